@@ -1148,6 +1148,167 @@ static hipError_t gemm_go(const GemmArgsD &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// activations as the matmuls take them: v_exp and v_rcp; exp(v) - 1 of xIELU loses what a bf16 output does not keep
+__device__ __forceinline__ float activate_fast(float v, int act, const Epilogue &e) {
+    switch (act) {
+        case BITNET_HIP_ACT_SILU: return v * __builtin_amdgcn_rcpf(1.0f + __expf(-v));
+        case BITNET_HIP_ACT_SIGMOID: return __builtin_amdgcn_rcpf(1.0f + __expf(-v));
+        case BITNET_HIP_ACT_GELU_TANH: return v * __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * gelu_argument(v)));
+        case BITNET_HIP_ACT_XIELU: return 0.5f * v + (v > 0.f ? e.act_a * v * v : e.act_b * (__expf(v) - 1.0f - v));
+        default: return activate(v, act);
+    }
+}
+
+// ---- few rows ---------------------------------------------------------------------------------------------------------
+// The same product where its tiles of 64 x 64 would leave most of the chip idle, or wait for K steps one by one (a step of such a tile takes 0.3 to
+// 0.4 us whatever is in flight: DMA, barrier, LDS reads and MFMAs of one workgroup follow one another).  A workgroup makes 16 FN columns of 16 FM rows;
+// its eight waves share the K columns out, 64 at a time in turn, each with its own buffers (R) and no barrier, and add up in LDS at the end.
+// Measured, us per launch, weights from HBM (this / 64 x 64 tiles): 16 x 2560 x 2560 7.3 / 13.2, 16 x 2560 x 6912 12.7 / 28.8, 61 x 2560 x 6912 19.4 / 34.1,
+// 61 x 6912 x 2560 14.8 / 17.3, 128 x 1536 x 4096 12.2 / 20.6, 1024 x 72 x 2560 7.1 / 13.4.
+template <int FN, int FM, int R>
+__global__ __launch_bounds__(512, 2) void k_dense_gemm_few(GemmArgsD p, int tiles_n, int tiles_m) {
+    extern __shared__ __attribute__((aligned(16))) f32x4 part[];  // [wave][fragment][lane]
+    constexpr int NW = 8;
+    const int units = p.k >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // each XCD a contiguous run of tiles, the row tiles of one weight tile side by side
+    const int total = tiles_n * tiles_m, per = (total + 7) >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
+    const int tn = id / tiles_m, tm = id % tiles_m;
+    const int m0 = tm * 16 * FM, n0 = tn * 16 * FN;
+    const int r16 = lane & 15, g = lane >> 4;
+    constexpr unsigned ROWS = 16 * (FM + FN), BUF = ROWS * 128;
+    const uint16_t *A = (const uint16_t *)p.a + (size_t)blockIdx.y * p.a_batch + (size_t)m0 * p.lda;
+    const uint16_t *W = p.w + (size_t)blockIdx.y * p.w_batch + (size_t)n0 * p.ldw;
+    const int rows_m = min(16 * FM, p.m - m0), rows_n = min(16 * FN, p.n - n0);
+    unsigned oa[2 * FM], ow[2 * FN];  // (lane offsets from the tile's first row, eight rows per instruction; rows past the end read the tile's own again)
+#pragma unroll
+    for (int i = 0; i < 2 * FM; ++i) {
+        const int r = i * 8 + (lane >> 3);
+        oa[i] = (unsigned)(min(r, rows_m - 1) * p.lda + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * FN; ++i) {
+        const int r = i * 8 + (lane >> 3);
+        ow[i] = (unsigned)(min(r, rows_n - 1) * p.ldw + ((lane & 7) ^ ((r >> 1) & 7)) * 8) * 2;
+    }
+    uint8_t *mine = (uint8_t *)part + wave * R * BUF;
+    const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)mine;
+    auto stage = [&](int u, int slot) {
+        const int k = min(u, units - 1) * 64;
+#pragma unroll
+        for (int i = 0; i < 2 * FN; ++i) dma1k(ow[i], W + k, base + slot * BUF + i * 1024);
+#pragma unroll
+        for (int i = 0; i < 2 * FM; ++i) dma1k(oa[i], A + k, base + slot * BUF + (2 * FN + i) * 1024);
+    };
+    f32x4 acc[FN][FM];
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < R; ++r) stage(wave + NW * r, r);
+    const int sw = (r16 >> 1) & 7;
+    for (int u = wave; u < units; u += NW * R) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * 2 * (FM + FN)) : "memory");
+            const uint8_t *lw = mine + r * BUF, *la = lw + FN * 2048;
+            bf16x8 fa[2][FM], fw[2][FN];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int q = ((h * 4 + g) ^ sw) * 16;
+#pragma unroll
+                for (int i = 0; i < FN; ++i) fw[h][i] = *reinterpret_cast<const bf16x8 *>(lw + (i * 16 + r16) * 128 + q);
+#pragma unroll
+                for (int j = 0; j < FM; ++j) fa[h][j] = *reinterpret_cast<const bf16x8 *>(la + (j * 16 + r16) * 128 + q);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            stage(u + NW * (r + R), r);
+            if (u + NW * r < units) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int i = 0; i < FN; ++i)
+#pragma unroll
+                        for (int j = 0; j < FM; ++j) acc[i][j] = mfma_bf16(fw[h][i], fa[h][j], acc[i][j]);
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j) part[(wave * FN * FM + i * FM + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    const bool vec = (p.ldc & 3) == 0 && (p.c_batch & 3) == 0 && ((uintptr_t)p.c & 15) == 0;
+    for (int f = wave; f < FN * FM; f += NW) {
+        f32x4 v = part[f * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += part[(w * FN * FM + f) * 64 + lane];
+        const int n = n0 + f / FM * 16 + g * 4, m = m0 + f % FM * 16 + r16;
+        if (m >= p.m) continue;
+        const size_t row = (size_t)blockIdx.y * p.c_batch + (size_t)m * p.ldc;
+        if (p.bias)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += p.bias[min(n + e, p.n - 1)];
+        if (p.gated) {
+            float r[2];
+#pragma unroll
+            for (int e = 0; e < 4; e += 2) r[e / 2] = activate_fast(v[e], p.act0, p.more) * v[e + 1];
+            uint16_t *dst = (uint16_t *)p.c + row + n / 2;
+            if (vec && n + 3 < p.n) {
+                *reinterpret_cast<uint32_t *>(dst) = (uint32_t)f2bf(r[0]) | (uint32_t)f2bf(r[1]) << 16;
+            } else {
+                if (n < p.n) dst[0] = f2bf(r[0]);
+                if (n + 2 < p.n) dst[1] = f2bf(r[1]);
+            }
+            continue;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = activate_fast(v[e], n + e < p.act_split ? p.act0 : p.act1, p.more);
+        if (p.more.mul) {
+            const int token = min(max(p.more.mul_tokens[*p.more.mul_at + m], 0), p.more.mul_rows - 1);
+            const uint16_t *mul = p.more.mul + (size_t)token * p.more.ld_mul;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] *= bf2f(mul[min(n + e, p.n - 1)]);
+        }
+        if (p.c_f32) {
+            float *dst = (float *)p.c + row + n;
+            if (vec && n + 3 < p.n) {
+                *reinterpret_cast<f32x4 *>(dst) = v;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < p.n) dst[e] = v[e];
+            }
+        } else {
+            uint16_t *dst = (uint16_t *)p.c + row + n;
+            if (vec && n + 3 < p.n) {
+                *reinterpret_cast<bf16x4 *>(dst) = bf16x4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < p.n) dst[e] = f2bf(v[e]);
+            }
+        }
+    }
+}
+
+template <int FN, int FM, int R>
+static hipError_t gemm_few_go(const GemmArgsD &a, hipStream_t s) {
+    const int tn = (a.n + 16 * FN - 1) / (16 * FN), tm = (a.m + 16 * FM - 1) / (16 * FM);
+    constexpr size_t lds = 8 * 1024 * (FN * FM > 2 * R * (FN + FM) ? FN * FM : 2 * R * (FN + FM));
+    if (lds > 65536) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_dense_gemm_few<FN, FM, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((k_dense_gemm_few<FN, FM, R>), dim3((tn * tm + 7) / 8 * 8, a.batch), dim3(512), lds, s, a, tn, tm);
+    return hipGetLastError();
+}
+
 // f32 activations: f32 multiply-adds on a 64 x 64 tile, 4 x 4 per thread
 template <bool GROUPED>
 __global__ __launch_bounds__(256) void k_dense_gemm_f32(GemmArgsD p) {
@@ -1226,7 +1387,16 @@ hipError_t launch_dense_gemm(const GemmArgsD &args, hipStream_t s) {
         hipLaunchKernelGGL(k_dense_gemm_f32<false>, dim3((a.n + 63) / 64, (a.m + 63) / 64, a.batch), dim3(256), 0, s, a);
         return hipGetLastError();
     }
-    if (a.more.mul) return a.c_f32 || a.gated ? hipErrorInvalidValue : gemm_go<64, 2, 2, 4, true>(a, s);
+    if (a.more.mul && (a.c_f32 || a.gated)) return hipErrorInvalidValue;
+    // one round of workgroups of the form for few rows, its smallest tile first (two per CU fit but share the CU's LDS-DMA: behind 256 the larger tile is ahead, and behind
+    // that the tiles of 64 x 64: 61 x 10240 x 2560 takes 20.3 to 25.5 us in this form and 18.3 in the other); short K leaves its waves without work (256: 5.2 / 4.3 us)
+    auto rounds = [&](int tn, int tm) { return ((long)(a.n + tn - 1) / tn * ((a.m + tm - 1) / tm) * a.batch + 255) / 256; };
+    if (a.k >= 512) {
+        if (rounds(16, 16) == 1) return gemm_few_go<1, 1, 2>(a, s);
+        if (rounds(32, 32) == 1) return gemm_few_go<2, 2, 1>(a, s);
+        if (rounds(32, 64) == 1) return gemm_few_go<2, 4, 1>(a, s);
+    }
+    if (a.more.mul) return gemm_go<64, 2, 2, 4, true>(a, s);
     auto tiles = [&](int t) { return (long)((a.n + t - 1) / t) * ((a.m + t - 1) / t) * a.batch; };
     if (a.k <= 1024 && tiles(64) >= 1024) return gemm_go<64, 2, 2, 2>(a, s);  // few steps: what counts is how many workgroups overlap their ends
     if (tiles(128) >= 200) {

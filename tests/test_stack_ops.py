@@ -83,6 +83,32 @@ def test_matmul(hip, pkg, m, n, k, f32):
         assert not got[:, n:].any()
 
 
+# the form for few rows: its three tiles at the edges of their ranges (one round of 256 workgroups), K that does not go round its eight waves, rows and columns
+# that end inside a tile, batches; the last two lie just behind the ranges.  Tolerances as in test_matmul: sums of k products in f32, one rounding to bf16.
+@pytest.mark.parametrize("m,n,k,batch", [(1, 1, 512, 1), (16, 4096, 576, 1), (17, 2048, 512, 1), (19, 40, 1984, 3), (33, 1000, 640, 1), (61, 4096, 512, 1), (64, 130, 4096, 2),
+                                         (65, 4090, 512, 1), (257, 1600, 768, 1), (2048, 72, 1536, 1), (64, 8200, 512, 1), (64, 100, 448, 1)])
+@pytest.mark.parametrize("form", ["f32", "bf16", "gated"])
+def test_matmul_few_rows(hip, pkg, m, n, k, batch, form):
+    if form == "gated":
+        n = u.up_to(n, 2)
+    g = rng(m, n, k)
+    a, w, b = u.rounded(g.standard_normal((batch, m, k))), u.rounded(g.standard_normal((batch, n, k)) / np.sqrt(k)), g.standard_normal(n).astype(np.float32)
+    want = np.stack([x.astype(np.float64) @ y.T.astype(np.float64) for x, y in zip(a, w)]) + b
+    ldc, act0, split = n + 4, pkg.ACT_NONE, n // 3
+    want[:, :, split:] = so.silu(want[:, :, split:]) if form != "gated" else want[:, :, split:]
+    if form == "gated":
+        act0, split, ldc = pkg.ACT_SILU | pkg.ACT_GATED, 0, n // 2 + 3
+        want = so.silu(want[:, :, ::2]) * want[:, :, 1::2]
+    elif split == 0:  # (no split: the first activation for all)
+        act0 = pkg.ACT_SILU
+    c = u.zeros_f32(batch * m, ldc) if form == "f32" else u.zeros_bf16(batch * m, ldc)
+    hip.dense_matmul_dev(u.dev_bf16(a), k, False, u.dev_bf16(w), k, m, n, k, c, ldc, form == "f32", bias=u.dev_f32(b), act0=act0, act1=pkg.ACT_SILU if split else 0, act_split=split,
+                         batch=batch, a_batch=m * k, w_batch=n * k, c_batch=m * ldc)
+    got = u.host(c).reshape(batch, m, ldc)
+    assert u.rms_error(got[:, :, :want.shape[2]], want) < (F32_TOL if form == "f32" else 3e-3)
+    assert not got[:, :, want.shape[2]:].any()
+
+
 def test_matmul_batched_f32(hip):
     g = rng(9)
     heads, m, n, k, step = 3, 70, 64, 64, 96
