@@ -306,6 +306,18 @@ __device__ __forceinline__ float group_sum(float v, float *slot) {
     return t;
 }
 
+// the same where nobody has used these floats before
+template <int NW>
+__device__ __forceinline__ float group_total(float v, float *slot) {
+    v = wave_sum(v);
+    if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float t = slot[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) t += slot[i];
+    return t;
+}
+
 __device__ __forceinline__ float gelu_argument(float v) { return 0.7978845608028654f * (v + 0.044715f * v * v * v); }  // sqrt(2 / pi)
 // BITNET_HIP_ACT_* without constants
 __device__ __forceinline__ float activate(float v, int act) {

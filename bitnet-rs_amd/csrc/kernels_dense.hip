@@ -4,6 +4,7 @@
 // Precision: residual stream, norms and accumulation are f32 everywhere.  The matmul multiplies bf16 activations on the matrix
 // cores, or -- a_f32 -- f32 activations with f32 multiply-adds; the matrix-vector product always multiplies f32 activations.
 #include <algorithm>
+#include <type_traits>
 
 #include "dense.hpp"
 
@@ -454,7 +455,7 @@ hipError_t launch_latent_rows(const LatentRows &a, hipStream_t s) {
 // ---- matrix-vector product --------------------------------------------------------------------------------------------
 // One launch per product of the decode step.  Every workgroup forms the whole input vector (L2-resident, a few KiB) in LDS --
 // norm, residual + norm, or gated norm -- then its waves take rows: LPR lanes per row, 16 bytes of weights per lane and chunk,
-// R rows x U chunks in flight.  The first block of weights is requested ahead of the input transform.
+// R rows x U chunks in flight.  The first block of weights is requested ahead of the input transform, and behind its loads.
 struct GemvK {
     GemvArgs a;
     LatentRows lat;
@@ -463,146 +464,125 @@ struct GemvK {
     int lat_wg;    // workgroup index that writes the latent row, or -1
 };
 
-template <bool MORE>
-__device__ void form_input(const VecIn &in, const float *x, int cols, int kp, float *xs, float *slot, bool writer) {
+// Loads return in order, so whatever a wave asked for ahead of its input it also waits for: the input's loads go out first, `weights` (the first rows' requests)
+// behind them, the arithmetic last -- it runs while the weights are on their way.
+// NR: sixteen-byte registers per thread, for vectors of up to 1024 NR elements; longer ones are formed in LDS.  slot: twelve floats.
+template <bool MORE, int NR, class F>
+__device__ __forceinline__ void form_input(const VecIn &in, const float *x, int cols, int kp, float *xs, float *slot, bool writer, F weights) {
     const int tid = threadIdx.x;
     const int n = in.n;
     if (in.kind == BITNET_HIP_IN_PLAIN) {
         if ((cols & 3) == 0 && ((uintptr_t)x & 15) == 0) {
             constexpr int NV = 8;  // sixteen-byte loads in flight per thread
             const int c4 = cols >> 2, k4 = kp >> 2;
-            for (int i0 = tid; i0 < k4; i0 += 256 * NV) {
-                f32x4 v[NV];
+            f32x4 v[NV];
+            auto load = [&](int i0) {
 #pragma unroll
                 for (int j = 0; j < NV; ++j) v[j] = reinterpret_cast<const f32x4 *>(x)[min(i0 + 256 * j, c4 - 1)];
+            };
+            auto store = [&](int i0) {
 #pragma unroll
                 for (int j = 0; j < NV; ++j) {
                     const int i = i0 + 256 * j;
                     if (i < k4) reinterpret_cast<f32x4 *>(xs)[i] = i < c4 ? v[j] : f32x4{0.f, 0.f, 0.f, 0.f};
                 }
+            };
+            load(tid);
+            weights();
+            store(tid);
+            for (int i0 = tid + 256 * NV; i0 < k4; i0 += 256 * NV) {
+                load(i0);
+                store(i0);
             }
         } else {
+            weights();
             for (int i = tid; i < kp; i += 256) xs[i] = i < cols ? x[i] : 0.f;
         }
         __syncthreads();
         return;
     }
-    constexpr int NR = 4;  // float4 registers: vectors of up to 4096 elements
+    const bool added = in.kind >= BITNET_HIP_IN_RESIDUAL_NORM && in.y, normed = added && in.post_weight, last_norm = in.kind < BITNET_HIP_IN_CONCAT, two = in.kind == BITNET_HIP_IN_CONCAT;
     if ((n & 3) == 0 && n <= 1024 * NR) {
-        f32x4 xv[NR];
+        f32x4 xv[NR], yv[NR], pw[NR], sc[NR], yg[NR], wv[NR], bv[NR], gv[NR];
         const int n4 = n >> 2;
+        const bool scaled = normed && in.scale, y_gated = MORE && added && in.y_gate, shifted = last_norm && in.center && in.bias, gated = last_norm && in.gate;
+        auto load = [&](f32x4 (&v)[NR], const float *from) {
 #pragma unroll
-        for (int j = 0; j < NR; ++j) {
-            const int i = tid + 256 * j;
-            const f32x4 v = reinterpret_cast<const f32x4 *>(x)[min(i, n4 - 1)];
-            xv[j] = v * (i < n4 ? 1.0f : 0.0f);
-        }
-        if (in.kind >= BITNET_HIP_IN_RESIDUAL_NORM && in.y && !in.post_weight) {
-            f32x4 yv[NR], yg[NR];
-#pragma unroll
-            for (int j = 0; j < NR; ++j) {
-                yv[j] = reinterpret_cast<const f32x4 *>(in.y)[min(tid + 256 * j, n4 - 1)];
-                yg[j] = MORE && in.y_gate ? reinterpret_cast<const f32x4 *>(in.y_gate)[min(tid + 256 * j, n4 - 1)] : f32x4{1.f, 1.f, 1.f, 1.f};
-            }
-#pragma unroll
-            for (int j = 0; j < NR; ++j) {
-                const int i = tid + 256 * j;
-                if (i >= n4) continue;
-                xv[j] += in.mult * yv[j] * yg[j];
-                if (writer && in.x_out) reinterpret_cast<f32x4 *>(in.x_out)[i] = xv[j];
-            }
-        } else if (in.kind >= BITNET_HIP_IN_RESIDUAL_NORM && in.y) {
-            f32x4 yv[NR], pw[NR], sc[NR];
+            for (int j = 0; j < NR; ++j) v[j] = reinterpret_cast<const f32x4 *>(from)[min(tid + 256 * j, n4 - 1)];
+        };
+        load(xv, x);
+        if (added) load(yv, in.y);
+        if (normed) load(pw, in.post_weight);
+        if (scaled) load(sc, in.scale);
+        if (y_gated) load(yg, in.y_gate);
+        if (last_norm) load(wv, in.weight);
+        if (two) load(wv, in.x2);
+        if (shifted) load(bv, in.bias);
+        if (gated) load(gv, in.gate);
+        weights();
+        auto squares = [&](const f32x4 (&v)[NR]) {
             float ss = 0.f;
 #pragma unroll
-            for (int j = 0; j < NR; ++j) {
-                const int i = tid + 256 * j;
-                const int c = min(i, n4 - 1);
-                const f32x4 v = reinterpret_cast<const f32x4 *>(in.y)[c];
-                yv[j] = v * (i < n4 ? 1.0f : 0.0f);
-                pw[j] = reinterpret_cast<const f32x4 *>(in.post_weight)[c];
-            }
-            if (in.scale) {
-#pragma unroll
-                for (int j = 0; j < NR; ++j) sc[j] = reinterpret_cast<const f32x4 *>(in.scale)[min(tid + 256 * j, n4 - 1)];
-            } else {
-#pragma unroll
-                for (int j = 0; j < NR; ++j) sc[j] = f32x4{1.f, 1.f, 1.f, 1.f};
-            }
-            if (MORE && in.y_gate)
-#pragma unroll
-                for (int j = 0; j < NR; ++j) sc[j] *= reinterpret_cast<const f32x4 *>(in.y_gate)[min(tid + 256 * j, n4 - 1)];
-#pragma unroll
-            for (int j = 0; j < NR; ++j) ss += yv[j].x * yv[j].x + yv[j].y * yv[j].y + yv[j].z * yv[j].z + yv[j].w * yv[j].w;
-            const float inv = 1.0f / sqrtf(group_sum<4>(ss, slot) / (float)in.mean_n + in.eps);
+            for (int j = 0; j < NR; ++j) ss += tid + 256 * j < n4 ? (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w) : 0.f;
+            return ss;
+        };
+        const float count = (float)in.mean_n, eps = in.eps, offset = in.offset;
+        auto inverse = [=](float ss) { return 1.0f / sqrtf(ss / count + eps); };
+        if (added) {
+            const float inv = normed ? inverse(group_total<4>(squares(yv), slot)) : 1.0f;
 #pragma unroll
             for (int j = 0; j < NR; ++j) {
                 const int i = tid + 256 * j;
-                if (i >= n4) continue;
-                xv[j] += sc[j] * (yv[j] * inv * (in.offset + pw[j]));
-                if (writer && in.x_out) reinterpret_cast<f32x4 *>(in.x_out)[i] = xv[j];
+                f32x4 v = yv[j] * (normed ? inv : in.mult);
+                if (normed) v *= offset + pw[j];
+                if (scaled) v *= sc[j];
+                if (y_gated) v *= yg[j];
+                xv[j] += v;
+                if (writer && in.x_out && i < n4) reinterpret_cast<f32x4 *>(in.x_out)[i] = xv[j];
             }
         }
-        if (in.kind >= BITNET_HIP_IN_CONCAT) {
-            const bool two = in.kind == BITNET_HIP_IN_CONCAT;
+        if (!last_norm) {
 #pragma unroll
             for (int j = 0; j < NR; ++j) {
                 const int i = tid + 256 * j;
                 if (i >= n4) continue;
                 reinterpret_cast<f32x4 *>(xs)[i] = xv[j];
-                if (two) reinterpret_cast<f32x4 *>(xs)[n4 + i] = reinterpret_cast<const f32x4 *>(in.x2)[i];
+                if (two) reinterpret_cast<f32x4 *>(xs)[n4 + i] = wv[j];
             }
             for (int i = (two ? 2 : 1) * n + tid; i < kp; i += 256) xs[i] = 0.f;
             __syncthreads();
             return;
         }
-        f32x4 bv[NR];
         if (in.center) {
             float t = 0.f;
 #pragma unroll
-            for (int j = 0; j < NR; ++j) {
-                t += (xv[j].x + xv[j].y) + (xv[j].z + xv[j].w);
-                bv[j] = in.bias ? reinterpret_cast<const f32x4 *>(in.bias)[min(tid + 256 * j, n4 - 1)] : f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-            const float mean = group_sum<4>(t, slot) / (float)in.mean_n;
+            for (int j = 0; j < NR; ++j) t += tid + 256 * j < n4 ? (xv[j].x + xv[j].y) + (xv[j].z + xv[j].w) : 0.f;
+            const float mean = group_total<4>(t, slot + 4) / (float)in.mean_n;
 #pragma unroll
-            for (int j = 0; j < NR; ++j) xv[j] -= tid + 256 * j < n4 ? mean : 0.f;
+            for (int j = 0; j < NR; ++j) xv[j] -= mean;
         }
-        f32x4 wv[NR], gv[NR];
-        float ss = 0.f;
-#pragma unroll
-        for (int j = 0; j < NR; ++j) {
-            const int i = tid + 256 * j;
-            wv[j] = reinterpret_cast<const f32x4 *>(in.weight)[min(i, n4 - 1)];
-            ss += xv[j].x * xv[j].x + xv[j].y * xv[j].y + xv[j].z * xv[j].z + xv[j].w * xv[j].w;
-        }
-        if (in.gate) {
-#pragma unroll
-            for (int j = 0; j < NR; ++j) gv[j] = reinterpret_cast<const f32x4 *>(in.gate)[min(tid + 256 * j, n4 - 1)];
-        } else {
-#pragma unroll
-            for (int j = 0; j < NR; ++j) gv[j] = f32x4{1.f, 1.f, 1.f, 1.f};
-        }
-        const float inv = 1.0f / sqrtf(group_sum<4>(ss, slot) / (float)in.mean_n + in.eps);
+        const float inv = inverse(group_total<4>(squares(xv), slot + 8));
 #pragma unroll
         for (int j = 0; j < NR; ++j) {
             const int i = tid + 256 * j;
             if (i >= n4) continue;
-            f32x4 r = xv[j] * inv * (in.offset + wv[j]) * gv[j];
-            if (in.center) r += bv[j];
+            f32x4 r = xv[j] * inv * (offset + wv[j]);
+            if (gated) r *= gv[j];
+            if (shifted) r += bv[j];
             reinterpret_cast<f32x4 *>(xs)[i] = r;
             if (writer && in.h_out) reinterpret_cast<f32x4 *>(in.h_out)[i] = r;
         }
     } else {
+        weights();
         float ss = 0.f;
-        if (in.kind >= BITNET_HIP_IN_RESIDUAL_NORM && in.y && !in.post_weight) {
+        if (added && !normed) {
             for (int i = tid; i < n; i += 256) {
                 const float v = x[i] + in.mult * in.y[i] * (MORE && in.y_gate ? in.y_gate[i] : 1.0f);
                 xs[i] = v;
                 if (writer && in.x_out) in.x_out[i] = v;
                 ss += v * v;
             }
-        } else if (in.kind >= BITNET_HIP_IN_RESIDUAL_NORM && in.y) {
+        } else if (added) {
             for (int i = tid; i < n; i += 256) ss += in.y[i] * in.y[i];
             const float inv = 1.0f / sqrtf(group_sum<4>(ss, slot) / (float)in.mean_n + in.eps);
             ss = 0.f;
@@ -618,8 +598,7 @@ __device__ void form_input(const VecIn &in, const float *x, int cols, int kp, fl
                 ss += x[i] * x[i];
             }
         }
-        if (in.kind >= BITNET_HIP_IN_CONCAT) {
-            const bool two = in.kind == BITNET_HIP_IN_CONCAT;
+        if (!last_norm) {
             for (int i = tid; two && i < n; i += 256) xs[n + i] = in.x2[i];
             for (int i = (two ? 2 : 1) * n + tid; i < kp; i += 256) xs[i] = 0.f;
             __syncthreads();
@@ -657,14 +636,17 @@ __device__ __forceinline__ float lanes_total(float v) {
 }
 
 // MORE: whatever bitnet_hip_epilogue and a gate on the residual ask for
-template <int LPR, int R, int U, bool MORE>
+template <int LPR, int R, int U, bool MORE, int NR>
 __global__ __launch_bounds__(256) void k_dense_gemv(GemvK p) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
-    __shared__ float slot[4];
+    __shared__ float slot[12];
     __shared__ float wbv[4];
     __shared__ int wbi[4];
     const GemvArgs &a = p.a;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // (every argument at once: read where they are used, behind branches, they are a chain of scalar loads ahead of the first vector load)
+    asm volatile("" ::"s"(a.in.x), "s"(a.in.y), "s"(a.in.post_weight), "s"(a.in.scale), "s"(a.in.weight), "s"(a.in.bias), "s"(a.in.gate), "s"(a.in.x_out), "s"(a.in.kind), "s"(a.in.n),
+                 "s"(a.in.center), "s"(a.in.mean_n), "s"(a.in.x2), "s"(a.w), "s"(a.rows), "s"(a.cols), "s"(a.ld), "s"(p.kp), "s"(p.groups), "s"(p.lat_wg));
     if ((int)blockIdx.x == p.lat_wg) {  // (the whole workgroup)
         if (blockIdx.y > 0) return;
         if (p.lat.f32)
@@ -712,9 +694,11 @@ __global__ __launch_bounds__(256) void k_dense_gemv(GemvK p) {
             }
         }
     };
-    if (g < p.groups) fetch(g, 0);
-    if (conv && g < p.groups) fetch_past(g);
-    form_input<MORE>(a.in, a.in.x + (size_t)b * a.x_batch, a.cols, p.kp, xs, slot, blockIdx.x == 0 && b == 0);
+    // (the taps are summed as they arrive: ahead of the weights, too)
+    form_input<MORE, NR>(a.in, a.in.x + (size_t)b * a.x_batch, a.cols, p.kp, xs, slot, blockIdx.x == 0 && b == 0, [&] {
+        if (conv && g < p.groups) fetch_past(g);
+        if (g < p.groups) fetch(g, 0);
+    });
     float bv = -INFINITY;
     int bi = 0x7fffffff;
     for (; g < p.groups; g += n_wg * 4) {
@@ -824,11 +808,21 @@ __global__ __launch_bounds__(256) void k_dense_gemv(GemvK p) {
     }
 }
 
+// LPR lanes per row take rows of up to 64, 256 and any number of columns: one, two and five steps at the most are needed of them
 template <int LPR, int R, bool MORE>
 static void gemv_go(int u, const GemvK &k, dim3 grid, hipStream_t s) {
     const size_t lds = (size_t)k.kp * 4;
-    void (*fn)(GemvK) = u == 1 ? k_dense_gemv<LPR, R, 1, MORE> : u == 2 ? k_dense_gemv<LPR, R, 2, MORE> : u == 3 ? k_dense_gemv<LPR, R, 3, MORE>
-                      : u == 4 ? k_dense_gemv<LPR, R, 4, MORE> : k_dense_gemv<LPR, R, 5, MORE>;
+    void (*fn)(GemvK);
+    if constexpr (LPR == 64) {
+        auto pick = [&](auto nr) {
+            constexpr int NR = decltype(nr)::value;
+            return u == 1 ? k_dense_gemv<64, R, 1, MORE, NR> : u == 2 ? k_dense_gemv<64, R, 2, MORE, NR> : u == 3 ? k_dense_gemv<64, R, 3, MORE, NR>
+                 : u == 4 ? k_dense_gemv<64, R, 4, MORE, NR> : k_dense_gemv<64, R, 5, MORE, NR>;
+        };
+        fn = k.a.in.n <= 3072 ? pick(std::integral_constant<int, 3>()) : pick(std::integral_constant<int, 4>());
+    } else {
+        fn = LPR == 16 && u > 1 ? k_dense_gemv<LPR, R, 2, MORE, 1> : k_dense_gemv<LPR, R, 1, MORE, 1>;
+    }
     if (lds > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(fn, grid, dim3(256), lds, s, k);
 }

@@ -403,13 +403,12 @@ __global__ __launch_bounds__(256) void k_experts_out(OutK p) {
         }
     };
     int g = blockIdx.x * 4 + wave;
-    if (g < p.groups) fetch(g, 0);
     const int steps = (end + U - 1) / U * U, total = steps * CH / 4;  // (identity experts have no columns)
     const float through = a.identity ? *a.identity : 0.f, scale0 = a.x0_scale ? *a.x0_scale : 1.0f;
     constexpr int AH = 12;
-    for (int i0 = tid; i0 < total; i0 += 256 * AH) {
-        f32x4 v[AH];
-        float in[AH];  // zero: past a segment's columns
+    f32x4 v[AH];
+    float in[AH];  // zero: past a segment's columns
+    auto load = [&](int i0) {
 #pragma unroll
         for (int j = 0; j < AH; ++j) {
             const int i = i0 + 256 * j, c = i / (CH / 4), x = max(c - p.c0, 0), q = min((int)((unsigned)x * p.magic >> 20), max(n_real - 1, 0));
@@ -418,9 +417,19 @@ __global__ __launch_bounds__(256) void k_experts_out(OutK p) {
             in[j] = col < cols && c < end ? (first ? scale0 : 1.0f) : 0.f;
             v[j] = *reinterpret_cast<const f32x4 *>((first ? a.x0 : a.x1 + (size_t)q * a.ldx1) + min(col, cols - 4));
         }
+    };
+    auto store = [&](int i0) {
 #pragma unroll
         for (int j = 0; j < AH; ++j)
             if (i0 + 256 * j < total) reinterpret_cast<f32x4 *>(xs)[i0 + 256 * j] = in[j] != 0.f ? in[j] * v[j] : f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    // (loads return in order: the weights are requested behind the vector, which is stored while they are on their way)
+    load(tid);
+    if (g < p.groups) fetch(g, 0);
+    store(tid);
+    for (int i0 = tid + 256 * AH; i0 < total; i0 += 256 * AH) {
+        load(i0);
+        store(i0);
     }
     __syncthreads();
     const int n_wg = gridDim.x;
