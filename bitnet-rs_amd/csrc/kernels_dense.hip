@@ -33,8 +33,31 @@ __global__ void k_embed_bf16(const uint16_t *__restrict__ table, size_t ld, cons
         }
         return;
     }
+    // four columns at a time: a row of one token is a chain of three dependent loads (position, token, columns), and no loop of them
+    const uint16_t *row = table + (size_t)tok * ld;
+    const bool vec = width % 4 == 0 && ld % 4 == 0 && ((uintptr_t)table & 7) == 0 && (((uintptr_t)out | (uintptr_t)norm_w) & 15) == 0;
+    auto four = [&](int i) {
+        const u32x2 x = *reinterpret_cast<const u32x2 *>(row + i);
+        return scale * f32x4{bf2f(x.x & 0xffffu), bf2f(x.x >> 16), bf2f(x.y & 0xffffu), bf2f(x.y >> 16)};
+    };
+    if (norm_w && vec && width <= 4096) {
+        f32x4 v[4], w[4];
+        const int n4 = width / 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[j] = reinterpret_cast<const f32x4 *>(norm_w)[min((int)threadIdx.x + 256 * j, n4 - 1)];
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = four(4 * min((int)threadIdx.x + 256 * j, n4 - 1));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ss += (int)threadIdx.x + 256 * j < n4 ? (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w) : 0.f;
+        const float inv = 1.0f / sqrtf(group_total<4>(ss, slot) / (float)width + eps);
+        f32x4 *o = reinterpret_cast<f32x4 *>(out + (size_t)blockIdx.x * width);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if ((int)threadIdx.x + 256 * j < n4) o[threadIdx.x + 256 * j] = v[j] * inv * w[j];
+        return;
+    }
     if (norm_w) {
-        const uint16_t *row = table + (size_t)tok * ld;
         constexpr int NR = 16;  // rows of up to 4096 columns in registers, what lies behind is read again
         float ss = 0.f, v[NR], w[NR];
 #pragma unroll
@@ -54,12 +77,16 @@ __global__ void k_embed_bf16(const uint16_t *__restrict__ table, size_t ld, cons
         for (int i = threadIdx.x + 256 * NR; i < width; i += 256) o[i] = scale * bf2f(row[i]) * inv * norm_w[i];
         return;
     }
-    for (int i = threadIdx.x; i < width; i += blockDim.x) out[(size_t)blockIdx.x * width + i] = scale * bf2f(table[(size_t)tok * ld + i]);
+    if (vec) {
+        for (int i = 4 * (threadIdx.x + 256 * blockIdx.y); i < width; i += 1024 * gridDim.y) *reinterpret_cast<f32x4 *>(out + (size_t)blockIdx.x * width + i) = four(i);
+    } else {
+        for (int i = threadIdx.x + 256 * blockIdx.y; i < width; i += 256 * gridDim.y) out[(size_t)blockIdx.x * width + i] = scale * bf2f(row[i]);
+    }
 }
 
 hipError_t launch_embed_bf16(const uint16_t *table, size_t ld, const int *tokens, const int *offset, int n, int width, int vocab, float scale,
                              const float *norm_w, float eps, const TokenPairs &pairs, float *out, hipStream_t s) {
-    const int parts = pairs.table && n == 1 ? (width + 1023) / 1024 : 1;  // (one token: its row at once)
+    const int parts = !norm_w && n == 1 ? (width + 1023) / 1024 : 1;  // (one token: its row at once)
     hipLaunchKernelGGL(k_embed_bf16, dim3(n, parts), dim3(256), 0, s, table, ld, tokens, offset, width, vocab, scale, norm_w, eps, pairs, out);
     return hipGetLastError();
 }
