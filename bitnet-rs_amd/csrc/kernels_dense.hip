@@ -4,6 +4,8 @@
 // Precision: residual stream, norms and accumulation are f32 everywhere.  The matmul multiplies bf16 activations on the matrix
 // cores, or -- a_f32 -- f32 activations with f32 multiply-adds; the matrix-vector product always multiplies f32 activations.
 #include <algorithm>
+#include <cmath>
+#include <iterator>
 #include <type_traits>
 
 #include "dense.hpp"
@@ -907,9 +909,8 @@ hipError_t launch_dense_gemv(const GemvArgs &a, int *n_wg_out, hipStream_t s) {
 
 // ---- many-row matmul --------------------------------------------------------------------------------------------------
 // C[m][n] = act(A[m][k] . W[n][k]^T + bias).  Workgroup tile TN x TM in WN x WM waves, K steps of 64 columns staged in LDS by LDS-DMA,
-// ST buffers.  256 x 256 in eight waves of 128 x 64 where the launch has the tiles for it (half the bytes per
-// product of 128 x 128, and a fragment read from LDS feeds four to eight MFMAs), 128 x 128, and 64 x 64 with four buffers for launches
-// that do not fill the chip and would wait for memory at every step.  LDS image of a row: eight 16-byte units, unit q stored at
+// ST buffers; from 256 x 256 in eight waves of 128 x 64 (half the bytes per product of 128 x 128, and a fragment read from LDS feeds
+// four to eight MFMAs) down to 64 x 64 with four buffers, the one that fills the chip best (launch_dense_gemm).  LDS image of a row: eight 16-byte units, unit q stored at
 // q ^ ((row >> 1) & 7) (activations) or q ^ weight_key(row) (weights): the sixteen rows of a ds_read_b128 cover all 64 banks once.  The
 // MFMA's A operand is the weight tile (rows = output columns n), its B operand the activation tile; for bf16
 // outputs row r of weight fragment i is column 4 FN (r / 4) + 4 i + r % 4 of the wave's tile, so that a lane ends up with 4 FN consecutive
@@ -1153,14 +1154,14 @@ static hipError_t grouped_go(const GemmArgsD &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int T, int WN, int WM, int ST, bool MUL = false>
+template <int TN, int TM, int WN, int WM, int ST, bool MUL = false>
 static hipError_t gemm_go(const GemmArgsD &a, hipStream_t s) {
-    const int tn = (a.n + T - 1) / T, tm = (a.m + T - 1) / T, swz = (tn * tm) % 8 == 0 ? 1 : 0;
-    constexpr size_t lds = (size_t)ST * T * 256;
-    auto fn = MUL       ? k_dense_gemm<T, T, WN, WM, ST, false, false, false, MUL>
-              : a.gated ? k_dense_gemm<T, T, WN, WM, ST, false, false, true>
-              : a.c_f32 ? k_dense_gemm<T, T, WN, WM, ST, true>
-                        : k_dense_gemm<T, T, WN, WM, ST, false>;
+    const int tn = (a.n + TN - 1) / TN, tm = (a.m + TM - 1) / TM, swz = (tn * tm) % 8 == 0 ? 1 : 0;
+    constexpr size_t lds = (size_t)ST * (TN + TM) * 128;
+    auto fn = MUL       ? k_dense_gemm<TN, TM, WN, WM, ST, false, false, false, MUL>
+              : a.gated ? k_dense_gemm<TN, TM, WN, WM, ST, false, false, true>
+              : a.c_f32 ? k_dense_gemm<TN, TM, WN, WM, ST, true>
+                        : k_dense_gemm<TN, TM, WN, WM, ST, false>;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
@@ -1411,22 +1412,35 @@ hipError_t launch_dense_gemm(const GemmArgsD &args, hipStream_t s) {
     if (a.more.mul && (a.c_f32 || a.gated)) return hipErrorInvalidValue;
     // one round of workgroups of the form for few rows, its smallest tile first (two per CU fit but share the CU's LDS-DMA: behind 256 the larger tile is ahead, and behind
     // that the tiles of 64 x 64: 61 x 10240 x 2560 takes 20.3 to 25.5 us in this form and 18.3 in the other); short K leaves its waves without work (256: 5.2 / 4.3 us)
-    auto rounds = [&](int tn, int tm) { return ((long)(a.n + tn - 1) / tn * ((a.m + tm - 1) / tm) * a.batch + 255) / 256; };
+    auto one_round = [&](int tn, int tm) { return ((long)(a.n + tn - 1) / tn) * ((a.m + tm - 1) / tm) * a.batch <= 256; };
     if (a.k >= 512) {
-        if (rounds(16, 16) == 1) return gemm_few_go<1, 1, 2>(a, s);
-        if (rounds(32, 32) == 1) return gemm_few_go<2, 2, 1>(a, s);
-        if (rounds(32, 64) == 1) return gemm_few_go<2, 4, 1>(a, s);
+        if (one_round(16, 16)) return gemm_few_go<1, 1, 2>(a, s);
+        if (one_round(32, 32)) return gemm_few_go<2, 2, 1>(a, s);
+        if (one_round(32, 64)) return gemm_few_go<2, 4, 1>(a, s);
     }
-    if (a.more.mul) return gemm_go<64, 2, 2, 4, true>(a, s);
-    auto tiles = [&](int t) { return (long)((a.n + t - 1) / t) * ((a.m + t - 1) / t) * a.batch; };
-    if (a.k <= 1024 && tiles(64) >= 1024) return gemm_go<64, 2, 2, 2>(a, s);  // few steps: what counts is how many workgroups overlap their ends
-    if (tiles(128) >= 200) {
-        // measured per K step: 2.05 us for a round of 256 large tiles (one per CU), 1.15 us for a round of 512 of the others (two per CU);
-        // a column tile of the large kind that sticks out over the last column costs a third more
-        const double large = (a.n % 256 ? 2.7 : 2.05) * ((tiles(256) + 255) / 256), small = 1.15 * ((tiles(128) + 511) / 512);
-        return large <= small ? gemm_go<256, 2, 4, 2>(a, s) : gemm_go<128, 2, 2, 2>(a, s);
+    if (a.more.mul) return gemm_go<64, 64, 2, 2, 4, true>(a, s);
+    auto tiles = [&](int tn, int tm) { return (double)((a.n + tn - 1) / tn) * ((a.m + tm - 1) / tm) * a.batch; };
+    if (a.k <= 1024 && tiles(64, 64) >= 1024) return gemm_go<64, 64, 2, 2, 2>(a, s);  // few steps: what counts is how many workgroups overlap their ends
+    // The tile whose launch is the shortest by what was measured (us, bf16 and f32 outputs, m 400 to 4096, n 1536 to 12288, k 1536 to 8192): a step of 64 columns and a
+    // round's start and end.  The large ones stand alone on their CU and run in rounds of 256; of 64 x 128 two fit, but a second one costs more than half a round; a CU
+    // takes up to four of 64 x 64.  Three buffers where LDS has the room: 128 x 256 takes 0.80 us a step with them and 0.96 with two.  4096 x 3072 x 3072:
+    // 256 x 256 leaves a quarter of the CUs out (76 us), 192 x 256 is one full round (69); 2048 x 2560 x 6912: 128 x 192 80 us, 128 x 128 in four waves 114.
+    // Outputs whose rows do not start on sixteen bytes are stored one by one, which costs the most at the largest tiles.
+    const double steps = a.k / 64, slow = (a.ldc & 7) == 0 && (a.c_batch & 7) == 0 && ((uintptr_t)a.c & 15) == 0 ? 0.0 : 40.0 / 65536;
+    auto rounds = [&](int tn, int tm, double step, double ends) { return std::ceil(tiles(tn, tm) / 256) * (steps * step + ends + slow * tn * tm); };
+    const double t64 = tiles(64, 64) / 256, t128 = tiles(64, 128);
+    const double us[] = {slow ? 1e30 : rounds(256, 256, 1.27, 13), slow ? 1e30 : rounds(192, 256, 1.15, 12), rounds(128, 256, 0.80, 6), rounds(128, 192, 0.68, 4.5),
+                         rounds(128, 128, 0.48, 5.5), steps * (t128 <= 256 ? 0.40 : 0.62 * std::ceil(t128 / 512)) + 3.5 + slow * 64 * 128,
+                         steps * 0.27 * (t64 > 1 ? t64 : 1) + 3 + slow * 64 * 64};
+    switch (std::min_element(std::begin(us), std::end(us)) - us) {
+        case 0: return gemm_go<256, 256, 2, 4, 2>(a, s);
+        case 1: return gemm_go<192, 256, 2, 4, 2>(a, s);
+        case 2: return gemm_go<128, 256, 2, 4, 3>(a, s);
+        case 3: return gemm_go<128, 192, 2, 4, 3>(a, s);
+        case 4: return gemm_go<128, 128, 2, 4, 4>(a, s);
+        case 5: return gemm_go<64, 128, 2, 2, 3>(a, s);
+        default: return gemm_go<64, 64, 2, 2, 4>(a, s);
     }
-    return gemm_go<64, 2, 2, 4>(a, s);
 }
 
 }  // namespace bitnet_hip

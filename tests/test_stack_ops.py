@@ -109,6 +109,31 @@ def test_matmul_few_rows(hip, pkg, m, n, k, batch, form):
     assert not got[:, :, want.shape[2]:].any()
 
 
+# every tile of the matmul where the launcher takes it (a whole number of them and ends inside one), and outputs that start on no sixteen bytes
+@pytest.mark.parametrize("m,n", [(4096, 4096), (4000, 4080), (4096, 3072), (3900, 3060), (2048, 3072), (2040, 4056), (2048, 2560), (1537, 2570), (1500, 2568), (700, 2552), (1531, 1528)])
+@pytest.mark.parametrize("form", ["f32", "bf16", "gated", "unaligned"])
+def test_matmul_tiles(hip, pkg, m, n, form):
+    import torch
+    k, g = 1088, torch.Generator(device="cuda").manual_seed(m + n)
+    a, w = (torch.randn(r, k, device="cuda", generator=g).bfloat16() for r in (m, n))
+    b = torch.randn(n, device="cuda", generator=g)
+    wd = (w.double() / np.sqrt(k)).bfloat16()
+    want = a.double() @ wd.double().T + b.double()
+    gated, f32 = form == "gated", form == "f32"
+    if gated:
+        want = torch.nn.functional.silu(want[:, ::2]) * want[:, 1::2]
+    else:
+        want[:, n // 3:] = torch.nn.functional.silu(want[:, n // 3:])
+    cols = want.shape[1]
+    ldc = cols + 5 if form == "unaligned" else u.up_to(cols, 64)
+    c = torch.zeros(m, ldc, device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
+    hip.dense_matmul_dev(a, k, False, wd, k, m, n, k, c, ldc, f32, bias=b, act0=pkg.ACT_SILU | pkg.ACT_GATED if gated else pkg.ACT_NONE, act1=0 if gated else pkg.ACT_SILU,
+                         act_split=0 if gated else n // 3)
+    torch.cuda.synchronize()
+    assert ((c[:, :cols].double() - want).norm() / want.norm()).item() < (F32_TOL if f32 else 3e-3)
+    assert not c[:, cols:].any()
+
+
 def test_matmul_batched_f32(hip):
     g = rng(9)
     heads, m, n, k, step = 3, 70, 64, 64, 96
