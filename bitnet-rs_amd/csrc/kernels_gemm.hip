@@ -112,6 +112,7 @@ __device__ __forceinline__ double qwave_sum_d(double v) {
 // subnormals and the first two binades of e2m3 are contiguous), so a digit is stored as a 6-bit sign-magnitude integer.  Row layout:
 // [256-block][lane group g 4][digit 3][MFMA m 2][chunk of 8 columns 4][6 bytes] = 576 bytes per block; inside a chunk the column at
 // offset o sits at k-slot 2 (o & 3) + (o >> 2) -- the order in which the weight expansion leaves its fp4 nibbles (expand16_fp4).
+// FP6 = 2: int8 planes in the order of k_gemm_few's operands, [row / 16][digit][256-block][MFMA 4][lane 64][16]: a wave reads a kilobyte at a time.
 template <int NDIG, int NV, int FP6 = 0>
 __global__ __launch_bounds__(256) void k_quant_rows(QuantArgs p) {
     static_assert(!FP6 || NDIG == 2, "the fp6 form carries the 2-digit form's integer");
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256) void k_quant_rows(QuantArgs p) {
     const float sc = __uint_as_float((uint32_t)(254 + S - be) << 23);     // 2^(S - E)
     const float inv_s = __uint_as_float((uint32_t)(be - S) << 23);        // 2^(E - S)
     if (tid == 0) p.inv_scale[row] = live ? inv_s : 0.0f;
-    if (FP6) {
+    if (FP6 == 1) {
         // q = rint(x 2^(S - E)) as f32 goes through LDS so that ONE lane owns the 32 columns of an MFMA operand (lane group g, MFMA m
         // of a 256-block): columns 32 u .. 32 u + 31 live in units 9 u .. 9 u + 7 of 16 bytes (the ninth unit of every 144 bytes is
         // padding: with it the sixteen lanes of a ds_read_b128 service group touch sixteen different units)
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(256) void k_quant_rows(QuantArgs p) {
         for (int i = tid; i < (p.kp >> 8) * 36; i += 256) reinterpret_cast<uint4 *>(rbase)[i] = reinterpret_cast<const uint4 *>(orow)[i];
         return;
     }
-    int8_t *base = p.planes + ((size_t)(row >> 4) * NDIG * 16 + (row & 15)) * p.kp;
+    int8_t *base = p.planes + (FP6 == 2 ? (size_t)(row >> 4) * NDIG * 16 * p.kp + (row & 15) * 16 : ((size_t)(row >> 4) * NDIG * 16 + (row & 15)) * p.kp);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int idx = tid + 256 * i;
@@ -250,7 +251,10 @@ __global__ __launch_bounds__(256) void k_quant_rows(QuantArgs p) {
         dg[2] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
         dg[3] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
 #pragma unroll
-        for (int d = 0; d < NDIG; ++d) *reinterpret_cast<uint32_t *>(base + (size_t)d * 16 * p.kp + 4 * idx) = dg[d];
+        for (int d = 0; d < NDIG; ++d) {
+            const int at = FP6 == 2 ? (idx >> 6) * 4096 + ((idx >> 2) & 3) * 1024 + ((idx >> 4) & 3) * 256 + (idx & 3) * 4 : 4 * idx;
+            *reinterpret_cast<uint32_t *>(base + (size_t)d * 16 * p.kp + at) = dg[d];
+        }
     }
 }
 
@@ -2082,6 +2086,108 @@ static void launch_quant_rows_w(const QuantArgs &q, bool fp6, hipStream_t stream
     }
 }
 
+// ---- few activation rows: the 2-digit form of an unscaled matrix -------------------------------------------------------------------------------------------
+// A short prompt's launches have few tiles of 256 rows (10 of them at 2560), and each walked its K steps alone: 1.1 us a step, 31 us for the down-projection.  Here a
+// workgroup makes RT row tiles of 16 by 16 tokens; its eight waves share the 256-column blocks out, both operands straight to registers in whole kilobytes (the quantiser
+// left the planes in that order), and add up in LDS: exact int32 sums, so every output is bit for bit that of the other forms.  RT = 2 where gate and up tiles meet.
+// (Two token tiles per workgroup, which expand the codes once for both: no faster up to 192 rows.)
+template <int RT>
+__global__ __launch_bounds__(512, 4) void k_gemm_few(GemmArgs p) {
+    extern __shared__ __attribute__((aligned(16))) v4i sums[];  // [wave][RT][digit][lane]
+    constexpr int NW = 8, PER = RT * 2;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+    const int n_tiles = (p.rows + 15) >> 4, tile0 = blockIdx.x * RT, tok0 = blockIdx.y * 16;
+    const uint8_t *wp[RT];
+    const int8_t *bp = p.planes + (size_t)blockIdx.y * p.nblk * 8192 + lane * 16;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) wp[r] = p.tiles + ((size_t)min(tile0 + r, n_tiles - 1) * p.nblk * 64 + lane) * 16;
+    gv4u w[RT], b[2][4];
+    auto fetch = [&](int blk) {
+        const int k = min(blk, p.nblk - 1);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) w[r] = *reinterpret_cast<const gv4u *>(wp[r] + (size_t)k * 1024);
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+#pragma unroll
+            for (int m = 0; m < 4; ++m) b[d][m] = *reinterpret_cast<const gv4u *>(bp + ((size_t)d * p.nblk + k) * 4096 + m * 1024);
+    };
+    v4i acc[RT][2];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r][0] = acc[r][1] = (v4i){0, 0, 0, 0};
+    fetch(wave);
+    for (int blk = wave; blk < p.nblk; blk += NW) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                const v4i a = gdecode16(w[r][m], p.lut);
+#pragma unroll
+                for (int d = 0; d < 2; ++d) acc[r][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, __builtin_bit_cast(v4i, b[d][m]), acc[r][d], 0, 0, 0);
+            }
+        if (blk + NW < p.nblk) fetch(blk + NW);
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) sums[(wave * PER + r * 2 + d) * 64 + lane] = acc[r][d];
+    __syncthreads();
+    if (wave >= (p.silu_mul ? RT / 2 : RT)) return;  // a wave per output tile: gate and up make one
+    const float is = p.inv_scale[tok0 + c];          // (padding rows: 0)
+    auto value = [&](int r, float (&v)[4]) {
+        v4i s[2];
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            s[d] = sums[(r * 2 + d) * 64 + lane];
+#pragma unroll
+            for (int x = 1; x < NW; ++x) s[d] += sums[(x * PER + r * 2 + d) * 64 + lane];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = combine_digits<2>(s, j) * is;
+    };
+    const int token = tok0 + c, ld = p.silu_mul ? p.rows >> 1 : p.rows, row = 16 * (p.silu_mul ? tile0 >> 1 : tile0 + wave) + 4 * g;
+    float v[4];
+    value(p.silu_mul ? 0 : wave, v);
+    if (RT == 2 && p.silu_mul) {
+        float up[4];
+        value(RT - 1, up);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = gsilu_mul(v[j], up[j]);
+    }
+    if (token >= p.m) return;
+    const size_t off = (size_t)token * ld + row;
+    if (p.yh) {  // (with silu_mul; ld % 4 == 0 checked by the launcher)
+        typedef _Float16 sh4 __attribute__((ext_vector_type(4)));
+        if (row >= ld) return;
+        sh4 o;
+        bool sat = false;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = gclamp_f16(v[j], sat);
+        gflush_sat(sat);
+        *reinterpret_cast<sh4 *>(p.yh + off) = o;
+    } else if ((ld & 3) == 0) {
+        if (row >= ld) return;
+        gv4f o = (gv4f){v[0], v[1], v[2], v[3]};
+        if (p.residual) o += *reinterpret_cast<const gv4f *>(p.residual + off);
+        *reinterpret_cast<gv4f *>(p.y + off) = o;
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (row + j < ld) p.y[off + j] = v[j] + (p.residual ? p.residual[off + j] : 0.0f);
+    }
+}
+
+// Prompt of bitnet-b1.58-2B-4T (QK256), ms with this / without: 16 tokens 1.76 / 3.39, 64 2.29 / 3.56, 128 2.88 / 3.62, 192 3.52 / 3.97, 256 4.11 / 4.02 (every workgroup
+// reads its 16 tokens' planes for itself: from there on the wide tiles are ahead).
+constexpr size_t kFewTokens = 192;
+static hipError_t launch_gemm_few(const Weights &w, QuantArgs q, const GemmArgs &a, hipStream_t stream) {
+    const unsigned n_tok = (unsigned)(q.m + 15) / 16, rt = a.silu_mul ? 2 : 1;
+    q.m_pad = (int)(16 * n_tok);
+    hipLaunchKernelGGL((q.kp <= 3072 ? k_quant_rows<2, 3, 2> : k_quant_rows<2, 8, 2>), dim3(q.m_pad), dim3(256), 0, stream, q);
+    g_last_gemm_tile = GemmTileChoice{2, 16, 8, 0, (int)(16 * rt)};
+    hipLaunchKernelGGL(rt == 2 ? k_gemm_few<2> : k_gemm_few<1>, dim3((unsigned)div_ceil(div_ceil(w.rows, 16), rt), n_tok), dim3(512), (size_t)8 * rt * 2 * 1024, stream, a);
+    return hipGetLastError();
+}
+
 template <int NDIG, int TTW>
 static hipError_t launch_gemm_t(const Weights &w, const QuantArgs &q, const GemmArgs &a, hipStream_t stream) {
     const int nv = (int)div_ceil((size_t)q.kp / 4, 256);
@@ -2502,9 +2608,11 @@ hipError_t launch_gemm_mfma(const Weights &w, const float *x, float *y, size_t m
         static const int f16a_mode = [] { const char *e = getenv("BITNET_HIP_GEMM_F16A"); return e ? atoi(e) : 0; }();
         if (f16a_mode && ndig == 2 && !w.scaled && lut_fits_f16w(w.lut) && w.cols % 256 == 0)
             return launch_gemm_f16(w, q, a, stream);
-        // unscaled matrices at 2 digits: the same integer on the fp6 x fp4 MFMA, on request (flag) or by BITNET_HIP_GEMM_FP6=1
-        if (gemm_takes_fp6(w, fu, ndig)) return launch_gemm_fp6(w, q, a, stream);
     }
+    // unscaled matrices at 2 digits: the same integer on the fp6 x fp4 MFMA, on request (flag) or by BITNET_HIP_GEMM_FP6=1
+    if (!fu.int8_form && gemm_takes_fp6(w, fu, ndig)) return launch_gemm_fp6(w, q, a, stream);
+    // (rows past 8192 columns do not fit the quantiser's registers; a pair of gate and up tiles wants them both in the matrix)
+    if (ndig == 2 && !w.scaled && m <= kFewTokens && w.cols <= 8192 && (!fu.silu_mul || w.rows % 32 == 0)) return launch_gemm_few(w, q, a, stream);
     if (ndig == 2) return launch_gemm_t<2, 4>(w, q, a, stream);
     if (ndig == 3) return launch_gemm_t<3, 2>(w, q, a, stream);
     return launch_gemm_t<4, 2>(w, q, a, stream);

@@ -788,7 +788,8 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
     // matrix cores as they stand (k_gemm_f16a, 320-row workgroups: one round of the chip at 4096 tokens) -- no quantiser launch, no second
     // rounding of values that were rounded to f16 already; q|k|v and gate|up keep the faster int8 digit planes behind their LayerNorm.
     const bool hybrid = h16 && hybrid_applies(N);
-    const int f6 = (chain || qb) ? 0 : fp6_flag(digits);
+    // (up to 192 rows the int8 digits have a form of their own, k_gemm_few: faster, and the same outputs bit for bit)
+    const int f6 = (chain || qb || N <= 192) ? 0 : fp6_flag(digits);
     static const int f6od_env = getenv("BITNET_HOST_PREFILL_FP6_OD") ? atoi(getenv("BITNET_HOST_PREFILL_FP6_OD")) : 0;  // experiment: o / down on the fp6 form too (non-hybrid)
     const int f6od = f6od_env ? f6 : 0;
     for (auto &L : layers_) {

@@ -303,6 +303,7 @@ def test_x_f16_handover_under_the_f16a_env_route_reads_f16_rows():
     assert p.returncode == 0 and "F16A_X_F16_OK" in p.stdout, p.stdout[-2000:] + p.stderr[-4000:]
 
 
+SILU_MUL = 1  # BITNET_HIP_FUSE_SILU_MUL
 INT8_DIGITS, FP6_DIGITS = 8, 16  # BITNET_HIP_FUSE_INT8_DIGITS, BITNET_HIP_FUSE_FP6_DIGITS
 
 
@@ -337,6 +338,29 @@ def test_fp6_form_is_the_int8_two_digit_product_bit_for_bit(hip, oracle, torch_,
     for i in range(len(pick)):
         assert cosine(got[i], want[i]) >= 0.99999, int(pick[i])
     hip.weights_free(h)
+
+
+# k_gemm_few against k_gemm_fp6 on the same integers: token tiles and rows that end inside, K blocks that do not go round its eight waves, every kind of output
+@pytest.mark.parametrize("rows,cols,m", [(16, 256, 1), (40, 260, 15), (256, 2560, 16), (96, 2304, 17), (2560, 6912, 64), (36, 4100, 191), (64, 8192, 192)])
+@pytest.mark.parametrize("paired", [False, True])
+def test_few_rows_are_the_wide_tiles_product_bit_for_bit(hip, torch_, rows, cols, m, paired):
+    rng = np.random.default_rng(rows * 3 + cols + m)
+    stride = -(-cols // 256) * 64
+    x = (rng.normal(0.1, 1.0, (m, cols)) * np.exp(rng.uniform(-3, 3, (m, 1)))).astype(np.float32)
+    parts = [hip.weights_upload_qk256(rng.integers(0, 256, rows * stride, dtype=np.uint8), rows, cols, stride) for _ in range(2 if paired else 1)]
+    h = hip.weights_concat(parts, interleave16=True) if paired and rows % 16 == 0 else parts[0]
+    flags = SILU_MUL if h != parts[0] else 0
+    rd = torch_.from_numpy(rng.normal(0, 1, (m, rows)).astype(np.float32)).cuda()
+    gd = torch_.from_numpy((rng.uniform(0.5, 1.5, cols) / 80).astype(np.float32)).cuda()
+    for kw in ({}, dict(ln_gamma=gd, ln_eps=1e-5), *(() if flags else (dict(residual=rd),))):
+        few = run_gemm(hip, torch_, h, x, rows, 2, flags=flags, **kw)
+        t = hip.matmul_last_tile()
+        assert t["scale_mode"] == 0 and t["waves"] == 8 and t["wave_tokens"] == 16, t
+        wide = run_gemm(hip, torch_, h, x, rows, 2, flags=flags | FP6_DIGITS, **kw)
+        assert hip.matmul_last_tile()["scale_mode"] == 6
+        assert not np.isnan(few).any() and np.array_equal(few, wide), (sorted(kw), float(np.abs(few - wide).max()))
+    for i in {h, *parts}:
+        hip.weights_free(i)
 
 
 FP6_EXPAND = 32  # BITNET_HIP_FUSE_FP6_EXPAND
