@@ -690,13 +690,16 @@ hipError_t launch_gqa_merge(const Gqa &g, const int *pos, int q0, int nq, const 
 // ---- prompt -----------------------------------------------------------------------------------------------------------
 // One workgroup: one head, four waves; a wave holds two slots of 16 queries: both maps of one query tile, or two tiles of the only map.  Key tiles
 // of 64 (every map's) and the values of the tile staged through registers into LDS one step ahead.
+// G = 2: two such groups of four waves share the keys of the same queries, tile by tile in turn, and meet in LDS at the end.  A prompt's last queries see all of its keys and its
+// first next to none: one group per workgroup left the longest walk (47 tiles of a 3000-token prompt) twice as long as a CU's fair share (28), 2.9 us a tile whatever its
+// neighbour does.  Heads that need more than 256 registers keep one group.
 // FAR: with a distance penalty, gates per column, or both.
-template <int NK, int NV, int MAPS, bool FAR>
-__global__ __launch_bounds__(256, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(Gqa p, const uint16_t *Q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, int n_qb) {
+template <int NK, int NV, int MAPS, bool FAR, int G>
+__global__ __launch_bounds__(256 * G, G == 2 ? 2 : 1) void k_gqa_prefill(Gqa p, const uint16_t *Q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, int n_qb) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int SLOTS = 2, QW = 16 * SLOTS / MAPS, KS = NK * 64 + 16, VS = 64 * 2 + 16, NVL = NV / 2;
-    uint8_t *lk = lds, *lv = lds + MAPS * 64 * KS;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    const int grp = G == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
+    uint8_t *lk = lds + grp * (MAPS * 64 * KS + NV * 16 * VS), *lv = lk + MAPS * 64 * KS;
     const int heads = (int)p.heads, dimp = (int)p.dimp, vdimp = (int)p.vdimp;
     // Consecutive workgroups go to the eight XCDs in turn.  Longest blocks first; an XCD keeps heads / 8 neighbouring heads of its own (their keys
     // and values stay in its L2), the heads left over move from XCD to XCD with the block so that all eight carry the same work.
@@ -725,7 +728,7 @@ __global__ __launch_bounds__(256, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(G
 #pragma unroll
     for (int t = 0; t < SLOTS; ++t) {
         // (finite: with chunks a tile may hold no key that a query sees; the sink counts once per query, four lanes share one)
-        m[t] = MAPS == 1 && p.sink ? p.sink[h] * kLog2e : -1e30f, l[t] = MAPS == 1 && p.sink && g == 0 ? 1.0f : 0.f;
+        m[t] = MAPS == 1 && p.sink && grp == 0 ? p.sink[h] * kLog2e : -1e30f, l[t] = MAPS == 1 && p.sink && g == 0 && grp == 0 ? 1.0f : 0.f;
 #pragma unroll
         for (int v = 0; v < NV; ++v) o[v][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -751,9 +754,9 @@ __global__ __launch_bounds__(256, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(G
     const FarPenalty far = far_penalty(p, h);
     // tiles from the first key of the workgroup's first query on; a wave leaves out what lies ahead of its own first key
     const int t_first = gqa_first(p, pos0 + q0) >> 6, w_first = gqa_first(p, pos0 + qw), w_last = gqa_first(p, pos0 + qw + QW - 1);
-    fetch(t_first * 64);
-    for (int kt0 = t_first; kt0 < n_tiles; ++kt0) {
-        const int key0 = kt0 * 64;
+    fetch(min(t_first + grp, n_tiles - 1) * 64);
+    for (int t0 = t_first; t0 < n_tiles; t0 += G) {
+        const int kt0 = t0 + grp, key0 = kt0 * 64;
         __syncthreads();
 #pragma unroll
         for (int mp = 0; mp < MAPS; ++mp)
@@ -762,8 +765,8 @@ __global__ __launch_bounds__(256, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(G
 #pragma unroll
         for (int j = 0; j < NVL; ++j) *reinterpret_cast<u32x4 *>(lv + ((tid >> 3) + 32 * j) * VS + (tid & 7) * 16) = vreg[j];
         __syncthreads();
-        if (kt0 + 1 < n_tiles) fetch(key0 + 64);
-        if (key0 > pos0 + qw + QW - 1 || key0 + 63 < w_first) continue;  // no key of the tile is seen by this wave's queries
+        if (kt0 + G < n_tiles) fetch(key0 + G * 64);
+        if (key0 > pos0 + qw + QW - 1 || key0 + 63 < w_first || (G == 2 && kt0 >= n_tiles)) continue;  // no key of the tile is seen by this wave's queries
         f32x4 s[4][SLOTS];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
@@ -846,6 +849,29 @@ __global__ __launch_bounds__(256, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(G
                 }
             }
     }
+    if (G == 2) {
+        f32x4 *po = reinterpret_cast<f32x4 *>(lds);                                       // [wave][slot][NV][lane]
+        float2 *pm = reinterpret_cast<float2 *>(lds + (size_t)4 * SLOTS * NV * 64 * 16);  // [wave][slot][lane]
+        __syncthreads();
+        if (grp == 1) {
+#pragma unroll
+            for (int t = 0; t < SLOTS; ++t) {
+#pragma unroll
+                for (int v = 0; v < NV; ++v) po[((wave * SLOTS + t) * NV + v) * 64 + lane] = o[v][t];
+                pm[(wave * SLOTS + t) * 64 + lane] = float2{m[t], l[t]};
+            }
+        }
+        __syncthreads();
+        if (grp == 1) return;
+#pragma unroll
+        for (int t = 0; t < SLOTS; ++t) {
+            const float2 b = pm[(wave * SLOTS + t) * 64 + lane];
+            const float mx = fmaxf(m[t], b.x), wa = __builtin_amdgcn_exp2f(m[t] - mx), wb = __builtin_amdgcn_exp2f(b.x - mx);
+            l[t] = l[t] * wa + b.y * wb;
+#pragma unroll
+            for (int v = 0; v < NV; ++v) o[v][t] = o[v][t] * wa + po[((wave * SLOTS + t) * NV + v) * 64 + lane] * wb;
+        }
+    }
     float inv[SLOTS], gate[SLOTS / MAPS];
 #pragma unroll
     for (int t = 0; t < SLOTS / MAPS; ++t) gate[t] = 1.0f;
@@ -887,13 +913,15 @@ __global__ __launch_bounds__(256, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(G
 template <int NK, int NV>
 static hipError_t gqa_prefill_go(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, hipStream_t s) {
     const int rows = g.maps == 2 ? 64 : 128, n_qb = (nq + rows - 1) / rows;
-    const size_t lds = (size_t)g.maps * 64 * (NK * 64 + 16) + (size_t)NV * 16 * (64 * 2 + 16);
-    auto fn = g.maps == 2 ? k_gqa_prefill<NK, NV, 2, false> : g.far_weight || g.gate_columns ? k_gqa_prefill<NK, NV, 1, true> : k_gqa_prefill<NK, NV, 1, false>;
+    constexpr int G = NV > 8 || NK > 4 ? 1 : 2;
+    const size_t tiles = G * ((size_t)g.maps * 64 * (NK * 64 + 16) + (size_t)NV * 16 * (64 * 2 + 16)), sums = G == 2 ? (size_t)4 * 2 * 64 * (NV * 16 + 8) : 0;
+    const size_t lds = tiles > sums ? tiles : sums;
+    auto fn = g.maps == 2 ? k_gqa_prefill<NK, NV, 2, false, G> : g.far_weight || g.gate_columns ? k_gqa_prefill<NK, NV, 1, true, G> : k_gqa_prefill<NK, NV, 1, false, G>;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(fn, dim3(8 * ((g.heads + 7) / 8) * n_qb), dim3(256), lds, s, g, q, ldq, n_ctx, nq, out, ldo, n_qb);
+    hipLaunchKernelGGL(fn, dim3(8 * ((g.heads + 7) / 8) * n_qb), dim3(256 * G), lds, s, g, q, ldq, n_ctx, nq, out, ldo, n_qb);
     return hipGetLastError();
 }
 
