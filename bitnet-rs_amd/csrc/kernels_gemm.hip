@@ -1175,11 +1175,11 @@ __device__ __forceinline__ void f16_chain_epilogue(const GemmArgs &p, gv4f (&acc
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
             for (int j = 0; j < 4; ++j) val[rt][j] = (acc[rt][tt][j] * is - mr.x * lng[rt][j]) * mr.y;
-        if (RT == 4 && p.silu_mul) {
+        if (RT % 2 == 0 && p.silu_mul) {
             // row tiles alternate (gate, up): FeedForward::forward T:756-781; the product goes out as f16 rows for the down-projection
             const int half_rows = p.rows >> 1, ra = 16 * (tile0 >> 1) + 4 * g;
 #pragma unroll
-            for (int pr = 0; pr < 2; ++pr) {
+            for (int pr = 0; pr < RT / 2; ++pr) {
                 float r[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
@@ -1240,6 +1240,10 @@ __device__ __forceinline__ void f16_chain_epilogue(const GemmArgs &p, gv4f (&acc
         if (p.stats_out) {  // this wave's 16 RT rows of the token: the consumer's LayerNorm adds the slabs up
             s1 += __shfl_xor(s1, 16), s2 += __shfl_xor(s2, 16);
             s1 += __shfl_xor(s1, 32), s2 += __shfl_xor(s2, 32);
+            if (RT == 2) {  // (half a slab: two waves make one, behind the loop)
+                if (g == 0) reinterpret_cast<float2 *>(lds)[(tt * NW + rw) * 16 + c] = live ? float2{s1, s2} : float2{0.f, 0.f};
+                continue;
+            }
             if (g == 0) *reinterpret_cast<float2 *>(p.stats_out + 2 * ((size_t)(bx * NW + rw) * p.stats_stride + token)) = live ? float2{s1, s2} : float2{0.f, 0.f};
             // RT == 5: rows / 80 partials fill the first slabs of the [rows / 64] array the interface names; the first NW / 4 waves of
             // every workgroup clear the rows / 320 surplus ones (behind the NW gx real ones), so the consumer still adds rows / 64 entries up
@@ -1247,10 +1251,18 @@ __device__ __forceinline__ void f16_chain_epilogue(const GemmArgs &p, gv4f (&acc
                 *reinterpret_cast<float2 *>(p.stats_out + 2 * ((size_t)(NW * gridDim.x + bx * (NW / 4) + rw) * p.stats_stride + token)) = float2{0.f, 0.f};
         }
     }
+    if (RT == 2 && p.stats_out && !p.silu_mul) {  // (the tile buffers are free: the K loop ends on a barrier)
+        __syncthreads();
+        for (int i = tid; i < TTW * (NW / 2) * 16; i += NW * 64) {
+            const int tt = i / (NW / 2 * 16), pair = i / 16 % (NW / 2);
+            const float2 a = reinterpret_cast<const float2 *>(lds)[(tt * NW + 2 * pair) * 16 + (i & 15)], b = reinterpret_cast<const float2 *>(lds)[(tt * NW + 2 * pair + 1) * 16 + (i & 15)];
+            *reinterpret_cast<float2 *>(p.stats_out + 2 * ((size_t)(bx * (NW / 2) + pair) * p.stats_stride + (by * TTW + tt) * 16 + (i & 15))) = float2{a.x + b.x, a.y + b.y};
+        }
+    }
     gflush_sat(sat);
 }
 
-// RT = row tiles per wave: 4 (256-row workgroups), or 5 (320-row workgroups, chain form only): a 2560-row matrix x 4096 tokens is then
+// RT = row tiles per wave: 4 (256-row workgroups), 2 (128-row workgroups for short prompts: launch_gemm_f16_chain says when), or 5 (320-row workgroups, chain form only): a 2560-row matrix x 4096 tokens is then
 // 8 x 64 = 512 workgroups -- exactly one round of the 512 slots (two 4-wave workgroups per CU) instead of 640 in two rounds.
 template <int FMT, int TTW, int EPI = 0, int RT = 4>
 __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_hi) {
@@ -2431,8 +2443,15 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
     const int ttw = gemm_token_tiles(gx0, m_pad, false, kGemmCUs);
     const bool fmt1 = w.scaled;
     const bool rt5 = ttw == 4 && !io.silu_mul && gemm_five_tiles(w.rows, m_pad);
+    // Short prompts: waves of 32 rows while the waves of 64 leave most CUs one workgroup.  A K step of such a workgroup is a serial chain (staging, expansion, LDS reads, MFMAs,
+    // barrier: 3.2 us at 32 tokens, of which the units are busy a third), so two of half the rows on a CU take less than one.  BitNet32-F16 prompt of bitnet-b1.58-2B-4T, ms with
+    // this / without: 16 tokens 2.77 / 3.50, 128 3.28 / 3.98, 256 4.06 / 4.23, 400 5.40 / 5.99, 777 6.96 / 7.58, 1024 7.32 / 7.98.  From 390 workgroups on (q|k|v at 777
+    // tokens) both take the same time (37.2 / 37.6 us), and the waves of 64 expand each weight for twice the tokens.
+    const bool rt2 = ttw < 4 && gx0 * (m_pad / (16 * ttw)) <= 320;
     if (rt5) gx0 = w.rows / 320;
+    if (rt2) gx0 = w.rows / 128;
     void (*fk)(GemmArgs, uint32_t) = rt5    ? (fmt1 ? k_gemm_f16a<1, 4, 1, 5> : k_gemm_f16a<0, 4, 1, 5>)
+                                     : rt2  ? (fmt1 ? (ttw == 2 ? k_gemm_f16a<1, 2, 1, 2> : k_gemm_f16a<1, 1, 1, 2>) : (ttw == 2 ? k_gemm_f16a<0, 2, 1, 2> : k_gemm_f16a<0, 1, 1, 2>))
                                      : fmt1 ? (ttw == 4 ? k_gemm_f16a<1, 4, 1> : ttw == 2 ? k_gemm_f16a<1, 2, 1> : k_gemm_f16a<1, 1, 1>)
                                             : (ttw == 4 ? k_gemm_f16a<0, 4, 1> : ttw == 2 ? k_gemm_f16a<0, 2, 1> : k_gemm_f16a<0, 1, 1>);
     if (io.qb_out) {  // the outputs also leave as QB32 rows (the next fp6-form matmul's input): 64-token tiles only, no silu pairing, K' = rows % 256 == 0
@@ -2489,7 +2508,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
             return hipGetLastError();
         }
     }
-    a.wgroup = gemm_weight_group(gx0, rt5 ? 320 : 256, w.cols, fmt1);
+    a.wgroup = gemm_weight_group(gx0, rt5 ? 320 : rt2 ? 128 : 256, w.cols, fmt1);
     hipLaunchKernelGGL(fk, dim3((unsigned)gx0, (unsigned)(m_pad / (16 * ttw))), dim3(256), lds, stream, a, lut_f16_hi(w.lut));
     return hipGetLastError();
 }

@@ -118,6 +118,27 @@ def test_f16_chain_plain_residual_and_handover(hip, oracle, torch_, fmt, rows, c
 
 
 @pytest.mark.parametrize("fmt", ["qk256", "i2s"])
+@pytest.mark.parametrize("m", [17, 511, 800, 1025])
+def test_f16_chain_half_slab_waves(hip, torch_, fmt, m):
+    """2560 rows around the lines of the short-prompt forms: 32-row waves of 16 and 32 tokens (511: 320 workgroups of 256 rows, 800: 260), 64-row waves (1025: 340)"""
+    rows, cols, mp = 2560, 512, -(-m // 64) * 64
+    rng = np.random.default_rng(m)
+    h, w = make_matrix(hip, rng, fmt, rows, cols)
+    x = rng.normal(0, 1, (mp, cols)).astype(np.float16)
+    res = rng.normal(0, 1, (m, rows)).astype(np.float32)
+    y, st = torch_.from_numpy(res).cuda(), torch_.full((rows // 64, mp, 2), float("nan"), device="cuda")
+    hip.matmul_f16_dev(h, torch_.from_numpy(x).cuda(), m, y=y, residual=y, stats_out=st)
+    torch_.cuda.synchronize()
+    got, xd = y.cpu().numpy().astype(np.float64), x[:m].astype(np.float64)
+    assert np.max(np.abs(got - (res + xd @ w.T)) / (np.abs(xd) @ np.abs(w).T + np.abs(res) + 1e-6)) <= 2e-6  # f16 inputs: accumulation order alone
+    slabs, s = got.reshape(m, rows // 64, 64), st.cpu().numpy()
+    for e in (1, 2):  # f32 sums of 64 terms: 2^-24 per addition against the magnitudes
+        assert np.all(np.abs(s[:, :m, e - 1].T - (slabs ** e).sum(axis=2)) <= 4e-6 * (np.abs(slabs) ** e).sum(axis=2) + 1e-6)
+    assert np.all(s[:, m:] == 0)
+    hip.weights_free(h)
+
+
+@pytest.mark.parametrize("fmt", ["qk256", "i2s"])
 def test_f16_chain_layernorm_after_product_and_silu(hip, oracle, torch_, fmt):
     """qkv-like (LayerNorm -> f32 rows) and gate|up-like (LayerNorm -> silu(gate) * up -> f16 rows) launches at the 2B-4T widths,
     LayerNorm statistics from one partial (the chain's entry) and from 40 (a producer's slabs), against the oracle's LayerNorm + product"""
