@@ -932,6 +932,24 @@ __device__ __forceinline__ int weight_key(int row) {
     return CF32 ? (row >> 1) & 7 : ((row / (4 * FN)) & 3) * 2 + ((row >> 1) & 1);
 }
 
+// The activations of the matmul's epilogues, the same in every tile and in the form for few rows: a call's results do not hang on the launcher's choice.
+// v_exp and v_rcp where the call allows them; exp(v) - 1 of xIELU loses what a bf16 output does not keep.
+__device__ __forceinline__ float sigmoid_fast(float v) { return __builtin_amdgcn_rcpf(1.0f + __expf(-v)); }
+__device__ __forceinline__ float silu_fast(float v) { return v * sigmoid_fast(v); }
+__device__ __forceinline__ float gelu_fast(float v) { return v * sigmoid_fast(2.0f * gelu_argument(v)); }
+__device__ __forceinline__ float xielu_fast(float v, const Epilogue &e) { return 0.5f * v + (v > 0.f ? e.act_a * v * v : e.act_b * (__expf(v) - 1.0f - v)); }
+// gated columns
+__device__ __forceinline__ float activate_pair(float v, int act) {
+    return act == BITNET_HIP_ACT_SILU ? silu_fast(v) : act == BITNET_HIP_ACT_GELU_TANH ? gelu_fast(v) : activate(v, act);
+}
+// The fast GELU where one activation covers whole waves of columns in every tile (up to 128 of them); a wave that two activations or the last column run
+// through has always taken expf and a division, and its tile must not decide.
+__device__ __forceinline__ bool gelu_is_fast(const GemmArgsD &p) { return p.act_split >= p.n && p.n % 128 == 0; }
+__device__ __forceinline__ float activate_column(float v, int act, bool fast_gelu, const Epilogue &e) {
+    return act == BITNET_HIP_ACT_SILU ? silu_fast(v) : act == BITNET_HIP_ACT_SIGMOID ? sigmoid_fast(v) : act == BITNET_HIP_ACT_XIELU ? xielu_fast(v, e)
+         : act == BITNET_HIP_ACT_GELU_TANH && fast_gelu ? gelu_fast(v) : activate(v, act);
+}
+
 // GROUPED: the row tiles come from a device list, (matrix, first row, rows) each; a matrix's tiles follow one another.
 // GATED (bf16 outputs): columns 2 i and 2 i + 1 make column i of the output.
 // MUL (bf16 outputs): row i of the output is multiplied by a table's row, the one of its token.
@@ -1048,7 +1066,7 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void k_dense_gemm(GemmArgsD p, int
     const bool vec = (p.ldc & 7) == 0 && (p.c_batch & 7) == 0 && ((uintptr_t)p.c & 15) == 0;
     // the activation: one for the whole wave unless the split runs through its columns
     const int mine = nlast < p.act_split ? p.act0 : nl >= p.act_split ? p.act1 : -1, act0 = __builtin_amdgcn_readfirstlane(mine);
-    const int act = __all(mine == act0) ? act0 : -1;
+    const int act = __all(mine == act0) && (act0 != BITNET_HIP_ACT_GELU_TANH || gelu_is_fast(p)) ? act0 : -1;
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
         const int m = m0 + wm + j * 16 + r16;
@@ -1064,11 +1082,7 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void k_dense_gemm(GemmArgsD p, int
 #pragma unroll
             for (int i = 0; i < FN; ++i)
 #pragma unroll
-                for (int e = 0; e < 4; e += 2) {
-                    const float v = acc[i][j][e], z = p.act0 == BITNET_HIP_ACT_GELU_TANH ? 2.0f * gelu_argument(v) : v;
-                    const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
-                    r[2 * i + e / 2] = (p.act0 == BITNET_HIP_ACT_SILU || p.act0 == BITNET_HIP_ACT_GELU_TANH ? v * sg : activate(v, p.act0)) * acc[i][j][e + 1];
-                }
+                for (int e = 0; e < 4; e += 2) r[2 * i + e / 2] = activate_pair(acc[i][j][e], p.act0) * acc[i][j][e + 1];
             uint16_t *dst = (uint16_t *)p.c + (size_t)blockIdx.y * p.c_batch + (size_t)m * p.ldc + nl / 2;
 #pragma unroll
             for (int i = 0; i < 2 * FN; i += 4) {
@@ -1088,24 +1102,18 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void k_dense_gemm(GemmArgsD p, int
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[i][j][e] = f(acc[i][j][e], nl + i * FS + e);
         };
-        // (exp(v) - 1 loses what a bf16 output does not keep)
-        auto xielu = [&](float v) { return 0.5f * v + (v > 0.f ? p.more.act_a * v * v : p.more.act_b * (__expf(v) - 1.0f - v)); };
         if (act < 0)
-            apply([&](float v, int n) {
-                const int f = n < p.act_split ? p.act0 : p.act1;
-                const float sg = __builtin_amdgcn_rcpf(1.0f + __expf(-v)), r = fmaxf(v, 0.0f);
-                return f == BITNET_HIP_ACT_SILU ? v * sg : f == BITNET_HIP_ACT_SIGMOID ? sg : f == BITNET_HIP_ACT_RELU2 ? r * r : f == BITNET_HIP_ACT_XIELU ? xielu(v) : activate(v, f);
-            });
+            apply([&](float v, int n) { return activate_column(v, n < p.act_split ? p.act0 : p.act1, false, p.more); });
         else if (act == BITNET_HIP_ACT_SILU)
-            apply([](float v, int) { return v * __builtin_amdgcn_rcpf(1.0f + __expf(-v)); });
+            apply([](float v, int) { return silu_fast(v); });
         else if (act == BITNET_HIP_ACT_SIGMOID)
-            apply([](float v, int) { return __builtin_amdgcn_rcpf(1.0f + __expf(-v)); });
+            apply([](float v, int) { return sigmoid_fast(v); });
         else if (act == BITNET_HIP_ACT_RELU2)
             apply([](float v, int) { return activate(v, BITNET_HIP_ACT_RELU2); });
         else if (act == BITNET_HIP_ACT_GELU_TANH)
-            apply([](float v, int) { return v * __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * gelu_argument(v))); });
+            apply([](float v, int) { return gelu_fast(v); });
         else if (act == BITNET_HIP_ACT_XIELU)
-            apply([&](float v, int) { return xielu(v); });
+            apply([&](float v, int) { return xielu_fast(v, p.more); });
         if (MUL) {
             const int token = min(max(p.more.mul_tokens[*p.more.mul_at + m], 0), p.more.mul_rows - 1);
             const uint16_t *mul = p.more.mul + (size_t)token * p.more.ld_mul;
@@ -1168,17 +1176,6 @@ static hipError_t gemm_go(const GemmArgsD &a, hipStream_t s) {
     }
     hipLaunchKernelGGL(fn, dim3(tn * tm, a.batch), dim3(64 * WN * WM), lds, s, a, tn, tm, swz);
     return hipGetLastError();
-}
-
-// activations as the matmuls take them: v_exp and v_rcp; exp(v) - 1 of xIELU loses what a bf16 output does not keep
-__device__ __forceinline__ float activate_fast(float v, int act, const Epilogue &e) {
-    switch (act) {
-        case BITNET_HIP_ACT_SILU: return v * __builtin_amdgcn_rcpf(1.0f + __expf(-v));
-        case BITNET_HIP_ACT_SIGMOID: return __builtin_amdgcn_rcpf(1.0f + __expf(-v));
-        case BITNET_HIP_ACT_GELU_TANH: return v * __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * gelu_argument(v)));
-        case BITNET_HIP_ACT_XIELU: return 0.5f * v + (v > 0.f ? e.act_a * v * v : e.act_b * (__expf(v) - 1.0f - v));
-        default: return activate(v, act);
-    }
 }
 
 // ---- few rows ---------------------------------------------------------------------------------------------------------
@@ -1279,7 +1276,7 @@ __global__ __launch_bounds__(512, 2) void k_dense_gemm_few(GemmArgsD p, int tile
         if (p.gated) {
             float r[2];
 #pragma unroll
-            for (int e = 0; e < 4; e += 2) r[e / 2] = activate_fast(v[e], p.act0, p.more) * v[e + 1];
+            for (int e = 0; e < 4; e += 2) r[e / 2] = activate_pair(v[e], p.act0) * v[e + 1];
             uint16_t *dst = (uint16_t *)p.c + row + n / 2;
             if (vec && n + 3 < p.n) {
                 *reinterpret_cast<uint32_t *>(dst) = (uint32_t)f2bf(r[0]) | (uint32_t)f2bf(r[1]) << 16;
@@ -1290,7 +1287,7 @@ __global__ __launch_bounds__(512, 2) void k_dense_gemm_few(GemmArgsD p, int tile
             continue;
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = activate_fast(v[e], n + e < p.act_split ? p.act0 : p.act1, p.more);
+        for (int e = 0; e < 4; ++e) v[e] = activate_column(v[e], n + e < p.act_split ? p.act0 : p.act1, gelu_is_fast(p), p.more);
         if (p.more.mul) {
             const int token = min(max(p.more.mul_tokens[*p.more.mul_at + m], 0), p.more.mul_rows - 1);
             const uint16_t *mul = p.more.mul + (size_t)token * p.more.ld_mul;

@@ -109,6 +109,28 @@ def test_matmul_few_rows(hip, pkg, m, n, k, batch, form):
     assert not got[:, :, want.shape[2]:].any()
 
 
+# the same rows alone (the form for few rows) and among many (tiles of 64 columns and more): sums of these inputs are exact in any order, so that whatever differs comes from
+# the epilogue; whole and ragged columns, one activation and two, the split inside and between what a wave holds
+@pytest.mark.parametrize("n,split", [(256, 0), (384, 128), (384, 200), (390, 0)])
+@pytest.mark.parametrize("form", ["f32", "bf16", "gated"])
+def test_matmul_activations_are_those_of_the_call(hip, pkg, n, split, form):
+    k, m, g = 512, 4096, rng(n, split)
+    gated, f32 = form == "gated", form == "f32"
+    a, w = g.integers(-4, 5, (m, k)).astype(np.float32) / 8, g.integers(-4, 5, (n, k)).astype(np.float32) / 16
+    ad, wd, b = u.dev_bf16(a), u.dev_bf16(w), u.dev_f32(g.integers(-8, 9, n).astype(np.float32) / 8)
+    acts = [pkg.ACT_SILU, pkg.ACT_SIGMOID, pkg.ACT_RELU2, pkg.ACT_GELU_TANH] + ([] if gated else [pkg.ACT_XIELU])
+    for i, act in enumerate(acts):
+        if gated and split:
+            continue
+        got = []
+        for rows in (16, m):
+            c = (u.zeros_f32 if f32 else u.zeros_bf16)(rows, n)
+            hip.dense_matmul_dev(ad, k, False, wd, k, rows, n, k, c, n, f32, bias=b, act0=act | (pkg.ACT_GATED if gated else 0), act1=acts[i - 1] if split else 0, act_split=split,
+                                 more=pkg.Epilogue(act_a=0.7, act_b=0.9) if pkg.ACT_XIELU in (act, acts[i - 1]) and not gated else None)
+            got.append(u.host(c)[:16])
+        assert got[0].any() and np.array_equal(*got), (act, np.abs(got[0] - got[1]).max())
+
+
 # every tile of the matmul where the launcher takes it (a whole number of them and ends inside one), and outputs that start on no sixteen bytes
 @pytest.mark.parametrize("m,n", [(4096, 4096), (4000, 4080), (4096, 3072), (3900, 3060), (2048, 3072), (2040, 4056), (2048, 2560), (1537, 2570), (1500, 2568), (700, 2552), (1531, 1528)])
 @pytest.mark.parametrize("form", ["f32", "bf16", "gated", "unaligned"])
