@@ -694,6 +694,12 @@ class HipLib:
                    C.c_int(act1), _sz(act_split), _ptr(c), _sz(ldc), C.c_int(c_f32), _sz(batch), _sz(a_batch), _sz(w_batch), _sz(c_batch),
                    C.byref(more) if more is not None else None, _vp(stream))
 
+    def dense_matmul_last_tile(self) -> tuple:
+        """(columns, rows, waves, waves that share them) of this thread's last dense_matmul_dev launch"""
+        v = [C.c_int() for _ in range(4)]
+        self._call("dense_matmul_last_tile", *[C.byref(x) for x in v])
+        return tuple(x.value for x in v)
+
     def dense_gemv_dev(self, x, w, rows: int, cols: int, ld: int, y, kind: int = 0, eps: float = 0.0, weight_offset: float = 0.0, weight=None, res=None,
                        post_weight=None, scale=None, gate=None, x_out=None, n: int = 0, mean_n: int = 0, bias=None, act0: int = 0, act1: int = 0,
                        act_split: int = 0, batch: int = 1, w_batch: int = 0, x_batch: int = 0, y_batch: int = 0, latent=None, latent_f32: bool = False,

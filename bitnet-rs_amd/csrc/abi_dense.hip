@@ -176,6 +176,15 @@ int bitnet_hip_dense_matmul_dev(const void *a, size_t lda, int a_f32, const uint
     BH_GUARD_END
 }
 
+int bitnet_hip_dense_matmul_last_tile(int *columns, int *rows, int *waves, int *sharing) {
+    const DenseTile &t = g_last_dense_tile;
+    if (columns) *columns = t.columns;
+    if (rows) *rows = t.rows;
+    if (waves) *waves = t.waves;
+    if (sharing) *sharing = t.sharing;
+    return t.columns ? BITNET_HIP_OK : set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "no dense matmul has been launched on this thread");
+}
+
 int bitnet_hip_latent_rows_dev(const bitnet_hip_latent_rows *rows, size_t m, int f32, void *stream) {
     BH_GUARD_BEGIN
     LatentRows r;

@@ -213,6 +213,10 @@ hipError_t launch_gated_norm_rows(const float *o, size_t ldo, const float *w, co
 hipError_t launch_gather_rows(const float *x, const int *rows, int n, int width, float *out, hipStream_t s);
 hipError_t launch_dense_gemv(const GemvArgs &a, int *n_wg_out, hipStream_t s);
 hipError_t launch_dense_gemm(const GemmArgsD &a, hipStream_t s);
+struct DenseTile {
+    int columns = 0, rows = 0, waves = 0, sharing = 0;
+};
+extern thread_local DenseTile g_last_dense_tile;  // what launch_dense_gemm ran last on this thread
 hipError_t launch_latent_rows(const LatentRows &a, hipStream_t s);
 size_t latent_scratch_floats(int heads, int ldc, int nq);
 bool latent_prefill_supported(int qd, int vdimp);

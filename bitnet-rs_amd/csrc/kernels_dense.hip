@@ -1149,6 +1149,8 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void k_dense_gemm(GemmArgsD p, int
     }
 }
 
+thread_local DenseTile g_last_dense_tile;
+
 template <int T, int ST>
 static hipError_t grouped_go(const GemmArgsD &a, hipStream_t s) {
     const int tn = (a.n + T - 1) / T;
@@ -1158,6 +1160,7 @@ static hipError_t grouped_go(const GemmArgsD &a, hipStream_t s) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
+    g_last_dense_tile = {T, T, 4, 1};
     hipLaunchKernelGGL(fn, dim3((tn * a.max_tiles + 7) / 8 * 8), dim3(256), lds, s, a, tn, 0, 0);
     return hipGetLastError();
 }
@@ -1174,6 +1177,7 @@ static hipError_t gemm_go(const GemmArgsD &a, hipStream_t s) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
+    g_last_dense_tile = {TN, TM, WN * WM, 1};
     hipLaunchKernelGGL(fn, dim3(tn * tm, a.batch), dim3(64 * WN * WM), lds, s, a, tn, tm, swz);
     return hipGetLastError();
 }
@@ -1324,6 +1328,7 @@ static hipError_t gemm_few_go(const GemmArgsD &a, hipStream_t s) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_dense_gemm_few<FN, FM, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
+    g_last_dense_tile = {16 * FN, 16 * FM, 8, 8};
     hipLaunchKernelGGL((k_dense_gemm_few<FN, FM, R>), dim3((tn * tm + 7) / 8 * 8, a.batch), dim3(512), lds, s, a, tn, tm);
     return hipGetLastError();
 }
@@ -1396,6 +1401,7 @@ hipError_t launch_dense_gemm(const GemmArgsD &args, hipStream_t s) {
     if (a.tiles) {
         if (a.a_f32) {
             if (a.tile != 64) return hipErrorInvalidValue;
+            g_last_dense_tile = {64, 64, 4, 1};
             hipLaunchKernelGGL(k_dense_gemm_f32<true>, dim3((a.n + 63) / 64, a.max_tiles, 1), dim3(256), 0, s, a);
             return hipGetLastError();
         }
@@ -1403,6 +1409,7 @@ hipError_t launch_dense_gemm(const GemmArgsD &args, hipStream_t s) {
         return a.tile == 128 ? grouped_go<128, 2>(a, s) : a.tile == 64 ? grouped_go<64, 4>(a, s) : hipErrorInvalidValue;
     }
     if (a.a_f32) {
+        g_last_dense_tile = {64, 64, 4, 1};
         hipLaunchKernelGGL(k_dense_gemm_f32<false>, dim3((a.n + 63) / 64, (a.m + 63) / 64, a.batch), dim3(256), 0, s, a);
         return hipGetLastError();
     }

@@ -655,6 +655,9 @@ typedef struct bitnet_hip_epilogue {
 int bitnet_hip_dense_matmul_dev(const void *a_dev, size_t lda, int a_f32, const uint16_t *w_dev, size_t ldw, const float *bias_dev,
                                 size_t m, size_t n, size_t k, int act0, int act1, size_t act_split, void *c_dev, size_t ldc, int c_f32,
                                 size_t batch, size_t a_batch, size_t w_batch, size_t c_batch, const bitnet_hip_epilogue *more, void *stream);
+/* Which tile the calling thread's last launch of that product ran (any pointer may be null): columns and rows per workgroup, its waves, and how many of them share
+ * the same columns and rows (8: the form for few rows, whose waves take K in turns; else 1).  The tests assert that they compared the form they are about. */
+int bitnet_hip_dense_matmul_last_tile(int *columns, int *rows, int *waves, int *sharing);
 
 /* How a matrix-vector product forms its input (every workgroup does so: no launch of its own). */
 #define BITNET_HIP_IN_PLAIN 0

@@ -85,10 +85,11 @@ def test_matmul(hip, pkg, m, n, k, f32):
 
 # the form for few rows: its three tiles at the edges of their ranges (one round of 256 workgroups), K that does not go round its eight waves, rows and columns
 # that end inside a tile, batches; the last two lie just behind the ranges.  Tolerances as in test_matmul: sums of k products in f32, one rounding to bf16.
-@pytest.mark.parametrize("m,n,k,batch", [(1, 1, 512, 1), (16, 4096, 576, 1), (17, 2048, 512, 1), (19, 40, 1984, 3), (33, 1000, 640, 1), (61, 4096, 512, 1), (64, 130, 4096, 2),
-                                         (65, 4090, 512, 1), (257, 1600, 768, 1), (2048, 72, 1536, 1), (64, 8200, 512, 1), (64, 100, 448, 1)])
+@pytest.mark.parametrize("m,n,k,batch,tile", [(1, 1, 512, 1, (16, 16)), (16, 4096, 576, 1, (16, 16)), (17, 2048, 512, 1, (16, 16)), (19, 40, 1984, 3, (16, 16)), (33, 1000, 640, 1, (16, 16)),
+                                              (61, 4096, 512, 1, (32, 32)), (64, 130, 4096, 2, (16, 16)), (65, 4090, 512, 1, (32, 64)), (257, 1600, 768, 1, (32, 64)),
+                                              (2048, 72, 1536, 1, (32, 32)), (64, 8200, 512, 1, None), (64, 100, 448, 1, None)])
 @pytest.mark.parametrize("form", ["f32", "bf16", "gated"])
-def test_matmul_few_rows(hip, pkg, m, n, k, batch, form):
+def test_matmul_few_rows(hip, pkg, m, n, k, batch, tile, form):
     if form == "gated":
         n = u.up_to(n, 2)
     g = rng(m, n, k)
@@ -104,6 +105,8 @@ def test_matmul_few_rows(hip, pkg, m, n, k, batch, form):
     c = u.zeros_f32(batch * m, ldc) if form == "f32" else u.zeros_bf16(batch * m, ldc)
     hip.dense_matmul_dev(u.dev_bf16(a), k, False, u.dev_bf16(w), k, m, n, k, c, ldc, form == "f32", bias=u.dev_f32(b), act0=act0, act1=pkg.ACT_SILU if split else 0, act_split=split,
                          batch=batch, a_batch=m * k, w_batch=n * k, c_batch=m * ldc)
+    ran = hip.dense_matmul_last_tile()
+    assert ran == (*tile, 8, 8) if tile else ran[3] == 1, ran
     got = u.host(c).reshape(batch, m, ldc)
     assert u.rms_error(got[:, :, :want.shape[2]], want) < (F32_TOL if form == "f32" else 3e-3)
     assert not got[:, :, want.shape[2]:].any()
