@@ -1188,16 +1188,16 @@ static hipError_t gemm_go(const GemmArgsD &a, hipStream_t s) {
 // its eight waves share the K columns out, 64 at a time in turn, each with its own buffers (R) and no barrier, and add up in LDS at the end.
 // Measured, us per launch, weights from HBM (this / 64 x 64 tiles): 16 x 2560 x 2560 7.3 / 13.2, 16 x 2560 x 6912 12.7 / 28.8, 61 x 2560 x 6912 19.4 / 34.1,
 // 61 x 6912 x 2560 14.8 / 17.3, 128 x 1536 x 4096 12.2 / 20.6, 1024 x 72 x 2560 7.1 / 13.4.
-template <int FN, int FM, int R>
+template <int FN, int FM, int R, bool TALL>
 __global__ __launch_bounds__(512, 2) void k_dense_gemm_few(GemmArgsD p, int tiles_n, int tiles_m) {
     extern __shared__ __attribute__((aligned(16))) f32x4 part[];  // [wave][fragment][lane]
     constexpr int NW = 8;
     const int units = p.k >> 6;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // each XCD a contiguous run of tiles, the row tiles of one weight tile side by side
+    // each XCD a contiguous run of tiles: the row tiles of one weight tile side by side, or (TALL) the column tiles of one row tile
     const int total = tiles_n * tiles_m, per = (total + 7) >> 3, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
-    const int tn = id / tiles_m, tm = id % tiles_m;
+    const int tn = TALL ? id % tiles_n : id / tiles_m, tm = TALL ? id / tiles_n : id % tiles_m;
     const int m0 = tm * 16 * FM, n0 = tn * 16 * FN;
     const int r16 = lane & 15, g = lane >> 4;
     constexpr unsigned ROWS = 16 * (FM + FN), BUF = ROWS * 128;
@@ -1290,8 +1290,14 @@ __global__ __launch_bounds__(512, 2) void k_dense_gemm_few(GemmArgsD p, int tile
             }
             continue;
         }
+        if (p.act_split < p.n) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = activate_column(v[e], n + e < p.act_split ? p.act0 : p.act1, gelu_is_fast(p), p.more);
+            for (int e = 0; e < 4; ++e) v[e] = activate_column(v[e], n + e < p.act_split ? p.act0 : p.act1, false, p.more);
+        } else if (p.act0 != BITNET_HIP_ACT_NONE) {
+            const bool fast_gelu = gelu_is_fast(p);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = activate_column(v[e], p.act0, fast_gelu, p.more);
+        }
         if (p.more.mul) {
             const int token = min(max(p.more.mul_tokens[*p.more.mul_at + m], 0), p.more.mul_rows - 1);
             const uint16_t *mul = p.more.mul + (size_t)token * p.more.ld_mul;
@@ -1324,12 +1330,16 @@ template <int FN, int FM, int R>
 static hipError_t gemm_few_go(const GemmArgsD &a, hipStream_t s) {
     const int tn = (a.n + 16 * FN - 1) / (16 * FN), tm = (a.m + 16 * FM - 1) / (16 * FM);
     constexpr size_t lds = 8 * 1024 * (FN * FM > 2 * R * (FN + FM) ? FN * FM : 2 * R * (FN + FM));
+    // Activations that outgrow an XCD's L2 (4 MB) are read once, not once per column of tiles, where they are the larger operand.  us with this order / the other:
+    // 2048 x 256 x 6912 18.9 / 35.2, 2685 x 160 x 4096 12.6 / 21.7, 1531 x 320 x 2560 10.4 / 14.6, 605 x 320 x 8192 15.4 / 19.5.
+    const bool tall = (size_t)a.m * a.k * 2 > 4u << 20 && (size_t)a.m * 4 > (size_t)a.n * 5;
+    auto fn = tall ? k_dense_gemm_few<FN, FM, R, true> : k_dense_gemm_few<FN, FM, R, false>;
     if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_dense_gemm_few<FN, FM, R>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
     g_last_dense_tile = {16 * FN, 16 * FM, 8, 8};
-    hipLaunchKernelGGL((k_dense_gemm_few<FN, FM, R>), dim3((tn * tm + 7) / 8 * 8, a.batch), dim3(512), lds, s, a, tn, tm);
+    hipLaunchKernelGGL(fn, dim3((tn * tm + 7) / 8 * 8, a.batch), dim3(512), lds, s, a, tn, tm);
     return hipGetLastError();
 }
 
@@ -1415,12 +1425,14 @@ hipError_t launch_dense_gemm(const GemmArgsD &args, hipStream_t s) {
     }
     if (a.more.mul && (a.c_f32 || a.gated)) return hipErrorInvalidValue;
     // one round of workgroups of the form for few rows, its smallest tile first (two per CU fit but share the CU's LDS-DMA: behind 256 the larger tile is ahead, and behind
-    // that the tiles of 64 x 64: 61 x 10240 x 2560 takes 20.3 to 25.5 us in this form and 18.3 in the other); short K leaves its waves without work (256: 5.2 / 4.3 us)
+    // that the tiles of 64 x 64: 61 x 10240 x 2560 takes 20.3 to 25.5 us in this form and 18.3 in the other); short K leaves its waves without work (256: 5.2 / 4.3 us), and
+    // those of the largest tile below 1536 (36 x 8192 x 512 7.0 / 6.2, 145 x 2560 x 512 6.5 / 6.2, 52 x 8192 x 1024 8.4 / 8.0; 40 x 4608 x 1536 8.7 / 9.3) unless tiles of 64
+    // columns are a quarter wider than the matrix needs (3500 x 72 x 512 6.3 / 8.0)
     auto one_round = [&](int tn, int tm) { return ((long)(a.n + tn - 1) / tn) * ((a.m + tm - 1) / tm) * a.batch <= 256; };
     if (a.k >= 512) {
         if (one_round(16, 16)) return gemm_few_go<1, 1, 2>(a, s);
         if (one_round(32, 32)) return gemm_few_go<2, 2, 1>(a, s);
-        if (one_round(32, 64)) return gemm_few_go<2, 4, 1>(a, s);
+        if (one_round(32, 64) && (a.k >= 1536 || ((long)a.n + 63) / 64 * 8 >= ((long)a.n + 31) / 32 * 5)) return gemm_few_go<2, 4, 1>(a, s);
     }
     if (a.more.mul) return gemm_go<64, 64, 2, 2, 4, true>(a, s);
     auto tiles = [&](int tn, int tm) { return (double)((a.n + tn - 1) / tn) * ((a.m + tm - 1) / tm) * a.batch; };

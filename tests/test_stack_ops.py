@@ -86,7 +86,8 @@ def test_matmul(hip, pkg, m, n, k, f32):
 # the form for few rows: its three tiles at the edges of their ranges (one round of 256 workgroups), K that does not go round its eight waves, rows and columns
 # that end inside a tile, batches; the last two lie just behind the ranges.  Tolerances as in test_matmul: sums of k products in f32, one rounding to bf16.
 @pytest.mark.parametrize("m,n,k,batch,tile", [(1, 1, 512, 1, (16, 16)), (16, 4096, 576, 1, (16, 16)), (17, 2048, 512, 1, (16, 16)), (19, 40, 1984, 3, (16, 16)), (33, 1000, 640, 1, (16, 16)),
-                                              (61, 4096, 512, 1, (32, 32)), (64, 130, 4096, 2, (16, 16)), (65, 4090, 512, 1, (32, 64)), (257, 1600, 768, 1, (32, 64)),
+                                              (61, 4096, 512, 1, (32, 32)), (64, 130, 4096, 2, (16, 16)), (65, 4090, 512, 1, None), (257, 1600, 768, 1, None),
+                                              (65, 4090, 1536, 1, (32, 64)), (257, 1600, 1600, 1, (32, 64)), (2760, 72, 512, 1, (32, 64)), (1400, 160, 2560, 1, (32, 32)), (1500, 320, 1536, 1, (32, 64)),
                                               (2048, 72, 1536, 1, (32, 32)), (64, 8200, 512, 1, None), (64, 100, 448, 1, None)])
 @pytest.mark.parametrize("form", ["f32", "bf16", "gated"])
 def test_matmul_few_rows(hip, pkg, m, n, k, batch, tile, form):
