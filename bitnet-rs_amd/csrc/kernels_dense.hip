@@ -950,6 +950,11 @@ __device__ __forceinline__ float activate_column(float v, int act, bool fast_gel
          : act == BITNET_HIP_ACT_GELU_TANH && fast_gelu ? gelu_fast(v) : activate(v, act);
 }
 
+__host__ __device__ __forceinline__ bool rows_on_16_bytes(const void *c, size_t ldc, size_t c_batch, bool f32) {
+    const size_t mask = f32 ? 3 : 7;
+    return ((ldc | c_batch) & mask) == 0 && ((uintptr_t)c & 15) == 0;
+}
+
 // GROUPED: the row tiles come from a device list, (matrix, first row, rows) each; a matrix's tiles follow one another.
 // GATED (bf16 outputs): columns 2 i and 2 i + 1 make column i of the output.
 // MUL (bf16 outputs): row i of the output is multiplied by a table's row, the one of its token.
@@ -1063,7 +1068,7 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void k_dense_gemm(GemmArgsD p, int
     }
     // this lane's columns: nl + i * FS + e
     const int nl = n0 + wn + g * (CF32 ? 4 : 4 * FN), nlast = nl + (FN - 1) * FS + 3;
-    const bool vec = (p.ldc & 7) == 0 && (p.c_batch & 7) == 0 && ((uintptr_t)p.c & 15) == 0;
+    const bool vec = rows_on_16_bytes(p.c, p.ldc, p.c_batch, CF32);
     // the activation: one for the whole wave unless the split runs through its columns
     const int mine = nlast < p.act_split ? p.act0 : nl >= p.act_split ? p.act1 : -1, act0 = __builtin_amdgcn_readfirstlane(mine);
     const int act = __all(mine == act0) && (act0 != BITNET_HIP_ACT_GELU_TANH || gelu_is_fast(p)) ? act0 : -1;
@@ -1437,24 +1442,34 @@ hipError_t launch_dense_gemm(const GemmArgsD &args, hipStream_t s) {
     if (a.more.mul) return gemm_go<64, 64, 2, 2, 4, true>(a, s);
     auto tiles = [&](int tn, int tm) { return (double)((a.n + tn - 1) / tn) * ((a.m + tm - 1) / tm) * a.batch; };
     if (a.k <= 1024 && tiles(64, 64) >= 1024) return gemm_go<64, 64, 2, 2, 2>(a, s);  // few steps: what counts is how many workgroups overlap their ends
-    // The tile whose launch is the shortest by what was measured (us, bf16 and f32 outputs, m 400 to 4096, n 1536 to 12288, k 1536 to 8192): a step of 64 columns and a
-    // round's start and end.  The large ones stand alone on their CU and run in rounds of 256; of 64 x 128 two fit, but a second one costs more than half a round; a CU
-    // takes up to four of 64 x 64.  Three buffers where LDS has the room: 128 x 256 takes 0.80 us a step with them and 0.96 with two.  4096 x 3072 x 3072:
-    // 256 x 256 leaves a quarter of the CUs out (76 us), 192 x 256 is one full round (69); 2048 x 2560 x 6912: 128 x 192 80 us, 128 x 128 in four waves 114.
-    // Outputs whose rows do not start on sixteen bytes are stored one by one, which costs the most at the largest tiles.
-    const double steps = a.k / 64, slow = (a.ldc & 7) == 0 && (a.c_batch & 7) == 0 && ((uintptr_t)a.c & 15) == 0 ? 0.0 : 40.0 / 65536;
-    auto rounds = [&](int tn, int tm, double step, double ends) { return std::ceil(tiles(tn, tm) / 256) * (steps * step + ends + slow * tn * tm); };
-    const double t64 = tiles(64, 64) / 256, t128 = tiles(64, 128);
-    const double us[] = {slow ? 1e30 : rounds(256, 256, 1.27, 13), slow ? 1e30 : rounds(192, 256, 1.15, 12), rounds(128, 256, 0.80, 6), rounds(128, 192, 0.68, 4.5),
-                         rounds(128, 128, 0.48, 5.5), steps * (t128 <= 256 ? 0.40 : 0.62 * std::ceil(t128 / 512)) + 3.5 + slow * 64 * 128,
-                         steps * 0.27 * (t64 > 1 ? t64 : 1) + 3 + slow * 64 * 64};
+    // The tile whose launch is the shortest by what was measured (us; every tile at 330 shapes, m 24 to 4100, n 320 to 13824, k 512 to 8192, each kind of output; the choice is 1.4 % behind
+    // the best of them in the mean): a step of 64 columns and a round's start and end.  The large ones stand alone on their CU and run in rounds of 256.  Of 128 x 128 in four
+    // waves two fit, which overlap their ends: ahead of the others where those fill their last round badly (565 x 12288 x 3072 52 us, 128 x 128 in eight waves 59;
+    // 3667 x 2112 x 1024 23 / 28).  Of 64 x 128 two fit as well, but a second one costs more than half a round; a CU takes up to four of 64 x 64.  Three buffers where LDS has the
+    // room: 128 x 256 takes 0.80 us a step with them and 0.96 with two.  4096 x 3072 x 3072: 256 x 256 leaves a quarter of the CUs out (76 us), 192 x 256 is one full round (69);
+    // 2048 x 2560 x 6912: 128 x 192 80 us, 128 x 128 in four waves 114.
+    // What is stored one by one: every tile's outputs, 25 us per 65536 of them, where rows do not start on sixteen bytes (4096 x 13824 x 2560: 256 x 256 412 us, 128 x 256 476,
+    // 64 x 128 513), else those of the last column of tiles where it sticks out, which lengthen the launch by 25 us (256 x 256), 14, 6, 3.5 (128 x 192) or 1.6
+    // (2297 x 4096 x 1536: 192 x 256 52 us, 128 x 192 42).
+    const double steps = a.k / 64, slow = a.gated ? 12.5 / 65536 : 25.0 / 65536;
+    const bool aligned = rows_on_16_bytes(a.c, a.ldc, a.c_batch, a.c_f32);
+    auto stores = [&](int tn, int tm, double rounds) { return aligned ? (a.n % tn && !a.gated ? 25.0 / 65536 / 65536 * tn * tm * tn * tm : 0.0) : slow * tn * tm * std::max(rounds, 1.0); };
+    auto alone = [&](int tn, int tm, double step, double ends) {
+        const double rounds = std::ceil(tiles(tn, tm) / 256);
+        return rounds * (steps * step + ends) + stores(tn, tm, rounds);
+    };
+    const double t64 = tiles(64, 64) / 256, t128 = tiles(64, 128) / 256, pairs = tiles(128, 128) / 512, whole = std::floor(pairs), rest = pairs - whole;
+    const double us[] = {alone(256, 256, 1.27, 13), alone(192, 256, 1.06, 11), alone(128, 256, 0.80, 6), alone(128, 192, 0.68, 4.5), alone(128, 128, 0.48, 5.5),
+                         whole * (0.88 * steps + 6) + (rest == 0 ? 0 : rest <= 0.5 ? 0.62 * steps + 6 : 0.88 * steps + 6) + stores(128, 128, 2 * pairs),
+                         steps * (t128 <= 1 ? 0.40 : 0.62 * std::ceil(t128 / 2)) + 3.5 + stores(64, 128, t128), steps * 0.27 * std::max(t64, 1.0) + 3 + stores(64, 64, t64)};
     switch (std::min_element(std::begin(us), std::end(us)) - us) {
         case 0: return gemm_go<256, 256, 2, 4, 2>(a, s);
         case 1: return gemm_go<192, 256, 2, 4, 2>(a, s);
         case 2: return gemm_go<128, 256, 2, 4, 3>(a, s);
         case 3: return gemm_go<128, 192, 2, 4, 3>(a, s);
         case 4: return gemm_go<128, 128, 2, 4, 4>(a, s);
-        case 5: return gemm_go<64, 128, 2, 2, 3>(a, s);
+        case 5: return gemm_go<128, 128, 2, 2, 2>(a, s);
+        case 6: return gemm_go<64, 128, 2, 2, 3>(a, s);
         default: return gemm_go<64, 64, 2, 2, 4>(a, s);
     }
 }

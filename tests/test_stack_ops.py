@@ -160,6 +160,40 @@ def test_matmul_tiles(hip, pkg, m, n, form):
     assert not c[:, cols:].any()
 
 
+# every tile by name, for whole and for ragged columns: (columns, rows, waves) of plain outputs, of gated ones and of those whose rows do not start on sixteen bytes; f32 rows
+# a multiple of four apart do.  A moved constant of the launcher's costs shows up here.
+BY_TILE = [(2000, 7680, 1088, (256, 256, 8), (256, 256, 8), (256, 256, 8)), (1500, 7680, 1088, (192, 256, 8), (192, 256, 8), (192, 256, 8)),
+           (1000, 7680, 1088, (128, 256, 8), (128, 256, 8), (128, 256, 8)), (520, 7680, 1088, (128, 192, 8), (128, 192, 8), (128, 192, 8)),
+           (700, 4096, 4096, (128, 128, 8), (128, 128, 8), (128, 128, 8)), (2000, 7700, 1088, (128, 128, 4), (256, 256, 8), (256, 256, 8)),
+           (1500, 4100, 1088, (128, 128, 4), (128, 256, 8), (128, 128, 4)), (700, 2560, 1088, (64, 128, 4), (64, 128, 4), (64, 128, 4)),
+           (520, 4100, 4096, (128, 128, 8), (128, 128, 8), (128, 128, 8)), (1000, 7700, 2048, (128, 128, 4), (128, 256, 8), (128, 256, 8)),
+           (300, 1500, 1088, (64, 64, 4), (64, 64, 4), (64, 64, 4)), (4096, 1088, 1024, (64, 64, 4), (64, 64, 4), (64, 64, 4))]
+
+
+@pytest.mark.parametrize("m,n,k,plain,pairs,odd", BY_TILE)
+@pytest.mark.parametrize("form", ["f32", "f32 + 4", "f32 + 3", "bf16", "bf16 + 4", "gated", "gated + 1"])
+def test_matmul_by_tile(hip, pkg, m, n, k, plain, pairs, odd, form):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    a, w = (torch.randn(r, k, device="cuda", generator=g).bfloat16() for r in (m, n))
+    b = torch.randn(n, device="cuda", generator=g)
+    w = (w.double() / np.sqrt(k)).bfloat16()
+    want = a.double() @ w.double().T + b.double()
+    gated, f32 = form.startswith("gated"), form.startswith("f32")
+    if gated:
+        want = torch.nn.functional.silu(want[:, ::2]) * want[:, 1::2]
+    cols, more = want.shape[1], int(form[form.index("+") + 2:]) if "+" in form else 0
+    ldc = u.up_to(cols, 8) + more
+    c = torch.zeros(m, ldc, device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
+    hip.dense_matmul_dev(a, k, False, w, k, m, n, k, c, ldc, f32, bias=b, act0=pkg.ACT_SILU | pkg.ACT_GATED if gated else pkg.ACT_NONE)
+    ran = hip.dense_matmul_last_tile()
+    torch.cuda.synchronize()
+    assert ((c[:, :cols].double() - want).norm() / want.norm()).item() < (F32_TOL if f32 else 3e-3)
+    assert not c[:, cols:].any()
+    if not (more and gated):  # (half the elements to store one by one: its own choice)
+        assert ran == (*(odd if more and form != "f32 + 4" else pairs if gated else plain), 1), ran
+
+
 def test_matmul_batched_f32(hip):
     g = rng(9)
     heads, m, n, k, step = 3, 70, 64, 64, 96
