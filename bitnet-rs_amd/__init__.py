@@ -630,6 +630,9 @@ class HipLib:
     def gqa_prefill_dev(self, a: "Gqa", q, ldq: int, n_ctx: int, nq: int, out, ldo: int, stream: int = 0) -> None:
         self._call("gqa_prefill_dev", C.byref(a), _ptr(q), _sz(ldq), _sz(n_ctx), _sz(nq), _ptr(out), _sz(ldo), _vp(stream))
 
+    def gqa_prefill_last_groups(self) -> int:
+        return int(self.c.bitnet_hip_gqa_prefill_last_groups())
+
     def delta_step_dev(self, d: "Delta", row, ba, pos, out, stream: int = 0) -> None:
         self._call("delta_step_dev", C.byref(d), _ptr(row), _ptr(ba), _ptr(pos), _ptr(out), _vp(stream))
 

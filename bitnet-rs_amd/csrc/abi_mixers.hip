@@ -137,6 +137,8 @@ int bitnet_hip_gqa_merge_dev(const bitnet_hip_gqa *a, const int32_t *pos, size_t
     BH_GUARD_END
 }
 
+int bitnet_hip_gqa_prefill_last_groups(void) { return g_last_gqa_groups; }
+
 int bitnet_hip_gqa_prefill_dev(const bitnet_hip_gqa *a, const uint16_t *q, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out, size_t ldo, void *stream) {
     BH_GUARD_BEGIN
     if (int rc = check_gqa(a)) return rc;

@@ -11,6 +11,8 @@
 //   k_gqa_merge    records of the decode forms -> output
 // Scores, maxima, sums and weights are f32; a weight (and the decode step's query) enters the matrix cores as a (high, low) pair of bf16 values.
 // Scores are kept in base 2: the score times log2(e).
+#include <algorithm>
+
 #include "dense.hpp"
 
 namespace bitnet_hip {
@@ -18,9 +20,9 @@ namespace bitnet_hip {
 constexpr float kLog2e = 1.44269504088896f;
 
 // the first key a query at this position sees
-__device__ __forceinline__ int gqa_first(const Gqa &p, int pos) {
+__host__ __device__ __forceinline__ int gqa_first(const Gqa &p, int pos) {
     const int first = p.chunk ? pos - (int)((unsigned)pos % (unsigned)p.chunk) : 0;
-    return p.window ? max(first, pos - (int)p.window + 1) : first;
+    return p.window && pos - (int)p.window + 1 > first ? pos - (int)p.window + 1 : first;
 }
 
 // The records of a query at `pos`: tiles of keys from `base` (the tile that holds its first key) on, `per` tiles each.
@@ -691,11 +693,11 @@ hipError_t launch_gqa_merge(const Gqa &g, const int *pos, int q0, int nq, const 
 // One workgroup: one head, four waves; a wave holds two slots of 16 queries: both maps of one query tile, or two tiles of the only map.  Key tiles
 // of 64 (every map's) and the values of the tile staged through registers into LDS one step ahead.
 // G = 2: two such groups of four waves share the keys of the same queries, tile by tile in turn, and meet in LDS at the end.  A prompt's last queries see all of its keys and its
-// first next to none: one group per workgroup left the longest walk (47 tiles of a 3000-token prompt) twice as long as a CU's fair share (28), 2.9 us a tile whatever its
-// neighbour does.  Heads that need more than 256 registers keep one group.
+// first next to none: with one group per workgroup the longest walk takes 2.6 us a tile whatever its neighbour does, with two it is half as long at 4.1 us a step.
+// Heads that need more than 256 registers keep one group; two_groups says when the others take two.
 // FAR: with a distance penalty, gates per column, or both.
 template <int NK, int NV, int MAPS, bool FAR, int G>
-__global__ __launch_bounds__(256 * G, G == 2 ? 2 : 1) void k_gqa_prefill(Gqa p, const uint16_t *Q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, int n_qb) {
+__global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(Gqa p, const uint16_t *Q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, int n_qb) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int SLOTS = 2, QW = 16 * SLOTS / MAPS, KS = NK * 64 + 16, VS = 64 * 2 + 16, NVL = NV / 2;
     const int grp = G == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
@@ -910,10 +912,31 @@ __global__ __launch_bounds__(256 * G, G == 2 ? 2 : 1) void k_gqa_prefill(Gqa p, 
     }
 }
 
-template <int NK, int NV>
+thread_local int g_last_gqa_groups;
+
+// Two groups fill a CU, and halve its walks; of one group two workgroups fit.  They pay while the launch is as long as its longest walk: with four tiles or more in it, a CU's
+// share of all tiles not much above it, and no second round behind walks that are all long (the shortest walk of the first round and the longest of the second one in turn).
+// Heads count as a multiple of eight, as the launch deals them to the XCDs (20 heads take what 24 do).  us with two / with one, measured over 200 shapes: 12 heads, 3000 tokens
+// 90 / 118 (share / walk 0.8), 32 heads, 2048 77 / 90 (1.06), 40 heads, 1664 73 / 73 (1.09), 24 heads, 3328 147 / 138 (1.27), 4096 207 / 169 (1.55); two maps, 24 heads, 1280 50 / 57,
+// 1531 71 / 68, 2048 113 / 94; 10 blocks of 24 heads behind 2700 keys (240 workgroups) 119 / 150, 11 blocks 168 / 161; one tile 8.8 / 7.2, three 12.2 / 11.8, five 15.6 / 16.3.
+static bool two_groups(const Gqa &g, int rows, int n_ctx, int nq) {
+    const int at_once = 256, pos0 = n_ctx - nq, heads = ((int)g.heads + 7) / 8 * 8, blocks = (nq + rows - 1) / rows, all_tiles = (n_ctx + 63) / 64;
+    long longest = 0, total = 0, second = 0;
+    for (int qb = blocks - 1, done = 0; qb >= 0 && total <= 2l * at_once * all_tiles; --qb, done += heads) {
+        const int q0 = qb * rows, tiles = (std::min(n_ctx, pos0 + q0 + rows) + 63) / 64 - (gqa_first(g, pos0 + q0) >> 6);
+        longest = std::max<long>(longest, tiles), total += (long)heads * tiles;
+        for (int i : {at_once - 1, at_once})
+            if ((long)heads * blocks > at_once && done <= i && i < done + heads) second += tiles;
+    }
+    return longest >= 4 && 16 * total <= 17 * at_once * longest && 10 * second <= 11 * longest;
+}
+
+template <int NK, int NV, int G>
 static hipError_t gqa_prefill_go(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, hipStream_t s) {
     const int rows = g.maps == 2 ? 64 : 128, n_qb = (nq + rows - 1) / rows;
-    constexpr int G = NV > 8 || NK > 4 ? 1 : 2;
+    if constexpr (G == 2)
+        if (!two_groups(g, rows, n_ctx, nq)) return gqa_prefill_go<NK, NV, 1>(g, q, ldq, n_ctx, nq, out, ldo, s);
+    g_last_gqa_groups = G;
     const size_t tiles = G * ((size_t)g.maps * 64 * (NK * 64 + 16) + (size_t)NV * 16 * (64 * 2 + 16)), sums = G == 2 ? (size_t)4 * 2 * 64 * (NV * 16 + 8) : 0;
     const size_t lds = tiles > sums ? tiles : sums;
     auto fn = g.maps == 2 ? k_gqa_prefill<NK, NV, 2, false, G> : g.far_weight || g.gate_columns ? k_gqa_prefill<NK, NV, 1, true, G> : k_gqa_prefill<NK, NV, 1, false, G>;
@@ -927,10 +950,10 @@ static hipError_t gqa_prefill_go(const Gqa &g, const uint16_t *q, size_t ldq, in
 
 hipError_t launch_gqa_prefill(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, hipStream_t s) {
     if (!gqa_supported((int)g.dimp, (int)g.vdimp)) return hipErrorInvalidValue;
-    if (g.dimp <= 64 && g.vdimp <= 64) return gqa_prefill_go<2, 4>(g, q, ldq, n_ctx, nq, out, ldo, s);
-    if (g.dimp <= 64 && g.vdimp <= 128) return gqa_prefill_go<2, 8>(g, q, ldq, n_ctx, nq, out, ldo, s);
-    if (g.dimp <= 128 && g.vdimp <= 128) return gqa_prefill_go<4, 8>(g, q, ldq, n_ctx, nq, out, ldo, s);
-    return gqa_prefill_go<8, 16>(g, q, ldq, n_ctx, nq, out, ldo, s);
+    if (g.dimp <= 64 && g.vdimp <= 64) return gqa_prefill_go<2, 4, 2>(g, q, ldq, n_ctx, nq, out, ldo, s);
+    if (g.dimp <= 64 && g.vdimp <= 128) return gqa_prefill_go<2, 8, 2>(g, q, ldq, n_ctx, nq, out, ldo, s);
+    if (g.dimp <= 128 && g.vdimp <= 128) return gqa_prefill_go<4, 8, 2>(g, q, ldq, n_ctx, nq, out, ldo, s);
+    return gqa_prefill_go<8, 16, 1>(g, q, ldq, n_ctx, nq, out, ldo, s);
 }
 
 }  // namespace bitnet_hip

@@ -801,6 +801,8 @@ int bitnet_hip_gqa_merge_dev(const bitnet_hip_gqa *attn, const int32_t *pos_dev,
 /* A portion of a prompt, bf16: the LAST nq of n_ctx positions attend (all of them in the caches); q as gqa_rows leaves it. */
 int bitnet_hip_gqa_prefill_dev(const bitnet_hip_gqa *attn, const uint16_t *q_dev, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out_dev, size_t ldo,
                                void *stream);
+/* Groups of four waves that shared a query block's keys in the calling thread's last launch of it: 2, or 1 (few keys, or enough workgroups to fill the chip); 0: none yet. */
+int bitnet_hip_gqa_prefill_last_groups(void);
 
 /* Gated delta rule.  A row of projections is [q kv_heads * dimp | k kv_heads * dimp | v heads * vdimp | gate heads * vdimp], and apart from it
  * [b heads | a heads] f32; heads zero-padded to multiples of 32.  q, k, v pass a causal convolution of `taps` tokens per channel and

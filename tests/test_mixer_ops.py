@@ -386,6 +386,22 @@ def test_attention_portion(hip, pkg, shape, n, nq):
     t.check(out, n - nq, 2e-2)
 
 
+# two groups of waves and one, on either side of each line between them: three and four tiles of keys; as many workgroups as the chip takes at once and a second round of long walks;
+# more tiles than the longest walk has room for; heads too large for two groups
+@pytest.mark.parametrize("shape,n,nq,groups", [((2, 1, 64, 64, 1), 192, 192, 1), ((2, 1, 64, 64, 1), 193, 193, 2), ((4, 2, 24, 40, 2), 256, 20, 2), ((4, 2, 24, 40, 2), 180, 20, 1),
+                                               ((64, 4, 16, 24, 2), 500, 256, 2), ((64, 4, 16, 24, 2), 500, 257, 1), ((57, 3, 16, 24, 2), 500, 257, 1), ((56, 4, 16, 24, 2), 500, 256, 2),
+                                               ((136, 8, 16, 16, 2), 256, 256, 1), ((100, 4, 24, 16, 1), 320, 320, 2), ((2, 1, 200, 256, 2), 300, 300, 1)])
+def test_attention_portion_in_groups(hip, pkg, shape, n, nq, groups):
+    t = Attention(pkg, n, *shape, False)
+    t.fill(hip, 0, n)
+    rows = t.put(t.rows[n - nq:])
+    hip.gqa_rows_dev(t.attn, rows, t.ld, False, False, pos_dev(n - nq), nq)
+    out = t.new(nq, t.heads * t.vdimp)
+    hip.gqa_prefill_dev(t.attn, rows, t.ld, n, nq, out, t.heads * t.vdimp)
+    assert hip.gqa_prefill_last_groups() == groups
+    t.check(out, n - nq, 2e-2)
+
+
 @pytest.mark.parametrize("f32", [True, False])
 @pytest.mark.parametrize("n,nq", [(1, 1), (130, 130), (300, 2)])
 @pytest.mark.parametrize("shape", SHAPES + [(2, 1, 300, 270, 2)])
