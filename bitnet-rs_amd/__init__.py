@@ -442,6 +442,11 @@ class HipLib:
         self._check(self.c.bitnet_hip_matmul_last_tile(*[C.byref(x) for x in v]))
         return dict(zip(("digits", "wave_tokens", "waves", "scale_mode"), (x.value for x in v)))
 
+    def matmul_takes_few_rows(self, h: int, m: int, flags: int, digits: int) -> bool:
+        """Would matmul_fused_dev run the form for few rows?"""
+        self.c.bitnet_hip_matmul_takes_few_rows.argtypes = [C.c_uint64, _sz, C.c_int, C.c_int]
+        return self.c.bitnet_hip_matmul_takes_few_rows(h, m, flags, digits) == 1
+
     def matmul_last_wave_rows(self) -> int:
         """Output rows per wave of this thread's last tiled matmul: 64, or 80 (320-row workgroups)."""
         return int(self.c.bitnet_hip_matmul_last_wave_rows())

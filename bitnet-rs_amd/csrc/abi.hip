@@ -381,6 +381,24 @@ size_t bitnet_hip_matmul_workspace_bytes(size_t m, size_t k, int digits) {
     return gemm_workspace_bytes(m, k, digits >= 2 && digits <= 4 ? digits : 4);
 }
 
+static GemvFusion matmul_flags(int flags) {
+    GemvFusion fu;
+    fu.silu_mul = (flags & BITNET_HIP_FUSE_SILU_MUL) != 0;
+    fu.x_f16 = (flags & BITNET_HIP_FUSE_X_F16) != 0;
+    fu.y_f16 = (flags & BITNET_HIP_FUSE_Y_F16) != 0;
+    fu.int8_form = (flags & BITNET_HIP_FUSE_INT8_DIGITS) != 0;
+    fu.fp6_form = (flags & BITNET_HIP_FUSE_FP6_DIGITS) != 0;
+    fu.fp6_expand = (flags & BITNET_HIP_FUSE_FP6_EXPAND) != 0;
+    return fu;
+}
+
+int bitnet_hip_matmul_takes_few_rows(bitnet_hip_weights_t h, size_t m, int flags, int digits) {
+    BH_GUARD_BEGIN
+    const WeightsRef w = lookup(h);
+    return w && m > 0 && gemm_takes_few(*w, matmul_flags(flags), m, digits) ? 1 : 0;
+    BH_GUARD_END
+}
+
 int bitnet_hip_matmul_fused_dev(bitnet_hip_weights_t h, const float *x_dev, float *y_dev, size_t m,
                                 const float *ln_gamma_dev, float ln_eps, const float *residual_dev, int flags, int digits,
                                 void *workspace_dev, size_t workspace_bytes, void *stream) {
@@ -390,16 +408,10 @@ int bitnet_hip_matmul_fused_dev(bitnet_hip_weights_t h, const float *x_dev, floa
     if (!x_dev || !y_dev) return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "Null pointer passed to matmul_fused_dev");
     if (m == 0) return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "dimensions must be > 0: m=0");
     if (digits < 2 || digits > 4) return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "digits must be 2, 3 or 4, got %d", digits);
-    GemvFusion fu;
+    GemvFusion fu = matmul_flags(flags);
     fu.ln_gamma = ln_gamma_dev;
     fu.ln_eps = ln_eps;
     fu.residual = residual_dev;
-    fu.silu_mul = (flags & BITNET_HIP_FUSE_SILU_MUL) != 0;
-    fu.x_f16 = (flags & BITNET_HIP_FUSE_X_F16) != 0;
-    fu.y_f16 = (flags & BITNET_HIP_FUSE_Y_F16) != 0;
-    fu.int8_form = (flags & BITNET_HIP_FUSE_INT8_DIGITS) != 0;
-    fu.fp6_form = (flags & BITNET_HIP_FUSE_FP6_DIGITS) != 0;
-    fu.fp6_expand = (flags & BITNET_HIP_FUSE_FP6_EXPAND) != 0;
     if (fu.fp6_form && (fu.int8_form || digits != 2 || !gemm_fp6_supported(*w)))
         return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "FUSE_FP6_DIGITS needs digits = 2, an unscaled matrix with a code map in -2..2, and no FUSE_INT8_DIGITS");
     if (fu.silu_mul && (!w->paired || residual_dev))

@@ -203,6 +203,7 @@ bool gemm_fp6_supported(const Weights &w);
 bool gemm_fp4_resident_enabled();                            // BITNET_HIP_FP4_RESIDENT != 0 (default on)
 hipError_t ensure_fp4_image(Weights &w, hipStream_t stream);  // builds Weights::tiles4 once (under the handle's mutex)
 void drop_fp4_image(Weights &w);
+bool gemm_takes_few(const Weights &w, const GemvFusion &fu, size_t m, int ndig);  // ... k_gemm_few?
 bool gemm_takes_fp6(const Weights &w, const GemvFusion &fu, int ndig);  // would launch_gemm_mfma run k_gemm_fp6 for this call?  // unscaled, code map in -2 .. 2: the fp6 x fp4 form of the 2-digit product (k_gemm_fp6)
 bool gemm_needs_row_major_scales(const Weights &w);  // 256-block scales and non-f16 32-block scales: the others read the scale tiles
 size_t gemm_workspace_bytes(size_t m, size_t cols, int ndig);

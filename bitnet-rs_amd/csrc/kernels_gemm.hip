@@ -2188,9 +2188,6 @@ __global__ __launch_bounds__(512, 4) void k_gemm_few(GemmArgs p) {
     }
 }
 
-// Prompt of bitnet-b1.58-2B-4T (QK256), ms with this / without: 16 tokens 1.76 / 3.39, 64 2.29 / 3.56, 128 2.88 / 3.62, 192 3.52 / 3.97, 256 4.11 / 4.02 (every workgroup
-// reads its 16 tokens' planes for itself: from there on the wide tiles are ahead).
-constexpr size_t kFewTokens = 192;
 static hipError_t launch_gemm_few(const Weights &w, QuantArgs q, const GemmArgs &a, hipStream_t stream) {
     const unsigned n_tok = (unsigned)(q.m + 15) / 16, rt = a.silu_mul ? 2 : 1;
     q.m_pad = (int)(16 * n_tok);
@@ -2309,6 +2306,10 @@ static uint32_t lut_fp4(uint32_t lut) {
     }
     return out;
 }
+static int gemm_f16a_mode() {
+    static const int mode = [] { const char *e = getenv("BITNET_HIP_GEMM_F16A"); return e ? atoi(e) : 0; }();
+    return mode;
+}
 int gemm_fp6_mode() {
     static const int mode = [] { const char *e = getenv("BITNET_HIP_GEMM_FP6"); return e ? atoi(e) : 0; }();
     return mode;
@@ -2349,9 +2350,22 @@ void drop_fp4_image(Weights &w) {
 bool gemm_takes_fp6(const Weights &w, const GemvFusion &fu, int ndig) {
     if (fu.int8_form || ndig != 2 || !gemm_fp6_supported(w)) return false;
     if (gemm_k32(w)) return false;
-    static const int f16a_mode = [] { const char *e = getenv("BITNET_HIP_GEMM_F16A"); return e ? atoi(e) : 0; }();
-    if (f16a_mode && w.cols % 256 == 0) return false;
+    if (gemm_f16a_mode() && w.cols % 256 == 0) return false;
     return fu.fp6_form || gemm_fp6_mode();
+}
+// would it send this call to k_gemm_few?  (the prompt forward asks, too: the fp6 digits are for the launches that do not)
+// A workgroup of that form reads its 16 tokens' planes for itself, so it costs by workgroups: 0.35 ns per 256 columns each, with the chip full, and its weights once.  The wide
+// tiles cost by their K steps, one chain however few rows there are (0.92 us per 256 columns), until their row blocks fill the chip.  us per launch, quantiser included, this / the
+// wide form (the faster of int8 and fp6): 2560 x 2560 rows x columns, 192 tokens 15.7 / 17.2, 2560 x 6912, 192 27 / 33, 3840 x 2560, 128 14.9 / 16.7, 160 16.6 / 17.2, 192 18.7 / 17.1,
+// 4096 x 4096, 128 20.2 / 22.0, 192 25.9 / 22.5; pairs of 13824 x 2560, 64 16.1 / 19.8, 100 22.0 / 19.9, 160 26.6 / 27.5, 192 30.2 / 27.3, of 28672 x 4096, 64 35 / 40, 128 57 / 40.
+bool gemm_takes_few(const Weights &w, const GemvFusion &fu, size_t m, int ndig) {
+    if (!gemm_supported(w) || ndig != 2 || w.scaled || gemm_takes_fp6(w, fu, ndig)) return false;
+    if (!fu.int8_form && gemm_f16a_mode() && lut_fits_f16w(w.lut) && w.cols % 256 == 0) return false;
+    // (a pair of gate and up tiles wants them both in the matrix; measured up to 192 rows)
+    if (m > 192 || (fu.silu_mul && w.rows % 32 != 0)) return false;
+    const double blocks = (double)div_ceil(w.cols, 256), workgroups = (double)div_ceil(div_ceil(w.rows, 16), fu.silu_mul ? 2 : 1) * div_ceil(m, 16);
+    const double row_blocks = (double)div_ceil(w.rows, 256) * div_ceil(m, 128), rounds = std::max(1.0, 0.55 + 0.016 * std::min(row_blocks, 180.0));
+    return workgroups * (0.2 + 0.35 * blocks) + (double)(w.rows * w.cols / 4) / 4800 <= 920 * blocks * rounds;
 }
 
 static hipError_t launch_gemm_fp6(const Weights &w, const QuantArgs &q, const GemmArgs &a, hipStream_t stream) {
@@ -2624,14 +2638,12 @@ hipError_t launch_gemm_mfma(const Weights &w, const float *x, float *y, size_t m
     }
     if (takes_f16) return launch_gemm_f16(w, q, a, stream);  // BitNet32-F16 at f16 activation precision: the f16 matrix cores
     if (!fu.int8_form) {
-        static const int f16a_mode = [] { const char *e = getenv("BITNET_HIP_GEMM_F16A"); return e ? atoi(e) : 0; }();
-        if (f16a_mode && ndig == 2 && !w.scaled && lut_fits_f16w(w.lut) && w.cols % 256 == 0)
+        if (gemm_f16a_mode() && ndig == 2 && !w.scaled && lut_fits_f16w(w.lut) && w.cols % 256 == 0)
             return launch_gemm_f16(w, q, a, stream);
     }
     // unscaled matrices at 2 digits: the same integer on the fp6 x fp4 MFMA, on request (flag) or by BITNET_HIP_GEMM_FP6=1
     if (!fu.int8_form && gemm_takes_fp6(w, fu, ndig)) return launch_gemm_fp6(w, q, a, stream);
-    // (rows past 8192 columns do not fit the quantiser's registers; a pair of gate and up tiles wants them both in the matrix)
-    if (ndig == 2 && !w.scaled && m <= kFewTokens && w.cols <= 8192 && (!fu.silu_mul || w.rows % 32 == 0)) return launch_gemm_few(w, q, a, stream);
+    if (gemm_takes_few(w, fu, m, ndig)) return launch_gemm_few(w, q, a, stream);
     if (ndig == 2) return launch_gemm_t<2, 4>(w, q, a, stream);
     if (ndig == 3) return launch_gemm_t<3, 2>(w, q, a, stream);
     return launch_gemm_t<4, 2>(w, q, a, stream);

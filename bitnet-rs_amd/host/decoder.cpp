@@ -788,13 +788,13 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
     // matrix cores as they stand (k_gemm_f16a, 320-row workgroups: one round of the chip at 4096 tokens) -- no quantiser launch, no second
     // rounding of values that were rounded to f16 already; q|k|v and gate|up keep the faster int8 digit planes behind their LayerNorm.
     const bool hybrid = h16 && hybrid_applies(N);
-    // (up to 192 rows the int8 digits have a form of their own, k_gemm_few: faster, and the same outputs bit for bit)
-    const int f6 = (chain || qb || N <= 192) ? 0 : fp6_flag(digits);
+    // (with few rows the int8 digits have a form of their own, k_gemm_few: the kernel library says where it is the faster one; the same outputs bit for bit)
+    auto f6 = [&](bitnet_hip_weights_t h, int flags) { return bitnet_hip_matmul_takes_few_rows(h, N, flags, digits) == 1 ? 0 : fp6_flag(digits); };
     static const int f6od_env = getenv("BITNET_HOST_PREFILL_FP6_OD") ? atoi(getenv("BITNET_HOST_PREFILL_FP6_OD")) : 0;  // experiment: o / down on the fp6 form too (non-hybrid)
-    const int f6od = f6od_env ? f6 : 0;
+    auto f6od = [&](bitnet_hip_weights_t h, int flags) { return f6od_env ? f6(h, flags) : 0; };
     for (auto &L : layers_) {
         if (chain || qb) break;
-        BCHK(bitnet_hip_matmul_fused_dev(L.qkv, pf_x_, pf_qkv_, N, L.attn_norm, c_.eps, nullptr, f6, digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
+        BCHK(bitnet_hip_matmul_fused_dev(L.qkv, pf_x_, pf_qkv_, N, L.attn_norm, c_.eps, nullptr, f6(L.qkv, 0), digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
         if (h16) {
             BCHK(bitnet_hip_attention_prefill_flags_dev(pf_qkv_, rope_sin_, rope_cos_, L.kcache, L.vcache, (size_t)c_.n_heads, (size_t)c_.n_kv_heads, (size_t)c_.head_dim,
                                                         (size_t)c_.max_pos, N, pf_attn_ws_, pf_attn_ws_bytes_, pf_atth_,
@@ -802,13 +802,13 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
             if (hybrid)
                 BCHK(bitnet_hip_matmul_f16_dev(L.o, pf_atth_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, 0, nullptr, nullptr, nullptr, s));
             else
-                BCHK(bitnet_hip_matmul_fused_dev(L.o, (const float *)pf_atth_, pf_x_, N, nullptr, 0.f, pf_x_, BITNET_HIP_FUSE_X_F16 | f6od, digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
-            BCHK(bitnet_hip_matmul_fused_dev(L.gateup, pf_x_, (float *)pf_hh_, N, L.ffn_norm, c_.eps, nullptr, BITNET_HIP_FUSE_SILU_MUL | BITNET_HIP_FUSE_Y_F16 | f6, digits,
+                BCHK(bitnet_hip_matmul_fused_dev(L.o, (const float *)pf_atth_, pf_x_, N, nullptr, 0.f, pf_x_, BITNET_HIP_FUSE_X_F16 | f6od(L.o, BITNET_HIP_FUSE_X_F16), digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
+            BCHK(bitnet_hip_matmul_fused_dev(L.gateup, pf_x_, (float *)pf_hh_, N, L.ffn_norm, c_.eps, nullptr, BITNET_HIP_FUSE_SILU_MUL | BITNET_HIP_FUSE_Y_F16 | f6(L.gateup, BITNET_HIP_FUSE_SILU_MUL), digits,
                                              pf_gemm_ws_, pf_gemm_ws_bytes_, s));
             if (hybrid)
                 BCHK(bitnet_hip_matmul_f16_dev(L.down, pf_hh_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, 0, nullptr, nullptr, nullptr, s));
             else
-                BCHK(bitnet_hip_matmul_fused_dev(L.down, (const float *)pf_hh_, pf_x_, N, nullptr, 0.f, pf_x_, BITNET_HIP_FUSE_X_F16 | f6od, digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
+                BCHK(bitnet_hip_matmul_fused_dev(L.down, (const float *)pf_hh_, pf_x_, N, nullptr, 0.f, pf_x_, BITNET_HIP_FUSE_X_F16 | f6od(L.down, BITNET_HIP_FUSE_X_F16), digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
             continue;
         }
         if (kv_f16_)
@@ -818,7 +818,7 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
             BCHK(bitnet_hip_attention_prefill_dev(pf_qkv_, rope_sin_, rope_cos_, L.kcache, L.vcache, (size_t)c_.n_heads, (size_t)c_.n_kv_heads,
                                                   (size_t)c_.head_dim, (size_t)c_.max_pos, N, pf_attn_ws_, pf_attn_ws_bytes_, pf_att_, s));
         BCHK(bitnet_hip_matmul_fused_dev(L.o, pf_att_, pf_x_, N, nullptr, 0.f, pf_x_, 0, digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
-        BCHK(bitnet_hip_matmul_fused_dev(L.gateup, pf_x_, pf_h_, N, L.ffn_norm, c_.eps, nullptr, BITNET_HIP_FUSE_SILU_MUL | f6, digits, pf_gemm_ws_,
+        BCHK(bitnet_hip_matmul_fused_dev(L.gateup, pf_x_, pf_h_, N, L.ffn_norm, c_.eps, nullptr, BITNET_HIP_FUSE_SILU_MUL | f6(L.gateup, BITNET_HIP_FUSE_SILU_MUL), digits, pf_gemm_ws_,
                                          pf_gemm_ws_bytes_, s));
         BCHK(bitnet_hip_matmul_fused_dev(L.down, pf_h_, pf_x_, N, nullptr, 0.f, pf_x_, 0, digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
     }

@@ -246,6 +246,9 @@ int bitnet_hip_matmul_fused_dev(bitnet_hip_weights_t w, const float *x_dev, floa
                                 const float *ln_gamma_dev, float ln_eps, const float *residual_dev,
                                 int flags, int digits, void *workspace_dev, size_t workspace_bytes,
                                 void *stream);
+/* 1 when bitnet_hip_matmul_fused_dev would run the form for few rows with these flags (k_gemm_few: int8 digit planes, digits = 2 on an unscaled matrix, up to 192 rows, where it is
+ * the faster one for this matrix), else 0.  Without it a prompt forward sets BITNET_HIP_FUSE_FP6_DIGITS: the same outputs bit for bit whichever form runs. */
+int bitnet_hip_matmul_takes_few_rows(bitnet_hip_weights_t w, size_t m, int flags, int digits);
 /* Which tile form the calling thread's last bitnet_hip_matmul_[fused_]dev launch ran (any pointer may be null): digits,
  * tokens per wave tile (16 / 32 / 64), waves per workgroup (4 / 8), weight-scale mode (0 none, 1 per 256-block, 2 per
  * 32-block on the masked K = 64 MFMA, 3 per 32-block on the K = 32 int8 MFMA with f16 scale tiles, 4 the f16 MFMA with the block

@@ -363,6 +363,28 @@ def test_few_rows_are_the_wide_tiles_product_bit_for_bit(hip, torch_, rows, cols
         hip.weights_free(i)
 
 
+# either side of the lines between k_gemm_few and the wide tiles: a narrow matrix, a wide one in one and in two rounds, a long K, 192 rows
+@pytest.mark.parametrize("rows,cols,m,few", [(3840, 2560, 128, True), (3840, 2560, 192, False), (2560, 6912, 192, True), (2560, 6912, 193, False), (4096, 4096, 144, True),
+                                             (4096, 4096, 176, False), (-13824, 2560, 80, True), (-13824, 2560, 112, False), (-13824, 2560, 144, True),
+                                             (-13824, 2560, 192, False)])
+def test_few_rows_only_where_they_are_faster(hip, torch_, rows, cols, m, few):
+    """rows < 0: pairs of gate and up tiles.  The query, the launch and the outputs agree: the wide int8 tiles' and the fp6 digits' bit for bit"""
+    paired, rows = rows < 0, abs(rows)
+    rng = np.random.default_rng(rows + cols + m)
+    stride, n = -(-cols // 256) * 64, rows // 2 if paired else rows
+    parts = [hip.weights_upload_qk256(rng.integers(0, 256, n * stride, dtype=np.uint8), n, cols, stride) for _ in range(2 if paired else 1)]
+    h, flags = (hip.weights_concat(parts, interleave16=True), SILU_MUL) if paired else (parts[0], 0)
+    x = (rng.normal(0.1, 1.0, (m, cols)) * np.exp(rng.uniform(-3, 3, (m, 1)))).astype(np.float32)
+    assert hip.matmul_takes_few_rows(h, m, flags, 2) == few == hip.matmul_takes_few_rows(h, m, flags | INT8_DIGITS, 2)
+    assert not hip.matmul_takes_few_rows(h, m, flags | FP6_DIGITS, 2) and not hip.matmul_takes_few_rows(h, m, flags, 3)
+    got = run_gemm(hip, torch_, h, x, n, 2, flags=flags)
+    t = hip.matmul_last_tile()
+    assert t["scale_mode"] == 0 and (t["waves"] == 8) == few, t
+    assert not np.isnan(got).any() and np.array_equal(got, run_gemm(hip, torch_, h, x, n, 2, flags=flags | FP6_DIGITS))
+    for i in {h, *parts}:
+        hip.weights_free(i)
+
+
 FP6_EXPAND = 32  # BITNET_HIP_FUSE_FP6_EXPAND
 
 
