@@ -493,6 +493,20 @@ struct GemvK {
     int lat_wg;    // workgroup index that writes the latent row, or -1
 };
 
+// An argument's value as if it were read here: a condition on it is then made where it is used.  Made once and kept, the conditions of the instances with MORE took a pair of
+// scalar registers each from the first load to the last store; eight to twelve were spilled, with scratch memory reserved for them.
+template <bool MORE, class T>
+__device__ __forceinline__ T here(T v) {
+    if constexpr (MORE) asm volatile("" : "+s"(v));
+    return v;
+}
+
+template <bool FIRST, class T>
+__device__ __forceinline__ T &either(T &a, T &b) {
+    if constexpr (FIRST) return a;
+    return b;
+}
+
 // Loads return in order, so whatever a wave asked for ahead of its input it also waits for: the input's loads go out first, `weights` (the first rows' requests)
 // behind them, the arithmetic last -- it runs while the weights are on their way.
 // NR: sixteen-byte registers per thread, for vectors of up to 1024 NR elements; longer ones are formed in LDS.  slot: twelve floats.
@@ -530,24 +544,33 @@ __device__ __forceinline__ void form_input(const VecIn &in, const float *x, int 
         __syncthreads();
         return;
     }
-    const bool added = in.kind >= BITNET_HIP_IN_RESIDUAL_NORM && in.y, normed = added && in.post_weight, last_norm = in.kind < BITNET_HIP_IN_CONCAT, two = in.kind == BITNET_HIP_IN_CONCAT;
+    auto added = [&] { return here<MORE>(in.kind) >= BITNET_HIP_IN_RESIDUAL_NORM && here<MORE>(in.y); };
+    auto normed = [&] { return added() && here<MORE>(in.post_weight); };
+    auto last_norm = [&] { return here<MORE>(in.kind) < BITNET_HIP_IN_CONCAT; };
+    auto two = [&] { return here<MORE>(in.kind) == BITNET_HIP_IN_CONCAT; };
     if ((n & 3) == 0 && n <= 1024 * NR) {
-        f32x4 xv[NR], yv[NR], pw[NR], sc[NR], yg[NR], wv[NR], bv[NR], gv[NR];
+        // (MORE: a bias waits for the registers of a gate on what is added, a gate on the norm for those of the added norm's weight; with registers of their own two workgroups
+        // of 13824 x 4096 fit a CU instead of three: 28.4 us, 23.1 without a gate)
+        f32x4 xv[NR], yv[NR], pw[NR], sc[NR], yg[NR], wv[NR], b_own[NR], g_own[NR];
+        auto &bv = either<MORE>(yg, b_own), &gv = either<MORE>(pw, g_own);
         const int n4 = n >> 2;
-        const bool scaled = normed && in.scale, y_gated = MORE && added && in.y_gate, shifted = last_norm && in.center && in.bias, gated = last_norm && in.gate;
+        auto scaled = [&] { return normed() && here<MORE>(in.scale); };
+        auto y_gated = [&] { return MORE && added() && here<MORE>(in.y_gate); };
+        auto shifted = [&] { return last_norm() && here<MORE>(in.center) && here<MORE>(in.bias); };
+        auto gated = [&] { return last_norm() && here<MORE>(in.gate); };
         auto load = [&](f32x4 (&v)[NR], const float *from) {
 #pragma unroll
             for (int j = 0; j < NR; ++j) v[j] = reinterpret_cast<const f32x4 *>(from)[min(tid + 256 * j, n4 - 1)];
         };
         load(xv, x);
-        if (added) load(yv, in.y);
-        if (normed) load(pw, in.post_weight);
-        if (scaled) load(sc, in.scale);
-        if (y_gated) load(yg, in.y_gate);
-        if (last_norm) load(wv, in.weight);
-        if (two) load(wv, in.x2);
-        if (shifted) load(bv, in.bias);
-        if (gated) load(gv, in.gate);
+        if (added()) load(yv, in.y);
+        if (normed()) load(pw, in.post_weight);
+        if (scaled()) load(sc, in.scale);
+        if (y_gated()) load(yg, in.y_gate);
+        if (last_norm()) load(wv, in.weight);
+        if (two()) load(wv, in.x2);
+        if (shifted() && !y_gated()) load(bv, in.bias);
+        if (gated() && !(MORE && normed())) load(gv, in.gate);
         weights();
         auto squares = [&](const f32x4 (&v)[NR]) {
             float ss = 0.f;
@@ -557,32 +580,36 @@ __device__ __forceinline__ void form_input(const VecIn &in, const float *x, int 
         };
         const float count = (float)in.mean_n, eps = in.eps, offset = in.offset;
         auto inverse = [=](float ss) { return 1.0f / sqrtf(ss / count + eps); };
-        if (added) {
-            const float inv = normed ? inverse(group_total<4>(squares(yv), slot)) : 1.0f;
+        if (added()) {
+            const bool of_norm = normed(), of_scale = scaled(), of_gate = y_gated();
+            const float inv = of_norm ? inverse(group_total<4>(squares(yv), slot)) : 1.0f;
 #pragma unroll
             for (int j = 0; j < NR; ++j) {
                 const int i = tid + 256 * j;
-                f32x4 v = yv[j] * (normed ? inv : in.mult);
-                if (normed) v *= offset + pw[j];
-                if (scaled) v *= sc[j];
-                if (y_gated) v *= yg[j];
+                f32x4 v = yv[j] * (of_norm ? inv : in.mult);
+                if (of_norm) v *= offset + pw[j];
+                if (of_scale) v *= sc[j];
+                if (of_gate) v *= yg[j];
                 xv[j] += v;
                 if (writer && in.x_out && i < n4) reinterpret_cast<f32x4 *>(in.x_out)[i] = xv[j];
             }
         }
-        if (!last_norm) {
+        if (shifted() && y_gated()) load(bv, in.bias);
+        if (MORE && gated() && normed()) load(gv, in.gate);
+        if (!last_norm()) {
+            const bool concat = two();
 #pragma unroll
             for (int j = 0; j < NR; ++j) {
                 const int i = tid + 256 * j;
                 if (i >= n4) continue;
                 reinterpret_cast<f32x4 *>(xs)[i] = xv[j];
-                if (two) reinterpret_cast<f32x4 *>(xs)[n4 + i] = wv[j];
+                if (concat) reinterpret_cast<f32x4 *>(xs)[n4 + i] = wv[j];
             }
-            for (int i = (two ? 2 : 1) * n + tid; i < kp; i += 256) xs[i] = 0.f;
+            for (int i = (concat ? 2 : 1) * n + tid; i < kp; i += 256) xs[i] = 0.f;
             __syncthreads();
             return;
         }
-        if (in.center) {
+        if (here<MORE>(in.center)) {
             float t = 0.f;
 #pragma unroll
             for (int j = 0; j < NR; ++j) t += tid + 256 * j < n4 ? (xv[j].x + xv[j].y) + (xv[j].z + xv[j].w) : 0.f;
@@ -591,27 +618,28 @@ __device__ __forceinline__ void form_input(const VecIn &in, const float *x, int 
             for (int j = 0; j < NR; ++j) xv[j] -= mean;
         }
         const float inv = inverse(group_total<4>(squares(xv), slot + 8));
+        const bool of_gate = gated(), of_bias = shifted();
 #pragma unroll
         for (int j = 0; j < NR; ++j) {
             const int i = tid + 256 * j;
             if (i >= n4) continue;
             f32x4 r = xv[j] * inv * (offset + wv[j]);
-            if (gated) r *= gv[j];
-            if (shifted) r += bv[j];
+            if (of_gate) r *= gv[j];
+            if (of_bias) r += bv[j];
             reinterpret_cast<f32x4 *>(xs)[i] = r;
             if (writer && in.h_out) reinterpret_cast<f32x4 *>(in.h_out)[i] = r;
         }
     } else {
         weights();
         float ss = 0.f;
-        if (added && !normed) {
+        if (added() && !normed()) {
             for (int i = tid; i < n; i += 256) {
                 const float v = x[i] + in.mult * in.y[i] * (MORE && in.y_gate ? in.y_gate[i] : 1.0f);
                 xs[i] = v;
                 if (writer && in.x_out) in.x_out[i] = v;
                 ss += v * v;
             }
-        } else if (added) {
+        } else if (added()) {
             for (int i = tid; i < n; i += 256) ss += in.y[i] * in.y[i];
             const float inv = 1.0f / sqrtf(group_sum<4>(ss, slot) / (float)in.mean_n + in.eps);
             ss = 0.f;
@@ -627,9 +655,10 @@ __device__ __forceinline__ void form_input(const VecIn &in, const float *x, int 
                 ss += x[i] * x[i];
             }
         }
-        if (!last_norm) {
-            for (int i = tid; two && i < n; i += 256) xs[n + i] = in.x2[i];
-            for (int i = (two ? 2 : 1) * n + tid; i < kp; i += 256) xs[i] = 0.f;
+        if (!last_norm()) {
+            const bool concat = two();
+            for (int i = tid; concat && i < n; i += 256) xs[n + i] = in.x2[i];
+            for (int i = (concat ? 2 : 1) * n + tid; i < kp; i += 256) xs[i] = 0.f;
             __syncthreads();
             return;
         }
@@ -666,7 +695,7 @@ __device__ __forceinline__ float lanes_total(float v) {
 
 // MORE: whatever bitnet_hip_epilogue and a gate on the residual ask for
 template <int LPR, int R, int U, bool MORE, int NR>
-__global__ __launch_bounds__(256) void k_dense_gemv(GemvK p) {
+__global__ __launch_bounds__(256, MORE && R * U >= 20 ? 2 : 1) void k_dense_gemv(GemvK p) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
     __shared__ float slot[12];
     __shared__ float wbv[4];
@@ -709,7 +738,14 @@ __global__ __launch_bounds__(256) void k_dense_gemv(GemvK p) {
     // the earlier positions of a convolution's rows, a tap per lane; summed behind the product
     const Epilogue &e = a.more;
     const bool conv = MORE && e.conv, mul = MORE && e.mul;
-    const int pos = conv ? *e.pos : 0, mul_at = mul ? *e.mul_at : 0;
+    // (arguments read where they are used: with a convolution's they do not all fit the scalar registers)
+    auto late = [] {
+        auto *k = (const __attribute__((address_space(4))) GemvK *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(k));
+        return k;
+    };
+    const int pos = conv ? *e.pos : 0;
+    int mul_at = 0;
     float past[R];
     auto fetch_past = [&](int grp) {
 #pragma unroll
@@ -727,6 +763,7 @@ __global__ __launch_bounds__(256) void k_dense_gemv(GemvK p) {
     form_input<MORE, NR>(a.in, a.in.x + (size_t)b * a.x_batch, a.cols, p.kp, xs, slot, blockIdx.x == 0 && b == 0, [&] {
         if (conv && g < p.groups) fetch_past(g);
         if (g < p.groups) fetch(g, 0);
+        if (mul) mul_at = *e.mul_at;
     });
     float bv = -INFINITY;
     int bi = 0x7fffffff;
@@ -796,8 +833,11 @@ __global__ __launch_bounds__(256) void k_dense_gemv(GemvK p) {
                 float v = acc[r];
                 if (a.bias && (!conv || ch < 0 || ch >= e.channels)) v += a.bias[row];
                 const int act = MORE && row >= e.act2_from ? e.act2 : row < a.act_split ? a.act0 : a.act1;
-                v = MORE ? activate(v, act, e.act_a, e.act_b) : activate(v, act);
-                if (mul) v *= bf2f(e.mul[(size_t)min(max(e.mul_tokens[mul_at], 0), e.mul_rows - 1) * e.ld_mul + row]);
+                v = MORE && act == BITNET_HIP_ACT_XIELU ? activate(v, act, late()->a.more.act_a, late()->a.more.act_b) : activate(v, act);
+                if (mul) {
+                    const auto &f = late()->a.more;
+                    v *= bf2f(f.mul[(size_t)min(max(f.mul_tokens[mul_at], 0), f.mul_rows - 1) * f.ld_mul + row]);
+                }
                 a.y[(size_t)b * a.y_batch + row - (MORE ? a.gated >> 1 : 0)] = v;
                 if (a.best_val) {
                     const float t = v != v ? -INFINITY : v;

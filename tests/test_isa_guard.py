@@ -228,3 +228,15 @@ def test_fp6w_k_loop_mixes_dma_and_tracked_loads_without_a_counted_wait(isa):
     assert not any(t.startswith(("scratch_", "global_store", "buffer_store")) for _, _, t in ins)
     waits = [t for _, _, t in ins if "vmcnt" in t]
     assert len(waits) == 1 and "vmcnt(0)" in waits[0], waits
+
+
+def test_matrix_vector_products_keep_no_scratch(tmp_path):
+    """Every instance of k_dense_gemv, those with convolutions, tables, pairs and gates too, keeps its arguments in registers; and an instance alone on its SIMD has nothing to run
+    while it waits for weights"""
+    if not os.path.exists(HIPCC):
+        pytest.skip("no hipcc")
+    _, usage = _compile("kernels_dense.hip", str(tmp_path))
+    gemv = {name: u for name, u in usage.items() if "k_dense_gemv" in name}
+    assert len(gemv) >= 60
+    for name, u in gemv.items():
+        assert u["ScratchSize"] == 0 and u["Occupancy"] >= 2, (name, u)

@@ -26,7 +26,7 @@ def test_gemv_plain(hip, pkg, rows, cols):
     assert u.rms_error(u.host(y), want) < F32_TOL
 
 
-@pytest.mark.parametrize("n", [80, 96, 384, 1001, 2560, 4096, 5000])
+@pytest.mark.parametrize("n", [80, 96, 384, 1001, 2560, 2564, 3072, 3076, 4096, 5000])
 @pytest.mark.parametrize("kind", ["norm", "gated", "residual", "first"])
 def test_gemv_input_transforms(hip, pkg, n, kind):
     g = rng(n, len(kind))

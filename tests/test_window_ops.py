@@ -142,6 +142,24 @@ def test_gemv_adds_a_gated_sublayer(hip, pkg, n):
         assert u.rms_error(u.host(xo), x2) < F32_TOL and u.rms_error(u.host(out), w @ so.layer_norm(x2, nw, nb, eps)) < F32_TOL
 
 
+# every vector an input can be formed of, in one call: some of them share registers; three and four registers per thread (3072) and none (4096)
+@pytest.mark.parametrize("n", [80, 1001, 2560, 3072, 3076, 4096, 4100])
+@pytest.mark.parametrize("gated,biased,scaled", [(True, True, True), (True, False, False), (False, True, False), (True, False, True)])
+def test_gemv_forms_its_input_of_everything(hip, pkg, n, gated, biased, scaled):
+    g = rng(n, 5)
+    rows, ld, cols, eps = 70, u.up_to(n, 64), u.up_to(n, 8), 1e-3
+    w = u.rounded(g.standard_normal((rows, n)) / np.sqrt(n))
+    x, y, nw, nb, pw, sc, gate = (g.standard_normal(n).astype(np.float32) for _ in range(7))
+    y_gate = g.random(n).astype(np.float32)
+    out, xo, ho = u.zeros_f32(rows), u.zeros_f32(n), u.zeros_f32(n)
+    hip.dense_gemv_dev(u.dev_f32(x), u.dev_bf16(u.padded(w, ld)), rows, cols, ld, out, kind=pkg.IN_RESIDUAL_NORM, eps=eps, weight=u.dev_f32(nw), center=True, res=u.dev_f32(y),
+                       norm_bias=u.dev_f32(nb) if biased else None, post_weight=u.dev_f32(pw), scale=u.dev_f32(sc) if scaled else None, gate=u.dev_f32(gate) if gated else None,
+                       y_gate=u.dev_f32(y_gate), x_out=xo, h_out=ho, n=n)
+    x2 = x + so.norm_plain(y.astype(f64), pw, eps) * y_gate * (sc if scaled else 1.0)
+    want = so.layer_norm(x2, nw, np.zeros(n), eps) * (gate if gated else 1.0) + (nb if biased else 0.0)
+    assert u.rms_error(u.host(xo), x2) < F32_TOL and u.rms_error(u.host(ho), want) < F32_TOL and u.rms_error(u.host(out), w @ want) < F32_TOL
+
+
 @pytest.mark.parametrize("width", [96, 90, 1000, 2560, 4096, 5000])
 @pytest.mark.parametrize("f32", [True, False])
 def test_rows_add_a_gated_sublayer(hip, pkg, width, f32):
