@@ -448,8 +448,12 @@ class HipLib:
         return self.c.bitnet_hip_matmul_takes_few_rows(h, m, flags, digits) == 1
 
     def matmul_last_wave_rows(self) -> int:
-        """Output rows per wave of this thread's last tiled matmul: 64, or 80 (320-row workgroups)."""
+        """Output rows per slab of LayerNorm partials of this thread's last tiled matmul: 64, or 80 (320-row workgroups)."""
         return int(self.c.bitnet_hip_matmul_last_wave_rows())
+
+    def matmul_last_workgroup_rows(self) -> int:
+        """Output rows per workgroup of this thread's last tiled matmul: 256, 320, 128, 32 or 16."""
+        return int(self.c.bitnet_hip_matmul_last_workgroup_rows())
 
     def matmul_last_resident_fp4(self) -> bool:
         self.c.bitnet_hip_matmul_last_resident_fp4.restype = C.c_int

@@ -578,6 +578,11 @@ int bitnet_hip_matmul_last_tile(int *digits, int *wave_tokens, int *waves, int *
 
 int bitnet_hip_matmul_last_wave_rows(void) { return g_last_gemm_tile.digits ? g_last_gemm_tile.wave_rows : 0; }
 
+int bitnet_hip_matmul_last_workgroup_rows(void) {
+    const GemmTileChoice &t = g_last_gemm_tile;
+    return !t.digits ? 0 : t.group_rows ? t.group_rows : 4 * t.wave_rows;
+}
+
 int bitnet_hip_matmul_last_resident_fp4(void) { return g_last_gemm_tile.resident_fp4; }
 
 int bitnet_hip_gemv_fused_dev(bitnet_hip_weights_t h, const float *x_dev, float *y_dev, size_t m,

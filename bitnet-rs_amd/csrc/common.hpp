@@ -241,6 +241,7 @@ hipError_t launch_gemm_mfma(const Weights &w, const float *x, float *y, size_t m
 struct GemmTileChoice {
     int digits = 0, wave_tokens = 0, waves = 0, scale_mode = 0, wave_rows = 64;
     int resident_fp4 = 0;  // the fp6 form read its weight operands from the resident fp4 image
+    int group_rows = 0;    // output rows per workgroup where they are not 4 wave_rows
 };
 extern thread_local GemmTileChoice g_last_gemm_tile;
 extern unsigned long long *g_mfma_stamps;  // diagnostic build only

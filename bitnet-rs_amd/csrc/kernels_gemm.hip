@@ -2192,7 +2192,7 @@ static hipError_t launch_gemm_few(const Weights &w, QuantArgs q, const GemmArgs 
     const unsigned n_tok = (unsigned)(q.m + 15) / 16, rt = a.silu_mul ? 2 : 1;
     q.m_pad = (int)(16 * n_tok);
     hipLaunchKernelGGL((q.kp <= 3072 ? k_quant_rows<2, 3, 2> : k_quant_rows<2, 8, 2>), dim3(q.m_pad), dim3(256), 0, stream, q);
-    g_last_gemm_tile = GemmTileChoice{2, 16, 8, 0, (int)(16 * rt)};
+    g_last_gemm_tile = GemmTileChoice{2, 16, 8, 0, (int)(16 * rt), 0, (int)(16 * rt)};
     hipLaunchKernelGGL(rt == 2 ? k_gemm_few<2> : k_gemm_few<1>, dim3((unsigned)div_ceil(div_ceil(w.rows, 16), rt), n_tok), dim3(512), (size_t)8 * rt * 2 * 1024, stream, a);
     return hipGetLastError();
 }
@@ -2399,7 +2399,7 @@ static hipError_t launch_gemm_fp6(const Weights &w, const QuantArgs &q, const Ge
     if (fp6w_mode && res && ttw == 4 && !rt5 && w.rows % 256 == 0 && (size_t)div_ceil(w.rows, 16) * (w.cols / 256) * 2048 < ((size_t)1 << 31)) {
         static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_fp6w), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);  // (72 KiB of tile buffers; once, thread-safe)
         if (raised != hipSuccess) return raised;
-        g_last_gemm_tile.wave_rows = 128;  // the 2 x 2 arrangement: a wave owns 128 rows x 32 tokens of the 256 x 64 tile
+        g_last_gemm_tile.wave_rows = 128, g_last_gemm_tile.group_rows = 256;  // the 2 x 2 arrangement: a wave owns 128 rows x 32 tokens of the 256 x 64 tile
         hipLaunchKernelGGL(k_gemm_fp6w, dim3((unsigned)gx0, (unsigned)(q.m_pad / 64)), dim3(256), (size_t)2 * 64 * 576, stream, aw);
         return hipGetLastError();
     }
@@ -2484,7 +2484,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
             f_raised.insert((const void *)fk);
         }
     }
-    g_last_gemm_tile = GemmTileChoice{2, 16 * ttw, 4, fmt1 ? 4 : 5, rt5 ? 80 : 64};
+    g_last_gemm_tile = GemmTileChoice{2, 16 * ttw, 4, fmt1 ? 4 : 5, rt5 ? 80 : 64, 0, rt2 ? 128 : 0};
     const size_t lds = (size_t)2 * ttw * 16 * 512 + (size_t)ttw * 16 * 8 + 4096;  // two tile buffers + the tokens' (mean, 1 / denom) + the statistics scratch
     // Wide launches (gate|up: 54 row blocks): 128-token workgroups (k_gemm_f16h: half the code expansion per MFMA) on as many row blocks as fill WHOLE rounds
     // of the 512 slots, this kernel's 64-token workgroups on the rest -- 13824 rows x 4096 tokens: 48 x 32 = 1536 workgroups = 3 rounds, then 6 x 64 = 384

@@ -255,11 +255,14 @@ int bitnet_hip_matmul_takes_few_rows(bitnet_hip_weights_t w, size_t m, int flags
  * scale folded into f16 weights and f16 activations: BitNet32-F16 at digits = 2).  The parity tests assert
  * that the instance bench.py times (2 digits, 64-token tile) is the one they compared with the oracle. */
 int bitnet_hip_matmul_last_tile(int *digits, int *wave_tokens, int *waves, int *scale_mode);
-/* Output rows per wave of that launch: 64 (four 16-row tiles, 256-row workgroups; also two waves of 32 that share a slab) or 80 (five: the 320-row workgroups the forms with
+/* Output rows that one slab of LayerNorm partials covers in that launch, a wave's: 64 (four 16-row tiles, 256-row workgroups; in the f16 chain's 128-row workgroups two waves of
+ * 32 make a slab) or 80 (five: the 320-row workgroups the forms with
  * f32 accumulators take when they need fewer rounds of the chip -- 2560 output rows x 4096 tokens = 512 workgroups, one round);
- * or 128 (the fp6 x fp4 form's 2 x 2 wave arrangement, k_gemm_fp6w: a wave owns 128 rows x 32 tokens of the 256 x 64 workgroup tile);
- * 0 before the thread's first tiled matmul.  scale_mode 5 = the f16 MFMA on an unscaled matrix, 6 = the fp6 x fp4 form (k_gemm_fp6). */
+ * or 128 (the fp6 x fp4 form's 2 x 2 wave arrangement, k_gemm_fp6w: a wave owns 128 rows x 32 tokens of the 256 x 64 workgroup tile); 16, or 32 in pairs (the form for few
+ * rows, whose eight waves share them); 0 before the thread's first tiled matmul.  scale_mode 5 = the f16 MFMA on an unscaled matrix, 6 = the fp6 x fp4 form (k_gemm_fp6). */
 int bitnet_hip_matmul_last_wave_rows(void);
+/* Output rows per workgroup of that launch: 256, 320, 128 (the f16 chain's short prompts), 16 or 32 (few rows); 0 before the first. */
+int bitnet_hip_matmul_last_workgroup_rows(void);
 /* 1 when that launch was the fp6 x fp4 form reading its weight operands from the resident fp4 image (below), else 0. */
 int bitnet_hip_matmul_last_resident_fp4(void);
 /* The resident fp4 image of an unscaled matrix whose code map lies in -2..2 (QK256: every value is exact in fp4 e2m1): 4 bits per

@@ -128,6 +128,7 @@ def test_f16_chain_half_slab_waves(hip, torch_, fmt, m):
     res = rng.normal(0, 1, (m, rows)).astype(np.float32)
     y, st = torch_.from_numpy(res).cuda(), torch_.full((rows // 64, mp, 2), float("nan"), device="cuda")
     hip.matmul_f16_dev(h, torch_.from_numpy(x).cuda(), m, y=y, residual=y, stats_out=st)
+    assert (hip.matmul_last_workgroup_rows(), hip.matmul_last_tile()["wave_tokens"]) == {17: (128, 16), 511: (128, 32), 800: (128, 32), 1025: (256, 32)}[m]
     torch_.cuda.synchronize()
     got, xd = y.cpu().numpy().astype(np.float64), x[:m].astype(np.float64)
     assert np.max(np.abs(got - (res + xd @ w.T)) / (np.abs(xd) @ np.abs(w).T + np.abs(res) + 1e-6)) <= 2e-6  # f16 inputs: accumulation order alone

@@ -355,7 +355,7 @@ def test_few_rows_are_the_wide_tiles_product_bit_for_bit(hip, torch_, rows, cols
     for kw in ({}, dict(ln_gamma=gd, ln_eps=1e-5), *(() if flags else (dict(residual=rd),))):
         few = run_gemm(hip, torch_, h, x, rows, 2, flags=flags, **kw)
         t = hip.matmul_last_tile()
-        assert t["scale_mode"] == 0 and t["waves"] == 8 and t["wave_tokens"] == 16, t
+        assert t["scale_mode"] == 0 and t["waves"] == 8 and t["wave_tokens"] == 16 and hip.matmul_last_workgroup_rows() == (32 if flags else 16), t
         wide = run_gemm(hip, torch_, h, x, rows, 2, flags=flags | FP6_DIGITS, **kw)
         assert hip.matmul_last_tile()["scale_mode"] == 6
         assert not np.isnan(few).any() and np.array_equal(few, wide), (sorted(kw), float(np.abs(few - wide).max()))
