@@ -558,6 +558,7 @@ __device__ __forceinline__ void store_wave_tiles(const GemmArgs &p, float (&val)
             if (token < p.m) {
 #pragma unroll
                 for (int pr = 0; pr < 2; ++pr) {
+                    if (ra + 16 * pr >= half_rows) continue;  // (a surplus tile: its place is in the next token's row, or behind the last one)
                     sh4 o;
                     bool sat = false;
 #pragma unroll

@@ -385,6 +385,47 @@ def test_few_rows_only_where_they_are_faster(hip, torch_, rows, cols, m, few):
         hip.weights_free(i)
 
 
+# rows handed over as f16, in and out, as the short and the longer prompts' forward does: the form for few rows (eight waves) and the wide int8 tiles (four)
+@pytest.mark.parametrize("n,k,m,waves", [(512, 1024, 1, 8), (512, 1024, 70, 8), (48, 1100, 33, 8), (2560, 6912, 19, 8), (2560, 6912, 177, 8), (512, 1024, 200, 4), (48, 1100, 215, 4),
+                                         (2560, 6912, 193, 4)])
+def test_f16_rows_in_and_out_of_few_and_many_rows(hip, torch_, n, k, m, waves):
+    """the down-projection, n x k, its rows in f16, with a residual; the pair of n x n in front of it hands f16 rows out.  Bit for bit the fp6 form's, and the f16 rows are the f32 outputs
+    rounded; n that ends inside a workgroup's rows writes into no other token's and nothing behind the last one"""
+    rng = np.random.default_rng(n + k + m)
+    stride, kc = -(-k // 256) * 64, n // 4 * 4
+    cs = -(-kc // 256) * 64
+    hd = hip.weights_upload_qk256(rng.integers(0, 256, n * stride, dtype=np.uint8), n, k, stride)
+    pair = [hip.weights_upload_qk256(rng.integers(0, 256, n * cs, dtype=np.uint8), n, kc, cs) for _ in range(2)]
+    hg = hip.weights_concat(pair, interleave16=True)
+    xh = torch_.from_numpy(rng.normal(0, 1.5, (m, k)).astype(np.float16)).cuda()
+    xf, res = torch_.from_numpy(rng.normal(0, 1, (m, kc)).astype(np.float32)).cuda(), torch_.from_numpy(rng.normal(0, 1, (m, n)).astype(np.float32)).cuda()
+    gd = torch_.from_numpy((rng.uniform(0.5, 1.5, kc) / 80).astype(np.float32)).cuda()
+    wsb = hip.matmul_workspace_bytes(m, max(k, kc), 2)
+    ws = torch_.empty(wsb, dtype=torch_.uint8, device="cuda")
+    outs = []
+    for fl in (INT8_DIGITS, FP6_DIGITS):
+        yx, yf, yh = (torch_.full((m + 8, n), float("nan"), dtype=t, device="cuda") for t in (torch_.float32, torch_.float32, torch_.float16))
+        tiles = []
+        hip.matmul_fused_dev(hd, xh, yx, m, ws, wsb, residual=res, flags=2 | fl, digits=2)
+        tiles.append(hip.matmul_last_tile())
+        hip.matmul_fused_dev(hg, xf, yf, m, ws, wsb, ln_gamma=gd, ln_eps=1e-5, flags=SILU_MUL | fl, digits=2)
+        hip.matmul_fused_dev(hg, xf, yh, m, ws, wsb, ln_gamma=gd, ln_eps=1e-5, flags=SILU_MUL | 4 | fl, digits=2)
+        tiles.append(hip.matmul_last_tile())
+        torch_.cuda.synchronize()
+        for h, t in ((hd, tiles[0]), (hg, tiles[1])):
+            few = fl == INT8_DIGITS and hip.matmul_takes_few_rows(h, m, fl | (SILU_MUL if h == hg else 0), 2)
+            assert t["scale_mode"] == (0 if fl == INT8_DIGITS else 6) and (t["waves"] == 8) == few, t
+        if fl == INT8_DIGITS:
+            assert tiles[0]["waves"] == waves
+        assert all(bool(y[m:].isnan().all()) for y in (yx, yf, yh))
+        outs.append([y[:m].cpu().numpy() for y in (yx, yf, yh)])
+    for a, b in zip(*outs):
+        assert np.isfinite(a.astype(np.float32)).all() and np.array_equal(a, b)
+    assert np.array_equal(outs[0][1].astype(np.float16), outs[0][2])
+    for h in (hg, hd, *pair):
+        hip.weights_free(h)
+
+
 FP6_EXPAND = 32  # BITNET_HIP_FUSE_FP6_EXPAND
 
 
