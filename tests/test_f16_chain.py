@@ -120,7 +120,7 @@ def test_f16_chain_plain_residual_and_handover(hip, oracle, torch_, fmt, rows, c
 @pytest.mark.parametrize("fmt", ["qk256", "i2s"])
 @pytest.mark.parametrize("m", [17, 511, 800, 1025])
 def test_f16_chain_half_slab_waves(hip, torch_, fmt, m):
-    """2560 rows around the lines of the short-prompt forms: 32-row waves of 16 and 32 tokens (511: 320 workgroups of 256 rows, 800: 260), 64-row waves (1025: 340)"""
+    """2560 rows around the lines of the short-prompt forms: 32-row waves of 16 tokens (17; 511: 320 workgroups if they had 256 rows) and of 32 (800: 260), 64-row waves (1025: 340)"""
     rows, cols, mp = 2560, 512, -(-m // 64) * 64
     rng = np.random.default_rng(m)
     h, w = make_matrix(hip, rng, fmt, rows, cols)
@@ -128,7 +128,7 @@ def test_f16_chain_half_slab_waves(hip, torch_, fmt, m):
     res = rng.normal(0, 1, (m, rows)).astype(np.float32)
     y, st = torch_.from_numpy(res).cuda(), torch_.full((rows // 64, mp, 2), float("nan"), device="cuda")
     hip.matmul_f16_dev(h, torch_.from_numpy(x).cuda(), m, y=y, residual=y, stats_out=st)
-    assert (hip.matmul_last_workgroup_rows(), hip.matmul_last_tile()["wave_tokens"]) == {17: (128, 16), 511: (128, 32), 800: (128, 32), 1025: (256, 32)}[m]
+    assert (hip.matmul_last_workgroup_rows(), hip.matmul_last_tile()["wave_tokens"]) == {17: (128, 16), 511: (128, 16), 800: (128, 32), 1025: (256, 32)}[m]
     torch_.cuda.synchronize()
     got, xd = y.cpu().numpy().astype(np.float64), x[:m].astype(np.float64)
     assert np.max(np.abs(got - (res + xd @ w.T)) / (np.abs(xd) @ np.abs(w).T + np.abs(res) + 1e-6)) <= 2e-6  # f16 inputs: accumulation order alone
