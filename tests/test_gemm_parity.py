@@ -385,6 +385,29 @@ def test_few_rows_only_where_they_are_faster(hip, torch_, rows, cols, m, few):
         hip.weights_free(i)
 
 
+# the wide int8 tiles where few rows no longer take them: rows, columns and tokens that end inside a tile, behind 192 rows
+@pytest.mark.parametrize("rows,cols,m", [(1000, 1100, 257), (48, 512, 200), (320, 6912, 230), (33, 260, 193), (2570, 2564, 1030)])
+def test_wide_int8_tiles_on_ragged_shapes(hip, oracle, torch_, rows, cols, m):
+    """k_gemm_mfma<2> against k_gemm_fp6 on the same integers, bit for bit, and against the oracle on sampled rows"""
+    rng = np.random.default_rng(rows * 5 + cols + m)
+    stride = -(-cols // 256) * 64
+    qs = rng.integers(0, 256, rows * stride, dtype=np.uint8)
+    x = (rng.normal(0.1, 1.0, (m, cols)) * np.exp(rng.uniform(-3, 3, (m, 1)))).astype(np.float32)
+    gd = torch_.from_numpy((rng.uniform(0.5, 1.5, cols) / 80).astype(np.float32)).cuda()
+    rd = torch_.from_numpy(rng.normal(0, 1, (m, rows)).astype(np.float32)).cuda()
+    h = hip.weights_upload_qk256(qs, rows, cols, stride)
+    for kw in (dict(ln_gamma=gd, ln_eps=1e-5), dict(residual=rd), {}):
+        wide = run_gemm(hip, torch_, h, x, rows, 2, flags=INT8_DIGITS, **kw)
+        t = hip.matmul_last_tile()
+        assert t["scale_mode"] == 0 and t["waves"] == 4 and t["digits"] == 2, t
+        six = run_gemm(hip, torch_, h, x, rows, 2, flags=FP6_DIGITS, **kw)
+        assert hip.matmul_last_tile()["scale_mode"] == 6
+        assert not np.isnan(wide).any() and np.array_equal(wide, six), (sorted(kw), float(np.abs(wide - six).max()))
+    for i in np.unique(np.r_[0, m - 1, rng.integers(0, m, 4)]):
+        assert cosine(wide[i], oracle.gemv_qk256(qs, x[i], rows, cols, stride)) >= 0.99999, int(i)
+    hip.weights_free(h)
+
+
 # rows handed over as f16, in and out, as the short and the longer prompts' forward does: the form for few rows (eight waves) and the wide int8 tiles (four)
 @pytest.mark.parametrize("n,k,m,waves", [(512, 1024, 1, 8), (512, 1024, 70, 8), (48, 1100, 33, 8), (2560, 6912, 19, 8), (2560, 6912, 177, 8), (512, 1024, 200, 4), (48, 1100, 215, 4),
                                          (2560, 6912, 193, 4)])

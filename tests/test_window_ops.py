@@ -124,6 +124,52 @@ def test_products_weighed_by_the_tokens(hip, pkg, n, f32):
         assert u.rms_error(u.host(y), want[i]) < F32_TOL
 
 
+# the form for few rows in each of its tiles, whole ones and ends inside them: the token table's factor, and everything an output can be put through on its way
+FEW = [(70, 90, 512, (16, 16)), (160, 256, 576, (16, 16)), (300, 250, 640, (32, 32)), (277, 416, 512, (32, 32)), (2000, 250, 1536, (32, 64)), (300, 1100, 1536, (32, 64))]
+
+
+@pytest.mark.parametrize("m,n,k,tile", FEW)
+def test_few_rows_weighed_by_the_tokens(hip, pkg, m, n, k, tile):
+    g = rng(m, n, k, 2)
+    vocab, first = 30, 7
+    x, w = u.rounded(g.standard_normal((m, k))), u.rounded(2.0 * g.standard_normal((n, k)) / np.sqrt(k))
+    table, tokens = u.rounded(g.standard_normal((vocab, 2 * n))), g.integers(0, vocab, first + m).astype(np.int32)
+    tokens[first + 1], tokens[first + m - 1] = vocab + 5, -3  # (the last row of the table and its first)
+    ld, ldc = u.up_to(2 * n, 64), u.up_to(n + 1, 64)
+    td, tok, pos, b = u.dev_bf16(u.padded(table, ld)), u.dev(tokens), pos_dev(first), g.standard_normal(n).astype(np.float32)
+    z = x.astype(f64) @ w.T.astype(f64) + b
+    for act, fn in ((pkg.ACT_GELU_TANH, so.gelu_tanh), (pkg.ACT_SIGMOID, so.sigmoid)):
+        out = u.zeros_bf16(m, ldc)
+        out[:, n:] = 3
+        hip.dense_matmul_dev(u.dev_bf16(x), k, False, u.dev_bf16(w), k, m, n, k, out, ldc, False, bias=u.dev_f32(b), act0=act,
+                             more=pkg.Epilogue(mul=ptr(td, 2 * n), ld_mul=ld, mul_rows=vocab, mul_tokens=ptr(tok), mul_at=ptr(pos)))
+        assert hip.dense_matmul_last_tile() == (*tile, 8, 8)
+        want = fn(z) * table[np.clip(tokens[first:], 0, vocab - 1), n:2 * n]
+        assert u.rms_error(u.host(out)[:, :n], want) < 4e-3 and bool((out[:, n:] == 3).all())
+
+
+@pytest.mark.parametrize("m,n,k,tile", FEW)
+@pytest.mark.parametrize("form", ["f32", "bf16", "gated"])
+def test_few_rows_activations(hip, pkg, m, n, k, tile, form):
+    """alone, and with another one from a column inside a lane's four on"""
+    g = rng(m, n, k, 3)
+    gated, f32 = form == "gated", form == "f32"
+    x, w, b = u.rounded(g.standard_normal((m, k))), u.rounded(3.0 * g.standard_normal((n, k)) / np.sqrt(k)), g.standard_normal(n).astype(np.float32)
+    xd, wd, bd, z = u.dev_bf16(x), u.dev_bf16(w), u.dev_f32(b), x.astype(f64) @ w.T.astype(f64) + b
+    acts = [(pkg.ACT_GELU_TANH, so.gelu_tanh), (pkg.ACT_SIGMOID, so.sigmoid), (pkg.ACT_RELU2, lambda v: np.maximum(v, 0) ** 2), (pkg.ACT_SILU, so.silu)]
+    acts += [] if gated else [(pkg.ACT_XIELU, xielu)]
+    more = None if gated else pkg.Epilogue(act_a=XIELU[0], act_b=XIELU[1])
+    for i, (act, fn) in enumerate(acts):
+        for split in (0,) if gated else (0, n // 3 + 1):
+            out = (u.zeros_f32 if f32 else u.zeros_bf16)(m, n + 3)
+            hip.dense_matmul_dev(xd, k, False, wd, k, m, n, k, out, n + 3, f32, bias=bd, act0=act | (pkg.ACT_GATED if gated else 0), act1=acts[i - 1][0] if split else 0, act_split=split, more=more)
+            assert hip.dense_matmul_last_tile() == (*tile, 8, 8)
+            want = fn(z[:, ::2]) * z[:, 1::2] if gated else np.where(np.arange(n) < (split or n), fn(z), acts[i - 1][1](z))
+            got = u.host(out)
+            assert u.rms_error(got[:, :want.shape[1]], want) < (F32_TOL if f32 else 4e-3), (act, split)
+            assert not got[:, want.shape[1]:].any()
+
+
 # ---- rows and vectors of the residual stream -----------------------------------------------------------------------------
 @pytest.mark.parametrize("n", [80, 90, 1001, 2560, 4096, 5000])
 def test_gemv_adds_a_gated_sublayer(hip, pkg, n):
