@@ -986,7 +986,8 @@ __device__ __forceinline__ float activate_pair(float v, int act) {
 // through has always taken expf and a division, and its tile must not decide.
 __device__ __forceinline__ bool gelu_is_fast(const GemmArgsD &p) { return p.act_split >= p.n && p.n % 128 == 0; }
 __device__ __forceinline__ float activate_column(float v, int act, bool fast_gelu, const Epilogue &e) {
-    return act == BITNET_HIP_ACT_SILU ? silu_fast(v) : act == BITNET_HIP_ACT_SIGMOID ? sigmoid_fast(v) : act == BITNET_HIP_ACT_XIELU ? xielu_fast(v, e)
+    const float sg = sigmoid_fast(v), r = fmaxf(v, 0.0f);
+    return act == BITNET_HIP_ACT_SILU ? v * sg : act == BITNET_HIP_ACT_SIGMOID ? sg : act == BITNET_HIP_ACT_RELU2 ? r * r : act == BITNET_HIP_ACT_XIELU ? xielu_fast(v, e)
          : act == BITNET_HIP_ACT_GELU_TANH && fast_gelu ? gelu_fast(v) : activate(v, act);
 }
 
