@@ -2359,14 +2359,18 @@ bool gemm_takes_fp6(const Weights &w, const GemvFusion &fu, int ndig) {
 // tiles cost by their K steps, one chain however few rows there are (0.92 us per 256 columns), until their row blocks fill the chip.  us per launch, quantiser included, this / the
 // wide form (the faster of int8 and fp6): 2560 x 2560 rows x columns, 192 tokens 15.7 / 17.2, 2560 x 6912, 192 27 / 33, 3840 x 2560, 128 14.9 / 16.7, 160 16.6 / 17.2, 192 18.7 / 17.1,
 // 4096 x 4096, 128 20.2 / 22.0, 192 25.9 / 22.5; pairs of 13824 x 2560, 64 16.1 / 19.8, 100 22.0 / 19.9, 160 26.6 / 27.5, 192 30.2 / 27.3, of 28672 x 4096, 64 35 / 40, 128 57 / 40.
+// Inside a prompt the wide tiles cost more than alone: their fp4 image is twice the codes, from HBM, and their f32 rows go past the caches (192 tokens of 3840 rows: the attention's
+// preparation takes 8.45 us behind them and 7.1 behind this form's).  The line lies where whole prompts of bitnet-b1.58-2B-4T change sides: q|k|v of 176 and 192 tokens this form,
+// 48 and 40 us a prompt; gate and up of 112 and 128 tokens the wide one, 40 and 70 us, of 144 to 192 this one.
 bool gemm_takes_few(const Weights &w, const GemvFusion &fu, size_t m, int ndig) {
     if (!gemm_supported(w) || ndig != 2 || w.scaled || gemm_takes_fp6(w, fu, ndig)) return false;
     if (!fu.int8_form && gemm_f16a_mode() && lut_fits_f16w(w.lut) && w.cols % 256 == 0) return false;
     // (a pair of gate and up tiles wants them both in the matrix; measured up to 192 rows)
     if (m > 192 || (fu.silu_mul && w.rows % 32 != 0)) return false;
     const double blocks = (double)div_ceil(w.cols, 256), workgroups = (double)div_ceil(div_ceil(w.rows, 16), fu.silu_mul ? 2 : 1) * div_ceil(m, 16);
-    const double row_blocks = (double)div_ceil(w.rows, 256) * div_ceil(m, 128), rounds = std::max(1.0, 0.55 + 0.016 * std::min(row_blocks, 180.0));
-    return workgroups * (0.2 + 0.35 * blocks) + (double)(w.rows * w.cols / 4) / 4800 <= 920 * blocks * rounds;
+    const double row_blocks = (double)div_ceil(w.rows, 256) * div_ceil(m, 128), rounds = std::max(1.0, 0.53 + 0.0164 * std::min(row_blocks, 180.0));
+    const double way_back = fu.silu_mul ? 0.0 : 0.6e-3 * (double)(4 * 16 * div_ceil(m, 16) * w.rows);
+    return workgroups * (0.2 + 0.35 * blocks) + (double)(w.rows * w.cols / 4) / 4800 <= 920 * blocks * rounds + way_back;
 }
 
 static hipError_t launch_gemm_fp6(const Weights &w, const QuantArgs &q, const GemmArgs &a, hipStream_t stream) {

@@ -364,9 +364,9 @@ def test_few_rows_are_the_wide_tiles_product_bit_for_bit(hip, torch_, rows, cols
 
 
 # either side of the lines between k_gemm_few and the wide tiles: a narrow matrix, a wide one in one and in two rounds, a long K, 192 rows
-@pytest.mark.parametrize("rows,cols,m,few", [(3840, 2560, 128, True), (3840, 2560, 192, False), (2560, 6912, 192, True), (2560, 6912, 193, False), (4096, 4096, 144, True),
-                                             (4096, 4096, 176, False), (-13824, 2560, 80, True), (-13824, 2560, 112, False), (-13824, 2560, 144, True),
-                                             (-13824, 2560, 192, False)])
+@pytest.mark.parametrize("rows,cols,m,few", [(3840, 2560, 128, True), (3840, 2560, 192, True), (2560, 6912, 192, True), (2560, 6912, 193, False), (4096, 4096, 144, True),
+                                             (4096, 4096, 192, False), (-13824, 2560, 80, True), (-13824, 2560, 112, False), (-13824, 2560, 128, False),
+                                             (-13824, 2560, 144, True), (-13824, 2560, 192, True), (-28672, 4096, 128, False), (4608, 3072, 192, False)])
 def test_few_rows_only_where_they_are_faster(hip, torch_, rows, cols, m, few):
     """rows < 0: pairs of gate and up tiles.  The query, the launch and the outputs agree: the wide int8 tiles' and the fp6 digits' bit for bit"""
     paired, rows = rows < 0, abs(rows)
