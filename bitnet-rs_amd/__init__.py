@@ -448,7 +448,7 @@ class HipLib:
         return self.c.bitnet_hip_matmul_takes_few_rows(h, m, flags, digits) == 1
 
     def matmul_last_wave_rows(self) -> int:
-        """Output rows per slab of LayerNorm partials of this thread's last tiled matmul: 64, or 80 (320-row workgroups)."""
+        """Output rows per wave of this thread's last tiled matmul, or per slab of LayerNorm partials where two waves share one: 64, 80 (320-row workgroups), 128 (fp6 2 x 2 waves), 16 or 32 (few rows)."""
         return int(self.c.bitnet_hip_matmul_last_wave_rows())
 
     def matmul_last_workgroup_rows(self) -> int:

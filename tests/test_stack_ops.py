@@ -135,7 +135,7 @@ def test_matmul_activations_are_those_of_the_call(hip, pkg, n, split, form):
         assert got[0].any() and np.array_equal(*got), (act, np.abs(got[0] - got[1]).max())
 
 
-# every tile of the matmul where the launcher takes it (a whole number of them and ends inside one), and outputs that start on no sixteen bytes
+# whole numbers of the matmul's tiles and ends inside one, two activations, and outputs that start on no sixteen bytes; test_matmul_by_tile says which tile takes a shape
 @pytest.mark.parametrize("m,n", [(4096, 4096), (4000, 4080), (4096, 3072), (3900, 3060), (2048, 3072), (2040, 4056), (2048, 2560), (1537, 2570), (1500, 2568), (700, 2552), (1531, 1528)])
 @pytest.mark.parametrize("form", ["f32", "bf16", "gated", "unaligned"])
 def test_matmul_tiles(hip, pkg, m, n, form):
