@@ -34,6 +34,7 @@ void free_weights(Weights *w) {
     if (w->scales) (void)hipFree(w->scales);
     if (w->tiles) (void)hipFree(w->tiles);
     if (w->tiles4) (void)hipFree(w->tiles4);
+    if (w->tiles4_pairs) (void)hipFree(w->tiles4_pairs);
     if (w->scale_tiles) (void)hipFree(w->scale_tiles);
     if (w->scale_tiles_h) (void)hipFree(w->scale_tiles_h);
     if (w->ln_g) (void)hipFree(w->ln_g);
@@ -504,6 +505,7 @@ int bitnet_hip_matmul_f16_dev(bitnet_hip_weights_t h, const void *xh_dev, size_t
     }
     if (io.silu_mul && (!w->paired || residual_dev))
         return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "FUSE_SILU_MUL needs a handle from weights_concat(..., interleave16=1) and no residual");
+    io.image = want_pair_image(*w, (hipStream_t)stream);
     hipError_t e = launch_gemm_f16_chain(*w, io, m, (hipStream_t)stream);
     if (e == hipErrorInvalidValue && io.qb_out)
         return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "FUSE_YH_QB32: this launch does not run 64-token tiles (too few rows for the QB32 hand-over)");

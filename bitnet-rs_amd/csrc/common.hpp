@@ -103,6 +103,7 @@ struct Weights {
     uint8_t *tiles = nullptr;
     // resident fp4 image for the prompt matmul's fp6 x fp4 form (kernels_gemm.hip k_retile_fp4 / ensure_fp4_image): optional, 4 bits per weight
     uint8_t *tiles4 = nullptr;
+    uint8_t *tiles4_pairs = nullptr;  // ... and the f16 chain's (k_retile_pairs / want_pair_image)
     float *scale_tiles = nullptr;  // 32-block scales in tile order (kernels_mfma.hip k_retile_scales)
     // Every scale is exactly an f16 value (BitNet32-F16 files store them so): the streaming layout
     // keeps them as f16 (2 bytes per 32 weights instead of 4) -- same numbers, fewer bytes.
@@ -203,6 +204,7 @@ bool gemm_fp6_supported(const Weights &w);
 bool gemm_fp4_resident_enabled();                            // BITNET_HIP_FP4_RESIDENT != 0 (default on)
 hipError_t ensure_fp4_image(Weights &w, hipStream_t stream);  // builds Weights::tiles4 once (under the handle's mutex)
 void drop_fp4_image(Weights &w);
+const uint8_t *want_pair_image(Weights &w, hipStream_t stream);  // Weights::tiles4_pairs, built on first use; null where that is not possible
 bool gemm_takes_few(const Weights &w, const GemvFusion &fu, size_t m, int ndig);  // ... k_gemm_few?
 bool gemm_takes_fp6(const Weights &w, const GemvFusion &fu, int ndig);  // would launch_gemm_mfma run k_gemm_fp6 for this call?  // unscaled, code map in -2 .. 2: the fp6 x fp4 form of the 2-digit product (k_gemm_fp6)
 bool gemm_needs_row_major_scales(const Weights &w);  // 256-block scales and non-f16 32-block scales: the others read the scale tiles
@@ -223,6 +225,7 @@ struct GemmF16Io {
     const float *gamma_out = nullptr; // [rows]: yh = f16(gamma_out * y)
     float *stats_out = nullptr;       // float2 [rows / 64][m_pad]
     void *qb_out = nullptr;           // QB32 buffer (qb32_bytes(m, rows)) receiving gamma_out * y (launch_gemm_f16_chain only; not with silu_mul)
+    const uint8_t *image = nullptr;   // want_pair_image's (launch_gemm_f16_chain only)
 };
 // QB32 activation rows (kernels_gemm.hip): digit records [m_pad][cols / 256][576] then one exponent byte per (token, 32 columns); m_pad = m up to 64
 size_t qb32_bytes(size_t m, size_t cols);

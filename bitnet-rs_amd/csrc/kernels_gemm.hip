@@ -72,7 +72,7 @@ struct GemmArgs {
     // records [m_pad][nblk][592]: 576 bytes of digits (the fp6 form's layout) + the block's eight E8M0-ready exponent bytes (one per 32-column unit) + 8 pad ----
     uint8_t *qb_out = nullptr;         // producer: records of the OUTPUT rows [m_pad][qb_nblk_out][592] (gamma_out * y, the next matmul's K = rows)
     int qb_nblk_out = 0;
-    const uint8_t *tiles4 = nullptr;  // k_gemm_fp6<.., RES = 1>: the resident fp4 image [n_tiles][nblk][m 2][64][16] (k_retile_fp4)
+    const uint8_t *tiles4 = nullptr;  // k_gemm_fp6<.., RES = 1>: the resident fp4 image [n_tiles][nblk][m 2][64][16] (k_retile_fp4); k_gemm_f16a / f16h: k_retile_pairs'
     int bx_off = 0;  // first row block of this launch (the wide gate|up launch is split in two: k_gemm_f16h on the first blocks, k_gemm_f16a on the rest)
     int wgroup = 0;  // > 0: an XCD walks `wgroup` weight row blocks x all token tiles before the next group (gridDim.x % wgroup == 0): gemm_weight_group
 };
@@ -995,6 +995,19 @@ __device__ __forceinline__ gh8 expand8_f16(uint32_t w, int h, uint32_t lut_hi, g
     return (gh8){w2[0][0], w2[0][1], w2[1][0], w2[1][1], w2[2][0], w2[2][1], w2[3][0], w2[3][1]};
 }
 
+// The same eight values from eight fp4 codes (the image of k_retile_pairs): v_cvt_scalef32_pk_f16_fp4 makes two of a byte, exactly (-2 .. 2).  4 VALU per 8 weights, 8 with a block
+// scale, where the codes of two bits take 12 and 16 -- and VALU of one wave hardly hides behind another's MFMAs: eight weights and four MFMAs 42 and 51 ns per SIMD with two waves
+// from the codes, 34 and 36 from the image, 31 for the MFMAs alone.
+template <bool SCALED>
+__device__ __forceinline__ gh8 expand8_pairs(uint32_t w, gh2 s2) {
+    gh2 v[4] = {__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 0), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 1), __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 2),
+                __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 1.0f, 3)};
+    if (SCALED)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[q] *= s2;
+    return (gh8){v[0][0], v[0][1], v[1][0], v[1][1], v[2][0], v[2][1], v[3][0], v[3][1]};
+}
+
 // ================================================================================================================================
 // QB32: block-scaled fixed-point activation rows for the fp6 x fp4 prompt matmul, written by the PRODUCER of the activations (round 5).
 // The row quantiser of the digit forms needs the row maximum -- a value no producing workgroup has -- so it stayed a launch of its own
@@ -1265,10 +1278,13 @@ __device__ __forceinline__ void f16_chain_epilogue(const GemmArgs &p, gv4f (&acc
 
 // RT = row tiles per wave: 4 (256-row workgroups), 2 (128-row workgroups for short prompts: launch_gemm_f16_chain says when), or 5 (320-row workgroups, chain form only): a 2560-row matrix x 4096 tokens is then
 // 8 x 64 = 512 workgroups -- exactly one round of the 512 slots (two 4-wave workgroups per CU) instead of 640 in two rounds.
+// FMT + 2: the weights from the resident image (GemmArgs::tiles4, k_retile_pairs): sixteen bytes per lane, row tile and half K step.
 template <int FMT, int TTW, int EPI = 0, int RT = 4>
 __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_hi) {
     static_assert(RT == 4 || EPI >= 1, "the 5-tile wave exists for the chain's epilogue only");  // EPI 2 = chain epilogue + QB32 hand-over
+    constexpr bool SC = FMT & 1, RES = FMT & 2;
     constexpr int WG_TOK = TTW * 16, NB = WG_TOK * 32 / 256, ROWB = 512, kBuf = WG_TOK * ROWB;
+    constexpr int NP = RES ? 2 : 1;  // pieces of a row tile's weights per K step
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c = lane & 15, g = lane >> 4, rw = wave;
@@ -1295,8 +1311,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_h
     for (int rt = 0; rt < RT; ++rt) {
         int t = bx * (4 * RT) + rw * RT + rt;
         t = t < n_tiles ? t : n_tiles - 1;
-        wptr[rt] = p.tiles + ((size_t)t * p.nblk * 64 + lane) * 16;
-        sptr[rt] = FMT == 1 ? reinterpret_cast<const uint32_t *>(p.stiles_h) + (size_t)t * p.nblk * 64 + g * 16 + c : nullptr;
+        wptr[rt] = (RES ? p.tiles4 : p.tiles) + ((size_t)t * p.nblk * 64 * NP + lane) * 16;
+        sptr[rt] = SC ? reinterpret_cast<const uint32_t *>(p.stiles_h) + (size_t)t * p.nblk * 64 + g * 16 + c : nullptr;
     }
     const _Float16 *planes = reinterpret_cast<const _Float16 *>(p.planes);
     const uint8_t *bsrc[NB];
@@ -1318,11 +1334,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_h
     ChainLnStats<WG_TOK, 4> lnst;
     const bool ln_in = EPI && p.stats_in;
     if (ln_in) lnst.issue(p, by, tid);
-    gv4u wn[RT], bn[NB];
+    gv4u wn[NP][RT], bn[NB];
     uint32_t sn[RT];
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) wn[rt] = *reinterpret_cast<const gv4u *>(wptr[rt]), sn[rt] = 0;
-    if (FMT == 1) {
+    for (int q = 0; q < NP; ++q)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) wn[q][rt] = *reinterpret_cast<const gv4u *>(wptr[rt] + 1024 * q), sn[rt] = 0;
+    if (SC) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) sn[rt] = sptr[rt][0];
     }
@@ -1373,13 +1391,20 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_h
         F16A_PHASE(0);
         gv4u wc[RT];
         uint32_t sc[RT];
+        const int n1 = blk + 1 < p.nblk ? blk + 1 : p.nblk - 1;
+        auto next_piece = [&](int q) {
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) wc[rt] = wn[rt], sc[rt] = sn[rt];
+            for (int rt = 0; rt < RT; ++rt) {
+                wc[rt] = wn[q][rt];
+                wn[q][rt] = *reinterpret_cast<const gv4u *>(wptr[rt] + ((size_t)n1 * NP + q) * 1024);
+            }
+        };
+        if (!RES) next_piece(0);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) sc[rt] = sn[rt];
         {
-            const int n1 = blk + 1 < p.nblk ? blk + 1 : p.nblk - 1, n2 = blk + 2 < p.nblk ? blk + 2 : p.nblk - 1;
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) wn[rt] = *reinterpret_cast<const gv4u *>(wptr[rt] + (size_t)n1 * 1024);
-            if (FMT == 1) {
+            const int n2 = blk + 2 < p.nblk ? blk + 2 : p.nblk - 1;
+            if (SC) {
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) sn[rt] = sptr[rt][(size_t)n1 * 64];
             }
@@ -1392,15 +1417,15 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_h
 #endif
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
+            if (RES && (m & 1) == 0) next_piece(m >> 1);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 gh8 a[RT];
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) {
-                    const uint32_t wd = m == 0 ? wc[rt].x : m == 1 ? wc[rt].y : m == 2 ? wc[rt].z : wc[rt].w;
                     // (s, s) of this lane's 32-block 2 g + (m >> 1): low / high half of its scale dword
                     const gh2 s2 = __builtin_bit_cast(gh2, __builtin_amdgcn_perm(0u, sc[rt], (m >> 1) ? 0x03020302u : 0x01000100u));
-                    a[rt] = expand8_f16<FMT>(wd, h, lut_hi, s2);
+                    a[rt] = RES ? expand8_pairs<SC>(wc[rt][2 * (m & 1) + h], s2) : expand8_f16<SC>(wc[rt][m], h, lut_hi, s2);
                 }
 #pragma unroll
                 for (int ct = 0; ct < TTW; ++ct) {
@@ -1472,6 +1497,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t gbuf_rsrc(const void *base) {
 
 template <int FMT>
 __global__ __launch_bounds__(256, 2) void k_gemm_f16h(GemmArgs p, uint32_t lut_hi) {
+    constexpr bool SC = FMT & 1, RES = FMT & 2;
     constexpr int RT = 4, TTW = 8, WG_TOK = TTW * 16, ROWB = 256, kBuf = WG_TOK * ROWB;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (scalar: the tile bases stay in SGPRs)
@@ -1495,13 +1521,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16h(GemmArgs p, uint32_t lut_h
     bx += p.bx_off;
     // wave-uniform bases (SGPR pairs) + 32-bit lane offsets: 128 accumulators leave no room for 64-bit per-lane pointers -- nor for a register-staged
     // activation tile (32 registers: hipcc spilled 144-228 bytes), so the tile goes global -> LDS by LDS-DMA, one half-K step ahead of its MFMAs
-    const __amdgpu_buffer_rsrc_t rs_w = gbuf_rsrc(p.tiles), rs_s = gbuf_rsrc(FMT == 1 ? (const void *)p.stiles_h : (const void *)p.tiles);
+    const __amdgpu_buffer_rsrc_t rs_w = gbuf_rsrc(RES ? p.tiles4 : p.tiles), rs_s = gbuf_rsrc(SC ? (const void *)p.stiles_h : (const void *)p.tiles);
     int wptr[RT], sptr[RT];  // scalar byte offsets of this wave's row tiles in the code / scale tile arrays
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         int t = bx * (4 * RT) + rw * RT + rt;
         t = t < n_tiles ? t : n_tiles - 1;
-        wptr[rt] = t * p.nblk * 1024;
+        wptr[rt] = t * p.nblk * (RES ? 2048 : 1024);
         sptr[rt] = t * p.nblk * 256;
     }
     const uint32_t woff = (uint32_t)lane * 16u, soff = (uint32_t)(g * 16 + c) * 4u;
@@ -1533,7 +1559,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16h(GemmArgs p, uint32_t lut_h
     uint32_t sn[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) wn[rt] = __builtin_bit_cast(gv4u, __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff, wptr[rt], 0)), sn[rt] = 0;
-    if (FMT == 1) {
+    if (SC) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) sn[rt] = __builtin_amdgcn_raw_buffer_load_b32(rs_s, soff, sptr[rt], 0);
     }
@@ -1551,16 +1577,22 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16h(GemmArgs p, uint32_t lut_h
 #pragma unroll
         for (int ct = 0; ct < TTW; ++ct) acc[rt][ct] = (gv4f){0.f, 0.f, 0.f, 0.f};
     for (int blk = 0; blk < p.nblk; ++blk) {
-        // this block's weights / scales become current; the next block's are requested
+        // this block's weights / scales become current; the next block's are requested (RES: the next half's)
         gv4u wc[RT];
         uint32_t sc[RT];
+        auto next_weights = [&](int at) {
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) wc[rt] = wn[rt], sc[rt] = sn[rt];
+            for (int rt = 0; rt < RT; ++rt) {
+                wc[rt] = wn[rt];
+                wn[rt] = __builtin_bit_cast(gv4u, __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff, wptr[rt] + at * 1024, 0));
+            }
+        };
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) sc[rt] = sn[rt];
         {
             const int n1 = blk + 1 < p.nblk ? blk + 1 : p.nblk - 1;
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt) wn[rt] = __builtin_bit_cast(gv4u, __builtin_amdgcn_raw_buffer_load_b128(rs_w, woff, wptr[rt] + n1 * 1024, 0));
-            if (FMT == 1) {
+            if (!RES) next_weights(n1);
+            if (SC) {
 #pragma unroll
                 for (int rt = 0; rt < RT; ++rt) sn[rt] = __builtin_amdgcn_raw_buffer_load_b32(rs_s, soff, sptr[rt] + n1 * 256, 0);
             }
@@ -1569,6 +1601,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16h(GemmArgs p, uint32_t lut_h
         for (int hs = 0; hs < 2; ++hs) {  // (compile-time after unrolling: the half tile of step s = 2 blk + hs sits in buffer hs)
             const int s = 2 * blk + hs;
             const uint8_t *bcur = lds + hs * kBuf;
+            if (RES) next_weights(s + 1 < n_steps ? s + 1 : s);
             if (s + 1 < n_steps) stage(s + 1, hs ^ 1);  // (every wave is past the barrier that ended step s - 1: nobody reads that buffer)
 #pragma unroll
             for (int mm = 0; mm < 2; ++mm) {
@@ -1578,9 +1611,8 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16h(GemmArgs p, uint32_t lut_h
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt) {
                         // dword m = 2 hs + mm of the lane's 16 bytes; (s, s) of its 32-block 2 g + hs: low / high half of the scale dword
-                        const uint32_t wd = hs == 0 ? (mm == 0 ? wc[rt].x : wc[rt].y) : (mm == 0 ? wc[rt].z : wc[rt].w);
                         const gh2 s2v = __builtin_bit_cast(gh2, __builtin_amdgcn_perm(0u, sc[rt], hs ? 0x03020302u : 0x01000100u));
-                        a[rt] = expand8_f16<FMT>(wd, h, lut_hi, s2v);
+                        a[rt] = RES ? expand8_pairs<SC>(wc[rt][2 * mm + h], s2v) : expand8_f16<SC>(wc[rt][2 * hs + mm], h, lut_hi, s2v);
                     }
 #pragma unroll
                     for (int ct = 0; ct < TTW; ++ct) {
@@ -1637,6 +1669,24 @@ __global__ void k_retile_fp4(const uint8_t *__restrict__ tiles, uint8_t *__restr
     const size_t tb = i >> 6, lane = i & 63;
     *reinterpret_cast<v4i *>(tiles4 + ((tb * 2 + 0) * 64 + lane) * 16) = (v4i){e[0], e[1], e[2], e[3]};
     *reinterpret_cast<v4i *>(tiles4 + ((tb * 2 + 1) * 64 + lane) * 16) = (v4i){e[4], e[5], e[6], e[7]};
+}
+
+// The image that k_gemm_f16a / k_gemm_f16h read: the same nibbles in the order of those kernels' operands, [row tile][256-block][half 2][lane 64][16 B]; dword 2 m + h of a lane
+// (half m >> 1) holds the codes of its columns 64 g + 16 m + 8 h .. + 7 in turn.
+__global__ void k_retile_pairs(const uint8_t *__restrict__ tiles, uint8_t *__restrict__ image, uint32_t lut4, size_t total16) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // one 16-byte lane segment of the streaming tiles each
+    if (i >= total16) return;
+    const gv4u w = *reinterpret_cast<const gv4u *>(tiles + i * 16);
+    gv4u o[2];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const uint32_t lo = __builtin_amdgcn_perm(0u, lut4, (w[u >> 1] >> (4 * (u & 1))) & 0x03030303u), hi = __builtin_amdgcn_perm(0u, lut4, (w[u >> 1] >> (4 * (u & 1) + 2)) & 0x03030303u);
+        auto packed = [](uint32_t b) { return (b & 0xfu) | (b >> 4 & 0xf0u) | (b >> 8 & 0xf00u) | (b >> 12 & 0xf000u); };  // four bytes' nibbles side by side
+        o[u >> 2][u & 3] = packed(lo) | packed(hi) << 16;
+    }
+    const size_t tb = i >> 6, lane = i & 63;
+    *reinterpret_cast<gv4u *>(image + ((tb * 2 + 0) * 64 + lane) * 16) = o[0];
+    *reinterpret_cast<gv4u *>(image + ((tb * 2 + 1) * 64 + lane) * 16) = o[1];
 }
 
 // RT = row tiles per wave: 4, or 5 (320-row workgroups: gemm_five_tiles; no silu * mul pairing with it).
@@ -2270,6 +2320,13 @@ static uint32_t lut_f16_hi(uint32_t lut) {
     return out;
 }
 
+// pick(FMT of k_gemm_f16a and k_gemm_f16h)
+template <class F>
+static auto f16_instance(bool scaled, bool image, F pick) {
+    return scaled ? (image ? pick(std::integral_constant<int, 3>()) : pick(std::integral_constant<int, 1>()))
+                  : image ? pick(std::integral_constant<int, 2>()) : pick(std::integral_constant<int, 0>());
+}
+
 // f16 activations on the f16 matrix cores (k_gemm_f16a): BitNet32-F16 at 2 digits; QK256 only on request (BITNET_HIP_GEMM_F16A=1:
 // measured 5-13 % slower than the int8 digit form there -- twice the expansion VALU for the same MFMA count)
 static hipError_t launch_gemm_f16(const Weights &w, const QuantArgs &q, const GemmArgs &a, hipStream_t stream) {
@@ -2324,23 +2381,46 @@ bool gemm_fp4_resident_enabled() {
     static const int mode = [] { const char *e = getenv("BITNET_HIP_FP4_RESIDENT"); return e ? atoi(e) : 1; }();
     return mode != 0;
 }
-hipError_t ensure_fp4_image(Weights &w, hipStream_t stream) {
-    if (!gemm_fp6_supported(w)) return hipErrorInvalidValue;
+static hipError_t build_image(Weights &w, uint8_t *Weights::*image, void (*retile)(const uint8_t *, uint8_t *, uint32_t, size_t), hipStream_t stream) {
     std::lock_guard<std::mutex> lk(*w.mu);
-    if (w.tiles4) return hipSuccess;
+    if (w.*image) return hipSuccess;
     const size_t n_tiles = div_ceil(w.rows, 16), nblk = div_ceil(w.cols, 256), total16 = n_tiles * nblk * 64;
     uint8_t *img = nullptr;
     hipError_t e = hipMalloc((void **)&img, total16 * 32);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_retile_fp4, dim3((unsigned)div_ceil(total16, 256)), dim3(256), 0, stream, w.tiles, img, lut_fp4(w.lut), total16);
+    hipLaunchKernelGGL(retile, dim3((unsigned)div_ceil(total16, 256)), dim3(256), 0, stream, w.tiles, img, lut_fp4(w.lut), total16);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(stream);  // other threads / streams may launch on the image the moment the lock is gone
     if (e != hipSuccess) {
         (void)hipFree(img);
         return e;
     }
-    w.tiles4 = img;
+    w.*image = img;
     return hipSuccess;
+}
+hipError_t ensure_fp4_image(Weights &w, hipStream_t stream) { return gemm_fp6_supported(w) ? build_image(w, &Weights::tiles4, k_retile_fp4, stream) : hipErrorInvalidValue; }
+// The image of the f16 chain's kernels (Weights::tiles4_pairs; it stays as long as the matrix does), or null where it cannot be had -- the stream captures, or memory is short --:
+// then the kernels expand the codes themselves, to the same values.  Another thread may be capturing: an allocation on behalf of this stream does not concern it.
+const uint8_t *want_pair_image(Weights &w, hipStream_t stream) {
+    if (!gemm_fp4_resident_enabled() || !gemm_f16_chain_supported(w)) return nullptr;
+    {
+        std::lock_guard<std::mutex> lk(*w.mu);
+        if (w.tiles4_pairs) return w.tiles4_pairs;
+    }
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone || hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    const hipError_t e = build_image(w, &Weights::tiles4_pairs, k_retile_pairs, stream);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    std::lock_guard<std::mutex> lk(*w.mu);
+    return w.tiles4_pairs;
 }
 void drop_fp4_image(Weights &w) {
     std::lock_guard<std::mutex> lk(*w.mu);
@@ -2460,7 +2540,8 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
 #endif
     size_t gx0 = w.rows / 256;
     const int ttw = gemm_token_tiles(gx0, m_pad, false, kGemmCUs);
-    const bool fmt1 = w.scaled;
+    const bool fmt1 = w.scaled, image = io.image != nullptr;
+    a.tiles4 = io.image;
     const bool rt5 = ttw == 4 && !io.silu_mul && gemm_five_tiles(w.rows, m_pad);
     // Short prompts: waves of 32 rows while the waves of 64 leave most CUs one workgroup.  A K step of such a workgroup is a serial chain (staging, expansion, LDS reads, MFMAs,
     // barrier: 3.2 us at 32 tokens, of which the units are busy a third), so two of half the rows on a CU take less than one.  BitNet32-F16 prompt of bitnet-b1.58-2B-4T, ms with
@@ -2469,13 +2550,16 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
     const bool rt2 = ttw < 4 && gx0 * (m_pad / (16 * ttw)) <= 320;
     if (rt5) gx0 = w.rows / 320;
     if (rt2) gx0 = w.rows / 128;
-    void (*fk)(GemmArgs, uint32_t) = rt5    ? (fmt1 ? k_gemm_f16a<1, 4, 1, 5> : k_gemm_f16a<0, 4, 1, 5>)
-                                     : rt2  ? (fmt1 ? (ttw == 2 ? k_gemm_f16a<1, 2, 1, 2> : k_gemm_f16a<1, 1, 1, 2>) : (ttw == 2 ? k_gemm_f16a<0, 2, 1, 2> : k_gemm_f16a<0, 1, 1, 2>))
-                                     : fmt1 ? (ttw == 4 ? k_gemm_f16a<1, 4, 1> : ttw == 2 ? k_gemm_f16a<1, 2, 1> : k_gemm_f16a<1, 1, 1>)
-                                            : (ttw == 4 ? k_gemm_f16a<0, 4, 1> : ttw == 2 ? k_gemm_f16a<0, 2, 1> : k_gemm_f16a<0, 1, 1>);
+    auto of_tile = [&](auto fmt) {
+        constexpr int F = decltype(fmt)::value;
+        return rt5   ? k_gemm_f16a<F, 4, 1, 5>
+               : rt2 ? (ttw == 2 ? k_gemm_f16a<F, 2, 1, 2> : k_gemm_f16a<F, 1, 1, 2>)
+                     : ttw == 4 ? k_gemm_f16a<F, 4, 1> : ttw == 2 ? k_gemm_f16a<F, 2, 1> : k_gemm_f16a<F, 1, 1>;
+    };
+    void (*fk)(GemmArgs, uint32_t) = f16_instance(fmt1, image, of_tile);
     if (io.qb_out) {  // the outputs also leave as QB32 rows (the next fp6-form matmul's input): 64-token tiles only, no silu pairing, K' = rows % 256 == 0
         if (ttw != 4 || io.silu_mul || w.rows % 256 != 0) return hipErrorInvalidValue;
-        fk = rt5 ? (fmt1 ? k_gemm_f16a<1, 4, 2, 5> : k_gemm_f16a<0, 4, 2, 5>) : (fmt1 ? k_gemm_f16a<1, 4, 2> : k_gemm_f16a<0, 4, 2>);
+        fk = f16_instance(fmt1, image, [&](auto fmt) { return rt5 ? k_gemm_f16a<decltype(fmt)::value, 4, 2, 5> : k_gemm_f16a<decltype(fmt)::value, 4, 2>; });
         a.qb_nblk_out = (int)(w.rows / 256);
         a.qb_out = static_cast<uint8_t *>(io.qb_out);
     }
@@ -2497,7 +2581,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
     // output element whichever kernel computes it (k-order, f32 accumulation): bit-identical to the one-kernel launch.  BITNET_HIP_GEMM_F16H=0: off.
     static const int f16h_mode = [] { const char *e = getenv("BITNET_HIP_GEMM_F16H"); return e ? atoi(e) : 1; }();
     const size_t slots = 2 * kGemmCUs;
-    if (f16h_mode && ttw == 4 && !rt5 && !io.qb_out && m_pad % 128 == 0 && w.rows * w.cols / 4 < ((size_t)1 << 31)) {
+    if (f16h_mode && ttw == 4 && !rt5 && !io.qb_out && m_pad % 128 == 0 && w.rows * w.cols / (image ? 2 : 4) < ((size_t)1 << 31)) {
         const size_t t128 = m_pad / 128;
         size_t n_a = (gx0 * t128 / slots) * slots / t128;  // row blocks whose 128-token workgroups fill whole rounds
         // a launch whose 128-token workgroups fit ONE round that is at least three quarters full (q|k|v: 15 x 32 = 480 of 512 slots, against 960 = 1.9 rounds of
@@ -2505,7 +2589,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
         if (gx0 * t128 <= slots && 4 * gx0 * t128 >= 3 * slots) n_a = gx0;
         if (gx0 < 24 && n_a != gx0) n_a = 0;
         if (n_a >= gx0 / 2 && n_a > 0) {
-            void (*hk)(GemmArgs, uint32_t) = fmt1 ? k_gemm_f16h<1> : k_gemm_f16h<0>;
+            void (*hk)(GemmArgs, uint32_t) = f16_instance(fmt1, image, [](auto fmt) { return k_gemm_f16h<decltype(fmt)::value>; });
             {
                 static std::mutex h_mu;
                 static std::unordered_set<const void *> h_raised;
@@ -2517,7 +2601,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
                 }
             }
             GemmArgs aa = a;
-            aa.wgroup = gemm_weight_group(n_a, 256, w.cols, fmt1);
+            aa.wgroup = gemm_weight_group(n_a, 256, image ? 2 * w.cols : w.cols, fmt1);
             hipLaunchKernelGGL(hk, dim3((unsigned)n_a, (unsigned)t128), dim3(256), (size_t)2 * 128 * 256 + 128 * 8 + 4096, stream, aa, lut_f16_hi(w.lut));
             g_last_gemm_tile = GemmTileChoice{2, 128, 4, fmt1 ? 4 : 5, 64};
             if (n_a == gx0) return hipGetLastError();
@@ -2527,7 +2611,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
             return hipGetLastError();
         }
     }
-    a.wgroup = gemm_weight_group(gx0, rt5 ? 320 : rt2 ? 128 : 256, w.cols, fmt1);
+    a.wgroup = gemm_weight_group(gx0, rt5 ? 320 : rt2 ? 128 : 256, image ? 2 * w.cols : w.cols, fmt1);
     hipLaunchKernelGGL(fk, dim3((unsigned)gx0, (unsigned)(m_pad / (16 * ttw))), dim3(256), lds, stream, a, lut_f16_hi(w.lut));
     return hipGetLastError();
 }

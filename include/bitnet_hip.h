@@ -289,6 +289,9 @@ int bitnet_hip_weights_fp4_image(bitnet_hip_weights_t h, int enable, void *strea
  *                  (sum, sum of squares) over disjoint row ranges that together cover the row -- one per wave of the producing launch
  *                  (64 rows, or 80 in 320-row workgroups: then the first rows / 80 entries are used and the others are written as zero);
  *                  the consumer adds all rows / 64 entries up (n_stats = rows / 64).
+ * The first call on a matrix builds an image of it, the codes as fp4 in the order of this form's operands, 4 bits per weight that bitnet_hip_weights_device_bytes counts (an
+ * allocation + one kernel, synchronises `stream`); under stream capture, without memory for it or with BITNET_HIP_FP4_RESIDENT=0 the codes are expanded in the K loop instead, to
+ * the same values.
  * bitnet_hip_matmul_f16_supported: rows % 256 == 0, cols % 256 == 0, code map values in -2..2, no scales or f16 32-block scales.
  * bitnet_hip_rows_to_f16_dev: the chain's entry (the embedding rows): xh = f16(gamma * x) (gamma nullable) + stats partial 0. */
 /* f16 hand-over rows carry no row scale: a value beyond +-65504 is clamped -- and COUNTED.  Returns the number of lanes (up to four elements each)

@@ -334,3 +334,39 @@ def test_f16h_wide_tile_instances_match_oracle_and_the_64_token_kernel(hip, orac
     assert p.returncode == 0, p.stdout[-1500:] + p.stderr[-3000:]
     h0 = [l.split()[1] for l in p.stdout.splitlines() if l.startswith("HASH ")][0]
     assert h0 == h1, "k_gemm_f16h's outputs differ from k_gemm_f16a's"
+
+
+# rows x cols x tokens: every form of the launch -- 128-row workgroups of 16 and 32 tokens, 256-row ones of 16, 32 and 64, 320-row ones, 128-token wave tiles whole and beside the others
+@pytest.mark.parametrize("fmt", ["qk256", "i2s"])
+@pytest.mark.parametrize("rows,cols,m,silu", [(256, 256, 1, 0), (2560, 512, 17, 0), (2560, 768, 300, 0), (5376, 256, 200, 0), (13824, 256, 130, 1), (10240, 512, 513, 1), (2560, 256, 4000, 0),
+                                              (3840, 512, 4096, 0), (13824, 256, 2048, 1)])
+def test_chain_on_the_image_is_the_expanding_one_bit_for_bit(hip, torch_, fmt, rows, cols, m, silu):
+    """A captured launch builds no image and expands the codes in its K loop; the first eager one builds it and reads its operands from there: the same values, the same order of sums."""
+    rng = np.random.default_rng(rows + cols + m)
+    parts = [make_matrix(hip, rng, fmt, rows // 2, cols)[0] for _ in range(2)]
+    h = hip.weights_concat(parts, interleave16=bool(silu))
+    mp, out = -(-m // 64) * 64, rows // 2 if silu else rows
+    xh = torch_.from_numpy(rng.normal(0, 1, (mp, cols)).astype(np.float16)).cuda()
+    flags = 1 if silu else 0
+
+    def buffers():
+        return (None if silu else torch_.full((m, out), 7.0, device="cuda")), torch_.full((mp, out), 7.0, dtype=torch_.float16, device="cuda")
+
+    def launch(b, stream):
+        hip.matmul_f16_dev(h, xh, m, y=b[0], yh=b[1], flags=flags, stream=stream)
+
+    expanded, image, b0 = buffers(), buffers(), hip.weights_device_bytes(h)
+    torch_.cuda.synchronize()
+    graph, s = torch_.cuda.CUDAGraph(), torch_.cuda.Stream()
+    with torch_.cuda.graph(graph, stream=s):
+        launch(expanded, s.cuda_stream)
+    assert hip.weights_device_bytes(h) == b0
+    graph.replay()
+    torch_.cuda.synchronize()
+    launch(image, torch_.cuda.current_stream().cuda_stream)
+    torch_.cuda.synchronize()
+    assert hip.weights_device_bytes(h) == b0 + rows // 16 * (cols // 256) * 2048
+    for a, b in zip(expanded, image):
+        assert a is None or (torch_.isfinite(a).all() and torch_.equal(a, b))
+    for w in (h, *parts):
+        hip.weights_free(w)
