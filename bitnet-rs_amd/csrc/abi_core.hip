@@ -115,6 +115,16 @@ int bitnet_hip_advance_pos_dev(int32_t *pos_dev, void *stream) {
     BH_GUARD_END
 }
 
+int bitnet_hip_sequence_update_dev(int32_t *history_dev, size_t first, size_t n, const int32_t *tokens, int32_t *n_forced_dev, int32_t forced, int32_t *pos_dev, int32_t position,
+                                   const float *row_dev, float *x_dev, size_t width, void *stream) {
+    BH_GUARD_BEGIN
+    if ((row_dev != nullptr) != (x_dev != nullptr) || (tokens && !history_dev)) return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "sequence_update_dev: a source without its destination");
+    if (n > (size_t)INT32_MAX || width > (size_t)INT32_MAX) return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "sequence_update_dev: n=%zu, width=%zu", n, width);
+    BH_HIP_TRY(launch_sequence_update(SequenceUpdate{history_dev, first, n, tokens, n_forced_dev, pos_dev, forced, position, row_dev, x_dev, width}, (hipStream_t)stream));
+    return BITNET_HIP_OK;
+    BH_GUARD_END
+}
+
 int bitnet_hip_argmax_dev(const float *v, size_t n, void *scratch, size_t n_wg, int32_t *token_dev, void *stream) {
     BH_GUARD_BEGIN
     if (!v || !scratch || !token_dev) return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "Null pointer passed to argmax_dev");

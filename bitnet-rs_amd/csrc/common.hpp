@@ -234,6 +234,7 @@ bool gemm_qb32_supported(const Weights &w);
 // the fp6 x fp4 form on QB32 rows (io.xh = the QB32 buffer) with the f16 chain's epilogue (LayerNorm after the product, residual, silu * up -> f16 rows)
 hipError_t launch_gemm_qb32(const Weights &w, const GemmF16Io &io, size_t m, hipStream_t stream);
 bool gemm_f16_chain_supported(const Weights &w);
+hipError_t launch_f16_saturations(uint32_t *count, hipStream_t stream);
 unsigned long long f16_saturations(bool reset);  // f16 hand-over values clamped to +-65504 since the last reset (lanes, not elements); synchronises the device
 hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m, hipStream_t stream);
 hipError_t launch_rows_to_f16(const float *x, const float *gamma, size_t m, size_t cols, void *xh, float *stats, hipStream_t stream);
@@ -266,6 +267,17 @@ hipError_t launch_dequant_i2s(const uint8_t *bytes, size_t rows, size_t cols, si
 hipError_t launch_embed_f16(const void *table, const int *tokens, const int *offset_ptr, int n, int hidden,
                             int vocab, float *out, hipStream_t stream);
 hipError_t launch_advance_pos(int *pos_ptr, hipStream_t stream);
+struct SequenceUpdate {  // null: left out
+    int *history;
+    size_t first, n;
+    const int *tokens;  // null: zeros
+    int *n_forced, *pos;
+    int forced, position;
+    const float *row;
+    float *x;
+    size_t width;
+};
+hipError_t launch_sequence_update(const SequenceUpdate &u, hipStream_t stream);
 hipError_t launch_add(const float *a, const float *b, float *out, size_t n, hipStream_t stream);
 // out[i] = silu(gate[.]) * up[.]; tile == 0: gate[i], up[i]; tile > 0: both live in ONE buffer of alternating
 // tile-row groups (gate tile, up tile, ...), gate = the buffer, up = gate + tile (weights_concat interleave16)

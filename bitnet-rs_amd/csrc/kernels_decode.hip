@@ -288,6 +288,22 @@ hipError_t launch_advance_pos(int *pos_ptr, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// what a host notes down between portions: a launch of its own would cost more than the bytes
+__global__ __launch_bounds__(256) void k_sequence_update(SequenceUpdate u) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (u.history && i < u.n) u.history[u.first + i] = u.tokens ? u.tokens[i] : 0;
+    if (u.x && i < u.width) u.x[i] = u.row[i];
+    if (i == 0) {
+        if (u.n_forced) *u.n_forced = u.forced;
+        if (u.pos) *u.pos = u.position;
+    }
+}
+hipError_t launch_sequence_update(const SequenceUpdate &u, hipStream_t stream) {
+    const size_t n = u.history ? u.n : 0, m = u.x ? u.width : 0, most = n > m ? n : m;
+    hipLaunchKernelGGL(k_sequence_update, dim3((unsigned)(most ? (most + 255) / 256 : 1)), dim3(256), 0, stream, u);
+    return hipGetLastError();
+}
+
 // Plain argmax over a logits vector (host-visible entry point).
 __global__ __launch_bounds__(256) void k_argmax_partial(const float *__restrict__ v, int n, float *__restrict__ best_val,
                                                         int *__restrict__ best_idx) {

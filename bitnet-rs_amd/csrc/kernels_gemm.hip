@@ -480,6 +480,14 @@ __device__ __forceinline__ _Float16 gclamp_f16(float v, bool &sat) {
 __device__ __forceinline__ void gflush_sat(bool sat) {
     if (sat) atomicAdd(&g_f16_saturations, 1u);  // (rare: one atomic per lane that clamped, none otherwise)
 }
+__global__ void k_take_saturations(uint32_t *count) {
+    const uint32_t v = atomicExch(&g_f16_saturations, 0u);
+    if (count) *count = v;
+}
+hipError_t launch_f16_saturations(uint32_t *count, hipStream_t stream) {
+    hipLaunchKernelGGL(k_take_saturations, dim3(1), dim3(1), 0, stream, count);
+    return hipGetLastError();
+}
 unsigned long long f16_saturations(bool reset) {
     unsigned int v = 0;
     if (hipMemcpyFromSymbol(&v, HIP_SYMBOL(g_f16_saturations), sizeof(v)) != hipSuccess) return ~0ull;  // (synchronises the device)

@@ -455,9 +455,11 @@ int Decoder::trace_step(const char *dir, bool with_logits) {
     tr.dir = dir;
     tr.seq = p;  // token position of this step (the reference counts 0 = first position)
     tr.stream = stream_;
+    host_pos_ = -1;
     const int rc = step_launches(with_logits, form_at(p), &tr);
     if (rc) return rc;
-    HCHK(hipStreamSynchronize((hipStream_t)stream_));
+    if (int rs = settle()) return rs;
+    moved_to(p + 1);
     return 0;
 }
 
@@ -506,11 +508,13 @@ int Decoder::run_reference(int n, bool with_logits) {
         err_ = "KV cache overflow";
         return BITNET_HIP_ERR_INVALID_ARGUMENT;
     }
+    host_pos_ = -1;
     for (int i = 0; i < n; ++i) {
         const int rc = step_launches_reference(with_logits);
         if (rc) return rc;
     }
-    HCHK(hipStreamSynchronize((hipStream_t)stream_));
+    if (int rc = settle()) return rc;
+    moved_to(p + n);
     // the reference-order kernels rebuilt a row-major copy of every matrix: give them back (one copy of the weights on the device)
     for (auto &L : layers_)
         for (bitnet_hip_weights_t h : {L.qkv, L.o, L.gateup, L.down})
@@ -760,12 +764,8 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
         pf_cap_ = n;
     }
     hipStream_t s = (hipStream_t)stream_;
-    Event ev0, ev1;
-    HCHK(hipEventCreate(&ev0.e));
-    HCHK(hipEventCreate(&ev1.e));
-    hipEvent_t e0 = ev0.e, e1 = ev1.e;
-    if (!force_scaled_) (void)bitnet_hip_f16_saturations(1);  // a fresh count for this prompt
-    HCHK(hipEventRecord(e0, s));
+    HCHK(hipEventRecord(begin_.e, s));
+    if (!force_scaled_) BCHK(bitnet_hip_f16_saturations_dev(nullptr, s));  // a fresh count for this prompt
     const size_t N = (size_t)n;
     BCHK(bitnet_hip_embed_f16_dev(embed_, history_, pos_, N, H, (size_t)c_.vocab, pf_x_, s));  // *pos_ == 0
     const bool chain = chain_applies(digits);
@@ -826,25 +826,26 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
         // f16 hand-over rows carry no row scale: a value beyond +-65504 (outlier channels x gamma: none in the synthetic models, possible in a real
         // checkpoint) is clamped AND counted (bitnet_hip_f16_saturations).  A prompt that clamped anything is repeated on the digit planes --
         // 30-bit fixed point behind a per-row power-of-two scale (digits = 4: a row whose outlier is 10^5 times its typical element still keeps 13 bits of
-        // those; the 2-digit and row-scaled f16 forms would flush them) -- before its logits are taken (no silent saturation).
-        HCHK(hipStreamSynchronize(s));
-        if (bitnet_hip_f16_saturations(1) > 0) {
-            force_scaled_ = true;
-            ++saturation_fallbacks_;
-            const int rc = prefill(n, with_logits, 4, elapsed_ms);
-            force_scaled_ = false;
-            return rc;
-        }
+        // those; the 2-digit and row-scaled f16 forms would flush them): no silent saturation.  The count is looked at once the logits are there, too, which
+        // a second pass then writes over: the device does not wait for the host in between.
+        BCHK(bitnet_hip_f16_saturations_dev((uint32_t *)pinned_, s));
     }
     {
-        const int rc = finish_prefill(n, pf_x_ + (N - 1) * H, with_logits);
+        const int rc = hand_over(n, pf_x_ + (N - 1) * H, with_logits);
         if (rc) return rc;
     }
-    HCHK(hipEventRecord(e1, s));
-    HCHK(hipStreamSynchronize(s));
-    float ms = 0.f;
-    HCHK(hipEventElapsedTime(&ms, e0, e1));
-    if (elapsed_ms) *elapsed_ms = ms;
+    HCHK(hipEventRecord(end_.e, s));
+    if (int rc = settle()) return rc;
+    if ((chain || qb || h16) && pinned_[0] != 0) {
+        if (int rc = update(0, 0, nullptr, false, 0)) return rc;
+        force_scaled_ = true;
+        ++saturation_fallbacks_;
+        const int rc = prefill(n, with_logits, 4, elapsed_ms);
+        force_scaled_ = false;
+        return rc;
+    }
+    moved_to(n);
+    if (elapsed_ms) HCHK(hipEventElapsedTime(elapsed_ms, begin_.e, end_.e));
     return 0;
 }
 
@@ -938,7 +939,7 @@ int Decoder::prefill_sharded(int n, int rank, int world, bitnet_host_allgather_f
     {
         // this rank's rows: chunk `rank`, then chunk 2 world - 1 - rank
         std::vector<int32_t> hist((size_t)n), tok(N), bp(N / 64);
-        HCHK(hipMemcpy(hist.data(), history_, (size_t)n * 4, hipMemcpyDeviceToHost));
+        if (int rc = history(hist.data(), n)) return rc;
         const int starts[2] = {rank * chunk, (2 * world - 1 - rank) * chunk};
         for (int h = 0; h < 2; ++h)
             for (int i = 0; i < chunk; ++i) {
@@ -1070,24 +1071,28 @@ int Decoder::prefill_sharded(int n, int rank, int world, bitnet_host_allgather_f
 }
 
 int Decoder::finish_prefill(int n, const float *last_row, bool with_logits) {
-    // hand over to the single-token state: residual stream of the last position, position counter
     if (n <= 0 || n > c_.max_pos - 1) {
         err_ = "KV cache overflow";
         return BITNET_HIP_ERR_INVALID_ARGUMENT;
     }
+    if (int rc = hand_over(n, last_row, with_logits)) return rc;
+    if (int rc = settle()) return rc;
+    moved_to(n);
+    return 0;
+}
+
+// to the single-token state: residual stream of the last position, position counter
+int Decoder::hand_over(int n, const float *last_row, bool with_logits) {
     hipStream_t s = (hipStream_t)stream_;
     const size_t H = c_.hidden;
-    if (last_row) HCHK(hipMemcpyAsync(x_, last_row, H * 4, hipMemcpyDeviceToDevice, s));
-    const int32_t last = n - 1;
-    HCHK(hipMemcpyAsync(pos_, &last, 4, hipMemcpyHostToDevice, s));
-    HCHK(hipStreamSynchronize(s));  // `last` is a stack variable
+    if (int rc = update(0, 0, nullptr, false, n - 1, last_row, last_row ? x_ : nullptr)) return rc;
+    host_pos_ = -1;
     if (with_logits && last_row) {
         BCHK(bitnet_hip_logits_f16_dev(embed_, x_, final_norm_, c_.eps, H, (size_t)c_.vocab, logits_, scratch_, (size_t)logits_wgs_, token_,
                                        pos_, history_, n_forced_, s));
     } else {
         BCHK(bitnet_hip_advance_pos_dev(pos_, s));
     }
-    HCHK(hipStreamSynchronize(s));
     return 0;
 }
 
@@ -1102,6 +1107,7 @@ void Decoder::layer_objects(int layer, uint64_t handles[4], void *ptrs[4]) const
 }
 
 void Decoder::global_objects(void *ptrs[7]) const {
+    expose();
     ptrs[0] = embed_, ptrs[1] = final_norm_, ptrs[2] = rope_sin_, ptrs[3] = rope_cos_, ptrs[4] = history_, ptrs[5] = pos_, ptrs[6] = stream_;
 }
 

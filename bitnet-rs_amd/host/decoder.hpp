@@ -104,6 +104,7 @@ class Decoder : public Sequence {
     // the KV cache already holds positions 0..n-1; last_row (device, [hidden]) is the residual stream
     // of position n-1 or null on ranks that do not own it (then only the position counter moves).
     int finish_prefill(int n, const float *last_row, bool with_logits);
+    int hand_over(int n, const float *last_row, bool with_logits);  // its launches
     bool chain_applies(int digits) const;
     bool handover16_applies(int digits) const;
     bool hybrid_applies(size_t n_rows) const;

@@ -2,6 +2,7 @@
 #include "sequence.hpp"
 
 #include <cstdio>
+#include <cstring>
 #include <vector>
 
 namespace bitnet_host {
@@ -28,6 +29,9 @@ int Sequence::init_sequence(int vocab, int width, int max_pos) {
     HCHK(hipMalloc((void **)&n_forced_, 4));
     HCHK(hipMalloc((void **)&token_, 4));
     HCHK(hipMalloc((void **)&history_, ((size_t)max_pos + 2) * 4));
+    HCHK(hipHostMalloc((void **)&pinned_, (1 + (size_t)kStaged) * 4, hipHostMallocCoherent));
+    HCHK(hipEventCreate(&begin_.e));
+    HCHK(hipEventCreate(&end_.e));
     return 0;
 }
 
@@ -35,6 +39,7 @@ Sequence::~Sequence() {
     drop_graphs();
     for (void *p : {(void *)logits_, (void *)pos_, (void *)n_forced_, (void *)history_, (void *)token_})
         if (p) hipFree(p);
+    if (pinned_) hipHostFree(pinned_);
     if (stream_) hipStreamDestroy((hipStream_t)stream_);
 }
 
@@ -46,12 +51,26 @@ void Sequence::drop_graphs() {
     }
 }
 
+int Sequence::settle() {
+    HCHK(hipStreamSynchronize((hipStream_t)stream_));
+    staged_ = false;
+    return 0;
+}
+
+// the tokens, position and row a step reads, in stream order: nothing here waits for the device
+int Sequence::update(int first, int n, const int32_t *tokens, bool forced, int pos, const float *row, float *x) {
+    host_pos_ = pos >= 0 ? -1 : host_pos_;
+    BCHK(bitnet_hip_sequence_update_dev(n > 0 ? history_ : nullptr, (size_t)first, (size_t)n, n > 0 ? tokens : nullptr, forced ? n_forced_ : nullptr, host_forced_, pos >= 0 ? pos_ : nullptr, pos, row, x,
+                                        x ? (size_t)width_ : 0, stream_));
+    if (pos >= 0) moved_to(pos);
+    return 0;
+}
+
 int Sequence::reset() {
     host_forced_ = 0;
-    HCHK(hipMemset(pos_, 0, 4));
-    HCHK(hipMemset(n_forced_, 0, 4));
-    HCHK(hipMemset(history_, 0, ((size_t)max_pos_ + 2) * 4));
-    return clear_state();
+    if (int rc = update(0, max_pos_ + 2, nullptr, true, 0)) return rc;
+    if (int rc = clear_state()) return rc;
+    return exposed_ ? settle() : 0;
 }
 
 int Sequence::feed(const int32_t *tokens, int n) {
@@ -66,23 +85,34 @@ int Sequence::feed(const int32_t *tokens, int n) {
             return fail_arg(b);
         }
     if (base + n > max_pos_) return fail_arg("KV cache overflow");  // T:1190-1194
-    HCHK(hipMemcpy(history_ + base, tokens, (size_t)n * 4, hipMemcpyHostToDevice));
-    host_forced_ = base + n;
-    HCHK(hipMemcpy(n_forced_, &host_forced_, 4, hipMemcpyHostToDevice));
-    return 0;
+    if (staged_)
+        if (int rc = settle()) return rc;
+    for (int i = 0; i == 0 || i < n; i += kStaged) {
+        const int part = n - i < kStaged ? n - i : kStaged;
+        if (i > 0)
+            if (int rc = settle()) return rc;
+        if (part > 0) memcpy(pinned_ + 1, tokens + i, (size_t)part * 4);
+        host_forced_ = base + i + part;
+        if (int rc = update(base + i, part, pinned_ + 1, true, -1)) return rc;
+        staged_ = true;
+    }
+    return exposed_ ? settle() : 0;
 }
 
 int Sequence::position() {
+    if (host_pos_ >= 0) return host_pos_;
     int p = -1;
-    if (hipMemcpy(&p, pos_, 4, hipMemcpyDeviceToHost) != hipSuccess) {
+    if (settle() != 0 || hipMemcpy(&p, pos_, 4, hipMemcpyDeviceToHost) != hipSuccess) {
         err_ = "position readback failed";
         return -1;
     }
+    moved_to(p);
     return p;
 }
 
 int Sequence::history(int32_t *out, int n) {
     if (!out || n < 0 || n > max_pos_ + 2) return fail_arg("history: n out of range");
+    if (int rc = settle()) return rc;
     HCHK(hipMemcpy(out, history_, (size_t)n * 4, hipMemcpyDeviceToHost));
     return 0;
 }
@@ -142,10 +172,8 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
             if (rc) return rc;
         }
     }
-    Event ev0, ev1;
-    HCHK(hipEventCreate(&ev0.e));
-    HCHK(hipEventCreate(&ev1.e));
-    HCHK(hipEventRecord(ev0.e, s));
+    host_pos_ = -1;
+    HCHK(hipEventRecord(begin_.e, s));
     for (int i = 0; i < n; ++i) {
         if (use_graph) {
             HCHK(hipGraphLaunch((hipGraphExec_t)graph_exec_[2 * form_at(p + i) + (with_logits ? 1 : 0)], s));
@@ -154,11 +182,10 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
             if (rc) return rc;
         }
     }
-    HCHK(hipEventRecord(ev1.e, s));
-    HCHK(hipStreamSynchronize(s));
-    float ms = 0.f;
-    HCHK(hipEventElapsedTime(&ms, ev0.e, ev1.e));
-    if (elapsed_ms) *elapsed_ms = ms;
+    HCHK(hipEventRecord(end_.e, s));
+    if (int rc = settle()) return rc;
+    moved_to(p + n);
+    if (elapsed_ms) HCHK(hipEventElapsedTime(elapsed_ms, begin_.e, end_.e));
     return 0;
 }
 

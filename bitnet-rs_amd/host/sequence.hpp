@@ -66,7 +66,7 @@ class Sequence {
     // Captures and instantiates the step graph of every form a sequence can reach ahead of time, so that no run() pays for a
     // capture in the middle of a generation.  Nothing executes.
     int prepare_graphs(bool with_logits);
-    int position();                    // tokens consumed so far
+    int position();                    // tokens consumed so far; -1: it could not be read
     int history(int32_t *out, int n);  // first n tokens of the sequence
     int last_logits(float *out);       // [vocab], of the last step run with logits
     virtual int last_hidden(float *out) = 0;  // residual stream after the last block (pre final norm)
@@ -81,6 +81,10 @@ class Sequence {
     int check_run(int n, bool with_logits);
     int ensure_graph(bool with_logits, int form);
     void drop_graphs();
+    int settle();                       // waits for the stream
+    void moved_to(int p) { host_pos_ = exposed_ ? -1 : p; }
+    void expose() const { exposed_ = true, host_pos_ = -1; }  // somebody else may write the device's position and read its history from now on
+    int update(int first, int n, const int32_t *tokens, bool forced, int pos, const float *row = nullptr, float *x = nullptr);  // (pos < 0: stays)
 
     virtual bool ready() const = 0;                            // weights are there
     virtual int step(bool with_logits, int form) = 0;          // the launches of one single-token step
@@ -94,6 +98,13 @@ class Sequence {
     float *logits_ = nullptr;
     int32_t *pos_ = nullptr, *n_forced_ = nullptr, *history_ = nullptr, *token_ = nullptr;
     int host_forced_ = 0;
+    mutable int host_pos_ = -1;  // *pos_ where it is known: every call that moves it knows where to
+    mutable bool exposed_ = false;
+    // pinned: a clamp count for the model's use, then tokens on their way to the history (staged_: a launch that reads them may be waiting)
+    static constexpr int kStaged = 16384;
+    int32_t *pinned_ = nullptr;
+    bool staged_ = false;
+    Event begin_, end_;  // of the last run or prefill
     static constexpr int kForms = 3;
     void *graph_exec_[2 * kForms] = {};  // [2 * form + with_logits]
     void *graph_[2 * kForms] = {};

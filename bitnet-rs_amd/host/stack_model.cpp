@@ -645,7 +645,6 @@ int StackModel::clear_state() {
     for (const Layer &L : layers_)
         for (const Slot &slot : L.slots)
             if (slot.state) HCHK(hipMemsetAsync(slot.state, 0, slot.state_bytes, (hipStream_t)stream_));
-    HCHK(hipStreamSynchronize((hipStream_t)stream_));
     hidden_ = nullptr;
     return 0;
 }
@@ -1237,12 +1236,6 @@ int StackModel::portion(int rows, int pos0) {
     return 0;
 }
 
-int StackModel::set_position(int p) {
-    HCHK(hipMemcpyAsync(pos_, &p, 4, hipMemcpyHostToDevice, (hipStream_t)stream_));
-    HCHK(hipStreamSynchronize((hipStream_t)stream_));  // `p` is a stack variable
-    return 0;
-}
-
 int StackModel::prefill(int n, bool with_logits, int, float *elapsed_ms) {
     if (!ready()) return fail_arg("model globals not set");
     const int p = position();
@@ -1251,23 +1244,20 @@ int StackModel::prefill(int n, bool with_logits, int, float *elapsed_ms) {
     if (p + n > max_pos_ - 1) return fail_arg("KV cache overflow");
     TRY(portion_buffers(n));
     hipStream_t s = (hipStream_t)stream_;
-    Event e0, e1;
-    HCHK(hipEventCreate(&e0.e));
-    HCHK(hipEventCreate(&e1.e));
-    HCHK(hipEventRecord(e0.e, s));
+    HCHK(hipEventRecord(begin_.e, s));
     TRY(portion(n, p));
-    TRY(set_position(with_logits ? p + n - 1 : p + n));
+    TRY(update(0, 0, nullptr, false, with_logits ? p + n - 1 : p + n));
+    host_pos_ = -1;
     if (with_logits) {
         bitnet_hip_vector_input in = plain_input(hidden_);
         in.kind = BITNET_HIP_IN_NORM;
         in.eps = spec_.eps, in.weight_offset = spec_.norm_offset, in.weight = final_norm_.w, in.bias = final_norm_.bias, in.center = spec_.center, in.n = width_;
         BCHK(bitnet_hip_dense_logits_dev(&in, head_m_.w, vocab_, head_m_.cols, head_m_.ld, logits_, argmax_, token_, pos_, history_, n_forced_, s));
     }
-    HCHK(hipEventRecord(e1.e, s));
-    HCHK(hipStreamSynchronize(s));
-    float ms = 0.f;
-    HCHK(hipEventElapsedTime(&ms, e0.e, e1.e));
-    if (elapsed_ms) *elapsed_ms = ms;
+    HCHK(hipEventRecord(end_.e, s));
+    TRY(settle());
+    moved_to(p + n);
+    if (elapsed_ms) HCHK(hipEventElapsedTime(elapsed_ms, begin_.e, end_.e));
     return 0;
 }
 

@@ -279,7 +279,6 @@ class StackModel : public Sequence {
     int portion_block(size_t i, int pass, int which, size_t n, size_t pos0);
     int portion_loop_in(size_t n);
     int portion_buffers(size_t n);
-    int set_position(int p);
 
     StackSpec spec_;
     bool f32_ = false;

@@ -300,6 +300,8 @@ int bitnet_hip_weights_fp4_image(bitnet_hip_weights_t h, int enable, void *strea
  * activations out (outlier channels x gamma beyond the f16 range) checks it behind a prompt and repeats the prompt on the row-scaled forms
  * (bitnet_hip_matmul_fused_dev), as Decoder::prefill does. */
 unsigned long long bitnet_hip_f16_saturations(int reset);
+/* The same count stored at `count` (device or pinned host memory; nullable) and cleared, in stream order and without a synchronisation. */
+int bitnet_hip_f16_saturations_dev(uint32_t *count, void *stream);
 int bitnet_hip_matmul_f16_supported(bitnet_hip_weights_t w);
 int bitnet_hip_rows_to_f16_dev(const float *x_dev, const float *gamma_dev, size_t m, size_t cols, void *xh_dev, float *stats_dev, void *stream);
 int bitnet_hip_matmul_f16_dev(bitnet_hip_weights_t w, const void *xh_dev, size_t m, const float *stats_in_dev, size_t n_stats,
@@ -394,6 +396,10 @@ int bitnet_hip_silu_mul_dev(const float *gate_dev, const float *up_dev, float *o
                             void *stream);
 /* *pos_dev += 1 (prompt positions whose logits nobody reads). */
 int bitnet_hip_advance_pos_dev(int32_t *pos_dev, void *stream);
+/* A sequence's bookkeeping in one launch, in stream order; what is null is left out.  history_dev[first .. first + n) = tokens, or zeros without them (tokens: device memory, or pinned
+ * host memory that stays as it is until the launch has run); *n_forced_dev = forced; *pos_dev = position; x_dev[0 .. width) = row_dev. */
+int bitnet_hip_sequence_update_dev(int32_t *history_dev, size_t first, size_t n, const int32_t *tokens, int32_t *n_forced_dev, int32_t forced, int32_t *pos_dev, int32_t position,
+                                   const float *row_dev, float *x_dev, size_t width, void *stream);
 /* One new token through MultiHeadAttention::forward's core (T:373-540): RoPE on q,k with
  * the split-half layout (T:134-163) at position *pos_dev, append k,v to the f32 cache
  * (T:1171-1202; n_kv*ceil(max_pos/64)*64*head_dim floats each, layout private to this library: K is kept

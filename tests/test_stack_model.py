@@ -617,3 +617,29 @@ def test_trace_runner_matches_the_library(cases, pkg, tmp_path, name):
         if w:
             assert np.array_equal(np.fromfile(str(tmp_path / f"{i}.f32"), np.float32).reshape(want.shape), want)
     assert not (tmp_path / "1.f32").exists()
+
+
+def test_tokens_of_many_feeds_reach_the_history(pkg, tmp_path):
+    """Tokens wait in pinned memory for the launch that copies them (16384 at a time): feeds that follow one another at once, ones of more than that, a reset behind them; the
+    position as the host keeps it through portions, steps and refused calls."""
+    path = u.save_model(str(tmp_path / "m"), MODELS["latent_without_ff"], u.random_tensors(MODELS["latent_without_ff"], 3))
+    m = pkg.open_model(path, "float32", 40000)
+    tokens = np.random.default_rng(1).integers(0, m.vocab, 36000).astype(np.int32)
+    for cuts in ([0, 36000], [0, 1, 2, 5, 5, 16389, 16390, 36000], [0, 16384, 32768, 36000]):
+        m.reset()
+        for a, b in zip(cuts, cuts[1:]):
+            m.feed(tokens[a:b])
+        assert np.array_equal(m.history(36000), tokens) and m.position() == 0
+    m.reset()
+    assert not m.history(40002).any()
+    m.feed(tokens[:60])
+    m.prefill(20, with_logits=False)
+    assert m.position() == 20
+    m.prefill(7)
+    m.run(3)
+    for refused in (lambda: m.prefill(31), lambda: m.feed([m.vocab]), lambda: m.run(39990)):
+        with pytest.raises(Exception):
+            refused()
+    assert m.position() == 30
+    m.run(30)
+    assert m.position() == 60 and np.array_equal(m.history(60), tokens[:60]) and m.history(61)[60] == int(np.argmax(m.last_logits()))

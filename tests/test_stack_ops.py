@@ -1,5 +1,7 @@
 """The bf16-weight operators and sequence mixers (include/bitnet_hip.h section 5), one at a time through the C ABI, against the
 plain restatement in oracle/stack_oracle.py or f64 numpy."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -427,3 +429,25 @@ def test_gated_norm_rows(hip):
     o64 = o.astype(np.float64)
     want = o64 / np.sqrt((o64 ** 2).sum(1, keepdims=True) / mean_n + eps) * w * gate[:, :n]
     assert u.rms_error(u.host(h)[:, :n], want) < F32_TOL and not u.host(h)[:, n:].any()
+
+
+@pytest.mark.parametrize("n,width", [(0, 0), (1, 0), (255, 256), (257, 1), (3000, 2560)])
+def test_sequence_update(hip, n, width):
+    import torch
+
+    history, scalars, x = torch.full((4000,), 9, dtype=torch.int32, device="cuda"), torch.tensor([5, 6], dtype=torch.int32, device="cuda"), torch.full((width + 2,), 3.0, device="cuda")
+    tokens, row = torch.arange(n + 1, dtype=torch.int32).pin_memory(), torch.randn(width + 1, device="cuda")
+    P = lambda t, at=0: C.c_void_p(t.data_ptr() + 4 * at)
+    call = lambda *a: hip._call("sequence_update_dev", *a, C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    call(P(history), C.c_size_t(7), C.c_size_t(n), P(tokens), P(scalars), C.c_int32(11), None, C.c_int32(0), P(row), P(x, 1), C.c_size_t(width))
+    torch.cuda.synchronize()
+    want = torch.full((4000,), 9, dtype=torch.int32)
+    want[7:7 + n] = tokens[:n]
+    assert torch.equal(history.cpu(), want) and scalars.tolist() == [11, 6]
+    assert torch.equal(x[1:1 + width], row[:width]) and x[0] == 3 and x[-1] == 3
+    call(P(history), C.c_size_t(8), C.c_size_t(n), None, None, C.c_int32(1), P(scalars, 1), C.c_int32(12), None, None, C.c_size_t(0))
+    torch.cuda.synchronize()
+    want[8:8 + n] = 0
+    assert torch.equal(history.cpu(), want) and scalars.tolist() == [11, 12]
+    with pytest.raises(Exception):
+        call(None, C.c_size_t(0), C.c_size_t(1), P(tokens), None, C.c_int32(0), None, C.c_int32(0), None, None, C.c_size_t(0))
