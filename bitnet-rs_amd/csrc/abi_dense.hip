@@ -124,8 +124,10 @@ int bitnet_hip_residual_norm_rows_dev(float *x, const float *y, size_t ldy, cons
     BH_REQUIRE(x && (!y || (post_weight && ldy >= width)) && (!h || ldh >= width), "residual_norm_rows: bad arguments");
     BH_REQUIRE(m > 0 && width > 0, "residual_norm_rows: empty");
     BH_CHECK_DIMS(m, width);
-    BH_HIP_TRY(launch_residual_norm_rows(x, y, ldy, post_weight, scale, next_weight, weight_offset, eps, (int)m, (int)width, h, ldh, h_f32,
-                                         (hipStream_t)stream));
+    SumRows r{};
+    r.x = x, r.m = m, r.width = width, r.y = y, r.ldy = y ? ldy : 0, r.eps = eps, r.h = h, r.ldh = h ? ldh : 0, r.h_f32 = h_f32, r.weight = next_weight;
+    r.weight_offset = weight_offset, r.post_weight = y ? post_weight : nullptr, r.scale = y ? scale : nullptr;
+    BH_HIP_TRY(launch_sum_norm_rows(r, (hipStream_t)stream));
     return BITNET_HIP_OK;
     BH_GUARD_END
 }

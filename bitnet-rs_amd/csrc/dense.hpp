@@ -206,8 +206,6 @@ hipError_t launch_embed_bf16(const uint16_t *table, size_t ld, const int *tokens
                              const float *norm_w, float eps, const TokenPairs &pairs, float *out, hipStream_t s);
 hipError_t launch_conv_keep(const void *rows, size_t ld, int rows_f32, int channels, int taps, float *ring, const int *pos, int n, hipStream_t s);
 hipError_t launch_sum_norm_rows(const SumRows &a, hipStream_t s);
-hipError_t launch_residual_norm_rows(float *x, const float *y, size_t ldy, const float *post_w, const float *scale, const float *next_w,
-                                     float offset, float eps, int m, int width, void *h, size_t ldh, int h_f32, hipStream_t s);
 hipError_t launch_gated_norm_rows(const float *o, size_t ldo, const float *w, const void *gate, size_t ldg, int gate_f32, float eps, int m, int n,
                                   int mean_n, void *h, size_t ldh, int h_f32, hipStream_t s);
 hipError_t launch_gather_rows(const float *x, const int *rows, int n, int width, float *out, hipStream_t s);

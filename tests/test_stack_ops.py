@@ -451,3 +451,62 @@ def test_sequence_update(hip, n, width):
     assert torch.equal(history.cpu(), want) and scalars.tolist() == [11, 12]
     with pytest.raises(Exception):
         call(None, C.c_size_t(0), C.c_size_t(1), P(tokens), None, C.c_int32(0), None, C.c_int32(0), None, None, C.c_size_t(0))
+
+
+@pytest.mark.parametrize("shift", [0, 1])  # rows that start off their alignment go column by column
+@pytest.mark.parametrize("width", [4, 1024, 1028, 2048, 2052, 3072, 3076, 3073, 4100])
+def test_row_norms_at_register_edges(hip, width, shift):
+    g = rng(width, shift)
+    m, ldh, eps = 3, u.up_to(width, 64) + 4, 1e-2
+    x, y = (g.standard_normal((m, width)).astype(np.float32) for _ in range(2))
+    pw, nw = (g.standard_normal(width).astype(np.float32) for _ in range(2))
+    gate = u.rounded(g.standard_normal((m, width)))
+    y64, gate_ld = y.astype(np.float64), u.up_to(width, 4)
+
+    def off(a, zeros):  # a device tensor whose first element lies `shift` past an aligned place
+        d = zeros(a.size + 8)
+        d[shift:shift + a.size] = (u.dev_f32(a) if zeros is u.zeros_f32 else u.dev_bf16(a)).reshape(-1)
+        return d[shift:shift + a.size]
+
+    for f32, tol in ((True, F32_TOL), (False, BF_TOL)):
+        h, xd = (u.zeros_f32 if f32 else u.zeros_bf16)(m, ldh) + 7, off(x, u.zeros_f32)
+        hip.residual_norm_rows_dev(xd, m, width, eps, 0.5, y=off(y, u.zeros_f32), ldy=width, post_weight=off(pw, u.zeros_f32), next_weight=u.dev_f32(nw), h=h, ldh=ldh, h_f32=f32)
+        want = x + y64 / np.sqrt((y64 ** 2).mean(1, keepdims=True) + eps) * (0.5 + pw)
+        assert u.rms_error(u.host(xd).reshape(m, width), want) < F32_TOL
+        want = want / np.sqrt((want ** 2).mean(1, keepdims=True) + eps) * (0.5 + nw)
+        assert u.rms_error(u.host(h)[:, :width], want) < tol and not u.host(h)[:, width:].any()
+
+        h = (u.zeros_f32 if f32 else u.zeros_bf16)(m, ldh) + 7
+        hip.gated_norm_rows_dev(off(y, u.zeros_f32), width, u.dev_f32(pw), (u.dev_f32 if f32 else u.dev_bf16)(u.padded(gate, gate_ld)), gate_ld, eps, f32, m, width, width, h, ldh, f32)
+        want = y64 / np.sqrt((y64 ** 2).mean(1, keepdims=True) + eps) * pw * gate
+        assert u.rms_error(u.host(h)[:, :width], want) < tol and not u.host(h)[:, width:].any()
+
+
+@pytest.mark.parametrize("q_rank,kv_rank", [(0, 1024), (2048, 0), (2049, 1025), (257, 1), (1536, 512)])
+def test_latent_rows_at_register_edges(hip, pkg, q_rank, kv_rank):
+    import torch
+
+    g = rng(q_rank, kv_rank)
+    m, rot, pos, eps, cap = 5, 8, 3, 1e-2, 16
+    rd = rot if kv_rank else 0
+    ldz, ldcq = q_rank + kv_rank + rd, q_rank + 3
+    z = g.standard_normal((m, ldz)).astype(np.float32)
+    qw, kw = g.standard_normal(max(q_rank, 1)).astype(np.float32), g.standard_normal(max(kv_rank, 1)).astype(np.float32)
+    angle = g.standard_normal((cap, rot // 2)).astype(np.float32)
+    dev = dict(z=u.dev_f32(z), qw=u.dev_f32(qw), kw=u.dev_f32(kw), cs=u.dev_f32(np.cos(angle)), sn=u.dev_f32(np.sin(angle)), cq=u.zeros_f32(m, ldcq) + 7, c=u.zeros_f32(cap, max(kv_rank, 1)),
+               r=u.zeros_f32(cap, rot), pos=torch.tensor([pos], dtype=torch.int32, device="cuda"))
+    P = {k: v.data_ptr() for k, v in dev.items()}
+    fields = dict(z=P["z"], ldz=ldz, q_rank=q_rank, eps=eps, pos=P["pos"])
+    if q_rank:
+        fields.update(q_weight=P["qw"], cq=P["cq"], ldcq=ldcq)
+    if kv_rank:
+        fields.update(kv_rank=kv_rank, rot_dim=rd, kv_weight=P["kw"], ccache=P["c"], rcache=P["r"], ldc=kv_rank, ldr=rot, rope_cos=P["cs"], rope_sin=P["sn"])
+    hip.latent_rows_dev(pkg.LatentRows(**fields), m, True)
+    z64 = z.astype(np.float64)
+    unit = lambda a: a / np.sqrt((a ** 2).mean(1, keepdims=True) + eps)
+    if q_rank:
+        assert u.rms_error(u.host(dev["cq"])[:, :q_rank], unit(z64[:, :q_rank]) * qw) < F32_TOL and not u.host(dev["cq"])[:, q_rank:].any()
+    if kv_rank:
+        assert u.rms_error(u.host(dev["c"])[pos:pos + m], unit(z64[:, q_rank:q_rank + kv_rank]) * kw) < F32_TOL
+        a, b, cs, sn = z64[:, ldz - rot:ldz - rot // 2], z64[:, ldz - rot // 2:], np.cos(angle[pos:pos + m]), np.sin(angle[pos:pos + m])
+        assert u.rms_error(u.host(dev["r"])[pos:pos + m], np.concatenate([a * cs - b * sn, b * cs + a * sn], 1)) < F32_TOL
