@@ -405,6 +405,11 @@ class HipLib:
         self._check(self.c.bitnet_hip_matmul_f16_dev(h, _ptr(xh), m, _optr(stats_in), n_stats, _optr(ln_gamma), ln_eps, _optr(y), _optr(residual), flags,
                                                      _optr(yh), _optr(gamma_out), _optr(stats_out), _vp(stream)))
 
+    def matmul_f16_takes_few_rows(self, h: int, m: int, flags: int = 0) -> bool:
+        """Is the form for few rows the faster one, so that matmul_f16_dev takes FUSE_FEW_ROWS?"""
+        self.c.bitnet_hip_matmul_f16_takes_few_rows.argtypes = [C.c_uint64, _sz, C.c_int]
+        return self.c.bitnet_hip_matmul_f16_takes_few_rows(h, m, flags) == 1
+
     def f16_saturations(self, reset: bool = True) -> int:
         self.c.bitnet_hip_f16_saturations.restype = C.c_uint64
         self.c.bitnet_hip_f16_saturations.argtypes = [C.c_int]

@@ -497,6 +497,9 @@ int bitnet_hip_matmul_f16_dev(bitnet_hip_weights_t h, const void *xh_dev, size_t
     io.yh = yh_dev;
     io.gamma_out = gamma_out_dev;
     io.stats_out = stats_out_dev;
+    io.few = (flags & BITNET_HIP_FUSE_FEW_ROWS) != 0;
+    if (io.few && ((flags & BITNET_HIP_FUSE_YH_QB32) || !gemm_f16_takes_few(*w, io.silu_mul, m)))
+        return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "FUSE_FEW_ROWS: only where bitnet_hip_matmul_f16_takes_few_rows says so, and without FUSE_YH_QB32");
     if (flags & BITNET_HIP_FUSE_YH_QB32) {  // yh_dev is a QB32 buffer (bitnet_hip_qb32_bytes(m, rows)): the next fp6-form matmul's input
         if (!yh_dev || io.silu_mul || w->rows % 256 != 0)
             return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "FUSE_YH_QB32 needs a QB32 buffer in yh_dev, rows %% 256 == 0 and no FUSE_SILU_MUL");
@@ -505,13 +508,18 @@ int bitnet_hip_matmul_f16_dev(bitnet_hip_weights_t h, const void *xh_dev, size_t
     }
     if (io.silu_mul && (!w->paired || residual_dev))
         return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "FUSE_SILU_MUL needs a handle from weights_concat(..., interleave16=1) and no residual");
-    io.image = want_pair_image(*w, (hipStream_t)stream);
+    if (!io.few) io.image = want_pair_image(*w, (hipStream_t)stream);
     hipError_t e = launch_gemm_f16_chain(*w, io, m, (hipStream_t)stream);
     if (e == hipErrorInvalidValue && io.qb_out)
         return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "FUSE_YH_QB32: this launch does not run 64-token tiles (too few rows for the QB32 hand-over)");
     if (e != hipSuccess) return set_error(BITNET_HIP_ERR_GPU, "kernel launch failed: %s", hipGetErrorString(e));
     return BITNET_HIP_OK;
     BH_GUARD_END
+}
+
+int bitnet_hip_matmul_f16_takes_few_rows(bitnet_hip_weights_t h, size_t m, int flags) {
+    const WeightsRef w = lookup(h);
+    return w && !(flags & BITNET_HIP_FUSE_YH_QB32) && gemm_f16_takes_few(*w, (flags & BITNET_HIP_FUSE_SILU_MUL) != 0, m) ? 1 : 0;
 }
 
 unsigned long long bitnet_hip_f16_saturations(int reset) { return f16_saturations(reset != 0); }

@@ -223,7 +223,8 @@ struct GemmF16Io {
     bool silu_mul = false;
     void *yh = nullptr;               // f16 [m_pad][rows] (rows / 2 with silu_mul), nullable
     const float *gamma_out = nullptr; // [rows]: yh = f16(gamma_out * y)
-    float *stats_out = nullptr;       // float2 [rows / 64][m_pad]
+    float *stats_out = nullptr;       // float2 [rows / 64][m_pad] ([rows / 16][m_pad] with few)
+    bool few = false;                 // k_gemm_f16_few (where gemm_f16_takes_few)
     void *qb_out = nullptr;           // QB32 buffer (qb32_bytes(m, rows)) receiving gamma_out * y (launch_gemm_f16_chain only; not with silu_mul)
     const uint8_t *image = nullptr;   // want_pair_image's (launch_gemm_f16_chain only)
 };
@@ -234,6 +235,7 @@ bool gemm_qb32_supported(const Weights &w);
 // the fp6 x fp4 form on QB32 rows (io.xh = the QB32 buffer) with the f16 chain's epilogue (LayerNorm after the product, residual, silu * up -> f16 rows)
 hipError_t launch_gemm_qb32(const Weights &w, const GemmF16Io &io, size_t m, hipStream_t stream);
 bool gemm_f16_chain_supported(const Weights &w);
+bool gemm_f16_takes_few(const Weights &w, bool silu_mul, size_t m);
 hipError_t launch_f16_saturations(uint32_t *count, hipStream_t stream);
 unsigned long long f16_saturations(bool reset);  // f16 hand-over values clamped to +-65504 since the last reset (lanes, not elements); synchronises the device
 hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m, hipStream_t stream);

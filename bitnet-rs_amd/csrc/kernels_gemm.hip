@@ -1474,6 +1474,167 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_h
     f16_chain_epilogue<RT, TTW, 4, EPI == 2>(p, acc, lds, mu_rs, bx, by, rw, c, g, tid);
 }
 
+// ---- few activation rows on the chain -----------------------------------------------------------------------------------------------------------------------
+// A short prompt has few tiles of 128 rows (20 at 2560), and each walks its K steps alone, whatever the bytes: 13 to 17 us a launch of the 2B model's layers at 16 tokens, 30 us of
+// the down-projection, where 2 to 11 MB of weights take under 2 us.
+// Here a workgroup makes RT row tiles of 16 by 16 tokens; its eight waves take the half blocks of 128 columns in turns, operands straight to registers, D half blocks
+// ahead, and add up in LDS in the order of the waves.  The LayerNorm partials it leaves are of 16 rows each: no workgroup has 64.  Bound by the dependent loads and by the tokens'
+// rows, which every workgroup reads for itself: 6.3 (q|k|v), 5 (o), 10.5 (gate|up) and 11 us (down) at 16 tokens; prompt of 16 tokens 2.63 -> 1.44 ms, 64 2.75 -> 2.36.
+// From the two-bit codes: the fp4 image's cheaper expansion is equal here (gate|up 0.2 us behind, o at 96 tokens 0.1 ahead) and twice the bytes.
+template <bool SC, int RT>
+__global__ __launch_bounds__(512, RT == 4 ? 2 : 4) void k_gemm_f16_few(GemmArgs p, uint32_t lut_hi) {
+    constexpr int NW = 8, D = 2, TOK = 16, NG = NW * 64 / TOK, NS = 5;  // NS: partials per thread and batch (160 at K = 2560 are one)
+    __shared__ __attribute__((aligned(16))) uint8_t rows[NW][4096];     // a wave's half block of the tokens
+    __shared__ __attribute__((aligned(16))) gv4f sums[NW][RT][64];
+    __shared__ double red[2 * NW * 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+    int l = blockIdx.x;  // an XCD takes consecutive workgroups, token tiles of the same rows beside each other
+    if ((gridDim.x & 7) == 0) l = (l & 7) * (gridDim.x >> 3) + (l >> 3);
+    const int n_tok = (p.m + TOK - 1) / TOK, bx = l / n_tok, tile0 = bx * RT, tok0 = (l - bx * n_tok) * TOK;
+    const int q = wave & 1;  // this wave's half of its blocks
+    const uint8_t *wbase = p.tiles + (size_t)tile0 * p.nblk * 1024, *bbase = reinterpret_cast<const uint8_t *>(p.planes) + (size_t)tok0 * p.nblk * 512;
+    const uint8_t *sbase = SC ? reinterpret_cast<const uint8_t *>(p.stiles_h) + (size_t)tile0 * p.nblk * 256 : nullptr;
+    const uint32_t woff = lane * 16 + 8 * q, soff = lane * 4;
+    uint32_t boff[4];
+    // A lane's operands are 64 bytes of one token, 128 bytes from the next lane group's: four requests of sixteen bytes each would look up 64 lines apiece.  The rows come in
+    // pieces of 64 bytes instead, four lanes each, and pass through LDS: unit 4 g + u of token c at (4 g + u) ^ c.
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int tok = 4 * i + g, unit = c ^ tok;
+        boff[i] = (uint32_t)tok * p.nblk * 512 + (unit >> 2) * 128 + 64 * q + (unit & 3) * 16;
+    }
+    uint8_t *stage = rows[wave] + lane * 16;
+    const uint8_t *operand = rows[wave] + c * 256;
+    typedef unsigned gv2u __attribute__((ext_vector_type(2)));
+    gv2u w[D][RT];
+    gv4u b[D][4];
+    uint32_t sc[D][RT];
+    auto fetch = [&](int s, int blk) {
+        if (blk >= p.nblk) return;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[s][i] = *reinterpret_cast<const gv4u *>(bbase + (size_t)blk * 512 + boff[i]);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            w[s][r] = *reinterpret_cast<const gv2u *>(wbase + (size_t)(r * p.nblk + blk) * 1024 + woff);
+            sc[s][r] = SC ? *reinterpret_cast<const uint32_t *>(sbase + (size_t)(r * p.nblk + blk) * 256 + soff) : 0u;
+        }
+    };
+    gv4f acc[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r] = (gv4f){0.f, 0.f, 0.f, 0.f};
+    const int first = wave >> 1;
+#pragma unroll
+    for (int s = 0; s < D; ++s) fetch(s, first + 4 * s);
+    float2 st[NS];  // (sum, sum of squares) partials of the input rows
+    const int stok = tid % TOK, sgrp = tid / TOK;
+    const float2 *stats = reinterpret_cast<const float2 *>(p.stats_in) + tok0 + stok;
+    if (p.stats_in)
+#pragma unroll
+        for (int k = 0; k < NS; ++k) st[k] = stats[(size_t)min(sgrp + k * NG, p.n_stats - 1) * p.stats_stride];
+    for (int blk = first; blk < p.nblk; blk += 4 * D) {
+#pragma unroll
+        for (int s = 0; s < D; ++s) {
+            if (blk + 4 * s < p.nblk) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) *reinterpret_cast<gv4u *>(stage + i * 1024) = b[s][i];
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the wave's own LDS accesses come in order)
+                __builtin_amdgcn_wave_barrier();
+                gh8 x[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const gh8 *>(operand + ((4 * g + u) ^ c) * 16);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int r = 0; r < RT; ++r) {
+                        // (s, s) of this lane's 32-block 2 g + q: low / high half of its scale dword
+                        const gh2 s2 = __builtin_bit_cast(gh2, __builtin_amdgcn_perm(0u, sc[s][r], q ? 0x03020302u : 0x01000100u));
+                        const gh8 a = expand8_f16<SC ? 1 : 0>(w[s][r][u >> 1], u & 1, lut_hi, s2);
+                        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, x[u], acc[r], 0, 0, 0);
+                    }
+                fetch(s, blk + 4 * (s + D));
+            }
+        }
+    }
+    if (p.stats_in) {  // this thread's share of a token's partials, in a fixed order
+        double s1 = 0.0, s2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            asm volatile("" : "+v"(st[k].x), "+v"(st[k].y));  // (hipcc converts them where they are requested otherwise, and waits there)
+            const bool in = sgrp + k * NG < p.n_stats;
+            s1 += (double)(in ? st[k].x : 0.0f), s2 += (double)(in ? st[k].y : 0.0f);
+        }
+        for (int i = sgrp + NS * NG; i < p.n_stats; i += NG) {
+            const float2 v = stats[(size_t)i * p.stats_stride];
+            s1 += (double)v.x, s2 += (double)v.y;
+        }
+        red[2 * tid] = s1, red[2 * tid + 1] = s2;
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r) sums[wave][r][lane] = acc[r];
+    __syncthreads();
+    if (wave >= (p.silu_mul ? RT / 2 : RT)) return;  // a wave per output tile: gate and up make one
+    const int r0 = p.silu_mul ? 2 * wave : wave, token = tok0 + c;
+    const bool live = token < p.m;
+    float mean = 0.f, rs = 1.f;
+    if (p.stats_in) {
+        double s1 = 0.0, s2 = 0.0;  // the four lanes of a token share its partials
+#pragma unroll
+        for (int k = 0; k < NG / 4; ++k) {
+            const int i = (g * (NG / 4) + k) * TOK + c;
+            s1 += red[2 * i], s2 += red[2 * i + 1];
+        }
+        s1 += __shfl_xor(s1, 16), s2 += __shfl_xor(s2, 16);
+        s1 += __shfl_xor(s1, 32), s2 += __shfl_xor(s2, 32);
+        const double mean_d = s1 / (double)p.cols, var_d = s2 / (double)p.cols - mean_d * mean_d;
+        mean = (float)mean_d, rs = 1.0f / sqrtf((float)(var_d > 0.0 ? var_d : 0.0) + p.ln_eps);
+    }
+    auto value = [&](int r, float (&v)[4]) {
+        gv4f x = sums[0][r][lane];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) x += sums[k][r][lane];
+        const int row0 = 16 * (tile0 + r) + 4 * g;
+        const gv4f lng = p.stats_in ? *reinterpret_cast<const gv4f *>(p.ln_g + row0) : (gv4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = (x[j] - mean * lng[j]) * rs;
+    };
+    typedef _Float16 fh4 __attribute__((ext_vector_type(4)));
+    bool sat = false;
+    float v[4];
+    value(r0, v);
+    const int ld = p.silu_mul ? p.rows >> 1 : p.rows, row0 = (p.silu_mul ? 16 * ((tile0 + r0) >> 1) : 16 * (tile0 + r0)) + 4 * g;
+    const size_t off = (size_t)(live ? token : 0) * ld + row0;
+    if (p.silu_mul) {
+        float up[4];
+        value(r0 + 1, up);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = gsilu_mul(v[j], up[j]);
+    } else if (p.residual) {
+        const gv4f x = *reinterpret_cast<const gv4f *>(p.residual + off);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += x[j];
+    }
+    if (live) {
+        if (p.y) *reinterpret_cast<gv4f *>(p.y + off) = (gv4f){v[0], v[1], v[2], v[3]};
+        if (p.yh) {
+            const gv4f go = p.gamma_out && !p.silu_mul ? *reinterpret_cast<const gv4f *>(p.gamma_out + row0) : (gv4f){1.f, 1.f, 1.f, 1.f};
+            fh4 o;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = gclamp_f16(v[j] * go[j], sat);
+            *reinterpret_cast<fh4 *>(p.yh + off) = o;
+        }
+    }
+    if (p.stats_out && !p.silu_mul) {
+        float s1 = (v[0] + v[1]) + (v[2] + v[3]), s2 = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+        s1 += __shfl_xor(s1, 16), s2 += __shfl_xor(s2, 16);
+        s1 += __shfl_xor(s1, 32), s2 += __shfl_xor(s2, 32);
+        if (g == 0) *reinterpret_cast<float2 *>(p.stats_out + 2 * ((size_t)(tile0 + r0) * p.stats_stride + token)) = live ? float2{s1, s2} : float2{0.f, 0.f};
+    }
+    gflush_sat(sat);
+}
+
+
 // ================================================================================================================================
 // k_gemm_f16h: k_gemm_f16a's arithmetic on a 64-row x 128-TOKEN wave tile (round 5).  The code expansion is a fixed cost per
 // weight and K step (17 VALU per 8 weights: 544 per wave and step against 128 MFMAs at 64 tokens -- the VALU issue port was the unit closest to
@@ -2508,6 +2669,32 @@ bool gemm_f16_chain_supported(const Weights &w) {
     return true;
 }
 
+// Row tiles per workgroup of k_gemm_f16_few for a caller that allows it (BITNET_HIP_FUSE_FEW_ROWS), 0: the wide tiles are faster.  The fewest that make one round of 256 workgroups;
+// past that two as long as the launch stays under about three rounds (long rows: four), which the wide tiles need longer for.  A launch's us against the wide tiles of the f16 chain,
+// whole prompts of bitnet-b1.58-2B-4T, 1 / 2 / 4 row tiles: o at 16 tokens -7.4 / -6.1 / -5.0, 32 -6.2 / -6.6 / -5.1, 96 -2.1 / -5.0 / -5.6, 128 +0.4 / -1.5 / -0.3, 160 +3.7 /
+// +0.7 / +1.1; q|k|v at 16 -7.4 / -6.7 / -4.8, 64 -1.2 / -4.5 / -5.2, 96 +3.0 / -1.1 / +0.1, 128 +7 / +1.2 / +0.7; down at 16 -18.5 / -16 / -12.5, 96 -7.7 / -12.7 / -13.8,
+// 128 -3.3 / -6.8 / -2.3, 192 +7.3 / -1.6 / -1.5, 256 +15 / +2.7 / +8.6; gate|up at 16 - / -5.2 / -6.4, 32 - / +1.3 / 0, 64 - / +10 / +11.
+static int f16_few_tiles(const Weights &w, bool silu_mul, size_t m) {
+    const size_t tiles = w.rows / 16 * div_ceil(m, 16);
+    for (int rt = silu_mul ? 2 : 1; rt <= 4; rt *= 2)
+        if (tiles / rt <= 256) return rt;
+    return tiles / 2 <= (w.cols > 4096 ? 960 : 720) ? 2 : 0;
+}
+bool gemm_f16_takes_few(const Weights &w, bool silu_mul, size_t m) {
+    return gemm_f16_chain_supported(w) && m > 0 && m <= 4096 && (!silu_mul || w.paired) && f16_few_tiles(w, silu_mul, m) > 0;
+}
+
+static hipError_t launch_gemm_f16_few(const Weights &w, const GemmArgs &a, hipStream_t stream) {
+    const bool scaled = a.stiles_h != nullptr;
+    const int rt = f16_few_tiles(w, a.silu_mul, (size_t)a.m);
+    if (rt == 0) return hipErrorInvalidValue;
+    void (*fk)(GemmArgs, uint32_t) = rt == 4 ? (scaled ? k_gemm_f16_few<true, 4> : k_gemm_f16_few<false, 4>)
+                                   : rt == 2 ? (scaled ? k_gemm_f16_few<true, 2> : k_gemm_f16_few<false, 2>) : scaled ? k_gemm_f16_few<true, 1> : k_gemm_f16_few<false, 1>;
+    g_last_gemm_tile = GemmTileChoice{2, 16, 8, scaled ? 4 : 5, 16 * rt, 0, 16 * rt};
+    hipLaunchKernelGGL(fk, dim3((unsigned)(w.rows / 16 / rt * div_ceil((size_t)a.m, 16))), dim3(512), 0, stream, a, lut_f16_hi(w.lut));
+    return hipGetLastError();
+}
+
 hipError_t launch_rows_to_f16(const float *x, const float *gamma, size_t m, size_t cols, void *xh, float *stats, hipStream_t stream) {
     if (cols % 4 != 0 || m == 0) return hipErrorInvalidValue;
     const size_t m_pad = div_ceil(m, 64) * 64;
@@ -2550,6 +2737,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
     const int ttw = gemm_token_tiles(gx0, m_pad, false, kGemmCUs);
     const bool fmt1 = w.scaled, image = io.image != nullptr;
     a.tiles4 = io.image;
+    if (io.few) return io.qb_out ? hipErrorInvalidValue : launch_gemm_f16_few(w, a, stream);
     const bool rt5 = ttw == 4 && !io.silu_mul && gemm_five_tiles(w.rows, m_pad);
     // Short prompts: waves of 32 rows while the waves of 64 leave most CUs one workgroup.  A K step of such a workgroup is a serial chain (staging, expansion, LDS reads, MFMAs,
     // barrier: 3.2 us at 32 tokens, of which the units are busy a third), so two of half the rows on a CU take less than one.  BitNet32-F16 prompt of bitnet-b1.58-2B-4T, ms with

@@ -619,7 +619,7 @@ bool Decoder::hybrid_applies(size_t n_rows) const {
 
 int Decoder::ensure_chain_buffers(size_t N) {
     const size_t H = c_.hidden, QD = (size_t)c_.n_heads * c_.head_dim, F = c_.ffn;
-    const size_t NP = (N + 63) / 64 * 64, nst = H / 64;
+    const size_t NP = (N + 63) / 64 * 64, nst = H / 16;  // (partials of 64 rows, or of 16 from the form for few rows)
     hipStream_t s = (hipStream_t)stream_;
     if ((int)NP > pfc_cap_) {
         for (void *q : {pf_xh_, pf_atth_, pf_hh_, (void *)pf_stats_})
@@ -642,7 +642,7 @@ int Decoder::ensure_chain_buffers(size_t N) {
 }
 
 int Decoder::prefill_chain_layers(size_t N) {
-    const size_t H = c_.hidden, nst = H / 64;
+    const size_t H = c_.hidden;
     hipStream_t s = (hipStream_t)stream_;
     {
         const int rc = ensure_chain_buffers(N);
@@ -651,18 +651,22 @@ int Decoder::prefill_chain_layers(size_t N) {
     BCHK(bitnet_hip_rows_to_f16_dev(pf_x_, layers_[0].attn_norm, N, H, pf_xh_, pf_stats_, s));
     size_t n_stats = 1;
     const int aflags = (kv_f16_ ? BITNET_HIP_ATTN_CACHE_F16 : 0) | BITNET_HIP_ATTN_OUT_F16;
+    // few rows: the kernel library says for which launches it has the faster form
+    auto few = [&](bitnet_hip_weights_t h, int flags) { return flags | (bitnet_hip_matmul_f16_takes_few_rows(h, N, flags) == 1 ? BITNET_HIP_FUSE_FEW_ROWS : 0); };
     for (size_t l = 0; l < layers_.size(); ++l) {
         auto &L = layers_[l];
-        BCHK(bitnet_hip_matmul_f16_dev(L.qkv, pf_xh_, N, pf_stats_, n_stats, L.attn_norm, c_.eps, pf_qkv_, nullptr, 0, nullptr, nullptr, nullptr, s));
+        BCHK(bitnet_hip_matmul_f16_dev(L.qkv, pf_xh_, N, pf_stats_, n_stats, L.attn_norm, c_.eps, pf_qkv_, nullptr, few(L.qkv, 0), nullptr, nullptr, nullptr, s));
         BCHK(bitnet_hip_attention_prefill_flags_dev(pf_qkv_, rope_sin_, rope_cos_, L.kcache, L.vcache, (size_t)c_.n_heads, (size_t)c_.n_kv_heads,
                                                     (size_t)c_.head_dim, (size_t)c_.max_pos, N, pf_attn_ws_, pf_attn_ws_bytes_, pf_atth_, aflags, s));
-        BCHK(bitnet_hip_matmul_f16_dev(L.o, pf_atth_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, 0, pf_xh_, L.ffn_norm, pf_stats_, s));
-        n_stats = nst;
-        BCHK(bitnet_hip_matmul_f16_dev(L.gateup, pf_xh_, N, pf_stats_, n_stats, L.ffn_norm, c_.eps, nullptr, nullptr, BITNET_HIP_FUSE_SILU_MUL, pf_hh_, nullptr,
+        const int of = few(L.o, 0), df = few(L.down, 0);
+        BCHK(bitnet_hip_matmul_f16_dev(L.o, pf_atth_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, of, pf_xh_, L.ffn_norm, pf_stats_, s));
+        n_stats = of ? H / 16 : H / 64;
+        BCHK(bitnet_hip_matmul_f16_dev(L.gateup, pf_xh_, N, pf_stats_, n_stats, L.ffn_norm, c_.eps, nullptr, nullptr, few(L.gateup, BITNET_HIP_FUSE_SILU_MUL), pf_hh_, nullptr,
                                        nullptr, s));
         const bool last = l + 1 == layers_.size();
-        BCHK(bitnet_hip_matmul_f16_dev(L.down, pf_hh_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, 0, last ? nullptr : pf_xh_,
+        BCHK(bitnet_hip_matmul_f16_dev(L.down, pf_hh_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, df, last ? nullptr : pf_xh_,
                                        last ? nullptr : layers_[l + 1].attn_norm, last ? nullptr : pf_stats_, s));
+        n_stats = df ? H / 16 : H / 64;
     }
     return 0;
 }

@@ -307,6 +307,10 @@ int bitnet_hip_rows_to_f16_dev(const float *x_dev, const float *gamma_dev, size_
 int bitnet_hip_matmul_f16_dev(bitnet_hip_weights_t w, const void *xh_dev, size_t m, const float *stats_in_dev, size_t n_stats,
                               const float *ln_gamma_dev, float ln_eps, float *y_dev, const float *residual_dev, int flags, void *yh_dev,
                               const float *gamma_out_dev, float *stats_out_dev, void *stream);
+/* With BITNET_HIP_FUSE_FEW_ROWS in flags: the form for few activation rows, where bitnet_hip_matmul_f16_takes_few_rows says that it is the faster one (else the call is
+ * refused).  The same product with its sums in another order, and stats_out holds [rows / 16][m up to 64] partials, of 16 rows each. */
+#define BITNET_HIP_FUSE_FEW_ROWS 128
+int bitnet_hip_matmul_f16_takes_few_rows(bitnet_hip_weights_t w, size_t m, int flags);
 
 /* QB32 ACTIVATIONS (round 5): the producer-quantised input of the fp6 x fp4 prompt matmul -- what QAct is to the decode GEMV.  The digit forms'
  * row quantiser needs the row maximum, which no producing workgroup has, so it stayed a launch of its own (two per layer, 6 % of the QK256

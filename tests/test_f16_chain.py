@@ -370,3 +370,64 @@ def test_chain_on_the_image_is_the_expanding_one_bit_for_bit(hip, torch_, fmt, r
         assert a is None or (torch_.isfinite(a).all() and torch_.equal(a, b))
     for w in (h, *parts):
         hip.weights_free(w)
+
+
+FEW_ROWS = 128
+
+
+# rows x cols x tokens: one, two and four row tiles per workgroup, one block of K (waves without work) to 27, whole and ragged token tiles, pairs
+@pytest.mark.parametrize("fmt", ["qk256", "i2s"])
+@pytest.mark.parametrize("rows,cols,m,silu,tile", [(256, 256, 1, 0, 16), (2560, 2560, 16, 0, 16), (2560, 768, 17, 0, 32), (2560, 6912, 100, 0, 32), (3840, 2304, 64, 0, 64), (13824, 512, 16, 1, 64),
+                                                   (512, 2560, 5, 1, 32), (2560, 1024, 1, 0, 16)])
+def test_f16_chain_few_rows(hip, torch_, fmt, rows, cols, m, silu, tile):
+    """The form for few rows behind a LayerNorm (partials of 16 and of 64 columns, and one), its residual, f16 copy and partials of 16 rows, against float64."""
+    rng = np.random.default_rng(rows + cols + m)
+    parts = [make_matrix(hip, rng, fmt, rows // 2, cols) for _ in range(2)]
+    h, mp, out = hip.weights_concat([a for a, _ in parts], interleave16=bool(silu)), -(-m // 64) * 64, rows // 2 if silu else rows
+    gamma, eps = rng.uniform(0.5, 1.5, cols).astype(np.float32), 1e-5
+    gd = torch_.from_numpy(gamma).cuda()
+    hip.weights_bind_ln(h, gd)
+    x = (rng.normal(0, 1, (m, cols)) * np.exp(rng.uniform(-1, 1, (m, 1))) + 0.3).astype(np.float32)
+    xh = torch_.zeros(mp, cols, dtype=torch_.float16, device="cuda")
+    xh[:m] = torch_.from_numpy((x * gamma).astype(np.float16)).cuda()
+    flags = (1 if silu else 0) | FEW_ROWS
+    assert hip.matmul_f16_takes_few_rows(h, m, flags)
+    w = np.concatenate([d for _, d in parts])
+    xd, x16 = x.astype(np.float64), (x * gamma).astype(np.float16).astype(np.float64)
+    mean, denom = xd.mean(1, keepdims=True), np.sqrt(xd.var(1, keepdims=True) + eps)
+    g64 = w @ gamma.astype(np.float64)
+    plain = (x16 @ w.T - mean * g64) / denom  # f16 inputs are given: accumulation order, and the f32 of mean * g
+    mag = (np.abs(x16) @ np.abs(w).T + np.abs(mean) * np.abs(g64)) / denom + 1e-6
+    res, gout = rng.normal(0, 1, (m, rows)).astype(np.float32), rng.uniform(0.5, 1.5, rows).astype(np.float32)
+    for part in (16, 64, cols):
+        n = cols // part
+        st = torch_.zeros(n, mp, 2, device="cuda")
+        sums = xd.reshape(m, n, part)
+        st[:, :m] = torch_.from_numpy(np.stack([sums.sum(2).T, (sums ** 2).sum(2).T], 2).astype(np.float32)).cuda()
+        yh = torch_.full((mp, out), 7.0, dtype=torch_.float16, device="cuda")
+        so = torch_.full((rows // 16, mp, 2), 7.0, device="cuda")
+        if silu:
+            hip.matmul_f16_dev(h, xh, m, stats_in=st, n_stats=n, ln_gamma=gd, ln_eps=eps, flags=flags, yh=yh)
+        else:
+            y = torch_.from_numpy(res).cuda()
+            hip.matmul_f16_dev(h, xh, m, stats_in=st, n_stats=n, ln_gamma=gd, ln_eps=eps, y=y, residual=y, flags=flags, yh=yh, gamma_out=torch_.from_numpy(gout).cuda(), stats_out=so)
+        torch_.cuda.synchronize()
+        assert hip.matmul_last_workgroup_rows() == tile and hip.matmul_last_tile()["wave_tokens"] == 16
+        if silu:
+            a, b = plain[:, :out], plain[:, out:]
+            want = a / (1 + np.exp(-a)) * b
+            # the product's 4e-6 through silu * up (slope at most 1.1), and the result's f16
+            assert np.all(np.abs(yh[:m].cpu().numpy() - want) <= 1.1 * 4e-6 * (mag[:, :out] * np.abs(b) + mag[:, out:] * np.abs(a)) + 2.0 ** -11 * np.abs(want) + 1e-6)
+        else:
+            got = y.cpu().numpy()
+            assert np.all(np.abs(got - (res + plain)) <= 4e-6 * (mag + np.abs(res)))
+            assert np.array_equal(yh[:m].cpu().numpy(), (got * gout).astype(np.float16))
+            s, slabs = so.cpu().numpy(), got.reshape(m, rows // 16, 16).astype(np.float64)
+            for e in (1, 2):  # f32 sums of 16 terms
+                assert np.all(np.abs(s[:, :m, e - 1].T - (slabs ** e).sum(axis=2)) <= 1e-6 * (np.abs(slabs) ** e).sum(axis=2) + 1e-6)
+            assert np.all(s[:, m:-(-m // 16) * 16] == 0)
+    most = next(k for k in range(m, 5000) if not hip.matmul_f16_takes_few_rows(h, k, flags))
+    with pytest.raises(Exception, match="FEW_ROWS"):
+        hip.matmul_f16_dev(h, torch_.zeros(-(-most // 64) * 64, cols, dtype=torch_.float16, device="cuda"), most, yh=torch_.zeros(-(-most // 64) * 64, out, dtype=torch_.float16, device="cuda"), flags=flags)
+    for a in (h, *(a for a, _ in parts)):
+        hip.weights_free(a)
