@@ -372,24 +372,79 @@ hipError_t launch_gqa_any(const Gqa &g, const void *q, size_t ldq, int q_f32, in
 // lane's weights of both tiles are the eight consecutive keys 8 g .. 8 g + 7 which it needs as an operand of O^T = V^T P^T.
 // Exponentials are the hardware's: exp2f scales its argument and result so that what lies under 2^-126 of the largest weight stays a number; here it is zero, which no sum that
 // holds a one can tell.  12 and 24 heads of two maps of 64 / 128 columns, 200 and 1000 keys: 9.4 -> 9.1 us; one map of 128 / 128: 8.25 -> 8.05.
+// The launch is a chain of latencies (150 and 2090 keys take the same): arguments -> position -> rotation and keys -> scores -> weights -> output.  Hence: what the host knows is
+// divided there (64-bit divisions by arguments were a quarter of the launch), all arguments are requested at once, raw rows and norms' weights ahead of the position, and the
+// new key's row is one more of the rows that the waves share out.  Beside another launch, 12 heads of 128 / 128 at 2090 keys 8.6 -> 6.2 us, 24 of two maps of 64 / 128 at 216 keys 12.2 -> 10.2.
+struct GqaStepK {
+    const float *row, *q_weight, *k_weight, *q_factor, *rope_cos, *rope_sin, *far_weight, *far_rate;
+    const int *pos;
+    uint16_t *K, *V;
+    float *scratch, eps;
+    int heads, group, dim, dimp, vdimp, capacity, turned, chunk, window, normed, append, k_at, v_at;  // normed: 1 queries, 2 keys
+};
+
 template <int NK, int NV, int MAPS>
-__global__ __launch_bounds__(256, NV > 8 || NK * MAPS >= 8 ? 1 : 2) void k_gqa_step(Gqa p, GqaStep a) {
+__global__ __launch_bounds__(256, NV > 8 || NK * MAPS >= 8 ? 1 : 2) void k_gqa_step(GqaStepK p) {
     extern __shared__ __attribute__((aligned(16))) float area[];  // queries [maps][16][NK * 32]; then the waves' outputs
     __shared__ float sm[4][MAPS][16], sl[4][MAPS][16];
     __shared__ __attribute__((aligned(16))) uint16_t newk[MAPS][NK * 32], newv[NV * 16];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
-    const int group = (int)(p.heads / p.kv_heads), ht = (group + 15) / 16, kv = blockIdx.y / ht, h0 = kv * group + (blockIdx.y - kv * ht) * 16;
-    const int nh = min(16, (kv + 1) * group - h0), dim = (int)p.dim, dimp = (int)p.dimp, vdimp = (int)p.vdimp;
-    constexpr int QS = NK * 32 + 4;
-    const int pos = *a.pos, n_keys = pos + 1;
-    const GqaRange range = gqa_range(p, pos);
+    // (every argument at once: read where they are used they are a chain of scalar loads)
+    asm volatile("" ::"s"(p.row), "s"(p.q_weight), "s"(p.k_weight), "s"(p.q_factor), "s"(p.rope_cos), "s"(p.rope_sin), "s"(p.far_weight), "s"(p.far_rate), "s"(p.pos), "s"(p.K), "s"(p.V),
+                 "s"(p.scratch), "s"(p.eps), "s"(p.heads), "s"(p.group), "s"(p.dim), "s"(p.dimp), "s"(p.vdimp), "s"(p.capacity), "s"(p.turned), "s"(p.chunk), "s"(p.window), "s"(p.normed),
+                 "s"(p.append), "s"(p.k_at), "s"(p.v_at));
+    const int posv = *p.pos;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
+    const int kv = blockIdx.z, first_head = blockIdx.y * 16, h0 = kv * p.group + first_head, nh = min(16, p.group - first_head);
+    const int dimp = p.dimp, vdimp = p.vdimp;
+    constexpr int QS = NK * 32 + 4, J = (NK + 1) / 2, QR = NK > 4 ? 1 : 4;  // QR: rows of a wave at a time
+    uint16_t *K = p.K + (size_t)kv * MAPS * p.capacity * dimp, *V = p.V + (size_t)kv * vdimp * p.capacity;
+    // row i of a wave: of the only map, or of its own of two
+    const int map = MAPS == 2 ? wave & 1 : 0;
+    auto head_of = [&](int i) { return MAPS == 2 ? (wave >> 1) + 2 * i : wave + 4 * i; };
+    const bool keys = 3 - wave < MAPS && p.append;  // this wave's row of the new key: map 3 - wave
+    float qv[QR][J], kv_[J], wq[J], wk[J];
+    auto rows = [&](int i0) {
+#pragma unroll
+        for (int i = 0; i < QR; ++i)
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                const float v = p.row[((size_t)(h0 + min(head_of(i0 + i), nh - 1)) * MAPS + map) * dimp + min(lane + 64 * j, dimp - 1)];
+                qv[i][j] = lane + 64 * j < dimp ? v : 0.f;
+            }
+    };
+    rows(0);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int at = min(lane + 64 * j, p.dim - 1);
+        kv_[j] = 0.f, wq[j] = wk[j] = 1.0f;
+        if (keys && lane + 64 * j < dimp) kv_[j] = p.row[p.k_at + (kv * MAPS + 3 - wave) * dimp + lane + 64 * j];
+        if (p.q_weight) wq[j] = p.q_weight[at];
+        if (p.k_weight) wk[j] = p.k_weight[at];
+    }
+    float raw_v = 0.f;
+    if (p.append && tid < vdimp) raw_v = p.row[p.v_at + kv * vdimp + tid];  // (vdimp <= 256)
+    const int pos = __builtin_amdgcn_readfirstlane(posv), n_keys = pos + 1;
+    struct {
+        int first, base, per, used;
+    } range;  // gqa_range
+    range.first = p.chunk ? pos - (int)((unsigned)pos % (unsigned)p.chunk) : 0;
+    if (p.window && pos - p.window + 1 > range.first) range.first = pos - p.window + 1;
+    range.base = range.first & ~(kGqaTile - 1);
+    const int tiles = (n_keys - range.base + kGqaTile - 1) / kGqaTile;
+    range.per = (tiles + kGqaSplits - 1) / kGqaSplits;
+    range.used = range.per == 1 ? tiles : (tiles + range.per - 1) / range.per;
     if ((int)blockIdx.x >= range.used) return;
     const int k0 = range.base + blockIdx.x * range.per * kGqaTile, k1 = min(k0 + range.per * kGqaTile, n_keys);
-    uint16_t *K = (uint16_t *)p.kcache + (size_t)kv * MAPS * p.capacity * dimp, *V = (uint16_t *)p.vcache + (size_t)kv * vdimp * p.capacity;
-    const float *kraw = a.row + (p.heads * MAPS + (size_t)kv * MAPS) * dimp,
-                *vraw = p.values_are_keys ? kraw : a.row + (p.heads + p.kv_heads) * MAPS * dimp + (size_t)kv * vdimp;
-    const int turned = (int)p.rot_dims;
-    const float *cs = p.rope_cos + (size_t)pos * (turned >> 1), *sn = p.rope_sin + (size_t)pos * (turned >> 1);
+    float cs[J], sn[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        cs[j] = 1.0f, sn[j] = 0.f;
+        if (p.turned && 64 * j < p.turned) {
+            const size_t at = (size_t)pos * (p.turned >> 1) + (min(lane + 64 * j, p.turned - 1) >> 1);
+            cs[j] = p.rope_cos[at], sn[j] = p.rope_sin[at];
+        }
+    }
+    const float factor = p.q_factor[pos];
     u32x4 kf[2][MAPS][NK], vf[NV];
     auto fetch = [&](int kb) {  // (blocks lie below the capacity, a multiple of 128)
 #pragma unroll
@@ -403,62 +458,55 @@ __global__ __launch_bounds__(256, NV > 8 || NK * MAPS >= 8 ? 1 : 2) void k_gqa_s
         for (int v = 0; v < NV; ++v) vf[v] = *reinterpret_cast<const u32x4 *>(V + (size_t)min(v * 16 + r16, vdimp - 1) * p.capacity + kb + g * 8);
     };
     constexpr bool kAhead = NK <= 4;  // the first block is requested ahead of the norms (registers allow it)
-    const bool owner = k1 == n_keys && !p.queries_only;
+    const bool owner = k1 == n_keys && p.append;
     if (kAhead) fetch(k0 + wave * 32);
+    // a row's element lane + 64 j: norm, weight, rotation by pairs of neighbours
+    auto finished = [&](float v, float norm, float weight, int j) {
+        const int i = lane + 64 * j;
+        const float t = v * norm * (i < p.dim ? weight : 1.0f);
+        if (!p.turned) return t;
+        const float o = dpp<0xb1>(t);  // quad_perm [1,0,3,2]
+        return i >= p.turned ? t : (i & 1) ? t * cs[j] + o * sn[j] : t * cs[j] - o * sn[j];
+    };
+    auto norm_of = [&](const float (&v)[J], bool normed) {
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < J; ++j) ss += v[j] * v[j];
+        return normed ? 1.0f / sqrtf(wave_sum(ss) / (float)p.dim + p.eps) : 1.0f;
+    };
     if (owner) {  // the record that holds the new position appends it (and puts it into its own fragments below)
-        if (wave < MAPS) {
-            float v[NK], ss = 0.f;
+        if (keys) {
+            const float norm = norm_of(kv_, p.normed & 2);
 #pragma unroll
-            for (int j = 0; j < (NK + 1) / 2; ++j) {
-                v[j] = lane + 64 * j < dimp ? kraw[wave * dimp + lane + 64 * j] : 0.f;
-                ss += v[j] * v[j];
-            }
-            const float norm = p.k_weight || p.unit_norm ? 1.0f / sqrtf(wave_sum(ss) / (float)dim + p.eps) : 1.0f;
-#pragma unroll
-            for (int j = 0; j < (NK + 1) / 2; ++j) {
+            for (int j = 0; j < J; ++j) {
                 const int i = lane + 64 * j;
-                float k = v[j] * norm * (p.k_weight && i < dim ? p.k_weight[i] : 1.0f);
-                if (turned) k = turn_neighbours(k, i, cs, sn, turned);
+                const float k = finished(kv_[j], norm, wk[j], j);
                 if (i < dimp) {
                     const uint16_t b = f2bf(k);
-                    K[((size_t)wave * p.capacity + pos) * dimp + i] = b;
-                    newk[wave][i] = b;
+                    K[((size_t)(3 - wave) * p.capacity + pos) * dimp + i] = b;
+                    newk[3 - wave][i] = b;
                 }
             }
         }
-        for (int i = tid; i < vdimp; i += 256) {
-            const uint16_t b = f2bf(vraw[i]);
-            V[(size_t)i * p.capacity + pos] = b;
-            newv[i] = b;
+        if (tid < vdimp) {
+            const uint16_t b = f2bf(raw_v);
+            V[(size_t)tid * p.capacity + pos] = b;
+            newv[tid] = b;
         }
     }
-    {
-        const float factor = p.q_factor[pos];
-        for (int r = wave; r < MAPS * 16; r += 4) {
-            const int map = r >> 4, hh = r & 15;
-            if (hh >= nh) {
-                for (int i = lane; i < NK * 32; i += 64) area[r * QS + i] = 0.f;
-                continue;
-            }
-            const float *q = a.row + ((size_t)(h0 + hh) * MAPS + map) * dimp;
-            float v[NK], ss = 0.f;
+    for (int i0 = 0; head_of(i0) < nh; i0 += QR) {
+        if (i0) rows(i0);
 #pragma unroll
-            for (int j = 0; j < (NK + 1) / 2; ++j) {
-                v[j] = lane + 64 * j < dimp ? q[lane + 64 * j] : 0.f;
-                ss += v[j] * v[j];
-            }
-            const float norm = (p.q_weight || p.unit_norm ? 1.0f / sqrtf(wave_sum(ss) / (float)dim + p.eps) : 1.0f) * factor;
+        for (int i = 0; i < QR; ++i) {
+            if (head_of(i0 + i) >= nh) continue;
+            const float norm = norm_of(qv[i], p.normed & 1) * factor;
 #pragma unroll
-            for (int j = 0; j < (NK + 1) / 2; ++j) {
-                const int i = lane + 64 * j;
-                float t = v[j] * norm * (p.q_weight && i < dim ? p.q_weight[i] : 1.0f);
-                if (turned) t = turn_neighbours(t, i, cs, sn, turned);
-                if (i < NK * 32) area[r * QS + i] = t;
-            }
+            for (int j = 0; j < J; ++j)
+                if (lane + 64 * j < NK * 32) area[(map * 16 + head_of(i0 + i)) * QS + lane + 64 * j] = finished(qv[i][j], norm, wq[j], j);
         }
     }
     __syncthreads();
-    SplitFrag q[MAPS][NK];
+    SplitFrag q[MAPS][NK];  // (lanes past the last head: whatever lies there; a column of the products is a head of its own)
 #pragma unroll
     for (int m = 0; m < MAPS; ++m)
 #pragma unroll
@@ -466,8 +514,8 @@ __global__ __launch_bounds__(256, NV > 8 || NK * MAPS >= 8 ? 1 : 2) void k_gqa_s
             const float *src = area + (m * 16 + r16) * QS + kk * 32 + g * 8;
             q[m][kk] = split8(*reinterpret_cast<const f32x4 *>(src), *reinterpret_cast<const f32x4 *>(src + 4));
         }
-    __syncthreads();  // (the area is used again)
-    const FarPenalty far = far_penalty(p, min(h0 + r16, (int)p.heads - 1));
+    FarPenalty far{0.f, 0.f};
+    if (p.far_weight) far.weight = p.far_weight[min(h0 + r16, p.heads - 1)] * 0.69314718055994531f, far.rate = p.far_rate[min(h0 + r16, p.heads - 1)];
     f32x4 o[NV][MAPS];
     float m[MAPS], l[MAPS];
 #pragma unroll
@@ -558,16 +606,17 @@ __global__ __launch_bounds__(256, NV > 8 || NK * MAPS >= 8 ? 1 : 2) void k_gqa_s
                 if (v * 16 < vdimp) *reinterpret_cast<f32x4 *>(area + ((size_t)(wave * MAPS + j) * nh + r16) * vdimp + v * 16 + g * 4) = o[v][j] * w;
     }
     __syncthreads();
-    const int v4 = vdimp / 4, rows = MAPS * nh;
-    for (int i = tid; i < rows * v4; i += 256) {
-        const int r = i / v4, c = (i - r * v4) * 4, j = r / nh, hh = r - j * nh;
-        const float *src = area + (size_t)r * vdimp + c;
-        const size_t step = (size_t)rows * vdimp;
-        const f32x4 sum = (*reinterpret_cast<const f32x4 *>(src) + *reinterpret_cast<const f32x4 *>(src + step)) +
-                          (*reinterpret_cast<const f32x4 *>(src + 2 * step) + *reinterpret_cast<const f32x4 *>(src + 3 * step));
-        float *rec = a.scratch + ((size_t)((h0 + hh) * MAPS + j) * kGqaSplits + blockIdx.x) * (kGqaRecHead + vdimp);
-        *reinterpret_cast<f32x4 *>(rec + kGqaRecHead + c) = sum;
-        if (c == 0) {
+    const int n_rows = MAPS * nh;
+    for (int r = tid >> 5; r < n_rows; r += 8) {
+        const int j = MAPS == 2 && r >= nh ? 1 : 0, hh = r - j * nh;
+        float *rec = p.scratch + ((size_t)((h0 + hh) * MAPS + j) * kGqaSplits + blockIdx.x) * (kGqaRecHead + vdimp);
+        for (int c = (tid & 31) * 4; c < vdimp; c += 128) {
+            const float *src = area + (size_t)r * vdimp + c;
+            const size_t step = (size_t)n_rows * vdimp;
+            *reinterpret_cast<f32x4 *>(rec + kGqaRecHead + c) = (*reinterpret_cast<const f32x4 *>(src) + *reinterpret_cast<const f32x4 *>(src + step)) +
+                                                                (*reinterpret_cast<const f32x4 *>(src + 2 * step) + *reinterpret_cast<const f32x4 *>(src + 3 * step));
+        }
+        if ((tid & 31) == 0) {
             const float M = fmaxf(fmaxf(sm[0][j][hh], sm[1][j][hh]), fmaxf(sm[2][j][hh], sm[3][j][hh]));
             float L = 0.f;
 #pragma unroll
@@ -586,7 +635,14 @@ static hipError_t step_go(const Gqa &g, const GqaStep &a, hipStream_t s) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(fn, dim3(splits, g.kv_heads * ((group + 15) / 16)), dim3(256), lds, s, g, a);
+    GqaStepK k;
+    k.row = a.row, k.q_weight = g.q_weight, k.k_weight = g.k_weight, k.q_factor = g.q_factor, k.rope_cos = g.rope_cos, k.rope_sin = g.rope_sin, k.far_weight = g.far_weight;
+    k.far_rate = g.far_rate, k.pos = a.pos, k.K = (uint16_t *)g.kcache, k.V = (uint16_t *)g.vcache, k.scratch = a.scratch, k.eps = g.eps, k.heads = (int)g.heads, k.group = group;
+    k.dim = (int)g.dim, k.dimp = (int)g.dimp, k.vdimp = (int)g.vdimp, k.capacity = (int)g.capacity, k.turned = (int)g.rot_dims, k.append = !g.queries_only;
+    k.chunk = g.chunk < g.capacity ? (int)g.chunk : 0, k.window = g.window < g.capacity ? (int)g.window : 0;  // (as large as the cache: no position has keys outside)
+    k.normed = (g.q_weight || g.unit_norm ? 1 : 0) | (g.k_weight || g.unit_norm ? 2 : 0);
+    k.k_at = (int)(g.heads * g.maps * g.dimp), k.v_at = g.values_are_keys ? k.k_at : (int)((g.heads + g.kv_heads) * g.maps * g.dimp);
+    hipLaunchKernelGGL(fn, dim3(splits, (group + 15) / 16, g.kv_heads), dim3(256), lds, s, k);
     return hipGetLastError();
 }
 
