@@ -625,6 +625,15 @@ def test_route(hip, pkg, m, experts, top, tile):
         assert np.array_equal(expert_of[slots], ids.reshape(-1))
 
 
+# one workgroup for choices and plan: a full one, one token past its last, rows and whole waves of lanes
+@pytest.mark.parametrize("m,experts,top,tile", [(64, 64, 8, 64), (65, 64, 8, 128), (63, 100, 5, 64), (5, 100, 16, 64), (16, 200, 20, 64), (17, 200, 20, 64), (16, 1024, 32, 64), (15, 300, 4, 64),
+                                               (64, 16, 16, 64)])
+def test_route_in_one_workgroup(hip, pkg, m, experts, top, tile):
+    test_route(hip, pkg, m, experts, top, tile)
+    if experts > 2 * top:
+        test_corrected_route(hip, pkg, m, experts - 3, 3, top, tile)
+
+
 @pytest.mark.parametrize("m,experts,top,tile", [(1, 4, 2, 64), (2, 6, 3, 64), (130, 5, 2, 64), (300, 6, 4, 128), (90, 40, 3, 128)])
 @pytest.mark.parametrize("width,ff", [(112, 24), (256, 136)])
 @pytest.mark.parametrize("f32", [True, False])
