@@ -55,7 +55,14 @@ __device__ __forceinline__ float delta_token(StepLds &w, float (&s)[NJ], int dim
     float o = 0.f;
     if (tid < vdimp) {
         a = b = 0.f;
-        for (int i = 0; i < SL; ++i) a += w.a[i * vdimp + tid], b += w.b[i * vdimp + tid];
+        constexpr int AH = 8;  // slices in flight
+        for (int i0 = 0; i0 < SL; i0 += AH) {
+            float x[AH], y[AH];
+#pragma unroll
+            for (int i = 0; i < AH; ++i) x[i] = w.a[min(i0 + i, SL - 1) * vdimp + tid], y[i] = w.b[min(i0 + i, SL - 1) * vdimp + tid];
+#pragma unroll
+            for (int i = 0; i < AH; ++i) a += i0 + i < SL ? x[i] : 0.f, b += i0 + i < SL ? y[i] : 0.f;
+        }
         const float u = beta * (w.v[tid] - g * a);
         w.u[tid] = u;
         o = g * b + kq * u;
@@ -79,18 +86,22 @@ __device__ __forceinline__ float head_sum(float v, float *slot) {
     return (slot[0] + slot[1]) + (slot[2] + slot[3]);
 }
 
+// A chain of latencies like the attention's step: what the host knows is divided there (shift: log2 of vdimp, or -1), the grid holds the key head and the head within it, and slices meet
+// in LDS eight at a time: 24 heads of 128 / 128 inside a step 8.4 -> 7.7 us.
 template <int NJ>
-__global__ __launch_bounds__(kStepThreads) void k_delta_step(Delta p, const float *row, const float *ba, const int *pos_ptr, float *out) {
+__global__ __launch_bounds__(kStepThreads) void k_delta_step(Delta p, int SL, int shift, const float *row, const float *ba, const int *pos_ptr, float *out) {
     __shared__ StepLds w;
-    const int tid = threadIdx.x, h = blockIdx.x, heads = (int)p.heads, kvh = (int)p.kv_heads, dimp = (int)p.dimp, vdimp = (int)p.vdimp, taps = (int)p.taps;
-    const int per = heads / kvh, kv = h / per, C = 2 * kvh * dimp + heads * vdimp;
-    const int SL = kStepThreads / vdimp, sl = tid / vdimp, v = tid - sl * vdimp;
+    const int tid = threadIdx.x, per = gridDim.x, kv = blockIdx.y, h = kv * per + blockIdx.x, heads = (int)p.heads, kvh = (int)p.kv_heads, dimp = (int)p.dimp, vdimp = (int)p.vdimp,
+              taps = (int)p.taps, C = 2 * kvh * dimp + heads * vdimp;
+    const int pos = *pos_ptr;
+    const int sl = shift >= 0 ? tid >> shift : tid / vdimp, v = tid - sl * vdimp;
     const bool live = sl < SL;
     float *st = p.state + (size_t)h * dimp * vdimp;
     float s[NJ];
 #pragma unroll
     for (int j = 0; j < NJ; ++j) s[j] = live && sl + SL * j < dimp ? st[(size_t)(sl + SL * j) * vdimp + v] : 0.f;
-    const int part = tid >> 8, c = tid & 255, pos = *pos_ptr;
+    const int part = tid >> 8, c = tid & 255;
+    const int newest = (taps & (taps - 1)) == 0 ? pos & (taps - 1) : (int)((unsigned)pos % (unsigned)taps);  // the position's place in the ring
     const int off = part == 0 ? kv * dimp + c : part == 1 ? (kvh + kv) * dimp + c : 2 * kvh * dimp + h * vdimp + c;
     const float gate = row[C + (size_t)h * vdimp + min(tid, vdimp - 1)], weight = p.norm[min(tid, vdimp - 1)], araw = ba[heads + h], braw = ba[h];
     float y = 0.f;
@@ -104,14 +115,14 @@ __global__ __launch_bounds__(kStepThreads) void k_delta_step(Delta p, const floa
             for (int e = 0; e < AH; ++e) {
                 const int j = min(j0 + e, taps - 1);
                 f[e] = p.conv[(size_t)(taps - 1 - j) * C + off];
-                in[e] = p.ring[(size_t)((pos - j + taps) % taps) * C + off];
+                in[e] = p.ring[(size_t)(newest >= j ? newest - j : newest - j + taps) * C + off];
             }
 #pragma unroll
             for (int e = 0; e < AH; ++e)
                 if (j0 + e < taps && j0 + e <= pos) y += f[e] * in[e];
         }
         // (the slot written is none of those read: taps slots, taps - 1 earlier tokens)
-        if (part == 2 || h == kv * per) p.ring[(size_t)(pos % taps) * C + off] = x;
+        if (part == 2 || h == kv * per) p.ring[(size_t)newest * C + off] = x;
         y = silu(y);
     }
     const float ss = wave_sum(part < 2 ? y * y : 0.f);
@@ -181,7 +192,8 @@ hipError_t launch_delta_step(const Delta &d, const float *row, const float *ba, 
     if (!delta_supported((int)d.dimp, (int)d.vdimp)) return hipErrorInvalidValue;
     const int nj = step_keys(d);
     auto fn = nj <= 4 ? k_delta_step<4> : nj <= 16 ? k_delta_step<16> : nj <= 32 ? k_delta_step<32> : k_delta_step<64>;
-    hipLaunchKernelGGL(fn, dim3(d.heads), dim3(kStepThreads), 0, s, d, row, ba, pos, out);
+    const int vdimp = (int)d.vdimp, shift = (vdimp & (vdimp - 1)) == 0 ? __builtin_ctz(vdimp) : -1;
+    hipLaunchKernelGGL(fn, dim3(d.heads / d.kv_heads, d.kv_heads), dim3(kStepThreads), 0, s, d, kStepThreads / vdimp, shift, row, ba, pos, out);
     return hipGetLastError();
 }
 

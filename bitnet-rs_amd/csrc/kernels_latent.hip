@@ -16,7 +16,7 @@ namespace bitnet_hip {
 __device__ __forceinline__ void split_range(int n_keys, int &per, int &used) {
     const int tiles = (n_keys + kLatentTile - 1) / kLatentTile;
     per = (tiles + kLatentSplits - 1) / kLatentSplits;
-    used = (tiles + per - 1) / per;
+    used = per == 1 ? tiles : (tiles + per - 1) / per;
 }
 
 // element i of the rotated part of a query head (raw part at q); elements past 2 * half are zero
@@ -307,7 +307,9 @@ hipError_t launch_latent_decode(const LatentAttn &a, hipStream_t s) {
 }
 
 // ---- the records of a head -> its value vector --------------------------------------------------------------------------
-// Every workgroup merges the head's records (running maxima, sums, the sink) in LDS and takes a share of W_uv's rows.
+// Every workgroup merges the head's records (running maxima, sums, the sink) in LDS and takes a share of W_uv's rows.  The position is wanted last: the records' first numbers and
+// vectors are requested whether they are used or not (scratch has room for all of them), and so are the wave's first rows of W_uv.  Inside
+// a step, 20 heads at 61 to 85 keys: 5.2 -> 4.6 us.
 template <class TO>
 __global__ __launch_bounds__(512) void k_latent_merge(LatentMerge p) {
     extern __shared__ __attribute__((aligned(16))) float o[];  // [ldc], then four partial vectors
@@ -315,18 +317,31 @@ __global__ __launch_bounds__(512) void k_latent_merge(LatentMerge p) {
     __shared__ float ws[kLatentSplits], sden;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = blockIdx.x, qi = blockIdx.z;
-    int per, used;
-    split_range(*p.pos + p.q0 + qi + 1, per, used);
+    const int posv = *p.pos;
     const size_t stride = kLatentRecHead + p.ldc;
     const float *rec = p.scratch + ((size_t)qi * p.heads + h) * kLatentSplits * stride;
+    const int share = (p.vdimp + gridDim.y - 1) / gridDim.y, v0 = blockIdx.y * share, v1 = min(v0 + share, p.vdimp);
+    constexpr int AW = 4, AR = 2;  // rows of W_uv, records per group
+    u32x4 uw[AW];
+#pragma unroll
+    for (int j = 0; j < AW; ++j) uw[j] = *reinterpret_cast<const u32x4 *>(p.uv + ((size_t)h * p.vdimp + min(v0 + wave + 8 * j, p.vdimp - 1)) * p.ldc + min(lane * 8, p.ldc - 8));
+    const int grp = tid >> 7, t = tid & 127;
+    f32x4 ahead[AR];
+#pragma unroll
+    for (int j = 0; j < AR; ++j) ahead[j] = *reinterpret_cast<const f32x4 *>(rec + (grp + 4 * j) * stride + kLatentRecHead + min(t * 4, p.ldc - 4));
+    float mv[2] = {-INFINITY, -INFINITY}, lv[2] = {0.f, 0.f};
+    if (wave == 0)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) mv[e] = rec[(lane + 64 * e) * stride], lv[e] = rec[(lane + 64 * e) * stride + 1];
+    const float sink = p.sink ? p.sink[h] : -INFINITY;
+    int per, used;
+    split_range(posv + p.q0 + qi + 1, per, used);
     if (wave == 0) {
-        const float sink = p.sink ? p.sink[h] : -INFINITY;
-        float mv[2], lv[2], M = sink;
+        float M = sink;
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            const int r = lane + 64 * e;
-            mv[e] = r < used ? rec[r * stride] : -INFINITY;
-            lv[e] = r < used ? rec[r * stride + 1] : 0.f;
+            const bool live = lane + 64 * e < used;
+            mv[e] = live ? mv[e] : -INFINITY, lv[e] = live ? lv[e] : 0.f;
             M = fmaxf(M, mv[e]);
         }
         M = rows_max(row_max(M));
@@ -342,31 +357,46 @@ __global__ __launch_bounds__(512) void k_latent_merge(LatentMerge p) {
     }
     __syncthreads();
     float *part = o + p.ldc;
-    const int grp = tid >> 7, t = tid & 127;
     for (int i = t * 4; i < p.ldc; i += 512) {
         f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
+        int r = grp;
+        if (i == t * 4) {
+#pragma unroll
+            for (int j = 0; j < AR; ++j)
+                if (grp + 4 * j < used) a += ws[grp + 4 * j] * ahead[j];
+            r += 4 * AR;
+        }
 #pragma unroll 16
-        for (int r = grp; r < used; r += 4) a += ws[r] * *reinterpret_cast<const f32x4 *>(rec + r * stride + kLatentRecHead + i);
+        for (; r < used; r += 4) a += ws[r] * *reinterpret_cast<const f32x4 *>(rec + r * stride + kLatentRecHead + i);
         *reinterpret_cast<f32x4 *>(part + grp * p.ldc + i) = a;
     }
     __syncthreads();
     const float inv = 1.0f / sden;
     for (int i = tid; i < p.ldc; i += 512) o[i] = ((part[i] + part[p.ldc + i]) + (part[2 * p.ldc + i] + part[3 * p.ldc + i])) * inv;
     __syncthreads();
-    const int share = (p.vdimp + gridDim.y - 1) / gridDim.y, v0 = blockIdx.y * share, v1 = min(v0 + share, p.vdimp);
     TO *out = (TO *)p.out + (size_t)qi * p.ldo + (size_t)h * p.vdimp;
-    for (int v = v0 + wave; v < v1; v += 8) {
+    auto product = [&](const u32x4 &wv, int i, float acc) {
+        const f32x4 x0 = *reinterpret_cast<const f32x4 *>(o + i), x1 = *reinterpret_cast<const f32x4 *>(o + i + 4);
+        acc = fmaf(x0.x, bf2f(wv.x & 0xffffu), fmaf(x0.y, bf2f(wv.x >> 16), acc));
+        acc = fmaf(x0.z, bf2f(wv.y & 0xffffu), fmaf(x0.w, bf2f(wv.y >> 16), acc));
+        acc = fmaf(x1.x, bf2f(wv.z & 0xffffu), fmaf(x1.y, bf2f(wv.z >> 16), acc));
+        return fmaf(x1.z, bf2f(wv.w & 0xffffu), fmaf(x1.w, bf2f(wv.w >> 16), acc));
+    };
+    auto rest = [&](int v, float acc) {  // the columns behind the first 512
         const uint16_t *w = p.uv + ((size_t)h * p.vdimp + v) * p.ldc;
-        float acc = 0.f;
-        for (int i = lane * 8; i < p.ldc; i += 512) {
-            const u32x4 wv = *reinterpret_cast<const u32x4 *>(w + i);
-            const f32x4 x0 = *reinterpret_cast<const f32x4 *>(o + i), x1 = *reinterpret_cast<const f32x4 *>(o + i + 4);
-            acc = fmaf(x0.x, bf2f(wv.x & 0xffffu), fmaf(x0.y, bf2f(wv.x >> 16), acc));
-            acc = fmaf(x0.z, bf2f(wv.y & 0xffffu), fmaf(x0.w, bf2f(wv.y >> 16), acc));
-            acc = fmaf(x1.x, bf2f(wv.z & 0xffffu), fmaf(x1.y, bf2f(wv.z >> 16), acc));
-            acc = fmaf(x1.z, bf2f(wv.w & 0xffffu), fmaf(x1.w, bf2f(wv.w >> 16), acc));
-        }
-        acc = wave_sum(acc);
+        for (int i = lane * 8 + 512; i < p.ldc; i += 512) acc = product(*reinterpret_cast<const u32x4 *>(w + i), i, acc);
+        return acc;
+    };
+#pragma unroll
+    for (int j = 0; j < AW; ++j) {
+        const int v = v0 + wave + 8 * j;
+        if (v >= v1) break;
+        const float acc = wave_sum(rest(v, lane * 8 < p.ldc ? product(uw[j], lane * 8, 0.f) : 0.f));
+        if (lane == 0) st_act(out, v, acc);
+    }
+    for (int v = v0 + wave + 8 * AW; v < v1; v += 8) {
+        const u32x4 wv = *reinterpret_cast<const u32x4 *>(p.uv + ((size_t)h * p.vdimp + v) * p.ldc + min(lane * 8, p.ldc - 8));
+        const float acc = wave_sum(rest(v, lane * 8 < p.ldc ? product(wv, lane * 8, 0.f) : 0.f));
         if (lane == 0) st_act(out, v, acc);
     }
 }
