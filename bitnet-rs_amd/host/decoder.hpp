@@ -107,6 +107,7 @@ class Decoder : public Sequence {
     int hand_over(int n, const float *last_row, bool with_logits);  // its launches
     bool chain_applies(int digits) const;
     bool handover16_applies(int digits) const;
+    bool f16_rows_apply() const;
     bool hybrid_applies(size_t n_rows) const;
     int last_prefill_path() const { return last_prefill_path_; }
     int saturation_fallbacks() const { return saturation_fallbacks_; }
