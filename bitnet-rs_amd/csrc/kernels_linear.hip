@@ -200,7 +200,8 @@ __global__ __launch_bounds__(256) void k_linear_scan(LinearAttn p, LinearWs w) {
     p.state[(size_t)h * size + e] = s;
 }
 
-// o = d^(i + 1) S q_i + sum over j <= i of d^(i - j) (k_j . q_i) v_j; four waves of 32 queries
+// o = d^(i + 1) S q_i + sum over j <= i of d^(i - j) (k_j . q_i) v_j; four waves of 32 queries.  blockIdx.z: a share of 16 NV value columns.  With few workgroups the launch is the walk
+// over a head's value tiles, whose operands arrive one tile ahead: shares of 64 columns instead of all 128, 24 heads at 64 tokens inside a prompt 12.6 -> 9.0 us.
 template <int NK, int NV>
 __global__ __launch_bounds__(256, NV > 8 ? 1 : 2) void k_linear_out(LinearAttn p, LinearWs w) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -210,7 +211,8 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : 2) void k_linear_out(LinearAttn p
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
     const int blk = blockIdx.x, h = blockIdx.y, t0 = blk * kLinBlock, len = min(kLinBlock, p.n - t0);
     const uint16_t *Q = (const uint16_t *)p.qkv + (size_t)h * p.dimp, *K = Q + (size_t)p.heads * p.dimp;
-    const uint16_t *V = (const uint16_t *)p.qkv + 2 * (size_t)p.heads * p.dimp + (size_t)h * p.vdimp;
+    const int vz = blockIdx.z * NV * 16, vdimp = p.vdimp - vz;
+    const uint16_t *V = (const uint16_t *)p.qkv + 2 * (size_t)p.heads * p.dimp + (size_t)h * p.vdimp + vz;
     Q += (size_t)t0 * p.ld, K += (size_t)t0 * p.ld, V += (size_t)t0 * p.ld;
     if (tid <= kLinBlock) pw[kLinBlock + tid] = p.decay_pow[(size_t)h * (kLinBlock + 1) + tid];
     if (tid < kLinBlock) pw[tid] = 0.f;
@@ -231,14 +233,14 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : 2) void k_linear_out(LinearAttn p
 #pragma unroll
         for (int j = 0; j < NV / 4; ++j)  // eight threads per pair of tokens
 #pragma unroll
-            for (int e = 0; e < 2; ++e) vr[j][e] = load_at(V, p.ld, tv + e, len, j * 64 + (tid & 7) * 8, p.vdimp);
+            for (int e = 0; e < 2; ++e) vr[j][e] = load_at(V, p.ld, tv + e, len, j * 64 + (tid & 7) * 8, vdimp);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < NK; ++j) kr[j] = zero_outside(kr[j], tk, len, j * 32 + (tid & 3) * 8, p.dimp);
 #pragma unroll
         for (int j = 0; j < NV / 4; ++j)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) vr[j][e] = zero_outside(vr[j][e], tv + e, len, j * 64 + (tid & 7) * 8, p.vdimp);
+            for (int e = 0; e < 2; ++e) vr[j][e] = zero_outside(vr[j][e], tv + e, len, j * 64 + (tid & 7) * 8, vdimp);
 #pragma unroll
         for (int j = 0; j < NK; ++j) *reinterpret_cast<u32x4 *>(lk + tk * KS + j * 64 + (tid & 3) * 16) = kr[j];
 #pragma unroll
@@ -257,13 +259,13 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : 2) void k_linear_out(LinearAttn p
         for (int kk = 0; kk < NK; ++kk)
             q[t][kk] = __builtin_bit_cast(bf16x8, zero_outside(__builtin_bit_cast(u32x4, q[t][kk]), qi[t], len, kk * 32 + g * 8, p.dimp));
     f32x4 o[NV][QT];
-    const size_t sb = ((size_t)h * w.nb + blk) * p.vdimp * p.dimp;
+    const size_t sb = (((size_t)h * w.nb + blk) * p.vdimp + vz) * p.dimp;
     bf16x8 hi[2][NK], lo[2][NK];
     auto request = [&](int v) {
 #pragma unroll
         for (int kk = 0; kk < NK; ++kk) {
             // (rows past vdimp are never stored, columns past dimp meet a zero query: clamped addresses, no branches around the loads)
-            const size_t at = sb + (size_t)min(v * 16 + r16, p.vdimp - 1) * p.dimp + min(kk * 32 + g * 8, p.dimp - 8);
+            const size_t at = sb + (size_t)min(v * 16 + r16, vdimp - 1) * p.dimp + min(kk * 32 + g * 8, p.dimp - 8);
             hi[v & 1][kk] = *reinterpret_cast<const bf16x8 *>(w.hi + at);
             lo[v & 1][kk] = *reinterpret_cast<const bf16x8 *>(w.lo + at);
         }
@@ -337,10 +339,10 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : 2) void k_linear_out(LinearAttn p
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
         if (qi[t] >= len) continue;
-        float *dst = p.out + (size_t)(t0 + qi[t]) * p.ldo + (size_t)h * p.vdimp + g * 4;
+        float *dst = p.out + (size_t)(t0 + qi[t]) * p.ldo + (size_t)h * p.vdimp + vz + g * 4;
 #pragma unroll
         for (int v = 0; v < NV; ++v)
-            if (v * 16 < p.vdimp) *reinterpret_cast<f32x4 *>(dst + v * 16) = o[v][t];
+            if (v * 16 < vdimp) *reinterpret_cast<f32x4 *>(dst + v * 16) = o[v][t];
     }
 }
 
@@ -355,7 +357,7 @@ static hipError_t out_go(const LinearAttn &a, const LinearWs &w, hipStream_t s) 
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_linear_out<NK, NV>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_linear_out<NK, NV>), dim3(w.nb, a.heads), dim3(256), lds, s, a, w);
+    hipLaunchKernelGGL((k_linear_out<NK, NV>), dim3(w.nb, a.heads, (a.vdimp + 16 * NV - 1) / (16 * NV)), dim3(256), lds, s, a, w);
     return hipGetLastError();
 }
 
@@ -371,6 +373,7 @@ hipError_t launch_linear_chunked(const LinearAttn &a, hipStream_t s) {
     hipLaunchKernelGGL(k_linear_sums, dim3(w.nb, a.heads, pieces), dim3(256), 3 * 64 * kTileBytes, s, a, w);
     hipLaunchKernelGGL(k_linear_scan, dim3((a.dimp * a.vdimp + 255) / 256, a.heads), dim3(256), 0, s, a, w);
     const int nk = a.dimp / 32, nv = a.vdimp / 16;
+    if (nv > 4 && w.nb * a.heads < 256) return nk <= 2 ? out_go<2, 4>(a, w, s) : nk <= 4 ? out_go<4, 4>(a, w, s) : out_go<8, 4>(a, w, s);
     if (nk <= 2) return nv <= 4 ? out_go<2, 4>(a, w, s) : nv <= 8 ? out_go<2, 8>(a, w, s) : out_go<2, 16>(a, w, s);
     if (nk <= 4) return nv <= 4 ? out_go<4, 4>(a, w, s) : nv <= 8 ? out_go<4, 8>(a, w, s) : out_go<4, 16>(a, w, s);
     return nv <= 8 ? out_go<8, 8>(a, w, s) : out_go<8, 16>(a, w, s);

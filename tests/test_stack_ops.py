@@ -420,6 +420,24 @@ def test_linear_attention_forms_hand_the_state_over(hip):
     assert at == n and u.rms_error(np.concatenate(got)[:, :, :vdim], want) < 1e-4
 
 
+@pytest.mark.parametrize("dim,vdim", [(32, 128), (96, 160), (160, 96)])
+def test_linear_attention_in_shares_of_value_columns(hip, dim, vdim):
+    """Many workgroups take all of a head's value columns each, few of them 64 columns: the same outputs, bit for bit."""
+    n, heads = 129, 129
+    dimp, vdimp, qkv, state, pw, want, S = linear_case(n, heads, dim, vdim, [0.5 + 0.49 * h / heads for h in range(heads)])
+
+    def run(h0, count):
+        cut = [qkv[:, o + h0 * w:o + (h0 + count) * w] for o, w in ((0, dimp), (heads * dimp, dimp), (2 * heads * dimp, vdimp))]
+        part = np.ascontiguousarray(np.concatenate(cut, axis=1))
+        out, nb = u.zeros_f32(n, count, vdimp), hip.linear_workspace_bytes(n, count, dimp, vdimp)
+        hip.linear_chunked_dev(u.dev_bf16(part), part.shape[1], n, count, dimp, vdimp, u.dev_f32(pw[h0:h0 + count]), u.dev_f32(state[h0:h0 + count]), out, count * vdimp, u.zeros_f32(nb // 4), nb)
+        return u.host(out)
+
+    got = run(0, heads)
+    assert all(u.rms_error(got[:, h, :vdim], want[:, h]) < 1e-4 for h in (0, 64, 128))
+    assert np.array_equal(got[:, 3:5], run(3, 2)) and np.array_equal(got[:, 128:], run(128, 1))
+
+
 def test_gated_norm_rows(hip):
     g = rng(3)
     m, n, mean_n, ldh, eps = 4, 96, 80, 128, 1e-2
