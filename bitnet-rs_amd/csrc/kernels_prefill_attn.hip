@@ -18,6 +18,7 @@
 //                   leave registers: an S^T accumulator (lane: query c, keys 4g..4g+3) is
 //                   already in B-operand form for the second product once the V^T operand
 //                   uses the same key -> k-slot map.
+//                   Contexts of one key tile skip k_prefill_prep (its comment: ONE).
 //   k_prefill_merge combines the key-split partials of launches too small to fill the chip.
 // q, k, v and the probabilities are rounded to f16 for the matrix cores (relative 2^-11);
 // the f32 KV cache the decode steps read afterwards holds the exact f32 values.
@@ -86,13 +87,20 @@ __device__ __forceinline__ int zz_row(const PrefillArgs &p, int t) {
     return r * 2 * p.zz_chunk + (first ? 0 : p.zz_chunk) + off;
 }
 
-// grid (max(nq_pad, Tpad) / 64, heads + 2 kv): slot < heads: query head (rows of p.q, positions from
-// q_block_pos); then k heads, then v heads (rows of p.kv, position = row).
-__global__ __launch_bounds__(256) void k_prefill_prep(PrefillArgs p) {
-    // one 64-token x 128-dim slab through LDS; every global access is 16 bytes wide (8 for f16 rows) and contiguous along the
-    // fastest index of its tensor (the scalar version of this kernel took 48 us per layer for 115 MB of traffic)
-    __shared__ __attribute__((aligned(16))) float tile[kQB][kPD + 4];  // + 4: float4 rows stay 16-byte aligned, columns spread over the banks
-    const int slot = blockIdx.y + p.slot0, t0 = blockIdx.x * kQB, tid = threadIdx.x;
+// A rotation pair (split-half RoPE).  The contractions are written out: left to hipcc they fall differently from kernel to kernel, and a
+// prompt's rows would depend on which of them rotated it.
+__device__ __forceinline__ float rope_lo(float x0, float x1, float s, float c) { return __builtin_fmaf(x0, c, -(x1 * s)); }
+__device__ __forceinline__ float rope_hi(float x0, float x1, float s, float c) { return __builtin_fmaf(x0, s, x1 * c); }
+
+typedef float SlabRow[kPD + 4];  // + 4: float4 rows stay 16-byte aligned, columns spread over the banks
+
+// One 64-token x 128-dim slab through LDS (`tile`: 64 rows); every global access is 16 bytes wide (8 for f16 rows) and contiguous along the
+// fastest index of its tensor (the scalar version took 48 us per layer for 115 MB of traffic).  Slot < heads: query head (rows of p.q,
+// positions from q_block_pos); then k heads, then v heads (rows of p.kv, position = row).  IMAGES: the f16 images that
+// k_prefill_attn reads are written as well; without, the decode cache alone.
+template <bool IMAGES>
+__device__ __forceinline__ void prefill_slab(const PrefillArgs &p, int slot, int block, SlabRow *tile) {
+    const int t0 = block * kQB, tid = threadIdx.x;
     const bool is_q = slot < p.n_heads, is_k = !is_q && slot < p.n_heads + p.n_kv;
     if ((p.phase == 1 && !is_q) || (p.phase == 2 && is_q)) return;
     const int n_rows = is_q ? p.nq : p.T;
@@ -101,7 +109,7 @@ __global__ __launch_bounds__(256) void k_prefill_prep(PrefillArgs p) {
                      : is_k ? p.k + (size_t)(slot - p.n_heads) * p.hs_kv : p.v + (size_t)(slot - p.n_heads - p.n_kv) * p.hs_kv;
     const int ld = is_q ? p.ld_q : p.ld_kv;
     // absolute position of row t0 (padding blocks past the last real one hold zeros: any position will do)
-    const int pos0 = is_q && p.q_block_pos ? ((int)blockIdx.x < (p.nq + kQB - 1) / kQB ? p.q_block_pos[blockIdx.x] : 0) : t0;
+    const int pos0 = is_q && p.q_block_pos ? (block < (p.nq + kQB - 1) / kQB ? p.q_block_pos[block] : 0) : t0;
     const int r0 = is_q ? t0 : zz_row(p, t0);  // a 64-row block of positions is 64 consecutive gathered rows (chunk % 64 == 0)
     const bool vec_ok = (ld & 3) == 0 && ((uintptr_t)src & 15) == 0;  // rows 16-byte aligned (always, for the decoder's buffers)
     if (!is_q && p.kv_f16) {
@@ -134,8 +142,8 @@ __global__ __launch_bounds__(256) void k_prefill_prep(PrefillArgs p) {
             const int pos = t0 + tok < n_rows ? pos0 + tok : 0;
             const float4 s = *reinterpret_cast<const float4 *>(p.rope_sin + (size_t)pos * 64 + j), c = *reinterpret_cast<const float4 *>(p.rope_cos + (size_t)pos * 64 + j);
             const float4 x0 = *reinterpret_cast<const float4 *>(&tile[tok][j]), x1 = *reinterpret_cast<const float4 *>(&tile[tok][64 + j]);
-            *reinterpret_cast<float4 *>(&tile[tok][j]) = float4{x0.x * c.x - x1.x * s.x, x0.y * c.y - x1.y * s.y, x0.z * c.z - x1.z * s.z, x0.w * c.w - x1.w * s.w};
-            *reinterpret_cast<float4 *>(&tile[tok][64 + j]) = float4{x0.x * s.x + x1.x * c.x, x0.y * s.y + x1.y * c.y, x0.z * s.z + x1.z * c.z, x0.w * s.w + x1.w * c.w};
+            *reinterpret_cast<float4 *>(&tile[tok][j]) = float4{rope_lo(x0.x, x1.x, s.x, c.x), rope_lo(x0.y, x1.y, s.y, c.y), rope_lo(x0.z, x1.z, s.z, c.z), rope_lo(x0.w, x1.w, s.w, c.w)};
+            *reinterpret_cast<float4 *>(&tile[tok][64 + j]) = float4{rope_hi(x0.x, x1.x, s.x, c.x), rope_hi(x0.y, x1.y, s.y, c.y), rope_hi(x0.z, x1.z, s.z, c.z), rope_hi(x0.w, x1.w, s.w, c.w)};
         }
         __syncthreads();
     }
@@ -154,7 +162,7 @@ __global__ __launch_bounds__(256) void k_prefill_prep(PrefillArgs p) {
         store_rows_f16(p.qh + ((size_t)slot * p.nq_pad + t0) * kPD);
     } else if (is_k) {
         const int kvh = slot - p.n_heads;
-        store_rows_f16(p.kh + ((size_t)kvh * p.Tpad + t0) * kPD);
+        if constexpr (IMAGES) store_rows_f16(p.kh + ((size_t)kvh * p.Tpad + t0) * kPD);
         // decode cache: K transposed in 64-position tiles [chunk][128][64] (kernels_attn.hip); t0 is a tile start
         const size_t head_floats = (size_t)((p.max_pos + 63) / 64) * 64 * kPD;
         float *kt = p.kcache + (size_t)kvh * head_floats + (size_t)(t0 >> 6) * kPD * 64;
@@ -194,13 +202,19 @@ __global__ __launch_bounds__(256) void k_prefill_prep(PrefillArgs p) {
         // (a < 4, b < 2, j < 4) at slot 8 a + 4 b + j, so that a lane's 8 k-slots (keys 4 g .. 4 g + 3 and 16 + 4 g .. 16 + 4 g + 3: the
         // S^T accumulator layout) are ONE 16-byte unit.  4 adjacent positions of one dim = 8 contiguous bytes here as well.
         _Float16 *vt = p.vt + (size_t)kvh * kPD * p.Tpad;
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < 8 && IMAGES; ++i) {
             const int idx = tid + 256 * i, d = idx >> 4, t4 = idx & 15, tok = t4 * 4;
             const int slot = 32 * (t4 >> 3) + 8 * (t4 & 3) + 4 * ((t4 >> 2) & 1);
             const v4h h = {(_Float16)tile[tok][d], (_Float16)tile[tok + 1][d], (_Float16)tile[tok + 2][d], (_Float16)tile[tok + 3][d]};
             *reinterpret_cast<v4h *>(vt + (size_t)d * p.Tpad + t0 + slot) = h;
         }
     }
+}
+
+// grid (max(nq_pad, Tpad) / 64, slots from p.slot0 on): a slab per workgroup
+__global__ __launch_bounds__(256) void k_prefill_prep(PrefillArgs p) {
+    __shared__ __attribute__((aligned(16))) SlabRow tile[kQB];
+    prefill_slab<true>(p, (int)blockIdx.y + p.slot0, (int)blockIdx.x, tile);
 }
 
 // NW waves per workgroup = HW query heads of ONE KV head x (NW / HW) wave columns; a wave owns NQ groups of 16 queries of its
@@ -245,29 +259,43 @@ __device__ __forceinline__ void gdma1k_s(unsigned lane_off, const void *sbase, u
                  : "memory");
 }
 
-template <int HW, int NW, int NQ>
+// ONE: the whole context is one key tile (T <= 64), and k_prefill_prep is not launched: a workgroup rotates and rounds its KV head's rows
+// into its own LDS tile (the values k_prefill_prep would have left), and 2 n_kv further workgroups of the launch write the decode cache
+// meanwhile.  Both launches were chains of latencies of 6 and 9 us; in one: prompts of 8 / 19 / 64 tokens (30 layers, QK256) 1602 / 1788 / 2161 ->
+// 1395 / 1525 / 1825 us, block-scaled weights 1513 / 1873 / 2157 -> 1313 / 1624 / 1833.  16 queries per wave (NQ = 1): every load in flight at
+// once (160 registers), and no padded second group.  Not beyond one tile: each workgroup would prepare all of them for itself.
+template <int HW, int NW, int NQ, bool ONE>
 __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_prefill_attn(PrefillArgs p) {
     constexpr int QW = NW / HW, QG = 16 * QW * NQ;  // wave columns per workgroup, queries per workgroup
     static_assert(NW == 4, "tile staging deals 32 pieces to 4 waves");
     extern __shared__ __attribute__((aligned(16))) uint8_t kv_lds[];  // [2][K tile | V^T tile]
+    if constexpr (ONE) {
+        const int n_qb = (p.nq + QG - 1) / QG;
+        if ((int)blockIdx.y >= n_qb) {
+            const int slot = p.n_heads + ((int)blockIdx.y - n_qb) * (int)gridDim.x + (int)blockIdx.x;
+            if (slot < p.n_heads + 2 * p.n_kv) prefill_slab<false>(p, slot, 0, reinterpret_cast<SlabRow *>(kv_lds));
+            return;
+        }
+    }
     __shared__ int s_last;
-    const int qg = p.head_fast ? (int)gridDim.y - 1 - (int)blockIdx.y : (int)gridDim.x - 1 - (int)blockIdx.x;  // long (late) blocks first
-    const int hg = p.head_fast ? blockIdx.x : blockIdx.y;
+    const int qg = ONE ? (int)blockIdx.y : p.head_fast ? (int)gridDim.y - 1 - (int)blockIdx.y : (int)gridDim.x - 1 - (int)blockIdx.x;  // long (late) blocks first
+    const int hg = ONE || p.head_fast ? blockIdx.x : blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
     const int h = hg * HW + wave % HW, kvh = h / (p.n_heads / p.n_kv);  // HW divides the group: one KV head per workgroup
     const int qbase = qg * QG + (wave / HW) * 16 * NQ;            // first query row of this wave (16 NQ rows inside one 64-row block)
     const int blk64 = qbase >> 6;                                 // the 64-row block the wave's rows lie in
     const int bpos = (p.q_block_pos ? p.q_block_pos[blk64 < (p.nq + kQB - 1) / kQB ? blk64 : 0] : blk64 * kQB) + (qbase & 63);
-    if (tid == 0) s_last = 0;
-    __syncthreads();
-    {   // last key tile any query of the workgroup sees
+    if constexpr (!ONE) {
+        if (tid == 0) s_last = 0;
+        __syncthreads();
+        // last key tile any query of the workgroup sees
         const int top = bpos + 16 * NQ - 1;
         const int need = p.causal ? (top < p.T ? top : p.T - 1) / kQB : (p.T - 1) / kQB;
         if (lane == 0) atomicMax(&s_last, need);
+        __syncthreads();
     }
-    __syncthreads();
-    int kt_first = 0, kt_last = s_last;
-    if (p.ksplit > 1) {
+    int kt_first = 0, kt_last = ONE ? 0 : s_last;
+    if (!ONE && p.ksplit > 1) {
         // this workgroup's share of the key tiles: a query block with n tiles is cut into ceil(n / kTilesPerSplit) parts (at most
         // ksplit), so early blocks (few tiles) stay whole and late ones spread over the chip; surplus workgroups only mark their
         // partial empty (m = -inf), which the merge skips
@@ -353,11 +381,33 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_prefill_attn(Prefi
     // B2 (before the V chunk 2 MFMAs = before the first K read of the NEXT tile is issued) waits for K(kt + 1) and requests K(kt + 2)
     // into the buffer K(kt) left (its last read was issued two chunks ago and consumed by K chunk 3).  Loads return in order, so
     // "the 4 pieces requested last may still be in flight" is s_waitcnt vmcnt(4).
-    stage_k(kt_first, 0);
-    stage_v(kt_first, 0);
-    if (kt_first < kt_last) stage_k(kt_first + 1, 1);
+    // ONE: a thread's four quads of rotation pairs of K (token 16 i + tid / 16) and its two 4 x 4 blocks of V (tokens 4 t4 .., dims 4 dq ..),
+    // every row clamped into the context and requested before the queries
+    float4 kx[ONE ? 4 : 1][2], ksn[ONE ? 4 : 1], kcs[ONE ? 4 : 1], vx[ONE ? 2 : 1][4];
+    if constexpr (ONE) {
+        const float *kr = p.k + (size_t)kvh * p.hs_kv, *vr = p.v + (size_t)kvh * p.hs_kv;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int tok = 16 * i + (tid >> 4), j = (tid & 15) * 4, row = tok < p.T ? tok : 0;
+            kx[i][0] = *reinterpret_cast<const float4 *>(kr + (size_t)row * p.ld_kv + j);
+            kx[i][1] = *reinterpret_cast<const float4 *>(kr + (size_t)row * p.ld_kv + 64 + j);
+            ksn[i] = *reinterpret_cast<const float4 *>(p.rope_sin + (size_t)row * 64 + j);
+            kcs[i] = *reinterpret_cast<const float4 *>(p.rope_cos + (size_t)row * 64 + j);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int tok = 4 * (8 * i + (tid >> 5)) + e, row = tok < p.T ? tok : 0;
+                vx[i][e] = *reinterpret_cast<const float4 *>(vr + (size_t)row * p.ld_kv + 4 * (tid & 31));
+            }
+    } else {
+        stage_k(kt_first, 0);
+        stage_v(kt_first, 0);
+        if (kt_first < kt_last) stage_k(kt_first + 1, 1);
+    }
     // the query operands, requested BEHIND the first K / V^T tiles so that their round trip (strided f32 rows + the RoPE tables) overlaps the tiles'
-    if (p.q_in_kernel) {
+    if (ONE || p.q_in_kernel) {
         // straight from the f32 rows of the q|k|v projection (round 4: two thirds of k_prefill_prep's traffic were the query slabs): a lane's
         // dims 32 ch + 8 g + i (ch < 4) hold both members of every rotation pair (d, d + 64) = (ch, ch + 2), so the split-half RoPE
         // (crates/bitnet-rope/src/lib.rs:59-93, T:134-163) needs no exchange; the same arithmetic as k_prefill_prep, the softmax scale and the
@@ -385,8 +435,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_prefill_attn(Prefi
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
                         const float x0 = x[ch][i], x1 = x[ch + 2][i];
-                        x[ch][i] = x0 * cs[i] - x1 * sn[i];
-                        x[ch + 2][i] = x0 * sn[i] + x1 * cs[i];
+                        x[ch][i] = rope_lo(x0, x1, sn[i], cs[i]);
+                        x[ch + 2][i] = rope_hi(x0, x1, sn[i], cs[i]);
                     }
                 }
             }
@@ -401,6 +451,36 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_prefill_attn(Prefi
             const _Float16 *qp = p.qh + ((size_t)h * p.nq_pad + qbase + 16 * q + c) * kPD + 8 * g;
 #pragma unroll
             for (int ch = 0; ch < 4; ++ch) qreg[q][ch] = *reinterpret_cast<const v8h *>(qp + 32 * ch);
+        }
+    }
+    if constexpr (ONE) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int tok = 16 * i + (tid >> 4), j = (tid & 15) * 4;
+            const bool live = tok < p.T;
+            const float4 x0 = kx[i][0], x1 = kx[i][1], s = ksn[i], cc = kcs[i];
+            float4 lo = {rope_lo(x0.x, x1.x, s.x, cc.x), rope_lo(x0.y, x1.y, s.y, cc.y), rope_lo(x0.z, x1.z, s.z, cc.z), rope_lo(x0.w, x1.w, s.w, cc.w)};
+            float4 hi = {rope_hi(x0.x, x1.x, s.x, cc.x), rope_hi(x0.y, x1.y, s.y, cc.y), rope_hi(x0.z, x1.z, s.z, cc.z), rope_hi(x0.w, x1.w, s.w, cc.w)};
+            // rounded to f32 before f16, as the rows of k_prefill_prep are (hipcc would take both roundings as one)
+            asm("" : "+v"(lo.x), "+v"(lo.y), "+v"(lo.z), "+v"(lo.w), "+v"(hi.x), "+v"(hi.y), "+v"(hi.z), "+v"(hi.w));
+            const v4h zero = {(_Float16)0.f, (_Float16)0.f, (_Float16)0.f, (_Float16)0.f};
+            const v4h hl = {(_Float16)lo.x, (_Float16)lo.y, (_Float16)lo.z, (_Float16)lo.w}, hh = {(_Float16)hi.x, (_Float16)hi.y, (_Float16)hi.z, (_Float16)hi.w};
+            // dims j .. j + 3 are half (j / 4) & 1 of unit j / 8, dims 64 + j .. of unit 8 + j / 8
+            uint8_t *kp = kv_lds + tok * 256 + 8 * ((j >> 2) & 1);
+            *reinterpret_cast<v4h *>(kp + (((j >> 3) ^ (tok & 15)) * 16)) = live ? hl : zero;
+            *reinterpret_cast<v4h *>(kp + (((8 + (j >> 3)) ^ (tok & 15)) * 16)) = live ? hh : zero;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int t4 = 8 * i + (tid >> 5), unit = 4 * (t4 >> 3) + (t4 & 3), half = (t4 >> 2) & 1;  // k_prefill_prep's order of keys
+            const bool l0 = 4 * t4 < p.T, l1 = 4 * t4 + 1 < p.T, l2 = 4 * t4 + 2 < p.T, l3 = 4 * t4 + 3 < p.T;
+            const float(*x)[4] = reinterpret_cast<const float(*)[4]>(&vx[i][0]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int dim = 4 * (tid & 31) + e;
+                const v4h hv = {(_Float16)(l0 ? x[0][e] : 0.f), (_Float16)(l1 ? x[1][e] : 0.f), (_Float16)(l2 ? x[2][e] : 0.f), (_Float16)(l3 ? x[3][e] : 0.f)};
+                *reinterpret_cast<v4h *>(kv_lds + kKTile + dim * 128 + ((unit ^ ((dim >> 1) & 7)) * 16) + 8 * half) = hv;
+            }
         }
     }
     // the builtin form, so that hipcc's own bookkeeping sees its q loads retired here: left to itself it re-waits for them with
@@ -550,7 +630,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_prefill_attn(Prefi
         l += __shfl_xor(l, 16);
         l += __shfl_xor(l, 32);
         const int qrow = qbase + 16 * q + c;
-        if (p.ksplit > 1) {  // un-normalised partial; padding rows are written too (the merge never reads them)
+        if (!ONE && p.ksplit > 1) {  // un-normalised partial; padding rows are written too (the merge never reads them)
             const size_t ro = ((size_t)blockIdx.z * p.nq_pad + qrow) * p.n_heads + h;
             float *op = p.part_o + ro * kPD + 4 * g;
 #pragma unroll
@@ -629,13 +709,13 @@ static hipError_t launch_attn_kernel(const PrefillArgs &p, hipStream_t stream) {
     void (*ak)(PrefillArgs);
     dim3 grid;
     if (group % 4 == 0) {  // 4 waves = the 4 heads of a KV head x 32 queries each; two such workgroups per CU
-        ak = k_prefill_attn<4, 4, 2>;
+        ak = k_prefill_attn<4, 4, 2, false>;
         grid = dim3((unsigned)(p.nq_pad / 32), (unsigned)(p.n_heads / 4), z);
     } else if (group % 2 == 0) {  // 2 heads x 2 wave columns x 32 queries
-        ak = k_prefill_attn<2, 4, 2>;
+        ak = k_prefill_attn<2, 4, 2, false>;
         grid = dim3((unsigned)(p.nq_pad / 64), (unsigned)(p.n_heads / 2), z);
     } else {
-        ak = k_prefill_attn<1, 4, 2>;
+        ak = k_prefill_attn<1, 4, 2, false>;
         grid = dim3((unsigned)(p.nq_pad / 128), (unsigned)p.n_heads, z);
     }
     // Workgroups are dispatched in linear id order (x fastest).  With the query groups in x, head group 0's blocks all start before head
@@ -729,6 +809,19 @@ hipError_t launch_attn_prefill(const float *q, int ld_q, const int *q_block_pos,
     p.slot0 = 0;
     if (phase == 1) {  // the query slabs alone (nothing to do when the attention kernel prepares them itself)
         if (!p.q_in_kernel) hipLaunchKernelGGL(k_prefill_prep, dim3(nbq, (unsigned)n_heads), dim3(256), 0, stream, p);
+        return hipGetLastError();
+    }
+    // One key tile and a group of heads that fills a workgroup: one launch (k_prefill_attn, ONE).  The rows of k and v are then read while
+    // other workgroups write `out`: an `out` that lies over them keeps the two launches, as do rows off 16 bytes and f16 rows.
+    const auto clear_of_out = [&](const float *b, size_t n) {
+        const uintptr_t o0 = (uintptr_t)out, o1 = o0 + (size_t)nq * n_heads * kPD * 4, b0 = (uintptr_t)b;
+        return b0 + n * 4 <= o0 || o1 <= b0;
+    };
+    if (T <= kQB && phase == 0 && p.q_in_kernel && !kv_f16 && zz_world == 0 && (n_heads / n_kv) % 4 == 0 && (ld_kv & 3) == 0 && ((uintptr_t)kv & 15) == 0 &&
+        clear_of_out(kv, (size_t)(T - 1) * ld_kv + 2 * (size_t)n_kv * kPD)) {
+        const unsigned x = (unsigned)(n_heads / 4);
+        hipLaunchKernelGGL((k_prefill_attn<4, 4, 1, true>), dim3(x, (unsigned)(div_ceil((size_t)nq, 16) + div_ceil((size_t)2 * n_kv, x))), dim3(256),
+                           sizeof(SlabRow) * kQB, stream, p);
         return hipGetLastError();
     }
     if (p.q_in_kernel) {

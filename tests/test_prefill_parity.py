@@ -527,3 +527,34 @@ def test_gathered_attention_world8_8k_matches_unsharded_and_f64(hip, oracle, tor
             pm = np.exp(s - s.max())
             want = (pm / pm.sum()) @ v[: t + 1, h // 4]
             assert np.max(np.abs(base[t, h * D:(h + 1) * D] - want)) <= 6e-3, (t, h)
+
+
+@pytest.mark.parametrize("T,n_heads,n_kv", [(1, 4, 1), (15, 20, 5), (16, 8, 2), (17, 16, 2), (37, 20, 5), (63, 4, 1), (64, 20, 5)])
+@pytest.mark.parametrize("flags", [0, 1, 2, 3])
+def test_prefill_attention_of_one_key_tile_is_the_start_of_a_longer_prompt(hip, oracle, torch_, T, n_heads, n_kv, flags):
+    """Up to 64 tokens one launch attends and fills the cache; its rows and its cache are those that the two launches of a longer prompt
+    leave for the same tokens (causal: the later ones do not reach them), digit for digit, in either cache and output type."""
+    D, max_pos, T2 = 128, 200, 130
+    rng = np.random.default_rng(1000 * T + flags)
+    ld = (n_heads + 2 * n_kv) * D
+    x = torch_.from_numpy(rng.normal(0, 1.5, (T2, ld)).astype(np.float32)).cuda()
+    sin, cos = (torch_.from_numpy(np.ascontiguousarray(a, np.float32)).cuda() for a in oracle.rope_tables(D, max_pos, 10000.0))
+    kt = torch_.float16 if flags & 1 else torch_.float32
+    n_cache, n_tiles = n_kv * 256 * D, 256 // 64
+    got = []
+    for n in (T, T2):
+        kc, vc = torch_.zeros(n_cache, dtype=kt, device="cuda"), torch_.zeros(n_cache, dtype=kt, device="cuda")
+        out = torch_.full((n, n_heads * D), 7.0, dtype=torch_.float16 if flags & 2 else torch_.float32, device="cuda")
+        wsb = hip.attention_prefill_workspace_bytes(n_heads, n_kv, n)
+        ws = torch_.empty(wsb, dtype=torch_.uint8, device="cuda")
+        hip.attention_prefill_flags_dev(x[:n].contiguous(), sin, cos, kc, vc, n_heads, n_kv, D, max_pos, n, ws, wsb, out, flags)
+        torch_.cuda.synchronize()
+        if flags & 1:  # [kv][tile][D / 2][64][2]
+            k = kc.view(n_kv, n_tiles, D // 2, 64, 2).permute(0, 1, 3, 2, 4).reshape(n_kv, 256, D)
+        else:  # [kv][tile][D][64]
+            k = kc.view(n_kv, n_tiles, D, 64).permute(0, 1, 3, 2).reshape(n_kv, 256, D)
+        got.append((out, k, vc.view(n_kv, 256, D)))
+    (o, k, v), (o2, k2, v2) = got
+    assert torch_.equal(o, o2[:T])
+    assert torch_.equal(k[:, :T], k2[:, :T]) and torch_.equal(v[:, :T], v2[:, :T])
+    assert not k[:, T:].any() and not v[:, T:].any()
