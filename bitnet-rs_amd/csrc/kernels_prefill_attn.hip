@@ -261,7 +261,7 @@ __device__ __forceinline__ void gdma1k_s(unsigned lane_off, const void *sbase, u
 
 // ONE: the whole context is one key tile (T <= 64), and k_prefill_prep is not launched: a workgroup rotates and rounds its KV head's rows
 // into its own LDS tile (the values k_prefill_prep would have left), and 2 n_kv further workgroups of the launch write the decode cache
-// meanwhile.  Both launches were chains of latencies of 6 and 9 us; in one: prompts of 8 / 19 / 64 tokens (30 layers, QK256) 1602 / 1788 / 2161 ->
+// meanwhile.  Two launches of 6.2 and 9.2 us, chains of latencies both (19 tokens), become one of 7.9: prompts of 8 / 19 / 64 tokens (30 layers, QK256) 1602 / 1788 / 2161 ->
 // 1395 / 1525 / 1825 us, block-scaled weights 1513 / 1873 / 2157 -> 1313 / 1624 / 1833.  16 queries per wave (NQ = 1): every load in flight at
 // once (160 registers), and no padded second group.  Not beyond one tile: each workgroup would prepare all of them for itself.
 template <int HW, int NW, int NQ, bool ONE>
