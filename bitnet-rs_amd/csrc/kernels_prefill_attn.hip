@@ -259,13 +259,14 @@ __device__ __forceinline__ void gdma1k_s(unsigned lane_off, const void *sbase, u
                  : "memory");
 }
 
-// ONE: the whole context is one key tile (T <= 64), and k_prefill_prep is not launched: a workgroup rotates and rounds its KV head's rows
+// ONE (NQ = 1): the whole context is one key tile (T <= 64), and k_prefill_prep is not launched: a workgroup rotates and rounds its KV head's rows
 // into its own LDS tile (the values k_prefill_prep would have left), and 2 n_kv further workgroups of the launch write the decode cache
 // meanwhile.  Two launches of 6.2 and 9.2 us, chains of latencies both (19 tokens), become one of 7.9: prompts of 8 / 19 / 64 tokens (30 layers, QK256) 1602 / 1788 / 2161 ->
-// 1395 / 1525 / 1825 us, block-scaled weights 1513 / 1873 / 2157 -> 1313 / 1624 / 1833.  16 queries per wave (NQ = 1): every load in flight at
+// 1395 / 1525 / 1825 us, block-scaled weights 1513 / 1873 / 2157 -> 1313 / 1624 / 1833.  16 queries per wave: every load in flight at
 // once (160 registers), and no padded second group.  Not beyond one tile: each workgroup would prepare all of them for itself.
-template <int HW, int NW, int NQ, bool ONE>
+template <int HW, int NW, int NQ>
 __global__ __launch_bounds__(NW * 64, NW == 4 ? 2 : 1) void k_prefill_attn(PrefillArgs p) {
+    constexpr bool ONE = NQ == 1;
     constexpr int QW = NW / HW, QG = 16 * QW * NQ;  // wave columns per workgroup, queries per workgroup
     static_assert(NW == 4, "tile staging deals 32 pieces to 4 waves");
     extern __shared__ __attribute__((aligned(16))) uint8_t kv_lds[];  // [2][K tile | V^T tile]
@@ -709,13 +710,13 @@ static hipError_t launch_attn_kernel(const PrefillArgs &p, hipStream_t stream) {
     void (*ak)(PrefillArgs);
     dim3 grid;
     if (group % 4 == 0) {  // 4 waves = the 4 heads of a KV head x 32 queries each; two such workgroups per CU
-        ak = k_prefill_attn<4, 4, 2, false>;
+        ak = k_prefill_attn<4, 4, 2>;
         grid = dim3((unsigned)(p.nq_pad / 32), (unsigned)(p.n_heads / 4), z);
     } else if (group % 2 == 0) {  // 2 heads x 2 wave columns x 32 queries
-        ak = k_prefill_attn<2, 4, 2, false>;
+        ak = k_prefill_attn<2, 4, 2>;
         grid = dim3((unsigned)(p.nq_pad / 64), (unsigned)(p.n_heads / 2), z);
     } else {
-        ak = k_prefill_attn<1, 4, 2, false>;
+        ak = k_prefill_attn<1, 4, 2>;
         grid = dim3((unsigned)(p.nq_pad / 128), (unsigned)p.n_heads, z);
     }
     // Workgroups are dispatched in linear id order (x fastest).  With the query groups in x, head group 0's blocks all start before head
@@ -820,7 +821,7 @@ hipError_t launch_attn_prefill(const float *q, int ld_q, const int *q_block_pos,
     if (T <= kQB && phase == 0 && p.q_in_kernel && !kv_f16 && zz_world == 0 && (n_heads / n_kv) % 4 == 0 && (ld_kv & 3) == 0 && ((uintptr_t)kv & 15) == 0 &&
         clear_of_out(kv, (size_t)(T - 1) * ld_kv + 2 * (size_t)n_kv * kPD)) {
         const unsigned x = (unsigned)(n_heads / 4);
-        hipLaunchKernelGGL((k_prefill_attn<4, 4, 1, true>), dim3(x, (unsigned)(div_ceil((size_t)nq, 16) + div_ceil((size_t)2 * n_kv, x))), dim3(256),
+        hipLaunchKernelGGL((k_prefill_attn<4, 4, 1>), dim3(x, (unsigned)(div_ceil((size_t)nq, 16) + div_ceil((size_t)2 * n_kv, x))), dim3(256),
                            sizeof(SlabRow) * kQB, stream, p);
         return hipGetLastError();
     }
