@@ -296,8 +296,9 @@ int Decoder::set_kv_f16(bool on) {
         drop_graphs();
         for (auto &L : layers_) {  // stale bytes of the other type could be NaN / Inf patterns in this one
             const size_t n = (size_t)c_.n_kv_heads * (((size_t)c_.max_pos + 63) / 64 * 64) * c_.head_dim;
-            HCHK(hipMemset(L.kcache, 0, n * sizeof(float)));
-            HCHK(hipMemset(L.vcache, 0, n * sizeof(float)));
+            // (on the model's own stream: the null stream is not ordered with it, and the next prompt waits for nothing else)
+            HCHK(hipMemsetAsync(L.kcache, 0, n * sizeof(float), (hipStream_t)stream_));
+            HCHK(hipMemsetAsync(L.vcache, 0, n * sizeof(float), (hipStream_t)stream_));
         }
     }
     kv_f16_ = on;

@@ -1,0 +1,138 @@
+// A HIP runtime of promises for the host code (tests/test_host_order.py): work is done as late as HIP allows it -- a stream's when somebody waits for that stream, the null stream's when a
+// blocking copy follows it -- so that whatever relies on an order that nothing establishes is seen.  The kernels are stand-ins that leave a mark.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <deque>
+#include <functional>
+#include <vector>
+
+#include "decoder.hpp"
+
+namespace {
+typedef std::deque<std::function<void()>> Queue;
+Queue g_null;
+std::vector<Queue *> g_streams;
+Queue &queue(void *s) { return s ? *static_cast<Queue *>(s) : g_null; }
+void run(Queue &q) {
+    while (!q.empty()) {
+        auto f = std::move(q.front());
+        q.pop_front();
+        f();
+    }
+}
+void run_all() {
+    run(g_null);
+    for (Queue *q : g_streams) run(*q);
+}
+uint64_t g_clamped = 0, g_taken = 0;  // the device's count, and what of it f16_saturations_dev has given out
+int g_clamping = 0;                   // the next product clamps, and somebody else takes the count at once
+uint64_t take() {
+    const uint64_t n = g_clamped - g_taken;
+    g_taken = g_clamped;
+    return n;
+}
+void product(void *s) {
+    if (g_clamping == 0) return;
+    --g_clamping;
+    queue(s).push_back([] { ++g_clamped, take(); });
+}
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) { return *p = malloc(n + 64), memset(*p, 0x5a, n + 64), hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipFree(void *p) { return run_all(), free(p), hipSuccess; }
+hipError_t hipHostFree(void *p) { return hipFree(p); }
+hipError_t hipDeviceSynchronize() { return run_all(), hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+    g_streams.push_back(new Queue);
+    return *s = reinterpret_cast<hipStream_t>(g_streams.back()), hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) { return run(queue(s)), hipSuccess; }
+hipError_t hipMemset(void *p, int v, size_t n) { return g_null.push_back([=] { memset(p, v, n); }), hipSuccess; }
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t s) { return queue(s).push_back([=] { memset(p, v, n); }), hipSuccess; }
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return run(g_null), memcpy(d, s, n), hipSuccess; }
+
+size_t bitnet_hip_qact_bytes(size_t) { return 64; }
+size_t bitnet_hip_qact_stats_bytes(size_t) { return 64; }
+size_t bitnet_hip_attention_scratch_bytes(size_t, size_t) { return 64; }
+size_t bitnet_hip_attention_prefill_workspace_bytes(size_t, size_t, size_t) { return 64; }
+size_t bitnet_hip_matmul_workspace_bytes(size_t, size_t, int) { return 64; }
+int bitnet_hip_matmul_f16_supported(bitnet_hip_weights_t) { return 1; }
+int bitnet_hip_weights_info(bitnet_hip_weights_t, size_t *rows, size_t *cols, size_t *bytes) {
+    if (rows) *rows = 512;
+    if (cols) *cols = 512;
+    if (bytes) *bytes = 512 * 128;
+    return 0;
+}
+int bitnet_hip_weights_upload_qk256(const uint8_t *, size_t, size_t, size_t, size_t, bitnet_hip_weights_t *h) { return *h = 1, 0; }
+int bitnet_hip_weights_concat(const bitnet_hip_weights_t *, size_t, int, bitnet_hip_weights_t *h) { return *h = 1, 0; }
+int bitnet_hip_sequence_update_dev(int32_t *history, size_t first, size_t n, const int32_t *tokens, int32_t *n_forced, int32_t forced, int32_t *pos, int32_t position, const float *row,
+                                   float *x, size_t width, void *s) {
+    queue(s).push_back([=] {
+        if (history)
+            for (size_t i = 0; i < n; ++i) history[first + i] = tokens ? tokens[i] : 0;
+        if (n_forced) *n_forced = forced;
+        if (pos) *pos = position;
+        if (x) memcpy(x, row, width * 4);
+    });
+    return 0;
+}
+int bitnet_hip_attention_prefill_flags_dev(const float *, const float *, const float *, void *k, void *v, size_t, size_t, size_t, size_t, size_t, void *, size_t, void *, int, void *s) {
+    queue(s).push_back([=] { *(float *)k = 7.f, *(float *)v = 8.f; });
+    return 0;
+}
+int bitnet_hip_attention_prefill_dev(const float *, const float *, const float *, float *k, float *v, size_t, size_t, size_t, size_t, size_t, void *, size_t, float *, void *s) {
+    queue(s).push_back([=] { *k = 7.f, *v = 8.f; });
+    return 0;
+}
+int bitnet_hip_matmul_f16_dev(bitnet_hip_weights_t, const void *, size_t, const float *, size_t, const float *, float, float *, const float *, int, void *, const float *, float *, void *s) {
+    return product(s), 0;
+}
+int bitnet_hip_advance_pos_dev(int32_t *pos, void *s) { return queue(s).push_back([=] { ++*pos; }), 0; }
+int bitnet_hip_f16_saturations_dev(uint32_t *count, void *s) {
+    queue(s).push_back([=] {
+        const uint64_t n = take();
+        if (count) *count = (uint32_t)n;
+    });
+    return 0;
+}
+}
+
+using bitnet_host::Decoder;
+
+#define CHECK(x) \
+    if (!(x)) return printf("%s:%d: %s\n", __FILE__, __LINE__, #x), 1
+
+int main(int argc, char **argv) {
+    bitnet_host::Config c;
+    c.hidden = 512, c.n_layers = 2, c.n_heads = 4, c.n_kv_heads = 1, c.head_dim = 128, c.ffn = 512, c.vocab = 64, c.max_pos = 128, c.eps = 1e-5f, c.rope_theta = 1e4f;
+    std::vector<uint8_t> zeros(1 << 20);
+    const float *f = reinterpret_cast<const float *>(zeros.data());
+    const int32_t tokens[3] = {11, 12, 13};
+    Decoder d(c);
+    CHECK(!d.dead());
+    for (int l = 0; l < c.n_layers; ++l) {
+        const uint8_t *z = zeros.data();
+        CHECK(d.set_layer_qk256(l, bitnet_host::LayerWeightsQk256{f, f, z, z, z, z, z, z, z}) == 0);
+    }
+    CHECK(d.set_globals(reinterpret_cast<const uint16_t *>(zeros.data()), f) == 0);
+    const char *what = argc > 1 ? argv[1] : "";
+    auto prompt = [&] { return d.feed(tokens, 3) || d.prefill(3, false, 2, nullptr); };
+    if (!strcmp(what, "cache_type")) {  // the caches are clear ahead of the prompt that fills them, whichever stream did it
+        for (bool f16 : {true, false, true}) {
+            CHECK(d.reset() == 0 && d.set_kv_f16(f16) == 0 && prompt() == 0);
+            hipDeviceSynchronize();
+            for (int l = 0; l < c.n_layers; ++l) {
+                uint64_t h[4];
+                void *p[4];
+                d.layer_objects(l, h, p);
+                CHECK(*(float *)p[2] == 7.f && *(float *)p[3] == 8.f && ((float *)p[2])[1] == 0.f && ((float *)p[3])[1] == 0.f);
+            }
+        }
+    } else {
+        CHECK(!"a case of this name");
+    }
+    return 0;
+}

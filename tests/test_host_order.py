@@ -1,0 +1,37 @@
+"""What the host layer orders, and what it only hopes for: its own sources on a runtime that does everything as late as HIP allows (tests/host_order.cpp), on the CPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HOST = os.path.join(ROOT, "bitnet-rs_amd", "host")
+RUNTIME_HEADER = "/opt/rocm/include/hip/hip_runtime_api.h"
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    if shutil.which("g++") is None or not os.path.exists(RUNTIME_HEADER):
+        pytest.skip("needs g++ and the runtime's headers")
+    d = tmp_path_factory.mktemp("host_order")
+    objs = [str(d / name) for name in ("decoder.o", "sequence.o", "host_order.o")]
+    flags = ["-O1", "-g", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-Wno-unused-result", "-Wno-int-in-bool-context", f"-I{HOST}", f"-I{ROOT}/include", "-I/opt/rocm/include"]
+    jobs = [subprocess.Popen(["g++", *flags, "-c", src, "-o", obj])
+            for src, obj in zip([f"{HOST}/decoder.cpp", f"{HOST}/sequence.cpp", f"{ROOT}/tests/host_order.cpp"], objs)]
+    assert all([j.wait() == 0 for j in jobs])
+    # whatever else the sources call succeeds and does nothing
+    names = [set(), set()]
+    for line in subprocess.run(["nm", *objs], capture_output=True, text=True, check=True).stdout.splitlines():
+        if len(line.split()) >= 2 and line.split()[-1].startswith(("hip", "bitnet_hip_")):
+            names[line.split()[-2] in "TW"].add(line.split()[-1])
+    (d / "rest.c").write_text("".join(f"long {n}(void) {{ return 0; }}\n" for n in sorted(names[0] - names[1])))
+    subprocess.run(["gcc", "-c", str(d / "rest.c"), "-o", str(d / "rest.o")], check=True)
+    subprocess.run(["g++", *objs, str(d / "rest.o"), "-o", str(d / "host_order"), "-ldl"], check=True)
+    return str(d / "host_order")
+
+
+@pytest.mark.parametrize("case", ["cache_type"])
+def test_nothing_relies_on_an_order_that_is_not_there(program, case):
+    out = subprocess.run([program, case], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout + out.stderr
