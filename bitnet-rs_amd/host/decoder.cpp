@@ -300,6 +300,7 @@ int Decoder::set_kv_f16(bool on) {
             HCHK(hipMemsetAsync(L.kcache, 0, n * sizeof(float), (hipStream_t)stream_));
             HCHK(hipMemsetAsync(L.vcache, 0, n * sizeof(float), (hipStream_t)stream_));
         }
+        if (int rc = settle()) return rc;  // (the caches' addresses may have been handed out)
     }
     kv_f16_ = on;
     return 0;
@@ -1124,8 +1125,11 @@ void Decoder::layer_objects(int layer, uint64_t handles[4], void *ptrs[4]) const
     ptrs[0] = L.attn_norm, ptrs[1] = L.ffn_norm, ptrs[2] = L.kcache, ptrs[3] = L.vcache;
 }
 
-void Decoder::global_objects(void *ptrs[7]) const {
-    expose();
+void Decoder::global_objects(void *ptrs[7]) {
+    if (expose() != 0) {
+        for (int i = 0; i < 7; ++i) ptrs[i] = nullptr;
+        return;
+    }
     ptrs[0] = embed_, ptrs[1] = final_norm_, ptrs[2] = rope_sin_, ptrs[3] = rope_cos_, ptrs[4] = history_, ptrs[5] = pos_, ptrs[6] = stream_;
 }
 

@@ -124,7 +124,7 @@ class Decoder : public Sequence {
     // pointers {attn_norm, ffn_norm, kcache, vcache}; globals {embed, final_norm, rope_sin, rope_cos,
     // history, pos, stream}.
     void layer_objects(int layer, uint64_t handles[4], void *ptrs[4]) const;
-    void global_objects(void *ptrs[7]) const;
+    void global_objects(void *ptrs[7]);
     int last_hidden(float *out) override;
     // Activation trace of ONE decode step in the reference's format (crates/bitnet-trace/src/lib.rs:46-168: one JSON file per
     // tensor -- name, shape, dtype, blake3 of the raw f32 bytes, rms, num_elements, seq, layer, stage -- in `dir`): the step

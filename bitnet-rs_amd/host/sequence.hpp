@@ -83,7 +83,12 @@ class Sequence {
     void drop_graphs();
     int settle();                       // waits for the stream
     void moved_to(int p) { host_pos_ = exposed_ ? -1 : p; }
-    void expose() const { exposed_ = true, host_pos_ = -1; }  // somebody else may write the device's position and read its history from now on
+    // Somebody else may write the device's position and read its history from now on, on a stream of their own: what was asked for before is done first, and every later call that moves them
+    // waits for it.
+    int expose() {
+        exposed_ = true, host_pos_ = -1;
+        return settle();
+    }
     int update(int first, int n, const int32_t *tokens, bool forced, int pos, const float *row = nullptr, float *x = nullptr);  // (pos < 0: stays)
 
     virtual bool ready() const = 0;                            // weights are there
@@ -98,8 +103,8 @@ class Sequence {
     float *logits_ = nullptr;
     int32_t *pos_ = nullptr, *n_forced_ = nullptr, *history_ = nullptr, *token_ = nullptr;
     int host_forced_ = 0;
-    mutable int host_pos_ = -1;  // *pos_ where it is known: every call that moves it knows where to
-    mutable bool exposed_ = false;
+    int host_pos_ = -1;  // *pos_ where it is known: every call that moves it knows where to
+    bool exposed_ = false;
     // pinned: a clamp count for the model's use, then tokens on their way to the history (staged_: a launch that reads them may be waiting)
     static constexpr int kStaged = 16384;
     int32_t *pinned_ = nullptr;

@@ -131,6 +131,21 @@ int main(int argc, char **argv) {
                 CHECK(*(float *)p[2] == 7.f && *(float *)p[3] == 8.f && ((float *)p[2])[1] == 0.f && ((float *)p[3])[1] == 0.f);
             }
         }
+    } else if (!strcmp(what, "objects")) {  // what is handed out holds what the calls before have put there, and so it stays
+        uint64_t h[4];
+        void *g[7], *p[4];
+        CHECK(d.reset() == 0 && d.feed(tokens, 2) == 0);
+        d.global_objects(g);
+        const int32_t *history = (int32_t *)g[4];
+        int32_t *pos = (int32_t *)g[5];
+        CHECK(history[0] == 11 && history[1] == 12 && *pos == 0);
+        CHECK(d.feed(tokens + 2, 1) == 0 && history[2] == 13);
+        CHECK(d.prefill(3, false, 2, nullptr) == 0 && *pos == 3 && d.position() == 3);
+        *pos = 2;
+        CHECK(d.position() == 2);
+        CHECK(d.reset() == 0 && *pos == 0 && history[0] == 0 && d.set_kv_f16(true) == 0);
+        d.layer_objects(1, h, p);
+        CHECK(*(float *)p[2] == 0.f && *(float *)p[3] == 0.f);
     } else {
         CHECK(!"a case of this name");
     }
