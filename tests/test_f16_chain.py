@@ -372,6 +372,39 @@ def test_chain_on_the_image_is_the_expanding_one_bit_for_bit(hip, torch_, fmt, r
         hip.weights_free(w)
 
 
+@pytest.mark.parametrize("fmt", ["qk256", "i2s"])
+@pytest.mark.parametrize("silu", [0, 1])
+def test_concatenation_of_parts_that_have_images(hip, torch_, fmt, silu):
+    """The images belong to the part: the fused matrix starts without one, builds its own, and either may be freed first."""
+    rows, cols, m = 256, 512, 64
+    rng = np.random.default_rng(silu)
+    parts = [make_matrix(hip, rng, fmt, rows, cols)[0] for _ in range(2)]
+    xh = torch_.from_numpy(rng.normal(0, 1, (m, cols)).astype(np.float16)).cuda()
+    plain, fresh = hip.weights_device_bytes(parts[0]), hip.weights_concat(parts, interleave16=bool(silu))
+
+    def product(h, n):
+        y = torch_.full((m, n), 7.0, dtype=torch_.float16, device="cuda")
+        hip.matmul_f16_dev(h, xh, m, yh=y, flags=0)
+        torch_.cuda.synchronize()
+        return y
+
+    before = product(parts[0], rows)
+    if fmt == "qk256":
+        hip.weights_fp4_image(parts[0], True)
+    image = rows // 16 * (cols // 256) * 2048
+    assert hip.weights_device_bytes(parts[0]) == plain + image * (2 if fmt == "qk256" else 1)
+    h = hip.weights_concat(parts, interleave16=bool(silu))
+    assert hip.weights_device_bytes(h) == 2 * plain
+    want = product(fresh, 2 * rows)
+    assert torch_.equal(product(h, 2 * rows), want) and hip.weights_device_bytes(h) == 2 * plain + 2 * image
+    hip.weights_free(h)
+    assert torch_.equal(product(parts[0], rows), before)
+    hip.weights_free(parts[0])
+    assert torch_.equal(product(fresh, 2 * rows), want)
+    for w in (fresh, parts[1]):
+        hip.weights_free(w)
+
+
 FEW_ROWS = 128
 
 
