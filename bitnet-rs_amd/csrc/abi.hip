@@ -532,6 +532,15 @@ int bitnet_hip_f16_saturations_dev(uint32_t *count, void *stream) {
     BH_GUARD_END
 }
 
+int bitnet_hip_f16_saturations_total_dev(uint32_t *total, void *stream) {
+    BH_GUARD_BEGIN
+    if (!total) return set_error(BITNET_HIP_ERR_INVALID_ARGUMENT, "Null pointer passed to f16_saturations_total_dev");
+    const hipError_t e = launch_f16_saturations_total(total, (hipStream_t)stream);
+    if (e != hipSuccess) return set_error(BITNET_HIP_ERR_GPU, "kernel launch failed: %s", hipGetErrorString(e));
+    return BITNET_HIP_OK;
+    BH_GUARD_END
+}
+
 size_t bitnet_hip_qb32_bytes(size_t m, size_t cols) { return qb32_bytes(m, cols); }
 
 int bitnet_hip_rows_to_qb32_dev(const float *x_dev, const float *gamma_dev, size_t m, size_t cols, void *qb_dev, float *stats_dev, void *stream) {

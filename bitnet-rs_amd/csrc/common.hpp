@@ -237,6 +237,7 @@ hipError_t launch_gemm_qb32(const Weights &w, const GemmF16Io &io, size_t m, hip
 bool gemm_f16_chain_supported(const Weights &w);
 bool gemm_f16_takes_few(const Weights &w, bool silu_mul, size_t m);
 hipError_t launch_f16_saturations(uint32_t *count, hipStream_t stream);
+hipError_t launch_f16_saturations_total(uint32_t *total, hipStream_t stream);
 unsigned long long f16_saturations(bool reset);  // f16 hand-over values clamped to +-65504 since the last reset (lanes, not elements); synchronises the device
 hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m, hipStream_t stream);
 hipError_t launch_rows_to_f16(const float *x, const float *gamma, size_t m, size_t cols, void *xh, float *stats, hipStream_t stream);

@@ -472,7 +472,9 @@ __device__ __forceinline__ void store_out4(float *dst, float a, float b, float c
 
 // f16 hand-over rows are clamped to +-65504 (an f16 element carries its own exponent: no row scale).  A clamp is COUNTED, not silent: the
 // decoder reads the counter behind a prompt forward and repeats the prompt on the row-scaled forms when it is not zero (Decoder::prefill).
-__device__ unsigned int g_f16_saturations = 0;
+// The count only grows: several sequences watch it at once, each for what it added since a look of its own (launch_f16_saturations_total).  What has been given out by those calls that
+// clear it stands beside it.
+__device__ unsigned int g_f16_saturations = 0, g_f16_given = 0;
 __device__ __forceinline__ _Float16 gclamp_f16(float v, bool &sat) {
     sat = sat || !(fabsf(v) <= 65504.0f);  // (also true for NaN)
     return (_Float16)__builtin_amdgcn_fmed3f(v, -65504.0f, 65504.0f);
@@ -481,21 +483,29 @@ __device__ __forceinline__ void gflush_sat(bool sat) {
     if (sat) atomicAdd(&g_f16_saturations, 1u);  // (rare: one atomic per lane that clamped, none otherwise)
 }
 __global__ void k_take_saturations(uint32_t *count) {
-    const uint32_t v = atomicExch(&g_f16_saturations, 0u);
-    if (count) *count = v;
+    uint32_t given, v;
+    do {  // (again only when another taker came in between, who then has got on)
+        given = __hip_atomic_load(&g_f16_given, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+        v = __hip_atomic_load(&g_f16_saturations, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } while (atomicCAS(&g_f16_given, given, v) != given);
+    if (count) *count = v - given;
 }
+__global__ void k_total_saturations(uint32_t *total) { *total = __hip_atomic_load(&g_f16_saturations, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 hipError_t launch_f16_saturations(uint32_t *count, hipStream_t stream) {
     hipLaunchKernelGGL(k_take_saturations, dim3(1), dim3(1), 0, stream, count);
     return hipGetLastError();
 }
+hipError_t launch_f16_saturations_total(uint32_t *total, hipStream_t stream) {
+    hipLaunchKernelGGL(k_total_saturations, dim3(1), dim3(1), 0, stream, total);
+    return hipGetLastError();
+}
 unsigned long long f16_saturations(bool reset) {
-    unsigned int v = 0;
-    if (hipMemcpyFromSymbol(&v, HIP_SYMBOL(g_f16_saturations), sizeof(v)) != hipSuccess) return ~0ull;  // (synchronises the device)
-    if (reset && v) {
-        const unsigned int z = 0;
-        (void)hipMemcpyToSymbol(HIP_SYMBOL(g_f16_saturations), &z, sizeof(z));
-    }
-    return v;
+    unsigned int v = 0, given = 0;
+    if (hipDeviceSynchronize() != hipSuccess || hipMemcpyFromSymbol(&given, HIP_SYMBOL(g_f16_given), sizeof(given)) != hipSuccess ||
+        hipMemcpyFromSymbol(&v, HIP_SYMBOL(g_f16_saturations), sizeof(v)) != hipSuccess)
+        return ~0ull;
+    if (reset && v != given) (void)hipMemcpyToSymbol(HIP_SYMBOL(g_f16_given), &v, sizeof(v));
+    return v - given;
 }
 
 // silu(gate) * up (FeedForward::forward T:756-781, silu(v) = v / (1 + exp(-v))) as the decode GEMV's epilogue computes it (kernels_gemvq.hip):

@@ -779,7 +779,7 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
     }
     hipStream_t s = (hipStream_t)stream_;
     HCHK(hipEventRecord(begin_.e, s));
-    if (!force_scaled_) BCHK(bitnet_hip_f16_saturations_dev(nullptr, s));  // a fresh count for this prompt
+    if (!force_scaled_) BCHK(bitnet_hip_f16_saturations_total_dev((uint32_t *)pinned_, s));  // the clamps ahead of this prompt
     const size_t N = (size_t)n;
     BCHK(bitnet_hip_embed_f16_dev(embed_, history_, pos_, N, H, (size_t)c_.vocab, pf_x_, s));  // *pos_ == 0
     const bool chain = chain_applies(digits);
@@ -843,11 +843,11 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
     }
     if (chain || qb || h16) {
         // f16 hand-over rows carry no row scale: a value beyond +-65504 (outlier channels x gamma: none in the synthetic models, possible in a real
-        // checkpoint) is clamped AND counted (bitnet_hip_f16_saturations).  A prompt that clamped anything is repeated on the digit planes --
+        // checkpoint) is clamped AND counted (the device's count: another sequence's clamp may show here, too).  A prompt during which it grew is repeated on the digit planes --
         // 30-bit fixed point behind a per-row power-of-two scale (digits = 4: a row whose outlier is 10^5 times its typical element still keeps 13 bits of
         // those; the 2-digit and row-scaled f16 forms would flush them): no silent saturation.  The count is looked at once the logits are there, too, which
         // a second pass then writes over: the device does not wait for the host in between.
-        BCHK(bitnet_hip_f16_saturations_dev((uint32_t *)pinned_, s));
+        BCHK(bitnet_hip_f16_saturations_total_dev((uint32_t *)pinned_ + 1, s));
     }
     {
         const int rc = hand_over(n, pf_x_ + (N - 1) * H, with_logits);
@@ -855,7 +855,7 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
     }
     HCHK(hipEventRecord(end_.e, s));
     if (int rc = settle()) return rc;
-    if ((chain || qb || h16) && pinned_[0] != 0) {
+    if ((chain || qb || h16) && pinned_[0] != pinned_[1]) {
         if (int rc = update(0, 0, nullptr, false, 0)) return rc;
         force_scaled_ = true;
         ++saturation_fallbacks_;

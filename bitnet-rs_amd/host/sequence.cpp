@@ -29,7 +29,7 @@ int Sequence::init_sequence(int vocab, int width, int max_pos) {
     HCHK(hipMalloc((void **)&n_forced_, 4));
     HCHK(hipMalloc((void **)&token_, 4));
     HCHK(hipMalloc((void **)&history_, ((size_t)max_pos + 2) * 4));
-    HCHK(hipHostMalloc((void **)&pinned_, (1 + (size_t)kStaged) * 4, hipHostMallocCoherent));
+    HCHK(hipHostMalloc((void **)&pinned_, ((size_t)kCounts + kStaged) * 4, hipHostMallocCoherent));
     HCHK(hipEventCreate(&begin_.e));
     HCHK(hipEventCreate(&end_.e));
     return 0;
@@ -91,9 +91,9 @@ int Sequence::feed(const int32_t *tokens, int n) {
         const int part = n - i < kStaged ? n - i : kStaged;
         if (i > 0)
             if (int rc = settle()) return rc;
-        if (part > 0) memcpy(pinned_ + 1, tokens + i, (size_t)part * 4);
+        if (part > 0) memcpy(pinned_ + kCounts, tokens + i, (size_t)part * 4);
         host_forced_ = base + i + part;
-        if (int rc = update(base + i, part, pinned_ + 1, true, -1)) return rc;
+        if (int rc = update(base + i, part, pinned_ + kCounts, true, -1)) return rc;
         staged_ = true;
     }
     return exposed_ ? settle() : 0;

@@ -105,8 +105,8 @@ class Sequence {
     int host_forced_ = 0;
     int host_pos_ = -1;  // *pos_ where it is known: every call that moves it knows where to
     bool exposed_ = false;
-    // pinned: a clamp count for the model's use, then tokens on their way to the history (staged_: a launch that reads them may be waiting)
-    static constexpr int kStaged = 16384;
+    // pinned: clamp counts for the model's use, then tokens on their way to the history (staged_: a launch that reads them may be waiting)
+    static constexpr int kCounts = 2, kStaged = 16384;
     int32_t *pinned_ = nullptr;
     bool staged_ = false;
     Event begin_, end_;  // of the last run or prefill

@@ -298,10 +298,14 @@ int bitnet_hip_weights_fp4_image(bitnet_hip_weights_t h, int enable, void *strea
  * that clamped a value of a live token since the last reset, in any of the chain's writers (bitnet_hip_rows_to_f16_dev, the yh outputs of
  * bitnet_hip_matmul_f16_dev / _matmul_qb32_dev / FUSE_Y_F16); reset != 0 clears it.  Synchronises the device.  A host that cannot rule such
  * activations out (outlier channels x gamma beyond the f16 range) checks it behind a prompt and repeats the prompt on the row-scaled forms
- * (bitnet_hip_matmul_fused_dev), as Decoder::prefill does. */
+ * (bitnet_hip_matmul_fused_dev), as Decoder::prefill does.
+ * The count is the device's: where several sequences run at once, a call that clears it takes it from all of them.  They compare
+ * bitnet_hip_f16_saturations_total_dev ahead of a prompt and behind it instead (a neighbour's clamp may cost a repeat, none is missed). */
 unsigned long long bitnet_hip_f16_saturations(int reset);
 /* The same count stored at `count` (device or pinned host memory; nullable) and cleared, in stream order and without a synchronisation. */
 int bitnet_hip_f16_saturations_dev(uint32_t *count, void *stream);
+/* All clamps since the library was loaded (modulo 2^32), stored at `total` (device or pinned host memory) in stream order: nothing clears it. */
+int bitnet_hip_f16_saturations_total_dev(uint32_t *total, void *stream);
 int bitnet_hip_matmul_f16_supported(bitnet_hip_weights_t w);
 int bitnet_hip_rows_to_f16_dev(const float *x_dev, const float *gamma_dev, size_t m, size_t cols, void *xh_dev, float *stats_dev, void *stream);
 int bitnet_hip_matmul_f16_dev(bitnet_hip_weights_t w, const void *xh_dev, size_t m, const float *stats_in_dev, size_t n_stats,

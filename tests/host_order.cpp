@@ -25,10 +25,10 @@ void run_all() {
     run(g_null);
     for (Queue *q : g_streams) run(*q);
 }
-uint64_t g_clamped = 0, g_taken = 0;  // the device's count, and what of it f16_saturations_dev has given out
+uint32_t g_clamped = 0, g_taken = 0;  // the device's count, and what of it f16_saturations_dev has given out
 int g_clamping = 0;                   // the next product clamps, and somebody else takes the count at once
-uint64_t take() {
-    const uint64_t n = g_clamped - g_taken;
+uint32_t take() {
+    const uint32_t n = g_clamped - g_taken;
     g_taken = g_clamped;
     return n;
 }
@@ -93,11 +93,12 @@ int bitnet_hip_matmul_f16_dev(bitnet_hip_weights_t, const void *, size_t, const 
 int bitnet_hip_advance_pos_dev(int32_t *pos, void *s) { return queue(s).push_back([=] { ++*pos; }), 0; }
 int bitnet_hip_f16_saturations_dev(uint32_t *count, void *s) {
     queue(s).push_back([=] {
-        const uint64_t n = take();
-        if (count) *count = (uint32_t)n;
+        const uint32_t n = take();
+        if (count) *count = n;
     });
     return 0;
 }
+int bitnet_hip_f16_saturations_total_dev(uint32_t *total, void *s) { return queue(s).push_back([=] { *total = g_clamped; }), 0; }
 }
 
 using bitnet_host::Decoder;
@@ -146,6 +147,14 @@ int main(int argc, char **argv) {
         CHECK(d.reset() == 0 && *pos == 0 && history[0] == 0 && d.set_kv_f16(true) == 0);
         d.layer_objects(1, h, p);
         CHECK(*(float *)p[2] == 0.f && *(float *)p[3] == 0.f);
+    } else if (!strcmp(what, "clamps")) {  // a clamp is not lost to a sequence beside this one that takes the count meanwhile
+        for (int n : {0, 1, 0, 2}) {
+            const int before = d.saturation_fallbacks();
+            g_clamping = n;
+            CHECK(d.reset() == 0 && prompt() == 0 && d.position() == 3);
+            CHECK(d.saturation_fallbacks() == before + (n > 0));
+            bitnet_hip_f16_saturations_dev(nullptr, d.stream());
+        }
     } else {
         CHECK(!"a case of this name");
     }

@@ -262,6 +262,37 @@ def test_f16_hand_over_saturation_is_counted_and_the_decoder_falls_back(pkg, hip
     dec.close()
 
 
+def test_clamps_seen_by_one_sequence_are_not_taken_from_another(hip, torch_):
+    """The running total on one stream, takers that clear the count on others: each taker gets what came since the last, the total misses nothing."""
+    import ctypes as C
+
+    streams = [torch_.cuda.Stream() for _ in range(3)]
+    m, cols = 64, 512
+    x, g = torch_.full((m, cols), 1e5, device="cuda"), torch_.ones(cols, device="cuda")
+    xh, out = torch_.zeros(m, cols, dtype=torch_.float16, device="cuda"), torch_.full((8,), 77, dtype=torch_.int32).pin_memory()
+    P = lambda i: C.c_void_p(out.data_ptr() + 4 * i)
+    S = lambda i: C.c_void_p(streams[i].cuda_stream)
+    torch_.cuda.synchronize()
+    hip.f16_saturations(True)
+    hip._call("f16_saturations_total_dev", P(0), S(0))
+    for i in (1, 2):
+        with torch_.cuda.stream(streams[i]):
+            hip.rows_to_f16_dev(x, g, m, cols, xh, None, stream=streams[i].cuda_stream)
+        hip._call("f16_saturations_dev", P(i), S(i))
+        torch_.cuda.synchronize()
+    hip._call("f16_saturations_dev", None, S(0))
+    hip._call("f16_saturations_total_dev", P(3), S(0))
+    torch_.cuda.synchronize()
+    before, a, b, after = out[:4].tolist()
+    lanes = m * cols // 4
+    assert (a, b) == (lanes, lanes) and (after - before) % 2 ** 32 == 2 * lanes
+    assert hip.f16_saturations(True) == 0
+    hip.rows_to_f16_dev(x, g, m, cols, xh, None)
+    assert hip.f16_saturations(False) == lanes and hip.f16_saturations(True) == lanes and hip.f16_saturations(True) == 0
+    with pytest.raises(Exception, match="Null pointer"):
+        hip._call("f16_saturations_total_dev", None, S(0))
+
+
 _F16H_HASH_SCRIPT = r"""
 import hashlib, importlib, sys
 import numpy as np, torch

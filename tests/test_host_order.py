@@ -31,7 +31,7 @@ def program(tmp_path_factory):
     return str(d / "host_order")
 
 
-@pytest.mark.parametrize("case", ["cache_type", "objects"])
+@pytest.mark.parametrize("case", ["cache_type", "objects", "clamps"])
 def test_nothing_relies_on_an_order_that_is_not_there(program, case):
     out = subprocess.run([program, case], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
