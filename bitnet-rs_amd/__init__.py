@@ -521,7 +521,7 @@ class HipLib:
         return int(self.c.bitnet_hip_weights_device_bytes(h))
 
     def weights_fp4_image(self, h: int, enable: bool = True, stream: int = 0) -> None:
-        """Build (or free) the resident fp4 image the fp6 x fp4 prompt matmul reads (include/bitnet_hip.h)."""
+        """Build the resident fp4 image the fp6 x fp4 prompt matmul reads, or free it and the f16 chain's (include/bitnet_hip.h)."""
         self.c.bitnet_hip_weights_fp4_image.argtypes = [C.c_uint64, C.c_int, C.c_void_p]
         self._check(self.c.bitnet_hip_weights_fp4_image(h, 1 if enable else 0, stream))
 

@@ -677,6 +677,7 @@ int bitnet_hip_weights_concat(const bitnet_hip_weights_t *parts, size_t n_parts,
     f->tiles = nullptr;
     f->tiles4 = nullptr;  // (a part may have images of its own by now)
     f->tiles4_pairs = nullptr;
+    f->pairs_failed = false;
     f->scale_tiles = nullptr;
     f->scale_tiles_h = nullptr;
     f->ln_g = nullptr;

@@ -104,6 +104,7 @@ struct Weights {
     // resident fp4 image for the prompt matmul's fp6 x fp4 form (kernels_gemm.hip k_retile_fp4 / ensure_fp4_image): optional, 4 bits per weight
     uint8_t *tiles4 = nullptr;
     uint8_t *tiles4_pairs = nullptr;  // ... and the f16 chain's (k_retile_pairs / want_pair_image)
+    bool pairs_failed = false;        // there was no memory for it
     float *scale_tiles = nullptr;  // 32-block scales in tile order (kernels_mfma.hip k_retile_scales)
     // Every scale is exactly an f16 value (BitNet32-F16 files store them so): the streaming layout
     // keeps them as f16 (2 bytes per 32 weights instead of 4) -- same numbers, fewer bytes.

@@ -2578,13 +2578,14 @@ static hipError_t build_image(Weights &w, uint8_t *Weights::*image, void (*retil
     return hipSuccess;
 }
 hipError_t ensure_fp4_image(Weights &w, hipStream_t stream) { return gemm_fp6_supported(w) ? build_image(w, &Weights::tiles4, k_retile_fp4, stream) : hipErrorInvalidValue; }
-// The image of the f16 chain's kernels (Weights::tiles4_pairs; it stays as long as the matrix does), or null where it cannot be had -- the stream captures, or memory is short --:
-// then the kernels expand the codes themselves, to the same values.  Another thread may be capturing: an allocation on behalf of this stream does not concern it.
+// The image of the f16 chain's kernels (Weights::tiles4_pairs; until the matrix goes or a host gives it back: drop_fp4_image), or null where it cannot be had -- the stream captures, or
+// memory is short, which is asked for once and not on every launch --: then the kernels expand the codes themselves, to the same values.  Another thread may be capturing: an allocation
+// on behalf of this stream does not concern it.
 const uint8_t *want_pair_image(Weights &w, hipStream_t stream) {
     if (!gemm_fp4_resident_enabled() || !gemm_f16_chain_supported(w)) return nullptr;
     {
         std::lock_guard<std::mutex> lk(*w.mu);
-        if (w.tiles4_pairs) return w.tiles4_pairs;
+        if (w.tiles4_pairs || w.pairs_failed) return w.tiles4_pairs;
     }
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
@@ -2594,17 +2595,18 @@ const uint8_t *want_pair_image(Weights &w, hipStream_t stream) {
     }
     const hipError_t e = build_image(w, &Weights::tiles4_pairs, k_retile_pairs, stream);
     (void)hipThreadExchangeStreamCaptureMode(&mode);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    if (e != hipSuccess) (void)hipGetLastError();
     std::lock_guard<std::mutex> lk(*w.mu);
+    w.pairs_failed = e == hipErrorOutOfMemory;
     return w.tiles4_pairs;
 }
 void drop_fp4_image(Weights &w) {
     std::lock_guard<std::mutex> lk(*w.mu);
-    if (w.tiles4) (void)hipFree(w.tiles4);
-    w.tiles4 = nullptr;
+    for (uint8_t **image : {&w.tiles4, &w.tiles4_pairs}) {
+        if (*image) (void)hipFree(*image);
+        *image = nullptr;
+    }
+    w.pairs_failed = false;
 }
 // would launch_gemm_mfma send this call to k_gemm_fp6? (the ABI asks before the launch, to build the image outside it)
 bool gemm_takes_fp6(const Weights &w, const GemvFusion &fu, int ndig) {

@@ -270,8 +270,9 @@ int bitnet_hip_matmul_last_resident_fp4(void);
  * bitnet_hip_weights_device_bytes counts both; QK256 2B-4T: q|k|v + gate|up of 30 layers = 678 MB, all seven projections 1.04 GB --
  * HBM is 288 GB).  With it bitnet_hip_matmul_fused_dev's BITNET_HIP_FUSE_FP6_DIGITS form loads its weight operands directly: no code
  * expansion in the K loop; the integers multiplied are the same, so the results stay bit-identical to the int8 digit planes.
- * enable = 1 builds it (idempotent; an allocation + one kernel, synchronises `stream`), 0 frees it.  Without this call the first
- * fp6-form launch on the handle builds it (not under stream capture); BITNET_HIP_FP4_RESIDENT=0 disables the image altogether.
+ * enable = 1 builds it (idempotent; an allocation + one kernel, synchronises `stream`), 0 frees it, and with it the image of the f16 chain (bitnet_hip_matmul_f16_dev, below; the
+ * only one of a matrix with block scales): no captured launch may hold them.  Without this call the first
+ * fp6-form launch on the handle builds it (not under stream capture); BITNET_HIP_FP4_RESIDENT=0 disables the images altogether.
  * Replaces nothing in the reference: its loader keeps one packed copy (crates/bitnet-quantization/src/i2s_qk256.rs:66-128). */
 int bitnet_hip_weights_fp4_image(bitnet_hip_weights_t h, int enable, void *stream);
 
@@ -289,9 +290,10 @@ int bitnet_hip_weights_fp4_image(bitnet_hip_weights_t h, int enable, void *strea
  *                  (sum, sum of squares) over disjoint row ranges that together cover the row -- one per wave of the producing launch
  *                  (64 rows, or 80 in 320-row workgroups: then the first rows / 80 entries are used and the others are written as zero);
  *                  the consumer adds all rows / 64 entries up (n_stats = rows / 64).
- * The first call on a matrix builds an image of it, the codes as fp4 in the order of this form's operands, 4 bits per weight that bitnet_hip_weights_device_bytes counts (an
- * allocation + one kernel, synchronises `stream`); under stream capture, without memory for it or with BITNET_HIP_FP4_RESIDENT=0 the codes are expanded in the K loop instead, to
- * the same values.
+ * The first call on a matrix (but with BITNET_HIP_FUSE_FEW_ROWS) builds an image of it, the codes as fp4 in the order of this form's operands, 4 bits per weight that
+ * bitnet_hip_weights_device_bytes counts (an allocation + one kernel, synchronises `stream`; 1.04 GB for all projections of the 2B-4T model, 363 MB for QK256's o and down);
+ * bitnet_hip_weights_fp4_image(w, 0) gives it back, and a later call builds it again.  Under stream capture, without memory for it (then it is not tried again until that call) or with
+ * BITNET_HIP_FP4_RESIDENT=0 the codes are expanded in the K loop instead, to the same values: a host that captures makes one call outside of the capture first.
  * bitnet_hip_matmul_f16_supported: rows % 256 == 0, cols % 256 == 0, code map values in -2..2, no scales or f16 32-block scales.
  * bitnet_hip_rows_to_f16_dev: the chain's entry (the embedding rows): xh = f16(gamma * x) (gamma nullable) + stats partial 0. */
 /* f16 hand-over rows carry no row scale: a value beyond +-65504 is clamped -- and COUNTED.  Returns the number of lanes (up to four elements each)

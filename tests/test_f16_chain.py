@@ -399,6 +399,13 @@ def test_chain_on_the_image_is_the_expanding_one_bit_for_bit(hip, torch_, fmt, r
     assert hip.weights_device_bytes(h) == b0 + rows // 16 * (cols // 256) * 2048
     for a, b in zip(expanded, image):
         assert a is None or (torch_.isfinite(a).all() and torch_.equal(a, b))
+    hip.weights_fp4_image(h, False)  # given back, and built again where it is wanted again
+    assert hip.weights_device_bytes(h) == b0
+    again = buffers()
+    launch(again, torch_.cuda.current_stream().cuda_stream)
+    torch_.cuda.synchronize()
+    assert hip.weights_device_bytes(h) == b0 + rows // 16 * (cols // 256) * 2048
+    assert all(a is None or torch_.equal(a, b) for a, b in zip(again, image))
     for w in (h, *parts):
         hip.weights_free(w)
 
