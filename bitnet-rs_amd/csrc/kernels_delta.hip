@@ -35,8 +35,8 @@ struct StepLds {
     float slot[16];
 };
 
-// S and the output of one token from q, k, v in LDS; threads below vdimp return o
-template <int NJ>
+// S and the output of one token from q, k, v in LDS, AH slices in flight where they meet; threads below vdimp return o
+template <int NJ, int AH>
 __device__ __forceinline__ float delta_token(StepLds &w, float (&s)[NJ], int dimp, int vdimp, int v, int sl, int SL, bool live, float g, float beta) {
     const int tid = threadIdx.x, lane = tid & 63;
     float a = 0.f, b = 0.f, kq = 0.f;
@@ -55,7 +55,6 @@ __device__ __forceinline__ float delta_token(StepLds &w, float (&s)[NJ], int dim
     float o = 0.f;
     if (tid < vdimp) {
         a = b = 0.f;
-        constexpr int AH = 8;  // slices in flight
         for (int i0 = 0; i0 < SL; i0 += AH) {
             float x[AH], y[AH];
 #pragma unroll
@@ -87,7 +86,8 @@ __device__ __forceinline__ float head_sum(float v, float *slot) {
 }
 
 // A chain of latencies like the attention's step: what the host knows is divided there (shift: log2 of vdimp, or -1), the grid holds the key head and the head within it, and slices meet
-// in LDS eight at a time: 24 heads of 128 / 128 inside a step 8.4 -> 7.7 us.
+// in LDS eight at a time: 24 heads of 128 / 128 inside a step 8.4 -> 7.7 us, 8 of 256 / 128 11.0 -> 10.2.  One at a time where the state fills the registers, which eight would be spilled
+// for: 24 heads of 256 / 256 24.4 us (eight: 27.2), 16 of 192 / 256 17.2 (19.4).
 template <int NJ>
 __global__ __launch_bounds__(kStepThreads) void k_delta_step(Delta p, int SL, int shift, const float *row, const float *ba, const int *pos_ptr, float *out) {
     __shared__ StepLds w;
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(kStepThreads) void k_delta_step(Delta p, int SL, in
     }
     const float g = expf(log_decay(p, h, araw)), beta = 1.0f / (1.0f + expf(-braw));
     __syncthreads();
-    const float o = delta_token<NJ>(w, s, dimp, vdimp, v, sl, SL, live, g, beta);
+    const float o = delta_token<NJ, (NJ > 32 ? 1 : 8)>(w, s, dimp, vdimp, v, sl, SL, live, g, beta);
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
         if (live && sl + SL * j < dimp) st[(size_t)(sl + SL * j) * vdimp + v] = s[j];
@@ -148,6 +148,7 @@ __global__ __launch_bounds__(kStepThreads) void k_delta_step(Delta p, int SL, in
     if (tid < vdimp) out[(size_t)h * vdimp + tid] = o * inv * weight * silu(gate);
 }
 
+// (eight slices here, spills and all: 64 tokens of 24 heads of 256 / 256 824 us with eight, 797 one at a time, 16 heads of 192 / 256 606 and 748, of 256 / 160 534 and 736)
 template <int NJ, class T>
 __global__ __launch_bounds__(kStepThreads) void k_delta_recurrent(Delta p, const float *qk, const T *vr, const float *gates, const T *rows, size_t ld, int n, T *out,
                                                                   size_t ldo) {
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(kStepThreads) void k_delta_recurrent(Delta p, const
         }
         const float g = expf(gates[(size_t)t * 2 * heads + h]), beta = gates[(size_t)t * 2 * heads + heads + h];
         __syncthreads();
-        const float o = delta_token<NJ>(w, s, dimp, vdimp, v, sl, SL, live, g, beta);
+        const float o = delta_token<NJ, 8>(w, s, dimp, vdimp, v, sl, SL, live, g, beta);
         const float inv = 1.0f / sqrtf(head_sum(o * o, w.slot) / (float)p.vdim + p.eps);  // (its barriers also end this token's reads of q, k, v)
         if (tid < vdimp) st_act(out + (size_t)t * ldo, (size_t)h * vdimp + tid, o * inv * p.norm[tid] * silu(ld_act(rows + (size_t)t * ld, C + (size_t)h * vdimp + tid)));
     }

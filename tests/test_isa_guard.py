@@ -230,6 +230,16 @@ def test_fp6w_k_loop_mixes_dma_and_tracked_loads_without_a_counted_wait(isa):
     assert len(waits) == 1 and "vmcnt(0)" in waits[0], waits
 
 
+def test_delta_rule_spills_only_where_a_head_fills_the_registers(tmp_path):
+    """Heads of 256 x 256 hold 64 numbers of the state per thread and 16 waves share a CU: what is spilled there is bounded, nothing else spills."""
+    if not os.path.exists(HIPCC):
+        pytest.skip("no hipcc")
+    _, usage = _compile("kernels_delta.hip", str(tmp_path))
+    for name, u in usage.items():
+        limit = 84 if "k_delta_stepILi64E" in name else 188 if "k_delta_recurrentILi64E" in name else 0
+        assert u["ScratchSize"] <= limit, (name, u)
+
+
 def test_matrix_vector_products_keep_no_scratch(tmp_path):
     """Every instance of k_dense_gemv, those with convolutions, tables, pairs and gates too, keeps its arguments in registers; and an instance alone on its SIMD has nothing to run
     while it waits for weights"""
