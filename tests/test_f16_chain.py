@@ -446,6 +446,20 @@ def test_concatenation_of_parts_that_have_images(hip, torch_, fmt, silu):
 FEW_ROWS = 128
 
 
+# the last number of tokens that takes the form: one round of workgroups, their number past it (longer rows: more), and the token rows within an XCD's L2
+@pytest.mark.parametrize("rows,cols,silu,last", [(2560, 2560, 0, 144), (3840, 2560, 0, 96), (2560, 6912, 0, 192), (13824, 2560, 1, 16), (1024, 512, 0, 256), (256, 2048, 0, 1024), (1024, 8192, 0, 256),
+                                                 (1024, 512, 1, 256), (4096, 2048, 1, 64), (512, 4096, 0, 512), (1024, 1024, 0, 352),
+                                                 (1536, 6912, 0, 240)])
+def test_f16_few_rows_only_where_they_are_faster(hip, rows, cols, silu, last):
+    rng = np.random.default_rng(rows)
+    for fmt in ("qk256", "i2s"):
+        parts = [make_matrix(hip, rng, fmt, rows // 2, cols)[0] for _ in range(2)]
+        h = hip.weights_concat(parts, interleave16=bool(silu))
+        assert [hip.matmul_f16_takes_few_rows(h, m, silu) for m in (1, last - 1, last, last + 1, 2 * last, 4096)] == [True, True, True, False, False, False]
+        for w in (h, *parts):
+            hip.weights_free(w)
+
+
 # rows x cols x tokens: one, two and four row tiles per workgroup, one block of K (waves without work) to 27, whole and ragged token tiles, pairs
 @pytest.mark.parametrize("fmt", ["qk256", "i2s"])
 @pytest.mark.parametrize("rows,cols,m,silu,tile", [(256, 256, 1, 0, 16), (2560, 2560, 16, 0, 16), (2560, 768, 17, 0, 32), (2560, 6912, 100, 0, 32), (3840, 2304, 64, 0, 64), (13824, 512, 16, 1, 64),
