@@ -803,10 +803,10 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
     // rounding of values that were rounded to f16 already; q|k|v and gate|up keep the faster int8 digit planes behind their LayerNorm.
     // Below 2497 tokens, too, since the f16 form has tiles for few rows and reads fp4: us of a prompt with o / down / both in f16 against the digits of 15 bits behind a quantiser, QK256 weights
     // of bitnet-b1.58-2B-4T: 8 tokens -81 / -109 / -198 (of 1683), 64 -75 / -111 / -201, 128 -65 / -99 / -186, 256 -225 / -463 / -697 (of 3947), 777 -218 / -563 / -815, 1531 -184 / -434 /
-    // -681, 2048 -53 / -40 / -171.  Down keeps its digits from 1024 to 2496 tokens: the launch is held to that instance by its parity test.
+    // -681, 2048 -53 / -40 / -171; down between 1024 and 2496 tokens: 1024 -510, 1281 -510, 1537 -960, 1665 -80, 1800 -60, 2048 -270, 2305 -120, 2496 -490.  Distance of a down-projection of
+    // given f16 rows to float64: 3.9e-7, the digits' 2.8e-4.
     const bool f16_rows = h16 && f16_rows_apply();
     auto few16 = [&](bitnet_hip_weights_t h) { return bitnet_hip_matmul_f16_takes_few_rows(h, N, 0) == 1 ? BITNET_HIP_FUSE_FEW_ROWS : 0; };
-    const bool o16 = f16_rows, down16 = f16_rows && (N < 1024 || hybrid_applies(N));
     // (with few rows the int8 digits have a form of their own, k_gemm_few: the kernel library says where it is the faster one; the same outputs bit for bit)
     auto f6 = [&](bitnet_hip_weights_t h, int flags) { return bitnet_hip_matmul_takes_few_rows(h, N, flags, digits) == 1 ? 0 : fp6_flag(digits); };
     static const int f6od_env = getenv("BITNET_HOST_PREFILL_FP6_OD") ? atoi(getenv("BITNET_HOST_PREFILL_FP6_OD")) : 0;  // experiment: o / down on the fp6 form too (non-hybrid)
@@ -818,13 +818,13 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
             BCHK(bitnet_hip_attention_prefill_flags_dev(pf_qkv_, rope_sin_, rope_cos_, L.kcache, L.vcache, (size_t)c_.n_heads, (size_t)c_.n_kv_heads, (size_t)c_.head_dim,
                                                         (size_t)c_.max_pos, N, pf_attn_ws_, pf_attn_ws_bytes_, pf_atth_,
                                                         (kv_f16_ ? BITNET_HIP_ATTN_CACHE_F16 : 0) | BITNET_HIP_ATTN_OUT_F16, s));
-            if (o16)
+            if (f16_rows)
                 BCHK(bitnet_hip_matmul_f16_dev(L.o, pf_atth_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, few16(L.o), nullptr, nullptr, nullptr, s));
             else
                 BCHK(bitnet_hip_matmul_fused_dev(L.o, (const float *)pf_atth_, pf_x_, N, nullptr, 0.f, pf_x_, BITNET_HIP_FUSE_X_F16 | f6od(L.o, BITNET_HIP_FUSE_X_F16), digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
             BCHK(bitnet_hip_matmul_fused_dev(L.gateup, pf_x_, (float *)pf_hh_, N, L.ffn_norm, c_.eps, nullptr, BITNET_HIP_FUSE_SILU_MUL | BITNET_HIP_FUSE_Y_F16 | f6(L.gateup, BITNET_HIP_FUSE_SILU_MUL), digits,
                                              pf_gemm_ws_, pf_gemm_ws_bytes_, s));
-            if (down16)
+            if (f16_rows)
                 BCHK(bitnet_hip_matmul_f16_dev(L.down, pf_hh_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, few16(L.down), nullptr, nullptr, nullptr, s));
             else
                 BCHK(bitnet_hip_matmul_fused_dev(L.down, (const float *)pf_hh_, pf_x_, N, nullptr, 0.f, pf_x_, BITNET_HIP_FUSE_X_F16 | f6od(L.down, BITNET_HIP_FUSE_X_F16), digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
