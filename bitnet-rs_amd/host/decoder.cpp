@@ -606,8 +606,7 @@ int Decoder::fp6_flag(int digits) {
     return prefill_fp6_ ? BITNET_HIP_FUSE_FP6_DIGITS : 0;
 }
 
-// May o and down take their f16 rows as they stand?  (Decoder::prefill explains; BITNET_HOST_PREFILL_HYBRID=0 keeps the int8 digit planes for all four projections, =2 takes the f16 form
-// at any length.)
+// May o and down take their f16 rows as they stand?  (Decoder::prefill explains; BITNET_HOST_PREFILL_HYBRID=0 keeps the int8 digit planes for all four projections.)
 static int hybrid_mode() {
     static const int mode = getenv("BITNET_HOST_PREFILL_HYBRID") ? atoi(getenv("BITNET_HOST_PREFILL_HYBRID")) : 1;
     return mode;
@@ -619,13 +618,10 @@ bool Decoder::f16_rows_apply() const {
     return true;
 }
 
-// Both of them whatever the length, one rank's share included: only for long shares -- where the hidden-row launches of 64-token tiles come to 400 workgroups or more (from 2497 tokens at
-// hidden 2560: 40 token tiles x 10 row blocks): measured, QK256, same box -- 4096 tokens 21.5 -> 20.3 ms, 3072 tokens 17.3 -> 16.4, 8192 tokens 45.3 -> 43.4, but 2048
-// tokens 11.8 -> 12.0 and 1024 tokens (also one rank's share of the 8-GPU prompt) 7.2 -> 7.8 ms.
-bool Decoder::hybrid_applies(size_t n_rows) const {
-    if (hybrid_mode() != 2 && ((size_t)c_.hidden / 256) * ((n_rows + 63) / 64) < 400) return false;
-    return f16_rows_apply();
-}
+int Decoder::few_rows_flag(bitnet_hip_weights_t h, size_t m) const { return bitnet_hip_matmul_f16_takes_few_rows(h, m, 0) == 1 ? BITNET_HIP_FUSE_FEW_ROWS : 0; }
+
+// Do their launches run 64-token tiles, which the QB32 hand-over needs?  (from 400 workgroups on: 2497 tokens at hidden 2560, 40 token tiles x 10 row blocks)
+bool Decoder::wide_rows_apply(size_t n_rows) const { return ((size_t)c_.hidden / 256) * ((n_rows + 63) / 64) >= 400 && f16_rows_apply(); }
 
 int Decoder::ensure_chain_buffers(size_t N) {
     const size_t H = c_.hidden, QD = (size_t)c_.n_heads * c_.head_dim, F = c_.ffn;
@@ -683,9 +679,9 @@ int Decoder::prefill_chain_layers(size_t N) {
 
 // The QK256 prompt forward with NO row quantiser launch (round 5): q|k|v and gate|up run the fp6 x fp4 form on QB32 rows -- block-scaled 15-bit
 // fixed point, one exponent per 32 columns of a token -- that the kernel PRODUCING the residual stream wrote: the o- / down-projection (f16 matrix
-// cores, 320-row workgroups: the hybrid forward's launches) leaves x (f32), QB32(gamma_next * x) and the LayerNorm statistics partials in its
-// epilogue (BITNET_HIP_FUSE_YH_QB32); LayerNorm is applied after the product (as on the f16 chain and in the decode step).  Only where the hybrid
-// forward applies (long prompts: the producers then run 64-token tiles) and every q|k|v / gate|up matrix takes the form.  OPT-IN
+// cores, 320-row workgroups) leaves x (f32), QB32(gamma_next * x) and the LayerNorm statistics partials in its
+// epilogue (BITNET_HIP_FUSE_YH_QB32); LayerNorm is applied after the product (as on the f16 chain and in the decode step).  Only for long
+// prompts (wide_rows_apply: the producers then run 64-token tiles) and where every q|k|v / gate|up matrix takes the form.  OPT-IN
 // (BITNET_HOST_PREFILL_QB32=1): measured same-box it is a tie with the quantiser launches (18.91-18.93 vs 18.97-19.00 ms at 4096 tokens: the 41.5 us of
 // quantisers per layer come back as +17 / +6.5 us in gate|up / q|k|v and +9 us per producing launch -- the prompt forward runs at a power limit, and the
 // memory-bound quantisers were also the matrix pipes' rest: EXPERIMENTS 8.3), and the default keeps the form that is bit-identical to the int8 planes.
@@ -694,7 +690,7 @@ bool Decoder::qb32_applies(int digits, size_t n_rows) {
         const char *e = getenv("BITNET_HOST_PREFILL_QB32");
         prefill_qb32_ = e ? (atoi(e) != 0 ? 1 : 0) : 0;
     }
-    if (force_scaled_ || !prefill_qb32_ || digits != 2 || !handover16_applies(digits) || !hybrid_applies(n_rows) || !fp6_flag(digits)) return false;
+    if (force_scaled_ || !prefill_qb32_ || digits != 2 || !handover16_applies(digits) || !wide_rows_apply(n_rows) || !fp6_flag(digits)) return false;
     for (const auto &L : layers_)
         for (bitnet_hip_weights_t h : {L.qkv, L.gateup})
             if (!h || bitnet_hip_matmul_qb32_supported(h) != 1) return false;
@@ -806,7 +802,6 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
     // -681, 2048 -53 / -40 / -171; down between 1024 and 2496 tokens: 1024 -510, 1281 -510, 1537 -960, 1665 -80, 1800 -60, 2048 -270, 2305 -120, 2496 -490.  Distance of a down-projection of
     // given f16 rows to float64: 3.9e-7, the digits' 2.8e-4.
     const bool f16_rows = h16 && f16_rows_apply();
-    auto few16 = [&](bitnet_hip_weights_t h) { return bitnet_hip_matmul_f16_takes_few_rows(h, N, 0) == 1 ? BITNET_HIP_FUSE_FEW_ROWS : 0; };
     // (with few rows the int8 digits have a form of their own, k_gemm_few: the kernel library says where it is the faster one; the same outputs bit for bit)
     auto f6 = [&](bitnet_hip_weights_t h, int flags) { return bitnet_hip_matmul_takes_few_rows(h, N, flags, digits) == 1 ? 0 : fp6_flag(digits); };
     static const int f6od_env = getenv("BITNET_HOST_PREFILL_FP6_OD") ? atoi(getenv("BITNET_HOST_PREFILL_FP6_OD")) : 0;  // experiment: o / down on the fp6 form too (non-hybrid)
@@ -819,13 +814,13 @@ int Decoder::prefill(int n, bool with_logits, int digits, float *elapsed_ms) {
                                                         (size_t)c_.max_pos, N, pf_attn_ws_, pf_attn_ws_bytes_, pf_atth_,
                                                         (kv_f16_ ? BITNET_HIP_ATTN_CACHE_F16 : 0) | BITNET_HIP_ATTN_OUT_F16, s));
             if (f16_rows)
-                BCHK(bitnet_hip_matmul_f16_dev(L.o, pf_atth_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, few16(L.o), nullptr, nullptr, nullptr, s));
+                BCHK(bitnet_hip_matmul_f16_dev(L.o, pf_atth_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, few_rows_flag(L.o, N), nullptr, nullptr, nullptr, s));
             else
                 BCHK(bitnet_hip_matmul_fused_dev(L.o, (const float *)pf_atth_, pf_x_, N, nullptr, 0.f, pf_x_, BITNET_HIP_FUSE_X_F16 | f6od(L.o, BITNET_HIP_FUSE_X_F16), digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
             BCHK(bitnet_hip_matmul_fused_dev(L.gateup, pf_x_, (float *)pf_hh_, N, L.ffn_norm, c_.eps, nullptr, BITNET_HIP_FUSE_SILU_MUL | BITNET_HIP_FUSE_Y_F16 | f6(L.gateup, BITNET_HIP_FUSE_SILU_MUL), digits,
                                              pf_gemm_ws_, pf_gemm_ws_bytes_, s));
             if (f16_rows)
-                BCHK(bitnet_hip_matmul_f16_dev(L.down, pf_hh_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, few16(L.down), nullptr, nullptr, nullptr, s));
+                BCHK(bitnet_hip_matmul_f16_dev(L.down, pf_hh_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, few_rows_flag(L.down, N), nullptr, nullptr, nullptr, s));
             else
                 BCHK(bitnet_hip_matmul_fused_dev(L.down, (const float *)pf_hh_, pf_x_, N, nullptr, 0.f, pf_x_, BITNET_HIP_FUSE_X_F16 | f6od(L.down, BITNET_HIP_FUSE_X_F16), digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
             continue;
@@ -992,7 +987,9 @@ int Decoder::prefill_sharded(int n, int rank, int world, bitnet_host_allgather_f
         if (rc) return rc;
     }
     float *att_out = h16 ? static_cast<float *>(pf_atth_) : pf_att_;
-    const bool hybrid = h16 && hybrid_applies(N);  // o / down on the f16 matrix cores, as in the unsharded prefill (long shares only)
+    // o / down on the f16 matrix cores, as in the unsharded prefill: shares of 128 / 256 / 1024 / 2048 / 2560 rows of bitnet-b1.58-2B-4T 2.67 / 3.28 / 6.52 / 11.2 / 13.6 ms, on
+    // the digits 2.85 / 3.96 / 7.23 / 11.5 / 13.6
+    const bool f16_rows = h16 && f16_rows_apply();
     const int aflags = (kv_f16_ ? BITNET_HIP_ATTN_CACHE_F16 : 0) | (h16 ? BITNET_HIP_ATTN_OUT_F16 : 0);
     for (auto &L : layers_) {
         HCHK(mark(0, s));
@@ -1029,14 +1026,14 @@ int Decoder::prefill_sharded(int n, int rank, int world, bitnet_host_allgather_f
         HCHK(mark(4, s));
         const int xf = h16 ? BITNET_HIP_FUSE_X_F16 : 0, yf = h16 ? BITNET_HIP_FUSE_Y_F16 : 0;
         float *h_buf = h16 ? static_cast<float *>(pf_hh_) : pf_h_;
-        if (hybrid)
-            BCHK(bitnet_hip_matmul_f16_dev(L.o, pf_atth_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, 0, nullptr, nullptr, nullptr, s));
+        if (f16_rows)
+            BCHK(bitnet_hip_matmul_f16_dev(L.o, pf_atth_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, few_rows_flag(L.o, N), nullptr, nullptr, nullptr, s));
         else
             BCHK(bitnet_hip_matmul_fused_dev(L.o, att_out, pf_x_, N, nullptr, 0.f, pf_x_, xf, digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
         BCHK(bitnet_hip_matmul_fused_dev(L.gateup, pf_x_, h_buf, N, L.ffn_norm, c_.eps, nullptr, BITNET_HIP_FUSE_SILU_MUL | yf, digits, pf_gemm_ws_,
                                          pf_gemm_ws_bytes_, s));
-        if (hybrid)
-            BCHK(bitnet_hip_matmul_f16_dev(L.down, pf_hh_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, 0, nullptr, nullptr, nullptr, s));
+        if (f16_rows)
+            BCHK(bitnet_hip_matmul_f16_dev(L.down, pf_hh_, N, nullptr, 0, nullptr, 0.f, pf_x_, pf_x_, few_rows_flag(L.down, N), nullptr, nullptr, nullptr, s));
         else
             BCHK(bitnet_hip_matmul_fused_dev(L.down, h_buf, pf_x_, N, nullptr, 0.f, pf_x_, xf, digits, pf_gemm_ws_, pf_gemm_ws_bytes_, s));
         HCHK(mark(5, s));

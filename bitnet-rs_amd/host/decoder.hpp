@@ -108,7 +108,8 @@ class Decoder : public Sequence {
     bool chain_applies(int digits) const;
     bool handover16_applies(int digits) const;
     bool f16_rows_apply() const;
-    bool hybrid_applies(size_t n_rows) const;
+    bool wide_rows_apply(size_t n_rows) const;
+    int few_rows_flag(bitnet_hip_weights_t h, size_t m) const;
     int last_prefill_path() const { return last_prefill_path_; }
     int saturation_fallbacks() const { return saturation_fallbacks_; }
     int fp6_flag(int digits);  // BITNET_HIP_FUSE_FP6_DIGITS for the q|k|v and gate|up launches of the digit-plane prompt forward, or 0

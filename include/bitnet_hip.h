@@ -33,7 +33,7 @@
  * counts -- are constants tuned for MI355X: 256 CUs in 8 XCDs, 4 MiB of L2 per XCD, 160 KiB of
  * LDS per CU, 512 registers per SIMD lane.  Results do not depend on them (placement and tiling
  * change speed only); on another gfx950 part they would want re-tuning (kGemmCUs, the cover
- * thresholds, gemm_weight_group's 1.5 MiB in kernels_gemm.hip; Decoder::hybrid_applies' 400
+ * thresholds, gemm_weight_group's 1.5 MiB in kernels_gemm.hip; Decoder::wide_rows_apply's 400
  * workgroups in host/decoder.cpp).  Environment switches that steer them: INTEGRATION.md.
  */
 #ifndef BITNET_HIP_H
