@@ -27,7 +27,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ATTN = "_ZN10bitnet_hip14k_prefill_attnILi4ELi4ELi2EEEvNS_11PrefillArgsE"
 GEMM64 = "_ZN10bitnet_hip11k_gemm_mfmaILi2ELi4ELi0ELi2ELi1EEEvNS_8GemmArgsE"
 GEMM32 = "_ZN10bitnet_hip11k_gemm_mfmaILi2ELi2ELi0ELi2ELi1EEEvNS_8GemmArgsE"
-GEMMF16 = "_ZN10bitnet_hip11k_gemm_f16aILi1ELi4ELi1ELi4EEEvNS_8GemmArgsEj"  # the f16 chain instance (BitNet32-F16, 64-token tile, chain epilogues)
+ATTN_ONE = "_ZN10bitnet_hip14k_prefill_attnILi4ELi4ELi1EEEvNS_11PrefillArgsE"  # contexts of one key tile
+GEMMF16 = "_ZN10bitnet_hip11k_gemm_f16aILi1ELi4ELi1ELi4EEEvNS_8GemmArgsEj"  # the f16 chain instance (BitNet32-F16, 64-token tile, chain epilogues), expanding codes
 # the 320-row workgroups of the 2560-row launches (five row tiles per wave), BitNet32-F16 and QK256 (the hybrid prompt forward's o / down)
 GEMMF16_R5 = "_ZN10bitnet_hip11k_gemm_f16aILi1ELi4ELi1ELi5EEEvNS_8GemmArgsEj"
 GEMMF16_R5_QK = "_ZN10bitnet_hip11k_gemm_f16aILi0ELi4ELi1ELi5EEEvNS_8GemmArgsEj"
@@ -35,6 +36,11 @@ GEMMFP6 = "_ZN10bitnet_hip10k_gemm_fp6ILi4ELi4ELi1ELi0EEEvNS_8GemmArgsEj"  # the
 GEMMFP6_X = "_ZN10bitnet_hip10k_gemm_fp6ILi4ELi4ELi0ELi0EEEvNS_8GemmArgsEj"  # ... expanding the 2-bit tiles in its K loop (BITNET_HIP_FUSE_FP6_EXPAND)
 GEMMFP6_QB = "_ZN10bitnet_hip10k_gemm_fp6ILi4ELi4ELi1ELi1EEEvNS_8GemmArgsEj"  # ... on QB32 rows with the chain epilogue (opt-in)
 GEMMF16_QB = "_ZN10bitnet_hip11k_gemm_f16aILi0ELi4ELi2ELi5EEEvNS_8GemmArgsEj"  # the o- / down-projection handing QB32 rows over (opt-in)
+# what prompts run: the f16 products from the resident image (the first parameter + 2) in 64-token tiles and in the 128-row workgroups of short prompts, and the form for few rows
+IMAGE = {f"_ZN10bitnet_hip11k_gemm_f16aILi{fmt}ELi{ttw}ELi{epi}ELi{rt}EEEvNS_8GemmArgsEj": (ceiling, waves)
+         for fmt, ttw, epi, rt, ceiling, waves in ((3, 4, 1, 4, 216, 2), (2, 4, 1, 4, 200, 2), (3, 4, 1, 5, 248, 2), (2, 4, 1, 5, 226, 2), (3, 2, 1, 2, 128, 4), (2, 2, 1, 2, 128, 4),
+                                                   (3, 1, 1, 2, 112, 4), (2, 1, 1, 2, 102, 4), (3, 2, 1, 4, 168, 3), (2, 2, 1, 4, 160, 3), (2, 4, 2, 5, 254, 2))}
+FEW = {f"_ZN10bitnet_hip14k_gemm_f16_fewILb{sc}ELi{rt}EEEvNS_8GemmArgsEj": (140, 3) if rt == 4 else (128, 4) for sc in (0, 1) for rt in (1, 2, 4)}
 
 
 def _compile(src, tmp):
@@ -116,6 +122,10 @@ def test_resources_of_the_benchmarked_instantiations(isa):
         assert u["VGPRs"] + u.get("AGPRs", 0) <= ceiling, (name, u)
     assert ua[ATTN]["Occupancy"] >= 2 and ug[GEMM64]["Occupancy"] >= 2 and ug[GEMM32]["Occupancy"] >= 3 and ug[GEMMF16]["Occupancy"] >= 2
     assert ug[GEMMF16_R5]["Occupancy"] >= 2 and ug[GEMMF16_R5_QK]["Occupancy"] >= 2 and ug[GEMMFP6]["Occupancy"] >= 2
+    for usage, instances in ((ug, IMAGE), (ug, FEW), (ug, {GEMMF16H.replace("ILi1E", "ILi3E"): (254, 2)}), (ua, {ATTN_ONE: (168, 3)})):
+        for name, (ceiling, waves) in instances.items():
+            u = usage[name]
+            assert u["ScratchSize"] == 0 and u["VGPRs"] + u.get("AGPRs", 0) <= ceiling and u["Occupancy"] >= waves, (name, u)
 
 
 # the one instantiation hipcc 7.2 spills: 4 digits x 256-element block scales on the 8-wave tile (128 int32 + 64 f32 accumulators);
@@ -134,12 +144,16 @@ def test_no_scratch_anywhere_else_in_the_prefill_sources(isa):
             assert u["ScratchSize"] == 0 or name in KNOWN_SCRATCH, (src, name, u)
     lines, usage = isa["kernels_gemm.hip"]
     assert usage[GEMMF16H]["ScratchSize"] <= 96 and usage[GEMMF16H]["Occupancy"] >= 2, usage[GEMMF16H]
-    body = body_of(lines, GEMMF16H)
-    for a, b in inner_loops(body):  # the K loop (both half steps unrolled): at most one scratch access per half step, 128 MFMAs each, no stores
-        ins = [t for _, _, t in classify(body[a:b + 1])]
-        if sum(t.startswith("v_mfma") for t in ins) >= 128:
-            assert sum(t.startswith("scratch_") for t in ins) <= 2, [t for t in ins if t.startswith("scratch_")]
-            assert not any(t.startswith(("global_store", "buffer_store")) for t in ins)
+    for name, spills in ((GEMMF16H, 2), (GEMMF16H.replace("ILi1E", "ILi3E"), 0)):  # expanding codes, and from the image
+        body = body_of(lines, name)
+        found = 0
+        for a, b in inner_loops(body):  # the K loop (both half steps unrolled): at most one scratch access per half step, 128 MFMAs each, no stores
+            ins = [t for _, _, t in classify(body[a:b + 1])]
+            if sum(t.startswith("v_mfma") for t in ins) >= 128:
+                found += 1
+                assert sum(t.startswith("scratch_") for t in ins) <= spills, [t for t in ins if t.startswith("scratch_")]
+                assert not any(t.startswith(("global_store", "buffer_store")) for t in ins)
+        assert found == 1, (name, found)
     for name in (ATTN, GEMM64, GEMM32, GEMMF16, GEMMF16_R5, GEMMF16_R5_QK, GEMMFP6):
         src = "kernels_prefill_attn.hip" if name == ATTN else "kernels_gemm.hip"
         assert not any(re.match(r"\s*scratch_", l) for l in body_of(isa[src][0], name)), name
