@@ -558,3 +558,81 @@ def test_prefill_attention_of_one_key_tile_is_the_start_of_a_longer_prompt(hip, 
     assert torch_.equal(o, o2[:T])
     assert torch_.equal(k[:, :T], k2[:, :T]) and torch_.equal(v[:, :T], v2[:, :T])
     assert not k[:, T:].any() and not v[:, T:].any()
+
+
+@pytest.mark.parametrize("T", [1, 17, 64])
+@pytest.mark.parametrize("shift", [0, 1])  # rows that start off their 16 bytes
+def test_prefill_attention_of_one_key_tile_over_its_own_rows(hip, oracle, torch_, T, shift):
+    """Outputs that lie over the k and v rows, over their first or last row only, or right beside them: what separate buffers give, digit for digit.  So do the caches of rows off 16 bytes;
+    their queries pass through memory as f16, which may round a query's element the other way: a score moves by at most 2^-10 of |q| |k| / sqrt(D) (which the rotation
+    keeps), and an output by that much of twice the largest |v|."""
+    D, n_heads, n_kv, max_pos = 128, 8, 2, 128
+    rng = np.random.default_rng(T)
+    nq, nkv = T * n_heads * D, T * 2 * n_kv * D
+    sin, cos = (torch_.from_numpy(np.ascontiguousarray(a, np.float32)).cuda() for a in oracle.rope_tables(D, max_pos, 10000.0))
+    q, kv = (torch_.from_numpy(rng.normal(0, 1.5, n).astype(np.float32)).cuda() for n in (nq, nkv))
+    zero = torch_.zeros(1, dtype=torch_.int32, device="cuda")
+    wsb = hip.attention_prefill_sharded_workspace_bytes(n_heads, n_kv, T, T)
+    ws = torch_.empty(wsb, dtype=torch_.uint8, device="cuda")
+
+    def run(area, q_at, kv_at, out_at):
+        area[q_at:q_at + nq], area[kv_at:kv_at + nkv] = q, kv
+        kc, vc = (torch_.zeros(n_kv * 128 * D, device="cuda") for _ in range(2))
+        hip.attention_prefill_sharded_dev(area[q_at:], n_heads * D, zero, T, area[kv_at:], 2 * n_kv * D, T, sin, cos, kc, vc, n_heads, n_kv, D, max_pos, ws, wsb, area[out_at:])
+        torch_.cuda.synchronize()
+        return area[out_at:out_at + nq].clone(), kc, vc
+
+    size = 4 * (nq + nkv) + 64
+    want = run(torch_.zeros(size, device="cuda"), 0, nq, nq + nkv)
+    first = 2 * nq + nkv  # k and v lie in the middle of the area, the queries at its start
+    for out_at in (first, first + nkv - 128, first - nq + 128, first + nkv, first - nq):
+        got = run(torch_.zeros(size, device="cuda"), shift, first + shift, out_at + 4 * shift)
+        assert torch_.equal(got[1], want[1]) and torch_.equal(got[2], want[2]), out_at - first
+        if shift == 0:
+            assert torch_.equal(got[0], want[0]), out_at - first
+            continue
+        rows = kv.view(T, 2, n_kv, D)
+        scores = q.view(T, n_heads, D).norm(dim=2).max() * rows[:, 0].norm(dim=2).max() * D ** -0.5
+        assert (got[0] - want[0]).abs().max() <= 2.0 ** -10 * scores * 2 * rows[:, 1].abs().max(), out_at - first
+
+
+_HYBRID_SCRIPT = r"""
+import importlib, sys
+import numpy as np, torch
+sys.path.insert(0, {root!r})
+pkg = importlib.import_module("bitnet-rs_amd"); synth = importlib.import_module("bitnet-rs_amd.synth")
+hip = pkg.load(); hip.init(0)
+cfg = synth.ModelConfig(hidden=1024, n_layers=2, n_heads=8, n_kv_heads=2, head_dim=128, ffn=2048, vocab=512, max_pos=700, eps=1e-5, rope_theta=10000.0)
+dec = pkg.HostDecoder(cfg)
+for l in range(cfg.n_layers):
+    dec.set_layer_qk256(l, synth.make_layer(cfg, l, fmt="qk256"))
+dec.set_globals(synth.make_globals(cfg))
+out = []
+for T in (5, 300, 640):
+    for sharded in (False, True):
+        if sharded and T % 128:
+            continue
+        dec.reset(); dec.feed(synth.prompt(T, cfg.vocab))
+        dec.prefill_sharded(T, 0, 1, None, with_logits=True, digits=2) if sharded else dec.prefill(T, with_logits=True, digits=2)
+        out.append(dec.last_logits())
+        print("MODE", hip.matmul_last_tile()["scale_mode"])
+np.save(sys.argv[1], np.stack(out))
+"""
+
+
+def test_prefill_with_digits_behind_the_f16_rows(hip, tmp_path):
+    """BITNET_HOST_PREFILL_HYBRID=0 keeps o and down on int8 digits of their f16 rows, in whole and in sharded prompts: the instance that runs, and logits close to the default's."""
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    logits = []
+    for mode, scale_mode in (("1", "5"), ("0", "0")):
+        path = str(tmp_path / f"{mode}.npy")
+        p = subprocess.run([sys.executable, "-c", _HYBRID_SCRIPT.format(root=root), path], env=dict(os.environ, BITNET_HOST_PREFILL_HYBRID=mode), capture_output=True, text=True, timeout=100)
+        assert p.returncode == 0, p.stdout[-1500:] + p.stderr[-3000:]
+        assert [l.split()[1] for l in p.stdout.splitlines() if l.startswith("MODE ")] == [scale_mode] * 4, p.stdout
+        logits.append(np.load(path))
+    for a, b in zip(*logits):
+        assert cosine(a, b) >= 0.9999
