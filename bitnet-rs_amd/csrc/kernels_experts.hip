@@ -223,7 +223,8 @@ __global__ __launch_bounds__(256) void k_route_slots(ExpertsPlan p) {
 }
 
 // A short prompt's choices and their plan in one launch of one workgroup, LT lanes per token: counts, ranks and offsets stay in LDS.  The three launches above take 8.1 + 3.9 + 2.5 us at
-// 64 tokens and 64 experts, this one 8.4: the choices themselves.  One round of it only: with two tokens per LT lanes, 90 tokens and 72 outputs take 22 us, the three launches 20.
+// 64 tokens and 64 experts, this one 8.4: the choices themselves.  Above 256 experts in groups it spills 88 bytes per lane, and takes 17 us for 16 tokens where the three took 91.
+// One round of it only: with two tokens per LT lanes, 90 tokens and 72 outputs take 22 us, the three launches 20.
 template <int LT, int PL, bool GROUPED>
 __global__ __launch_bounds__(1024) void k_route_few(const float *__restrict__ z, size_t ldz, Router r, ExpertsPlan p) {
     __shared__ int count[kMaxExperts], first[kMaxExperts];

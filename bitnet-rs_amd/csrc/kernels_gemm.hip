@@ -2758,9 +2758,9 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
     if (io.few) return io.qb_out ? hipErrorInvalidValue : launch_gemm_f16_few(w, a, stream);
     const bool rt5 = ttw == 4 && !io.silu_mul && gemm_five_tiles(w.rows, m_pad);
     // Short prompts: waves of 32 rows while the waves of 64 leave most CUs one workgroup.  A K step of such a workgroup is a serial chain (staging, expansion, LDS reads, MFMAs,
-    // barrier: 3.2 us at 32 tokens, of which the units are busy a third), so two of half the rows on a CU take less than one.  BitNet32-F16 prompt of bitnet-b1.58-2B-4T, ms with
-    // this / without: 16 tokens 2.77 / 3.50, 128 3.28 / 3.98, 256 4.06 / 4.23, 400 5.40 / 5.99, 777 6.96 / 7.58, 1024 7.32 / 7.98.  From 390 workgroups on (q|k|v at 777
-    // tokens) both take the same time (37.2 / 37.6 us), and the waves of 64 expand each weight for twice the tokens.
+    // barrier), so two of half the rows on a CU take less than one.  BitNet32-F16 prompt of bitnet-b1.58-2B-4T, weights from the image, ms with the line at 320 / 448 workgroups / without:
+    // 193 tokens 3.30 / 3.30 / 3.79, 256 3.35 / 3.41 / 3.84, 257 3.79 / 3.80 / 4.29, 400 4.44 / 4.41 / 4.92, 512 4.60 / 4.61 / 5.04, 640 5.82 / 5.77 / 5.96, 777 6.16 / 6.13 / 6.51,
+    // 1024 6.57 / 6.57 / 6.91 (at 256: 3.91 at 257 tokens, 4.91 at 400); at 384 as at 320.
     const bool rt2 = ttw < 4 && gx0 * (m_pad / (16 * ttw)) <= 320;
     if (rt5) gx0 = w.rows / 320;
     if (rt2) gx0 = w.rows / 128;
@@ -2815,6 +2815,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
                 }
             }
             GemmArgs aa = a;
+            // (with the image 3 row blocks at gate|up, block scales counted twice like the codes; groups of 4, of 6 and none take the same, prompts of 1024 to 4096 tokens within 0.5 %)
             aa.wgroup = gemm_weight_group(n_a, 256, image ? 2 * w.cols : w.cols, fmt1);
             hipLaunchKernelGGL(hk, dim3((unsigned)n_a, (unsigned)t128), dim3(256), (size_t)2 * 128 * 256 + 128 * 8 + 4096, stream, aa, lut_f16_hi(w.lut));
             g_last_gemm_tile = GemmTileChoice{2, 128, 4, fmt1 ? 4 : 5, 64};
