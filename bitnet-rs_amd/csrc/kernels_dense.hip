@@ -281,6 +281,62 @@ __global__ __launch_bounds__(256) void k_sum_norm_rows(SumRows p) {
     for (int i = (x2 ? 2 : 1) * width + tid; i < (int)p.ldh; i += 256) st_act(h, i, 0.f);
 }
 
+// x += scale * norm(y), h = norm(x) or x, of rows that four columns at a time do not fit: an odd width, operands off their alignment, more than 4096 columns.  The kernel above goes over
+// experts, gates and biases in every column there, with a load at a time in flight: 8 rows of 3073 columns 10.1 us, here 6.6; 4096 of 5121 89 and 85.  (Without y it is the faster one up to
+// 2048 columns: 8 rows of 1022 2.6 and 2.9 us.)  REGS: up to 4096 columns in registers.
+template <class T, bool REGS>
+__global__ __launch_bounds__(256) void k_residual_norm_rows(SumRows p) {
+    constexpr int NJ = REGS ? 16 : 1;
+    __shared__ float slot[4];
+    const int tid = threadIdx.x, width = (int)p.width;
+    float *x = p.x + (size_t)blockIdx.x * width;
+    const float *y = p.y ? p.y + (size_t)blockIdx.x * p.ldy : nullptr, *__restrict__ post = p.post_weight, *__restrict__ scale = p.scale, *__restrict__ weight = p.weight;
+    T *h = p.h ? (T *)p.h + (size_t)blockIdx.x * p.ldh : nullptr;
+    float xv[NJ], yv[NJ];
+    auto columns = [&](auto f) {
+        if constexpr (REGS) {
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) f(tid + 256 * j, j, tid + 256 * j < width);
+        } else {
+            for (int i = tid; i < width; i += 256) f(i, 0, true);
+        }
+    };
+    auto x_at = [&](int i, int j) { return REGS ? xv[j] : x[i]; };
+    if (y) {
+        float ss = 0.f;
+        columns([&](int i, int j, bool in) {
+            yv[j] = in ? y[i] : 0.f;
+            if (REGS) xv[j] = in ? x[i] : 0.f;
+            ss += yv[j] * yv[j];
+        });
+        const float inv = 1.0f / sqrtf(group_sum<4>(ss, slot) / (float)width + p.eps);
+        columns([&](int i, int j, bool in) {
+            if (!in) return;
+            const float v = x_at(i, j) + (scale ? scale[i] : 1.0f) * ((REGS ? yv[j] : y[i]) * inv * (p.weight_offset + post[i]));
+            x[i] = v, xv[j] = v;
+        });
+    } else if (REGS) {
+        columns([&](int i, int j, bool in) { xv[j] = in ? x[i] : 0.f; });
+    }
+    if (!h) return;
+    if (weight) {
+        float ss = 0.f;
+        columns([&](int i, int j, bool) {
+            const float v = x_at(i, j);
+            ss += v * v;
+        });
+        const float inv = 1.0f / sqrtf(group_sum<4>(ss, slot) / (float)width + p.eps);
+        columns([&](int i, int j, bool in) {
+            if (in) st_act(h, i, x_at(i, j) * inv * (p.weight_offset + weight[i]));
+        });
+    } else {
+        columns([&](int i, int j, bool in) {
+            if (in) st_act(h, i, x_at(i, j));
+        });
+    }
+    for (int i = width + tid; i < (int)p.ldh; i += 256) st_act(h, i, 0.f);
+}
+
 template <class T, int NJ>
 static hipError_t sum_norm_go(const SumRows &a, hipStream_t s) {
     const bool g = a.gate || a.y_scale;
@@ -296,8 +352,14 @@ static hipError_t sum_norm_type(const SumRows &a, hipStream_t s) {
                     own = (uintptr_t)a.h | (uintptr_t)a.expert_rows | (uintptr_t)a.input | (uintptr_t)a.gate;
     const bool vec = wide % 16 == 0 && own % (4 * sizeof(T)) == 0 && a.width % 4 == 0 && a.width <= 1024 * kSumRegs && a.ldy % 4 == 0 && a.ld_expert % 4 == 0 && a.ldh % 4 == 0 &&
                      a.ld_input % 4 == 0 && a.ld_gate % 4 == 0;
+    if (!vec) {
+        const bool plain = (a.y ? a.post_weight != nullptr : a.width > 2048) && a.top == 0 && !a.x2 && !a.center && !a.bias && !a.gate && !a.y_scale && !a.identity;
+        if (!plain) return sum_norm_go<T, 0>(a, s);
+        auto fn = a.width <= 4096 ? k_residual_norm_rows<T, true> : k_residual_norm_rows<T, false>;
+        hipLaunchKernelGGL(fn, dim3(a.m), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
     // (a group more than the row needs costs its registers and its share of the instructions)
-    if (!vec) return sum_norm_go<T, 0>(a, s);
     return a.width <= 2048 ? sum_norm_go<T, 2>(a, s) : a.width <= 3072 ? sum_norm_go<T, 3>(a, s) : sum_norm_go<T, kSumRegs>(a, s);
 }
 
