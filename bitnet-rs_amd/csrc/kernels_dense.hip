@@ -381,7 +381,7 @@ __global__ __launch_bounds__(256) void k_gated_norm_rows(const float *__restrict
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const int at = 4 * min(tid + 256 * j, (n >> 2) - 1);
-            v[j] = ld4(orow, at), wv[j] = ld4(w, at), gv[j] = ld4(grow, at);
+            if (NJ > 1 || 4 * tid < n) v[j] = ld4(orow, at), wv[j] = ld4(w, at), gv[j] = ld4(grow, at);  // (narrow rows: most waves have none; 4096 rows of 64 3.0 us, 4.7 with two groups)
         }
 #pragma unroll
         for (int j = 0; j < NJ; ++j) ss += 4 * (tid + 256 * j) < n ? (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w) : 0.f;
@@ -404,7 +404,7 @@ hipError_t launch_gated_norm_rows(const float *o, size_t ldo, const float *w, co
         using TH = std::remove_pointer_t<decltype(out)>;
         const bool vec = ((uintptr_t)o | (uintptr_t)w) % 16 == 0 && (uintptr_t)g % (4 * sizeof(TG)) == 0 && (uintptr_t)out % (4 * sizeof(TH)) == 0 && n % 4 == 0 && n <= 1024 * kSumRegs &&
                          ldo % 4 == 0 && ldg % 4 == 0 && ldh % 4 == 0;
-        auto fn = !vec ? k_gated_norm_rows<TG, TH, 0> : n <= 2048 ? k_gated_norm_rows<TG, TH, 2> : n <= 3072 ? k_gated_norm_rows<TG, TH, 3> : k_gated_norm_rows<TG, TH, kSumRegs>;
+        auto fn = !vec ? k_gated_norm_rows<TG, TH, 0> : n <= 512 ? k_gated_norm_rows<TG, TH, 1> : n <= 2048 ? k_gated_norm_rows<TG, TH, 2> : n <= 3072 ? k_gated_norm_rows<TG, TH, 3> : k_gated_norm_rows<TG, TH, kSumRegs>;
         hipLaunchKernelGGL(fn, dim3(m), dim3(256), 0, s, o, ldo, w, g, ldg, eps, n, mean_n, out, ldh);
     };
     if (gate_f32 && h_f32)

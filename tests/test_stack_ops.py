@@ -500,6 +500,11 @@ def test_row_norms_at_register_edges(hip, width, shift):
         assert u.rms_error(u.host(h)[:, :width], want) < tol and not u.host(h)[:, width:].any()
 
 
+@pytest.mark.parametrize("width", [64, 252, 256, 260, 508, 512, 516])
+def test_row_norms_of_narrow_rows(hip, width):
+    test_row_norms_at_register_edges(hip, width, 0)
+
+
 @pytest.mark.parametrize("width,shift", [(255, 0), (3, 0), (1024, 1), (4095, 0), (4096, 1), (4097, 0), (4100, 1), (8192, 0)])
 def test_row_norms_of_single_columns(hip, width, shift):
     test_row_norms_at_register_edges(hip, width, shift)
