@@ -129,6 +129,12 @@ def test_sum_norm_rows_behind_experts(hip, pkg, width, f32):
     assert u.rms_error(xs, x + 0.6 * summed(x, np.zeros((m, width)))) < F32_TOL
 
 
+@pytest.mark.parametrize("width", [4, 1024, 1028, 2048, 2052, 3072, 3076, 4096])
+@pytest.mark.parametrize("f32", [True, False])
+def test_sum_norm_rows_behind_experts_at_register_edges(hip, pkg, width, f32):
+    test_sum_norm_rows_behind_experts(hip, pkg, width, f32)
+
+
 @pytest.mark.parametrize("width", [40, 77, 2560, 4500])
 def test_norm_behind_the_embedding(hip, width):
     g = rng(width, 4)
