@@ -309,8 +309,9 @@ hipError_t launch_latent_decode(const LatentAttn &a, hipStream_t s) {
 // ---- the records of a head -> its value vector --------------------------------------------------------------------------
 // Every workgroup merges the head's records (running maxima, sums, the sink) in LDS and takes a share of W_uv's rows.  The position is wanted last: the records' first numbers and
 // vectors are requested whether they are used or not (scratch has room for all of them), and so are the wave's first rows of W_uv.  Inside
-// a step, 20 heads at 61 to 85 keys: 5.2 -> 4.6 us.
-template <class TO>
+// a step, 20 heads at 61 to 85 keys: 5.2 -> 4.6 us.  Not AHEAD past 256 heads times queries: the chip is full, what is not used costs bytes, and registers cost waves: 64 queries of 20
+// heads at 85 keys 15.4 us (ahead: 19.3), of 128 heads 79 (121), 16 queries of 20 heads 8.4 (9.2), of 16 heads 4.9 (4.8); 64 of 20 heads at 1500 keys 23.6 (25.0), at 8000 82 (72).
+template <class TO, bool AHEAD>
 __global__ __launch_bounds__(512) void k_latent_merge(LatentMerge p) {
     extern __shared__ __attribute__((aligned(16))) float o[];  // [ldc], then four partial vectors
     static_assert(kLatentSplits == 128, "two records per lane of a wave");
@@ -323,19 +324,25 @@ __global__ __launch_bounds__(512) void k_latent_merge(LatentMerge p) {
     const int share = (p.vdimp + gridDim.y - 1) / gridDim.y, v0 = blockIdx.y * share, v1 = min(v0 + share, p.vdimp);
     constexpr int AW = 4, AR = 2;  // rows of W_uv, records per group
     u32x4 uw[AW];
-#pragma unroll
-    for (int j = 0; j < AW; ++j) uw[j] = *reinterpret_cast<const u32x4 *>(p.uv + ((size_t)h * p.vdimp + min(v0 + wave + 8 * j, p.vdimp - 1)) * p.ldc + min(lane * 8, p.ldc - 8));
     const int grp = tid >> 7, t = tid & 127;
     f32x4 ahead[AR];
-#pragma unroll
-    for (int j = 0; j < AR; ++j) ahead[j] = *reinterpret_cast<const f32x4 *>(rec + (grp + 4 * j) * stride + kLatentRecHead + min(t * 4, p.ldc - 4));
     float mv[2] = {-INFINITY, -INFINITY}, lv[2] = {0.f, 0.f};
-    if (wave == 0)
+    if constexpr (AHEAD) {
 #pragma unroll
-        for (int e = 0; e < 2; ++e) mv[e] = rec[(lane + 64 * e) * stride], lv[e] = rec[(lane + 64 * e) * stride + 1];
+        for (int j = 0; j < AW; ++j) uw[j] = *reinterpret_cast<const u32x4 *>(p.uv + ((size_t)h * p.vdimp + min(v0 + wave + 8 * j, p.vdimp - 1)) * p.ldc + min(lane * 8, p.ldc - 8));
+#pragma unroll
+        for (int j = 0; j < AR; ++j) ahead[j] = *reinterpret_cast<const f32x4 *>(rec + (grp + 4 * j) * stride + kLatentRecHead + min(t * 4, p.ldc - 4));
+        if (wave == 0)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) mv[e] = rec[(lane + 64 * e) * stride], lv[e] = rec[(lane + 64 * e) * stride + 1];
+    }
     const float sink = p.sink ? p.sink[h] : -INFINITY;
     int per, used;
     split_range(posv + p.q0 + qi + 1, per, used);
+    if (!AHEAD && wave == 0)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+            if (lane + 64 * e < used) mv[e] = rec[(lane + 64 * e) * stride], lv[e] = rec[(lane + 64 * e) * stride + 1];
     if (wave == 0) {
         float M = sink;
 #pragma unroll
@@ -360,7 +367,7 @@ __global__ __launch_bounds__(512) void k_latent_merge(LatentMerge p) {
     for (int i = t * 4; i < p.ldc; i += 512) {
         f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
         int r = grp;
-        if (i == t * 4) {
+        if (AHEAD && i == t * 4) {
 #pragma unroll
             for (int j = 0; j < AR; ++j)
                 if (grp + 4 * j < used) a += ws[grp + 4 * j] * ahead[j];
@@ -382,21 +389,22 @@ __global__ __launch_bounds__(512) void k_latent_merge(LatentMerge p) {
         acc = fmaf(x1.x, bf2f(wv.z & 0xffffu), fmaf(x1.y, bf2f(wv.z >> 16), acc));
         return fmaf(x1.z, bf2f(wv.w & 0xffffu), fmaf(x1.w, bf2f(wv.w >> 16), acc));
     };
-    auto rest = [&](int v, float acc) {  // the columns behind the first 512
+    auto rest = [&](int v, int i, float acc) {  // the columns from i on
         const uint16_t *w = p.uv + ((size_t)h * p.vdimp + v) * p.ldc;
-        for (int i = lane * 8 + 512; i < p.ldc; i += 512) acc = product(*reinterpret_cast<const u32x4 *>(w + i), i, acc);
+        for (; i < p.ldc; i += 512) acc = product(*reinterpret_cast<const u32x4 *>(w + i), i, acc);
         return acc;
     };
+    if constexpr (AHEAD) {
 #pragma unroll
-    for (int j = 0; j < AW; ++j) {
-        const int v = v0 + wave + 8 * j;
-        if (v >= v1) break;
-        const float acc = wave_sum(rest(v, lane * 8 < p.ldc ? product(uw[j], lane * 8, 0.f) : 0.f));
-        if (lane == 0) st_act(out, v, acc);
+        for (int j = 0; j < AW; ++j) {
+            const int v = v0 + wave + 8 * j;
+            if (v >= v1) break;
+            const float acc = wave_sum(rest(v, lane * 8 + 512, lane * 8 < p.ldc ? product(uw[j], lane * 8, 0.f) : 0.f));
+            if (lane == 0) st_act(out, v, acc);
+        }
     }
-    for (int v = v0 + wave + 8 * AW; v < v1; v += 8) {
-        const u32x4 wv = *reinterpret_cast<const u32x4 *>(p.uv + ((size_t)h * p.vdimp + v) * p.ldc + min(lane * 8, p.ldc - 8));
-        const float acc = wave_sum(rest(v, lane * 8 < p.ldc ? product(wv, lane * 8, 0.f) : 0.f));
+    for (int v = v0 + wave + (AHEAD ? 8 * AW : 0); v < v1; v += 8) {
+        const float acc = wave_sum(rest(v, lane * 8, 0.f));
         if (lane == 0) st_act(out, v, acc);
     }
 }
@@ -405,10 +413,8 @@ hipError_t launch_latent_merge(const LatentMerge &a, hipStream_t s) {
     const int shares = a.nq > 1 ? 1 : (a.vdimp >= 64 ? 4 : 1);
     const size_t lds = (size_t)5 * a.ldc * sizeof(float);
     if (lds > 65536) return hipErrorInvalidValue;
-    if (a.out_bf16)
-        hipLaunchKernelGGL(k_latent_merge<uint16_t>, dim3(a.heads, shares, a.nq), dim3(512), lds, s, a);
-    else
-        hipLaunchKernelGGL(k_latent_merge<float>, dim3(a.heads, shares, a.nq), dim3(512), lds, s, a);
+    auto fn = a.heads * a.nq <= 256 ? (a.out_bf16 ? k_latent_merge<uint16_t, true> : k_latent_merge<float, true>) : a.out_bf16 ? k_latent_merge<uint16_t, false> : k_latent_merge<float, false>;
+    hipLaunchKernelGGL(fn, dim3(a.heads, shares, a.nq), dim3(512), lds, s, a);
     return hipGetLastError();
 }
 

@@ -318,6 +318,13 @@ def test_latent_decode_long_and_several_queries(hip, pkg, f32):
     t.check(t.decode(hip), 1e-5 if f32 else 1e-4)
 
 
+@pytest.mark.parametrize("f32", [True, False])
+@pytest.mark.parametrize("shape,nq", [(SHAPES[2], 15), (SHAPES[2], 16), (SHAPES[3], 64), ((129, 32, 32, 32, 64), 2), ((65, 32, 32, 256, 1024), 4)])
+def test_latent_decode_of_more_queries_than_one_round(hip, pkg, shape, nq, f32):
+    t = Latent(pkg, 150, nq, *shape, f32)
+    t.check(t.decode(hip), 1e-5 if f32 else 1e-4)
+
+
 def test_latent_decode_large_latent_in_bf16(hip, pkg):
     t = Latent(pkg, 150, 2, 3, 64, 64, 32, 900, False)  # beyond the matrix-core form's latent
     t.check(t.decode(hip), 1e-4)
