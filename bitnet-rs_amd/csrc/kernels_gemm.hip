@@ -2688,15 +2688,16 @@ bool gemm_f16_chain_supported(const Weights &w) {
 // 128 -3.3 / -6.8 / -2.3, 192 +7.3 / -1.6 / -1.5, 256 +15 / +2.7 / +8.6; gate|up at 16 - / -5.2 / -6.4, 32 - / +1.3 / 0, 64 - / +10 / +11.  Whole prompts with o in this form and in the
 // wide tiles: 144 tokens 2.96 and 3.19 ms (QK256 2.74 and 2.87).
 // Past one round it is the token rows that a launch reads over and over: they have to stay in an XCD's L2 of 4 MiB, and a short K leaves the wide tiles little to wait for.  A launch's us
-// in this form / the wide one, back to back, at rows x columns and tokens, one round: 256 x 512, 720 3.4 / 3.8, 256 x 8192, 960 15.1 / 19.4; past it: 1536 x 6912, 240 (3.2 MiB) 16.5 / 21.3,
-// 2048 x 8192, 240 (3.8) 24.5 / 25.0, 1536 x 6912, 288 (864 workgroups) 21.0 / 19.0, 512 x 4096, 528 (4.1) 12.1 / 11.4, 1024 x 8192, 480 (7.5) 36 / 20, 256 x 8192, 1920 (30) 40 / 20; 2560 x 512, 144 4.8 / 4.7, 1024 x 512, 352
-// 4.8 / 4.5, 512 x 1024, 720 5.4 / 5.5; pairs 1024 x 512, 352 4.8 / 4.1, 2048 x 1024, 176 5.5 / 5.6, 4096 x 2048, 80 7.8 / 7.4.
+// in this form / the wide one, back to back, at rows x columns and tokens, one round: 256 x 512, 720 3.4 / 3.8, 256 x 8192, 960 15.1 / 19.4; past it: 1536 x 6912, 240 (3.2 MiB) 16.5 /
+// 21.3, 2048 x 8192, 240 (3.8) 24.5 / 25.0, 1536 x 6912, 288 (864 workgroups) 21.0 / 19.0, with block scales 24.0 / 25.2, 1536 x 8192 with block scales, 256 22.6 / 30.1, 512 x 4096, 528
+// (4.1) 12.1 / 11.4, 1024 x 8192, 480 (7.5) 36 / 20, 256 x 8192, 1920 (30) 40 / 20; 2560 x 512, 144 4.8 / 4.7, 1024 x 512, 352 4.8 / 4.5, 512 x 1024, 720 5.4 / 5.5; pairs 1024 x 512, 352
+// 4.8 / 4.1, 2048 x 1024, 176 5.5 / 5.6, 4096 x 2048, 80 7.8 / 7.4.
 static int f16_few_tiles(const Weights &w, bool silu_mul, size_t m) {
     const size_t tiles = w.rows / 16 * div_ceil(m, 16);
     for (int rt = silu_mul ? 2 : 1; rt <= 4; rt *= 2)
         if (tiles / rt <= 256) return rt;
     if (silu_mul || w.cols < 1024 || m * w.cols * 2 > (size_t)4 << 20) return 0;
-    return tiles / 2 <= (w.cols > 4096 && w.rows >= 2048 ? 960 : 720) ? 2 : 0;
+    return tiles / 2 <= (w.cols > 4096 && (w.rows >= 2048 || w.scaled) ? 960 : 720) ? 2 : 0;
 }
 bool gemm_f16_takes_few(const Weights &w, bool silu_mul, size_t m) {
     return gemm_f16_chain_supported(w) && m > 0 && m <= 4096 && (!silu_mul || w.paired) && f16_few_tiles(w, silu_mul, m) > 0;
