@@ -87,6 +87,22 @@ struct QuantArgs {
     float *inv_scale;
 };
 
+// Workgroups are dealt round-robin to the 8 XCDs (each with its own L2).  Renumber them so that one XCD works through CONSECUTIVE logical ids: the workgroups
+// that share an activation tile (same by, all bx) then find it in ONE L2 instead of pulling it into eight.  wgroup > 0: a weight-stationary walk, groups of
+// `wgroup` row blocks (a divisor of their number), inside a group the token tiles, inside a tile the group's blocks.  Placement only changes speed, never results.
+__device__ __forceinline__ void xcd_walk(int wgroup, int &bx, int &by) {
+    const int gx = gridDim.x, total = gx * gridDim.y, id = by * gx + bx, xcd = id & 7;
+    const int l = xcd * (total >> 3) + min(xcd, total & 7) + (id >> 3);  // (the first total & 7 of them take one more)
+    if (wgroup > 0) {
+        const int per = (int)gridDim.y * wgroup, grp = l / per, r = l - grp * per;
+        by = r / wgroup;
+        bx = grp * wgroup + (r - by * wgroup);
+    } else {
+        by = l / gx;
+        bx = l - by * gx;
+    }
+}
+
 template <int CTRL>
 __device__ __forceinline__ float qdpp_f(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
@@ -609,23 +625,8 @@ __global__ __launch_bounds__(256 * CW, MINW) void k_gemm_mfma(GemmArgs p) {
     const int c = lane & 15, g = lane >> 4, rw = wave & 3, cw = wave >> 2;
     const int n_tiles = (p.rows + 15) >> 4;
     const int kp = p.nblk * 256;
-    // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2).  Renumber them so that one XCD
-    // works through CONSECUTIVE logical ids: the workgroups that share an activation tile (same by, all bx)
-    // then find it in ONE L2 instead of pulling it into eight.  Placement only changes speed, never results.
     int bx = blockIdx.x, by = blockIdx.y;
-    {
-        const int gx = gridDim.x, total = gx * gridDim.y, id = by * gx + bx;
-        if ((total & 7) == 0) {
-            const int l = (id & 7) * (total >> 3) + (id >> 3);
-            bx = l % gx;
-            by = l / gx;
-            if (p.wgroup > 0) {  // weight-stationary walk: groups of `wgroup` row blocks, inside a group the token tiles, inside a tile the group's blocks
-                const int per = (int)gridDim.y * p.wgroup, grp = l / per, r = l - grp * per;
-                by = r / p.wgroup;
-                bx = grp * p.wgroup + (r - by * p.wgroup);
-            }
-        }
-    }
+    xcd_walk(p.wgroup, bx, by);
 
     // this wave's four weight row tiles (clamped: surplus tiles recompute the last one, never stored)
     const uint8_t *wptr[4];
@@ -1309,19 +1310,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_h
     const int n_tiles = (p.rows + 15) >> 4;
     const int kp = p.nblk * 256;
     int bx = blockIdx.x, by = blockIdx.y;
-    {  // one XCD works through consecutive logical ids (k_gemm_mfma explains)
-        const int gx = gridDim.x, total = gx * gridDim.y, id = by * gx + bx;
-        if ((total & 7) == 0) {
-            const int l = (id & 7) * (total >> 3) + (id >> 3);
-            bx = l % gx;
-            by = l / gx;
-            if (p.wgroup > 0) {  // weight-stationary walk: groups of `wgroup` row blocks, inside a group the token tiles, inside a tile the group's blocks
-                const int per = (int)gridDim.y * p.wgroup, grp = l / per, r = l - grp * per;
-                by = r / p.wgroup;
-                bx = grp * p.wgroup + (r - by * p.wgroup);
-            }
-        }
-    }
+    xcd_walk(p.wgroup, bx, by);
     bx += p.bx_off;
     const uint8_t *wptr[RT];
     const uint32_t *sptr[RT];
@@ -1482,6 +1471,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_h
         return;
     }
     f16_chain_epilogue<RT, TTW, 4, EPI == 2>(p, acc, lds, mu_rs, bx, by, rw, c, g, tid);
+    if (TTW < 4 && p.stats_out && !p.silu_mul && by == (int)gridDim.y - 1) {  // no workgroup has the token tiles behind the last token's: their partials are zero
+        const int slabs = RT == 2 ? 2 : 4;
+        for (int i = tid; i < slabs * 64; i += 256) {
+            const int token = (by + 1) * WG_TOK + (i & 63);
+            if (token < p.stats_stride) *reinterpret_cast<float2 *>(p.stats_out + 2 * ((size_t)(bx * slabs + (i >> 6)) * p.stats_stride + token)) = float2{0.f, 0.f};
+        }
+    }
 }
 
 // ---- few activation rows on the chain -----------------------------------------------------------------------------------------------------------------------
@@ -1684,19 +1680,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16h(GemmArgs p, uint32_t lut_h
     const int n_tiles = (p.rows + 15) >> 4;
     const int kp = p.nblk * 256;
     int bx = blockIdx.x, by = blockIdx.y;
-    {  // one XCD works through consecutive logical ids (k_gemm_mfma explains)
-        const int gx = gridDim.x, total = gx * gridDim.y, id = by * gx + bx;
-        if ((total & 7) == 0) {
-            const int l = (id & 7) * (total >> 3) + (id >> 3);
-            bx = l % gx;
-            by = l / gx;
-            if (p.wgroup > 0) {
-                const int per = (int)gridDim.y * p.wgroup, grp = l / per, r = l - grp * per;
-                by = r / p.wgroup;
-                bx = grp * p.wgroup + (r - by * p.wgroup);
-            }
-        }
-    }
+    xcd_walk(p.wgroup, bx, by);
     bx += p.bx_off;
     // wave-uniform bases (SGPR pairs) + 32-bit lane offsets: 128 accumulators leave no room for 64-bit per-lane pointers -- nor for a register-staged
     // activation tile (32 registers: hipcc spilled 144-228 bytes), so the tile goes global -> LDS by LDS-DMA, one half-K step ahead of its MFMAs
@@ -1883,19 +1867,7 @@ __global__ __launch_bounds__(256, (TTW >= 4 || EPI) ? 2 : TTW == 2 ? 3 : 4) void
     const int c = lane & 15, g = lane >> 4, rw = wave;
     const int n_tiles = (p.rows + 15) >> 4;
     int bx = blockIdx.x, by = blockIdx.y;
-    {  // one XCD works through consecutive logical ids (k_gemm_mfma explains)
-        const int gx = gridDim.x, total = gx * gridDim.y, id = by * gx + bx;
-        if ((total & 7) == 0) {
-            const int l = (id & 7) * (total >> 3) + (id >> 3);
-            bx = l % gx;
-            by = l / gx;
-            if (p.wgroup > 0) {  // weight-stationary walk: groups of `wgroup` row blocks, inside a group the token tiles, inside a tile the group's blocks
-                const int per = (int)gridDim.y * p.wgroup, grp = l / per, r = l - grp * per;
-                by = r / p.wgroup;
-                bx = grp * p.wgroup + (r - by * p.wgroup);
-            }
-        }
-    }
+    xcd_walk(p.wgroup, bx, by);
     constexpr int NM = RES ? 2 : 1;            // 16-byte weight loads per row tile and K step
     constexpr size_t WSTEP = RES ? 2048 : 1024;  // bytes of one (tile, 256-block) in the layout read
     // Addresses are a wave-uniform base (SGPR pair) + a 32-bit lane offset (round 5: 64-bit per-lane pointers for 4-5 weight tiles, 9 staging
@@ -2090,19 +2062,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_fp6w(GemmArgs p) {
     const int c = lane & 15, g = lane >> 4, wr = wave >> 1, wt = wave & 1;
     const int n_tiles = (p.rows + 15) >> 4;
     int bx = blockIdx.x, by = blockIdx.y;
-    {  // one XCD works through consecutive logical ids (k_gemm_mfma explains)
-        const int gx = gridDim.x, total = gx * gridDim.y, id = by * gx + bx;
-        if ((total & 7) == 0) {
-            const int l = (id & 7) * (total >> 3) + (id >> 3);
-            bx = l % gx;
-            by = l / gx;
-            if (p.wgroup > 0) {
-                const int per = (int)gridDim.y * p.wgroup, grp = l / per, r = l - grp * per;
-                by = r / p.wgroup;
-                bx = grp * p.wgroup + (r - by * p.wgroup);
-            }
-        }
-    }
+    xcd_walk(p.wgroup, bx, by);
     const __amdgpu_buffer_rsrc_t rs_w = gbuf_rsrc(p.tiles4);
     int wptr[RT];  // scalar byte offsets of this wave's row tiles in the fp4 image
 #pragma unroll
@@ -2269,6 +2229,26 @@ static bool gemm_five_tiles(size_t rows, size_t m_pad) {
     const size_t slots = 2 * kGemmCUs, tb = m_pad / 64;
     return div_ceil(rows / 320 * tb, slots) * 5 < div_ceil(div_ceil(rows, 256) * tb, slots) * 4;
 }
+// What a launch takes with a tile of 64 rt rows by 16 ttw tokens: `once` and, for each workgroup that its fullest CU gets, `end` (prologue and epilogue; `residual` on top where there is one);
+// a K block of 256 columns takes `chain` however few workgroups a CU has (a workgroup's steps follow one another) and `share` for each of them where they fill it; the tiles of 64 tokens
+// fit a CU twice, which is `pair`, and run in rounds of that.
+struct TileCost {
+    int rt, ttw;
+    double once, end, residual, chain, share, pair;
+};
+template <size_t N>
+static const TileCost *cheapest_tile(const TileCost (&costs)[N], size_t rows, size_t blocks, size_t m, bool residual, bool five) {
+    const TileCost *best = nullptr;
+    double least = 0.0;
+    for (const TileCost &c : costs) {
+        if (c.rt == 5 && !five) continue;
+        const size_t most = div_ceil(div_ceil(rows, 64 * (size_t)c.rt) * div_ceil(m, 16 * (size_t)c.ttw), kGemmCUs);
+        const double block = c.pair > 0 ? (double)(most / 2) * c.pair + (most % 2 ? (most > 1 ? c.share : c.chain) : 0.0) : std::max(c.chain, c.share * (double)most);
+        const double us = c.once + (c.end + (residual ? c.residual : 0.0)) * (double)most + (double)blocks * block;
+        if (!best || us < least) best = &c, least = us;
+    }
+    return best;
+}
 // Weight-stationary walk of a launch (EXPERIMENTS 4.6).  In the plain order an XCD takes a band of token tiles and walks ALL row blocks for each: the
 // activation tile stays in its L2, the whole weight matrix streams through once per token tile (gate|up: 8.85 MB x 64 tiles = 566 MB of L2 misses
 // per launch, served by the Infinity Cache).  Grouped, an XCD takes `wgroup` row blocks -- the largest divisor of the row-block count whose codes
@@ -2428,11 +2408,7 @@ static hipError_t launch_gemm_few(const Weights &w, QuantArgs q, const GemmArgs 
 }
 
 template <int NDIG, int TTW>
-static hipError_t launch_gemm_t(const Weights &w, const QuantArgs &q, const GemmArgs &a, hipStream_t stream) {
-    const int nv = (int)div_ceil((size_t)q.kp / 4, 256);
-    void (*qk)(QuantArgs) = nv <= 3 ? k_quant_rows<NDIG, 3> : k_quant_rows<NDIG, 8>;
-    if (NDIG == 2 && quant_rows_w_applies(q)) launch_quant_rows_w(q, false, stream);
-    else hipLaunchKernelGGL(qk, dim3(q.m_pad), dim3(256), 0, stream, q);
+static hipError_t launch_gemm_t(const Weights &w, QuantArgs q, const GemmArgs &a, hipStream_t stream) {
     constexpr int TTWS = 2;  // scaled variant: narrower token tile (f32 accumulators take the registers)
     const bool k32 = a.stiles_h != nullptr;
     const bool bs32 = (a.wscale && w.block_size == 32) || k32;  // 32-block scales: one token tile per wave (registers)
@@ -2471,7 +2447,13 @@ static hipError_t launch_gemm_t(const Weights &w, const QuantArgs &q, const Gemm
         }
     }
     g_last_gemm_tile = GemmTileChoice{NDIG, 16 * ttw, 4 * cw, k32 ? 3 : !a.wscale ? 0 : bs32 ? 2 : 1};
-    const unsigned gx = (unsigned)div_ceil(div_ceil(w.rows, 16), 16), gy = (unsigned)(q.m_pad / (16 * cw * ttw));
+    const unsigned gx = (unsigned)div_ceil(div_ceil(w.rows, 16), 16), gy = (unsigned)div_ceil((size_t)q.m, (size_t)16 * cw * ttw);
+    const int nv = (int)div_ceil((size_t)q.kp / 4, 256);
+    void (*qk)(QuantArgs) = nv <= 3 ? k_quant_rows<NDIG, 3> : k_quant_rows<NDIG, 8>;
+    const bool by_waves = NDIG == 2 && quant_rows_w_applies(q);
+    q.m_pad = (int)gy * 16 * cw * ttw;  // (rows that no tile reads are not quantised)
+    if (by_waves) launch_quant_rows_w(q, false, stream);
+    else hipLaunchKernelGGL(qk, dim3(q.m_pad), dim3(256), 0, stream, q);
     GemmArgs aw = a;
     if (!scaled_variant) aw.wgroup = gemm_weight_group(gx, 256, w.cols, false);
     hipLaunchKernelGGL(gk, dim3(gx, gy), dim3(256 * cw), lds, stream, aw);
@@ -2508,13 +2490,15 @@ static auto f16_instance(bool scaled, bool image, F pick) {
 
 // f16 activations on the f16 matrix cores (k_gemm_f16a): BitNet32-F16 at 2 digits; QK256 only on request (BITNET_HIP_GEMM_F16A=1:
 // measured 5-13 % slower than the int8 digit form there -- twice the expansion VALU for the same MFMA count)
-static hipError_t launch_gemm_f16(const Weights &w, const QuantArgs &q, const GemmArgs &a, hipStream_t stream) {
-    const int nv = (int)div_ceil((size_t)q.kp / 4, 256);
-    void (*qk)(QuantArgs) = nv <= 3 ? k_quant_rows_f16<3> : k_quant_rows_f16<8>;
-    hipLaunchKernelGGL(qk, dim3(q.m_pad), dim3(256), 0, stream, q);
+static hipError_t launch_gemm_f16(const Weights &w, QuantArgs q, const GemmArgs &a, hipStream_t stream) {
     // token tile: 64 (TTW 4) while the grid still covers the chip twice over, else narrower (short prompts, one rank's share)
     const size_t gx0 = div_ceil(div_ceil(w.rows, 16), 16);
     const int ttw = gemm_token_tiles(gx0, q.m_pad, false, kGemmCUs);
+    const unsigned gy = (unsigned)div_ceil((size_t)q.m, (size_t)16 * ttw);
+    const int nv = (int)div_ceil((size_t)q.kp / 4, 256);
+    void (*qk)(QuantArgs) = nv <= 3 ? k_quant_rows_f16<3> : k_quant_rows_f16<8>;
+    q.m_pad = (int)gy * 16 * ttw;
+    hipLaunchKernelGGL(qk, dim3(q.m_pad), dim3(256), 0, stream, q);
     const bool fmt1 = a.stiles_h != nullptr;
     void (*fk)(GemmArgs, uint32_t) = fmt1 ? (ttw == 4 ? k_gemm_f16a<1, 4> : ttw == 2 ? k_gemm_f16a<1, 2> : k_gemm_f16a<1, 1>)
                                           : (ttw == 4 ? k_gemm_f16a<0, 4> : ttw == 2 ? k_gemm_f16a<0, 2> : k_gemm_f16a<0, 1>);
@@ -2529,7 +2513,7 @@ static hipError_t launch_gemm_f16(const Weights &w, const QuantArgs &q, const Ge
         }
     }
     g_last_gemm_tile = GemmTileChoice{2, 16 * ttw, 4, fmt1 ? 4 : 5};
-    hipLaunchKernelGGL(fk, dim3((unsigned)gx0, (unsigned)(q.m_pad / (16 * ttw))), dim3(256), (size_t)2 * ttw * 16 * 512, stream, a, lut_f16_hi(w.lut));
+    hipLaunchKernelGGL(fk, dim3((unsigned)gx0, gy), dim3(256), (size_t)2 * ttw * 16 * 512, stream, a, lut_f16_hi(w.lut));
     return hipGetLastError();
 }
 
@@ -2634,17 +2618,28 @@ bool gemm_takes_few(const Weights &w, const GemvFusion &fu, size_t m, int ndig) 
     return workgroups * (0.2 + 0.35 * blocks) + (double)(w.rows * w.cols / 4) / 4800 <= 920 * blocks * rounds + way_back;
 }
 
-static hipError_t launch_gemm_fp6(const Weights &w, const QuantArgs &q, const GemmArgs &a, hipStream_t stream) {
+static hipError_t launch_gemm_fp6(const Weights &w, QuantArgs q, const GemmArgs &a, hipStream_t stream) {
+    size_t gx0 = div_ceil(div_ceil(w.rows, 16), 16);
+    static const size_t cover_asked = [] { const char *e = getenv("BITNET_HIP_FP6_COVER"); return e ? (size_t)atoi(e) : 0; }();  // (developer sweep of the token tile)
+    const size_t cover = cover_asked ? cover_asked : 2 * kGemmCUs;
+    int ttw = gemm_token_tiles(gx0, q.m_pad, false, cover);
+    bool rt5 = ttw == 4 && !a.silu_mul && w.rows % 4 == 0 && gemm_five_tiles(w.rows, q.m_pad);
+    if (!rt5) ttw = gemm_token_tiles(gx0, q.m_pad, true, cover);
+    // From 1024 columns on the tile whose launch is the shortest by what was measured (27 sizes from 100 to 2490 tokens, resident image); us with the rule above, which also counted the
+    // padding's tiles, and with this one: q|k|v at 850 to 1000 tokens 24.3 to 25.8 -> 19.3 to 20.7, 1800 38.6 -> 33.8; gate|up at 256 24.7 -> 20.1, 400 39.1 -> 28.1, 576 39.4 -> 35.5.
+    if (q.kp >= 1024 && !cover_asked) {
+        static const TileCost costs[] = {{4, 1, 2.5, 0.2, 0.0, 0.95, 0.55, 0}, {4, 2, 3.0, 0.0, 0.0, 1.35, 0.80, 0}, {4, 4, 4.5, 0.0, 0.0, 1.80, 1.65, 2.85}, {5, 4, 4.5, 0.0, 0.0, 2.30, 2.30, 3.60}};
+        const TileCost *c = cheapest_tile(costs, w.rows, (size_t)q.kp / 256, (size_t)q.m, a.residual != nullptr, !a.silu_mul && w.rows % 320 == 0);
+        ttw = c->ttw, rt5 = c->rt == 5;
+    }
+    if (rt5) gx0 = w.rows / 320;
+    const unsigned gy = (unsigned)div_ceil((size_t)q.m, (size_t)16 * ttw);
     const int nv = (int)div_ceil((size_t)q.kp / 4, 256);
     void (*qk)(QuantArgs) = nv <= 3 ? k_quant_rows<2, 3, 1> : k_quant_rows<2, 8, 1>;
-    if (quant_rows_w_applies(q)) launch_quant_rows_w(q, true, stream);
+    const bool by_waves = quant_rows_w_applies(q);
+    q.m_pad = (int)gy * 16 * ttw;  // (rows that no tile reads are not quantised)
+    if (by_waves) launch_quant_rows_w(q, true, stream);
     else hipLaunchKernelGGL(qk, dim3(q.m_pad), dim3(256), (size_t)(q.kp / 32) * 144 + (size_t)(q.kp / 256) * 576, stream, q);  // LDS: the row's integers (144 bytes per 32 columns) + its packed image
-    size_t gx0 = div_ceil(div_ceil(w.rows, 16), 16);
-    static const size_t cover = [] { const char *e = getenv("BITNET_HIP_FP6_COVER"); return e ? (size_t)atoi(e) : 2 * kGemmCUs; }();  // (developer sweep of the token tile)
-    int ttw = gemm_token_tiles(gx0, q.m_pad, false, cover);
-    const bool rt5 = ttw == 4 && !a.silu_mul && w.rows % 4 == 0 && gemm_five_tiles(w.rows, q.m_pad);
-    if (rt5) gx0 = w.rows / 320;
-    else ttw = gemm_token_tiles(gx0, q.m_pad, true, cover);
     const bool res = a.tiles4 != nullptr;
     void (*fk)(GemmArgs, uint32_t) = res ? (rt5 ? k_gemm_fp6<4, 5, 1> : ttw == 4 ? k_gemm_fp6<4, 4, 1> : ttw == 2 ? k_gemm_fp6<2, 4, 1> : k_gemm_fp6<1, 4, 1>)
                                          : (rt5 ? k_gemm_fp6<4, 5> : ttw == 4 ? k_gemm_fp6<4> : ttw == 2 ? k_gemm_fp6<2> : k_gemm_fp6<1>);
@@ -2666,10 +2661,10 @@ static hipError_t launch_gemm_fp6(const Weights &w, const QuantArgs &q, const Ge
         static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void *>(k_gemm_fp6w), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);  // (72 KiB of tile buffers; once, thread-safe)
         if (raised != hipSuccess) return raised;
         g_last_gemm_tile.wave_rows = 128, g_last_gemm_tile.group_rows = 256;  // the 2 x 2 arrangement: a wave owns 128 rows x 32 tokens of the 256 x 64 tile
-        hipLaunchKernelGGL(k_gemm_fp6w, dim3((unsigned)gx0, (unsigned)(q.m_pad / 64)), dim3(256), (size_t)2 * 64 * 576, stream, aw);
+        hipLaunchKernelGGL(k_gemm_fp6w, dim3((unsigned)gx0, gy), dim3(256), (size_t)2 * 64 * 576, stream, aw);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(fk, dim3((unsigned)gx0, (unsigned)(q.m_pad / (16 * ttw))), dim3(256), (size_t)2 * ttw * 16 * 576, stream, aw, lut_fp4(w.lut));
+    hipLaunchKernelGGL(fk, dim3((unsigned)gx0, gy), dim3(256), (size_t)2 * ttw * 16 * 576, stream, aw, lut_fp4(w.lut));
     return hipGetLastError();
 }
 
@@ -2722,6 +2717,29 @@ hipError_t launch_rows_to_f16(const float *x, const float *gamma, size_t m, size
     return hipGetLastError();
 }
 
+// ---- tiles of the chain launches ----------------------------------------------------------------------------------------
+// The one whose launch is the shortest (TileCost) by what was measured: us, all 32 sizes from 72 to 4000 tokens of the 2B model's o, down, q|k|v and gate|up, weights from the image; the
+// choice is 1.5 % behind the best in the mean.  Before, the tile halved until its workgroups, those of the padding included, covered the CUs once; us then and with this rule: down at 640
+// tokens 49 -> 37, 777 50 -> 39, 1800 98 -> 83, 2300 104 -> 92 (QK256 85 -> 68, 87 -> 72 at the last two), o at 1100 31 -> 26, 2300 50 -> 42, gate|up at 100 23 -> 19, 300 42 -> 36,
+// 400 44 -> 37, q|k|v at 400 24 -> 18; BitNet32-F16 prompt of 777 tokens 6.36 -> 5.73 ms.
+// Rows of fewer than 1024 columns have too few steps for that to count: there the former rule stands (tiles halve until they cover the CUs; rows halve up to 320 workgroups).
+struct F16Tile {
+    int rt, ttw;
+};
+static F16Tile f16_covering_tile(const Weights &w, bool silu_mul, size_t m_pad) {
+    const int ttw = gemm_token_tiles(w.rows / 256, m_pad, false, kGemmCUs);
+    if (ttw == 4 && !silu_mul && gemm_five_tiles(w.rows, m_pad)) return {5, 4};
+    return {ttw < 4 && w.rows / 256 * (m_pad / (16 * ttw)) <= 320 ? 2 : 4, ttw};
+}
+static F16Tile f16_tile(const Weights &w, bool silu_mul, bool residual, size_t m) {
+    static const TileCost costs[2][5] = {{{2, 1, 4.0, 0.2, 0.0, 0.73, 0.32, 0}, {2, 2, 5.0, 0.4, 0.3, 0.98, 0.475, 0}, {4, 2, 5.3, 0.6, 0.7, 1.12, 0.765, 0},
+                                          {4, 4, 6.0, 1.8, 1.5, 1.78, 1.54, 2.76}, {5, 4, 10.0, 1.4, 1.3, 2.04, 1.8, 3.30}},
+                                         {{2, 1, 6.0, 0.2, 0.1, 0.80, 0.405, 0}, {2, 2, 5.5, 0.5, 0.5, 1.09, 0.555, 0}, {4, 2, 6.5, 1.0, 1.1, 1.34, 0.96, 0},
+                                          {4, 4, 7.0, 2.7, 3.3, 2.04, 1.82, 3.03}, {5, 4, 11.0, 2.7, 2.8, 2.42, 2.3, 3.70}}};
+    const TileCost *c = cheapest_tile(costs[w.scaled ? 1 : 0], w.rows, w.cols / 256, m, residual, !silu_mul && w.rows % 320 == 0);
+    return {c->rt, c->ttw};
+}
+
 hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m, hipStream_t stream) {
     if (!gemm_f16_chain_supported(w) || m == 0 || !io.xh) return hipErrorInvalidValue;
     if (io.stats_in && !(w.ln_g && io.n_stats > 0)) return hipErrorInvalidValue;
@@ -2752,19 +2770,30 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
 #ifdef BH_STAMPS
     a.stamps = g_mfma_stamps;
 #endif
-    size_t gx0 = w.rows / 256;
-    const int ttw = gemm_token_tiles(gx0, m_pad, false, kGemmCUs);
     const bool fmt1 = w.scaled, image = io.image != nullptr;
     a.tiles4 = io.image;
     if (io.few) return io.qb_out ? hipErrorInvalidValue : launch_gemm_f16_few(w, a, stream);
-    const bool rt5 = ttw == 4 && !io.silu_mul && gemm_five_tiles(w.rows, m_pad);
-    // Short prompts: waves of 32 rows while the waves of 64 leave most CUs one workgroup.  A K step of such a workgroup is a serial chain (staging, expansion, LDS reads, MFMAs,
-    // barrier), so two of half the rows on a CU take less than one.  BitNet32-F16 prompt of bitnet-b1.58-2B-4T, weights from the image, ms with the line at 320 / 448 workgroups / without:
-    // 193 tokens 3.30 / 3.30 / 3.79, 256 3.35 / 3.41 / 3.84, 257 3.79 / 3.80 / 4.29, 400 4.44 / 4.41 / 4.92, 512 4.60 / 4.61 / 5.04, 640 5.82 / 5.77 / 5.96, 777 6.16 / 6.13 / 6.51,
-    // 1024 6.57 / 6.57 / 6.91 (at 256: 3.91 at 257 tokens, 4.91 at 400); at 384 as at 320.
-    const bool rt2 = ttw < 4 && gx0 * (m_pad / (16 * ttw)) <= 320;
-    if (rt5) gx0 = w.rows / 320;
-    if (rt2) gx0 = w.rows / 128;
+    // Wide launches (gate|up: 54 row blocks): 128-token workgroups (k_gemm_f16h: half the code expansion per MFMA) on as many row blocks as fill WHOLE rounds
+    // of the 512 slots, k_gemm_f16a's 64-token workgroups on the rest -- 13824 rows x 4096 tokens: 48 x 32 = 1536 workgroups = 3 rounds, then 6 x 64 = 384
+    // half-length ones (as one 128-token grid it would be 3.375 rounds: the 16 % idle tail would cost more than the expansion saves).  Same arithmetic per
+    // output element whichever kernel computes it (k-order, f32 accumulation): bit-identical to the one-kernel launch.  BITNET_HIP_GEMM_F16H=0: off.
+    static const int f16h_mode = [] { const char *e = getenv("BITNET_HIP_GEMM_F16H"); return e ? atoi(e) : 1; }();
+    const F16Tile covering = f16_covering_tile(w, io.silu_mul, m_pad);
+    size_t n_a = 0;  // row blocks of the 128-token workgroups
+    if (f16h_mode && covering.ttw == 4 && covering.rt == 4 && !io.qb_out && m_pad % 128 == 0 && w.rows * w.cols / (image ? 2 : 4) < ((size_t)1 << 31)) {
+        const size_t slots = 2 * kGemmCUs, t128 = m_pad / 128, blocks = w.rows / 256;
+        n_a = (blocks * t128 / slots) * slots / t128;  // those that fill whole rounds
+        // a launch whose 128-token workgroups fit ONE round that is at least three quarters full (q|k|v: 15 x 32 = 480 of 512 slots, against 960 = 1.9 rounds of
+        // 64-token ones: a 128-token workgroup takes 1.85 x a 64-token one) goes to k_gemm_f16h whole
+        if (blocks * t128 <= slots && 4 * blocks * t128 >= 3 * slots) n_a = blocks;
+        if (blocks < 24 && n_a != blocks) n_a = 0;
+        if (n_a < blocks / 2) n_a = 0;
+    }
+    // (a launch that also leaves QB32 rows wants whole tiles of 64 tokens)
+    const F16Tile tile = n_a > 0 || io.qb_out || w.cols < 1024 ? covering : f16_tile(w, io.silu_mul, io.residual != nullptr, m);
+    const int ttw = tile.ttw;
+    const bool rt5 = tile.rt == 5, rt2 = tile.rt == 2;
+    const size_t gx0 = w.rows / (64 * (size_t)tile.rt);
     auto of_tile = [&](auto fmt) {
         constexpr int F = decltype(fmt)::value;
         return rt5   ? k_gemm_f16a<F, 4, 1, 5>
@@ -2790,45 +2819,31 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
     }
     g_last_gemm_tile = GemmTileChoice{2, 16 * ttw, 4, fmt1 ? 4 : 5, rt5 ? 80 : 64, 0, rt2 ? 128 : 0};
     const size_t lds = (size_t)2 * ttw * 16 * 512 + (size_t)ttw * 16 * 8 + 4096;  // two tile buffers + the tokens' (mean, 1 / denom) + the statistics scratch
-    // Wide launches (gate|up: 54 row blocks): 128-token workgroups (k_gemm_f16h: half the code expansion per MFMA) on as many row blocks as fill WHOLE rounds
-    // of the 512 slots, this kernel's 64-token workgroups on the rest -- 13824 rows x 4096 tokens: 48 x 32 = 1536 workgroups = 3 rounds, then 6 x 64 = 384
-    // half-length ones (as one 128-token grid it would be 3.375 rounds: the 16 % idle tail would cost more than the expansion saves).  Same arithmetic per
-    // output element whichever kernel computes it (k-order, f32 accumulation): bit-identical to the one-kernel launch.  BITNET_HIP_GEMM_F16H=0: off.
-    static const int f16h_mode = [] { const char *e = getenv("BITNET_HIP_GEMM_F16H"); return e ? atoi(e) : 1; }();
-    const size_t slots = 2 * kGemmCUs;
-    if (f16h_mode && ttw == 4 && !rt5 && !io.qb_out && m_pad % 128 == 0 && w.rows * w.cols / (image ? 2 : 4) < ((size_t)1 << 31)) {
-        const size_t t128 = m_pad / 128;
-        size_t n_a = (gx0 * t128 / slots) * slots / t128;  // row blocks whose 128-token workgroups fill whole rounds
-        // a launch whose 128-token workgroups fit ONE round that is at least three quarters full (q|k|v: 15 x 32 = 480 of 512 slots, against 960 = 1.9 rounds of
-        // 64-token ones: a 128-token workgroup takes 1.85 x a 64-token one) goes to k_gemm_f16h whole
-        if (gx0 * t128 <= slots && 4 * gx0 * t128 >= 3 * slots) n_a = gx0;
-        if (gx0 < 24 && n_a != gx0) n_a = 0;
-        if (n_a >= gx0 / 2 && n_a > 0) {
-            void (*hk)(GemmArgs, uint32_t) = f16_instance(fmt1, image, [](auto fmt) { return k_gemm_f16h<decltype(fmt)::value>; });
-            {
-                static std::mutex h_mu;
-                static std::unordered_set<const void *> h_raised;
-                std::lock_guard<std::mutex> lk(h_mu);
-                if (!h_raised.count((const void *)hk)) {
-                    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(hk), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-                    if (e != hipSuccess) return e;
-                    h_raised.insert((const void *)hk);
-                }
+    if (n_a > 0) {
+        void (*hk)(GemmArgs, uint32_t) = f16_instance(fmt1, image, [](auto fmt) { return k_gemm_f16h<decltype(fmt)::value>; });
+        {
+            static std::mutex h_mu;
+            static std::unordered_set<const void *> h_raised;
+            std::lock_guard<std::mutex> lk(h_mu);
+            if (!h_raised.count((const void *)hk)) {
+                hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(hk), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+                if (e != hipSuccess) return e;
+                h_raised.insert((const void *)hk);
             }
-            GemmArgs aa = a;
-            // (with the image 3 row blocks at gate|up, block scales counted twice like the codes; groups of 4, of 6 and none take the same, prompts of 1024 to 4096 tokens within 0.5 %)
-            aa.wgroup = gemm_weight_group(n_a, 256, image ? 2 * w.cols : w.cols, fmt1);
-            hipLaunchKernelGGL(hk, dim3((unsigned)n_a, (unsigned)t128), dim3(256), (size_t)2 * 128 * 256 + 128 * 8 + 4096, stream, aa, lut_f16_hi(w.lut));
-            g_last_gemm_tile = GemmTileChoice{2, 128, 4, fmt1 ? 4 : 5, 64};
-            if (n_a == gx0) return hipGetLastError();
-            a.bx_off = (int)n_a;
-            a.wgroup = 0;
-            hipLaunchKernelGGL(fk, dim3((unsigned)(gx0 - n_a), (unsigned)(m_pad / 64)), dim3(256), lds, stream, a, lut_f16_hi(w.lut));
-            return hipGetLastError();
         }
+        GemmArgs aa = a;
+        // (with the image 3 row blocks at gate|up, block scales counted twice like the codes; groups of 4, of 6 and none take the same, prompts of 1024 to 4096 tokens within 0.5 %)
+        aa.wgroup = gemm_weight_group(n_a, 256, image ? 2 * w.cols : w.cols, fmt1);
+        hipLaunchKernelGGL(hk, dim3((unsigned)n_a, (unsigned)(m_pad / 128)), dim3(256), (size_t)2 * 128 * 256 + 128 * 8 + 4096, stream, aa, lut_f16_hi(w.lut));
+        g_last_gemm_tile = GemmTileChoice{2, 128, 4, fmt1 ? 4 : 5, 64};
+        if (n_a == gx0) return hipGetLastError();
+        a.bx_off = (int)n_a;
+        a.wgroup = 0;
+        hipLaunchKernelGGL(fk, dim3((unsigned)(gx0 - n_a), (unsigned)(m_pad / 64)), dim3(256), lds, stream, a, lut_f16_hi(w.lut));
+        return hipGetLastError();
     }
     a.wgroup = gemm_weight_group(gx0, rt5 ? 320 : rt2 ? 128 : 256, image ? 2 * w.cols : w.cols, fmt1);
-    hipLaunchKernelGGL(fk, dim3((unsigned)gx0, (unsigned)(m_pad / (16 * ttw))), dim3(256), lds, stream, a, lut_f16_hi(w.lut));
+    hipLaunchKernelGGL(fk, dim3((unsigned)gx0, (unsigned)div_ceil(m, (size_t)16 * ttw)), dim3(256), lds, stream, a, lut_f16_hi(w.lut));
     return hipGetLastError();
 }
 
@@ -2894,7 +2909,7 @@ hipError_t launch_gemm_qb32(const Weights &w, const GemmF16Io &io, size_t m, hip
     }
     g_last_gemm_tile = GemmTileChoice{2, 16 * ttw, 4, 8, rt5 ? 80 : 64, res ? 1 : 0};  // scale_mode 8: the fp6 form on QB32 rows
     a.wgroup = gemm_weight_group(gx0, rt5 ? 320 : 256, res ? 2 * w.cols : w.cols, false, res ? kFp4GroupBudget : (size_t)3 << 19);
-    hipLaunchKernelGGL(fk, dim3((unsigned)gx0, (unsigned)(m_pad / (16 * ttw))), dim3(256), (size_t)2 * ttw * 16 * (576 + 8) + (size_t)ttw * 16 * 8 + 4096, stream, a, lut_fp4(w.lut));
+    hipLaunchKernelGGL(fk, dim3((unsigned)gx0, (unsigned)div_ceil(m, (size_t)16 * ttw)), dim3(256), (size_t)2 * ttw * 16 * (576 + 8) + (size_t)ttw * 16 * 8 + 4096, stream, a, lut_fp4(w.lut));
     return hipGetLastError();
 }
 

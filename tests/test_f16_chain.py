@@ -139,6 +139,31 @@ def test_f16_chain_half_slab_waves(hip, torch_, fmt, m):
     hip.weights_free(h)
 
 
+@pytest.mark.parametrize("fmt,m,tile", [("qk256", 65, (128, 16)), ("i2s", 65, (128, 16)), ("qk256", 833, (128, 16)), ("i2s", 833, (128, 32)), ("qk256", 1281, (256, 32)), ("i2s", 1281, (256, 32))])
+def test_f16_chain_no_tile_past_the_last_token(hip, torch_, fmt, m, tile):
+    """Tiles chosen by their measured cost; token counts that end in a tile ahead of the padding's end, grids that are no multiple of eight workgroups: every live value is written, the
+    partials of the padding that no workgroup computes are zero, and nothing behind the last token's row is touched"""
+    rows, cols, mp = 2560, 1024, -(-m // 64) * 64
+    rng = np.random.default_rng(m)
+    h, w = make_matrix(hip, rng, fmt, rows, cols)
+    x = rng.normal(0, 1, (mp, cols)).astype(np.float16)
+    res = rng.normal(0, 1, (m, rows)).astype(np.float32)
+    y, st = torch_.full((mp, rows), 7.0, device="cuda"), torch_.full((rows // 64, mp, 2), float("nan"), device="cuda")
+    y[:m] = torch_.from_numpy(res).cuda()
+    hip.matmul_f16_dev(h, torch_.from_numpy(x).cuda(), m, y=y, residual=y, stats_out=st)
+    assert (hip.matmul_last_workgroup_rows(), hip.matmul_last_tile()["wave_tokens"]) == tile
+    torch_.cuda.synchronize()
+    out, xd = y.cpu().numpy().astype(np.float64), x[:m].astype(np.float64)
+    got = out[:m]
+    assert np.max(np.abs(got - (res + xd @ w.T)) / (np.abs(xd) @ np.abs(w).T + np.abs(res) + 1e-6)) <= 2e-6  # f16 inputs: accumulation order alone
+    assert np.all(out[m:] == 7.0)
+    slabs, s = got.reshape(m, rows // 64, 64), st.cpu().numpy()
+    for e in (1, 2):  # f32 sums of 64 terms: 2^-24 per addition against the magnitudes
+        assert np.all(np.abs(s[:, :m, e - 1].T - (slabs ** e).sum(axis=2)) <= 4e-6 * (np.abs(slabs) ** e).sum(axis=2) + 1e-6)
+    assert np.all(s[:, m:] == 0)
+    hip.weights_free(h)
+
+
 @pytest.mark.parametrize("fmt", ["qk256", "i2s"])
 def test_f16_chain_layernorm_after_product_and_silu(hip, oracle, torch_, fmt):
     """qkv-like (LayerNorm -> f32 rows) and gate|up-like (LayerNorm -> silu(gate) * up -> f16 rows) launches at the 2B-4T widths,

@@ -385,6 +385,27 @@ def test_few_rows_only_where_they_are_faster(hip, torch_, rows, cols, m, few):
         hip.weights_free(i)
 
 
+# the fp6 digits' tiles by their measured cost: one, two and four token tiles per wave and five row tiles, rows and tokens that end inside a tile
+@pytest.mark.parametrize("rows,cols,m,tokens", [(1000, 1100, 209, 16), (3840, 1280, 850, 32), (13824, 1280, 449, 64), (3840, 1100, 1793, 64), (960, 1024, 4133, 32)])
+def test_fp6_tiles_on_ragged_shapes(hip, torch_, rows, cols, m, tokens):
+    """bit for bit the int8 planes'; no row behind the last token's is touched"""
+    rng = np.random.default_rng(rows + cols + m)
+    stride = -(-cols // 256) * 64
+    x = (rng.normal(0.1, 1.0, (m, cols)) * np.exp(rng.uniform(-3, 3, (m, 1)))).astype(np.float32)
+    gd = torch_.from_numpy((rng.uniform(0.5, 1.5, cols) / 80).astype(np.float32)).cuda()
+    h = hip.weights_upload_qk256(rng.integers(0, 256, rows * stride, dtype=np.uint8), rows, cols, stride)
+    wsb = hip.matmul_workspace_bytes(m, cols, 2)
+    ws, outs = torch_.empty(wsb, dtype=torch_.uint8, device="cuda"), []
+    for flags in (FP6_DIGITS, INT8_DIGITS):
+        y = torch_.full((m + 70, rows), 7.0, device="cuda")
+        hip.matmul_fused_dev(h, torch_.from_numpy(x).cuda(), y, m, ws, wsb, ln_gamma=gd, ln_eps=1e-5, flags=flags, digits=2)
+        t = hip.matmul_last_tile()
+        assert (t["scale_mode"], t["wave_tokens"]) == (6, tokens) if flags == FP6_DIGITS else t["scale_mode"] == 0, t
+        outs.append(y.cpu().numpy())
+    assert not np.isnan(outs[0]).any() and np.all(outs[0][m:] == 7.0) and np.array_equal(*outs)
+    hip.weights_free(h)
+
+
 # the wide int8 tiles where few rows no longer take them: rows, columns and tokens that end inside a tile, behind 192 rows
 @pytest.mark.parametrize("rows,cols,m", [(1000, 1100, 257), (48, 512, 200), (320, 6912, 230), (33, 260, 193), (2570, 2564, 1030)])
 def test_wide_int8_tiles_on_ragged_shapes(hip, oracle, torch_, rows, cols, m):
