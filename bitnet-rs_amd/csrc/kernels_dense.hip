@@ -1238,18 +1238,31 @@ __global__ __launch_bounds__(64 * WN * WM, 2) void k_dense_gemm(GemmArgsD p, int
 
 thread_local DenseTile g_last_dense_tile;
 
-template <int T, int ST>
+// TM: the rows of the plan's tiles
+template <int TN, int TM, int WN, int WM, int ST>
 static hipError_t grouped_go(const GemmArgsD &a, hipStream_t s) {
-    const int tn = (a.n + T - 1) / T;
-    constexpr size_t lds = (size_t)ST * T * 256;
-    auto fn = a.gated ? k_dense_gemm<T, T, 2, 2, ST, false, true, true> : k_dense_gemm<T, T, 2, 2, ST, false, true>;
+    const int tn = (a.n + TN - 1) / TN;
+    constexpr size_t lds = (size_t)ST * (TN + TM) * 128;
+    auto fn = a.gated ? k_dense_gemm<TN, TM, WN, WM, ST, false, true, true> : k_dense_gemm<TN, TM, WN, WM, ST, false, true>;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    g_last_dense_tile = {T, T, 4, 1};
-    hipLaunchKernelGGL(fn, dim3((tn * a.max_tiles + 7) / 8 * 8), dim3(256), lds, s, a, tn, 0, 0);
+    g_last_dense_tile = {TN, TM, WN * WM, 1};
+    hipLaunchKernelGGL(fn, dim3((tn * a.max_tiles + 7) / 8 * 8), dim3(64 * WN * WM), lds, s, a, tn, 0, 0);
     return hipGetLastError();
+}
+// Experts' products, weights from HBM, us at 64 experts, n x k and rows per expert (64 x 64 in three buffers / 128 x 64 / 128 x 128 in four waves / in eight): 896 x 3072, 3 rows 67 / 62 /
+// 63 / 65, 50 78 / 70 / 72 / 74, 88 104 / 105 / 78 / 81, 125 131 / 113 / 123 / 110, 188 163 / 137 / 116 / 127; 3072 x 896, 3 61 / 60 / 63 / 71, 50 82 / 73 / 81 / 87, 88 107 / 95 / 89 /
+// 94; 448 x 1536, 3 18 / 25 / 26 / 20, 50 22 / 29 / 28 / 23, 88 31 / 28 / 29 / 25; 1360 x 3072 gated, 12 99 / 96 / 117 / 99, 88 160 / 139 / 132 / 117, 188 254 / 203 / 163 / 188.
+// Tiles of 64 rows: 128 columns while they reach every CU (a workgroup's activations serve twice the columns), else 64 in three buffers, of which a CU takes three (in four, two: 20 / 18).
+// Tiles of 128 rows: eight waves with four buffers for long K while an expert has one tile, and there is one round and a half of workgroups; else two workgroups per CU, which overlap
+// their ends.
+static hipError_t launch_grouped(const GemmArgsD &a, hipStream_t s) {
+    const int experts = a.max_tiles - a.m / a.tile;  // (how a plan counts its tiles)
+    if (a.tile == 64) return (long)experts * ((a.n + 127) / 128) >= 384 ? grouped_go<128, 64, 2, 2, 2>(a, s) : grouped_go<64, 64, 2, 2, 3>(a, s);
+    if (a.tile != 128) return hipErrorInvalidValue;
+    return a.k >= 1536 && a.m <= 112l * experts ? grouped_go<128, 128, 2, 4, 4>(a, s) : grouped_go<128, 128, 2, 2, 2>(a, s);
 }
 
 template <int TN, int TM, int WN, int WM, int ST, bool MUL = false>
@@ -1503,7 +1516,7 @@ hipError_t launch_dense_gemm(const GemmArgsD &args, hipStream_t s) {
             return hipGetLastError();
         }
         if (a.c_f32) return hipErrorInvalidValue;
-        return a.tile == 128 ? grouped_go<128, 2>(a, s) : a.tile == 64 ? grouped_go<64, 4>(a, s) : hipErrorInvalidValue;
+        return launch_grouped(a, s);
     }
     if (a.a_f32) {
         g_last_dense_tile = {64, 64, 4, 1};

@@ -665,6 +665,16 @@ def test_experts_of_a_portion(hip, pkg, m, experts, top, tile, width, ff, f32):
     assert u.rms_error(got, want) < (F32_TOL if f32 else 8e-3)
 
 
+# the forms of the grouped products: 128 columns by 64 rows where that reaches every CU, eight waves for long K and one tile per expert; last columns and rows inside a tile
+@pytest.mark.parametrize("m,experts,top,tile,width,ff,form", [(130, 200, 2, 64, 250, 72, (128, 64, 4, 1)), (90, 40, 3, 64, 250, 72, (64, 64, 4, 1)), (90, 40, 3, 128, 112, 1600, (128, 128, 8, 1)),
+                                                             (150, 5, 4, 128, 112, 1600, (128, 128, 4, 1))])
+def test_forms_of_the_experts_products(hip, pkg, m, experts, top, tile, width, ff, form):
+    test_experts_of_a_portion(hip, pkg, m, experts, top, tile, width, ff, False)
+    assert tuple(hip.dense_matmul_last_tile()) == form
+    test_gated_experts_of_a_portion(hip, pkg, m, experts, 2, top, tile, width, ff, False)
+    assert tuple(hip.dense_matmul_last_tile()) == form
+
+
 @pytest.mark.parametrize("experts,top,width,ff,cols0", [(4, 1, 64, 24, 8), (6, 6, 112, 40, 200), (12, 3, 320, 72, 160), (64, 8, 1000, 520, 1032), (128, 4, 2560, 768, 3328), (9, 3, 90, 16, 64)])
 def test_experts_of_one_token(hip, pkg, experts, top, width, ff, cols0):
     g = rng(experts, width, ff)
