@@ -231,6 +231,16 @@ hipError_t launch_gqa_rows(const Gqa &g, void *rows, size_t ld, int rows_f32, in
 hipError_t launch_gqa_step(const Gqa &g, const GqaStep &a, hipStream_t s);
 hipError_t launch_gqa_any(const Gqa &g, const void *q, size_t ldq, int q_f32, int cache_f32, const int *pos, int q0, int nq, float *scratch, hipStream_t s);
 hipError_t launch_gqa_merge(const Gqa &g, const int *pos, int q0, int nq, const float *scratch, void *out, size_t ldo, int out_bf16, hipStream_t s);
+struct GqaOut {  // records of one query -> output -> product
+    Gqa g;
+    const int *pos = nullptr;
+    const float *scratch = nullptr, *bias = nullptr;
+    const uint16_t *w = nullptr;
+    float *y = nullptr;
+    int rows = 0, cols = 0, ld = 0, records = 0;
+};
+int gqa_out_records(const Gqa &g, int cols);
+hipError_t launch_gqa_out(const GqaOut &a, hipStream_t s);
 extern thread_local int g_last_gqa_groups;  // groups of four waves per workgroup of launch_gqa_prefill's last launch on this thread
 hipError_t launch_gqa_prefill(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, hipStream_t s);
 bool delta_supported(int dimp, int vdimp);

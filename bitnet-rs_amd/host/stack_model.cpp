@@ -10,6 +10,8 @@
 namespace bitnet_host {
 
 namespace {
+// Records that a step's output products merge themselves, 128 keys each: one form of the step for up to two of them, one for up to four, all that is faster than a launch of its own.
+constexpr size_t kFewRecords = 2, kMostRecords = 4;
 constexpr size_t kDecodeSlice = 64;  // queries per call where a portion takes a decode form of its attention
 size_t up_to(size_t v, size_t a) { return (v + a - 1) / a * a; }
 }  // namespace
@@ -751,6 +753,32 @@ int StackModel::step_loop_in() {
     return 0;
 }
 
+// Does the block's output product take the attention's records as they are?  (nothing but them goes into it)
+bool StackModel::merges_in_out(size_t i, int which) const {
+    const Block &B = layers_[i].block[which];
+    if (f32_ || !B.used || !B.mixer || spec_.layers[i].mixer != LayerSpec::Attention || B.fs > 0 || B.expert_up.w) return false;
+    const bitnet_hip_gqa a = gqa_args(i, 0, row_[0], B.main, true);
+    return bitnet_hip_gqa_out_records(&a, B.out.cols) >= kMostRecords;
+}
+
+// records of a query at the position, over the layers
+size_t StackModel::records_at(int pos) const {
+    size_t most = 0;
+    for (size_t i = 0; i < layers_.size(); ++i) {
+        if (!merges_in_out(i, 0)) continue;
+        const AttentionSpec &m = spec_.layers[i].attention;
+        int first = m.chunk > 0 ? pos / m.chunk * m.chunk : 0;
+        if (m.window > 0) first = std::max(first, pos - m.window + 1);
+        most = std::max(most, (size_t)(pos - first / 128 * 128) / 128 + 1);
+    }
+    return most;
+}
+
+int StackModel::form_at(int pos) const {
+    const size_t n = records_at(pos);
+    return n == 0 || n > kMostRecords ? 0 : n <= kFewRecords ? 1 : 2;
+}
+
 // the sublayers of a block; their sum is left in y_[which]
 int StackModel::step_block(size_t i, int pass, int which) {
     const Layer &L = layers_[i];
@@ -787,6 +815,10 @@ int StackModel::step_block(size_t i, int pass, int which) {
         } else {
             BCHK(bitnet_hip_gqa_rows_dev(&a, proj, B.main, 1, f32_, pos_, 1, nullptr, 0, stream_));
             BCHK(bitnet_hip_gqa_any_dev(&a, proj, B.main, 1, f32_, pos_, 0, 1, scratch_, stream_));
+        }
+        if (records_ > 0 && merges_in_out(i, which)) {
+            BCHK(bitnet_hip_gqa_out_dev(&a, pos_, records_, scratch_, B.out.w, B.out.rows, B.out.cols, B.out.ld, B.out_bias, y_[which], stream_));
+            return 0;
         }
         BCHK(bitnet_hip_gqa_merge_dev(&a, pos_, 0, 1, scratch_, row, B.ko, 0, stream_));
     } else if (B.mixer) {
@@ -865,7 +897,8 @@ int StackModel::embed_rows(size_t n, float *out) {
     return 0;
 }
 
-int StackModel::step(bool with_logits, int) {
+int StackModel::step(bool with_logits, int form) {
+    records_ = form == 0 ? 0 : form == 1 ? kFewRecords : kMostRecords;
     cur_ = x0_;
     row_at_ = 0;
     pending_ = Pending();

@@ -150,6 +150,7 @@ class StackModel : public Sequence {
   protected:
     bool ready() const override { return head_ != nullptr && layers_set_ == spec_.layers.size(); }
     int step(bool with_logits, int form) override;
+    int form_at(int pos) const override;  // 0: the attention's records are merged by a launch of their own; 1, 2: by the output products, up to kFewRecords, kMostRecords of them
     int clear_state() override;
 
   private:
@@ -265,6 +266,8 @@ class StackModel : public Sequence {
     int step_side(size_t i);
     int step_linear(size_t i, int pass);
     int step_block(size_t i, int pass, int which);
+    bool merges_in_out(size_t i, int which) const;
+    size_t records_at(int pos) const;
     int step_loop_in();
     // portion of n tokens
     int matmul(const void *a, size_t lda, bool a_f32, const Matrix &m, const float *bias, size_t n, int act0, int act1, size_t split, void *c, size_t ldc,
@@ -303,6 +306,7 @@ class StackModel : public Sequence {
     float *x_[2] = {nullptr, nullptr}, *z_ = nullptr, *q_ = nullptr, *qabs_ = nullptr, *att_ = nullptr, *y_[2] = {nullptr, nullptr}, *act_ = nullptr,
           *lin_ = nullptr, *lino_ = nullptr, *scratch_ = nullptr;
     void *argmax_ = nullptr;
+    size_t records_ = 0;  // of the step at hand: merged by the output products; 0: by a launch of their own
     int row_at_ = 0;  // the row the last block used: its residual gate is read while the next block's is written
     const float *cur_ = nullptr;  // where the step's residual stream is
     float *next_x() const { return cur_ == x_[0] ? x_[1] : x_[0]; }

@@ -823,6 +823,11 @@ int bitnet_hip_gqa_any_dev(const bitnet_hip_gqa *attn, const void *q_dev, size_t
 /* The records of nq queries -> out [nq][ldo], f32 or bf16. */
 int bitnet_hip_gqa_merge_dev(const bitnet_hip_gqa *attn, const int32_t *pos_dev, size_t q0, size_t nq, const float *scratch_dev, void *out_dev,
                              size_t ldo, int out_bf16, void *stream);
+/* The records of one query, merged, and the product behind it in one launch: y = W . [out; 0] + bias, W bf16 [rows][ld].  records: at least as many as the query at *pos can
+ * have (one per 128 keys from a multiple of 128 on), at most bitnet_hip_gqa_out_records (0: not in one launch; one map, up to 4096 columns, an f32 gate). */
+size_t bitnet_hip_gqa_out_records(const bitnet_hip_gqa *attn, size_t cols);
+int bitnet_hip_gqa_out_dev(const bitnet_hip_gqa *attn, const int32_t *pos_dev, size_t records, const float *scratch_dev, const uint16_t *w_dev, size_t rows,
+                           size_t cols, size_t ld, const float *bias_dev, float *y_dev, void *stream);
 /* A portion of a prompt, bf16: the LAST nq of n_ctx positions attend (all of them in the caches); q as gqa_rows leaves it. */
 int bitnet_hip_gqa_prefill_dev(const bitnet_hip_gqa *attn, const uint16_t *q_dev, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out_dev, size_t ldo,
                                void *stream);

@@ -408,6 +408,39 @@ def test_attention_portion_in_groups(hip, pkg, shape, n, nq, groups):
     t.check(out, n - nq, 2e-2)
 
 
+# heads, columns of one, rows of the product, extra columns of its matrix; position, chunk, window; records asked for
+@pytest.mark.parametrize("heads,vdimp,rows,extra", [(1, 32, 5, 0), (12, 128, 1536, 0), (20, 128, 2560, 64), (24, 128, 3072, 0), (3, 160, 70, 32), (4, 1024, 9, 0), (7, 96, 2050, 32)])
+@pytest.mark.parametrize("pos,chunk,window,records", [(0, 0, 0, 1), (127, 0, 0, 2), (128, 0, 0, 2), (511, 0, 0, 4), (300, 256, 0, 1), (900, 0, 200, 3), (1000, 0, 400, 4)])
+@pytest.mark.parametrize("sink,gate", [(False, None), (True, "head"), (False, "column")])
+def test_records_merged_by_the_product(hip, pkg, heads, vdimp, rows, extra, pos, chunk, window, records, sink, gate):
+    """against the merge's own launch and a 64-bit product; what lies in the slots past the position's records is never used"""
+    g = rng(heads, vdimp, rows, pos)
+    n, first = heads * vdimp, max(pos // chunk * chunk if chunk else 0, pos - window + 1 if window else 0)
+    used = (pos - first // 128 * 128) // 128 + 1
+    assert used <= records
+    rec = np.full((heads, 128, 4 + vdimp), np.nan, np.float32)
+    rec[:, :used, 0], rec[:, :used, 1] = 3 * g.standard_normal((heads, used)), g.uniform(0.5, 60.0, (heads, used))
+    rec[:, :used, 4:] = g.standard_normal((heads, used, vdimp))
+    scratch = u.dev_f32(rec.reshape(-1))
+    keep = [u.zeros_f32(64), u.dev_f32(g.standard_normal(heads)), u.dev_f32(g.standard_normal(n))]
+    p = [t.data_ptr() for t in keep]
+    kw = dict(chunk=chunk, window=window)
+    if sink:
+        kw["sink"] = p[1]
+    if gate:
+        kw.update(gate=p[2], ldgate=n, gate_f32=1, gate_columns=int(gate == "column"))
+    attn = pkg.Gqa(heads, 1, 1, 32, 32, vdimp, vdimp, 1024, 1e-5, 0.0, 1.0, 0, 0, p[0], p[0], p[0], **kw)
+    cols = u.up_to(n, 64) + extra
+    ld = u.up_to(cols, 64)
+    w, bias = u.rounded(g.standard_normal((rows, cols)) / np.sqrt(n)), g.standard_normal(rows).astype(np.float32)
+    out, y = u.zeros_f32(1, n), u.zeros_f32(rows)
+    hip.gqa_merge_dev(attn, pos_dev(pos), 0, 1, scratch, out, n, False)
+    assert hip.gqa_out_records(attn, cols) == 4
+    hip.gqa_out_dev(attn, pos_dev(pos), records, scratch, u.dev_bf16(u.padded(w, ld)), rows, cols, ld, y, bias=u.dev_f32(bias))
+    want = w[:, :n].astype(np.float64) @ u.host(out)[0].astype(np.float64) + bias
+    assert u.rms_error(u.host(y), want) < F32_TOL
+
+
 @pytest.mark.parametrize("f32", [True, False])
 @pytest.mark.parametrize("n,nq", [(1, 1), (130, 130), (300, 2)])
 @pytest.mark.parametrize("shape", SHAPES + [(2, 1, 300, 270, 2)])
