@@ -305,13 +305,15 @@ hipError_t launch_experts_route(const float *logits, size_t ldz, const Router &r
 }
 
 // ---- one token --------------------------------------------------------------------------------------------------------
-// Both products in the manner of k_dense_gemv: LPR lanes per row, 16 bytes of weights per lane and chunk of LPR * 8 columns, R rows x U chunks in
-// flight, the input vector in LDS with every segment padded to whole chunks.
+// LPR lanes per row, 16 bytes of weights per lane and chunk of LPR * 8 columns, R rows x U chunks in flight.  The way up in the manner of k_dense_gemv: the input vector in LDS, a row
+// per wave.  On the way down the four waves of a workgroup share its rows' columns, chunk by chunk, so that a lane needs the vector at its own columns only and takes it to registers: no
+// stage in LDS, no barrier ahead of the products and every load of the rows requested at once, their addresses on the scalar unit.  With a row per wave and the vector of all segments in
+// LDS (45 KB for 3072 + 1024 + 8 x 896 columns, read by 768 workgroups, as many bytes as half of the weights) the launch was bound by that stage, its barrier and the waits between its
+// loads; us per step of 4 to 6 layer runs, that form / this one: Mimolix 1b 166.9 / 151.4, 2b 305.2 / 285.7, 3b 257.9 / 240.8, Lurepel 1b 157 / 151, 3b 238 / 229, Sipelorn 1b 246 / 232.
 constexpr int kStage = 4;  // sixteen-byte loads in flight per thread while the vector is staged (rows and segments start on 16 bytes)
 
 template <int R>
-__device__ __forceinline__ void multiply8(const u32x4 (&w)[R], const float *x, float (&acc)[R]) {
-    const f32x4 x0 = *reinterpret_cast<const f32x4 *>(x), x1 = *reinterpret_cast<const f32x4 *>(x + 4);
+__device__ __forceinline__ void multiply8(const u32x4 (&w)[R], f32x4 x0, f32x4 x1, float (&acc)[R]) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         acc[r] = fmaf(x0.x, __builtin_bit_cast(float, w[r].x << 16), acc[r]);
@@ -421,7 +423,10 @@ __global__ __launch_bounds__(256) void k_experts_up(UpK p) {
             else if (g + n_wg * 4 < p.groups)
                 fetch(g + n_wg * 4, 0);
 #pragma unroll
-            for (int u = 0; u < U; ++u) multiply8<R>(c[u], xs + k0 + (u * LPR + l) * 8, acc);
+            for (int u = 0; u < U; ++u) {
+                const f32x4 *x = reinterpret_cast<const f32x4 *>(xs + k0 + (u * LPR + l) * 8);
+                multiply8<R>(c[u], x[0], x[1], acc);
+            }
         }
         if (R > 1 && a.gated) {
 #pragma unroll
@@ -443,91 +448,76 @@ __global__ __launch_bounds__(256) void k_experts_up(UpK p) {
 
 struct OutK {
     ExpertsOut a;
-    int c0, ce, chunks;  // chunks of the first segment, of an expert's, of all (rounded up to whole steps)
+    int c0, ce;          // chunks of the first segment, of an expert's
     unsigned magic;      // ceil(2^20 / ce)
     int groups;
 };
 
 template <int LPR, int R, int U>
-__global__ __launch_bounds__(256) void k_experts_out(OutK p) {
-    extern __shared__ __attribute__((aligned(16))) float xs[];
+__global__ __launch_bounds__(256, 3) void k_experts_out(OutK p) {
     const ExpertsOut &a = p.a;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sub = lane / LPR, l = lane % LPR;
-    constexpr int G = 64 / LPR, CH = LPR * 8;
-    const int ids = lane < a.top ? a.ids[lane] : -1, n_real = __popcll(__ballot(ids >= 0)), end = p.c0 + n_real * p.ce;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), sub = LPR == 64 ? 0 : lane / LPR, l = lane % LPR;
+    constexpr int G = 64 / LPR, CH = LPR * 8, ROWS = G * R;
+    __shared__ float parts[4][ROWS];
+    const int cols0 = a.cols0, cols1 = a.cols1, ld0 = a.ld0, ld1 = a.ld1, ldx1 = a.ldx1, rows = a.rows, c0 = p.c0, ce = p.ce, top = a.top;
+    const unsigned magic = p.magic;
+    const uint16_t *w0 = a.w0, *w1 = a.w1;
+    const float *x0 = a.x0, *x1 = a.x1;
+    // (every argument at once: read where they are used they are a chain of scalar loads)
+    asm volatile("" ::"s"(cols0), "s"(cols1), "s"(ld0), "s"(ld1), "s"(ldx1), "s"(rows), "s"(c0), "s"(ce), "s"(top), "s"(magic), "s"(w0), "s"(w1), "s"(x0), "s"(x1), "s"(a.ids), "s"(a.x0_scale), "s"(a.identity), "s"(a.bias), "s"(a.input), "s"(a.y), "s"(p.groups));
+    int ids = a.ids[min(lane, top - 1)];
+    ids = lane < top ? ids : -1;
+    asm volatile("" : "+v"(ids));
+    const int n_real = __popcll(__ballot(ids >= 0)), end = c0 + n_real * ce;  // (identity experts have no columns)
+    const float through = a.identity ? *a.identity : 0.f, scale0 = a.x0_scale ? *a.x0_scale : 1.0f;
+    const size_t each = (size_t)rows * ld1;
     u32x4 w[U][R];
-    auto fetch = [&](int grp, int chunk0) {
+    f32x4 v[U][2];
+    float in[U];  // zero: past a segment's columns
+    const int row0 = blockIdx.x * ROWS, row = row0 + tid, batches = ((end + 3) / 4 + U - 1) / U;
+    auto fetch = [&](int u, int chunk) {
+        const int c = min(chunk, end - 1), x = max(c - c0, 0), q = min((int)((unsigned)x * magic >> 20), max(n_real - 1, 0)), e = max(__builtin_amdgcn_readlane(ids, q), 0);
+        const bool first = c < c0;
+        const uint16_t *mat = w1 + (size_t)e * each, *base = first ? w0 : mat;
+        const float *vec = x1 + (size_t)q * ldx1, *src = first ? x0 : vec;
+        const int ld = first ? ld0 : ld1, cols = first ? cols0 : cols1, from = c0 + q * ce, at = (c - (first ? 0 : from)) * CH + l * 8;
+        const unsigned col = min(at, cols - 8);
+        in[u] = at < cols && chunk < end ? (first ? scale0 : 1.0f) : 0.f;
+        v[u][0] = *reinterpret_cast<const f32x4 *>(src + col), v[u][1] = *reinterpret_cast<const f32x4 *>(src + col + 4);
+        base += (size_t)row0 * ld;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (LPR == 64) {
+                w[u][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(base + col));
+                if (row0 + r + 1 < rows) base += ld;
+            } else {
+                w[u][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(base + (unsigned)(min(sub * R + r, rows - 1 - row0) * ld) + col));
+            }
+        }
+    };
+    float bias = 0.f, input = 0.f, acc[R];  // (on their way while the products run)
+    if (a.bias) bias = a.bias[min(row, rows - 1)];
+    if (a.identity) input = a.input[min(row, rows - 1)];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+    for (int b = 0; b < batches; ++b) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) fetch(u, wave + 4 * (U * b + u));
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int c = chunk0 + u, x = max(c - p.c0, 0);
-            const int q = min((int)((unsigned)x * p.magic >> 20), max(n_real - 1, 0)), e = max(__builtin_amdgcn_readlane(ids, q), 0);
-            const bool first = c < p.c0;
-            const uint16_t *base = first ? a.w0 : a.w1 + (size_t)e * a.rows * a.ld1;
-            const int ld = first ? a.ld0 : a.ld1, col = min((first ? c : x - q * p.ce) * CH + l * 8, (first ? a.cols0 : a.cols1) - 8);
+            f32x4 x[2];
 #pragma unroll
-            for (int r = 0; r < R; ++r)
-                w[u][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(base + (size_t)min((grp * G + sub) * R + r, a.rows - 1) * ld + col));
+            for (int h = 0; h < 2; ++h) x[h] = in[u] != 0.f ? in[u] * v[u][h] : f32x4{0.f, 0.f, 0.f, 0.f};
+            multiply8<R>(w[u], x[0], x[1], acc);
         }
-    };
-    int g = blockIdx.x * 4 + wave;
-    const int steps = (end + U - 1) / U * U, total = steps * CH / 4;  // (identity experts have no columns)
-    const float through = a.identity ? *a.identity : 0.f, scale0 = a.x0_scale ? *a.x0_scale : 1.0f;
-    constexpr int AH = 12;
-    f32x4 v[AH];
-    float in[AH];  // zero: past a segment's columns
-    auto load = [&](int i0) {
+    }
 #pragma unroll
-        for (int j = 0; j < AH; ++j) {
-            const int i = i0 + 256 * j, c = i / (CH / 4), x = max(c - p.c0, 0), q = min((int)((unsigned)x * p.magic >> 20), max(n_real - 1, 0));
-            const bool first = c < p.c0;
-            const int col = (first ? i : i - (p.c0 + q * p.ce) * (CH / 4)) * 4, cols = first ? a.cols0 : a.cols1;
-            in[j] = col < cols && c < end ? (first ? scale0 : 1.0f) : 0.f;
-            v[j] = *reinterpret_cast<const f32x4 *>((first ? a.x0 : a.x1 + (size_t)q * a.ldx1) + min(col, cols - 4));
-        }
-    };
-    auto store = [&](int i0) {
-#pragma unroll
-        for (int j = 0; j < AH; ++j)
-            if (i0 + 256 * j < total) reinterpret_cast<f32x4 *>(xs)[i0 + 256 * j] = in[j] != 0.f ? in[j] * v[j] : f32x4{0.f, 0.f, 0.f, 0.f};
-    };
-    // (loads return in order: the weights are requested behind the vector, which is stored while they are on their way)
-    load(tid);
-    if (g < p.groups) fetch(g, 0);
-    store(tid);
-    for (int i0 = tid + 256 * AH; i0 < total; i0 += 256 * AH) {
-        load(i0);
-        store(i0);
+    for (int r = 0; r < R; ++r) {
+        const float t = lanes_sum<LPR>(acc[r]);
+        if (l == 0) parts[wave][sub * R + r] = t;
     }
     __syncthreads();
-    const int n_wg = gridDim.x;
-    for (; g < p.groups; g += n_wg * 4) {
-        float acc[R], more[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int row = min((g * G + sub) * R + r, a.rows - 1);
-            acc[r] = 0.f;
-            more[r] = (a.bias ? a.bias[row] : 0.f) + (a.identity ? through * a.input[row] : 0.f);
-        }
-        for (int c0 = 0; c0 < steps; c0 += U) {
-            u32x4 c[U][R];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int r = 0; r < R; ++r) c[u][r] = w[u][r];
-            if (c0 + U < steps)
-                fetch(g, c0 + U);
-            else if (g + n_wg * 4 < p.groups)
-                fetch(g + n_wg * 4, 0);
-#pragma unroll
-            for (int u = 0; u < U; ++u) multiply8<R>(c[u], xs + (c0 + u) * CH + l * 8, acc);
-        }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const float v = lanes_sum<LPR>(acc[r]);
-            const int row = (g * G + sub) * R + r;
-            if (l == 0 && row < a.rows) a.y[row] = v + more[r];
-        }
-    }
+    if (tid < ROWS && row < rows) a.y[row] = ((parts[0][tid] + parts[1][tid]) + (parts[2][tid] + parts[3][tid])) + (bias + through * input);
 }
 
 // workgroups of a product: all of them at once up to three per CU, whole rounds of row groups beyond
@@ -579,27 +569,24 @@ static hipError_t out_go(const ExpertsOut &a, hipStream_t s) {
     k.a = a;
     constexpr int CH = LPR * 8;
     k.c0 = (a.cols0 + CH - 1) / CH, k.ce = (a.cols1 + CH - 1) / CH;
-    const int chunks = k.c0 + a.top * k.ce, u = chunks >= 8 ? 8 : chunks >= 4 ? 4 : 2;
-    k.chunks = (chunks + u - 1) / u * u;
+    const int chunks = k.c0 + a.top * k.ce, each = (chunks + 3) / 4;
     k.magic = ((1u << 20) + k.ce - 1) / k.ce;
     k.groups = (a.rows + 64 / LPR * R - 1) / (64 / LPR * R);
-    const size_t lds = (size_t)k.chunks * CH * 4;
     // (the quotient by multiplication holds while chunks * ce stays below 2^20)
-    if (lds > 150 * 1024 || (long)k.chunks * k.ce >= 1 << 20) return hipErrorInvalidValue;
-    auto fn = u == 2 ? k_experts_out<LPR, R, 2> : u == 4 ? k_experts_out<LPR, R, 4> : k_experts_out<LPR, R, 8>;
-    if (lds > 65536) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(fn, dim3(gemv_grid(k.groups, 1)), dim3(256), lds, s, k);
+    if ((chunks + 7) / 8 * 8 * CH * 4 > 150 * 1024 || (long)(chunks + 7) * k.ce >= 1 << 20) return hipErrorInvalidValue;
+    auto fn = each <= 2 ? k_experts_out<LPR, R, 2> : each <= 3 ? k_experts_out<LPR, R, 3> : each <= 4 || each == 7 || each == 8 ? k_experts_out<LPR, R, 4> : k_experts_out<LPR, R, 6>;
+    hipLaunchKernelGGL(fn, dim3(k.groups), dim3(256), 0, s, k);
     return hipGetLastError();
 }
 
 hipError_t launch_experts_out(const ExpertsOut &a, hipStream_t s) {
     auto waste = [&](int ch) { return (double)((a.cols0 + ch - 1) / ch * ch + (long)a.top * ((a.cols1 + ch - 1) / ch * ch)) / (a.cols0 + (double)a.top * a.cols1); };
     auto fits = [&](int ch) { return ((a.cols0 + ch - 1) / ch + (long)a.top * ((a.cols1 + ch - 1) / ch) + 7) / 8 * 8 * ch * 4 <= 150 * 1024; };
-    // the longest rows of lanes whose chunks are not padding for the most part (lanes past a row's end load its last columns again: no traffic)
-    return waste(512) <= 1.4 * waste(256) && fits(512) ? out_go<64, 1>(a, s) : waste(256) <= 1.3 * waste(128) && fits(256) ? out_go<32, 1>(a, s) : out_go<16, 1>(a, s);
+    // four rows per workgroup from 3072 on, where that is still three workgroups per CU; us per step of Mimolix / Lurepel / Sipelorn with R = 4, 2, 1: 3072 rows 244.3 / 230.0 / 347.0,
+    // 248.2 / 232.0 / 348.2, 259.9 / 234.5 / 351.5; 2560 rows 290.7 / 278.2 / 391.6, 289.5 / 277.5 / 391.0, 297.6 / 280.0 / 394.0; 1536 rows 153.1 / 151.8 / 232.7, 151.5 / 150.1 / 233.0,
+    // 153.7 / 151.2 / 232.2.  The longest rows of lanes whose chunks are not padding for the most part (lanes past a row's end load its last columns again: no traffic)
+    if (waste(512) <= 1.4 * waste(256) && fits(512)) return a.rows >= 3072 ? out_go<64, 4>(a, s) : out_go<64, 2>(a, s);
+    return waste(256) <= 1.3 * waste(128) && fits(256) ? out_go<32, 1>(a, s) : out_go<16, 1>(a, s);
 }
 
 }  // namespace bitnet_hip

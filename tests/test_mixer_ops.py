@@ -726,6 +726,26 @@ def test_experts_of_one_token(hip, pkg, experts, top, width, ff, cols0):
     assert u.rms_error(u.host(y), want) < F32_TOL
 
 
+# the way down: two and four rows per workgroup, rows past the last one; one to six chunks per wave, twice four and more than one batch of six; last chunks partly or wholly past the columns
+@pytest.mark.parametrize("rows", [1, 2051, 3071, 3074])
+@pytest.mark.parametrize("top,colf,cols0", [(1, 8, 8), (3, 1024, 1000), (8, 520, 0), (7, 1024, 1032), (8, 1536, 520), (8, 1544, 1536)])
+def test_way_down_of_one_token(hip, rows, top, colf, cols0):
+    g = rng(rows, top, colf)
+    experts, ld1, ld0 = 9, colf + 64, cols0 + 8
+    down, w0 = u.rounded(g.standard_normal((experts, rows, colf))), u.rounded(g.standard_normal((rows, max(cols0, 8))))
+    x1, x0, y = g.standard_normal((top, colf)).astype(np.float32), g.standard_normal(max(cols0, 8)).astype(np.float32), u.zeros_f32(rows + 4)
+    ids = g.permutation(experts)[:top].astype(np.int32)
+    padded = lambda a, ld: np.concatenate([a, np.full(a.shape[:-1] + (ld - a.shape[-1],), np.nan, np.float32)], -1)  # what lies past the columns is never used
+    for real in (top, top - 1, 0):  # behind them identity experts
+        chosen = np.where(np.arange(top) < real, ids, -1).astype(np.int32)
+        first = (u.dev_f32(x0), u.dev_bf16(padded(w0, ld0))) if cols0 else (None, None)
+        hip.experts_out_dev(*first, cols0, ld0 if cols0 else 0, None, u.dev_f32(padded(x1, ld1)), ld1, u.dev_bf16(padded(down, ld1)), colf, ld1, u.dev(chosen), top, rows, y)
+        want = sum((down[e].astype(np.float64) @ x1[k] for k, e in enumerate(ids[:real])), w0.astype(np.float64) @ x0 if cols0 else np.zeros(rows))
+        got = u.host(y)
+        assert u.rms_error(got[:rows], want) < F32_TOL if np.any(want) else not np.any(got[:rows])
+        assert not np.any(got[rows:])
+
+
 # experts that hand their input through, choice by corrected scores, weights as the scores are, gated pairs
 def corrected(m, experts, identity, top, seed):
     n = experts + identity
