@@ -731,6 +731,13 @@ __device__ __forceinline__ float lanes_total(float v) {
     return LPR == 64 ? rows_sum(v) : v;
 }
 
+struct GemvPlainK {
+    const float *x, *bias;
+    const uint16_t *w;
+    float *y;
+    int rows, cols, ld, act0, act1, act_split;
+};
+
 // MORE: whatever bitnet_hip_epilogue and a gate on the residual ask for
 template <int LPR, int R, int U, bool MORE, int NR>
 __global__ __launch_bounds__(256, MORE && R * U >= 20 ? 2 : 1) void k_dense_gemv(GemvK p) {
@@ -918,6 +925,61 @@ __global__ __launch_bounds__(256, MORE && R * U >= 20 ? 2 : 1) void k_dense_gemv
     }
 }
 
+// A plain vector needs no norm ahead of the products, so it does not go through LDS either: the four waves of a workgroup share its R rows' columns, chunk by chunk of 512, a lane takes the
+// vector's elements at its own columns to registers, and vector, bias and weights are requested at once (U chunks per wave in flight).  Launch and one latency bound it below 1 MB of
+// weights, memory above.  us, k_dense_gemv / this form: 64 x 3072 3.7 / 2.7, 1536 x 1536 4.0 / 3.3, 2560 x 2560 5.4 / 5.2, 3072 x 8192 11.6 / 11.1, 6912 x 2560 9.4 / 8.8,
+// 32768 x 16384 195 / 159; steps: Lasapel 1b 176.6 -> 171.6, 3b 273.6 -> 268.9, Lurepel 1b at 900 keys 162.3 -> 158.3, Sipelorn 1b 242.7 -> 237.
+template <int R, int U>
+__global__ __launch_bounds__(256, 3) void k_dense_gemv_plain(GemvPlainK p) {
+    __shared__ float parts[4][R];
+    asm volatile("" ::"s"(p.x), "s"(p.w), "s"(p.bias), "s"(p.y), "s"(p.rows), "s"(p.cols), "s"(p.ld), "s"(p.act0), "s"(p.act1), "s"(p.act_split));
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row0 = blockIdx.x * R, row = row0 + tid;
+    const int chunks = (p.cols + 511) / 512, batches = ((chunks + 3) / 4 + U - 1) / U;
+    float bias = 0.f, acc[R];
+    if (p.bias) bias = p.bias[min(row, p.rows - 1)];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+    for (int b = 0; b < batches; ++b) {
+        u32x4 w[U][R];
+        f32x4 v[U][2];
+        bool in[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int at = (wave + 4 * (U * b + u)) * 512 + lane * 8;
+            const unsigned col = min(at, p.cols - 8);
+            in[u] = at < p.cols;
+            v[u][0] = *reinterpret_cast<const f32x4 *>(p.x + col), v[u][1] = *reinterpret_cast<const f32x4 *>(p.x + col + 4);
+            const uint16_t *wr = p.w + (size_t)row0 * p.ld;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                w[u][r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(wr + col));
+                if (row0 + r + 1 < p.rows) wr += p.ld;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            f32x4 x[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) x[h] = in[u] ? v[u][h] : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    acc[r] = fmaf(x[c >> 1][2 * c & 3], __builtin_bit_cast(float, w[u][r][c] << 16), acc[r]);
+                    acc[r] = fmaf(x[c >> 1][(2 * c & 3) + 1], __builtin_bit_cast(float, w[u][r][c] & 0xffff0000u), acc[r]);
+                }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const float t = lanes_total<64>(acc[r]);
+        if (lane == 0) parts[wave][r] = t;
+    }
+    __syncthreads();
+    if (tid < R && row < p.rows)
+        p.y[row] = activate(((parts[0][tid] + parts[1][tid]) + (parts[2][tid] + parts[3][tid])) + bias, row < p.act_split ? p.act0 : p.act1);
+}
+
 // LPR lanes per row take rows of up to 64, 256 and any number of columns: one, two and five steps at the most are needed of them
 template <int LPR, int R, bool MORE>
 static void gemv_go(int u, const GemvK &k, dim3 grid, hipStream_t s) {
@@ -947,7 +1009,25 @@ static void gemv_pick_u(int u, const GemvK &k, dim3 grid, hipStream_t s) {
         gemv_go<LPR, R, false>(u, k, grid, s);
 }
 
+// What k_dense_gemv_plain takes: a vector as it lies there, no epilogue beyond bias and activation, rows of more than half a wave.  Many short rows stay with k_dense_gemv, whose
+// workgroups take several groups of them (128256 x 264 / 512 columns: 23 / 26 us against 31 / 33; 16384 x 512: 7.1 / 6.7; 128256 x 1024: 47 / 41).  One, two or four rows per workgroup:
+// us with R = 1, 2, 4 at 512 x 1536 2.8, 2.9, 3.0, 1024 x 4096 4.0, 4.0, 4.0, 2560 x 6912 11.4, 9.0, 9.4, 3072 x 8192 14.3, 11.4, 11.1, 16384 x 4096 27.9, 24.8, 23.4.
+static bool gemv_is_plain(const GemvArgs &a) {
+    return a.in.kind == BITNET_HIP_IN_PLAIN && ((uintptr_t)a.in.x & 15) == 0 && a.batch == 1 && !a.gated && !a.best_val && !a.latent && !a.more.conv && !a.more.mul &&
+           a.cols > 256 && (a.rows <= 16384 || a.cols > 512) && a.more.act2_from >= a.rows && a.act0 != BITNET_HIP_ACT_XIELU && a.act1 != BITNET_HIP_ACT_XIELU;
+}
+
+template <int R>
+static hipError_t gemv_plain_go(const GemvArgs &a, hipStream_t s) {
+    GemvPlainK k{a.in.x, a.bias, a.w, a.y, a.rows, a.cols, a.ld, a.act0, a.act1, a.act_split ? a.act_split : a.rows};
+    const int each = ((a.cols + 511) / 512 + 3) / 4;
+    auto fn = each <= 1 ? k_dense_gemv_plain<R, 1> : each <= 2 ? k_dense_gemv_plain<R, 2> : each <= 3 || each == 5 || each == 6 ? k_dense_gemv_plain<R, 3> : k_dense_gemv_plain<R, 4>;
+    hipLaunchKernelGGL(fn, dim3((a.rows + R - 1) / R), dim3(256), 0, s, k);
+    return hipGetLastError();
+}
+
 hipError_t launch_dense_gemv(const GemvArgs &a, int *n_wg_out, hipStream_t s) {
+    if (gemv_is_plain(a)) return a.rows >= 3072 ? gemv_plain_go<4>(a, s) : a.rows > 512 ? gemv_plain_go<2>(a, s) : gemv_plain_go<1>(a, s);
     GemvK k;
     k.a = a;
     k.a.latent = nullptr;

@@ -18,6 +18,29 @@ def pos_dev(p):
     return u.dev(np.array([p], np.int32))
 
 
+# one, two and four rows per workgroup and rows past the last one; a wave's chunks of 512 columns: one to four, twice three, more than four; what stays with the general form
+@pytest.mark.parametrize("rows", [1, 511, 514, 3071, 3074])
+@pytest.mark.parametrize("cols", [256, 264, 2048, 2056, 4104, 6152, 8200, 12296, 20488])
+@pytest.mark.parametrize("off", [0, 1])
+def test_gemv_of_a_plain_vector(hip, pkg, rows, cols, off):
+    if off and cols > 4104:
+        pytest.skip("one length of a vector off sixteen bytes is enough")
+    g = rng(rows, cols)
+    ld = cols + 8
+    w, x, bias = u.rounded(g.standard_normal((rows, cols)) / np.sqrt(cols)), g.standard_normal(cols).astype(np.float32), g.standard_normal(rows).astype(np.float32)
+    wd = u.dev_bf16(np.concatenate([w, np.full((rows, 8), np.nan, np.float32)], 1))  # what lies past the columns is never used
+    xd, y = u.dev_f32(np.concatenate([np.full(off, np.nan, np.float32), x, np.full(8, np.nan, np.float32)]))[off:], u.zeros_f32(rows + 4)
+    split = rows // 3
+    hip.dense_gemv_dev(xd, wd, rows, cols, ld, y, bias=u.dev_f32(bias), act0=pkg.ACT_RELU2, act1=pkg.ACT_NONE, act_split=split, n=cols)
+    z, got = w.astype(np.float64) @ x + bias, u.host(y)
+    want = np.where(np.arange(rows) < (split or rows), so.relu_squared(z), z)
+    # the f32 sums of one row: nothing else to average their rounding over
+    assert u.rms_error(got[:rows], want) < (F32_TOL if rows > 1 else 1e-5) if np.any(want) else not np.any(got[:rows])
+    assert not np.any(got[rows:])
+    hip.dense_gemv_dev(xd, wd, rows, cols, ld, y, n=cols)
+    assert u.rms_error(u.host(y)[:rows], z - bias) < (F32_TOL if rows > 1 else 1e-5)
+
+
 # ---- rows and vectors of a block ---------------------------------------------------------------------------------------
 @pytest.mark.parametrize("n", [80, 90, 1001, 2560, 4096, 5000])
 def test_gemv_layer_norm_of_a_plain_residual(hip, pkg, n):
