@@ -750,7 +750,8 @@ hipError_t launch_gqa_merge(const Gqa &g, const int *pos, int q0, int nq, const 
 // The merge of up to four records and the product behind it in one launch: every workgroup forms the whole output in LDS, as k_dense_gemv forms its input, and its waves take rows of the
 // product.  Nothing that is requested hangs on the position: a thread asks for all NB records of its columns, with their maxima and sums, and makes their weights itself; what the position
 // says only masks them.  The product's weights go out behind.  us per layer with this launch against the merge's and the product's, steps of the layer stacks: 1536 columns of 12 heads
-// -3.0 (up to 256 keys) and -2.2 (512), 2560 of 20 -1.9 and -0.9, 3072 of 24 -2.2 and -1.5; with half waves that reduce up to 32 records over LDS, 1024 keys are even and 2000 lose 1.5 to 6.
+// -3.0 (up to 256 keys) and -2.2 (512), 2560 of 20 -1.9 and -0.9, 3072 of 24 -2.2 and -1.5; with half waves that reduce up to 32 records over LDS, 1024 keys are even and 2000 lose 1.5 to 6.  (Against k_dense_gemv's product;
+// k_dense_gemv_plain's is 0.7, 0.2 and 0.2 faster at these three widths, which leaves -2.3 / -1.5, -1.7 / -0.7 and -2.0 / -1.3.)
 struct GqaOutK {
     Gqa g;
     const int *pos;
