@@ -1292,6 +1292,13 @@ __device__ __forceinline__ void f16_chain_epilogue(const GemmArgs &p, gv4f (&acc
             *reinterpret_cast<float2 *>(p.stats_out + 2 * ((size_t)(bx * (NW / 2) + pair) * p.stats_stride + (by * TTW + tt) * 16 + (i & 15))) = float2{a.x + b.x, a.y + b.y};
         }
     }
+    if (TTW < 4 && p.stats_out && !p.silu_mul && by == (int)gridDim.y - 1) {  // no workgroup has the token tiles behind the last token's: their partials are zero
+        constexpr int slabs = NW * RT / 4;
+        for (int i = tid; i < slabs * 64; i += NW * 64) {
+            const int token = (by + 1) * WG_TOK + (i & 63);
+            if (token < p.stats_stride) *reinterpret_cast<float2 *>(p.stats_out + 2 * ((size_t)(bx * slabs + (i >> 6)) * p.stats_stride + token)) = float2{0.f, 0.f};
+        }
+    }
     gflush_sat(sat);
 }
 
@@ -1471,13 +1478,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_f16a(GemmArgs p, uint32_t lut_h
         return;
     }
     f16_chain_epilogue<RT, TTW, 4, EPI == 2>(p, acc, lds, mu_rs, bx, by, rw, c, g, tid);
-    if (TTW < 4 && p.stats_out && !p.silu_mul && by == (int)gridDim.y - 1) {  // no workgroup has the token tiles behind the last token's: their partials are zero
-        const int slabs = RT == 2 ? 2 : 4;
-        for (int i = tid; i < slabs * 64; i += 256) {
-            const int token = (by + 1) * WG_TOK + (i & 63);
-            if (token < p.stats_stride) *reinterpret_cast<float2 *>(p.stats_out + 2 * ((size_t)(bx * slabs + (i >> 6)) * p.stats_stride + token)) = float2{0.f, 0.f};
-        }
-    }
 }
 
 // ---- few activation rows on the chain -----------------------------------------------------------------------------------------------------------------------

@@ -106,6 +106,23 @@ def test_matmul_qb32_is_the_product_of_the_decoded_rows(hip, oracle, torch_, row
     hip.weights_free(h)
 
 
+@pytest.mark.parametrize("rows,cols,m,tokens", [(512, 512, 65, 16), (512, 256, 80, 16), (13824, 256, 257, 32), (13824, 256, 700, 64)])
+def test_matmul_qb32_leaves_partials_of_every_row(hip, torch_, rows, cols, m, tokens):
+    """tiles of 16, 32 and 64 tokens that end ahead of, and at, the padding to 64: the partials of the live tokens are their outputs' sums, those of the padding zero"""
+    rng, mp = np.random.default_rng(rows + m), -(-m // 64) * 64
+    h = hip.weights_upload_qk256(rng.integers(0, 256, rows * cols // 4, dtype=np.uint8), rows, cols, cols // 4)
+    qb = torch_.zeros(hip.qb32_bytes(m, cols), dtype=torch_.uint8, device="cuda")
+    hip.rows_to_qb32_dev(torch_.from_numpy(rng.normal(0.1, 1.0, (m, cols)).astype(np.float32)).cuda(), None, m, cols, qb, None)
+    y, st = torch_.full((m, rows), float("nan"), device="cuda"), torch_.full((rows // 64, mp, 2), float("nan"), device="cuda")
+    hip.matmul_qb32_dev(h, qb, m, y=y, stats_out=st)
+    assert hip.matmul_last_tile()["wave_tokens"] == tokens
+    slabs, s = y.cpu().numpy().astype(np.float64).reshape(m, rows // 64, 64), st.cpu().numpy()
+    for e in (1, 2):  # f32 sums of 64 terms: 2^-24 per addition against the magnitudes
+        assert np.all(np.abs(s[:, :m, e - 1].T - (slabs ** e).sum(axis=2)) <= 4e-6 * (np.abs(slabs) ** e).sum(axis=2) + 1e-6)
+    assert np.all(s[:, m:] == 0)
+    hip.weights_free(h)
+
+
 def test_matmul_qb32_silu_pair_writes_f16_rows(hip, oracle, torch_):
     rng = np.random.default_rng(12)
     K, F, m = 1024, 768, 130
