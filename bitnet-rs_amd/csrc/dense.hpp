@@ -266,6 +266,12 @@ __device__ __forceinline__ float ld_act(const uint16_t *p, size_t i) { return bf
 __device__ __forceinline__ void st_act(float *p, size_t i, float v) { p[i] = v; }
 __device__ __forceinline__ void st_act(uint16_t *p, size_t i, float v) { p[i] = f2bf(v); }
 
+// the `bytes` from base on (the same in all lanes), read by raw buffer loads: a load past their end takes no memory traffic and gives zero
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t bounded(const void *base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, bytes, 0x00020000);  // (word 3 of gfx94x / gfx950: dwords)
+}
+constexpr int kBufferNt = 2;  // a buffer load's nontemporal bit
+
 template <int CTRL>
 __device__ __forceinline__ float dpp(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));

@@ -41,6 +41,19 @@ def test_gemv_of_a_plain_vector(hip, pkg, rows, cols, off):
     assert u.rms_error(u.host(y)[:rows], z - bias) < (F32_TOL if rows > 1 else 1e-5)
 
 
+# a wave's chunks that lie partly and wholly past the columns, and none that does
+@pytest.mark.parametrize("rows,cols", [(5, 3072), (600, 1536), (3073, 2560), (9, 2048), (7, 520), (513, 6152)])
+def test_gemv_of_a_plain_vector_with_infinite_weights(hip, rows, cols):
+    """an infinite weight among a row's last ones makes that row infinite, with its column's sign, and no other: nothing past the columns is multiplied"""
+    g = rng(rows, cols)
+    w, x, y = u.rounded(g.standard_normal((rows, cols)) / np.sqrt(cols)), g.standard_normal(cols).astype(np.float32), u.zeros_f32(rows)
+    for k, row in enumerate(range(0, rows, max(rows // 8, 1))):
+        w[row, cols - 1 - k % 8] = np.inf
+    hip.dense_gemv_dev(u.dev_f32(x), u.dev_bf16(w), rows, cols, cols, y, n=cols)
+    want, got = w.astype(np.float64) @ x, u.host(y)
+    assert not np.any(np.isnan(got)) and np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
+
+
 # ---- rows and vectors of a block ---------------------------------------------------------------------------------------
 @pytest.mark.parametrize("n", [80, 90, 1001, 2560, 4096, 5000])
 def test_gemv_layer_norm_of_a_plain_residual(hip, pkg, n):
