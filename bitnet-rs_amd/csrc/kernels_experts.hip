@@ -473,7 +473,8 @@ __global__ __launch_bounds__(256, 3) void k_experts_out(OutK p) {
     const size_t each = (size_t)rows * ld1;
     u32x4 w[U][R];
     f32x4 v[U][2];
-    float in[U];  // zero: past a segment's columns
+    float scale[U];
+    bool in[U];  // a lane has columns of its own
     const int row0 = blockIdx.x * ROWS, row = row0 + tid, batches = ((end + 3) / 4 + U - 1) / U;
     auto fetch = [&](int u, int chunk) {
         const int c = min(chunk, end - 1), x = max(c - c0, 0), q = min((int)((unsigned)x * magic >> 20), max(n_real - 1, 0)), e = max(__builtin_amdgcn_readlane(ids, q), 0);
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(256, 3) void k_experts_out(OutK p) {
         const float *vec = x1 + (size_t)q * ldx1, *src = first ? x0 : vec;
         const int ld = first ? ld0 : ld1, cols = first ? cols0 : cols1, from = c0 + q * ce, at = (c - (first ? 0 : from)) * CH + l * 8;
         const unsigned col = min(at, cols - 8);
-        in[u] = at < cols && chunk < end ? (first ? scale0 : 1.0f) : 0.f;
+        in[u] = at < cols && chunk < end, scale[u] = first ? scale0 : 1.0f;
         v[u][0] = *reinterpret_cast<const f32x4 *>(src + col), v[u][1] = *reinterpret_cast<const f32x4 *>(src + col + 4);
         base += (size_t)row0 * ld;
 #pragma unroll
@@ -507,8 +508,16 @@ __global__ __launch_bounds__(256, 3) void k_experts_out(OutK p) {
         for (int u = 0; u < U; ++u) {
             f32x4 x[2];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) x[h] = in[u] != 0.f ? in[u] * v[u][h] : f32x4{0.f, 0.f, 0.f, 0.f};
-            multiply8<R>(w[u], x[0], x[1], acc);
+            for (int h = 0; h < 2; ++h) x[h] = scale[u] != 0.f ? scale[u] * v[u][h] : f32x4{0.f, 0.f, 0.f, 0.f};
+            float t[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) t[r] = acc[r];
+            multiply8<R>(w[u], x[0], x[1], t);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                asm volatile("" : "+v"(t[r]));  // (a choice, not a branch, which would take the loads along)
+                acc[r] = in[u] ? t[r] : acc[r];  // (else it has a segment's last ones again, which may be infinite)
+            }
         }
     }
 #pragma unroll

@@ -782,6 +782,26 @@ def test_way_down_of_one_token(hip, rows, top, colf, cols0):
         assert not np.any(got[rows:])
 
 
+# 64 lanes per row with chunks that lie partly and wholly past the columns, 32 and 16 lanes
+@pytest.mark.parametrize("rows,top,colf,cols0", [(9, 3, 512, 0), (3073, 5, 1024, 1024), (70, 1, 520, 1536), (33, 8, 200, 256), (17, 2, 72, 136)])
+def test_way_down_of_one_token_with_infinite_weights(hip, rows, top, colf, cols0):
+    """an infinite weight among a row's last ones, of the first segment or of an expert, makes that row infinite, with its column's sign, and no other"""
+    g = rng(rows, top, colf)
+    experts = top + 2
+    down, w0 = u.rounded(g.standard_normal((experts, rows, colf))), u.rounded(g.standard_normal((rows, max(cols0, 8))))
+    x1, x0, y = g.standard_normal((top, colf)).astype(np.float32), g.standard_normal(max(cols0, 8)).astype(np.float32), u.zeros_f32(rows)
+    ids = g.permutation(experts)[:top].astype(np.int32)
+    for k, row in enumerate(range(0, rows, max(rows // 8, 1))):
+        if cols0 and k % 2:
+            w0[row, cols0 - 1 - k % 8] = np.inf
+        else:
+            down[ids[k % top], row, colf - 1 - k % 8] = np.inf
+    first = (u.dev_f32(x0), u.dev_bf16(w0)) if cols0 else (None, None)
+    hip.experts_out_dev(*first, cols0, cols0, None, u.dev_f32(x1), colf, u.dev_bf16(down), colf, colf, u.dev(ids), top, rows, y)
+    want, got = sum((down[e].astype(np.float64) @ x1[k] for k, e in enumerate(ids)), w0.astype(np.float64) @ x0 if cols0 else np.zeros(rows)), u.host(y)
+    assert not np.any(np.isnan(got)) and np.array_equal(np.isinf(got), np.isinf(want)) and np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
+
+
 # experts that hand their input through, choice by corrected scores, weights as the scores are, gated pairs
 def corrected(m, experts, identity, top, seed):
     n = experts + identity
