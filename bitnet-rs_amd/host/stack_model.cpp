@@ -278,10 +278,16 @@ int StackModel::upload(T **dst, const std::vector<T> &src) {
 int StackModel::upload_matrix(Matrix &m, const std::vector<uint16_t> &rows, int n_rows, int cols) {
     m.rows = n_rows, m.cols = (int)up_to(cols, 8), m.ld = (int)up_to(cols, 64);
     void *p = nullptr;
-    HCHK(hipMalloc(&p, (size_t)n_rows * m.ld * 2));
+    const size_t bytes = (size_t)n_rows * m.ld * 2;
+    HCHK(hipMalloc(&p, bytes));
     owned_.push_back(p);
-    HCHK(hipMemset(p, 0, (size_t)n_rows * m.ld * 2));
-    HCHK(hipMemcpy2D(p, (size_t)m.ld * 2, rows.data(), (size_t)cols * 2, (size_t)cols * 2, n_rows, hipMemcpyHostToDevice));
+    // (padded on the host, one copy: a hipMemset ahead of a hipMemcpy2D has been seen to land behind it, under rocprofv3's kernel trace, and every later model's weights were zero)
+    std::vector<uint16_t> padded;
+    if (m.ld != cols) {
+        padded.resize((size_t)n_rows * m.ld);
+        for (int r = 0; r < n_rows; ++r) memcpy(&padded[(size_t)r * m.ld], &rows[(size_t)r * cols], (size_t)cols * 2);
+    }
+    HCHK(hipMemcpy(p, m.ld != cols ? padded.data() : rows.data(), bytes, hipMemcpyHostToDevice));
     m.w = static_cast<uint16_t *>(p);
     weight_bytes_ += (size_t)n_rows * cols * 2;
     return 0;

@@ -1,5 +1,6 @@
 // A HIP runtime of promises for the host code (tests/test_host_order.py): work is done as late as HIP allows it -- a stream's when somebody waits for that stream, the null stream's when a
-// blocking copy follows it -- so that whatever relies on an order that nothing establishes is seen.  The kernels are stand-ins that leave a mark.
+// blocking copy follows it -- so that whatever relies on an order that nothing establishes is seen.  The kernels are stand-ins that leave a mark.  A blocking copy of rows (hipMemcpy2D)
+// does not wait for the null stream's fills here, although it should: under rocprofv3's kernel trace the runtime's has overtaken a hipMemset of the same memory.
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -8,6 +9,7 @@
 #include <vector>
 
 #include "decoder.hpp"
+#include "stack_model.hpp"
 
 namespace {
 typedef std::deque<std::function<void()>> Queue;
@@ -25,6 +27,7 @@ void run_all() {
     run(g_null);
     for (Queue *q : g_streams) run(*q);
 }
+std::vector<std::pair<const uint8_t *, size_t>> g_memory;
 uint32_t g_clamped = 0, g_taken = 0;  // the device's count, and what of it f16_saturations_dev has given out
 int g_clamping = 0;                   // the next product clamps, and somebody else takes the count at once
 uint32_t take() {
@@ -40,9 +43,17 @@ void product(void *s) {
 }  // namespace
 
 extern "C" {
-hipError_t hipMalloc(void **p, size_t n) { return *p = malloc(n + 64), memset(*p, 0x5a, n + 64), hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) {
+    *p = malloc(n + 64), memset(*p, 0x5a, n + 64);
+    return g_memory.push_back({(const uint8_t *)*p, n}), hipSuccess;
+}
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipFree(void *p) { return run_all(), free(p), hipSuccess; }
+hipError_t hipFree(void *p) {
+    run_all();
+    for (auto &m : g_memory)
+        if (m.first == p) m = {nullptr, 0};
+    return free(p), hipSuccess;
+}
 hipError_t hipHostFree(void *p) { return hipFree(p); }
 hipError_t hipDeviceSynchronize() { return run_all(), hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
@@ -53,6 +64,10 @@ hipError_t hipStreamSynchronize(hipStream_t s) { return run(queue(s)), hipSucces
 hipError_t hipMemset(void *p, int v, size_t n) { return g_null.push_back([=] { memset(p, v, n); }), hipSuccess; }
 hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t s) { return queue(s).push_back([=] { memset(p, v, n); }), hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return run(g_null), memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpy2D(void *d, size_t ldd, const void *s, size_t lds, size_t n, size_t rows, hipMemcpyKind) {
+    for (size_t r = 0; r < rows; ++r) memcpy((char *)d + r * ldd, (const char *)s + r * lds, n);
+    return hipSuccess;
+}
 
 size_t bitnet_hip_qact_bytes(size_t) { return 64; }
 size_t bitnet_hip_qact_stats_bytes(size_t) { return 64; }
@@ -106,7 +121,37 @@ using bitnet_host::Decoder;
 #define CHECK(x) \
     if (!(x)) return printf("%s:%d: %s\n", __FILE__, __LINE__, #x), 1
 
+// a matrix of 6 rows lies on the device, with zeros behind its columns
+bool arrived(const std::vector<uint16_t> &w, size_t cols, size_t ld) {
+    std::vector<uint16_t> want(6 * ld, 0);
+    for (size_t r = 0; r < 6; ++r) memcpy(&want[r * ld], &w[r * cols], cols * 2);
+    for (const auto &m : g_memory)
+        if (m.second == 6 * ld * 2 && !memcmp(m.first, want.data(), m.second)) return true;
+    return false;
+}
+
+int matrices() {
+    for (int width : {40, 64, 200}) {
+        bitnet_host::StackSpec spec;
+        spec.width = width, spec.vocab = 6, spec.layers.resize(1);
+        auto &layer = spec.layers[0];
+        layer.mixer = bitnet_host::LayerSpec::Linear;
+        layer.linear.heads = 1, layer.linear.dim = layer.linear.vdim = 6, layer.linear.decay = {0.5};
+        bitnet_host::StackModel m(spec, false, 16);
+        CHECK(!m.dead());
+        std::vector<uint16_t> w(6 * width), head(6 * width);
+        for (size_t i = 0; i < w.size(); ++i) w[i] = (uint16_t)(i + 1), head[i] = (uint16_t)(i + 2000);
+        bitnet_host::StackGlobalWeights g;
+        g.embed = w.data(), g.head = head.data(), g.final_norm.resize(width);
+        CHECK(m.set_globals(g) == 0);
+        hipDeviceSynchronize();
+        CHECK(arrived(w, width, (width + 63) / 64 * 64) && arrived(head, width, (width + 63) / 64 * 64));
+    }
+    return 0;
+}
+
 int main(int argc, char **argv) {
+    if (argc > 1 && !strcmp(argv[1], "matrices")) return matrices();
     bitnet_host::Config c;
     c.hidden = 512, c.n_layers = 2, c.n_heads = 4, c.n_kv_heads = 1, c.head_dim = 128, c.ffn = 512, c.vocab = 64, c.max_pos = 128, c.eps = 1e-5f, c.rope_theta = 1e4f;
     std::vector<uint8_t> zeros(1 << 20);

@@ -15,10 +15,10 @@ def program(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.exists(RUNTIME_HEADER):
         pytest.skip("needs g++ and the runtime's headers")
     d = tmp_path_factory.mktemp("host_order")
-    objs = [str(d / name) for name in ("decoder.o", "sequence.o", "host_order.o")]
+    objs = [str(d / name) for name in ("decoder.o", "sequence.o", "stack_model.o", "host_order.o")]
     flags = ["-O1", "-g", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-Wno-unused-result", "-Wno-int-in-bool-context", f"-I{HOST}", f"-I{ROOT}/include", "-I/opt/rocm/include"]
     jobs = [subprocess.Popen(["g++", *flags, "-c", src, "-o", obj])
-            for src, obj in zip([f"{HOST}/decoder.cpp", f"{HOST}/sequence.cpp", f"{ROOT}/tests/host_order.cpp"], objs)]
+            for src, obj in zip([f"{HOST}/decoder.cpp", f"{HOST}/sequence.cpp", f"{HOST}/stack_model.cpp", f"{ROOT}/tests/host_order.cpp"], objs)]
     assert all([j.wait() == 0 for j in jobs])
     # whatever else the sources call succeeds and does nothing
     names = [set(), set()]
@@ -31,7 +31,7 @@ def program(tmp_path_factory):
     return str(d / "host_order")
 
 
-@pytest.mark.parametrize("case", ["cache_type", "objects", "clamps"])
+@pytest.mark.parametrize("case", ["cache_type", "objects", "clamps", "matrices"])
 def test_nothing_relies_on_an_order_that_is_not_there(program, case):
     out = subprocess.run([program, case], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
