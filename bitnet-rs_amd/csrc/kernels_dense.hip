@@ -1340,17 +1340,31 @@ static hipError_t grouped_go(const GemmArgsD &a, hipStream_t s) {
     hipLaunchKernelGGL(fn, dim3((tn * a.max_tiles + 7) / 8 * 8), dim3(64 * WN * WM), lds, s, a, tn, 0, 0);
     return hipGetLastError();
 }
-// Experts' products, weights from HBM, us at 64 experts, n x k and rows per expert (64 x 64 in three buffers / 128 x 64 / 128 x 128 in four waves / in eight): 896 x 3072, 3 rows 67 / 62 /
-// 63 / 65, 50 78 / 70 / 72 / 74, 88 104 / 105 / 78 / 81, 125 131 / 113 / 123 / 110, 188 163 / 137 / 116 / 127; 3072 x 896, 3 61 / 60 / 63 / 71, 50 82 / 73 / 81 / 87, 88 107 / 95 / 89 /
-// 94; 448 x 1536, 3 18 / 25 / 26 / 20, 50 22 / 29 / 28 / 23, 88 31 / 28 / 29 / 25; 1360 x 3072 gated, 12 99 / 96 / 117 / 99, 88 160 / 139 / 132 / 117, 188 254 / 203 / 163 / 188.
-// Tiles of 64 rows: 128 columns while they reach every CU (a workgroup's activations serve twice the columns), else 64 in three buffers, of which a CU takes three (in four, two: 20 / 18).
-// Tiles of 128 rows: eight waves with four buffers for long K while an expert has one tile, and there is one round and a half of workgroups; else two workgroups per CU, which overlap
-// their ends.
+// Experts' products.  wide: the workgroups of one row tile per expert, which is what decides; measured over 46 shapes (4 to 256 experts, 128 to 6400 columns of 128 to 5632, also in pairs) at
+// 2 to 400 rows per expert, us with 64 x 64 in four buffers / in three / 128 x 64 / 128 x 128 in four waves / in eight:
+//   64 x 64, four buffers: what the others do not take.  8 experts, 1024 x 4096, 16 rows 21 / 28 / 53; 128, 768 x 2048, 32 rows 79 / 81 / 89
+//   128 x 64 (activations serve twice the columns): where nearly every CU gets two, from as many rows on as K is long.  64, 896 x 3072, 44 rows 74 / 75 / 70; 64, 1024 x 1024, 16 rows
+//     31 / 30 / 27; 64, 1536 x 448, 8 rows 21 / 20 / 19.  Not with rows of whole 4 KiB, whose beginnings meet on the same channels: 256, 512 x 2048, 44 rows 114 / 117 / 136
+//   64 x 64, three buffers, of which a CU takes three: one to two workgroups per CU.  8, 4096 x 1024, 16 rows 17 / 15 / 19; not with such rows either
+//   128 x 128 in eight waves: one round of workgroups (64, 448 x 1536, 72 rows 31 / 31 / 28 / 29 / 23), or two to three of them for long K while an expert has one tile (64, 1408 x 2048,
+//     88 rows 108 / 109 / 96 / 99 / 91)
+//   128 x 128 in four waves, two workgroups per CU, which overlap their ends: 64, 896 x 3072, 88 rows 107 / 107 / 106 / 79 / 82
+// In the mean 3 % behind the best form; against 64 x 64 in four buffers below 96 rows per expert and 128 x 128 in four waves from there on 5.6 % ahead, nowhere more than 6 % behind.
 static hipError_t launch_grouped(const GemmArgsD &a, hipStream_t s) {
     const int experts = a.max_tiles - a.m / a.tile;  // (how a plan counts its tiles)
-    if (a.tile == 64) return (long)experts * ((a.n + 127) / 128) >= 384 ? grouped_go<128, 64, 2, 2, 2>(a, s) : grouped_go<64, 64, 2, 2, 3>(a, s);
+    const long tn = (a.n + 127) / 128, wide = experts * tn;
+    if (a.tile == 64) {
+        const bool spread = a.k % 2048 != 0;
+        const long rows_from = a.k <= 512 ? 0 : a.k <= 1024 ? 6 : 40;
+        if (wide >= 448 && (spread || a.k <= 1024) && a.m >= rows_from * experts) return grouped_go<128, 64, 2, 2, 2>(a, s);
+        const long all = (long)experts * ((a.n + 63) / 64);
+        return all > 256 && all <= 512 && spread ? grouped_go<64, 64, 2, 2, 3>(a, s) : grouped_go<64, 64, 2, 2, 4>(a, s);
+    }
     if (a.tile != 128) return hipErrorInvalidValue;
-    return a.k >= 1536 && a.m <= 112l * experts ? grouped_go<128, 128, 2, 4, 4>(a, s) : grouped_go<128, 128, 2, 2, 2>(a, s);
+    // (above 104 rows per expert some have a second tile)
+    const long likely = wide + (a.m > 104l * experts ? wide / 14 : 0);
+    const bool eight = a.max_tiles * tn <= 256 || (a.m <= 112l * experts && (likely <= 256 || (likely > 512 && likely <= 768 && a.k >= 1536)));
+    return eight ? grouped_go<128, 128, 2, 4, 4>(a, s) : grouped_go<128, 128, 2, 2, 2>(a, s);
 }
 
 template <int TN, int TM, int WN, int WM, int ST, bool MUL = false>

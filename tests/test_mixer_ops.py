@@ -734,9 +734,10 @@ def test_experts_of_a_portion(hip, pkg, m, experts, top, tile, width, ff, f32):
     assert u.rms_error(got, want) < (F32_TOL if f32 else 8e-3)
 
 
-# the forms of the grouped products: 128 columns by 64 rows where that reaches every CU, eight waves for long K and one tile per expert; last columns and rows inside a tile
-@pytest.mark.parametrize("m,experts,top,tile,width,ff,form", [(130, 200, 2, 64, 250, 72, (128, 64, 4, 1)), (90, 40, 3, 64, 250, 72, (64, 64, 4, 1)), (90, 40, 3, 128, 112, 1600, (128, 128, 8, 1)),
-                                                             (150, 5, 4, 128, 112, 1600, (128, 128, 4, 1))])
+# the forms of the grouped products: 128 columns by 64 rows where that gives nearly every CU two workgroups; 64 by 64 in four buffers and, from one workgroup per CU on, in three; 128 by 128 in
+# eight waves where there is one round of them or, for long K, two to three, else in four; last columns and rows inside a tile
+@pytest.mark.parametrize("m,experts,top,tile,width,ff,form", [(130, 230, 2, 64, 250, 72, (128, 64, 4, 1)), (90, 40, 3, 64, 250, 72, (64, 64, 4, 1)), (90, 80, 3, 64, 250, 72, (64, 64, 4, 1)),
+                                                             (90, 40, 3, 128, 112, 1600, (128, 128, 8, 1)), (150, 513, 4, 128, 8, 1600, (128, 128, 8, 1)), (150, 260, 4, 128, 112, 72, (128, 128, 4, 1))])
 def test_forms_of_the_experts_products(hip, pkg, m, experts, top, tile, width, ff, form):
     test_experts_of_a_portion(hip, pkg, m, experts, top, tile, width, ff, False)
     assert tuple(hip.dense_matmul_last_tile()) == form
