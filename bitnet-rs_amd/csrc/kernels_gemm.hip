@@ -2236,18 +2236,25 @@ struct TileCost {
     int rt, ttw;
     double once, end, residual, chain, share, pair;
 };
+static double tile_us(const TileCost &c, size_t rows, size_t blocks, size_t m, bool residual) {
+    const size_t most = div_ceil(div_ceil(rows, 64 * (size_t)c.rt) * div_ceil(m, 16 * (size_t)c.ttw), kGemmCUs);
+    const double block = c.pair > 0 ? (double)(most / 2) * c.pair + (most % 2 ? (most > 1 ? c.share : c.chain) : 0.0) : std::max(c.chain, c.share * (double)most);
+    return c.once + (c.end + (residual ? c.residual : 0.0)) * (double)most + (double)blocks * block;
+}
+// The shortest launch of `costs`, which were measured on the resident image.  Without it a workgroup expands its codes itself, and a narrower tile does so for fewer tokens: there one
+// narrower than `covering`, the choice by covering the CUs (of as many rows: the statistics' slabs follow from these), has to be ahead by a tenth (of 40 launches that are, by less, all took longer than with the covering tile: 13824 x 2560,
+// 1025 tokens, 78 us and 83; 1024 x 1024, 2300 tokens, 11.8 and 13.3; the 54 further ahead up to 2 % longer but one of 5 %, in the mean 9 % less).
 template <size_t N>
-static const TileCost *cheapest_tile(const TileCost (&costs)[N], size_t rows, size_t blocks, size_t m, bool residual, bool five) {
-    const TileCost *best = nullptr;
+static const TileCost *cheapest_tile(const TileCost (&costs)[N], size_t rows, size_t blocks, size_t m, bool residual, bool five, bool image, int covering_rt, int covering_ttw) {
+    const TileCost *best = nullptr, *covering = nullptr;
     double least = 0.0;
     for (const TileCost &c : costs) {
+        if (c.rt == covering_rt && c.ttw == covering_ttw) covering = &c;
         if (c.rt == 5 && !five) continue;
-        const size_t most = div_ceil(div_ceil(rows, 64 * (size_t)c.rt) * div_ceil(m, 16 * (size_t)c.ttw), kGemmCUs);
-        const double block = c.pair > 0 ? (double)(most / 2) * c.pair + (most % 2 ? (most > 1 ? c.share : c.chain) : 0.0) : std::max(c.chain, c.share * (double)most);
-        const double us = c.once + (c.end + (residual ? c.residual : 0.0)) * (double)most + (double)blocks * block;
+        const double us = tile_us(c, rows, blocks, m, residual);
         if (!best || us < least) best = &c, least = us;
     }
-    return best;
+    return !image && covering && best->rt == covering->rt && best->ttw < covering->ttw && least > 0.9 * tile_us(*covering, rows, blocks, m, residual) ? covering : best;
 }
 // Weight-stationary walk of a launch (EXPERIMENTS 4.6).  In the plain order an XCD takes a band of token tiles and walks ALL row blocks for each: the
 // activation tile stays in its L2, the whole weight matrix streams through once per token tile (gate|up: 8.85 MB x 64 tiles = 566 MB of L2 misses
@@ -2629,7 +2636,7 @@ static hipError_t launch_gemm_fp6(const Weights &w, QuantArgs q, const GemmArgs 
     // padding's tiles, and with this one: q|k|v at 850 to 1000 tokens 24.3 to 25.8 -> 19.3 to 20.7, 1800 38.6 -> 33.8; gate|up at 256 24.7 -> 20.1, 400 39.1 -> 28.1, 576 39.4 -> 35.5.
     if (q.kp >= 1024 && !cover_asked) {
         static const TileCost costs[] = {{4, 1, 2.5, 0.2, 0.0, 0.95, 0.55, 0}, {4, 2, 3.0, 0.0, 0.0, 1.35, 0.80, 0}, {4, 4, 4.5, 0.0, 0.0, 1.80, 1.65, 2.85}, {5, 4, 4.5, 0.0, 0.0, 2.30, 2.30, 3.60}};
-        const TileCost *c = cheapest_tile(costs, w.rows, (size_t)q.kp / 256, (size_t)q.m, a.residual != nullptr, !a.silu_mul && w.rows % 320 == 0);
+        const TileCost *c = cheapest_tile(costs, w.rows, (size_t)q.kp / 256, (size_t)q.m, a.residual != nullptr, !a.silu_mul && w.rows % 320 == 0, a.tiles4 != nullptr, rt5 ? 5 : 4, ttw);
         ttw = c->ttw, rt5 = c->rt == 5;
     }
     if (rt5) gx0 = w.rows / 320;
@@ -2731,12 +2738,12 @@ static F16Tile f16_covering_tile(const Weights &w, bool silu_mul, size_t m_pad) 
     if (ttw == 4 && !silu_mul && gemm_five_tiles(w.rows, m_pad)) return {5, 4};
     return {ttw < 4 && w.rows / 256 * (m_pad / (16 * ttw)) <= 320 ? 2 : 4, ttw};
 }
-static F16Tile f16_tile(const Weights &w, bool silu_mul, bool residual, size_t m) {
+static F16Tile f16_tile(const Weights &w, bool silu_mul, bool residual, size_t m, bool image, F16Tile covering) {
     static const TileCost costs[2][5] = {{{2, 1, 4.0, 0.2, 0.0, 0.73, 0.32, 0}, {2, 2, 5.0, 0.4, 0.3, 0.98, 0.475, 0}, {4, 2, 5.3, 0.6, 0.7, 1.12, 0.765, 0},
                                           {4, 4, 6.0, 1.8, 1.5, 1.78, 1.54, 2.76}, {5, 4, 10.0, 1.4, 1.3, 2.04, 1.8, 3.30}},
                                          {{2, 1, 6.0, 0.2, 0.1, 0.80, 0.405, 0}, {2, 2, 5.5, 0.5, 0.5, 1.09, 0.555, 0}, {4, 2, 6.5, 1.0, 1.1, 1.34, 0.96, 0},
                                           {4, 4, 7.0, 2.7, 3.3, 2.04, 1.82, 3.03}, {5, 4, 11.0, 2.7, 2.8, 2.42, 2.3, 3.70}}};
-    const TileCost *c = cheapest_tile(costs[w.scaled ? 1 : 0], w.rows, w.cols / 256, m, residual, !silu_mul && w.rows % 320 == 0);
+    const TileCost *c = cheapest_tile(costs[w.scaled ? 1 : 0], w.rows, w.cols / 256, m, residual, !silu_mul && w.rows % 320 == 0, image, covering.rt, covering.ttw);
     return {c->rt, c->ttw};
 }
 
@@ -2790,7 +2797,7 @@ hipError_t launch_gemm_f16_chain(const Weights &w, const GemmF16Io &io, size_t m
         if (n_a < blocks / 2) n_a = 0;
     }
     // (a launch that also leaves QB32 rows wants whole tiles of 64 tokens)
-    const F16Tile tile = n_a > 0 || io.qb_out || w.cols < 1024 ? covering : f16_tile(w, io.silu_mul, io.residual != nullptr, m);
+    const F16Tile tile = n_a > 0 || io.qb_out || w.cols < 1024 ? covering : f16_tile(w, io.silu_mul, io.residual != nullptr, m, image, covering);
     const int ttw = tile.ttw;
     const bool rt5 = tile.rt == 5, rt2 = tile.rt == 2;
     const size_t gx0 = w.rows / (64 * (size_t)tile.rt);

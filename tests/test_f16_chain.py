@@ -435,6 +435,27 @@ def test_chain_on_the_image_is_the_expanding_one_bit_for_bit(hip, torch_, fmt, r
         hip.weights_free(w)
 
 
+def test_tiles_with_and_without_the_image(hip, torch_):
+    """A tile that is a little shorter with the image only is not taken where the codes are expanded: the same values and the same statistics, bit for bit"""
+    rows, cols, m = 2304, 1024, 897
+    rng, mp = np.random.default_rng(7), -(-m // 64) * 64
+    h, _ = make_matrix(hip, rng, "qk256", rows, cols)
+    xh = torch_.from_numpy(rng.normal(0, 1, (mp, cols)).astype(np.float16)).cuda()
+    outs = [(torch_.full((m, rows), 7.0, device="cuda"), torch_.full((rows // 64, mp, 2), float("nan"), device="cuda")) for _ in range(2)]
+    torch_.cuda.synchronize()
+    graph, s = torch_.cuda.CUDAGraph(), torch_.cuda.Stream()
+    with torch_.cuda.graph(graph, stream=s):
+        hip.matmul_f16_dev(h, xh, m, y=outs[0][0], stats_out=outs[0][1], stream=s.cuda_stream)
+    assert hip.matmul_last_tile()["wave_tokens"] == 32
+    graph.replay()
+    torch_.cuda.synchronize()
+    hip.matmul_f16_dev(h, xh, m, y=outs[1][0], stats_out=outs[1][1])
+    assert hip.matmul_last_tile()["wave_tokens"] == 16
+    torch_.cuda.synchronize()
+    assert torch_.equal(outs[0][0], outs[1][0]) and torch_.equal(outs[0][1], outs[1][1])
+    hip.weights_free(h)
+
+
 @pytest.mark.parametrize("fmt", ["qk256", "i2s"])
 @pytest.mark.parametrize("silu", [0, 1])
 def test_concatenation_of_parts_that_have_images(hip, torch_, fmt, silu):

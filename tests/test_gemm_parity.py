@@ -473,6 +473,19 @@ def test_f16_rows_in_and_out_of_few_and_many_rows(hip, torch_, n, k, m, waves):
 FP6_EXPAND = 32  # BITNET_HIP_FUSE_FP6_EXPAND
 
 
+# tiles that are narrower by the image's costs than those that cover the CUs: a little shorter there, longer where the codes are expanded; and much shorter, which holds for both
+@pytest.mark.parametrize("rows,cols,m,expanding,image", [(6912, 1024, 577, 32, 16), (2304, 1024, 1793, 32, 16), (7680, 1024, 1025, 32, 32), (9472, 1024, 321, 32, 32)])
+def test_fp6_tiles_with_and_without_the_image(hip, torch_, rows, cols, m, expanding, image):
+    rng = np.random.default_rng(rows + m)
+    h = hip.weights_upload_qk256(rng.integers(0, 256, rows * cols // 4, dtype=np.uint8), rows, cols, cols // 4)
+    x, outs = rng.normal(0.1, 1.0, (m, cols)).astype(np.float32), []
+    for flags, tokens in ((FP6_DIGITS | FP6_EXPAND, expanding), (FP6_DIGITS, image)):
+        outs.append(run_gemm(hip, torch_, h, x, rows, 2, flags=flags))
+        assert hip.matmul_last_tile()["wave_tokens"] == tokens
+    assert not np.isnan(outs[0]).any() and np.array_equal(*outs)
+    hip.weights_free(h)
+
+
 @pytest.mark.parametrize("rows,cols,m", [(2560, 2560, 4096), (512, 1024, 70), (13824, 2560, 300), (336, 512, 33), (3840, 2560, 4096), (2048, 512, 8130), (13824, 2560, 4096)])
 def test_fp6_form_on_the_resident_fp4_image_is_the_expanding_form_bit_for_bit(hip, torch_, rows, cols, m):
     """Round 5: k_gemm_fp6<.., RES = 1> loads its A operands from the resident fp4 image (k_retile_fp4: exactly the nibbles expand16_fp4
