@@ -328,7 +328,7 @@ int bitnet_hip_experts_out_dev(const float *x0, const uint16_t *w0, size_t cols0
     a.x0 = x0, a.x1 = x1, a.bias = bias, a.w0 = w0, a.w1 = w1, a.cols0 = (int)cols0, a.ld0 = (int)ld0, a.cols1 = (int)cols1, a.ld1 = (int)ld1, a.ldx1 = (int)ldx1;
     a.top = (int)top, a.rows = (int)rows, a.ids = ids, a.identity = identity, a.input = input, a.x0_scale = x0_scale, a.y = y;
     const hipError_t e = launch_experts_out(a, (hipStream_t)stream);
-    if (e == hipErrorInvalidValue) return set_error(BITNET_HIP_ERR_UNSUPPORTED, "experts_out: %zu + %zu x %zu columns do not fit a workgroup's memory", cols0, top, cols1);
+    if (e == hipErrorInvalidValue) return set_error(BITNET_HIP_ERR_UNSUPPORTED, "experts_out: %zu + %zu x %zu columns are too many", cols0, top, cols1);
     BH_HIP_TRY(e);
     return BITNET_HIP_OK;
     BH_GUARD_END

@@ -581,8 +581,8 @@ static hipError_t out_go(const ExpertsOut &a, hipStream_t s) {
     const int chunks = k.c0 + a.top * k.ce, each = (chunks + 3) / 4;
     k.magic = ((1u << 20) + k.ce - 1) / k.ce;
     k.groups = (a.rows + 64 / LPR * R - 1) / (64 / LPR * R);
-    // (the quotient by multiplication holds while chunks * ce stays below 2^20)
-    if ((chunks + 7) / 8 * 8 * CH * 4 > 150 * 1024 || (long)(chunks + 7) * k.ce >= 1 << 20) return hipErrorInvalidValue;
+    // (the quotient by multiplication holds while chunks * ce stays below 2^20: 8 experts of 185000 columns)
+    if ((long)chunks * k.ce >= 1 << 20) return hipErrorInvalidValue;
     auto fn = each <= 2 ? k_experts_out<LPR, R, 2> : each <= 3 ? k_experts_out<LPR, R, 3> : each <= 4 || each == 7 || each == 8 ? k_experts_out<LPR, R, 4> : k_experts_out<LPR, R, 6>;
     hipLaunchKernelGGL(fn, dim3(k.groups), dim3(256), 0, s, k);
     return hipGetLastError();
@@ -590,12 +590,11 @@ static hipError_t out_go(const ExpertsOut &a, hipStream_t s) {
 
 hipError_t launch_experts_out(const ExpertsOut &a, hipStream_t s) {
     auto waste = [&](int ch) { return (double)((a.cols0 + ch - 1) / ch * ch + (long)a.top * ((a.cols1 + ch - 1) / ch * ch)) / (a.cols0 + (double)a.top * a.cols1); };
-    auto fits = [&](int ch) { return ((a.cols0 + ch - 1) / ch + (long)a.top * ((a.cols1 + ch - 1) / ch) + 7) / 8 * 8 * ch * 4 <= 150 * 1024; };
     // four rows per workgroup from 3072 on, where that is still three workgroups per CU; us per step of Mimolix / Lurepel / Sipelorn with R = 4, 2, 1: 3072 rows 244.3 / 230.0 / 347.0,
     // 248.2 / 232.0 / 348.2, 259.9 / 234.5 / 351.5; 2560 rows 290.7 / 278.2 / 391.6, 289.5 / 277.5 / 391.0, 297.6 / 280.0 / 394.0; 1536 rows 153.1 / 151.8 / 232.7, 151.5 / 150.1 / 233.0,
     // 153.7 / 151.2 / 232.2.  The longest rows of lanes whose chunks are not padding for the most part (lanes past a row's end load its last columns again: no traffic)
-    if (waste(512) <= 1.4 * waste(256) && fits(512)) return a.rows >= 3072 ? out_go<64, 4>(a, s) : out_go<64, 2>(a, s);
-    return waste(256) <= 1.3 * waste(128) && fits(256) ? out_go<32, 1>(a, s) : out_go<16, 1>(a, s);
+    if (waste(512) <= 1.4 * waste(256)) return a.rows >= 3072 ? out_go<64, 4>(a, s) : out_go<64, 2>(a, s);
+    return waste(256) <= 1.3 * waste(128) ? out_go<32, 1>(a, s) : out_go<16, 1>(a, s);
 }
 
 }  // namespace bitnet_hip

@@ -783,6 +783,11 @@ def test_way_down_of_one_token(hip, rows, top, colf, cols0):
         assert not np.any(got[rows:])
 
 
+def test_way_down_of_one_token_with_many_columns(hip):
+    test_way_down_of_one_token(hip, 5, 8, 6144, 1000)
+    test_way_down_of_one_token(hip, 3, 2, 40008, 8)
+
+
 # 64 lanes per row with chunks that lie partly and wholly past the columns, 32 and 16 lanes
 @pytest.mark.parametrize("rows,top,colf,cols0", [(9, 3, 512, 0), (3073, 5, 1024, 1024), (70, 1, 520, 1536), (33, 8, 200, 256), (17, 2, 72, 136)])
 def test_way_down_of_one_token_with_infinite_weights(hip, rows, top, colf, cols0):

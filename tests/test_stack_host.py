@@ -181,6 +181,7 @@ def test_entry_points_check_shapes_before_any_launch(built):
         (lambda: hip.experts_up_dev(8, built.Router(8, 4, 2, 1.0), 8, 8, 16, 8, 64, 0, 8, 16, 8), "experts_up"),
         (lambda: hip.experts_up_dev(8, built.Router(8, 0, 2, 1.0), 8, 8, 16, 12, 64, 0, 8, 16, 8), "experts_up"),
         (lambda: hip.experts_out_dev(8, 8, 64, 64, None, 8, 8, 8, 16, 64, 8, 2, 16, 8), "experts_out"),
+        (lambda: hip.experts_out_dev(8, 8, 64, 64, None, 8, 1 << 18, 8, 1 << 18, 1 << 18, 8, 8, 16, 8), "columns are too many"),
         (lambda: hip.sum_norm_rows_dev(built.SumRows(x=8, m=1, width=8, h=8, ldh=7)), "sum_norm_rows"),
         (lambda: hip.sum_norm_rows_dev(built.SumRows(x=8, m=1, width=8, h=8, ldh=8, gate=8, ld_gate=7)), "sum_norm_rows: bad gate"),
         (lambda: hip.gqa_step_dev(built.Gqa(4, 2, 2, 16, 32, 16, 32, 128, 1e-5, 0.1, 0.9, 8, 8, 8, 8, 8, far_weight=8, far_rate=8), 8, 8, 8), "gqa: bad window"),
