@@ -889,9 +889,13 @@ hipError_t launch_gqa_out(const GqaOut &a, hipStream_t s) {
         constexpr int N = decltype(nu)::value, B = decltype(nb)::value, R = decltype(rr)::value;
         return u == 1 ? k_gqa_out<R, 1, N, B> : u == 2 ? k_gqa_out<R, 2, N, B> : u == 3 ? k_gqa_out<R, 3, N, B> : u == 4 ? k_gqa_out<R, 4, N, B> : k_gqa_out<R, 5, N, B>;
     };
-    auto pick = [&](auto nu, auto nb) { return r == 2 ? pick_r(std::integral_constant<int, 2>(), nu, nb) : pick_r(std::integral_constant<int, 1>(), nu, nb); };
-    auto of = [&](auto nb) { return pieces <= 512 ? pick(std::integral_constant<int, 2>(), nb) : pieces <= 768 ? pick(std::integral_constant<int, 3>(), nb) : pick(std::integral_constant<int, 4>(), nb); };
-    auto fn = a.records <= 2 ? of(std::integral_constant<int, 2>()) : of(std::integral_constant<int, 4>());
+    auto of = [&](auto rr, auto nb) {
+        return pieces <= 512 ? pick_r(rr, std::integral_constant<int, 2>(), nb) : pieces <= 768 ? pick_r(rr, std::integral_constant<int, 3>(), nb) : pick_r(rr, std::integral_constant<int, 4>(), nb);
+    };
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
+    const std::integral_constant<int, 4> four;
+    auto fn = a.records <= 2 ? of(one, two) : r == 1 ? of(one, four) : of(two, four);
     hipLaunchKernelGGL(fn, dim3(n_wg), dim3(256), (size_t)k.kp * sizeof(float), s, k);
     return hipGetLastError();
 }
