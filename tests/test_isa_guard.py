@@ -264,3 +264,16 @@ def test_matrix_vector_products_keep_no_scratch(tmp_path):
     assert len(gemv) >= 60
     for name, u in gemv.items():
         assert u["ScratchSize"] == 0 and u["Occupancy"] >= 2, (name, u)
+
+
+def test_products_of_records_and_experts_keep_no_scratch(tmp_path):
+    """The way down of a token's experts requests up to 24 pieces of weights at once under a budget of three waves per SIMD (165 of 168 registers in the largest instance); the product that
+    merges the attention's records holds all of them in registers; both instantiated for what their launches choose and nothing else"""
+    if not os.path.exists(HIPCC):
+        pytest.skip("no hipcc")
+    for src, kernel, count, waves in (("kernels_experts.hip", "k_experts_out", 16, 3), ("kernels_gqa.hip", "k_gqa_out", 45, 2)):
+        _, usage = _compile(src, str(tmp_path))
+        found = {name: u for name, u in usage.items() if kernel in name}
+        assert len(found) == count, (kernel, len(found))
+        for name, u in found.items():
+            assert u["ScratchSize"] == 0 and u["Occupancy"] >= waves, (name, u)

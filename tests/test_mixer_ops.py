@@ -444,8 +444,8 @@ def test_attention_portion_in_groups(hip, pkg, shape, n, nq, groups):
     t.check(out, n - nq, 2e-2)
 
 
-# heads, columns of one, rows of the product, extra columns of its matrix; position, chunk, window; records asked for
-@pytest.mark.parametrize("heads,vdimp,rows,extra", [(1, 32, 5, 0), (12, 128, 1536, 0), (20, 128, 2560, 64), (24, 128, 3072, 0), (3, 160, 70, 32), (4, 1024, 9, 0), (7, 96, 2050, 32)])
+# heads, columns of one, rows of the product (the last two: more than the workgroups of one round take), extra columns of its matrix; position, chunk, window; records asked for
+@pytest.mark.parametrize("heads,vdimp,rows,extra", [(1, 32, 5, 0), (12, 128, 1536, 0), (20, 128, 2560, 64), (24, 128, 3072, 0), (3, 160, 70, 32), (4, 1024, 9, 0), (7, 96, 2050, 32), (2, 64, 3081, 0), (2, 96, 6161, 0)])
 @pytest.mark.parametrize("pos,chunk,window,records", [(0, 0, 0, 1), (127, 0, 0, 2), (128, 0, 0, 2), (511, 0, 0, 4), (300, 256, 0, 1), (900, 0, 200, 3), (1000, 0, 400, 4)])
 @pytest.mark.parametrize("sink,gate", [(False, None), (True, "head"), (False, "column")])
 def test_records_merged_by_the_product(hip, pkg, heads, vdimp, rows, extra, pos, chunk, window, records, sink, gate):

@@ -227,6 +227,70 @@ def test_graph_replays_match_eager_steps(cases, dtype, name):
     assert np.array_equal(out[0], out[1])
 
 
+# a chunk that every position lies in; one that ends behind 640 positions, where the records are few again; windows of 150 and 700 positions
+FORMS = {"chunks": u.lurepel([u.chunk_layer(chunk=5000), u.chunk_layer(heads=4, kv_heads=2, chunk=640, mlp=u.gated_mlp())], width=72, vocab=60),
+         "one_chunk": u.lurepel([u.chunk_layer(heads=4, kv_heads=2, chunk=640, mlp=u.gated_mlp())], width=72, vocab=60),
+         "windows": u.sipelorn([u.window_layer(window=150, taps=2, mlp=u.xielu_mlp()), u.window_layer(window=700, taps=3)], width=72, vocab=60)}
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", list(FORMS))
+def test_steps_where_the_number_of_records_changes_their_form(pkg, hip, tmp_path, dtype, name):
+    """Single tokens across 128, 256 and 512 keys and back to a few: the output products merge the attention's records up to two, up to four, or not at all.  Every position against
+    the oracle; one by one and in one run, replayed and launched, bit for bit the same."""
+    config = FORMS[name]
+    t = u.random_tensors(config, 45)
+    m = pkg.open_model(u.save_model(str(tmp_path), config, t), dtype, 720)
+    tokens = tokens_of(config, 660, 14)
+    want = so.forward(config, t, tokens)[0]
+    out = []
+    for use_graph in (True, False):
+        m.reset()
+        m.feed(tokens)
+        m.prefill(100, with_logits=False)
+        rows = []
+        for _ in range(560):
+            m.run(1, use_graph=use_graph)
+            rows.append(m.last_logits())
+        out.append(np.stack(rows))
+    assert error(out[0], want[100:]) < LIMIT[dtype]
+    assert np.array_equal(out[0], out[1])
+    for use_graph in (True, False):
+        m.reset()
+        m.feed(tokens)
+        m.prefill(240, with_logits=False)
+        m.run(420, use_graph=use_graph)
+        assert error(m.last_logits()[None], want[-1:]) < LIMIT[dtype]
+    m.close()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_several_models_at_once(pkg, hip, tmp_path, dtype):
+    """models opened one behind the other in one process, their prompts and steps in turn: each computes what it does alone, bit for bit"""
+    paths = {name: u.save_model(str(tmp_path / name), MODELS[name], u.random_tensors(MODELS[name], sum(map(ord, name)))) for name in SEQUENCES}
+    tokens = {name: tokens_of(MODELS[name], 90, 15) for name in SEQUENCES}
+
+    def calls(m, t):
+        yield lambda: m.forward(t[:70], [0, 69])
+        for i in range(70, 90):
+            yield lambda i=i: m.forward(t[i:i + 1], [0])
+
+    alone = {}
+    for name in SEQUENCES:
+        m = pkg.open_model(paths[name], dtype, 128)
+        alone[name] = [call() for call in calls(m, tokens[name])]
+        m.close()
+    models = {name: pkg.open_model(paths[name], dtype, 128) for name in SEQUENCES}
+    for _ in range(2):
+        for m in models.values():
+            m.reset()
+        for i, row in enumerate(zip(*(list(calls(models[name], tokens[name])) for name in SEQUENCES))):
+            for name, call in zip(SEQUENCES, row):
+                assert np.array_equal(call(), alone[name][i]), (name, i)
+    for m in models.values():
+        m.close()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("name", ["mixed", "lightning_only", "many_heads", "mimolix", "mimolix_delta", "lurepel", "lurepel_identities", "sipelorn", "sipelorn_narrow"])
 def test_greedy_generation(cases, name, dtype):
