@@ -1345,7 +1345,7 @@ static hipError_t grouped_go(const GemmArgsD &a, hipStream_t s) {
 // 2 to 400 rows per expert, us with 64 x 64 in four buffers / in three / 128 x 64 / 128 x 128 in four waves / in eight:
 //   64 x 64, four buffers: what the others do not take.  8 experts, 1024 x 4096, 16 rows 21 / 28 / 53; 128, 768 x 2048, 32 rows 79 / 81 / 89
 //   128 x 64 (activations serve twice the columns): where nearly every CU gets two, from as many rows on as K is long.  64, 896 x 3072, 44 rows 74 / 75 / 70; 64, 1024 x 1024, 16 rows
-//     31 / 30 / 27; 64, 1536 x 448, 8 rows 21 / 20 / 19.  Not with rows of whole 4 KiB, whose beginnings meet on the same channels: 256, 512 x 2048, 44 rows 114 / 117 / 136
+//     31 / 30 / 27; 64, 1536 x 448, 8 rows 21 / 20 / 19; 64, 768 x 2560, 52 rows 67 / 68 / 60.  Not with rows of whole 4 KiB, whose beginnings meet on the same channels: 256, 512 x 2048, 44 rows 114 / 117 / 136
 //   64 x 64, three buffers, of which a CU takes three: one to two workgroups per CU.  8, 4096 x 1024, 16 rows 17 / 15 / 19; not with such rows either
 //   128 x 128 in eight waves: one round of workgroups (64, 448 x 1536, 72 rows 31 / 31 / 28 / 29 / 23), or two to three of them for long K while an expert has one tile (64, 1408 x 2048,
 //     88 rows 108 / 109 / 96 / 99 / 91)
@@ -1356,8 +1356,8 @@ static hipError_t launch_grouped(const GemmArgsD &a, hipStream_t s) {
     const long tn = (a.n + 127) / 128, wide = experts * tn;
     if (a.tile == 64) {
         const bool spread = a.k % 2048 != 0;
-        const long rows_from = a.k <= 512 ? 0 : a.k <= 1024 ? 6 : 40;
-        if (wide >= 448 && (spread || a.k <= 1024) && a.m >= rows_from * experts) return grouped_go<128, 64, 2, 2, 2>(a, s);
+        const long rows_from = a.k <= 512 ? 0 : a.k <= 1024 ? 6 : wide >= 448 ? 40 : 50;
+        if (wide >= (a.k <= 1024 ? 448 : 384) && (spread || a.k <= 1024) && a.m >= rows_from * experts) return grouped_go<128, 64, 2, 2, 2>(a, s);
         const long all = (long)experts * ((a.n + 63) / 64);
         return all > 256 && all <= 512 && spread ? grouped_go<64, 64, 2, 2, 3>(a, s) : grouped_go<64, 64, 2, 2, 4>(a, s);
     }

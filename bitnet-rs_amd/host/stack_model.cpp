@@ -1147,8 +1147,9 @@ int StackModel::portion_block(size_t i, int pass, int which, size_t n, size_t po
     const bitnet_hip_router r = router_args(i);
     // Tiles of 128 rows from 56 per expert on, where a good share of the experts has more than 64 and their weights would be read twice; from 96 on where a tile per expert leaves CUs without
     // work (16 experts of 512 x 1024, 72 rows each: tiles of 64 rows 7.1 us, of 128 13.3).
+    // (identity experts, which have no rows, are chosen like the others)
     const size_t columns = std::min(e.gated ? 2 * e.ff : e.ff, width_), rows_from = e.count * ((columns + 127) / 128) >= 256 ? 56 : 96;
-    const size_t tile = !f32_ && n * e.top >= rows_from * e.count ? 128 : 64;
+    const size_t tile = !f32_ && n * e.top >= rows_from * (e.count + e.identity) ? 128 : 64;
     BCHK(bitnet_hip_experts_plan_make(pplan_.p, pplan_.bytes, n, e.count, e.top, tile, &plan_));
     BCHK(bitnet_hip_experts_route_dev(tail + B.gates, ldt, &r, &plan_, stream_));
     BCHK(bitnet_hip_experts_matmul_dev(&plan_, 1, ph_.p, ldh, f32_, B.expert_up.w, e.gated ? 2 * e.ff : e.ff, B.expert_up.ld, B.expert_up.ld,
