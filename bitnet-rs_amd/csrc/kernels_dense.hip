@@ -1017,12 +1017,12 @@ static void gemv_pick_u(int u, const GemvK &k, dim3 grid, hipStream_t s) {
         gemv_go<LPR, R, false>(u, k, grid, s);
 }
 
-// What k_dense_gemv_plain takes: a vector as it lies there, no epilogue beyond bias and activation, rows of more than half a wave.  Many short rows stay with k_dense_gemv, whose
+// What k_dense_gemv_plain takes: a vector as it lies there, it and the weights on 16 bytes, no epilogue beyond bias and activation, rows of more than half a wave.  Many short rows stay with k_dense_gemv, whose
 // workgroups take several groups of them, us there / here: 16384 x 512 6.8 / 6.1, 65536 x 520 17.5 / 17.5, x 768 20.1 / 18.7, 128256 x 264 23 / 31, x 512 26 / 33, x 520 27.9 / 31.6,
 // x 640 29.4 / 32.4, x 768 33.8 / 34.6, x 1024 43 / 38.  One, two or four rows per workgroup:
 // us with R = 1, 2, 4 at 512 x 1536 2.8, 2.9, 3.0, 1024 x 4096 4.0, 4.0, 4.0, 2560 x 6912 11.4, 9.0, 9.4, 3072 x 8192 14.3, 11.4, 11.1, 16384 x 4096 27.9, 24.8, 23.4.
 static bool gemv_is_plain(const GemvArgs &a) {
-    return a.in.kind == BITNET_HIP_IN_PLAIN && ((uintptr_t)a.in.x & 15) == 0 && a.batch == 1 && !a.gated && !a.best_val && !a.latent && !a.more.conv && !a.more.mul &&
+    return a.in.kind == BITNET_HIP_IN_PLAIN && (((uintptr_t)a.in.x | (uintptr_t)a.w) & 15) == 0 && a.batch == 1 && !a.gated && !a.best_val && !a.latent && !a.more.conv && !a.more.mul &&
            a.cols > (a.rows <= 16384 ? 256 : a.rows <= 65536 ? 512 : 768) && a.more.act2_from >= a.rows && a.act0 != BITNET_HIP_ACT_XIELU && a.act1 != BITNET_HIP_ACT_XIELU;
 }
 

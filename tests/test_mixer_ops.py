@@ -41,6 +41,14 @@ def test_gemv_of_a_plain_vector(hip, pkg, rows, cols, off):
     assert u.rms_error(u.host(y)[:rows], z - bias) < (F32_TOL if rows > 1 else 1e-5)
 
 
+@pytest.mark.parametrize("rows,cols", [(70, 520), (3074, 2560)])
+def test_gemv_of_a_plain_vector_and_weights_off_sixteen_bytes(hip, rows, cols):
+    g = rng(rows, cols)
+    w, x, y = u.rounded(g.standard_normal((rows, cols)) / np.sqrt(cols)), g.standard_normal(cols).astype(np.float32), u.zeros_f32(rows)
+    hip.dense_gemv_dev(u.dev_f32(x), u.dev_bf16(np.concatenate([np.full(4, np.nan, np.float32), w.reshape(-1)]))[4:], rows, cols, cols, y, n=cols)
+    assert u.rms_error(u.host(y), w.astype(np.float64) @ x) < F32_TOL
+
+
 # a wave's chunks that lie partly and wholly past the columns, and none that does
 @pytest.mark.parametrize("rows,cols", [(5, 3072), (600, 1536), (3073, 2560), (9, 2048), (7, 520), (513, 6152)])
 def test_gemv_of_a_plain_vector_with_infinite_weights(hip, rows, cols):
