@@ -1007,11 +1007,14 @@ static void gemv_go(int u, const GemvK &k, dim3 grid, hipStream_t s) {
     hipLaunchKernelGGL(fn, grid, dim3(256), lds, s, k);
 }
 
+static bool gemv_has_more(const GemvArgs &a) {
+    const bool pairs = a.gated && a.gated < a.rows;
+    return a.in.y_gate || pairs || a.more.conv || a.more.mul || a.more.act2_from < a.rows || a.act0 == BITNET_HIP_ACT_XIELU || a.act1 == BITNET_HIP_ACT_XIELU;
+}
+
 template <int LPR, int R>
 static void gemv_pick_u(int u, const GemvK &k, dim3 grid, hipStream_t s) {
-    const GemvArgs &a = k.a;
-    const bool pairs = a.gated && a.gated < a.rows;
-    if (a.in.y_gate || pairs || a.more.conv || a.more.mul || a.more.act2_from < a.rows || a.act0 == BITNET_HIP_ACT_XIELU || a.act1 == BITNET_HIP_ACT_XIELU)
+    if (gemv_has_more(k.a))
         gemv_go<LPR, R, true>(u, k, grid, s);
     else
         gemv_go<LPR, R, false>(u, k, grid, s);
@@ -1035,8 +1038,361 @@ static hipError_t gemv_plain_go(const GemvArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// A vector that is formed on the way -- summed, normed, gated -- without going through LDS: wave w of a workgroup takes the columns of the chunks w, w + waves, .. of 512 of ALL its rows, a lane forms
+// the vector at its own eight columns per chunk in registers, once, and keeps it for the workgroup's rows, which follow one another four at a time, the next four on their way.  Requests go out in the
+// order vectors, what the rows' ends need, weights.  What an rms norm divides by follows the product, so its sum costs no meeting of the waves; a layer norm's mean and squares about it are put together
+// from the waves' own means in one.  The waves' partial sums meet in LDS once, behind the last row, and a thread finishes each row.  Bound by the launch and two dependent latencies below some
+// 10 MB, by memory above.  us per launch in a chain, k_dense_gemv / this form, rms norm | added and normed twice | layer norm of a sum:
+//   256 x 2560 4.0 / 2.9 | 5.0 / 3.9 | 4.9 / 4.1    1932 x 1536 4.5 / 3.5 | 5.6 / 4.5 | 5.3 / 4.5    2112 x 2560 6.0 / 4.7 | 7.5 / 5.9 | 7.2 / 5.6    5376 x 1536 6.6 / 5.2 | 7.9 / 6.1 | 7.5 / 6.0
+//   6912 x 2560 9.5 / 8.1 | 10.4 / 9.1 | 10.2 / 9.1    10240 x 2560 13.4 / 11.2 | 15.0 / 12.0 | 14.4 / 11.7    12288 x 3072 15.4 / 15.8 | 16.4 / 16.0 | 15.8 / 15.4    3072 x 6144 14.5 / 8.3 | 22.8 / 9.9 | 21.6 / 10.3
+struct GemvFormK {
+    GemvArgs a;
+    LatentRows lat;
+    int rows_wg;  // rows of a workgroup, a multiple of R
+    int lat_wg;   // workgroup index that writes the latent row, or -1
+};
+constexpr int kFormedRows = 256;  // most rows of a workgroup (a thread finishes each, so no more than its threads either)
+
+// Four values per lane -> their sums over the wave, the i-th in the sixteen lanes from 32 (i % 2) + 16 (i / 2) on: pairs fold onto one another, 10 steps instead of 24.
+__device__ __forceinline__ float four_sums(float (&v)[4]) {
+    swap_rows32(v[0], v[1]), swap_rows32(v[2], v[3]);
+    float a = v[0] + v[1], b = v[2] + v[3];
+    swap_rows16(a, b);
+    return row_sum(a + b);
+}
+
+// R rows at a time, U chunks per wave; NORM: 0 none, 1 rms, 2 layer norm; MORE as k_dense_gemv's
+template <int R, int U, int NORM, bool MORE>
+__global__ __launch_bounds__(512) void k_dense_gemv_formed(GemvFormK p) {
+    __shared__ __attribute__((aligned(16))) float slots[4][8];
+    __shared__ __attribute__((aligned(16))) float parts[kFormedRows + R][8];
+    const GemvArgs &a = p.a;
+    const VecIn &in = a.in;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = (int)blockDim.x >> 6;
+    asm volatile("" ::"s"(in.x), "s"(in.y), "s"(in.post_weight), "s"(in.scale), "s"(in.weight), "s"(in.bias), "s"(in.gate), "s"(in.x_out), "s"(in.kind), "s"(in.n), "s"(in.mean_n), "s"(a.w),
+                 "s"(a.rows), "s"(a.cols), "s"(a.ld), "s"(p.rows_wg), "s"(p.lat_wg), "s"(a.bias));
+    if ((int)blockIdx.x == p.lat_wg) {  // (four waves)
+        if (p.lat.f32) {
+            if (p.lat.cq) latent_queries<float>(p.lat, 0, slots[0]);
+            latent_row<float>(p.lat, 0, slots[0]);
+        } else {
+            if (p.lat.cq) latent_queries<uint16_t>(p.lat, 0, slots[0]);
+            latent_row<uint16_t>(p.lat, 0, slots[0]);
+        }
+        return;
+    }
+    const int row0 = blockIdx.x * p.rows_wg, n_rows = min(p.rows_wg, a.rows - row0);
+    const bool writer = blockIdx.x == 0;
+    int col[U];
+    bool inside[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) col[u] = (wave + nw * u) * 512 + lane * 8, inside[u] = col[u] < a.cols;
+    typedef f32x4 Vec[U][2];
+    const int bytes = in.n * 4;
+    auto load = [&](Vec &v, const float *from, int behind = 0) {  // (elements ahead of `behind` have offsets past any buffer's end)
+        const auto r = bounded(from, bytes);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[u][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, 4 * (col[u] - behind) + 16 * h, 0, 0));
+    };
+    const bool added = in.kind >= BITNET_HIP_IN_RESIDUAL_NORM && in.y, normed = added && in.post_weight, scaled = normed && in.scale, y_gated = MORE && added && in.y_gate;
+    const bool gated = NORM && in.gate, shifted = NORM == 2 && in.bias, two = NORM == 0 && in.kind == BITNET_HIP_IN_CONCAT;
+    Vec xv, yv, pw, sc, yg, wv, bv, gv;
+    load(xv, in.x);
+    if (added) load(yv, in.y);
+    if (normed) load(pw, in.post_weight);
+    if (scaled) load(sc, in.scale);
+    if (y_gated) load(yg, in.y_gate);
+    if (NORM) load(wv, in.weight);
+    if (two) load(wv, in.x2, in.n);
+    if (shifted) load(bv, in.bias);
+    if (gated) load(gv, in.gate);
+    // a thread finishes one row: what it needs for that
+    const Epilogue &e = a.more;
+    const int row = row0 + tid;
+    const bool finishes = tid < n_rows;
+    const bool conv = MORE && e.conv, mul = MORE && e.mul;
+    float bias = 0.f;
+    if (a.bias && finishes) bias = a.bias[row];
+    constexpr int TAPS = 3;  // earlier positions of a convolution requested ahead
+    int pos = 0;
+    const int ch = MORE ? row - e.conv_from : -1;
+    const bool convolved = conv && finishes && ch >= 0 && ch < e.channels;
+    float past[TAPS], tap[TAPS], last_tap = 0.f;
+    if (conv) {
+        pos = *e.pos;
+        if (convolved) {
+            last_tap = e.conv[(size_t)(e.taps - 1) * e.channels + ch];
+#pragma unroll
+            for (int j = 0; j < TAPS; ++j) {  // (j + 1 positions back)
+                const int at = pos - 1 - j, t = e.taps - 2 - j;
+                past[j] = 0.f, tap[j] = 0.f;
+                if (t >= 0 && at >= 0) past[j] = e.ring[(size_t)(at % e.taps) * e.channels + ch], tap[j] = e.conv[(size_t)t * e.channels + ch];
+            }
+        }
+    }
+    int mul_token = 0;
+    if (mul) mul_token = e.mul_tokens[*e.mul_at];
+    // weights
+    const auto wr = bounded(a.w + (size_t)row0 * a.ld, n_rows * a.ld * 2);
+    int woff[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) woff[u] = inside[u] ? 2 * col[u] : 0x7fffffff;
+    u32x4 w0[R][U], w1[R][U];
+    auto fetch = [&](u32x4 (&w)[R][U], int i) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int u = 0; u < U; ++u) w[r][u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, woff[u], min(i + r, n_rows - 1) * a.ld * 2, kBufferNt));
+    };
+    fetch(w0, 0);
+    auto squares = [&](const Vec &v) {
+        float ss = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) ss += (v[u][h].x * v[u][h].x + v[u][h].y * v[u][h].y) + (v[u][h].z * v[u][h].z + v[u][h].w * v[u][h].w);
+        return ss;
+    };
+    auto total = [&](const float *slot) {
+        const f32x4 lo = *reinterpret_cast<const f32x4 *>(slot), hi = *reinterpret_cast<const f32x4 *>(slot + 4);
+        float t = lo.x;
+#pragma unroll
+        for (int i = 1; i < 8; ++i) t += i < nw ? (i < 4 ? lo[i & 3] : hi[i & 3]) : 0.f;
+        return t;
+    };
+    const float count = (float)in.mean_n;
+    auto inverse = [&](float ss) { return 1.0f / sqrtf(ss / count + in.eps); };
+    if (added) {
+        float inv = 1.f;
+        if (normed) {
+            const float t = wave_sum(squares(yv));
+            if (lane == 0) slots[0][wave] = t;
+            __syncthreads();
+            inv = inverse(total(slots[0]));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                f32x4 v = yv[u][h] * (normed ? inv : in.mult);
+                if (normed) v *= in.offset + pw[u][h];
+                if (scaled) v *= sc[u][h];
+                if (y_gated) v *= yg[u][h];
+                xv[u][h] += v;
+                if (writer && in.x_out && col[u] < in.n) *reinterpret_cast<f32x4 *>(in.x_out + col[u] + 4 * h) = xv[u][h];
+            }
+    }
+    if (two)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) xv[u][h] += wv[u][h];
+    if (NORM == 1) {  // what it is divided by follows the product
+        const float t = wave_sum(squares(xv));
+        if (lane == 0) slots[2][wave] = t;
+    }
+    float mean = 0.f, inv = 1.f;
+    if (NORM == 2) {
+        // sums of a wave's own columns and of its squares about its own mean, put together without a second meeting
+        auto columns = [&](int wv_) {
+            int c = 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) c += min(max(a.cols - (wv_ + nw * u) * 512, 0), 512);
+            return (float)c;
+        };
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) s += (xv[u][h].x + xv[u][h].y) + (xv[u][h].z + xv[u][h].w);
+        s = wave_sum(s);
+        const float own = s / fmaxf(columns(wave), 1.f);
+        Vec d;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) d[u][h] = inside[u] ? xv[u][h] - own : f32x4{0.f, 0.f, 0.f, 0.f};
+        const float m2 = wave_sum(squares(d));
+        if (lane == 0) slots[1][wave] = s, slots[3][wave] = m2;
+        __syncthreads();
+        mean = total(slots[1]) / count;
+        float ss = total(slots[3]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float c = columns(i), off = slots[1][i] / fmaxf(c, 1.f) - mean;
+            ss += i < nw && c > 0.f ? c * (off * off) : 0.f;
+        }
+        inv = inverse(ss);
+    }
+    if (NORM) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                f32x4 v = NORM == 2 ? (xv[u][h] - mean) * inv : xv[u][h];
+                v *= in.offset + wv[u][h];
+                if (gated) v *= gv[u][h];
+                if (shifted) v += bv[u][h];
+                xv[u][h] = v;
+                if (NORM == 2 && writer && in.h_out && inside[u]) *reinterpret_cast<f32x4 *>(in.h_out + col[u] + 4 * h) = v;
+            }
+    }
+    auto rows = [&](const u32x4 (&w)[R][U], int i) {
+        float acc[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            acc[r] = 0.f;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    acc[r] = fmaf(xv[u][c >> 1][2 * c & 3], __builtin_bit_cast(float, w[r][u][c] << 16), acc[r]);
+                    acc[r] = fmaf(xv[u][c >> 1][(2 * c & 3) + 1], __builtin_bit_cast(float, w[r][u][c] & 0xffff0000u), acc[r]);
+                }
+        }
+        if constexpr (R == 4) {
+            const float t = four_sums(acc);
+            if ((lane & 15) == 0) parts[i + (lane >> 5) + (lane >> 3 & 2)][wave] = t;
+        } else {
+            const float t = wave_sum(acc[0]);
+            if (lane == 0) parts[i][wave] = t;
+        }
+    };
+    for (int i = 0; i < n_rows; i += 2 * R) {
+        if (i + R < n_rows) fetch(w1, i + R);
+        rows(w0, i);
+        if (i + 2 * R < n_rows) fetch(w0, i + 2 * R);
+        if (i + R < n_rows) rows(w1, i + R);
+    }
+    __syncthreads();
+    if (NORM == 1) {
+        inv = inverse(total(slots[2]));
+        if (writer && in.h_out)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (inside[u]) *reinterpret_cast<f32x4 *>(in.h_out + col[u] + 4 * h) = xv[u][h] * inv;
+    }
+    auto sum = [&](int r) {
+        const float t = total(parts[r]);
+        return NORM == 1 ? t * inv : t;
+    };
+    float best = -INFINITY;
+    int best_row = 0x7fffffff;
+    if (finishes && row < a.gated) {  // (even, and so are the rows in pairs and those of a workgroup)
+        if (tid & 1) return;
+        const float up_bias = a.bias ? a.bias[row + 1] : 0.f;
+        a.y[row >> 1] = activate(sum(tid) + bias, a.act0) * (sum(tid + 1) + up_bias);
+    } else if (finishes) {
+        float v = sum(tid) + bias;
+        if (convolved) {
+            float f = 0.f;
+            for (int j = e.taps - 2; j >= TAPS; --j) {
+                const int at = pos - 1 - j;
+                if (at >= 0) f += e.conv[(size_t)(e.taps - 2 - j) * e.channels + ch] * e.ring[(size_t)(at % e.taps) * e.channels + ch];
+            }
+#pragma unroll
+            for (int j = TAPS - 1; j >= 0; --j) f += tap[j] * past[j];
+            e.ring[(size_t)(pos % e.taps) * e.channels + ch] = v;  // (no earlier position's slot)
+            v = v * last_tap + f;
+        }
+        const int act = MORE && row >= e.act2_from ? e.act2 : row < a.act_split ? a.act0 : a.act1;
+        v = MORE && act == BITNET_HIP_ACT_XIELU ? activate(v, act, e.act_a, e.act_b) : activate(v, act);
+        if (mul) v *= bf2f(e.mul[(size_t)min(max(mul_token, 0), e.mul_rows - 1) * e.ld_mul + row]);
+        a.y[row - (a.gated >> 1)] = v;
+        best = v != v ? -INFINITY : v;
+        best_row = row;
+    }
+    if (a.best_val) {  // (no pairs)
+        auto better = [&](float v, int i) {
+            if (v > best || (v == best && i < best_row)) best = v, best_row = i;
+        };
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const float v = __shfl_xor(best, off, 64);
+            const int i = __shfl_xor(best_row, off, 64);
+            better(v, i);
+        }
+        if (lane == 0) slots[0][wave] = best, slots[1][wave] = __builtin_bit_cast(float, best_row);
+        __syncthreads();
+        if (tid == 0) {
+            for (int i = 1; i < nw; ++i) better(slots[0][i], __builtin_bit_cast(int, slots[1][i]));
+            a.best_val[blockIdx.x] = best;
+            a.best_idx[blockIdx.x] = best_row;
+        }
+    }
+}
+
+struct FormedSplit {
+    int u, waves;  // chunks of 512 columns per wave
+};
+static FormedSplit formed_split(const GemvArgs &a) {
+    const int chunks = (a.cols + 511) / 512, most = a.latent ? 4 : 8, u = (chunks + most - 1) / most;
+    return {u, a.latent ? 4 : (chunks + u - 1) / u};
+}
+// What k_dense_gemv_formed takes: a vector to be formed, whole in eights, it and the weights on 16 bytes (a lane's columns are inside or outside as one, and loads past the end give zeros, so that an
+// infinite weight counts for its own row alone), more than half a wave's columns and no more than two chunks for each of eight waves.  Past 2^26 weights (a head) memory is all that
+// counts and k_dense_gemv, whose waves take whole rows, is as fast or faster: us there / here 32768 x 1536 21.7 / 18.9, 16384 x 2560 19.3 / 16.9, 32768 x 3072 35.9 / 36.7, 128256 x 2560 100.2 / 101.2.
+static bool gemv_is_formed(const GemvArgs &a) {
+    const VecIn &in = a.in;
+    const uintptr_t all = (uintptr_t)in.x | (uintptr_t)in.y | (uintptr_t)in.post_weight | (uintptr_t)in.scale | (uintptr_t)in.y_gate | (uintptr_t)in.weight | (uintptr_t)in.bias |
+                          (uintptr_t)in.gate | (uintptr_t)in.x2 | (uintptr_t)in.x_out | (uintptr_t)in.h_out | (uintptr_t)a.w;
+    return in.kind != BITNET_HIP_IN_PLAIN && in.n % 8 == 0 && (in.kind == BITNET_HIP_IN_CONCAT ? 2 : 1) * in.n == a.cols && a.cols > 256 && a.cols <= 8192 && (all & 15) == 0 && a.batch == 1 &&
+           (!a.latent || a.cols <= 4096) && (!a.best_val || a.rows <= 1024 * std::min(64 * formed_split(a).waves, kFormedRows)) && (size_t)a.rows * a.cols <= ((size_t)1 << 26) &&
+           (!a.more.conv || a.more.conv_from >= a.gated) && (size_t)kFormedRows * a.ld < ((size_t)1 << 30);
+}
+
+template <int R, int U>
+static void gemv_formed_go(const GemvFormK &k, dim3 grid, dim3 block, hipStream_t s) {
+    const GemvArgs &a = k.a;
+    const int norm = a.in.kind == BITNET_HIP_IN_RESIDUAL || a.in.kind == BITNET_HIP_IN_CONCAT ? 0 : a.in.center ? 2 : 1;
+    void (*fn)(GemvFormK) = gemv_has_more(a) ? (norm == 0 ? k_dense_gemv_formed<R, U, 0, true> : norm == 1 ? k_dense_gemv_formed<R, U, 1, true> : k_dense_gemv_formed<R, U, 2, true>)
+                                             : (norm == 0 ? k_dense_gemv_formed<R, U, 0, false> : norm == 1 ? k_dense_gemv_formed<R, U, 1, false> : k_dense_gemv_formed<R, U, 2, false>);
+    hipLaunchKernelGGL(fn, grid, block, 0, s, k);
+}
+
+static hipError_t launch_gemv_formed(const GemvArgs &a, int *n_wg_out, hipStream_t s) {
+    GemvFormK k;
+    k.a = a;
+    k.a.latent = nullptr;
+    if (a.act_split == 0) k.a.act_split = a.rows;
+    if (k.a.in.mean_n == 0) k.a.in.mean_n = a.in.n;
+    const auto [u, waves] = formed_split(a);
+    // Up to 256 rows a row per CU.  Else steps of four rows, one or two workgroups per CU (of one or two waves up to four), the count that leaves a CU the fewest steps in turn: a launch lasts as long as
+    // the CUs with the most.  One workgroup has no other's loads to hide its sums behind (1.15), but of five waves and more a second one is worth its forming from two steps on only.  us, rows per
+    // workgroup: 2112 x 2560 12 5.9, 8 6.3; 2560 x 2560 12 6.1, 8 6.3, 4 6.6; 4096 x 1536 8 5.3, 16 5.5, 4 5.7; 5000 x 3072 20 8.6, 12 8.9; 6912 x 2560 16 9.1, 28 9.6, 36 10.1;
+    // 3000 x 512 4 3.4, 12 4.6; 12000 x 1024 12 6.7, 16 7.1, 24 7.3.  One, two or four rows at a time: 1932 x 1536 5.2, 4.7, 4.5; 10240 x 2560 12.9, 12.4, 11.5.
+    const bool single = a.rows <= 256 && !a.gated;
+    int each = 1;
+    if (!single) {
+        double least = 0;
+        for (int per = 1; per <= (waves <= 2 ? 4 : 2); ++per) {
+            const int n = (a.rows + 1024 * per - 1) / (1024 * per);
+            if (per > 1 && n == 1 && waves >= 5) break;
+            const double cost = per * n * (per == 1 ? 1.15 : 1.0);
+            if (per == 1 || cost <= least) least = cost, each = 4 * n;
+        }
+        each = std::min({each, 64 * waves, kFormedRows});
+    }
+    k.rows_wg = each;
+    const int n_wg = (a.rows + each - 1) / each;
+    if (n_wg_out) *n_wg_out = n_wg;
+    k.lat_wg = a.latent ? n_wg : -1;
+    if (a.latent) k.lat = *a.latent;
+    const dim3 grid(n_wg + (a.latent ? 1 : 0)), block(64 * waves);
+    if (u == 1)
+        single ? gemv_formed_go<1, 1>(k, grid, block, s) : gemv_formed_go<4, 1>(k, grid, block, s);
+    else
+        single ? gemv_formed_go<1, 2>(k, grid, block, s) : gemv_formed_go<4, 2>(k, grid, block, s);
+    return hipGetLastError();
+}
+
 hipError_t launch_dense_gemv(const GemvArgs &a, int *n_wg_out, hipStream_t s) {
     if (gemv_is_plain(a)) return a.rows >= 3072 ? gemv_plain_go<4>(a, s) : a.rows > 512 ? gemv_plain_go<2>(a, s) : gemv_plain_go<1>(a, s);
+    if (gemv_is_formed(a)) return launch_gemv_formed(a, n_wg_out, s);
     GemvK k;
     k.a = a;
     k.a.latent = nullptr;
