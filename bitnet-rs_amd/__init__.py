@@ -645,6 +645,13 @@ class HipLib:
     def gqa_out_dev(self, a: "Gqa", pos, records: int, scratch, w, rows: int, cols: int, ld: int, y, bias=None, stream: int = 0) -> None:
         self._call("gqa_out_dev", C.byref(a), _ptr(pos), _sz(records), _ptr(scratch), _ptr(w), _sz(rows), _sz(cols), _sz(ld), _optr(bias), _ptr(y), _vp(stream))
 
+    def gqa_project_records(self, a: "Gqa", cols: int) -> int:
+        self.c.bitnet_hip_gqa_project_records.restype = _sz
+        return int(self.c.bitnet_hip_gqa_project_records(C.byref(a), _sz(cols)))
+
+    def gqa_project_dev(self, a: "Gqa", pos, records: int, scratch, w, rows: int, cols: int, ld: int, y, bias=None, stream: int = 0) -> None:
+        self._call("gqa_project_dev", C.byref(a), _ptr(pos), _sz(records), _ptr(scratch), _ptr(w), _sz(rows), _sz(cols), _sz(ld), _optr(bias), _ptr(y), _vp(stream))
+
     def gqa_merge_dev(self, a: "Gqa", pos, q0: int, nq: int, scratch, out, ldo: int, out_bf16: bool, stream: int = 0) -> None:
         self._call("gqa_merge_dev", C.byref(a), _ptr(pos), _sz(q0), _sz(nq), _ptr(scratch), _ptr(out), _sz(ldo), C.c_int(out_bf16), _vp(stream))
 

@@ -158,6 +158,27 @@ int bitnet_hip_gqa_out_dev(const bitnet_hip_gqa *a, const int32_t *pos, size_t r
     BH_GUARD_END
 }
 
+size_t bitnet_hip_gqa_project_records(const bitnet_hip_gqa *a, size_t cols) {
+    if (!a || check_gqa(a) != 0 || cols > 32768) return 0;
+    return (size_t)gqa_project_records(*a, (int)cols);
+}
+
+int bitnet_hip_gqa_project_dev(const bitnet_hip_gqa *a, const int32_t *pos, size_t records, const float *scratch, const uint16_t *w, size_t rows, size_t cols, size_t ld,
+                           const float *bias, float *y, void *stream) {
+    BH_GUARD_BEGIN
+    if (int rc = check_gqa(a)) return rc;
+    BH_REQUIRE(pos && scratch && w && y && rows > 0 && records > 0 && cols >= 8 && cols % 8 == 0 && cols <= ld && ld % 8 == 0 && ld <= 32768 && (((uintptr_t)scratch | (uintptr_t)w) & 15) == 0 &&
+                   (!a->gate || !a->gate_columns || (uintptr_t)a->gate % 16 == 0),
+               "gqa_project: bad arguments");
+    BH_CHECK_DIMS(rows, ld);
+    if (records > (size_t)gqa_project_records(*a, (int)cols)) return set_error(BITNET_HIP_ERR_UNSUPPORTED, "gqa_project: %zu records of %zu heads of %zu columns", records, a->heads, a->vdimp);
+    GqaOut o;
+    o.g = *a, o.pos = pos, o.scratch = scratch, o.bias = bias, o.w = w, o.y = y, o.rows = (int)rows, o.cols = (int)cols, o.ld = (int)ld, o.records = (int)records;
+    BH_HIP_TRY(launch_gqa_project(o, (hipStream_t)stream));
+    return BITNET_HIP_OK;
+    BH_GUARD_END
+}
+
 int bitnet_hip_gqa_prefill_last_groups(void) { return g_last_gqa_groups; }
 
 int bitnet_hip_gqa_prefill_dev(const bitnet_hip_gqa *a, const uint16_t *q, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out, size_t ldo, void *stream) {

@@ -241,6 +241,8 @@ struct GqaOut {  // records of one query -> output -> product
 };
 int gqa_out_records(const Gqa &g, int cols);
 hipError_t launch_gqa_out(const GqaOut &a, hipStream_t s);
+int gqa_project_records(const Gqa &g, int cols);
+hipError_t launch_gqa_project(const GqaOut &a, hipStream_t s);
 extern thread_local int g_last_gqa_groups;  // groups of four waves per workgroup of launch_gqa_prefill's last launch on this thread
 hipError_t launch_gqa_prefill(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, hipStream_t s);
 bool delta_supported(int dimp, int vdimp);
@@ -311,6 +313,73 @@ __device__ __forceinline__ float rows_max(float v) {
     return fmaxf(v, w);
 }
 __device__ __forceinline__ float wave_sum(float v) { return rows_sum(row_sum(v)); }
+
+// Four values per lane -> their sums over the wave, the i-th in the sixteen lanes from 32 (i % 2) + 16 (i / 2) on: pairs fold onto one another, 10 steps instead of 24.
+__device__ __forceinline__ float four_sums(float (&v)[4]) {
+    swap_rows32(v[0], v[1]), swap_rows32(v[2], v[3]);
+    float a = v[0] + v[1], b = v[2] + v[3];
+    swap_rows16(a, b);
+    return row_sum(a + b);
+}
+
+// Rows of bf16 weights times a vector that the waves of a workgroup share by columns: lane l of wave w holds the elements of the chunks w, w + waves, .. of 512 at 8 l, U chunks in all, in registers.
+// R (one or four) rows at a time, the next ones on their way.
+template <int R, int U>
+struct SharedRows {
+    __amdgpu_buffer_rsrc_t w;
+    int off[U], n_rows, pitch;  // bytes
+    u32x4 a[R][U], b[R][U];
+    // inside: does the lane have columns in the chunk?  (past the row's end a load gives zeros)
+    __device__ __forceinline__ SharedRows(const uint16_t *first, int n_rows_, int ld, const int (&col)[U], const bool (&inside)[U]) : w(bounded(first, n_rows_ * ld * 2)), n_rows(n_rows_), pitch(ld * 2) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) off[u] = inside[u] ? 2 * col[u] : 0x7fffffff;
+    }
+    __device__ __forceinline__ void fetch(u32x4 (&v)[R][U], int i) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[r][u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w, off[u], min(i + r, n_rows - 1) * pitch, kBufferNt));
+    }
+    __device__ __forceinline__ void request() { fetch(a, 0); }
+    __device__ __forceinline__ void products(const f32x4 (&x)[U][2], const u32x4 (&v)[R][U], int i, float (*parts)[8], int wave, int lane) {
+        float acc[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            acc[r] = 0.f;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    acc[r] = fmaf(x[u][c >> 1][2 * c & 3], __builtin_bit_cast(float, v[r][u][c] << 16), acc[r]);
+                    acc[r] = fmaf(x[u][c >> 1][(2 * c & 3) + 1], __builtin_bit_cast(float, v[r][u][c] & 0xffff0000u), acc[r]);
+                }
+        }
+        if constexpr (R == 4) {
+            const float t = four_sums(acc);
+            if ((lane & 15) == 0) parts[i + (lane >> 5) + (lane >> 3 & 2)][wave] = t;
+        } else {
+            const float t = wave_sum(acc[0]);
+            if (lane == 0) parts[i][wave] = t;
+        }
+    }
+    // behind request(); a wave's sums of row i in parts[i][wave] (n_rows of them, rounded up to whole R)
+    __device__ __forceinline__ void run(const f32x4 (&x)[U][2], float (*parts)[8], int wave, int lane) {
+        for (int i = 0; i < n_rows; i += 2 * R) {
+            if (i + R < n_rows) fetch(b, i + R);
+            products(x, a, i, parts, wave, lane);
+            if (i + 2 * R < n_rows) fetch(a, i + 2 * R);
+            if (i + R < n_rows) products(x, b, i + R, parts, wave, lane);
+        }
+    }
+};
+// the sum of up to eight waves' numbers, on 16 bytes of LDS
+__device__ __forceinline__ float waves_total(const float *slot, int waves) {
+    const f32x4 lo = *reinterpret_cast<const f32x4 *>(slot), hi = *reinterpret_cast<const f32x4 *>(slot + 4);
+    float t = lo.x;
+#pragma unroll
+    for (int i = 1; i < 8; ++i) t += i < waves ? (i < 4 ? lo[i & 3] : hi[i & 3]) : 0.f;
+    return t;
+}
 
 // sum over a workgroup of NW waves; slot: NW floats of LDS
 template <int NW>

@@ -1053,14 +1053,6 @@ struct GemvFormK {
 };
 constexpr int kFormedRows = 256;  // most rows of a workgroup (a thread finishes each, so no more than its threads either)
 
-// Four values per lane -> their sums over the wave, the i-th in the sixteen lanes from 32 (i % 2) + 16 (i / 2) on: pairs fold onto one another, 10 steps instead of 24.
-__device__ __forceinline__ float four_sums(float (&v)[4]) {
-    swap_rows32(v[0], v[1]), swap_rows32(v[2], v[3]);
-    float a = v[0] + v[1], b = v[2] + v[3];
-    swap_rows16(a, b);
-    return row_sum(a + b);
-}
-
 // R rows at a time, U chunks per wave; NORM: 0 none, 1 rms, 2 layer norm; MORE as k_dense_gemv's
 template <int R, int U, int NORM, bool MORE>
 __global__ __launch_bounds__(512) void k_dense_gemv_formed(GemvFormK p) {
@@ -1134,19 +1126,8 @@ __global__ __launch_bounds__(512) void k_dense_gemv_formed(GemvFormK p) {
     }
     int mul_token = 0;
     if (mul) mul_token = e.mul_tokens[*e.mul_at];
-    // weights
-    const auto wr = bounded(a.w + (size_t)row0 * a.ld, n_rows * a.ld * 2);
-    int woff[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) woff[u] = inside[u] ? 2 * col[u] : 0x7fffffff;
-    u32x4 w0[R][U], w1[R][U];
-    auto fetch = [&](u32x4 (&w)[R][U], int i) {
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int u = 0; u < U; ++u) w[r][u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, woff[u], min(i + r, n_rows - 1) * a.ld * 2, kBufferNt));
-    };
-    fetch(w0, 0);
+    SharedRows<R, U> weights(a.w + (size_t)row0 * a.ld, n_rows, a.ld, col, inside);
+    weights.request();
     auto squares = [&](const Vec &v) {
         float ss = 0.f;
 #pragma unroll
@@ -1155,13 +1136,7 @@ __global__ __launch_bounds__(512) void k_dense_gemv_formed(GemvFormK p) {
             for (int h = 0; h < 2; ++h) ss += (v[u][h].x * v[u][h].x + v[u][h].y * v[u][h].y) + (v[u][h].z * v[u][h].z + v[u][h].w * v[u][h].w);
         return ss;
     };
-    auto total = [&](const float *slot) {
-        const f32x4 lo = *reinterpret_cast<const f32x4 *>(slot), hi = *reinterpret_cast<const f32x4 *>(slot + 4);
-        float t = lo.x;
-#pragma unroll
-        for (int i = 1; i < 8; ++i) t += i < nw ? (i < 4 ? lo[i & 3] : hi[i & 3]) : 0.f;
-        return t;
-    };
+    auto total = [&](const float *slot) { return waves_total(slot, nw); };
     const float count = (float)in.mean_n;
     auto inverse = [&](float ss) { return 1.0f / sqrtf(ss / count + in.eps); };
     if (added) {
@@ -1239,33 +1214,7 @@ __global__ __launch_bounds__(512) void k_dense_gemv_formed(GemvFormK p) {
                 if (NORM == 2 && writer && in.h_out && inside[u]) *reinterpret_cast<f32x4 *>(in.h_out + col[u] + 4 * h) = v;
             }
     }
-    auto rows = [&](const u32x4 (&w)[R][U], int i) {
-        float acc[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            acc[r] = 0.f;
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    acc[r] = fmaf(xv[u][c >> 1][2 * c & 3], __builtin_bit_cast(float, w[r][u][c] << 16), acc[r]);
-                    acc[r] = fmaf(xv[u][c >> 1][(2 * c & 3) + 1], __builtin_bit_cast(float, w[r][u][c] & 0xffff0000u), acc[r]);
-                }
-        }
-        if constexpr (R == 4) {
-            const float t = four_sums(acc);
-            if ((lane & 15) == 0) parts[i + (lane >> 5) + (lane >> 3 & 2)][wave] = t;
-        } else {
-            const float t = wave_sum(acc[0]);
-            if (lane == 0) parts[i][wave] = t;
-        }
-    };
-    for (int i = 0; i < n_rows; i += 2 * R) {
-        if (i + R < n_rows) fetch(w1, i + R);
-        rows(w0, i);
-        if (i + 2 * R < n_rows) fetch(w0, i + 2 * R);
-        if (i + R < n_rows) rows(w1, i + R);
-    }
+    weights.run(xv, parts, wave, lane);
     __syncthreads();
     if (NORM == 1) {
         inv = inverse(total(slots[2]));

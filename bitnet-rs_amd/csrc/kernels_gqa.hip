@@ -900,6 +900,83 @@ hipError_t launch_gqa_out(const GqaOut &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Up to eight records on the lanes of k_dense_gemv_formed (dense.hpp, SharedRows): each merges the records of its own eight columns in registers, for all rows of its workgroup, and nothing goes
+// through LDS ahead of the products.  As above nothing that is requested hangs on the position.
+struct GqaProjectK {
+    Gqa g;
+    const int *pos;
+    const float *scratch, *bias;
+    const uint16_t *w;
+    float *y;
+    int rows, ld, rows_wg;
+    unsigned magic;  // ceil(2^20 / eights of a head)
+};
+constexpr int kProjectRows = 64;
+
+template <int NB>
+__global__ __launch_bounds__(512) void k_gqa_project(GqaProjectK p) {
+    __shared__ __attribute__((aligned(16))) float parts[kProjectRows + 4][8];
+    const Gqa &g = p.g;
+    const int here = *p.pos;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), vdimp = (int)g.vdimp, n = (int)g.heads * vdimp;
+    const unsigned stride = kGqaRecHead + vdimp;
+    const int row0 = blockIdx.x * p.rows_wg, n_rows = min(p.rows_wg, p.rows - row0);
+    const int at = wave * 512 + lane * 8, col[1] = {min(at, n - 8)}, head = (int)((unsigned)(col[0] >> 3) * p.magic >> 20);
+    const bool inside[1] = {at < n};
+    const float *rec = p.scratch + (unsigned)head * (kGqaSplits * stride), *v = rec + kGqaRecHead + (col[0] - head * vdimp);
+    float2 ml[NB];
+    f32x4 vec[NB][2], zc[2];
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+        ml[e] = *reinterpret_cast<const float2 *>(rec + e * stride);
+        vec[e][0] = *reinterpret_cast<const f32x4 *>(v + e * stride), vec[e][1] = *reinterpret_cast<const f32x4 *>(v + e * stride + 4);
+    }
+    const float sink = g.sink ? g.sink[head] * kLog2e : -INFINITY, z = g.gate && !g.gate_columns ? ((const float *)g.gate)[head] : 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) zc[h] = g.gate && g.gate_columns ? *reinterpret_cast<const f32x4 *>((const float *)g.gate + col[0] + 4 * h) : f32x4{0.f, 0.f, 0.f, 0.f};
+    const float bias = p.bias && tid < n_rows ? p.bias[row0 + tid] : 0.f;
+    SharedRows<4, 1> weights(p.w + (size_t)row0 * p.ld, n_rows, p.ld, col, inside);
+    weights.request();
+    const int used = gqa_range(g, here).used;
+    float M = sink;
+#pragma unroll
+    for (int e = 0; e < NB; ++e) M = e < used ? fmaxf(M, ml[e].x) : M;
+    float den = g.sink ? exp2f(sink - M) : 0.f;
+    f32x4 x[1][2] = {{f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}}};
+#pragma unroll
+    for (int e = 0; e < NB; ++e) {
+        if (e >= used) continue;
+        const float w = exp2f(ml[e].x - M);
+        den += w * ml[e].y;
+        x[0][0] += w * vec[e][0], x[0][1] += w * vec[e][1];
+    }
+    const float f = (g.gate && !g.gate_columns ? activate(z, BITNET_HIP_ACT_SIGMOID) : 1.0f) / den;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        x[0][h] *= f;
+        if (g.gate && g.gate_columns)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x[0][h][c] *= activate(zc[h][c], BITNET_HIP_ACT_SIGMOID);
+        if (!inside[0]) x[0][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    weights.run(x, parts, wave, lane);
+    __syncthreads();
+    if (tid < n_rows) p.y[row0 + tid] = waves_total(parts[tid], (int)blockDim.x >> 6) + bias;
+}
+
+int gqa_project_records(const Gqa &g, int cols) { return g.maps != 1 || g.heads * g.vdimp > 4096 || (size_t)cols < g.heads * g.vdimp || (g.gate && !g.gate_f32) ? 0 : 12; }
+
+hipError_t launch_gqa_project(const GqaOut &a, hipStream_t s) {
+    if (a.records < 1 || a.records > gqa_project_records(a.g, a.cols)) return hipErrorInvalidValue;
+    GqaProjectK k;
+    k.g = a.g, k.pos = a.pos, k.scratch = a.scratch, k.bias = a.bias, k.w = a.w, k.y = a.y, k.rows = a.rows, k.ld = a.ld;
+    k.magic = ((1u << 20) + a.g.vdimp / 8 - 1) / (unsigned)(a.g.vdimp / 8);
+    const int waves = ((int)(a.g.heads * a.g.vdimp) + 511) / 512;
+    k.rows_wg = std::min({(a.rows + 1023) / 1024 * 4, kProjectRows, 64 * waves});
+    hipLaunchKernelGGL(a.records <= 2 ? k_gqa_project<2> : a.records <= 4 ? k_gqa_project<4> : a.records <= 8 ? k_gqa_project<8> : k_gqa_project<12>, dim3((a.rows + k.rows_wg - 1) / k.rows_wg), dim3(64 * waves), 0, s, k);
+    return hipGetLastError();
+}
+
 // ---- prompt -----------------------------------------------------------------------------------------------------------
 // One workgroup: one head, four waves; a wave holds two slots of 16 queries: both maps of one query tile, or two tiles of the only map.  Key tiles
 // of 64 (every map's) and the values of the tile staged through registers into LDS one step ahead.

@@ -167,7 +167,7 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
     const int p = position();
     hipStream_t s = (hipStream_t)stream_;
     if (use_graph) {
-        for (int i = 0; i < n; ++i) {  // every form this run needs (at most three captures)
+        for (int i = 0; i < n; ++i) {  // every form this run needs
             int rc = ensure_graph(with_logits, form_at(p + i));
             if (rc) return rc;
         }

@@ -110,7 +110,7 @@ class Sequence {
     int32_t *pinned_ = nullptr;
     bool staged_ = false;
     Event begin_, end_;  // of the last run or prefill
-    static constexpr int kForms = 3;
+    static constexpr int kForms = 5;
     void *graph_exec_[2 * kForms] = {};  // [2 * form + with_logits]
     void *graph_[2 * kForms] = {};
 };

@@ -10,8 +10,8 @@
 namespace bitnet_host {
 
 namespace {
-// Records that a step's output products merge themselves, 128 keys each: one form of the step for up to two of them, one for up to four, all that is faster than a launch of its own.
-constexpr size_t kFewRecords = 2, kMostRecords = 4;
+// Forms of a step: 0, the attention's records are merged by a launch of their own; else by the output products, up to so many of them, 128 keys each
+constexpr size_t kStepRecords[] = {0, 2, 4, 8, 12}, kMostRecords = 12;
 constexpr size_t kDecodeSlice = 64;  // queries per call where a portion takes a decode form of its attention
 size_t up_to(size_t v, size_t a) { return (v + a - 1) / a * a; }
 }  // namespace
@@ -764,7 +764,7 @@ bool StackModel::merges_in_out(size_t i, int which) const {
     const Block &B = layers_[i].block[which];
     if (f32_ || !B.used || !B.mixer || spec_.layers[i].mixer != LayerSpec::Attention || B.fs > 0 || B.expert_up.w) return false;
     const bitnet_hip_gqa a = gqa_args(i, 0, row_[0], B.main, true);
-    return bitnet_hip_gqa_out_records(&a, B.out.cols) >= kMostRecords;
+    return bitnet_hip_gqa_supported(a.dimp, a.vdimp) && bitnet_hip_gqa_project_records(&a, B.out.cols) >= kMostRecords;
 }
 
 // records of a query at the position, over the layers
@@ -780,9 +780,15 @@ size_t StackModel::records_at(int pos) const {
     return most;
 }
 
+// (up to twelve records: us of attention and product at 300 / 600 / 1500 keys, merged by a launch / by the product: 12 heads of 128 on 3 14.1 / 14.1 / 14.2 -> 11.9 / 12.2 / 13.0, 24 on 6
+// 17.2 / 17.2 / 17.4 -> 14.3 / 15.3 / 16.2, 32 on 8 at 1500 19.8 -> 19.4; with sixteen requested at once and the rest in turn even at 17, slower from there on.  Records of 256 keys, from twice the
+// waves, would reach 3072 keys: 14.7 -> 13.7 where the keys lie in the L2, but a pass's steps got slower, 7.50 -> 7.69 ms)
 int StackModel::form_at(int pos) const {
     const size_t n = records_at(pos);
-    return n == 0 || n > kMostRecords ? 0 : n <= kFewRecords ? 1 : 2;
+    static_assert(sizeof(kStepRecords) / sizeof(kStepRecords[0]) == kForms, "a graph for each");
+    for (int f = 1; n > 0 && f < kForms; ++f)
+        if (n <= kStepRecords[f]) return f;
+    return 0;
 }
 
 // the sublayers of a block; their sum is left in y_[which]
@@ -816,15 +822,16 @@ int StackModel::step_block(size_t i, int pass, int which) {
         TRY(step_attend_latent(i, pass, proj, S.latent.kv_from < 0 ? &r : nullptr, row, B.ko));
     } else if (B.mixer && S.mixer == LayerSpec::Attention) {
         const bitnet_hip_gqa a = gqa_args(i, pass, proj, B.main, true);
+        if (form_ > 0 && merges_in_out(i, which)) {
+            BCHK(bitnet_hip_gqa_step_dev(&a, proj, pos_, scratch_, stream_));
+            BCHK(bitnet_hip_gqa_project_dev(&a, pos_, kStepRecords[form_], scratch_, B.out.w, B.out.rows, B.out.cols, B.out.ld, B.out_bias, y_[which], stream_));
+            return 0;
+        }
         if (!f32_ && bitnet_hip_gqa_supported(a.dimp, a.vdimp)) {
             BCHK(bitnet_hip_gqa_step_dev(&a, proj, pos_, scratch_, stream_));
         } else {
             BCHK(bitnet_hip_gqa_rows_dev(&a, proj, B.main, 1, f32_, pos_, 1, nullptr, 0, stream_));
             BCHK(bitnet_hip_gqa_any_dev(&a, proj, B.main, 1, f32_, pos_, 0, 1, scratch_, stream_));
-        }
-        if (records_ > 0 && merges_in_out(i, which)) {
-            BCHK(bitnet_hip_gqa_out_dev(&a, pos_, records_, scratch_, B.out.w, B.out.rows, B.out.cols, B.out.ld, B.out_bias, y_[which], stream_));
-            return 0;
         }
         BCHK(bitnet_hip_gqa_merge_dev(&a, pos_, 0, 1, scratch_, row, B.ko, 0, stream_));
     } else if (B.mixer) {
@@ -904,7 +911,7 @@ int StackModel::embed_rows(size_t n, float *out) {
 }
 
 int StackModel::step(bool with_logits, int form) {
-    records_ = form == 0 ? 0 : form == 1 ? kFewRecords : kMostRecords;
+    form_ = form;
     cur_ = x0_;
     row_at_ = 0;
     pending_ = Pending();

@@ -150,7 +150,7 @@ class StackModel : public Sequence {
   protected:
     bool ready() const override { return head_ != nullptr && layers_set_ == spec_.layers.size(); }
     int step(bool with_logits, int form) override;
-    int form_at(int pos) const override;  // 0: the attention's records are merged by a launch of their own; 1, 2: by the output products, up to kFewRecords, kMostRecords of them
+    int form_at(int pos) const override;  // how a step's attention records are merged: kStepRecords
     int clear_state() override;
 
   private:
@@ -306,7 +306,7 @@ class StackModel : public Sequence {
     float *x_[2] = {nullptr, nullptr}, *z_ = nullptr, *q_ = nullptr, *qabs_ = nullptr, *att_ = nullptr, *y_[2] = {nullptr, nullptr}, *act_ = nullptr,
           *lin_ = nullptr, *lino_ = nullptr, *scratch_ = nullptr;
     void *argmax_ = nullptr;
-    size_t records_ = 0;  // of the step at hand: merged by the output products; 0: by a launch of their own
+    int form_ = 0;  // of the step at hand
     int row_at_ = 0;  // the row the last block used: its residual gate is read while the next block's is written
     const float *cur_ = nullptr;  // where the step's residual stream is
     float *next_x() const { return cur_ == x_[0] ? x_[1] : x_[0]; }

@@ -828,6 +828,10 @@ int bitnet_hip_gqa_merge_dev(const bitnet_hip_gqa *attn, const int32_t *pos_dev,
 size_t bitnet_hip_gqa_out_records(const bitnet_hip_gqa *attn, size_t cols);
 int bitnet_hip_gqa_out_dev(const bitnet_hip_gqa *attn, const int32_t *pos_dev, size_t records, const float *scratch_dev, const uint16_t *w_dev, size_t rows,
                            size_t cols, size_t ld, const float *bias_dev, float *y_dev, void *stream);
+/* The same for more records (at most gqa_project_records) and weights on 16 bytes. */
+size_t bitnet_hip_gqa_project_records(const bitnet_hip_gqa *attn, size_t cols);
+int bitnet_hip_gqa_project_dev(const bitnet_hip_gqa *attn, const int32_t *pos_dev, size_t records, const float *scratch_dev, const uint16_t *w_dev, size_t rows,
+                               size_t cols, size_t ld, const float *bias_dev, float *y_dev, void *stream);
 /* A portion of a prompt, bf16: the LAST nq of n_ctx positions attend (all of them in the caches); q as gqa_rows leaves it. */
 int bitnet_hip_gqa_prefill_dev(const bitnet_hip_gqa *attn, const uint16_t *q_dev, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out_dev, size_t ldo,
                                void *stream);
