@@ -178,6 +178,9 @@ __global__ __launch_bounds__(NW * 64) void k_gemv_q(GemvQArgs p) {
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
             int e = 4 * (tid + NT * i);
+            // (a whole wave past the columns asks for nothing and merges nothing: at 2560 of them that is the second slot of six of eight waves, us per launch at 129 to 192 keys 5.3 -> 5.0; ten waves
+            // with a slot each give another 0.1)
+            if (i > 0 && 4 * (wave * 64 + NT * i) >= p.cols) break;
             e = e < p.cols ? e : p.cols - 4;
             const int h = e >> 7, d = e & 127, kvh = h >> p.attn_group_log2, hg = h & ((1 << p.attn_group_log2) - 1);
             const float *rb = p.attn_rec + (size_t)kvh * p.attn_chunks_max * kAttnRecFloats;
@@ -245,6 +248,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemv_q(GemvQArgs p) {
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
             const int e = 4 * (tid + NT * i);
+            if (i > 0 && 4 * (wave * 64 + NT * i) >= p.cols) break;
             // softmax merge: out = sum_c e^(m_c - M) o_c / sum_c e^(m_c - M) l_c   (k_attn_combine's value)
             float M = -INFINITY;
 #pragma unroll
