@@ -658,6 +658,13 @@ class HipLib:
     def gqa_prefill_dev(self, a: "Gqa", q, ldq: int, n_ctx: int, nq: int, out, ldo: int, stream: int = 0) -> None:
         self._call("gqa_prefill_dev", C.byref(a), _ptr(q), _sz(ldq), _sz(n_ctx), _sz(nq), _ptr(out), _sz(ldo), _vp(stream))
 
+    def gqa_prefill_scratch_bytes(self, a: "Gqa", n_ctx: int, nq: int) -> int:
+        self.c.bitnet_hip_gqa_prefill_scratch_bytes.restype = _sz
+        return int(self.c.bitnet_hip_gqa_prefill_scratch_bytes(C.byref(a), _sz(n_ctx), _sz(nq)))
+
+    def gqa_prefill_scratch_dev(self, a: "Gqa", q, ldq: int, n_ctx: int, nq: int, out, ldo: int, scratch, scratch_bytes: int, stream: int = 0) -> None:
+        self._call("gqa_prefill_scratch_dev", C.byref(a), _ptr(q), _sz(ldq), _sz(n_ctx), _sz(nq), _ptr(out), _sz(ldo), _optr(scratch), _sz(scratch_bytes), _vp(stream))
+
     def gqa_prefill_last_groups(self) -> int:
         return int(self.c.bitnet_hip_gqa_prefill_last_groups())
 

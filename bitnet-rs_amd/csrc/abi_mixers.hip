@@ -181,16 +181,33 @@ int bitnet_hip_gqa_project_dev(const bitnet_hip_gqa *a, const int32_t *pos, size
 
 int bitnet_hip_gqa_prefill_last_groups(void) { return g_last_gqa_groups; }
 
-int bitnet_hip_gqa_prefill_dev(const bitnet_hip_gqa *a, const uint16_t *q, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out, size_t ldo, void *stream) {
-    BH_GUARD_BEGIN
+static int gqa_prefill(const bitnet_hip_gqa *a, const uint16_t *q, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out, size_t ldo, float *scratch, hipStream_t stream) {
     if (int rc = check_gqa(a)) return rc;
     BH_REQUIRE(q && out && nq > 0 && nq <= n_ctx && n_ctx <= a->capacity && ldq % 8 == 0 && ldq >= a->heads * a->maps * a->dimp && ldo % 4 == 0 &&
                    ldo >= a->heads * a->vdimp,
                "gqa_prefill: bad arguments");
     BH_CHECK_DIMS(nq, ldq);
     if (!gqa_supported((int)a->dimp, (int)a->vdimp)) return set_error(BITNET_HIP_ERR_UNSUPPORTED, "gqa_prefill: head of %zu / %zu columns", a->dimp, a->vdimp);
-    BH_HIP_TRY(launch_gqa_prefill(*a, q, ldq, (int)n_ctx, (int)nq, out, ldo, (hipStream_t)stream));
+    BH_HIP_TRY(launch_gqa_prefill(*a, q, ldq, (int)n_ctx, (int)nq, out, ldo, scratch, stream));
     return BITNET_HIP_OK;
+}
+
+int bitnet_hip_gqa_prefill_dev(const bitnet_hip_gqa *a, const uint16_t *q, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out, size_t ldo, void *stream) {
+    BH_GUARD_BEGIN
+    return gqa_prefill(a, q, ldq, n_ctx, nq, out, ldo, nullptr, (hipStream_t)stream);
+    BH_GUARD_END
+}
+
+size_t bitnet_hip_gqa_prefill_scratch_bytes(const bitnet_hip_gqa *a, size_t n_ctx, size_t nq) {
+    if (!a || check_gqa(a) != 0 || nq == 0 || nq > n_ctx || n_ctx > a->capacity || !gqa_supported((int)a->dimp, (int)a->vdimp)) return 0;
+    return gqa_prefill_floats(*a, (int)n_ctx, (int)nq) * sizeof(float);
+}
+
+int bitnet_hip_gqa_prefill_scratch_dev(const bitnet_hip_gqa *a, const uint16_t *q, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out, size_t ldo, float *scratch, size_t scratch_bytes, void *stream) {
+    BH_GUARD_BEGIN
+    const size_t bytes = bitnet_hip_gqa_prefill_scratch_bytes(a, n_ctx, nq);
+    BH_REQUIRE(bytes == 0 || (scratch && (uintptr_t)scratch % 16 == 0 && scratch_bytes >= bytes), "gqa_prefill: scratch of %zu bytes, %zu needed", scratch_bytes, bytes);
+    return gqa_prefill(a, q, ldq, n_ctx, nq, out, ldo, bytes ? scratch : nullptr, (hipStream_t)stream);
     BH_GUARD_END
 }
 

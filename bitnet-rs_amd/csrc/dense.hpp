@@ -244,7 +244,8 @@ hipError_t launch_gqa_out(const GqaOut &a, hipStream_t s);
 int gqa_project_records(const Gqa &g, int cols);
 hipError_t launch_gqa_project(const GqaOut &a, hipStream_t s);
 extern thread_local int g_last_gqa_groups;  // groups of four waves per workgroup of launch_gqa_prefill's last launch on this thread
-hipError_t launch_gqa_prefill(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, hipStream_t s);
+size_t gqa_prefill_floats(const Gqa &g, int n_ctx, int nq);
+hipError_t launch_gqa_prefill(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, float *records, hipStream_t s);
 bool delta_supported(int dimp, int vdimp);
 bool delta_chunked_supported(int dimp, int vdimp);
 size_t delta_workspace_bytes(size_t n, size_t heads, size_t dimp, size_t vdimp);

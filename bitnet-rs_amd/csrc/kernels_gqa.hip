@@ -984,8 +984,9 @@ hipError_t launch_gqa_project(const GqaOut &a, hipStream_t s) {
 // first next to none: with one group per workgroup the longest walk takes 2.6 us a tile whatever its neighbour does, with two it is half as long at 4.1 us a step.
 // Heads that need more than 256 registers keep one group; two_groups says when the others take two.
 // FAR: with a distance penalty, gates per column, or both.
+// records: gridDim.y workgroups share a block's tiles of keys, in stretches, and each leaves its outputs, maxima and sums for k_gqa_merge_parts (which counts the sink).
 template <int NK, int NV, int MAPS, bool FAR, int G>
-__global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(Gqa p, const uint16_t *Q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, int n_qb) {
+__global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(Gqa p, const uint16_t *Q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, int n_qb, float *records) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int SLOTS = 2, QW = 16 * SLOTS / MAPS, KS = NK * 64 + 16, VS = 64 * 2 + 16, NVL = NV / 2;
     const int grp = G == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
@@ -1018,7 +1019,7 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
 #pragma unroll
     for (int t = 0; t < SLOTS; ++t) {
         // (finite: with chunks a tile may hold no key that a query sees; the sink counts once per query, four lanes share one)
-        m[t] = MAPS == 1 && p.sink && grp == 0 ? p.sink[h] * kLog2e : -1e30f, l[t] = MAPS == 1 && p.sink && g == 0 && grp == 0 ? 1.0f : 0.f;
+        m[t] = MAPS == 1 && p.sink && grp == 0 && !records ? p.sink[h] * kLog2e : -1e30f, l[t] = MAPS == 1 && p.sink && g == 0 && grp == 0 && !records ? 1.0f : 0.f;
 #pragma unroll
         for (int v = 0; v < NV; ++v) o[v][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -1040,11 +1041,16 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
         for (int j = 0; j < NVL; ++j)
             if (j * 32 < vdimp) vreg[j] = *reinterpret_cast<const u32x4 *>(vb + (size_t)j * 64 * p.capacity + voff);
     };
-    const int n_tiles = (min(n_ctx, pos0 + q0 + 4 * QW) + 63) / 64;
+    int n_tiles = (min(n_ctx, pos0 + q0 + 4 * QW) + 63) / 64;
     const FarPenalty far = far_penalty(p, h);
     // tiles from the first key of the workgroup's first query on; a wave leaves out what lies ahead of its own first key
-    const int t_first = gqa_first(p, pos0 + q0) >> 6, w_first = gqa_first(p, pos0 + qw), w_last = gqa_first(p, pos0 + qw + QW - 1);
-    fetch(min(t_first + grp, n_tiles - 1) * 64);
+    int t_first = gqa_first(p, pos0 + q0) >> 6;
+    const int w_first = gqa_first(p, pos0 + qw), w_last = gqa_first(p, pos0 + qw + QW - 1);
+    if (records) {
+        const int each = (n_tiles - t_first + (int)gridDim.y - 1) / (int)gridDim.y;
+        t_first = min(t_first + (int)blockIdx.y * each, n_tiles), n_tiles = min(t_first + each, n_tiles);
+    }
+    fetch(max(min(t_first + grp, n_tiles - 1), 0) * 64);
     for (int t0 = t_first; t0 < n_tiles; t0 += G) {
         const int kt0 = t0 + grp, key0 = kt0 * 64;
         __syncthreads();
@@ -1157,10 +1163,24 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
         for (int t = 0; t < SLOTS; ++t) {
             const float2 b = pm[(wave * SLOTS + t) * 64 + lane];
             const float mx = fmaxf(m[t], b.x), wa = __builtin_amdgcn_exp2f(m[t] - mx), wb = __builtin_amdgcn_exp2f(b.x - mx);
-            l[t] = l[t] * wa + b.y * wb;
+            m[t] = mx, l[t] = l[t] * wa + b.y * wb;
 #pragma unroll
             for (int v = 0; v < NV; ++v) o[v][t] = o[v][t] * wa + po[((wave * SLOTS + t) * NV + v) * 64 + lane] * wb;
         }
+    }
+    if (records) {
+#pragma unroll
+        for (int t = 0; t < SLOTS; ++t) {
+            const int qi = qw + t / MAPS * 16 + r16;
+            const float sum = rows_sum(l[t]);
+            if (qi >= nq) continue;
+            float *rec = records + ((((size_t)qi * heads + h) * MAPS + t % MAPS) * gridDim.y + blockIdx.y) * (kGqaRecHead + vdimp);
+            if (g == 0) rec[0] = m[t], rec[1] = sum;
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                if (v * 16 < vdimp) *reinterpret_cast<f32x4 *>(rec + kGqaRecHead + v * 16 + g * 4) = o[v][t];
+        }
+        return;
     }
     float inv[SLOTS], gate[SLOTS / MAPS];
 #pragma unroll
@@ -1219,11 +1239,71 @@ static bool two_groups(const Gqa &g, int rows, int n_ctx, int nq) {
     return longest >= 4 && 16 * total <= 17 * at_once * longest && 10 * second <= 11 * longest;
 }
 
+// The records of a query's head (gridDim.y of the launch above, one behind the other for every map) -> its output: a wave each, vdimp / 4 lanes of four columns, as many groups of them as fit a wave
+// sharing the records.
+template <int MAPS>
+__global__ __launch_bounds__(256) void k_gqa_merge_parts(Gqa p, const float *records, int parts, int nq, uint16_t *out, size_t ldo) {
+    const int lane = threadIdx.x & 63, at = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), heads = (int)p.heads, vdimp = (int)p.vdimp;
+    if (at >= nq * heads) return;
+    const int qi = at / heads, h = at - qi * heads, lanes = vdimp >> 2, groups = 64 / lanes, grp = lane / lanes, c = (lane - grp * lanes) * 4;
+    const size_t stride = kGqaRecHead + vdimp;
+    const float *rec = records + (size_t)at * MAPS * parts * stride;
+    f32x4 v[MAPS], z = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (p.gate)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z[e] = gate_logit(p, qi, h, c + e);
+    const float sink = p.sink ? p.sink[h] * kLog2e : -1e30f;
+#pragma unroll
+    for (int j = 0; j < MAPS; ++j) {
+        const float *r = rec + (size_t)j * parts * stride;
+        const float m = lane < parts ? r[lane * stride] : -1e30f, l = lane < parts ? r[lane * stride + 1] : 0.f;
+        const float M = fmaxf(sink, rows_max(row_max(m))), w = __builtin_amdgcn_exp2f(m - M);
+        v[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int i0 = 0; i0 < parts; i0 += groups) {  // (all lanes take part; past the last record the weight is zero)
+            const int i = i0 + grp;
+            v[j] += __shfl(w, min(i, 63), 64) * *reinterpret_cast<const f32x4 *>(r + min(i, parts - 1) * stride + kGqaRecHead + c);
+        }
+        f32x4 t = v[j];
+        const float den = wave_sum(w * l) + (p.sink ? __builtin_amdgcn_exp2f(sink - M) : 0.f);
+        for (int o = 1; o < groups; ++o)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) t[e] += __shfl(v[j][e], lane + o * lanes, 64);
+        v[j] = t * (1.0f / den);
+    }
+    f32x4 q = v[0];
+    if (MAPS == 2) {
+        q -= p.lambda * v[MAPS - 1];
+        q *= p.out_scale / sqrtf(wave_sum(grp == 0 ? (q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w) : 0.f) / (float)p.vdim + p.eps);
+    }
+    if (p.gate)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] *= activate(z[e], BITNET_HIP_ACT_SIGMOID);
+    if (grp == 0) *reinterpret_cast<bf16x4 *>(out + (size_t)qi * ldo + (size_t)h * vdimp + c) = bf16x4{(__bf16)q.x, (__bf16)q.y, (__bf16)q.z, (__bf16)q.w};
+}
+
+// Few queries behind many keys: a launch whose blocks leave CUs without a workgroup lasts as long as its longest walk, so a block's tiles are cut into stretches, of two tiles (a step of two
+// groups) at least and no more of them than there are CUs for (heads count as a multiple of eight, as the launch deals them to the XCDs: 12 heads in 21 stretches take 32 us where 15 take 24).
+// A step of a walk takes 4.1 us, the launch that puts the records together 5 and 0.8 ns for each query's head and map.  us without / with, heads, keys, queries: 12, 2090, 90 64 / 20; 24, 2090, 90
+// 64 / 24; 12, 600, 20 22.6 / 12.8; 12, 1000, 200 34.2 / 19.7; 12, 450, 130 20.7 / 15.8; 12, 1000, 1000 34.6 / 31.5; 12, 8000, 30 214 / 38; 24 of two maps, 2090, 90 59 / 30; 2 of 256 columns,
+// 2000, 50 162 / 24.  Queries without many keys stay: 24, 1531, 1531 50, in two stretches where CUs hold two workgroups 52; 12, 100, 3 8.4.
+static int gqa_prefill_parts(const Gqa &g, int n_ctx, int nq) {
+    const int rows = g.maps == 2 ? 64 : 128, blocks = (nq + rows - 1) / rows, heads = ((int)g.heads + 7) / 8 * 8;
+    const int tiles = (n_ctx + 63) / 64 - (gqa_first(g, n_ctx - nq + (blocks - 1) * rows) >> 6), most = std::min<long>(256 / ((long)heads * blocks), 32);
+    if (most < 2) return 1;
+    const int each = ((tiles + most - 1) / most + 1) & ~1, saved = (tiles + 1) / 2 - each / 2;
+    return 4.1 * saved > 5.0 + 8e-4 * (double)nq * (double)(g.heads * g.maps) ? (tiles + each - 1) / each : 1;
+}
+size_t gqa_prefill_floats(const Gqa &g, int n_ctx, int nq) {
+    const int parts = gqa_prefill_parts(g, n_ctx, nq);
+    return parts > 1 ? (size_t)nq * g.heads * g.maps * parts * (kGqaRecHead + g.vdimp) : 0;
+}
+
 template <int NK, int NV, int G>
-static hipError_t gqa_prefill_go(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, hipStream_t s) {
-    const int rows = g.maps == 2 ? 64 : 128, n_qb = (nq + rows - 1) / rows;
+static hipError_t gqa_prefill_go(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, float *records, hipStream_t s) {
+    const int rows = g.maps == 2 ? 64 : 128, n_qb = (nq + rows - 1) / rows, parts = records ? gqa_prefill_parts(g, n_ctx, nq) : 1;
     if constexpr (G == 2)
-        if (!two_groups(g, rows, n_ctx, nq)) return gqa_prefill_go<NK, NV, 1>(g, q, ldq, n_ctx, nq, out, ldo, s);
+        if (parts == 1 && !two_groups(g, rows, n_ctx, nq)) return gqa_prefill_go<NK, NV, 1>(g, q, ldq, n_ctx, nq, out, ldo, nullptr, s);
     g_last_gqa_groups = G;
     const size_t tiles = G * ((size_t)g.maps * 64 * (NK * 64 + 16) + (size_t)NV * 16 * (64 * 2 + 16)), sums = G == 2 ? (size_t)4 * 2 * 64 * (NV * 16 + 8) : 0;
     const size_t lds = tiles > sums ? tiles : sums;
@@ -1232,16 +1312,20 @@ static hipError_t gqa_prefill_go(const Gqa &g, const uint16_t *q, size_t ldq, in
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(fn, dim3(8 * ((g.heads + 7) / 8) * n_qb), dim3(256 * G), lds, s, g, q, ldq, n_ctx, nq, out, ldo, n_qb);
+    hipLaunchKernelGGL(fn, dim3(8 * ((g.heads + 7) / 8) * n_qb, parts), dim3(256 * G), lds, s, g, q, ldq, n_ctx, nq, out, ldo, n_qb, parts > 1 ? records : nullptr);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || parts == 1) return e;
+    hipLaunchKernelGGL(g.maps == 2 ? k_gqa_merge_parts<2> : k_gqa_merge_parts<1>, dim3((nq * (int)g.heads + 3) / 4), dim3(256), 0, s, g, records, parts, nq, out, ldo);
     return hipGetLastError();
 }
 
-hipError_t launch_gqa_prefill(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, hipStream_t s) {
+// records: gqa_prefill_floats(g, n_ctx, nq) of them, or none where a block's keys stay together
+hipError_t launch_gqa_prefill(const Gqa &g, const uint16_t *q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, float *records, hipStream_t s) {
     if (!gqa_supported((int)g.dimp, (int)g.vdimp)) return hipErrorInvalidValue;
-    if (g.dimp <= 64 && g.vdimp <= 64) return gqa_prefill_go<2, 4, 2>(g, q, ldq, n_ctx, nq, out, ldo, s);
-    if (g.dimp <= 64 && g.vdimp <= 128) return gqa_prefill_go<2, 8, 2>(g, q, ldq, n_ctx, nq, out, ldo, s);
-    if (g.dimp <= 128 && g.vdimp <= 128) return gqa_prefill_go<4, 8, 2>(g, q, ldq, n_ctx, nq, out, ldo, s);
-    return gqa_prefill_go<8, 16, 1>(g, q, ldq, n_ctx, nq, out, ldo, s);
+    if (g.dimp <= 64 && g.vdimp <= 64) return gqa_prefill_go<2, 4, 2>(g, q, ldq, n_ctx, nq, out, ldo, records, s);
+    if (g.dimp <= 64 && g.vdimp <= 128) return gqa_prefill_go<2, 8, 2>(g, q, ldq, n_ctx, nq, out, ldo, records, s);
+    if (g.dimp <= 128 && g.vdimp <= 128) return gqa_prefill_go<4, 8, 2>(g, q, ldq, n_ctx, nq, out, ldo, records, s);
+    return gqa_prefill_go<8, 16, 1>(g, q, ldq, n_ctx, nq, out, ldo, records, s);
 }
 
 }  // namespace bitnet_hip

@@ -1129,7 +1129,9 @@ int StackModel::portion_block(size_t i, int pass, int which, size_t n, size_t po
         BCHK(bitnet_hip_gqa_rows_dev(&a, proj, ld, f32_, f32_, pos_, n, conv ? pqc_.p : nullptr, ldq, stream_));
         if (conv) BCHK(bitnet_hip_conv_keep_dev(proj, ld, f32_, L.channels, a.taps, L.slots[(size_t)pass].ring, pos_, n, stream_));
         if (!f32_ && bitnet_hip_gqa_supported(a.dimp, a.vdimp)) {
-            BCHK(bitnet_hip_gqa_prefill_dev(&a, (const uint16_t *)q, ldq, pos0 + n, n, (uint16_t *)row, ld, stream_));
+            const size_t bytes = bitnet_hip_gqa_prefill_scratch_bytes(&a, pos0 + n, n);
+            TRY(grow(pscratch_, bytes));
+            BCHK(bitnet_hip_gqa_prefill_scratch_dev(&a, (const uint16_t *)q, ldq, pos0 + n, n, (uint16_t *)row, ld, (float *)pscratch_.p, pscratch_.bytes, stream_));
         } else {
             for (size_t s = 0; s < n; s += kDecodeSlice) {
                 const size_t k = std::min(kDecodeSlice, n - s);
