@@ -233,18 +233,46 @@ int bitnet_hip_dense_gemv_dev(const bitnet_hip_vector_input *input, const uint16
     BH_GUARD_END
 }
 
-int bitnet_hip_dense_logits_dev(const bitnet_hip_vector_input *input, const uint16_t *w, size_t vocab, size_t cols, size_t ld, float *logits,
-                                void *scratch, int32_t *token, int32_t *pos, int32_t *history, const int32_t *n_forced, void *stream) {
-    BH_GUARD_BEGIN
+static EmbedNext to_embed_next(const bitnet_hip_embedding &e) {
+    EmbedNext o;
+    o.table = e.table, o.ld = e.ld, o.width = (int)e.width, o.vocab = (int)e.vocab, o.scale = e.scale, o.eps = e.eps, o.norm_w = e.norm_weight, o.out = e.out;
+    o.pairs.table = e.pairs, o.pairs.ld = e.pairs ? e.ld_pairs : 0, o.pairs.buckets = e.buckets, o.pairs.mul_prev = e.mul_prev, o.pairs.mul_cur = e.mul_cur;
+    return o;
+}
+int bitnet_hip_embedding_follows(const bitnet_hip_embedding *e) {
+    return e && e->table && e->out && e->width <= 4096 && e->vocab > 0 && e->vocab < (size_t(1) << 31) && e->ld >= e->width &&
+           (!e->pairs || (e->ld_pairs >= e->width && e->buckets > 0 && e->mul_prev < (uint64_t(1) << 31) && e->mul_cur < (uint64_t(1) << 31))) && embed_follows(to_embed_next(*e));
+}
+
+static int dense_logits(const bitnet_hip_vector_input *input, const uint16_t *w, size_t vocab, size_t cols, size_t ld, float *logits, void *scratch, int32_t *token, int32_t *pos,
+                        int32_t *history, const int32_t *n_forced, const bitnet_hip_embedding *next, hipStream_t stream) {
     GemvArgs g;
     BH_REQUIRE(scratch, "Null pointer passed to dense_logits_dev");
+    BH_REQUIRE(!next || (pos && history && bitnet_hip_embedding_follows(next)), "dense_logits: an embedding row that cannot follow");
     if (int rc = gemv_args(input, w, vocab, cols, ld, logits, g)) return rc;
     g.best_val = static_cast<float *>(scratch);
     g.best_idx = reinterpret_cast<int *>(g.best_val + 1024);
     int n_wg = 0;
-    BH_HIP_TRY(launch_dense_gemv(g, &n_wg, (hipStream_t)stream));
-    if (token || pos) BH_HIP_TRY(launch_argmax_final(g.best_val, g.best_idx, n_wg, token, pos, history, n_forced, (hipStream_t)stream));
+    BH_HIP_TRY(launch_dense_gemv(g, &n_wg, stream));
+    if (next)
+        BH_HIP_TRY(launch_argmax_embed(g.best_val, g.best_idx, n_wg, token, pos, history, n_forced, to_embed_next(*next), stream));
+    else if (token || pos)
+        BH_HIP_TRY(launch_argmax_final(g.best_val, g.best_idx, n_wg, token, pos, history, n_forced, stream));
     return BITNET_HIP_OK;
+}
+
+int bitnet_hip_dense_logits_dev(const bitnet_hip_vector_input *input, const uint16_t *w, size_t vocab, size_t cols, size_t ld, float *logits,
+                                void *scratch, int32_t *token, int32_t *pos, int32_t *history, const int32_t *n_forced, void *stream) {
+    BH_GUARD_BEGIN
+    return dense_logits(input, w, vocab, cols, ld, logits, scratch, token, pos, history, n_forced, nullptr, (hipStream_t)stream);
+    BH_GUARD_END
+}
+
+int bitnet_hip_dense_logits_embed_dev(const bitnet_hip_vector_input *input, const uint16_t *w, size_t vocab, size_t cols, size_t ld, float *logits, void *scratch, int32_t *token,
+                                      int32_t *pos, int32_t *history, const int32_t *n_forced, const bitnet_hip_embedding *next, void *stream) {
+    BH_GUARD_BEGIN
+    BH_REQUIRE(next, "Null pointer passed to dense_logits_embed_dev");
+    return dense_logits(input, w, vocab, cols, ld, logits, scratch, token, pos, history, n_forced, next, (hipStream_t)stream);
     BH_GUARD_END
 }
 

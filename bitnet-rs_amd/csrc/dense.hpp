@@ -126,6 +126,17 @@ struct TokenPairs {
     uint64_t buckets = 0, mul_prev = 0, mul_cur = 0;
 };
 
+// the embedding row of a position that follows
+struct EmbedNext {
+    const uint16_t *table = nullptr;
+    size_t ld = 0;
+    int width = 0, vocab = 0;
+    float scale = 1.f, eps = 0.f;
+    const float *norm_w = nullptr;
+    TokenPairs pairs;
+    float *out = nullptr;
+};
+
 // rows of a down-projection output z -> normed query latent, normed key latent and rotated key part
 struct LatentRows {
     const float *z = nullptr;      // [m][ldz]: [q_rank | kv_rank | rot_dim] (the last two absent when kv_rank == 0)
@@ -204,6 +215,8 @@ constexpr int kMaxExperts = 1024, kMaxTop = 32;
 
 hipError_t launch_embed_bf16(const uint16_t *table, size_t ld, const int *tokens, const int *offset, int n, int width, int vocab, float scale,
                              const float *norm_w, float eps, const TokenPairs &pairs, float *out, hipStream_t s);
+bool embed_follows(const EmbedNext &e);
+hipError_t launch_argmax_embed(const float *best_val, const int *best_idx, int n, int *token, int *pos, int *history, const int *n_forced, const EmbedNext &e, hipStream_t s);
 hipError_t launch_conv_keep(const void *rows, size_t ld, int rows_f32, int channels, int taps, float *ring, const int *pos, int n, hipStream_t s);
 hipError_t launch_sum_norm_rows(const SumRows &a, hipStream_t s);
 hipError_t launch_gated_norm_rows(const float *o, size_t ldo, const float *w, const void *gate, size_t ldg, int gate_f32, float eps, int m, int n,

@@ -86,6 +86,88 @@ __global__ void k_embed_bf16(const uint16_t *__restrict__ table, size_t ld, cons
     }
 }
 
+// The greedy token out of a product's partial maxima (as k_argmax_final, position and history too) and the embedding row of the next position, which a step behind this one starts with: as
+// k_embed_bf16 gives it, bit for bit.  A chain of latencies: position, token, columns; a token that is there already is on its way beside the maxima.  Two launches of 3.9 and 4.4 to 4.7 us
+// become one of 4.5 to 5.2 us.
+__global__ __launch_bounds__(256) void k_argmax_embed(const float *best_val, const int *best_idx, int n, int *token_out, int *pos_ptr, int *history, const int *n_forced, EmbedNext e) {
+    __shared__ float sv[4], slot[4];
+    __shared__ int si[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, at = *pos_ptr + 1;
+    const bool forced = n_forced && at < *n_forced;
+    const int there = history[at], prev = min(max(history[at - 1], 0), e.vocab - 1), n4 = e.width / 4;
+    f32x4 v[4], w[4];
+    u32x2 x[4], y[4];
+    auto fetch = [&](int token) {
+        const uint16_t *row = e.table + (size_t)token * e.ld, *two = nullptr;
+        if (e.pairs.table) {
+            const uint64_t sum = (uint64_t)prev * e.pairs.mul_prev + (uint64_t)token * e.pairs.mul_cur;
+            two = e.pairs.table + (size_t)((sum | e.pairs.buckets) >> 32 ? sum % e.pairs.buckets : (uint32_t)sum % (uint32_t)e.pairs.buckets) * e.pairs.ld;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = 4 * min(tid + 256 * j, n4 - 1);
+            x[j] = *reinterpret_cast<const u32x2 *>(row + i);
+            y[j] = two ? *reinterpret_cast<const u32x2 *>(two + i) : u32x2{0u, 0u};
+        }
+    };
+    if (forced) fetch(min(max(there, 0), e.vocab - 1));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = e.norm_w ? reinterpret_cast<const f32x4 *>(e.norm_w)[min(tid + 256 * j, n4 - 1)] : f32x4{1.f, 1.f, 1.f, 1.f};
+    float bv = -INFINITY;
+    int bi = 0x7fffffff;
+    auto better = [&](float o, int i) {
+        if (o > bv || (o == bv && i < bi)) bv = o, bi = i;
+    };
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (tid + 256 * j < n) better(best_val[tid + 256 * j], best_idx[tid + 256 * j]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const float o = __shfl_xor(bv, off, 64);
+        const int i = __shfl_xor(bi, off, 64);
+        better(o, i);
+    }
+    if (lane == 0) sv[wave] = bv, si[wave] = bi;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) better(sv[i], si[i]);
+    const int token = bi == 0x7fffffff ? 0 : bi;
+    if (!forced) fetch(token);
+    if (tid == 0) {
+        if (token_out) *token_out = token;
+        if (!forced) history[at] = token;
+        *pos_ptr = at;
+    }
+    auto four = [&](u32x2 u) { return f32x4{bf2f(u.x & 0xffffu), bf2f(u.x >> 16), bf2f(u.y & 0xffffu), bf2f(u.y >> 16)}; };
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = e.scale * four(x[j]);
+    if (e.pairs.table)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = v[j] + four(y[j]);
+    if (e.norm_w) {
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ss += tid + 256 * j < n4 ? (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w) : 0.f;
+        const float inv = 1.0f / sqrtf(group_total<4>(ss, slot) / (float)e.width + e.eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = v[j] * inv * w[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (tid + 256 * j < n4) reinterpret_cast<f32x4 *>(e.out)[tid + 256 * j] = v[j];
+}
+
+bool embed_follows(const EmbedNext &e) {
+    const uintptr_t rows = (uintptr_t)e.table | (uintptr_t)e.pairs.table, vectors = (uintptr_t)e.norm_w | (uintptr_t)e.out;
+    return e.width > 0 && e.width % 4 == 0 && e.width <= 4096 && (e.ld | e.pairs.ld) % 4 == 0 && (rows & 7) == 0 && (vectors & 15) == 0 && !(e.norm_w && e.pairs.table);
+}
+
+hipError_t launch_argmax_embed(const float *best_val, const int *best_idx, int n, int *token, int *pos, int *history, const int *n_forced, const EmbedNext &e, hipStream_t s) {
+    if (n > 1024 || !embed_follows(e)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_argmax_embed, dim3(1), dim3(256), 0, s, best_val, best_idx, n, token, pos, history, n_forced, e);
+    return hipGetLastError();
+}
+
 hipError_t launch_embed_bf16(const uint16_t *table, size_t ld, const int *tokens, const int *offset, int n, int width, int vocab, float scale,
                              const float *norm_w, float eps, const TokenPairs &pairs, float *out, hipStream_t s) {
     const int parts = !norm_w && n == 1 ? (width + 1023) / 1024 : 1;  // (one token: its row at once)

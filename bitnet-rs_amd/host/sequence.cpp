@@ -49,6 +49,12 @@ void Sequence::drop_graphs() {
         if (graph_[i]) hipGraphDestroy((hipGraph_t)graph_[i]);
         graph_exec_[i] = graph_[i] = nullptr;
     }
+    for (int i = 0; i < kForms; ++i) {
+        if (chain_exec_[i]) hipGraphExecDestroy((hipGraphExec_t)chain_exec_[i]);
+        if (chain_graph_[i]) hipGraphDestroy((hipGraph_t)chain_graph_[i]);
+        chain_exec_[i] = chain_graph_[i] = nullptr;
+    }
+    chain_steps_ = 0;
 }
 
 int Sequence::settle() {
@@ -152,6 +158,39 @@ int Sequence::ensure_graph(bool with_logits, int form) {
     return 0;
 }
 
+int Sequence::ensure_chain(int form) {
+    if (int rc = ensure_graph(true, form)) return rc;
+    if (!chain_steps_) {
+        size_t nodes = 0;
+        HCHK(hipGraphGetNodes((hipGraph_t)graph_[2 * form + 1], nullptr, &nodes));
+        const int fit = nodes ? (int)(kChainNodes / nodes) : 1;
+        chain_steps_ = !chains() || fit < 1 ? 1 : fit < kChainMost ? fit : kChainMost;
+    }
+    if (chain_steps_ < 2 || chain_exec_[form]) return 0;
+    hipStream_t s = (hipStream_t)stream_;
+    hipGraph_t g = nullptr;
+    HCHK(hipStreamBeginCapture(s, hipStreamCaptureModeGlobal));
+    int rc = 0;
+    for (int i = 0; i < chain_steps_ && rc == 0; ++i) {
+        follows_ = i > 0, followed_ = i + 1 < chain_steps_;
+        rc = step(true, form);
+    }
+    follows_ = followed_ = false;
+    const hipError_t e = hipStreamEndCapture(s, &g);
+    if (rc != 0) {
+        if (g) hipGraphDestroy(g);
+        return rc;
+    }
+    HCHK(e);
+    hipGraphExec_t ex = nullptr;
+    const hipError_t made = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
+    if (made != hipSuccess) hipGraphDestroy(g);
+    HCHK(made);
+    chain_graph_[form] = g;
+    chain_exec_[form] = ex;
+    return 0;
+}
+
 int Sequence::check_run(int n, bool with_logits) {
     if (!ready()) return fail_arg("model globals not set");
     const int p = position();
@@ -166,20 +205,31 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
     if (int rc = check_run(n, with_logits)) return rc;
     const int p = position();
     hipStream_t s = (hipStream_t)stream_;
+    // steps from i on that one graph makes
+    auto together = [&](int i) {
+        const int form = form_at(p + i);
+        if (!with_logits || n - i < 2 || ensure_chain(form) != 0 || chain_steps_ < 2 || i + chain_steps_ > n) return 1;
+        for (int k = 1; k < chain_steps_; ++k)
+            if (form_at(p + i + k) != form) return 1;
+        return chain_steps_;
+    };
     if (use_graph) {
-        for (int i = 0; i < n; ++i) {  // every form this run needs
+        for (int i = 0; i < n; i += together(i)) {  // every form this run needs
             int rc = ensure_graph(with_logits, form_at(p + i));
             if (rc) return rc;
         }
     }
     host_pos_ = -1;
     HCHK(hipEventRecord(begin_.e, s));
-    for (int i = 0; i < n; ++i) {
+    for (int i = 0; i < n;) {
         if (use_graph) {
-            HCHK(hipGraphLaunch((hipGraphExec_t)graph_exec_[2 * form_at(p + i) + (with_logits ? 1 : 0)], s));
+            const int form = form_at(p + i), k = together(i);
+            HCHK(hipGraphLaunch((hipGraphExec_t)(k > 1 ? chain_exec_[form] : graph_exec_[2 * form + (with_logits ? 1 : 0)]), s));
+            i += k;
         } else {
             int rc = step(with_logits, form_at(p + i));
             if (rc) return rc;
+            ++i;
         }
     }
     HCHK(hipEventRecord(end_.e, s));

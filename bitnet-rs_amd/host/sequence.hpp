@@ -80,6 +80,7 @@ class Sequence {
     int fail_arg(const char *what);
     int check_run(int n, bool with_logits);
     int ensure_graph(bool with_logits, int form);
+    int ensure_chain(int form);
     void drop_graphs();
     int settle();                       // waits for the stream
     void moved_to(int p) { host_pos_ = exposed_ ? -1 : p; }
@@ -94,6 +95,7 @@ class Sequence {
     virtual bool ready() const = 0;                            // weights are there
     virtual int step(bool with_logits, int form) = 0;          // the launches of one single-token step
     virtual int form_at(int) const { return 0; }               // which form of them a step at this position takes
+    virtual bool chains() const { return false; }              // can a step with logits embed the next position's token?
     virtual int clear_state() { return 0; }
 
     bool dead_ = true;
@@ -111,6 +113,13 @@ class Sequence {
     bool staged_ = false;
     Event begin_, end_;  // of the last run or prefill
     static constexpr int kForms = 5;
+    // Several steps with logits as one graph (chain_exec_[form], chain_steps_ of them), the token chosen and the next one's row in one launch: as many as make kChainNodes launches, four at most (eight
+    // take the same; graphs of 600 launches and more were slower than one per step).  Answers of 24 to 48 tokens, four layers: Lasapel 2b 14.48 -> 14.12 ms, Mimolix 3b 8.75 -> 8.64, Lurepel 1b
+    // 7.30 -> 7.18, Sipelorn 1b 6.82 -> 6.76.
+    static constexpr int kChainNodes = 192, kChainMost = 4;
+    bool follows_ = false, followed_ = false;  // of the step at hand: the one ahead has embedded its token; it embeds the next one's
+    void *chain_exec_[kForms] = {}, *chain_graph_[kForms] = {};
+    int chain_steps_ = 0;  // (0: not known yet)
     void *graph_exec_[2 * kForms] = {};  // [2 * form + with_logits]
     void *graph_[2 * kForms] = {};
 };

@@ -910,12 +910,28 @@ int StackModel::embed_rows(size_t n, float *out) {
     return 0;
 }
 
+bitnet_hip_embedding StackModel::embedding(float *out) const {
+    bitnet_hip_embedding e = {};
+    e.table = embed_.w, e.ld = embed_.ld, e.width = width_, e.vocab = vocab_, e.scale = spec_.embed_scale, e.out = out;
+    if (pairs_.w)
+        e.pairs = pairs_.w, e.ld_pairs = pairs_.ld, e.buckets = spec_.pairs.buckets, e.mul_prev = spec_.pairs.mul_prev, e.mul_cur = spec_.pairs.mul_cur;
+    else
+        e.norm_weight = embed_norm_, e.eps = spec_.eps;
+    return e;
+}
+
+// (the row of the step behind is written while nobody reads this step's any more: the residual stream has left it with the first sum)
+bool StackModel::chains() const {
+    const bitnet_hip_embedding e = embedding(x0_);
+    return !runs_.empty() && bitnet_hip_embedding_follows(&e);
+}
+
 int StackModel::step(bool with_logits, int form) {
     form_ = form;
     cur_ = x0_;
     row_at_ = 0;
     pending_ = Pending();
-    TRY(embed_rows(1, x0_));
+    if (!follows_) TRY(embed_rows(1, x0_));
     for (const Run &run : runs_) {
         const size_t i = run.layer;
         const Layer &L = layers_[i];
@@ -944,7 +960,11 @@ int StackModel::step(bool with_logits, int form) {
     }
     if (with_logits) {
         const bitnet_hip_vector_input in = block_input(final_norm_);
-        BCHK(bitnet_hip_dense_logits_dev(&in, head_m_.w, vocab_, head_m_.cols, head_m_.ld, logits_, argmax_, token_, pos_, history_, n_forced_, stream_));
+        const bitnet_hip_embedding next = embedding(x0_);
+        if (followed_)
+            BCHK(bitnet_hip_dense_logits_embed_dev(&in, head_m_.w, vocab_, head_m_.cols, head_m_.ld, logits_, argmax_, token_, pos_, history_, n_forced_, &next, stream_));
+        else
+            BCHK(bitnet_hip_dense_logits_dev(&in, head_m_.w, vocab_, head_m_.cols, head_m_.ld, logits_, argmax_, token_, pos_, history_, n_forced_, stream_));
         hidden_ = cur_;
     } else {
         BCHK(bitnet_hip_advance_pos_dev(pos_, stream_));

@@ -150,6 +150,8 @@ class StackModel : public Sequence {
   protected:
     bool ready() const override { return head_ != nullptr && layers_set_ == spec_.layers.size(); }
     int step(bool with_logits, int form) override;
+    bool chains() const override;
+    bitnet_hip_embedding embedding(float *out) const;
     int form_at(int pos) const override;  // how a step's attention records are merged: kStepRecords
     int clear_state() override;
 

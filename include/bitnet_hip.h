@@ -731,6 +731,21 @@ int bitnet_hip_dense_gemv_dev(const bitnet_hip_vector_input *input, const uint16
 int bitnet_hip_dense_logits_dev(const bitnet_hip_vector_input *input, const uint16_t *w_dev, size_t vocab, size_t cols, size_t ld,
                                 float *logits_dev, void *scratch_dev, int32_t *token_dev, int32_t *pos_dev, int32_t *history_dev,
                                 const int32_t *n_forced_dev, void *stream);
+/* The same, and the embedding row of the next position (its token: the one chosen, or the one that history holds where that is forced) behind it in the same launch.  next: what
+ * embed_bf16, embed_norm_bf16 (norm_weight) or embed_pairs_bf16 (pairs) take; embedding_follows: rows of up to 4096 columns, whole in fours, tables on 8 bytes, vectors on 16. */
+typedef struct bitnet_hip_embedding {
+    const uint16_t *table;
+    size_t ld, width, vocab;
+    float scale, eps;
+    const float *norm_weight;
+    const uint16_t *pairs;
+    size_t ld_pairs, buckets;
+    uint64_t mul_prev, mul_cur;
+    float *out;
+} bitnet_hip_embedding;
+int bitnet_hip_embedding_follows(const bitnet_hip_embedding *next);
+int bitnet_hip_dense_logits_embed_dev(const bitnet_hip_vector_input *input, const uint16_t *w_dev, size_t vocab, size_t cols, size_t ld, float *logits_dev, void *scratch_dev,
+                                      int32_t *token_dev, int32_t *pos_dev, int32_t *history_dev, const int32_t *n_forced_dev, const bitnet_hip_embedding *next, void *stream);
 
 /* Attention over the latent cache.  Head h's query [qd = dimp + ldr]: dimp unrotated (zero-padded to a multiple of 32), then the part to
  * rotate (rot_dim of ldr).  score = (unrotated . W_uk c + rotated . r) * scale; the softmax's denominator also holds exp(sink[h]) (sink

@@ -1,0 +1,39 @@
+"""Several steps as one graph, each embedding the next one's token (host/sequence.cpp): the same, bit for bit, as steps one by one, for every kind of embedding, with tokens fed and chosen, across the
+end of what was fed and across the forms of a step; replayed with other work between."""
+import importlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+synth = importlib.import_module("bitnet-rs_amd.synth")
+
+
+@pytest.mark.parametrize("design", ["lasapel", "mimolix", "lurepel", "sipelorn"])
+@pytest.mark.parametrize("fed,prompt,steps", [(30, 6, 23), (6, 6, 9), (12, 3, 14), (140, 120, 19)])
+def test_chained_steps(pkg, tmp_path, design, fed, prompt, steps):
+    config = getattr(synth, design + "_config")("1b", 2 if design != "mimolix" else 4)
+    config["vocab"] = 640
+    getattr(synth, "write_" + design)(str(tmp_path), config)
+    m = pkg.open_model(str(tmp_path), max_pos=512)
+    tokens = np.random.default_rng(fed).integers(0, 640, fed).astype(np.int32)
+
+    def start():
+        m.reset()
+        m.feed(tokens)
+        m.prefill(prompt, with_logits=True, digits=2)
+
+    start()
+    one = []
+    for _ in range(steps):
+        m.run(1)
+        one.append(m.last_logits().copy())
+    history = m.history(prompt + steps + 1)
+    for again in range(3):
+        start()
+        at = 0
+        for n in (steps,) if again == 0 else (5, steps - 5) if again == 1 else (1, 4, steps - 5):
+            m.run(n)
+            at += n
+            assert np.array_equal(m.last_logits(), one[at - 1])
+        assert np.array_equal(m.history(prompt + steps + 1), history)
