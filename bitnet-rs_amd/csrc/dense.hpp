@@ -5,6 +5,8 @@
 // have ld a multiple of 64; what lies past their columns must be FINITE (a weight's zero column cancels it).
 #pragma once
 
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace bitnet_hip {
@@ -437,6 +439,22 @@ __device__ __forceinline__ float activate(float v, int act) {
 // all of them
 __device__ __forceinline__ float activate(float v, int act, float a, float b) {
     return act == BITNET_HIP_ACT_XIELU ? 0.5f * v + (v > 0.f ? a * v * v : b * (expm1f(v) - v)) : activate(v, act);
+}
+
+// The order of the workgroups of a launch over records of keys of which the device alone knows how many there are: eight records of all members (heads, queries), then the next eight, so
+// that what exists comes first and what ends at once comes last.  As the fastest index the 128 records of a head, most of them to end, lay ahead of the next head's: 24 heads of 128 columns
+// (bf16) at 200 keys 52 -> 22 us, at 2000 keys 53 -> 27, 16 queries at 200 keys 361 -> 36; at 8000 keys, where nearly all exist, 55.9 -> 56.8.
+// Up to 32 members, an XCD's compute units, take their record on one XCD, whose L2 has its keys for all; the next 32 on the next XCD, so that few records fill the chip too.  Members
+// of other sets of keys between them do no harm; dealing (record, set) pairs to the XCDs instead did: 24 heads of 6 sets at 8000 keys 56 -> 62 us.
+struct RecordPlace {
+    int record, member;
+};
+__device__ __forceinline__ RecordPlace record_place() {
+    return {(int)(blockIdx.z * 8 + ((blockIdx.x + blockIdx.y) & 7)), (int)(blockIdx.y * (gridDim.x >> 3) + (blockIdx.x >> 3))};
+}
+inline dim3 record_grid(int records, size_t members) {
+    const size_t chunks = std::min<size_t>((members + 31) / 32, 65535), each = (members + chunks - 1) / chunks;
+    return dim3(8 * each, chunks, (records + 7) / 8);
 }
 
 // a pair of floats as (high, low) bf16 pairs: high + low carries 16 of the 24 bits

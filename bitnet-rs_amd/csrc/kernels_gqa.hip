@@ -303,15 +303,17 @@ hipError_t launch_gqa_rows(const Gqa &g, void *rows, size_t ld, int rows_f32, in
 // ---- any size ---------------------------------------------------------------------------------------------------------
 // One workgroup per (record, head and map, query); a wave takes every fourth key, its lanes the columns.
 template <class TQ, class TC, int ND, int NV>
-__global__ __launch_bounds__(256) void k_gqa_any(Gqa p, const TQ *q, size_t ldq, const int *pos_ptr, int q0, float *scratch) {
+__global__ __launch_bounds__(256) void k_gqa_any(Gqa p, const TQ *q, size_t ldq, const int *pos_ptr, int q0, int nq, float *scratch) {
     extern __shared__ __attribute__((aligned(16))) float vec[];  // [4][vdimp]
     __shared__ float sm[4], sl[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hm = blockIdx.y, qi = blockIdx.z;
-    const int maps = (int)p.maps, h = hm / maps, map = hm - h * maps, kv = h / (int)(p.heads / p.kv_heads), dimp = (int)p.dimp, vdimp = (int)p.vdimp;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const RecordPlace at = record_place();
+    const int maps = (int)p.maps, each = (int)p.heads * maps, qi = at.member / each, hm = at.member - qi * each, h = hm / maps, map = hm - h * maps, kv = h / (int)(p.heads / p.kv_heads), dimp = (int)p.dimp, vdimp = (int)p.vdimp;
+    if (qi >= nq) return;
     const int pos = *pos_ptr + q0 + qi;
     const GqaRange range = gqa_range(p, pos);
-    if ((int)blockIdx.x >= range.used) return;
-    const int start = range.base + blockIdx.x * range.per * kGqaTile, k0 = max(start, range.first), k1 = min(start + range.per * kGqaTile, pos + 1);
+    if (at.record >= range.used) return;
+    const int start = range.base + at.record * range.per * kGqaTile, k0 = max(start, range.first), k1 = min(start + range.per * kGqaTile, pos + 1);
     const TQ *qr = q + (size_t)qi * ldq + (size_t)hm * dimp;
     const TC *K = (const TC *)p.kcache + (size_t)(kv * maps + map) * p.capacity * dimp, *V = (const TC *)p.vcache + (size_t)kv * vdimp * p.capacity;
     float qv[ND], acc[NV];
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(256) void k_gqa_any(Gqa p, const TQ *q, size_t ldq,
         w[i] = sm[i] == -INFINITY ? 0.f : exp2f(sm[i] - M);
         L += w[i] * sl[i];
     }
-    float *rec = scratch + (((size_t)qi * p.heads * maps + hm) * kGqaSplits + blockIdx.x) * (kGqaRecHead + vdimp);
+    float *rec = scratch + (((size_t)qi * p.heads * maps + hm) * kGqaSplits + at.record) * (kGqaRecHead + vdimp);
     for (int i = tid; i < vdimp; i += 256)
         rec[kGqaRecHead + i] = (w[0] * vec[i] + w[1] * vec[vdimp + i]) + (w[2] * vec[2 * vdimp + i] + w[3] * vec[3 * vdimp + i]);
     if (tid == 0) rec[0] = M, rec[1] = L;
@@ -358,7 +360,7 @@ static hipError_t any_go(const Gqa &g, const void *q, size_t ldq, const int *pos
     const size_t lds = 4 * g.vdimp * sizeof(float);
     if (g.dimp > 1024 || g.vdimp > 1024) return hipErrorInvalidValue;
     auto fn = g.dimp <= 64 && g.vdimp <= 64 ? k_gqa_any<TQ, TC, 1, 1> : g.dimp <= 256 && g.vdimp <= 256 ? k_gqa_any<TQ, TC, 4, 4> : k_gqa_any<TQ, TC, 16, 16>;
-    hipLaunchKernelGGL(fn, dim3(splits, g.heads * g.maps, nq), dim3(256), lds, s, g, (const TQ *)q, ldq, pos, q0, scratch);
+    hipLaunchKernelGGL(fn, record_grid(splits, g.heads * g.maps * nq), dim3(256), lds, s, g, (const TQ *)q, ldq, pos, q0, nq, scratch);
     return hipGetLastError();
 }
 
@@ -375,7 +377,9 @@ hipError_t launch_gqa_any(const Gqa &g, const void *q, size_t ldq, int q_f32, in
 // holds a one can tell.  12 and 24 heads of two maps of 64 / 128 columns, 200 and 1000 keys: 9.4 -> 9.1 us; one map of 128 / 128: 8.25 -> 8.05.
 // The launch is a chain of latencies (150 and 2090 keys take the same): arguments -> position -> rotation and keys -> scores -> weights -> output.  Hence: what the host knows is
 // divided there (64-bit divisions by arguments were a quarter of the launch), all arguments are requested at once, raw rows and norms' weights ahead of the position, and the
-// new key's row is one more of the rows that the waves share out.  Beside another launch, 12 heads of 128 / 128 at 2090 keys 8.6 -> 6.2 us, 24 of two maps of 64 / 128 at 216 keys 12.2 -> 10.2.
+// new key's row is one more of the rows that the waves share out.  Records are the slowest index of the launch, which has one for every 128 keys of the capacity: as the fastest
+// they put several of the workgroups that have keys on the same compute units at some capacities (24 heads of 6 kv heads at 2000 keys, us with this order / that: capacity 8192 6.0 / 8.2,
+// two maps 6.9 / 9.1, capacity 8320 7.0 / 8.9, 5888 and 9600 7.0 / 7.1).  Beside another launch, 12 heads of 128 / 128 at 2090 keys 8.6 -> 6.2 us, 24 of two maps of 64 / 128 at 216 keys 12.2 -> 10.2.
 struct GqaStepK {
     const float *row, *q_weight, *k_weight, *q_factor, *rope_cos, *rope_sin, *far_weight, *far_rate;
     const int *pos;
@@ -395,7 +399,7 @@ __global__ __launch_bounds__(256, NV > 8 || NK * MAPS >= 8 ? 1 : 2) void k_gqa_s
                  "s"(p.append), "s"(p.k_at), "s"(p.v_at));
     const int posv = *p.pos;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, g = lane >> 4;
-    const int kv = blockIdx.z, first_head = blockIdx.y * 16, h0 = kv * p.group + first_head, nh = min(16, p.group - first_head);
+    const int kv = blockIdx.x, first_head = blockIdx.y * 16, h0 = kv * p.group + first_head, nh = min(16, p.group - first_head);
     const int dimp = p.dimp, vdimp = p.vdimp;
     constexpr int QS = NK * 32 + 4, J = (NK + 1) / 2, QR = NK > 4 ? 1 : 4;  // QR: rows of a wave at a time
     uint16_t *K = p.K + (size_t)kv * MAPS * p.capacity * dimp, *V = p.V + (size_t)kv * vdimp * p.capacity;
@@ -434,8 +438,8 @@ __global__ __launch_bounds__(256, NV > 8 || NK * MAPS >= 8 ? 1 : 2) void k_gqa_s
     const int tiles = (n_keys - range.base + kGqaTile - 1) / kGqaTile;
     range.per = (tiles + kGqaSplits - 1) / kGqaSplits;
     range.used = range.per == 1 ? tiles : (tiles + range.per - 1) / range.per;
-    if ((int)blockIdx.x >= range.used) return;
-    const int k0 = range.base + blockIdx.x * range.per * kGqaTile, k1 = min(k0 + range.per * kGqaTile, n_keys);
+    if ((int)blockIdx.z >= range.used) return;
+    const int k0 = range.base + blockIdx.z * range.per * kGqaTile, k1 = min(k0 + range.per * kGqaTile, n_keys);
     float cs[J], sn[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -610,7 +614,7 @@ __global__ __launch_bounds__(256, NV > 8 || NK * MAPS >= 8 ? 1 : 2) void k_gqa_s
     const int n_rows = MAPS * nh;
     for (int r = tid >> 5; r < n_rows; r += 8) {
         const int j = MAPS == 2 && r >= nh ? 1 : 0, hh = r - j * nh;
-        float *rec = p.scratch + ((size_t)((h0 + hh) * MAPS + j) * kGqaSplits + blockIdx.x) * (kGqaRecHead + vdimp);
+        float *rec = p.scratch + ((size_t)((h0 + hh) * MAPS + j) * kGqaSplits + blockIdx.z) * (kGqaRecHead + vdimp);
         for (int c = (tid & 31) * 4; c < vdimp; c += 128) {
             const float *src = area + (size_t)r * vdimp + c;
             const size_t step = (size_t)n_rows * vdimp;
@@ -643,7 +647,7 @@ static hipError_t step_go(const Gqa &g, const GqaStep &a, hipStream_t s) {
     k.chunk = g.chunk < g.capacity ? (int)g.chunk : 0, k.window = g.window < g.capacity ? (int)g.window : 0;  // (as large as the cache: no position has keys outside)
     k.normed = (g.q_weight || g.unit_norm ? 1 : 0) | (g.k_weight || g.unit_norm ? 2 : 0);
     k.k_at = (int)(g.heads * g.maps * g.dimp), k.v_at = g.values_are_keys ? k.k_at : (int)((g.heads + g.kv_heads) * g.maps * g.dimp);
-    hipLaunchKernelGGL(fn, dim3(splits, (group + 15) / 16, g.kv_heads), dim3(256), lds, s, k);
+    hipLaunchKernelGGL(fn, dim3(g.kv_heads, (group + 15) / 16, splits), dim3(256), lds, s, k);
     return hipGetLastError();
 }
 

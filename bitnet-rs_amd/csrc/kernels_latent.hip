@@ -43,12 +43,14 @@ __global__ __launch_bounds__(256) void k_latent_decode_any(LatentAttn p) {
     extern __shared__ float vec[];  // [4][ldc]
     __shared__ float sm[4], sl[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int h = blockIdx.y, qi = blockIdx.z;
+    const RecordPlace at = record_place();
+    const int qi = at.member / p.heads, h = at.member - qi * p.heads;
+    if (qi >= p.nq) return;
     const int pos = *p.pos + p.q0 + qi, n_keys = pos + 1;
     int per, used;
     split_range(n_keys, per, used);
-    if ((int)blockIdx.x >= used) return;
-    const int k0 = blockIdx.x * per * kLatentTile, k1 = min(k0 + per * kLatentTile, n_keys);
+    if (at.record >= used) return;
+    const int k0 = at.record * per * kLatentTile, k1 = min(k0 + per * kLatentTile, n_keys);
     const int half = p.rot_dim / 2;
     const float *qa = p.qabs + ((size_t)qi * p.heads + h) * p.ldc;
     const float *qr = p.q + (size_t)qi * p.ldq + (size_t)h * p.qd + p.dimp;
@@ -100,7 +102,7 @@ __global__ __launch_bounds__(256) void k_latent_decode_any(LatentAttn p) {
         w[i] = sm[i] == -INFINITY ? 0.f : expf(sm[i] - M);
         L += w[i] * sl[i];
     }
-    float *rec = p.scratch + (((size_t)qi * p.heads + h) * kLatentSplits + blockIdx.x) * (kLatentRecHead + p.ldc);
+    float *rec = p.scratch + (((size_t)qi * p.heads + h) * kLatentSplits + at.record) * (kLatentRecHead + p.ldc);
     for (int i = tid; i < p.ldc; i += 256)
         rec[kLatentRecHead + i] = (w[0] * vec[i] + w[1] * vec[p.ldc + i]) + (w[2] * vec[2 * p.ldc + i] + w[3] * vec[3 * p.ldc + i]);
     if (tid == 0) rec[0] = M, rec[1] = L;
@@ -111,6 +113,10 @@ __global__ __launch_bounds__(256) void k_latent_decode_any(LatentAttn p) {
 // of the columns, the rows going from memory straight into the MFMA's B operand (a lane: one key, eight columns); the f32 query is a
 // (high, low) pair.  The same registers leave the tile transposed in LDS (key pairs from two neighbouring lanes), and the waves share
 // the columns of O += P C.
+// A workgroup's LDS leaves room for no second one on its compute unit, and the device alone knows how many of the launch's records exist: eight records of all heads and queries come
+// first, then the next eight, so that those that end at once come last.  With the records of the first heads ahead of the others' (all of 128, most to end at once) the last heads waited
+// for compute units that ended nothing: 40 heads at 100 keys 10.4 -> 8.4 us, 64 at 2000 keys 11.3 -> 9.4, 16 queries of 20 heads at 100 keys 59.7 -> 44.1; where every record exists the
+// order is worth nothing (40 heads at 8000 keys 17.3 -> 17.7).  The eight lie on eight XCDs, each with all heads of its records: L2 reads a record once.
 constexpr int kDecKK = 20;  // most 32-column steps of ldc + ldr
 constexpr int kDecNT = 5;   // most 16-column tiles of ldc per wave
 constexpr int kCtStride = kLatentTile * 2 + 16;
@@ -123,7 +129,7 @@ __global__ __launch_bounds__(512) void k_latent_decode(LatentAttn p) {
     __shared__ f32x4 spart[4][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
     const int kg = wave & 3, half_cols = wave >> 2;
-    const int h0 = blockIdx.y * 16, qi = blockIdx.z;
+    const int h0 = blockIdx.y * 16, qi = blockIdx.x >> 3, record = blockIdx.z * 8 + (blockIdx.x & 7);
     constexpr int MKK = NCK ? (NCK + NRK + 1) / 2 : kDecKK / 2, MNT = NCK ? NCK / 4 : kDecNT;
     const int nck = NCK ? NCK : p.ldc / 32, nkk = NCK ? NCK + NRK : nck + p.ldr / 32, kt = nkk * 32, ntiles = nck * 2, ldc = nck * 32;
     const int kk0 = half_cols * ((nkk + 1) / 2), kn = half_cols ? nkk / 2 : (nkk + 1) / 2;  // this wave's steps
@@ -141,12 +147,12 @@ __global__ __launch_bounds__(512) void k_latent_decode(LatentAttn p) {
         }
     };
     // up to kLatentSplits tiles a record is one tile: requested before the position is known (any tile below the capacity may be read)
-    fetch(blockIdx.x * kLatentTile);
+    fetch(min(record * kLatentTile, p.capacity - kLatentTile));
     const int pos = *p.pos + p.q0 + qi, n_keys = pos + 1;
     int per, used;
     split_range(n_keys, per, used);
-    if ((int)blockIdx.x >= used) return;
-    const int k0 = blockIdx.x * per * kLatentTile, k1 = min(k0 + per * kLatentTile, n_keys);
+    if (record >= used) return;
+    const int k0 = record * per * kLatentTile, k1 = min(k0 + per * kLatentTile, n_keys);
     if (per > 1) fetch(k0);
     {
         // the query rows, 32 threads each: latent part, then the rotated part
@@ -267,7 +273,7 @@ __global__ __launch_bounds__(512) void k_latent_decode(LatentAttn p) {
     for (int i = 0; i < 4; ++i) {
         const int row = g * 4 + i, h = h0 + row;
         if (h >= p.heads) continue;
-        float *rec = p.scratch + (((size_t)qi * p.heads + h) * kLatentSplits + blockIdx.x) * (kLatentRecHead + ldc);
+        float *rec = p.scratch + (((size_t)qi * p.heads + h) * kLatentSplits + record) * (kLatentRecHead + ldc);
 #pragma unroll
         for (int t = 0; t < MNT; ++t)
             if (t * 8 + wave < ntiles) rec[kLatentRecHead + (t * 8 + wave) * 16 + r16] = o[t][i];
@@ -293,16 +299,16 @@ static hipError_t decode_any(const LatentAttn &a, dim3 grid, hipStream_t s) {
 
 hipError_t launch_latent_decode(const LatentAttn &a, hipStream_t s) {
     const int splits = min(kLatentSplits, (a.capacity + kLatentTile - 1) / kLatentTile);
-    if (a.f32) return decode_any<float>(a, dim3(splits, a.heads, a.nq), s);
+    if (a.f32) return decode_any<float>(a, record_grid(splits, (size_t)a.heads * a.nq), s);
     const int kt = a.ldc + a.ldr;
-    if (kt > 32 * kDecKK || a.ldc > 128 * kDecNT || a.ldc % 64 || a.ldr % 32) return decode_any<uint16_t>(a, dim3(splits, a.heads, a.nq), s);
+    if (kt > 32 * kDecKK || a.ldc > 128 * kDecNT || a.ldc % 64 || a.ldr % 32) return decode_any<uint16_t>(a, record_grid(splits, (size_t)a.heads * a.nq), s);
     const size_t lds = (size_t)a.ldc * kCtStride + (size_t)32 * (kt * 2 + 16) + (size_t)32 * kCtStride;
     auto fn = a.ldc == 512 && a.ldr == 64 ? k_latent_decode<16, 2> : k_latent_decode<0, 0>;
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL(fn, dim3(splits, (a.heads + 15) / 16, a.nq), dim3(512), lds, s, a);
+    hipLaunchKernelGGL(fn, dim3(8 * a.nq, (a.heads + 15) / 16, (splits + 7) / 8), dim3(512), lds, s, a);
     return hipGetLastError();
 }
 
