@@ -981,20 +981,41 @@ hipError_t launch_gqa_project(const GqaOut &a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// The order of a chain of products whose operands come from LDS: AHEAD reads, then PER products and the next read in turn.  Left to itself the compiler asks for two operands and waits for them.
+template <int READS, int PER, int AHEAD>
+__device__ __forceinline__ void reads_ahead() {
+    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+    for (int i = 0; i < READS - AHEAD; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, PER * AHEAD, 0);
+}
+
+// buffers of a tile in LDS: two where the two tiles that are under way on a compute unit (one of the largest heads) leave room
+constexpr int prefill_buffers(int nk, int nv, int maps) { return (nv > 8 || nk > 4 ? 2 : 4) * (maps * 64 * (nk * 64 + 32) + nv * 16 * (64 * 2 + 32)) <= 163840 ? 2 : 1; }
+
 // ---- prompt -----------------------------------------------------------------------------------------------------------
 // One workgroup: one head, four waves; a wave holds two slots of 16 queries: both maps of one query tile, or two tiles of the only map.  Key tiles
 // of 64 (every map's) and the values of the tile staged through registers into LDS one step ahead.
 // G = 2: two such groups of four waves share the keys of the same queries, tile by tile in turn, and meet in LDS at the end.  A prompt's last queries see all of its keys and its
-// first next to none: with one group per workgroup the longest walk takes 2.6 us a tile whatever its neighbour does, with two it is half as long at 4.1 us a step.
+// first next to none: with one group per workgroup the longest walk takes 2.2 us a tile whatever its neighbour does, with two it is half as long at 3.3 us a step.
 // Heads that need more than 256 registers keep one group; two_groups says when the others take two.
+// Bound by the two waves of a SIMD and their waits, not by memory (16 heads, 4096 tokens: matrix cores 40 %, vector instructions half of the time).  Hence: rows of a tile lie 32 bytes past a
+// multiple of 64 apart (reads of 16 rows by 64 bytes without bank conflicts: 16 bytes past it they took twice the cycles), keys in the order in which a lane's weights are eight
+// neighbours (one 16-byte read of the values where two of 8 were), a key's row is written by neighbouring threads, operands are read four ahead of their products, and two
+// buffers take one barrier a step, with the stores between the weights and their products.  us, each of these in turn, 16 heads of 128 columns at 4096 tokens: 130.9, 124.5 (order), 121.0
+// (writes), 120.5 (rows), 111.9 (reads ahead), 109.7 (buffers).  24 heads, 3000 tokens 121 -> 105; 32 heads, 1531 49.4 -> 42; 24 of two maps, 1531 62 -> 53, 300 13.9 -> 12.5.
 // FAR: with a distance penalty, gates per column, or both.
 // records: gridDim.y workgroups share a block's tiles of keys, in stretches, and each leaves its outputs, maxima and sums for k_gqa_merge_parts (which counts the sink).
 template <int NK, int NV, int MAPS, bool FAR, int G>
 __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefill(Gqa p, const uint16_t *Q, size_t ldq, int n_ctx, int nq, uint16_t *out, size_t ldo, int n_qb, float *records) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    constexpr int SLOTS = 2, QW = 16 * SLOTS / MAPS, KS = NK * 64 + 16, VS = 64 * 2 + 16, NVL = NV / 2;
+    constexpr int SLOTS = 2, QW = 16 * SLOTS / MAPS, KS = NK * 64 + 32, VS = 64 * 2 + 32, NVL = NV / 2, AHEAD = 4;
     const int grp = G == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
-    uint8_t *lk = lds + grp * (MAPS * 64 * KS + NV * 16 * VS), *lv = lk + MAPS * 64 * KS;
+    constexpr int KB = MAPS * 64 * KS, TILE = KB + NV * 16 * VS, BUFS = prefill_buffers(NK, NV, MAPS);
+    uint8_t *lk = lds + grp * BUFS * TILE;
     const int heads = (int)p.heads, dimp = (int)p.dimp, vdimp = (int)p.vdimp;
     // Consecutive workgroups go to the eight XCDs in turn.  Longest blocks first; an XCD keeps heads / 8 neighbouring heads of its own (their keys
     // and values stay in its L2), the heads left over move from XCD to XCD with the block so that all eight carry the same work.
@@ -1029,7 +1050,15 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
     }
     const uint16_t *K = (const uint16_t *)p.kcache + (size_t)kv * MAPS * p.capacity * dimp, *V = (const uint16_t *)p.vcache + (size_t)kv * vdimp * p.capacity;
     u32x4 kreg[MAPS][NK], vreg[NVL];
-    const unsigned koff = (unsigned)((tid >> 2) * dimp * 2 + (tid & 3) * 16);
+    // keys: a row of the tile by KC neighbouring threads; row p of 32 in LDS is key 8 (p >> 2 & 3) + 4 (p >> 4) + (p & 3)
+    constexpr int KC = NK * 4, KR = 256 / KC;
+    const unsigned koff = (unsigned)((tid / KC) * dimp * 2 + min((tid % KC) * 16, dimp * 2 - 16));
+    uint8_t *kw[NK];
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+        const int key = tid / KC + j * KR, row = (key & 32) + (key >> 2 & 1) * 16 + (key >> 3 & 3) * 4 + (key & 3);
+        kw[j] = lk + row * KS + (tid % KC) * 16;
+    }
     const size_t voff = (size_t)(tid >> 3) * p.capacity * 2 + (tid & 7) * 16;
 #pragma unroll
     for (int j = 0; j < NVL; ++j) vreg[j] = u32x4{0u, 0u, 0u, 0u};
@@ -1038,7 +1067,7 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
         for (int mp = 0; mp < MAPS; ++mp) {
             const char *kb = (const char *)(K + ((size_t)mp * p.capacity + key0) * dimp);
 #pragma unroll
-            for (int j = 0; j < NK; ++j) kreg[mp][j] = *reinterpret_cast<const u32x4 *>(kb + min(j * 64, dimp * 2 - 64) + koff);
+            for (int j = 0; j < NK; ++j) kreg[mp][j] = *reinterpret_cast<const u32x4 *>(kb + (size_t)(j * KR * 2) * dimp + koff);
         }
         const char *vb = (const char *)(V + key0);
 #pragma unroll
@@ -1054,19 +1083,46 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
         const int each = (n_tiles - t_first + (int)gridDim.y - 1) / (int)gridDim.y;
         t_first = min(t_first + (int)blockIdx.y * each, n_tiles), n_tiles = min(t_first + each, n_tiles);
     }
-    fetch(max(min(t_first + grp, n_tiles - 1), 0) * 64);
-    for (int t0 = t_first; t0 < n_tiles; t0 += G) {
-        const int kt0 = t0 + grp, key0 = kt0 * 64;
-        __syncthreads();
+    auto store = [&](int at) {
 #pragma unroll
         for (int mp = 0; mp < MAPS; ++mp)
 #pragma unroll
-            for (int j = 0; j < NK; ++j) *reinterpret_cast<u32x4 *>(lk + (mp * 64 + (tid >> 2)) * KS + j * 64 + (tid & 3) * 16) = kreg[mp][j];
+            for (int j = 0; j < NK; ++j) *reinterpret_cast<u32x4 *>(kw[j] + at + mp * 64 * KS) = kreg[mp][j];
 #pragma unroll
-        for (int j = 0; j < NVL; ++j) *reinterpret_cast<u32x4 *>(lv + ((tid >> 3) + 32 * j) * VS + (tid & 7) * 16) = vreg[j];
+        for (int j = 0; j < NVL; ++j) *reinterpret_cast<u32x4 *>(lk + at + KB + ((tid >> 3) + 32 * j) * VS + (tid & 7) * 16) = vreg[j];
+    };
+    fetch(max(min(t_first + grp, n_tiles - 1), 0) * 64);
+    if (BUFS == 2) {
+        store(0);
+        if (t_first + grp + G < n_tiles) fetch((t_first + grp + G) * 64);
+    }
+    SplitFrag pf[2][SLOTS];
+    auto values = [&](const uint8_t *from) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const bf16x8 a = *reinterpret_cast<const bf16x8 *>(from + (v * 16 + r16) * VS + ks * 64 + g * 16);
+#pragma unroll
+                for (int t = 0; t < SLOTS; ++t) {
+                    o[v][t] = mfma_bf16(a, pf[ks][t].hi, o[v][t]);
+                    o[v][t] = mfma_bf16(a, pf[ks][t].lo, o[v][t]);
+                }
+            }
+        reads_ahead<NV * 2, 2 * SLOTS, AHEAD>();
+    };
+    int at = 0;  // the tile's buffer
+    for (int t0 = t_first; t0 < n_tiles; t0 += G) {
+        const int kt0 = t0 + grp, key0 = kt0 * 64;
         __syncthreads();
-        if (kt0 + G < n_tiles) fetch(key0 + G * 64);
-        if (key0 > pos0 + qw + QW - 1 || key0 + 63 < w_first || (G == 2 && kt0 >= n_tiles)) continue;  // no key of the tile is seen by this wave's queries
+        if (BUFS == 1) {
+            store(0);
+            __syncthreads();
+            if (kt0 + G < n_tiles) fetch(key0 + G * 64);
+        }
+        const bool seen = !(key0 > pos0 + qw + QW - 1 || key0 + 63 < w_first || (G == 2 && kt0 >= n_tiles));  // (else: no key of the tile is seen by this wave's queries)
+        const uint8_t *kt_ = lk + at;
+        if (seen) {
         f32x4 s[4][SLOTS];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
@@ -1076,31 +1132,33 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
             for (int kk = 0; kk < NK; ++kk)
 #pragma unroll
                 for (int t = 0; t < SLOTS; ++t) {
-                    const bf16x8 a = *reinterpret_cast<const bf16x8 *>(lk + ((t % MAPS) * 64 + kt * 16 + r16) * KS + kk * 64 + g * 16);
+                    const bf16x8 a = *reinterpret_cast<const bf16x8 *>(kt_ + ((t % MAPS) * 64 + kt * 16 + r16) * KS + kk * 64 + g * 16);
                     s[kt][t] = mfma_bf16(a, qf[t][kk], s[kt][t]);
                 }
         }
+        reads_ahead<4 * NK * MAPS, SLOTS / MAPS, AHEAD>();
+        __builtin_amdgcn_sched_barrier(0);
         if (FAR && p.far_weight)
 #pragma unroll
             for (int t = 0; t < SLOTS; ++t)
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s[kt][t][i] = nearer(s[kt][t][i], far, qpos[t] - (key0 + kt * 16 + g * 4 + i));
+                    for (int i = 0; i < 4; ++i) s[kt][t][i] = nearer(s[kt][t][i], far, qpos[t] - (key0 + (kt >> 1) * 32 + g * 8 + (kt & 1) * 4 + i));
         if (key0 + 63 > pos0 + qw)  // the diagonal
 #pragma unroll
             for (int t = 0; t < SLOTS; ++t)
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s[kt][t][i] = key0 + kt * 16 + g * 4 + i > qpos[t] ? -INFINITY : s[kt][t][i];
+                    for (int i = 0; i < 4; ++i) s[kt][t][i] = key0 + (kt >> 1) * 32 + g * 8 + (kt & 1) * 4 + i > qpos[t] ? -INFINITY : s[kt][t][i];
         if (key0 < w_last)  // an earlier chunk of some of the queries
 #pragma unroll
             for (int t = 0; t < SLOTS; ++t)
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s[kt][t][i] = key0 + kt * 16 + g * 4 + i < qfirst[t] ? -INFINITY : s[kt][t][i];
+                    for (int i = 0; i < 4; ++i) s[kt][t][i] = key0 + (kt >> 1) * 32 + g * 8 + (kt & 1) * 4 + i < qfirst[t] ? -INFINITY : s[kt][t][i];
         float mn[SLOTS];
         bool grows = false;
 #pragma unroll
@@ -1121,7 +1179,6 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
                 for (int v = 0; v < NV; ++v) o[v][t] *= al;
             }
         }
-        SplitFrag pf[2][SLOTS];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
@@ -1135,19 +1192,13 @@ __global__ __launch_bounds__(256 * G, NV > 8 || NK > 4 ? 1 : 2) void k_gqa_prefi
                 }
                 pf[ks][t] = split8(w[0], w[1]);
             }
-#pragma unroll
-        for (int v = 0; v < NV; ++v)
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                const uint8_t *row = lv + (v * 16 + r16) * VS + ks * 64 + g * 8;
-                const u32x2 a0 = *reinterpret_cast<const u32x2 *>(row), a1 = *reinterpret_cast<const u32x2 *>(row + 32);
-                const bf16x8 a = __builtin_bit_cast(bf16x8, u32x4{a0.x, a0.y, a1.x, a1.y});
-#pragma unroll
-                for (int t = 0; t < SLOTS; ++t) {
-                    o[v][t] = mfma_bf16(a, pf[ks][t].hi, o[v][t]);
-                    o[v][t] = mfma_bf16(a, pf[ks][t].lo, o[v][t]);
-                }
-            }
+        }
+        if (BUFS == 2) {
+            at ^= TILE;
+            if (kt0 + G < n_tiles) store(at);
+            if (kt0 + 2 * G < n_tiles) fetch(key0 + 2 * G * 64);
+        }
+        if (seen) values(kt_ + KB);
     }
     if (G == 2) {
         f32x4 *po = reinterpret_cast<f32x4 *>(lds);                                       // [wave][slot][NV][lane]
@@ -1228,9 +1279,9 @@ thread_local int g_last_gqa_groups;
 
 // Two groups fill a CU, and halve its walks; of one group two workgroups fit.  They pay while the launch is as long as its longest walk: with four tiles or more in it, a CU's
 // share of all tiles not much above it, and no second round behind walks that are all long (the shortest walk of the first round and the longest of the second one in turn).
-// Heads count as a multiple of eight, as the launch deals them to the XCDs (20 heads take what 24 do).  us with two / with one, measured over 200 shapes: 12 heads, 3000 tokens
-// 90 / 118 (share / walk 0.8), 32 heads, 2048 77 / 90 (1.06), 40 heads, 1664 73 / 73 (1.09), 24 heads, 3328 147 / 138 (1.27), 4096 207 / 169 (1.55); two maps, 24 heads, 1280 50 / 57,
-// 1531 71 / 68, 2048 113 / 94; 10 blocks of 24 heads behind 2700 keys (240 workgroups) 119 / 150, 11 blocks 168 / 161; one tile 8.8 / 7.2, three 12.2 / 11.8, five 15.6 / 16.3.
+// Heads count as a multiple of eight, as the launch deals them to the XCDs (20 heads take what 24 do).  us with two / with one: 24 heads, 2600 tokens
+// 80 / 90 (share / walk 1.05), 32 heads, 2048 63 / 75 (1.06), 40 heads, 1664 63 / 62 (1.09), 24 heads, 3000 105 / 105 (1.19), 3328 124 / 121 (1.27), 4096 173 / 153 (1.55); two maps,
+// 24 heads, 1280 39 / 44, 1531 57 / 53, 2048 88 / 75; five tiles 13.1 / 13.9, four 13.0 / 12.4.
 static bool two_groups(const Gqa &g, int rows, int n_ctx, int nq) {
     const int at_once = 256, pos0 = n_ctx - nq, heads = ((int)g.heads + 7) / 8 * 8, blocks = (nq + rows - 1) / rows, all_tiles = (n_ctx + 63) / 64;
     long longest = 0, total = 0, second = 0;
@@ -1288,15 +1339,16 @@ __global__ __launch_bounds__(256) void k_gqa_merge_parts(Gqa p, const float *rec
 
 // Few queries behind many keys: a launch whose blocks leave CUs without a workgroup lasts as long as its longest walk, so a block's tiles are cut into stretches, of two tiles (a step of two
 // groups) at least and no more of them than there are CUs for (heads count as a multiple of eight, as the launch deals them to the XCDs: 12 heads in 21 stretches take 32 us where 15 take 24).
-// A step of a walk takes 4.1 us, the launch that puts the records together 5 and 0.8 ns for each query's head and map.  us without / with, heads, keys, queries: 12, 2090, 90 64 / 20; 24, 2090, 90
-// 64 / 24; 12, 600, 20 22.6 / 12.8; 12, 1000, 200 34.2 / 19.7; 12, 450, 130 20.7 / 15.8; 12, 1000, 1000 34.6 / 31.5; 12, 8000, 30 214 / 38; 24 of two maps, 2090, 90 59 / 30; 2 of 256 columns,
-// 2000, 50 162 / 24.  Queries without many keys stay: 24, 1531, 1531 50, in two stretches where CUs hold two workgroups 52; 12, 100, 3 8.4.
+// A step of a walk that is saved is worth 2.7 us (7 of one group); the launch that puts the records together costs 5 and 0.7 ns for each query's head, 1.4 for each of a head's two maps.
+// us without / with, heads, keys, queries: 12, 2090, 90 51 / 18; 24, 2090, 90 52 / 22; 12, 600, 20 18.3 / 11.1; 12, 1000, 200 28.7 / 18.9; 12, 450, 130 17.7 / 14.5; 12, 8000, 30 168 / 27;
+// 24 of two maps, 2090, 90 49 / 28; 2 of 256 columns, 2000, 50 131 / 22; 8, 2000, 2000 50 / 40.  What stays whole: 12, 400, 400 15.9 / 18.1; 16, 512, 512 18.6 / 21.2; 24 of two maps,
+// 600, 100 18.3 / 20.6; 12, 100, 3 8.4.
 static int gqa_prefill_parts(const Gqa &g, int n_ctx, int nq) {
     const int rows = g.maps == 2 ? 64 : 128, blocks = (nq + rows - 1) / rows, heads = ((int)g.heads + 7) / 8 * 8;
     const int tiles = (n_ctx + 63) / 64 - (gqa_first(g, n_ctx - nq + (blocks - 1) * rows) >> 6), most = std::min<long>(256 / ((long)heads * blocks), 32);
     if (most < 2) return 1;
     const int each = ((tiles + most - 1) / most + 1) & ~1, saved = (tiles + 1) / 2 - each / 2;
-    return 4.1 * saved > 5.0 + 8e-4 * (double)nq * (double)(g.heads * g.maps) ? (tiles + each - 1) / each : 1;
+    return 2.7 * saved > 5.0 + (g.maps == 2 ? 1.4e-3 : 7e-4) * (double)nq * (double)(g.heads * g.maps) ? (tiles + each - 1) / each : 1;
 }
 size_t gqa_prefill_floats(const Gqa &g, int n_ctx, int nq) {
     const int parts = gqa_prefill_parts(g, n_ctx, nq);
@@ -1309,7 +1361,7 @@ static hipError_t gqa_prefill_go(const Gqa &g, const uint16_t *q, size_t ldq, in
     if constexpr (G == 2)
         if (parts == 1 && !two_groups(g, rows, n_ctx, nq)) return gqa_prefill_go<NK, NV, 1>(g, q, ldq, n_ctx, nq, out, ldo, nullptr, s);
     g_last_gqa_groups = G;
-    const size_t tiles = G * ((size_t)g.maps * 64 * (NK * 64 + 16) + (size_t)NV * 16 * (64 * 2 + 16)), sums = G == 2 ? (size_t)4 * 2 * 64 * (NV * 16 + 8) : 0;
+    const size_t tiles = (size_t)G * prefill_buffers(NK, NV, (int)g.maps) * ((size_t)g.maps * 64 * (NK * 64 + 32) + (size_t)NV * 16 * (64 * 2 + 32)), sums = G == 2 ? (size_t)4 * 2 * 64 * (NV * 16 + 8) : 0;
     const size_t lds = tiles > sums ? tiles : sums;
     auto fn = g.maps == 2 ? k_gqa_prefill<NK, NV, 2, false, G> : g.far_weight || g.gate_columns ? k_gqa_prefill<NK, NV, 1, true, G> : k_gqa_prefill<NK, NV, 1, false, G>;
     if (lds > 65536) {
