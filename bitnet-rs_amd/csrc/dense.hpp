@@ -441,6 +441,18 @@ __device__ __forceinline__ float activate(float v, int act, float a, float b) {
     return act == BITNET_HIP_ACT_XIELU ? 0.5f * v + (v > 0.f ? a * v * v : b * (expm1f(v) - v)) : activate(v, act);
 }
 
+// The order of a chain of products whose operands come from LDS: AHEAD reads, then PER products and the next read in turn.  Left to itself the compiler asks for two operands and waits for them.
+template <int READS, int PER, int AHEAD>
+__device__ __forceinline__ void reads_ahead() {
+    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+#pragma unroll
+    for (int i = 0; i < READS - AHEAD; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, PER * AHEAD, 0);
+}
+
 // The order of the workgroups of a launch over records of keys of which the device alone knows how many there are: eight records of all members (heads, queries), then the next eight, so
 // that what exists comes first and what ends at once comes last.  As the fastest index the 128 records of a head, most of them to end, lay ahead of the next head's: 24 heads of 128 columns
 // (bf16) at 200 keys 52 -> 22 us, at 2000 keys 53 -> 27, 16 queries at 200 keys 361 -> 36; at 8000 keys, where nearly all exist, 55.9 -> 56.8.

@@ -981,18 +981,6 @@ hipError_t launch_gqa_project(const GqaOut &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// The order of a chain of products whose operands come from LDS: AHEAD reads, then PER products and the next read in turn.  Left to itself the compiler asks for two operands and waits for them.
-template <int READS, int PER, int AHEAD>
-__device__ __forceinline__ void reads_ahead() {
-    __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
-#pragma unroll
-    for (int i = 0; i < READS - AHEAD; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-    __builtin_amdgcn_sched_group_barrier(0x008, PER * AHEAD, 0);
-}
-
 // buffers of a tile in LDS: two where the two tiles that are under way on a compute unit (one of the largest heads) leave room
 constexpr int prefill_buffers(int nk, int nv, int maps) { return (nv > 8 || nk > 4 ? 2 : 4) * (maps * 64 * (nk * 64 + 32) + nv * 16 * (64 * 2 + 32)) <= 163840 ? 2 : 1; }
 

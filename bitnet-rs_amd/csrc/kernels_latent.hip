@@ -27,6 +27,23 @@ __device__ __forceinline__ float rotated(const T *q, const float *cs, const floa
     return (x * cs[c] + (a < half ? -y : y) * s) * live;
 }
 
+// eight neighbours of it, i and half multiples of eight and rows and tables on 16 bytes: six loads where the elements one by one take 32, each with a wait of its own
+__device__ __forceinline__ bf16x8 rotated8(const uint16_t *q, const float *cs, const float *sn, int half, int i, float sign) {
+    const int n = 2 * half, a = min(i, n - 8), b = a < half ? a + half : a - half, c = a < half ? a : a - half;
+    const u32x4 xv = *reinterpret_cast<const u32x4 *>(q + a), yv = *reinterpret_cast<const u32x4 *>(q + b);
+    const f32x4 c0 = *reinterpret_cast<const f32x4 *>(cs + c), c1 = *reinterpret_cast<const f32x4 *>(cs + c + 4), s0 = *reinterpret_cast<const f32x4 *>(sn + c),
+                s1 = *reinterpret_cast<const f32x4 *>(sn + c + 4);
+    const float live = i < n ? sign : 0.0f;
+    bf16x8 r;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float x = bf2f(xv[e >> 1] >> (e & 1) * 16 & 0xffff), y = bf2f(yv[e >> 1] >> (e & 1) * 16 & 0xffff);
+        const float k = e < 4 ? c0[e & 3] : c1[e & 3], s = e < 4 ? s0[e & 3] : s1[e & 3];
+        r[e] = (__bf16)((x * k + (a < half ? -y : y) * s) * live);
+    }
+    return r;
+}
+
 // (no canonicalising v_max of an MFMA result ahead of it; no NaNs here)
 __device__ __forceinline__ float max3(float a, float b, float c) {
     float r;
@@ -426,11 +443,14 @@ hipError_t launch_latent_merge(const LatentMerge &a, hipStream_t s) {
 
 // ---- prompt -----------------------------------------------------------------------------------------------------------
 // One workgroup: one head, 64 QT queries, four waves of 16 QT; key tiles of 64 staged through registers into LDS one step ahead.
+// Rows of a tile 32 bytes past a multiple of 64 apart, keys in the order in which a lane's weights are eight neighbours and operands read four ahead of their products, as in k_gqa_prefill;
+// 16 heads of 192 + 64 columns and values of 256, 3000 tokens 298 -> 226 us, 24 heads of 128 + 64 and 128 at 2000 tokens 117 -> 113.  The queries' rotated part by eight elements where the
+// tables allow it: one by one it was 128 loads, each waited for, 9 us ahead of every walk: 20 heads at 61 tokens 17.1 -> 8.4 us, 24 at 2000 113 -> 94.6, at 4096 226 -> 191.
 // NK: 32-column steps of a key (dimp + ldr), NV: 16-row tiles of V^T.
 template <int NK, int NV, int QT>
 __global__ __launch_bounds__(256, NV > 8 ? 1 : QT == 1 ? 3 : 2) void k_latent_prefill(LatentAttn p, int n_qb) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    constexpr int KS = NK * 64 + 16, VS = kLatentTile * 2 + 16, NVL = NV / 2;
+    constexpr int KS = NK * 64 + 32, VS = kLatentTile * 2 + 32, NVL = NV / 2;
     uint8_t *lk = lds, *lv = lds + kLatentTile * KS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g = lane >> 4;
     // Consecutive workgroups go to the eight XCDs in turn.  Longest blocks first; an XCD keeps heads / 8 heads of its own (their keys
@@ -442,6 +462,7 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : QT == 1 ? 3 : 2) void k_latent_pr
     const int q0 = qb * 64 * QT, pos0 = p.n_ctx - p.nq;
     const int qw = q0 + wave * 16 * QT;  // this wave's first query
     const int half = p.rot_dim / 2;
+    const bool by_eight = half > 0 && half % 8 == 0 && (((uintptr_t)p.rope_cos | (uintptr_t)p.rope_sin | (uintptr_t)p.qb | p.ldq * 2) & 15) == 0;
     bf16x8 qf[QT][NK];
     int qpos[QT];
 #pragma unroll
@@ -460,8 +481,13 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : QT == 1 ? 3 : 2) void k_latent_pr
 #pragma unroll
                     for (int e = 0; e < 8; ++e) qf[t][kk][e] = -qf[t][kk][e];
             } else {
+                if (by_eight) {
+                    const bf16x8 v = rotated8(q + p.dimp, cs, sn, half, d - p.dimp, sign);
+                    qf[t][kk] = v;
+                } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) qf[t][kk][e] = (__bf16)(sign * rotated(q + p.dimp, cs, sn, half, d + e - p.dimp));
+                    for (int e = 0; e < 8; ++e) qf[t][kk][e] = (__bf16)(sign * rotated(q + p.dimp, cs, sn, half, d + e - p.dimp));
+                }
             }
         }
     }
@@ -485,6 +511,7 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : QT == 1 ? 3 : 2) void k_latent_pr
     // columns: one address form per step); eight threads per row of V^T
     const unsigned koff = (unsigned)((tid >> 2) * ldk * 2 + (tid & 3) * 16), roff = (unsigned)((tid >> 2) * p.ldr * 2 + (tid & 3) * 16);
     const unsigned voff = (unsigned)((tid >> 3) * p.ldvt * 2 + (tid & 7) * 16);
+    const int key = tid >> 2, krow = (key & 32) + (key >> 2 & 1) * 16 + (key >> 3 & 3) * 4 + (key & 3);  // row i of 32 in LDS: key 8 (i >> 2 & 3) + 4 (i >> 4) + (i & 3)
     auto fetch = [&](int key0) {
         const char *kb = (const char *)(K + (size_t)key0 * ldk), *rb = (const char *)(R + (size_t)key0 * p.ldr), *vb = (const char *)(V + key0);
 #pragma unroll
@@ -508,7 +535,7 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : QT == 1 ? 3 : 2) void k_latent_pr
         const int key0 = kt0 * kLatentTile;
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < NK; ++j) *reinterpret_cast<u32x4 *>(lk + (tid >> 2) * KS + j * 64 + (tid & 3) * 16) = kreg[j];
+        for (int j = 0; j < NK; ++j) *reinterpret_cast<u32x4 *>(lk + krow * KS + j * 64 + (tid & 3) * 16) = kreg[j];
 #pragma unroll
         for (int j = 0; j < NVL; ++j) *reinterpret_cast<u32x4 *>(lv + ((tid >> 3) + 32 * j) * VS + (tid & 7) * 16) = vreg[j];
         __syncthreads();
@@ -526,13 +553,15 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : QT == 1 ? 3 : 2) void k_latent_pr
                 for (int t = 0; t < QT; ++t) s[kt][t] = mfma_bf16(a, qf[t][kk], s[kt][t]);
             }
         }
+        reads_ahead<4 * NK, QT, 4>();
+        __builtin_amdgcn_sched_barrier(0);
         if (key0 + kLatentTile - 1 > pos0 + qw)  // the diagonal
 #pragma unroll
             for (int t = 0; t < QT; ++t)
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) s[kt][t][i] = key0 + kt * 16 + g * 4 + i > qpos[t] ? -INFINITY : s[kt][t][i];
+                    for (int i = 0; i < 4; ++i) s[kt][t][i] = key0 + (kt >> 1) * 32 + g * 8 + (kt & 1) * 4 + i > qpos[t] ? -INFINITY : s[kt][t][i];
         float mn[QT];
         bool grows = false;
 #pragma unroll
@@ -583,15 +612,14 @@ __global__ __launch_bounds__(256, NV > 8 ? 1 : QT == 1 ? 3 : 2) void k_latent_pr
         for (int v = 0; v < NV; ++v)
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
-                const uint8_t *row = lv + (v * 16 + r16) * VS + ks * 64 + g * 8;
-                const u32x2 a0 = *reinterpret_cast<const u32x2 *>(row), a1 = *reinterpret_cast<const u32x2 *>(row + 32);
-                const bf16x8 a = __builtin_bit_cast(bf16x8, u32x4{a0.x, a0.y, a1.x, a1.y});
+                const bf16x8 a = *reinterpret_cast<const bf16x8 *>(lv + (v * 16 + r16) * VS + ks * 64 + g * 16);
 #pragma unroll
                 for (int t = 0; t < QT; ++t) {
                     o[v][t] = mfma_bf16(a, ph[ks][t], o[v][t]);
                     o[v][t] = mfma_bf16(a, pl[ks][t], o[v][t]);
                 }
             }
+        reads_ahead<NV * 2, 2 * QT, 4>();
     }
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
@@ -613,7 +641,7 @@ bool latent_prefill_supported(int qd, int vdimp) { return qd <= 256 && vdimp <= 
 template <int NK, int NV, int QT>
 static hipError_t prefill_go(const LatentAttn &a, hipStream_t s) {
     const int n_qb = (a.nq + 64 * QT - 1) / (64 * QT);
-    const size_t lds = (size_t)kLatentTile * (NK * 64 + 16) + (size_t)NV * 16 * (kLatentTile * 2 + 16);
+    const size_t lds = (size_t)kLatentTile * (NK * 64 + 32) + (size_t)NV * 16 * (kLatentTile * 2 + 32);
     if (lds > 65536) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k_latent_prefill<NK, NV, QT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
