@@ -232,6 +232,7 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
             ++i;
         }
     }
+    if (n > 0) ran(with_logits);
     HCHK(hipEventRecord(end_.e, s));
     if (int rc = settle()) return rc;
     moved_to(p + n);

@@ -96,6 +96,7 @@ class Sequence {
     virtual int step(bool with_logits, int form) = 0;          // the launches of one single-token step
     virtual int form_at(int) const { return 0; }               // which form of them a step at this position takes
     virtual bool chains() const { return false; }              // can a step with logits embed the next position's token?
+    virtual void ran(bool) {}                                  // the launches of steps, with logits or without, are out: replayed, or by step() itself
     virtual int clear_state() { return 0; }
 
     bool dead_ = true;

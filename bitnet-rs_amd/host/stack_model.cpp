@@ -965,10 +965,9 @@ int StackModel::step(bool with_logits, int form) {
             BCHK(bitnet_hip_dense_logits_embed_dev(&in, head_m_.w, vocab_, head_m_.cols, head_m_.ld, logits_, argmax_, token_, pos_, history_, n_forced_, &next, stream_));
         else
             BCHK(bitnet_hip_dense_logits_dev(&in, head_m_.w, vocab_, head_m_.cols, head_m_.ld, logits_, argmax_, token_, pos_, history_, n_forced_, stream_));
-        hidden_ = cur_;
+        step_hidden_ = cur_;
     } else {
         BCHK(bitnet_hip_advance_pos_dev(pos_, stream_));
-        hidden_ = nullptr;  // the last sublayer's output was not added: nobody asked for it
     }
     return 0;
 }
@@ -977,6 +976,7 @@ int StackModel::step(bool with_logits, int form) {
 
 int StackModel::portion_buffers(size_t n) {
     if (n <= rows_cap_) return 0;
+    hidden_ = nullptr;  // (it may lie in what is given back here)
     n = up_to(n, 64);
     const size_t es = f32_ ? 4 : 2;
     size_t z = 0, cq = 0, q = 0, qabs = 0, att = 0, act = 0, k = 0, vt = 0, lin = 0, linf = 0, lino = 0, gate = 0, ws = 0, scratch = 0, qf = 0;

@@ -151,6 +151,7 @@ class StackModel : public Sequence {
     bool ready() const override { return head_ != nullptr && layers_set_ == spec_.layers.size(); }
     int step(bool with_logits, int form) override;
     bool chains() const override;
+    void ran(bool with_logits) override { hidden_ = with_logits ? step_hidden_ : nullptr; }  // (without: the last sublayer's output was not added)
     bitnet_hip_embedding embedding(float *out) const;
     int form_at(int pos) const override;  // how a step's attention records are merged: kStepRecords
     int clear_state() override;
@@ -314,6 +315,7 @@ class StackModel : public Sequence {
     float *next_x() const { return cur_ == x_[0] ? x_[1] : x_[0]; }
     Pending pending_;
     const float *hidden_ = nullptr;  // residual stream of the last position run
+    const float *step_hidden_ = nullptr;  // where every step with logits leaves it
     // portion buffers; T = bf16, or f32 in 32-bit mode
     size_t rows_cap_ = 0;
     Buffer px_, ph_, pz_, pcq_, pq_, pqf_, pqabs_, patt_, py_, pact_, pk_, pvt_, plin_, plinf_, plino_, pgate_, pscratch_, plws_, pwant_, pxw_, phw_, plog_;

@@ -37,3 +37,27 @@ def test_chained_steps(pkg, tmp_path, design, fed, prompt, steps):
             at += n
             assert np.array_equal(m.last_logits(), one[at - 1])
         assert np.array_equal(m.history(prompt + steps + 1), history)
+
+
+@pytest.mark.parametrize("design", ["lasapel", "lurepel"])
+def test_last_hidden_of_replayed_steps(pkg, tmp_path, design):
+    """the row of the last position, not of the prompt, on every sequence of a model: as steps without graphs leave it"""
+    config = getattr(synth, design + "_config")("1b", 2)
+    config["vocab"] = 640
+    getattr(synth, "write_" + design)(str(tmp_path), config)
+    m = pkg.open_model(str(tmp_path), max_pos=256)
+    tokens = np.random.default_rng(3).integers(0, 640, 20).astype(np.int32)
+    for again in range(2):
+        for n in (1, 9):
+            rows = []
+            for use_graph in (False, True):
+                m.reset()
+                m.feed(tokens)
+                m.prefill(6, with_logits=True, digits=2)
+                prompt = m.last_hidden()
+                m.run(n, use_graph=use_graph)
+                rows.append(m.last_hidden())
+            assert np.array_equal(*rows) and not np.array_equal(prompt, rows[1])
+        m.run(1, with_logits=False)
+        with pytest.raises(pkg.BitNetHipError, match="without logits"):
+            m.last_hidden()
