@@ -155,18 +155,24 @@ int Sequence::ensure_graph(bool with_logits, int form) {
     HCHK(hipGraphInstantiate(&ex, g, nullptr, nullptr, 0));
     graph_[gi] = g;
     graph_exec_[gi] = ex;
-    return 0;
-}
-
-int Sequence::ensure_chain(int form) {
-    if (int rc = ensure_graph(true, form)) return rc;
-    if (!chain_steps_) {
+    if (with_logits && !chain_steps_) {
         size_t nodes = 0;
-        HCHK(hipGraphGetNodes((hipGraph_t)graph_[2 * form + 1], nullptr, &nodes));
+        HCHK(hipGraphGetNodes(g, nullptr, &nodes));
         const int fit = nodes ? (int)(kChainNodes / nodes) : 1;
         chain_steps_ = !chains() || fit < 1 ? 1 : fit < kChainMost ? fit : kChainMost;
     }
-    if (chain_steps_ < 2 || chain_exec_[form]) return 0;
+    return 0;
+}
+
+int Sequence::steps_together(const int *forms, int n) {
+    if (chain_steps_ < 2 || chain_steps_ > n) return 1;
+    for (int k = 1; k < chain_steps_; ++k)
+        if (forms[k] != forms[0]) return 1;
+    return ensure_chain(forms[0]) == 0 ? chain_steps_ : 1;
+}
+
+int Sequence::ensure_chain(int form) {
+    if (chain_exec_[form]) return 0;
     hipStream_t s = (hipStream_t)stream_;
     hipGraph_t g = nullptr;
     HCHK(hipStreamBeginCapture(s, hipStreamCaptureModeGlobal));
@@ -205,17 +211,12 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
     if (int rc = check_run(n, with_logits)) return rc;
     const int p = position();
     hipStream_t s = (hipStream_t)stream_;
-    // steps from i on that one graph makes
-    auto together = [&](int i) {
-        const int form = form_at(p + i);
-        if (!with_logits || n - i < 2 || ensure_chain(form) != 0 || chain_steps_ < 2 || i + chain_steps_ > n) return 1;
-        for (int k = 1; k < chain_steps_; ++k)
-            if (form_at(p + i + k) != form) return 1;
-        return chain_steps_;
-    };
+    std::vector<int> forms((size_t)n);
+    for (int i = 0; i < n; ++i) forms[(size_t)i] = form_at(p + i);
+    auto together = [&](int i) { return with_logits ? steps_together(&forms[(size_t)i], n - i) : 1; };
     if (use_graph) {
         for (int i = 0; i < n; i += together(i)) {  // every form this run needs
-            int rc = ensure_graph(with_logits, form_at(p + i));
+            int rc = ensure_graph(with_logits, forms[(size_t)i]);
             if (rc) return rc;
         }
     }
@@ -223,11 +224,11 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
     HCHK(hipEventRecord(begin_.e, s));
     for (int i = 0; i < n;) {
         if (use_graph) {
-            const int form = form_at(p + i), k = together(i);
+            const int form = forms[(size_t)i], k = together(i);
             HCHK(hipGraphLaunch((hipGraphExec_t)(k > 1 ? chain_exec_[form] : graph_exec_[2 * form + (with_logits ? 1 : 0)]), s));
             i += k;
         } else {
-            int rc = step(with_logits, form_at(p + i));
+            int rc = step(with_logits, forms[(size_t)i]);
             if (rc) return rc;
             ++i;
         }

@@ -81,6 +81,7 @@ class Sequence {
     int check_run(int n, bool with_logits);
     int ensure_graph(bool with_logits, int form);
     int ensure_chain(int form);
+    int steps_together(const int *forms, int n);  // of the next n steps, which take these forms: as many as one graph makes
     void drop_graphs();
     int settle();                       // waits for the stream
     void moved_to(int p) { host_pos_ = exposed_ ? -1 : p; }
@@ -120,7 +121,7 @@ class Sequence {
     static constexpr int kChainNodes = 192, kChainMost = 4;
     bool follows_ = false, followed_ = false;  // of the step at hand: the one ahead has embedded its token; it embeds the next one's
     void *chain_exec_[kForms] = {}, *chain_graph_[kForms] = {};
-    int chain_steps_ = 0;  // (0: not known yet)
+    int chain_steps_ = 0;  // (0: not known yet, no step with logits has been captured)
     void *graph_exec_[2 * kForms] = {};  // [2 * form + with_logits]
     void *graph_[2 * kForms] = {};
 };

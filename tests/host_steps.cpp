@@ -194,9 +194,30 @@ int last_row() {
     return 0;
 }
 
+// several steps make one graph where as many are asked for and all of one form; nothing is captured that is not launched
+int chain_use() {
+    Model m(600);
+    START(m);
+    CHECK(m.start(590, 4) == 0);
+    for (int n : {1, 2, 3}) CHECK(m.run(n, true, true, nullptr) == 0 && g_made.size() == 1);
+    const size_t one = g_made[0], four = 4 * one - 3;  // (three embeddings go with the logits ahead of them)
+    g_replayed.clear();
+    CHECK(m.run(9, true, true, nullptr) == 0 && g_made.size() == 2 && g_made[1] == four && g_replayed == (std::vector<size_t>{four, four, one}));
+    CHECK(m.start(590, 254) == 0);  // behind two steps the next form
+    g_made.clear(), g_replayed.clear();
+    CHECK(m.run(5, true, true, nullptr) == 0 && g_made == std::vector<size_t>{one} && g_replayed == std::vector<size_t>(5, one));
+    CHECK(m.run(4, false, true, nullptr) == 0 && g_replayed.size() == 9);
+    g_follows = false;
+    Model alone(600);
+    START(alone);
+    CHECK(alone.start(590, 4) == 0 && alone.run(20, true, true, nullptr) == 0 && g_made.size() == 1 && g_replayed == std::vector<size_t>(20, g_made[0]));
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, int (*)()> cases = {
         {"last_row", last_row},
+        {"chain_use", chain_use},
     };
     const auto it = cases.find(argc > 1 ? argv[1] : "");
     CHECK(it != cases.end());

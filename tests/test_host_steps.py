@@ -37,3 +37,7 @@ def check(program, case):
 
 def test_last_hidden_is_of_the_position_that_ran_last(program):
     check(program, "last_row")
+
+
+def test_steps_make_one_graph_where_it_is_launched(program):
+    check(program, "chain_use")
