@@ -52,7 +52,7 @@ void Sequence::drop_graphs() {
     for (int i = 0; i < kForms; ++i) {
         if (chain_exec_[i]) hipGraphExecDestroy((hipGraphExec_t)chain_exec_[i]);
         if (chain_graph_[i]) hipGraphDestroy((hipGraph_t)chain_graph_[i]);
-        chain_exec_[i] = chain_graph_[i] = nullptr;
+        chain_exec_[i] = chain_graph_[i] = nullptr, chain_refused_[i] = false;
     }
     chain_steps_ = 0;
 }
@@ -168,7 +168,13 @@ int Sequence::steps_together(const int *forms, int n) {
     if (chain_steps_ < 2 || chain_steps_ > n) return 1;
     for (int k = 1; k < chain_steps_; ++k)
         if (forms[k] != forms[0]) return 1;
-    return ensure_chain(forms[0]) == 0 ? chain_steps_ : 1;
+    if (chain_refused_[forms[0]]) return 1;
+    const std::string err = err_;
+    if (ensure_chain(forms[0]) == 0) return chain_steps_;
+    chain_refused_[forms[0]] = true;  // (steps one by one do the same: nobody's error)
+    (void)hipGetLastError();
+    err_ = err;
+    return 1;
 }
 
 int Sequence::ensure_chain(int form) {

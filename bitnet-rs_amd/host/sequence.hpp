@@ -121,6 +121,7 @@ class Sequence {
     static constexpr int kChainNodes = 192, kChainMost = 4;
     bool follows_ = false, followed_ = false;  // of the step at hand: the one ahead has embedded its token; it embeds the next one's
     void *chain_exec_[kForms] = {}, *chain_graph_[kForms] = {};
+    bool chain_refused_[kForms] = {};  // could not be made (memory): not tried again until the graphs are dropped
     int chain_steps_ = 0;  // (0: not known yet, no step with logits has been captured)
     void *graph_exec_[2 * kForms] = {};  // [2 * form + with_logits]
     void *graph_[2 * kForms] = {};

@@ -214,10 +214,24 @@ int chain_use() {
     return 0;
 }
 
+// a chain that cannot be made is tried once, its error is nobody's, and the steps run one by one
+int chain_refused() {
+    Model m(600);
+    START(m);
+    g_largest_graph = 8;
+    for (int again = 0; again < 3; ++again) {
+        CHECK(m.start(200, 4) == 0 && m.run(20, true, true, nullptr) == 0 && m.position() == 24 && m.last() == m.tokens[23]);
+        CHECK(g_made.size() == 2 && g_made[0] <= 8 && g_made[1] > 8 && m.error().empty() && g_last_error == hipSuccess);
+        for (size_t n : g_replayed) CHECK(n == g_made[0]);
+    }
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, int (*)()> cases = {
         {"last_row", last_row},
         {"chain_use", chain_use},
+        {"chain_refused", chain_refused},
     };
     const auto it = cases.find(argc > 1 ? argv[1] : "");
     CHECK(it != cases.end());

@@ -41,3 +41,7 @@ def test_last_hidden_is_of_the_position_that_ran_last(program):
 
 def test_steps_make_one_graph_where_it_is_launched(program):
     check(program, "chain_use")
+
+
+def test_a_graph_of_several_steps_that_cannot_be_made_is_tried_once(program):
+    check(program, "chain_refused")
