@@ -3,7 +3,6 @@
 
 #include <cstdio>
 #include <cstring>
-#include <vector>
 
 namespace bitnet_host {
 
@@ -130,11 +129,19 @@ int Sequence::last_logits(float *out) {
 
 int Sequence::prepare_graphs(bool with_logits) {
     if (!ready()) return fail_arg("model globals not set");
-    unsigned forms = 0;
-    for (int pos = 0; pos + 1 < max_pos_; ++pos) forms |= 1u << form_at(pos);
-    for (int f = 0; f < kForms; ++f)
-        if (forms & (1u << f))
-            if (int rc = ensure_graph(with_logits, f)) return rc;
+    std::vector<int> forms;
+    for (int pos = 0; pos + 1 < max_pos_; ++pos) forms.push_back(form_at(pos));
+    return make_graphs(forms, with_logits, true);
+}
+
+// what steps of these forms, one behind the other, are launched with; any: from wherever a run may start among them, and however far it may go
+int Sequence::make_graphs(const std::vector<int> &forms, bool with_logits, bool any) {
+    const int n = (int)forms.size();
+    for (int i = 0, k; i < n; i += k) {
+        if (int rc = ensure_graph(with_logits, forms[(size_t)i])) return rc;
+        k = with_logits ? steps_together(&forms[(size_t)i], n - i) : 1;
+        if (any) k = 1;
+    }
     return 0;
 }
 
@@ -220,12 +227,8 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
     std::vector<int> forms((size_t)n);
     for (int i = 0; i < n; ++i) forms[(size_t)i] = form_at(p + i);
     auto together = [&](int i) { return with_logits ? steps_together(&forms[(size_t)i], n - i) : 1; };
-    if (use_graph) {
-        for (int i = 0; i < n; i += together(i)) {  // every form this run needs
-            int rc = ensure_graph(with_logits, forms[(size_t)i]);
-            if (rc) return rc;
-        }
-    }
+    if (use_graph)
+        if (int rc = make_graphs(forms, with_logits, false)) return rc;
     host_pos_ = -1;
     HCHK(hipEventRecord(begin_.e, s));
     for (int i = 0; i < n;) {

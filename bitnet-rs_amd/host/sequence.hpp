@@ -8,6 +8,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <string>
+#include <vector>
 
 #include <hip/hip_runtime_api.h>
 
@@ -63,8 +64,8 @@ class Sequence {
     virtual int prefill(int n, bool with_logits, int digits, float *elapsed_ms) = 0;
     // The next n tokens of the sequence, forced; logits [n_want][vocab] (host) of the places `want` among them.
     virtual int forward(const int32_t *tokens, int n, const int32_t *want, int n_want, float *logits);
-    // Captures and instantiates the step graph of every form a sequence can reach ahead of time, so that no run() pays for a
-    // capture in the middle of a generation.  Nothing executes.
+    // Captures and instantiates the graphs of a step and of several, of every form a sequence can reach, ahead of time, so that no
+    // run() pays for a capture in the middle of a generation.  Nothing executes.
     int prepare_graphs(bool with_logits);
     int position();                    // tokens consumed so far; -1: it could not be read
     int history(int32_t *out, int n);  // first n tokens of the sequence
@@ -81,6 +82,7 @@ class Sequence {
     int check_run(int n, bool with_logits);
     int ensure_graph(bool with_logits, int form);
     int ensure_chain(int form);
+    int make_graphs(const std::vector<int> &forms, bool with_logits, bool any);
     int steps_together(const int *forms, int n);  // of the next n steps, which take these forms: as many as one graph makes
     void drop_graphs();
     int settle();                       // waits for the stream

@@ -227,11 +227,31 @@ int chain_refused() {
     return 0;
 }
 
+// behind prepare_graphs no run captures anything, wherever it starts and however long it is
+int prepared() {
+    for (int max_pos : {3, 40, 130, 600}) {
+        Model m(max_pos);
+        START(m);
+        CHECK(m.prepare_graphs(true) == 0 && m.prepare_graphs(false) == 0);
+        const size_t made = g_made.size();
+        for (int from = 0; from < max_pos - 1; from += 7)
+            for (int n : {1, 2, 4, 9, max_pos - 1 - from}) {
+                if (from + n > max_pos - 2) continue;
+                CHECK(m.start(max_pos - 2, from) == 0 && m.run(n, true, true, nullptr) == 0 && m.last() == m.tokens[(size_t)(from + n - 1)]);
+                CHECK(m.start(max_pos - 2, from) == 0 && m.run(n, false, true, nullptr) == 0);
+            }
+        CHECK(g_made.size() == made);
+        for (size_t a : g_made) CHECK(max_pos > 4 || a <= g_made[0]);  // no chain where no sequence has room for one
+    }
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, int (*)()> cases = {
         {"last_row", last_row},
         {"chain_use", chain_use},
         {"chain_refused", chain_refused},
+        {"prepared", prepared},
     };
     const auto it = cases.find(argc > 1 ? argv[1] : "");
     CHECK(it != cases.end());

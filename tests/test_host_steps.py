@@ -45,3 +45,7 @@ def test_steps_make_one_graph_where_it_is_launched(program):
 
 def test_a_graph_of_several_steps_that_cannot_be_made_is_tried_once(program):
     check(program, "chain_refused")
+
+
+def test_no_run_captures_behind_prepare_graphs(program):
+    check(program, "prepared")
