@@ -953,6 +953,7 @@ def _host_lib(path: str = HOST_LIB_PATH):
     L.bitnet_host_prefill.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_int, fp]
     L.bitnet_host_forward.argtypes = [C.c_void_p, i32p, C.c_int, i32p, C.c_int, fp]
     L.bitnet_host_prepare_graphs.argtypes = [C.c_void_p, C.c_int]
+    L.bitnet_host_last_graph_steps.argtypes = [C.c_void_p]
     L.bitnet_host_position.argtypes = [C.c_void_p]
     L.bitnet_host_history.argtypes = [C.c_void_p, i32p, C.c_int]
     L.bitnet_host_last_logits.argtypes = [C.c_void_p, _f32p]
@@ -1028,6 +1029,10 @@ class HostSequence:
     def prepare_graphs(self, with_logits: bool = True) -> None:
         """capture + instantiate the step graph of every form a sequence can reach, ahead of time (nothing executes)"""
         self._check(self.c.bitnet_host_prepare_graphs(self.h, int(with_logits)))
+
+    def last_graph_steps(self) -> int:
+        """the most steps that one graph of the last run made; 0: it launched none"""
+        return int(self.c.bitnet_host_last_graph_steps(self.h))
 
     def position(self) -> int:
         return int(self.c.bitnet_host_position(self.h))

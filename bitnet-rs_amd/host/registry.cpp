@@ -102,6 +102,7 @@ int bitnet_host_forward(void *d, const int32_t *tokens, int n, const int32_t *wa
     SEQ(BITNET_HIP_ERR_INVALID_ARGUMENT);
     return S->forward(tokens, n, want, n_want, logits);
 }
+int bitnet_host_last_graph_steps(void *d) { SEQ(0); return S->last_graph_steps(); }
 int bitnet_host_prepare_graphs(void *d, int with_logits) { SEQ(BITNET_HIP_ERR_INVALID_ARGUMENT); return S->prepare_graphs(with_logits != 0); }
 int bitnet_host_position(void *d) { SEQ(-1); return S->position(); }
 int bitnet_host_history(void *d, int32_t *out, int n) { SEQ(BITNET_HIP_ERR_INVALID_ARGUMENT); return S->history(out, n); }

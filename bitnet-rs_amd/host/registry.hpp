@@ -49,6 +49,7 @@ int bitnet_host_prefill(void *d, int n, int with_logits, int digits, float *elap
 // the next n tokens, forced; logits [n_want][vocab] of the places `want` among them
 int bitnet_host_forward(void *d, const int32_t *tokens, int n, const int32_t *want, int n_want, float *logits);
 int bitnet_host_prepare_graphs(void *d, int with_logits);
+int bitnet_host_last_graph_steps(void *d);  // the most steps that one graph of the last run made; 0: it launched none
 int bitnet_host_position(void *d);
 int bitnet_host_history(void *d, int32_t *out, int n);
 int bitnet_host_last_logits(void *d, float *out);

@@ -230,12 +230,14 @@ int Sequence::run(int n, bool with_logits, bool use_graph, float *elapsed_ms) {
     if (use_graph)
         if (int rc = make_graphs(forms, with_logits, false)) return rc;
     host_pos_ = -1;
+    graph_steps_ = 0;
     HCHK(hipEventRecord(begin_.e, s));
     for (int i = 0; i < n;) {
         if (use_graph) {
             const int form = forms[(size_t)i], k = together(i);
             HCHK(hipGraphLaunch((hipGraphExec_t)(k > 1 ? chain_exec_[form] : graph_exec_[2 * form + (with_logits ? 1 : 0)]), s));
             i += k;
+            if (k > graph_steps_) graph_steps_ = k;
         } else {
             int rc = step(with_logits, forms[(size_t)i]);
             if (rc) return rc;

@@ -67,6 +67,7 @@ class Sequence {
     // Captures and instantiates the graphs of a step and of several, of every form a sequence can reach, ahead of time, so that no
     // run() pays for a capture in the middle of a generation.  Nothing executes.
     int prepare_graphs(bool with_logits);
+    int last_graph_steps() const { return graph_steps_; }  // the most steps that one graph of the last run() made; 0: it launched none
     int position();                    // tokens consumed so far; -1: it could not be read
     int history(int32_t *out, int n);  // first n tokens of the sequence
     int last_logits(float *out);       // [vocab], of the last step run with logits
@@ -125,6 +126,7 @@ class Sequence {
     void *chain_exec_[kForms] = {}, *chain_graph_[kForms] = {};
     bool chain_refused_[kForms] = {};  // could not be made (memory): not tried again until the graphs are dropped
     int chain_steps_ = 0;  // (0: not known yet, no step with logits has been captured)
+    int graph_steps_ = 0;
     void *graph_exec_[2 * kForms] = {};  // [2 * form + with_logits]
     void *graph_[2 * kForms] = {};
 };

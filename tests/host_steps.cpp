@@ -202,7 +202,7 @@ int chain_use() {
     for (int n : {1, 2, 3}) CHECK(m.run(n, true, true, nullptr) == 0 && g_made.size() == 1);
     const size_t one = g_made[0], four = 4 * one - 3;  // (three embeddings go with the logits ahead of them)
     g_replayed.clear();
-    CHECK(m.run(9, true, true, nullptr) == 0 && g_made.size() == 2 && g_made[1] == four && g_replayed == (std::vector<size_t>{four, four, one}));
+    CHECK(m.run(9, true, true, nullptr) == 0 && g_made.size() == 2 && g_made[1] == four && g_replayed == (std::vector<size_t>{four, four, one}) && m.last_graph_steps() == 4);
     CHECK(m.start(590, 254) == 0);  // behind two steps the next form
     g_made.clear(), g_replayed.clear();
     CHECK(m.run(5, true, true, nullptr) == 0 && g_made == std::vector<size_t>{one} && g_replayed == std::vector<size_t>(5, one));
@@ -210,7 +210,7 @@ int chain_use() {
     g_follows = false;
     Model alone(600);
     START(alone);
-    CHECK(alone.start(590, 4) == 0 && alone.run(20, true, true, nullptr) == 0 && g_made.size() == 1 && g_replayed == std::vector<size_t>(20, g_made[0]));
+    CHECK(alone.start(590, 4) == 0 && alone.run(20, true, true, nullptr) == 0 && g_made.size() == 1 && g_replayed == std::vector<size_t>(20, g_made[0]) && alone.last_graph_steps() == 1);
     return 0;
 }
 

@@ -61,3 +61,20 @@ def test_last_hidden_of_replayed_steps(pkg, tmp_path, design):
         m.run(1, with_logits=False)
         with pytest.raises(pkg.BitNetHipError, match="without logits"):
             m.last_hidden()
+
+
+@pytest.mark.parametrize("design", ["lasapel", "mimolix", "lurepel", "sipelorn"])
+def test_steps_are_chained(pkg, tmp_path, design):
+    """one graph does make several steps where as many are asked for, and is there behind prepare_graphs"""
+    config = getattr(synth, design + "_config")("1b", 2 if design != "mimolix" else 4)
+    config["vocab"] = 640
+    getattr(synth, "write_" + design)(str(tmp_path), config)
+    m = pkg.open_model(str(tmp_path), max_pos=128)
+    m.prepare_graphs(True)
+    m.feed(np.arange(40, dtype=np.int32))
+    m.prefill(10, with_logits=True, digits=2)
+    for n in (9, 1, 4):
+        m.run(n)
+        assert (m.last_graph_steps() > 1) == (n > 1)
+    m.run(4, use_graph=False)
+    assert m.last_graph_steps() == 0
