@@ -764,7 +764,7 @@ bool StackModel::merges_in_out(size_t i, int which) const {
     const Block &B = layers_[i].block[which];
     if (f32_ || !B.used || !B.mixer || spec_.layers[i].mixer != LayerSpec::Attention || B.fs > 0 || B.expert_up.w) return false;
     const bitnet_hip_gqa a = gqa_args(i, 0, row_[0], B.main, true);
-    return bitnet_hip_gqa_supported(a.dimp, a.vdimp) && bitnet_hip_gqa_project_records(&a, B.out.cols) >= kMostRecords;
+    return bitnet_hip_gqa_project_records(&a, B.out.cols) >= kMostRecords;
 }
 
 // records of a query at the position, over the layers
@@ -782,7 +782,8 @@ size_t StackModel::records_at(int pos) const {
 
 // (up to twelve records: us of attention and product at 300 / 600 / 1500 keys, merged by a launch / by the product: 12 heads of 128 on 3 14.1 / 14.1 / 14.2 -> 11.9 / 12.2 / 13.0, 24 on 6
 // 17.2 / 17.2 / 17.4 -> 14.3 / 15.3 / 16.2, 32 on 8 at 1500 19.8 -> 19.4; with sixteen requested at once and the rest in turn even at 17, slower from there on.  Records of 256 keys, from twice the
-// waves, would reach 3072 keys: 14.7 -> 13.7 where the keys lie in the L2, but a pass's steps got slower, 7.50 -> 7.69 ms)
+// waves, would reach 3072 keys: 14.7 -> 13.7 where the keys lie in the L2, but a pass's steps got slower, 7.50 -> 7.69 ms.  Heads of more than 256 columns, whose records come from
+// gqa_any, at 100 / 500 / 1500 keys: 8 of 512 69.5 / 85.9 / 88.2 -> 65.7 / 81.8 / 86.4, 12 of 320 50.3 / 61.8 / 63.6 -> 46.7 / 58.6 / 62.6)
 int StackModel::form_at(int pos) const {
     const size_t n = records_at(pos);
     static_assert(sizeof(kStepRecords) / sizeof(kStepRecords[0]) == kForms, "a graph for each");
@@ -822,16 +823,15 @@ int StackModel::step_block(size_t i, int pass, int which) {
         TRY(step_attend_latent(i, pass, proj, S.latent.kv_from < 0 ? &r : nullptr, row, B.ko));
     } else if (B.mixer && S.mixer == LayerSpec::Attention) {
         const bitnet_hip_gqa a = gqa_args(i, pass, proj, B.main, true);
-        if (form_ > 0 && merges_in_out(i, which)) {
-            BCHK(bitnet_hip_gqa_step_dev(&a, proj, pos_, scratch_, stream_));
-            BCHK(bitnet_hip_gqa_project_dev(&a, pos_, kStepRecords[form_], scratch_, B.out.w, B.out.rows, B.out.cols, B.out.ld, B.out_bias, y_[which], stream_));
-            return 0;
-        }
         if (!f32_ && bitnet_hip_gqa_supported(a.dimp, a.vdimp)) {
             BCHK(bitnet_hip_gqa_step_dev(&a, proj, pos_, scratch_, stream_));
         } else {
             BCHK(bitnet_hip_gqa_rows_dev(&a, proj, B.main, 1, f32_, pos_, 1, nullptr, 0, stream_));
             BCHK(bitnet_hip_gqa_any_dev(&a, proj, B.main, 1, f32_, pos_, 0, 1, scratch_, stream_));
+        }
+        if (form_ > 0 && merges_in_out(i, which)) {
+            BCHK(bitnet_hip_gqa_project_dev(&a, pos_, kStepRecords[form_], scratch_, B.out.w, B.out.rows, B.out.cols, B.out.ld, B.out_bias, y_[which], stream_));
+            return 0;
         }
         BCHK(bitnet_hip_gqa_merge_dev(&a, pos_, 0, 1, scratch_, row, B.ko, 0, stream_));
     } else if (B.mixer) {

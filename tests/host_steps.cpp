@@ -246,12 +246,29 @@ int prepared() {
     return 0;
 }
 
+// the output product merges the records, whichever kernel has left them
+int wide_heads() {
+    for (bool narrow : {true, false}) {
+        g_narrow = narrow;
+        Model m(2000, narrow ? 32 : 288);
+        START(m);
+        for (int at : {0, 127, 128, 500, 900, 1500, 1600}) {
+            CHECK(m.reset() == 0 && m.feed(m.tokens.data(), at + 2) == 0 && (at == 0 || m.prefill(at, false, 0, nullptr) == 0));
+            g_done.clear();
+            CHECK(m.run(1, true, true, nullptr) == 0 && count(narrow ? "step" : "any") == 2 && count(narrow ? "any" : "step") == 0);
+            CHECK(count("project") == (at < 1536 ? 2 : 0) && count("merge") == (at < 1536 ? 0 : 2));
+        }
+    }
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, int (*)()> cases = {
         {"last_row", last_row},
         {"chain_use", chain_use},
         {"chain_refused", chain_refused},
         {"prepared", prepared},
+        {"wide_heads", wide_heads},
     };
     const auto it = cases.find(argc > 1 ? argv[1] : "");
     CHECK(it != cases.end());

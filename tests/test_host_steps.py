@@ -49,3 +49,7 @@ def test_a_graph_of_several_steps_that_cannot_be_made_is_tried_once(program):
 
 def test_no_run_captures_behind_prepare_graphs(program):
     check(program, "prepared")
+
+
+def test_output_products_merge_the_records_of_any_head(program):
+    check(program, "wide_heads")

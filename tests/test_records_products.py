@@ -69,3 +69,21 @@ def test_steps_across_the_forms(pkg, tmp_path):
         m.feed(tokens[:at + 5])
         m.prefill(at + 5, with_logits=True, digits=2)
         assert u.rms_error(got, m.last_logits()) < 2e-2, at
+
+
+def test_steps_of_wide_heads_across_the_forms(pkg, tmp_path):
+    """heads of 288 columns, whose records come from gqa_any: the same, a prompt of the last five tokens against steps"""
+    config = u.lurepel([u.chunk_layer(heads=3, kv_heads=1, dim=288, scale=0.05, chunk=4096, dims=64)], width=112, vocab=150)
+    path = u.save_model(str(tmp_path), config, u.random_tensors(config, 8))
+    m = pkg.open_model(path, max_pos=2048)
+    tokens = np.random.default_rng(6).integers(0, 150, 1550).astype(np.int32)
+    for at in (126, 254, 510, 1022, 1534):
+        m.reset()
+        m.feed(tokens[:at + 5])
+        m.prefill(at, with_logits=False, digits=2)
+        m.run(5)
+        got = m.last_logits().copy()
+        m.reset()
+        m.feed(tokens[:at + 5])
+        m.prefill(at + 5, with_logits=True, digits=2)
+        assert u.rms_error(got, m.last_logits()) < 2e-2, at
