@@ -13,6 +13,7 @@ namespace {
 // Forms of a step: 0, the attention's records are merged by a launch of their own; else by the output products, up to so many of them, 128 keys each
 constexpr size_t kStepRecords[] = {0, 2, 4, 8, 12}, kMostRecords = 12;
 constexpr size_t kDecodeSlice = 64;  // queries per call where a portion takes a decode form of its attention
+constexpr size_t kRecordStep = size_t(8) << 20;  // bytes that the room of a portion's records grows by (17 to 34 MB at most, for heads of 128 to 256 columns)
 size_t up_to(size_t v, size_t a) { return (v + a - 1) / a * a; }
 }  // namespace
 
@@ -253,7 +254,9 @@ int StackModel::grow(Buffer &b, size_t bytes) {
     }
     b.p = nullptr;
     b.bytes = 0;
-    HCHK(hipMalloc(&b.p, bytes));
+    const hipError_t e = hipMalloc(&b.p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();  // (the call's error, not the next launch's)
+    HCHK(e);
     HCHK(hipMemset(b.p, 0, bytes));
     HCHK(hipDeviceSynchronize());
     b.bytes = bytes;
@@ -974,8 +977,22 @@ int StackModel::step(bool with_logits, int form) {
 
 // ---- a portion of n tokens --------------------------------------------------------------------------------------------
 
-int StackModel::portion_buffers(size_t n) {
-    if (n <= rows_cap_) return 0;
+// what n tokens behind pos0 others need; nothing is allocated behind the first launch
+int StackModel::portion_buffers(size_t n, size_t pos0) {
+    if (n > rows_cap_) TRY(portion_rows(n));
+    size_t records = 0;
+    for (size_t i = 0; i < layers_.size(); ++i) {
+        if (f32_ || spec_.layers[i].mixer != LayerSpec::Attention) continue;
+        const bitnet_hip_gqa a = gqa_args(i, 0, prow_.p, layers_[i].block[0].main, false);
+        if (bitnet_hip_gqa_supported(a.dimp, a.vdimp)) records = std::max(records, bitnet_hip_gqa_prefill_scratch_bytes(&a, pos0 + n, n));
+    }
+    const int rc = grow(pscratch_, up_to(records, kRecordStep));  // (in few steps: what a later portion of the sequence needs is mostly there)
+    if (rc != 0) rows_cap_ = 0;  // (what lay there for others is gone, too)
+    return rc;
+}
+
+// buffers by a portion's tokens alone
+int StackModel::portion_rows(size_t n) {
     hidden_ = nullptr;  // (it may lie in what is given back here)
     n = up_to(n, 64);
     const size_t es = f32_ ? 4 : 2;
@@ -1149,8 +1166,6 @@ int StackModel::portion_block(size_t i, int pass, int which, size_t n, size_t po
         BCHK(bitnet_hip_gqa_rows_dev(&a, proj, ld, f32_, f32_, pos_, n, conv ? pqc_.p : nullptr, ldq, stream_));
         if (conv) BCHK(bitnet_hip_conv_keep_dev(proj, ld, f32_, L.channels, a.taps, L.slots[(size_t)pass].ring, pos_, n, stream_));
         if (!f32_ && bitnet_hip_gqa_supported(a.dimp, a.vdimp)) {
-            const size_t bytes = bitnet_hip_gqa_prefill_scratch_bytes(&a, pos0 + n, n);
-            TRY(grow(pscratch_, bytes));
             BCHK(bitnet_hip_gqa_prefill_scratch_dev(&a, (const uint16_t *)q, ldq, pos0 + n, n, (uint16_t *)row, ld, (float *)pscratch_.p, pscratch_.bytes, stream_));
         } else {
             for (size_t s = 0; s < n; s += kDecodeSlice) {
@@ -1265,7 +1280,6 @@ int StackModel::portion_linear(size_t i, int pass, size_t n) {
 // tokens pos0 .. pos0 + n - 1 of the history through every layer; px_ holds the residual stream, *pos_ stays at pos0
 int StackModel::portion(int rows, int pos0) {
     const size_t n = rows, ldh = up_to(width_, 64);
-    TRY(portion_buffers(n));
     float *x = (float *)px_.p;
     const float *y = (const float *)py_.p;
     TRY(embed_rows(n, x));
@@ -1314,7 +1328,7 @@ int StackModel::prefill(int n, bool with_logits, int, float *elapsed_ms) {
     if (p < 0) return BITNET_HIP_ERR_GPU;
     if (n <= 0 || p + n > host_forced_) return fail_arg("prefill: feed() the prompt tokens first");
     if (p + n > max_pos_ - 1) return fail_arg("KV cache overflow");
-    TRY(portion_buffers(n));
+    TRY(portion_buffers(n, p));
     hipStream_t s = (hipStream_t)stream_;
     HCHK(hipEventRecord(begin_.e, s));
     TRY(portion(n, p));

@@ -284,7 +284,8 @@ class StackModel : public Sequence {
     int portion_linear(size_t i, int pass, size_t n);
     int portion_block(size_t i, int pass, int which, size_t n, size_t pos0);
     int portion_loop_in(size_t n);
-    int portion_buffers(size_t n);
+    int portion_buffers(size_t n, size_t pos0);
+    int portion_rows(size_t n);
 
     StackSpec spec_;
     bool f32_ = false;

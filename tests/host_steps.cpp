@@ -76,7 +76,7 @@ hipError_t hipGraphExecDestroy(hipGraphExec_t e) { return delete reinterpret_cas
 hipError_t hipGraphDestroy(hipGraph_t g) { return delete reinterpret_cast<Graph *>(g), hipSuccess; }
 
 size_t bitnet_hip_gqa_scratch_bytes(size_t, size_t, size_t, size_t) { return 256; }
-size_t bitnet_hip_gqa_prefill_scratch_bytes(const bitnet_hip_gqa *, size_t n_ctx, size_t nq) { return n_ctx > nq ? n_ctx * 4096 : 0; }
+size_t bitnet_hip_gqa_prefill_scratch_bytes(const bitnet_hip_gqa *, size_t n_ctx, size_t nq) { return n_ctx > nq ? n_ctx * 16384 : 0; }
 int bitnet_hip_gqa_supported(size_t, size_t) { return g_narrow; }
 size_t bitnet_hip_gqa_out_records(const bitnet_hip_gqa *, size_t) { return 4; }
 size_t bitnet_hip_gqa_project_records(const bitnet_hip_gqa *, size_t) { return 12; }
@@ -262,6 +262,32 @@ int wide_heads() {
     return 0;
 }
 
+// everything that a portion needs is there ahead of its first launch; where it cannot be had, nothing has run
+int portion_room() {
+    Model m(4000);
+    START(m);
+    for (int n : {100, 300, 64, 700, 20, 1000}) {
+        const int p = m.position();
+        CHECK(m.feed(m.tokens.data() + p, n) == 0);
+        g_done.clear();
+        CHECK(m.prefill(n, false, 0, nullptr) == 0 && count("prefill") == 2);
+        bool launched = false;
+        for (const std::string &s : g_done) {
+            launched = launched || (s != "malloc" && s != "free");
+            CHECK(!launched || (s != "malloc" && s != "free"));
+        }
+    }
+    g_largest_block = 45 << 20;  // (the records of 2184 + 900 positions take more)
+    const int p = m.position();
+    CHECK(m.feed(m.tokens.data() + p, 900) == 0);
+    g_done.clear();
+    CHECK(m.prefill(900, false, 0, nullptr) != 0 && m.position() == p && g_last_error == hipSuccess);
+    for (const std::string &s : g_done) CHECK(s == "malloc" || s == "free");
+    g_largest_block = ~size_t(0);
+    CHECK(m.prefill(900, false, 0, nullptr) == 0 && m.position() == p + 900 && m.last() == m.tokens[(size_t)p + 899]);
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, int (*)()> cases = {
         {"last_row", last_row},
@@ -269,6 +295,7 @@ int main(int argc, char **argv) {
         {"chain_refused", chain_refused},
         {"prepared", prepared},
         {"wide_heads", wide_heads},
+        {"portion_room", portion_room},
     };
     const auto it = cases.find(argc > 1 ? argv[1] : "");
     CHECK(it != cases.end());

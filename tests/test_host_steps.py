@@ -53,3 +53,7 @@ def test_no_run_captures_behind_prepare_graphs(program):
 
 def test_output_products_merge_the_records_of_any_head(program):
     check(program, "wide_heads")
+
+
+def test_a_portion_allocates_nothing_behind_its_first_launch(program):
+    check(program, "portion_room")
