@@ -132,7 +132,7 @@ __global__ __launch_bounds__(256) void k_argmax_embed(const float *best_val, con
 #pragma unroll
     for (int i = 0; i < 4; ++i) better(sv[i], si[i]);
     const int token = bi == 0x7fffffff ? 0 : bi;
-    if (!forced) fetch(token);
+    if (!forced) fetch(min(token, e.vocab - 1));  // (there may be more logits than rows)
     if (tid == 0) {
         if (token_out) *token_out = token;
         if (!forced) history[at] = token;
