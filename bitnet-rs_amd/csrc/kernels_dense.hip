@@ -1366,7 +1366,9 @@ static FormedSplit formed_split(const GemvArgs &a) {
 }
 // What k_dense_gemv_formed takes: a vector to be formed, whole in eights, it and the weights on 16 bytes (a lane's columns are inside or outside as one, and loads past the end give zeros, so that an
 // infinite weight counts for its own row alone), more than half a wave's columns and no more than two chunks for each of eight waves.  Past 2^26 weights (a head) memory is all that
-// counts and k_dense_gemv, whose waves take whole rows, is as fast or faster: us there / here 32768 x 1536 21.7 / 18.9, 16384 x 2560 19.3 / 16.9, 32768 x 3072 35.9 / 36.7, 128256 x 2560 100.2 / 101.2.
+// counts and k_dense_gemv, whose waves take whole rows, is as fast or faster: us there / here 32768 x 1536 21.7 / 18.9, 16384 x 2560 17.8 / 15.8, 32768 x 3072 35.9 / 36.7, 128256 x 2560 100.2 / 101.2.
+// Below, of 10 widths from 1024 to 8192 columns by 8 sizes from 4 to 64 million weights and 28 round shapes, this form is faster at all but one: 3072 columns behind one rms norm where k_dense_gemv's
+// rounds of 3072 rows are whole, 11264 rows 14.56 / 14.60, 12000 14.5 / 14.9, 12288 15.2 / 15.4, and 12289 15.6 / 15.2, 13029 17.4 / 15.7 again; no line by sizes keeps those rows and no others.
 static bool gemv_is_formed(const GemvArgs &a) {
     const VecIn &in = a.in;
     const uintptr_t all = (uintptr_t)in.x | (uintptr_t)in.y | (uintptr_t)in.post_weight | (uintptr_t)in.scale | (uintptr_t)in.y_gate | (uintptr_t)in.weight | (uintptr_t)in.bias |
@@ -1407,6 +1409,10 @@ static hipError_t launch_gemv_formed(const GemvArgs &a, int *n_wg_out, hipStream
             if (per == 1 || cost <= least) least = cost, each = 4 * n;
         }
         each = std::min({each, 64 * waves, kFormedRows});
+        // Workgroups that begin a multiple of 256 KiB apart wait for the same memory where two per CU run at once, or nearly: four rows more.  us, k_dense_gemv / without / with it, rms norm | added and
+        // normed twice: 16384 x 4096 25.6 / 27.7 / 23.3 | 25.7 / 26.4 / 24.1, 15000 x 4096 23.5 / 23.9 / 22.0 | 25.0 / 23.6 / 22.6, 8192 x 8192 32.5 / 30.8 / 24.8 | 43.6 / 31.6 / 26.9.  Fewer
+        // workgroups: 7000 x 8192 (438) 24.6 / 23.8 | 25.9 / 25.8, 6200 x 8192 (388) 23.1 / 23.3 | 24.7 / 25.3.
+        if ((size_t)each * a.ld * 2 % ((size_t)1 << 18) == 0 && (a.rows + each - 1) / each > 448 && each + 4 <= std::min(64 * waves, kFormedRows)) each += 4;
     }
     k.rows_wg = each;
     const int n_wg = (a.rows + each - 1) / each;

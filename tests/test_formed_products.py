@@ -103,3 +103,16 @@ def test_formed_input_and_greedy_token(hip, pkg, vocab, cols):
     hip._call("dense_logits_dev", C.byref(vi), C.c_void_p(p[2]), C.c_size_t(vocab), C.c_size_t(cols), C.c_size_t(ld), C.c_void_p(p[3]), C.c_void_p(p[4]), C.c_void_p(p[5]), None, None, None, None)
     want = w.astype(np.float64) @ so.norm_plain(x.astype(np.float64), nw, 1e-3)
     assert u.rms_error(u.host(logits), want) < F32_TOL and int(u.host(token)[0]) == int(np.argmax(want))
+
+
+@pytest.mark.parametrize("rows,cols,ld", [(16001, 520, 8192), (7300, 1032, 16384)])
+def test_formed_input_of_rows_a_power_of_two_apart(hip, pkg, rows, cols, ld):
+    """workgroups that would begin a multiple of 256 KiB apart take four rows more: of two waves, and of three"""
+    import torch
+
+    g, (x, _, nw, *_) = vectors(cols, rows)
+    w, out = u.rounded(g.standard_normal((rows, cols)) / np.sqrt(cols)), u.zeros_f32(rows)
+    wd = torch.zeros((rows, ld), dtype=torch.int16, device="cuda")
+    wd[:, :cols] = u.dev_bf16(w).view(torch.int16).reshape(rows, cols)
+    hip.dense_gemv_dev(u.dev_f32(x), wd, rows, cols, ld, out, n=cols, kind=pkg.IN_NORM, eps=1e-3, weight=u.dev_f32(nw))
+    assert u.rms_error(u.host(out), w.astype(np.float64) @ so.norm_plain(x.astype(np.float64), nw, 1e-3)) < F32_TOL
