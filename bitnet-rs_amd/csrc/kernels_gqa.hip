@@ -751,25 +751,23 @@ hipError_t launch_gqa_merge(const Gqa &g, const int *pos, int q0, int nq, const 
 }
 
 // ---- records -> output -> product -------------------------------------------------------------------------------------
-// The merge of up to four records and the product behind it in one launch: every workgroup forms the whole output in LDS, as k_dense_gemv forms its input, and its waves take rows of the
-// product.  Nothing that is requested hangs on the position: a thread asks for all NB records of its columns, with their maxima and sums, and makes their weights itself; what the position
-// says only masks them.  The product's weights go out behind.  us per layer with this launch against the merge's and the product's, steps of the layer stacks: 1536 columns of 12 heads
-// -3.0 (up to 256 keys) and -2.2 (512), 2560 of 20 -1.9 and -0.9, 3072 of 24 -2.2 and -1.5; with half waves that reduce up to 32 records over LDS, 1024 keys are even and 2000 lose 1.5 to 6.  (Against k_dense_gemv's product;
-// k_dense_gemv_plain's is 0.7, 0.2 and 0.2 faster at these three widths, which leaves -2.3 / -1.5, -1.7 / -0.7 and -2.0 / -1.3.)
+// The merge of up to four records and the product behind it in one launch, for weights that begin off four bytes (k_gqa_project below takes all others, more records and every step of the models): every
+// workgroup forms the whole output in LDS, as k_dense_gemv forms its input, and its waves take rows of the product.  Nothing that is requested hangs on the position: a thread asks for all records
+// of its columns, with their maxima and sums, and makes their weights itself; what the position says only masks them.  The product's weights go out behind.
 struct GqaOutK {
     Gqa g;
     const int *pos;
     const float *scratch, *bias;
     const uint16_t *w;
     float *y;
-    int rows, cols, ld, kp;
+    int rows, cols, ld, kp, records;
     unsigned magic;  // ceil(2^20 / pieces of a head)
 };
+constexpr int kOutRecords = 4, kOutPieces = 4, kOutChunks = 3;  // records, pieces of four columns per thread, chunks of 512 columns in flight
 
-// R rows per wave, U chunks of 512 columns in flight; NU: pieces of four columns per thread
-template <int R, int U, int NU, int NB>
 __global__ __launch_bounds__(256) void k_gqa_out(GqaOutK p) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
+    constexpr int NU = kOutPieces, NB = kOutRecords, U = kOutChunks;
     const Gqa &g = p.g;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, vdimp = (int)g.vdimp, pieces = (int)g.heads * (vdimp >> 2);
     const int here = *p.pos;
@@ -779,10 +777,12 @@ __global__ __launch_bounds__(256) void k_gqa_out(GqaOutK p) {
     float sink[NU], z[NU];
 #pragma unroll
     for (int j = 0; j < NU; ++j) {
+        if (j > 0 && 256 * j >= pieces) continue;
         const int u = min(tid + 256 * j, pieces - 1), h = (int)((unsigned)u * p.magic >> 20);
         const float *rec = p.scratch + (unsigned)h * (kGqaSplits * stride), *v = rec + kGqaRecHead + (u - h * (vdimp >> 2)) * 4;
 #pragma unroll
         for (int e = 0; e < NB; ++e) {
+            if (e >= 2 && p.records <= 2) continue;
             ml[j][e] = *reinterpret_cast<const float2 *>(rec + e * stride);
             vec[j][e] = *reinterpret_cast<const f32x4 *>(v + e * stride);
         }
@@ -791,21 +791,19 @@ __global__ __launch_bounds__(256) void k_gqa_out(GqaOutK p) {
         zc[j] = g.gate && g.gate_columns ? *reinterpret_cast<const f32x4 *>((const float *)g.gate + 4 * u) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
     const int l8 = lane * 8, last_col = p.cols - 8;
-    u32x4 w[R][U];
-    auto fetch = [&](int grp, int k0) {
+    u32x4 w[U];
+    auto fetch = [&](int row, int k0) {
+        const uint16_t *wr = p.w + (size_t)row * p.ld;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const uint16_t *wr = p.w + (size_t)min(grp * R + r, p.rows - 1) * p.ld;
-#pragma unroll
-            for (int u = 0; u < U; ++u) w[r][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(wr + min(k0 + u * 512 + l8, last_col)));
-        }
+        for (int u = 0; u < U; ++u) w[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(wr + min(k0 + u * 512 + l8, last_col)));
     };
-    int grp = blockIdx.x * 4 + wave;
-    const int n = gridDim.x * 4, groups = (p.rows + R - 1) / R;
-    if (grp < groups) fetch(grp, 0);
-    const int used = gqa_range(g, here).used;
+    int row = blockIdx.x * 4 + wave;
+    const int n = gridDim.x * 4;
+    if (row < p.rows) fetch(row, 0);
+    const int used = min(gqa_range(g, here).used, p.records <= 2 ? 2 : NB);
 #pragma unroll
     for (int j = 0; j < NU; ++j) {
+        if (j > 0 && 256 * j >= pieces) continue;
         float M = sink[j], den = 0.f, e2[NB];
 #pragma unroll
         for (int e = 0; e < NB; ++e) M = e < used ? fmaxf(M, ml[j][e].x) : M;
@@ -828,83 +826,56 @@ __global__ __launch_bounds__(256) void k_gqa_out(GqaOutK p) {
     }
     for (int i = 4 * pieces + tid; i < p.kp; i += 256) xs[i] = 0.f;
     __syncthreads();
-    for (; grp < groups; grp += n) {
-        float acc[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] = 0.f;
+    for (; row < p.rows; row += n) {
+        float acc = 0.f;
         for (int k0 = 0; k0 < p.kp; k0 += U * 512) {
-            u32x4 c[R][U];
+            u32x4 c[U];
 #pragma unroll
-            for (int r = 0; r < R; ++r)
-#pragma unroll
-                for (int u = 0; u < U; ++u) c[r][u] = w[r][u];
+            for (int u = 0; u < U; ++u) c[u] = w[u];
             if (k0 + U * 512 < p.kp)
-                fetch(grp, k0 + U * 512);
-            else if (grp + n < groups)
-                fetch(grp + n, 0);
+                fetch(row, k0 + U * 512);
+            else if (row + n < p.rows)
+                fetch(row + n, 0);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const f32x4 x0 = *reinterpret_cast<const f32x4 *>(xs + k0 + u * 512 + l8), x1 = *reinterpret_cast<const f32x4 *>(xs + k0 + u * 512 + l8 + 4);
+                const f32x4 x[2] = {*reinterpret_cast<const f32x4 *>(xs + k0 + u * 512 + l8), *reinterpret_cast<const f32x4 *>(xs + k0 + u * 512 + l8 + 4)};
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const u32x4 q = c[r][u];
-                    acc[r] = fmaf(x0.x, __builtin_bit_cast(float, q.x << 16), acc[r]);
-                    acc[r] = fmaf(x0.y, __builtin_bit_cast(float, q.x & 0xffff0000u), acc[r]);
-                    acc[r] = fmaf(x0.z, __builtin_bit_cast(float, q.y << 16), acc[r]);
-                    acc[r] = fmaf(x0.w, __builtin_bit_cast(float, q.y & 0xffff0000u), acc[r]);
-                    acc[r] = fmaf(x1.x, __builtin_bit_cast(float, q.z << 16), acc[r]);
-                    acc[r] = fmaf(x1.y, __builtin_bit_cast(float, q.z & 0xffff0000u), acc[r]);
-                    acc[r] = fmaf(x1.z, __builtin_bit_cast(float, q.w << 16), acc[r]);
-                    acc[r] = fmaf(x1.w, __builtin_bit_cast(float, q.w & 0xffff0000u), acc[r]);
+                for (int i = 0; i < 4; ++i) {
+                    acc = fmaf(x[i >> 1][2 * i & 3], __builtin_bit_cast(float, c[u][i] << 16), acc);
+                    acc = fmaf(x[i >> 1][(2 * i & 3) + 1], __builtin_bit_cast(float, c[u][i] & 0xffff0000u), acc);
                 }
             }
         }
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
-        if (lane == 0)
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                if (grp * R + r < p.rows) p.y[grp * R + r] = acc[r] + (p.bias ? p.bias[grp * R + r] : 0.f);
+        acc = wave_sum(acc);
+        if (lane == 0) p.y[row] = acc + (p.bias ? p.bias[row] : 0.f);
     }
 }
 
 // the most records that one launch may take in place of two; 0: none
 int gqa_out_records(const Gqa &g, int cols) {
     if (g.maps != 1 || g.heads * g.vdimp > 4096 || (size_t)cols < g.heads * g.vdimp || cols > 4096 || (g.gate && !g.gate_f32)) return 0;
-    return 4;
+    return kOutRecords;
 }
 
 hipError_t launch_gqa_out(const GqaOut &a, hipStream_t s) {
     if (a.records < 1 || a.records > gqa_out_records(a.g, a.cols)) return hipErrorInvalidValue;
+    // (its loads want four bytes; us, an instance of k_gqa_out for these sizes / this, weights on sixteen bytes and on eight, at 200 | 500 keys: 12 heads of 128, 1536 rows 3.3 / 2.9 | 3.9 / 3.0; 24, 3072 rows
+    // 5.2 / 4.3 | 6.3 / 4.7; 32 of 64, 3072 rows 4.0 / 4.1 | 5.1 / 4.4.  The one instance that is left, against those: 3.3 / 3.8 | 4.0 / 4.1; 5.3 / 6.0 | 6.5 / 6.8; 4.1 / 5.1 | 5.1 / 5.8)
+    if ((uintptr_t)a.w % 4 == 0 && a.ld <= 32768) return launch_gqa_project(a, s);
     GqaOutK k;
-    k.g = a.g, k.pos = a.pos, k.scratch = a.scratch, k.bias = a.bias, k.w = a.w, k.y = a.y, k.rows = a.rows, k.cols = a.cols, k.ld = a.ld;
-    const int chunks = (a.cols + 511) / 512, u = chunks % 3 == 0 ? 3 : chunks % 4 == 0 ? 4 : chunks < 3 ? chunks : 5, pieces = (int)(a.g.heads * a.g.vdimp / 4);
-    k.kp = (chunks + u - 1) / u * u * 512;
+    k.g = a.g, k.pos = a.pos, k.scratch = a.scratch, k.bias = a.bias, k.w = a.w, k.y = a.y, k.rows = a.rows, k.cols = a.cols, k.ld = a.ld, k.records = a.records;
+    k.kp = (a.cols + 512 * kOutChunks - 1) / (512 * kOutChunks) * (512 * kOutChunks);
     k.magic = ((1u << 20) + a.g.vdimp / 4 - 1) / (unsigned)(a.g.vdimp / 4);
-    // (four records of many heads: half the workgroups, which each merge them; us per layer of Lurepel 3b, R = 1 / 2: up to two records -2.2 / -1.7 against the two launches, up to four
-    // -0.8 / -1.5; of its 1b, 1536 rows, -3.0 / -3.0 and -2.2 / -2.1)
-    const int r = a.records > 2 && a.rows >= 2048 ? 2 : 1;
-    int n_wg = (a.rows + 4 * r - 1) / (4 * r);
+    int n_wg = (a.rows + 3) / 4;
     if (n_wg > 768) {
         const int rounds = (n_wg + 767) / 768;
         n_wg = (n_wg + rounds - 1) / rounds;
     }
-    auto pick_r = [&](auto rr, auto nu, auto nb) {
-        constexpr int N = decltype(nu)::value, B = decltype(nb)::value, R = decltype(rr)::value;
-        return u == 1 ? k_gqa_out<R, 1, N, B> : u == 2 ? k_gqa_out<R, 2, N, B> : u == 3 ? k_gqa_out<R, 3, N, B> : u == 4 ? k_gqa_out<R, 4, N, B> : k_gqa_out<R, 5, N, B>;
-    };
-    auto of = [&](auto rr, auto nb) {
-        return pieces <= 512 ? pick_r(rr, std::integral_constant<int, 2>(), nb) : pieces <= 768 ? pick_r(rr, std::integral_constant<int, 3>(), nb) : pick_r(rr, std::integral_constant<int, 4>(), nb);
-    };
-    const std::integral_constant<int, 1> one;
-    const std::integral_constant<int, 2> two;
-    const std::integral_constant<int, 4> four;
-    auto fn = a.records <= 2 ? of(one, two) : r == 1 ? of(one, four) : of(two, four);
-    hipLaunchKernelGGL(fn, dim3(n_wg), dim3(256), (size_t)k.kp * sizeof(float), s, k);
+    hipLaunchKernelGGL(k_gqa_out, dim3(n_wg), dim3(256), (size_t)k.kp * sizeof(float), s, k);
     return hipGetLastError();
 }
 
-// Up to eight records on the lanes of k_dense_gemv_formed (dense.hpp, SharedRows): each merges the records of its own eight columns in registers, for all rows of its workgroup, and nothing goes
+// Up to twelve records on the lanes of k_dense_gemv_formed (dense.hpp, SharedRows): each merges the records of its own eight columns in registers, for all rows of its workgroup, and nothing goes
 // through LDS ahead of the products.  As above nothing that is requested hangs on the position.
 struct GqaProjectK {
     Gqa g;

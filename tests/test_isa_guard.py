@@ -271,7 +271,7 @@ def test_products_of_records_and_experts_keep_no_scratch(tmp_path):
     merges the attention's records holds all of them in registers; both instantiated for what their launches choose and nothing else"""
     if not os.path.exists(HIPCC):
         pytest.skip("no hipcc")
-    for src, kernel, count, waves in (("kernels_experts.hip", "k_experts_out", 16, 3), ("kernels_gqa.hip", "k_gqa_out", 45, 2)):
+    for src, kernel, count, waves in (("kernels_experts.hip", "k_experts_out", 16, 3), ("kernels_gqa.hip", "k_gqa_out", 1, 2)):
         _, usage = _compile(src, str(tmp_path))
         found = {name: u for name, u in usage.items() if kernel in name}
         assert len(found) == count, (kernel, len(found))

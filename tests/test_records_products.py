@@ -49,6 +49,31 @@ def test_records_merged_by_lanes(hip, pkg, heads, vdimp, rows, extra, pos, chunk
     assert u.rms_error(u.host(y), w[:, :n].astype(np.float64) @ out.reshape(-1) + bias) < F32_TOL
 
 
+@pytest.mark.parametrize("heads,vdimp,rows,extra,pos", [(1, 32, 5, 0, 0), (12, 128, 1536, 0, 200), (3, 160, 70, 32, 511), (4, 1024, 9, 0, 300), (7, 96, 3100, 32, 130)])
+def test_weights_off_sixteen_bytes(hip, pkg, heads, vdimp, rows, extra, pos):
+    """gqa_out's own kernel (weights off four bytes), and the lanes' product of weights on eight: as of the same weights on sixteen bytes, up to the order of sums"""
+    g = np.random.default_rng([heads, vdimp, rows])
+    n, used = heads * vdimp, pos // 128 + 1
+    rec = np.full((heads, 128, 4 + vdimp), np.nan, np.float32)
+    rec[:, :used, 0], rec[:, :used, 1] = 3 * g.standard_normal((heads, used)), g.uniform(0.5, 60.0, (heads, used))
+    rec[:, :used, 4:] = g.standard_normal((heads, used, vdimp))
+    scratch, some, gate = u.dev_f32(rec.reshape(-1)), u.zeros_f32(64), u.dev_f32(g.standard_normal(n))
+    attn = pkg.Gqa(heads, 1, 1, 32, 32, vdimp, vdimp, 1024, 1e-5, 0.0, 1.0, 0, 0, *[some.data_ptr()] * 3, gate=gate.data_ptr(), ldgate=n, gate_f32=1, gate_columns=1)
+    cols = u.up_to(n, 64) + extra
+    ld = u.up_to(cols, 64)
+    w = u.bf16_bits(u.padded(u.rounded(g.standard_normal((rows, cols)) / np.sqrt(n)), ld)).view(np.int16).reshape(-1)
+    on, eight, off = (u.dev(np.concatenate([np.zeros(k, np.int16), w]))[k:] for k in (0, 4, 1))
+    assert off.data_ptr() % 16 == 2
+    got = []
+    for weights in (on, eight, off):
+        y = u.zeros_f32(rows)
+        hip.gqa_out_dev(attn, pos_dev(pos), used, scratch, weights, rows, cols, ld, y)
+        got.append(u.host(y))
+    assert np.array_equal(got[1], got[0]) and u.rms_error(got[2], got[0]) < F32_TOL
+    with pytest.raises(pkg.BitNetHipError, match="bad arguments"):
+        hip.gqa_project_dev(attn, pos_dev(pos), used, scratch, eight, rows, cols, ld, u.zeros_f32(rows))
+
+
 def test_steps_across_the_forms(pkg, tmp_path):
     """a Lurepel model's steps around 128, 256, 512, 1024 and 1536 keys: as a prompt of all tokens gives them"""
     import importlib
