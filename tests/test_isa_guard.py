@@ -277,3 +277,20 @@ def test_products_of_records_and_experts_keep_no_scratch(tmp_path):
         assert len(found) == count, (kernel, len(found))
         for name, u in found.items():
             assert u["ScratchSize"] == 0 and u["Occupancy"] >= waves, (name, u)
+
+
+def test_prompt_attention_and_merging_products_fit_their_registers(tmp_path):
+    """k_gqa_prefill counts on two waves per SIMD (one where a head has 256 columns, whose two maps spill 52 bytes), k_gqa_project on its records in registers; in exactly the instances that launches choose"""
+    if not os.path.exists(HIPCC):
+        pytest.skip("no hipcc")
+    _, usage = _compile("kernels_gqa.hip", str(tmp_path))
+    prefill = {name: u for name, u in usage.items() if "k_gqa_prefill" in name}
+    assert len(prefill) == 21
+    for name, u in prefill.items():
+        wide = "k_gqa_prefillILi8ELi16E" in name
+        assert u["ScratchSize"] <= (52 if "k_gqa_prefillILi8ELi16ELi2E" in name else 0) and u["Occupancy"] >= (1 if wide else 2), (name, u)
+        assert wide or u["VGPRs"] + u["AGPRs"] <= 230, (name, u)
+    project = {name: u for name, u in usage.items() if "k_gqa_project" in name}
+    assert len(project) == 4
+    for name, u in project.items():
+        assert u["ScratchSize"] == 0 and u["Occupancy"] >= 3, (name, u)
