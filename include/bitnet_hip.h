@@ -850,8 +850,8 @@ int bitnet_hip_gqa_project_dev(const bitnet_hip_gqa *attn, const int32_t *pos_de
 /* A portion of a prompt, bf16: the LAST nq of n_ctx positions attend (all of them in the caches); q as gqa_rows leaves it. */
 int bitnet_hip_gqa_prefill_dev(const bitnet_hip_gqa *attn, const uint16_t *q_dev, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out_dev, size_t ldo,
                                void *stream);
-/* The same with room (on 16 bytes) for records of stretches of a block's keys, merged behind it: few queries behind many keys leave most of the chip idle otherwise.  scratch_bytes 0: the
- * keys stay together, and scratch may be NULL. */
+/* The same with room (on 16 bytes) for records of stretches of a block's keys, merged behind it: few queries behind many keys leave most of the chip idle otherwise.  Where
+ * gqa_prefill_scratch_bytes gives 0 the keys stay together, and scratch may be NULL; elsewhere the call wants at least that many bytes (gqa_prefill wants none). */
 size_t bitnet_hip_gqa_prefill_scratch_bytes(const bitnet_hip_gqa *attn, size_t n_ctx, size_t nq);
 int bitnet_hip_gqa_prefill_scratch_dev(const bitnet_hip_gqa *attn, const uint16_t *q_dev, size_t ldq, size_t n_ctx, size_t nq, uint16_t *out_dev, size_t ldo, float *scratch_dev,
                                        size_t scratch_bytes, void *stream);

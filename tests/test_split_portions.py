@@ -43,3 +43,22 @@ def test_chunked_portion_in_stretches(hip, pkg, shape, n, nq):
     outs, _ = both(hip, t, rows, t.ld, n, nq)
     t.check(outs[1], n - nq, 2e-2)
     assert u.rms_error(u.host(outs[1]), u.host(outs[0])) < 4e-3
+
+
+def test_room_is_wanted_where_there_are_stretches(hip, pkg):
+    """no room, too little of it or room off sixteen bytes is refused where keys are shared out, and none is needed where they are not"""
+    t = Attention(pkg, 700, 4, 2, 24, 40, 2, False)
+    t.fill(hip, 0, 700)
+    rows, out = t.put(t.rows[570:]), t.new(130, 4 * t.vdimp)
+    size = hip.gqa_prefill_scratch_bytes(t.attn, 700, 130)
+    room = u.zeros_f32(size // 4 + 4)
+    for scratch, n in ((None, 0), (None, size), (room, size - 1), (room[1:], size)):
+        with pytest.raises(pkg.BitNetHipError, match="scratch of"):
+            hip.gqa_prefill_scratch_dev(t.attn, rows, t.ld, 700, 130, out, 4 * t.vdimp, scratch, n)
+    assert not u.host(out).any()
+    hip.gqa_rows_dev(t.attn, rows, t.ld, False, False, pos_dev(570), 130)
+    assert hip.gqa_prefill_scratch_bytes(t.attn, 130, 130) == 0
+    hip.gqa_prefill_scratch_dev(t.attn, rows, t.ld, 130, 130, out, 4 * t.vdimp, None, 0)
+    want = t.new(130, 4 * t.vdimp)
+    hip.gqa_prefill_dev(t.attn, rows, t.ld, 130, 130, want, 4 * t.vdimp)
+    assert u.host(want).any() and (u.host(out) == u.host(want)).all()
