@@ -762,35 +762,33 @@ int StackModel::step_loop_in() {
     return 0;
 }
 
-// Does the block's output product take the attention's records as they are?  (nothing but them goes into it)
-bool StackModel::merges_in_out(size_t i, int which) const {
+// The attention's records that the block's output product merges as they are, at most; 0: none (nothing but them goes into it).  Every workgroup reads the records of all columns, a launch of its
+// own reads them once: past 3072 columns of heads of up to 128, nine to twelve are faster there.  us of attention and product at 1300 keys, 2048 rows, merged by a launch / by the product: 24 heads
+// of 128 12.4 / 12.3, 28 12.6 / 12.8, 32 12.8 / 13.3, 40 of 96 13.8 / 14.6, 64 of 64 11.9 / 12.6; 16 of 256 17.3 / 16.9; at 700 keys 32 of 128 12.9 / 12.4.
+size_t StackModel::merged_in_out(size_t i, int which) const {
     const Block &B = layers_[i].block[which];
-    if (f32_ || !B.used || !B.mixer || spec_.layers[i].mixer != LayerSpec::Attention || B.fs > 0 || B.expert_up.w) return false;
+    if (f32_ || !B.used || !B.mixer || spec_.layers[i].mixer != LayerSpec::Attention || B.fs > 0 || B.expert_up.w) return 0;
     const bitnet_hip_gqa a = gqa_args(i, 0, row_[0], B.main, true);
-    return bitnet_hip_gqa_project_records(&a, B.out.cols) >= kMostRecords;
-}
-
-// records of a query at the position, over the layers
-size_t StackModel::records_at(int pos) const {
-    size_t most = 0;
-    for (size_t i = 0; i < layers_.size(); ++i) {
-        if (!merges_in_out(i, 0)) continue;
-        const AttentionSpec &m = spec_.layers[i].attention;
-        int first = m.chunk > 0 ? pos / m.chunk * m.chunk : 0;
-        if (m.window > 0) first = std::max(first, pos - m.window + 1);
-        most = std::max(most, (size_t)(pos - first / 128 * 128) / 128 + 1);
-    }
-    return most;
+    if (bitnet_hip_gqa_project_records(&a, B.out.cols) < kMostRecords) return 0;
+    return a.vdimp <= 128 && a.heads * a.vdimp > 3072 ? 8 : kMostRecords;
 }
 
 // (up to twelve records: us of attention and product at 300 / 600 / 1500 keys, merged by a launch / by the product: 12 heads of 128 on 3 14.1 / 14.1 / 14.2 -> 11.9 / 12.2 / 13.0, 24 on 6
-// 17.2 / 17.2 / 17.4 -> 14.3 / 15.3 / 16.2, 32 on 8 at 1500 19.8 -> 19.4; with sixteen requested at once and the rest in turn even at 17, slower from there on.  Records of 256 keys, from twice the
+// 17.2 / 17.2 / 17.4 -> 14.3 / 15.3 / 16.2; with sixteen requested at once and the rest in turn even at 17, slower from there on.  Records of 256 keys, from twice the
 // waves, would reach 3072 keys: 14.7 -> 13.7 where the keys lie in the L2, but a pass's steps got slower, 7.50 -> 7.69 ms.  Heads of more than 256 columns, whose records come from
 // gqa_any, at 100 / 500 / 1500 keys: 8 of 512 69.5 / 85.9 / 88.2 -> 65.7 / 81.8 / 86.4, 12 of 320 50.3 / 61.8 / 63.6 -> 46.7 / 58.6 / 62.6)
 int StackModel::form_at(int pos) const {
-    const size_t n = records_at(pos);
     static_assert(sizeof(kStepRecords) / sizeof(kStepRecords[0]) == kForms, "a graph for each");
-    for (int f = 1; n > 0 && f < kForms; ++f)
+    size_t n = 0, most = 0;  // records of the layers whose products merge them, and what one of those products takes
+    for (size_t i = 0; i < layers_.size(); ++i) {
+        const size_t merged = merged_in_out(i, 0);
+        if (merged == 0) continue;
+        const AttentionSpec &m = spec_.layers[i].attention;
+        int first = m.chunk > 0 ? pos / m.chunk * m.chunk : 0;
+        if (m.window > 0) first = std::max(first, pos - m.window + 1);
+        n = std::max(n, (size_t)(pos - first / 128 * 128) / 128 + 1), most = std::max(most, merged);
+    }
+    for (int f = 1; n > 0 && n <= most && f < kForms; ++f)
         if (n <= kStepRecords[f]) return f;
     return 0;
 }
@@ -832,7 +830,7 @@ int StackModel::step_block(size_t i, int pass, int which) {
             BCHK(bitnet_hip_gqa_rows_dev(&a, proj, B.main, 1, f32_, pos_, 1, nullptr, 0, stream_));
             BCHK(bitnet_hip_gqa_any_dev(&a, proj, B.main, 1, f32_, pos_, 0, 1, scratch_, stream_));
         }
-        if (form_ > 0 && merges_in_out(i, which)) {
+        if (form_ > 0 && kStepRecords[form_] <= merged_in_out(i, which)) {
             BCHK(bitnet_hip_gqa_project_dev(&a, pos_, kStepRecords[form_], scratch_, B.out.w, B.out.rows, B.out.cols, B.out.ld, B.out_bias, y_[which], stream_));
             return 0;
         }

@@ -269,8 +269,7 @@ class StackModel : public Sequence {
     int step_side(size_t i);
     int step_linear(size_t i, int pass);
     int step_block(size_t i, int pass, int which);
-    bool merges_in_out(size_t i, int which) const;
-    size_t records_at(int pos) const;
+    size_t merged_in_out(size_t i, int which) const;
     int step_loop_in();
     // portion of n tokens
     int matmul(const void *a, size_t lda, bool a_f32, const Matrix &m, const float *bias, size_t n, int act0, int act1, size_t split, void *c, size_t ldc,

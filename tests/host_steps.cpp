@@ -140,15 +140,15 @@ using bitnet_host::LayerSpec;
     if (!(x)) return printf("%s:%d: %s\n", __FILE__, __LINE__, #x), 1
 
 struct Model : bitnet_host::StackModel {
-    static bitnet_host::StackSpec spec(int dim) {
+    static bitnet_host::StackSpec spec(int dim, int heads) {
         bitnet_host::StackSpec s;
         s.width = 64, s.vocab = 100, s.layers.resize(2);
-        for (LayerSpec &l : s.layers) l.mixer = LayerSpec::Attention, l.attention.heads = 2, l.attention.kv_heads = 1, l.attention.dim = l.attention.vdim = dim;
+        for (LayerSpec &l : s.layers) l.mixer = LayerSpec::Attention, l.attention.heads = heads, l.attention.kv_heads = 1, l.attention.dim = l.attention.vdim = dim;
         return s;
     }
     int rc = 0;
     std::vector<int32_t> tokens;
-    Model(int max_pos, int dim = 32) : StackModel(spec(dim), false, max_pos) {
+    Model(int max_pos, int dim = 32, int heads = 2) : StackModel(spec(dim, heads), false, max_pos) {
         std::vector<uint16_t> zeros(64 * 64 * 64);
         for (int i = 0; i < 2; ++i) {
             bitnet_host::StackLayerWeights w;
@@ -288,6 +288,19 @@ int portion_room() {
     return 0;
 }
 
+// nine to twelve records of many columns are merged by a launch of their own, fewer by the product, and no form of a step is made that is another's twin
+int many_columns() {
+    Model m(2000, 128, 28);
+    START(m);
+    CHECK(m.prepare_graphs(true) == 0 && g_made.size() == 8);  // forms of 2, 4 and 8 records and of a launch, one step and several
+    for (int at : {0, 500, 1023, 1024, 1500, 1600}) {
+        CHECK(m.reset() == 0 && m.feed(m.tokens.data(), at + 2) == 0 && (at == 0 || m.prefill(at, false, 0, nullptr) == 0));
+        g_done.clear();
+        CHECK(m.run(1, true, true, nullptr) == 0 && count("step") == 2 && count("project") == (at < 1024 ? 2 : 0) && count("merge") == (at < 1024 ? 0 : 2));
+    }
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const std::map<std::string, int (*)()> cases = {
         {"last_row", last_row},
@@ -296,6 +309,7 @@ int main(int argc, char **argv) {
         {"prepared", prepared},
         {"wide_heads", wide_heads},
         {"portion_room", portion_room},
+        {"many_columns", many_columns},
     };
     const auto it = cases.find(argc > 1 ? argv[1] : "");
     CHECK(it != cases.end());

@@ -57,3 +57,7 @@ def test_output_products_merge_the_records_of_any_head(program):
 
 def test_a_portion_allocates_nothing_behind_its_first_launch(program):
     check(program, "portion_room")
+
+
+def test_many_records_of_many_columns_take_a_launch_of_their_own(program):
+    check(program, "many_columns")

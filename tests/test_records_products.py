@@ -96,9 +96,10 @@ def test_steps_across_the_forms(pkg, tmp_path):
         assert u.rms_error(got, m.last_logits()) < 2e-2, at
 
 
-def test_steps_of_wide_heads_across_the_forms(pkg, tmp_path):
-    """heads of 288 columns, whose records come from gqa_any: the same, a prompt of the last five tokens against steps"""
-    config = u.lurepel([u.chunk_layer(heads=3, kv_heads=1, dim=288, scale=0.05, chunk=4096, dims=64)], width=112, vocab=150)
+@pytest.mark.parametrize("heads,kv_heads,dim", [(3, 1, 288), (28, 7, 128)])
+def test_steps_of_other_heads_across_the_forms(pkg, tmp_path, heads, kv_heads, dim):
+    """heads of 288 columns, whose records come from gqa_any, and 3584 columns, whose records past eight take a launch of their own: the same, a prompt of the last five tokens against steps"""
+    config = u.lurepel([u.chunk_layer(heads=heads, kv_heads=kv_heads, dim=dim, scale=0.05, chunk=4096, dims=64)], width=112, vocab=150)
     path = u.save_model(str(tmp_path), config, u.random_tensors(config, 8))
     m = pkg.open_model(path, max_pos=2048)
     tokens = np.random.default_rng(6).integers(0, 150, 1550).astype(np.int32)
