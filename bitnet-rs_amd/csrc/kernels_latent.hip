@@ -133,7 +133,8 @@ __global__ __launch_bounds__(256) void k_latent_decode_any(LatentAttn p) {
 // A workgroup's LDS leaves room for no second one on its compute unit, and the device alone knows how many of the launch's records exist: eight records of all heads and queries come
 // first, then the next eight, so that those that end at once come last.  With the records of the first heads ahead of the others' (all of 128, most to end at once) the last heads waited
 // for compute units that ended nothing: 40 heads at 100 keys 10.4 -> 8.4 us, 64 at 2000 keys 11.3 -> 9.4, 16 queries of 20 heads at 100 keys 59.7 -> 44.1; where every record exists the
-// order is worth nothing (40 heads at 8000 keys 17.3 -> 17.7).  The eight lie on eight XCDs, each with all heads of its records: L2 reads a record once.
+// order costs 1 to 4 % (40 heads at 8000 keys 17.3 -> 17.7, 16 queries of 64 heads at 4000 keys 156 -> 162; of 128 at 2000 225 -> 232), and 16 or 32 records at a time give that back only
+// together with what the order gains (16 queries of 20 heads at 100 keys 60.1 -> 44.7 with eight, 48.6 with 16, 57.7 with 32).  The eight lie on eight XCDs, each with all heads of its records: L2 reads a record once.
 constexpr int kDecKK = 20;  // most 32-column steps of ldc + ldr
 constexpr int kDecNT = 5;   // most 16-column tiles of ldc per wave
 constexpr int kCtStride = kLatentTile * 2 + 16;
